@@ -27,16 +27,9 @@
 // and `split`.
 #include <limits.h>
 
-#include "common.h"
+#include "mfma_attention.h"
 
 using namespace jle;
-
-typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
-typedef __attribute__((ext_vector_type(4))) float f32x4;
-typedef __attribute__((ext_vector_type(2))) unsigned int u32x2;
-typedef __attribute__((ext_vector_type(4))) unsigned int u32x4;  // (register arrays of HIP's uint4 may end up in scratch)
-
-constexpr float kLog2e = 1.4426950408889634f;
 
 __device__ __forceinline__ int first_key(int mode, int param, int pos) {
   if (mode == 1) return (pos / param) * param;
@@ -71,26 +64,6 @@ __device__ __forceinline__ float capped_log2(float v, const Biasing& b) {
 // the penalty in the exponent's base-2 units: r1 ln(x) log2(e) = r1 log2(x)
 __device__ __forceinline__ float penalty_log2(float r1, float r2, float back) {
   return r1 * __builtin_amdgcn_logf(fmaf(r2, back, 1.0f));
-}
-
-// Maximum / sum over the four lanes that hold one column (equal lane % 16), in all of them.  The two swaps
-// exchange the halves of the wavefront and neighbouring rows of 16 lanes: no trip through shared memory.
-__device__ __forceinline__ float column_max(float v) {
-  uint32_t u = __float_as_uint(v);
-  auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
-  v = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-  u = __float_as_uint(v);
-  r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
-  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-}
-
-__device__ __forceinline__ float column_sum(float v) {
-  uint32_t u = __float_as_uint(v);
-  auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
-  v = __uint_as_float(r[0]) + __uint_as_float(r[1]);
-  u = __float_as_uint(v);
-  r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
-  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
 // One step of 32 keys for the columns of a wavefront: mask the scores (MASKED; without it every key of the
@@ -826,14 +799,6 @@ __global__ __launch_bounds__(WAVES * 64, DH <= 128 ? 2 : 1) void attention_prefi
 // registers), the variants taking turns call by call: 26 % faster at 2,048 tokens, 24 % at 8,192 and 16,384; of that
 // 3 % are the loads (32 keys a step, three steps ahead), 14 % the 64 keys a step, 7 to 12 % the values as one 16-byte
 // read per element and the keys of a half asked for at once.
-// where piece p of key row r of a page tile lies: p ^ key_swizzle(r); the eight rows that eight neighbouring lanes read
-// (r % 4, r / 8 varying) then differ in the low three bits
-__device__ __forceinline__ int key_swizzle(int r) { return (r & 3) | ((r >> 3) << 2) | (((r >> 2) & 1) << 3); }
-
-__device__ __forceinline__ void load_to_lds16(const void* base, uint32_t byte_off, uint32_t lds_addr) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1\n" ::"v"(byte_off), "s"(base), "s"(lds_addr) : "memory");
-}
-
 // One step of 64 keys (four tiles of 16) for the columns of a wavefront: softmax_and_values for twice the keys, so
 // that the maxima, the sums and the accumulators' correction are done once per 64 keys.  st[ct][2 h + t][i]: the
 // score of key 32 h + 8 g + 4 t + i of the step (g: the lane's group of 16), so the lane's eight probabilities of a

@@ -109,6 +109,8 @@ _SIGNATURES = {
     "jle_mamba2_chunked_supported": [_i, _i],
     "jle_latent_down_prepare": [_vp, _i, _i, _vp, _f, _vp, _i, _i, _vp, _vp, _i, _i, _f, _vp, _f, _vp, _vp, _vp, _i, _vp,
                                 _i, _i, _i, _vp],
+    "jle_latent_expanded_gather": [_vp, _vp, _vp, _i, _vp, _i, _vp, _vp, _i, _i, _i, _vp],
+    "jle_latent_expanded_attention": [_vp, _i, _vp, _vp, _vp, _i, _vp, _vp, _vp, _i, _i, _f, _i, _vp, _vp],
     "jle_relu2": [_vp, _vp, _i, _ll, _vp],
     "jle_attention_prefill_kept": [_vp, _vp, _vp, _vp, _vp, _vp, _i, _vp, _i, _i, _i, _i, _f, _i, _i, _i, _i, _vp],
     "jle_paged_attention_kept": [_vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _f, _i, _i, _i, _i, _i, _i, _i, _i, _vp,
@@ -176,7 +178,8 @@ def _bind(path: str):
             fn.restype = ctypes.c_int
     for name, args in (("jle_attention_mfma_supported", [_i, _i, _i, _i]),  # queries, not launches: no stream
                        ("jle_gemm_stream_supported", [_i, _i, _i]), ("jle_gemm_f32_stream_supported", [_i, _i, _i]),
-                       ("jle_latent_attention_mfma_supported", [_i, _i, _i, _i, _i]), ("jle_attention_group_waves", []),
+                       ("jle_latent_attention_mfma_supported", [_i, _i, _i, _i, _i]),
+                       ("jle_latent_expanded_supported", [_i, _i, _i, _i, _i]), ("jle_attention_group_waves", []),
                        ("jle_mlstm_chunked_supported", [_i, _i]), ("jle_mlstm_chunk_tokens", []),
                        ("jle_gated_delta_padded", [_i]), ("jle_gated_unit_chunk_tokens", []),
                        ("jle_retention_chunk_tokens", []), ("jle_retention_chunked_supported", [_i, _i]),
@@ -699,6 +702,92 @@ class HipOps:
                    _p(rope_pages), _p(out), _p(positions), _p(token_segment), _p(block_table), block_table.shape[1],
                    window, float(scale), _p(plan), tiles, n, H, r, ps, splits, steps_per_split, _p(ws_ml), _p(ws_o),
                    _p(sink))
+        return out
+
+    # Which steps form every head's keys and values (attention_expanded.hip) instead of staying in the latent's space
+    # (attention_latent.hip).  Forming a key's costs as much as about 160 (query, key) pairs save where the step's tokens
+    # alone do not fill the card; where a token has at most 8 gathered keys both take what their launches take or the
+    # expanded form less.  One call with all it launches, 32 heads, latent 512, page 16 (latent's space | expanded,
+    # microseconds): one prompt of 512 tokens 129 | 59, of 2,048 837 | 107; 64 prompts of 20 107 | 74, of 40 196 | 80;
+    # behind cached tokens: 128 behind 1,024 101 | 72, 64 behind 2,048 95 | 101 (63 pairs a key), 64 behind 8,192
+    # 233 | 347, 512 behind 8,192 1,405 | 363, 256 behind 16,384 1,523 | 658 (254 pairs a key).
+    # The formed keys and values take no more than LATENT_EXPAND_BYTES.
+    LATENT_EXPAND_ROWS = 8
+    LATENT_EXPAND_PAIRS = 160
+    LATENT_EXPAND_BYTES = 1 << 30
+
+    @staticmethod
+    def expanded_plan(seg_lens, seg_starts, window: int):
+        """The gathered keys and the work of ``attention_expanded.hip``: ``(spans, blocks, rows, pairs)``.  ``spans``: per 64
+        gathered keys (segment, first position, first position a query needs, end); ``blocks``: (first token, tokens,
+        gathered row of position 0, 0), up to 128 consecutive tokens of a segment each, those with the most keys first;
+        ``rows``: the gathered keys, a multiple of 64; ``pairs``: the visible (query, key) pairs."""
+        spans, keyed, base, o, pairs = [], [], 0, 0, 0
+        for s, (ln, start) in enumerate(zip(seg_lens, seg_starts)):
+            end = start + ln
+            need = max(0, start - window + 1) if window else 0
+            lo = need // 64 * 64
+            for p in range(lo, end, 64):
+                spans += [s, p, need, end]
+            for t in range(0, ln, 128):
+                nt = min(128, ln - t)
+                first = max(0, start + t - window + 1) if window else 0
+                keyed.append((first - (start + t + nt), len(keyed), o + t, nt, base - lo))
+            full = max(0, end - max(start, window - 1)) if window else 0  # (queries whose window is full)
+            rest = ln - full
+            pairs += full * window + rest * (start + 1) + rest * (rest - 1) // 2
+            base += -(-(end - lo) // 64) * 64
+            o += ln
+        keyed.sort()
+        return spans, [v for _, _, n0, nt, off in keyed for v in (n0, nt, off, 0)], base, pairs
+
+    def latent_attention_expanded(self, q, nope_dim: int, w_uk, w_uv, latent_pages, rope_pages, block_table, positions,
+                                  token_segment, window, scale: float, meta=None, sink=None):
+        """The heads' outputs ``[N, H * value_dim]`` with every head's keys and values formed from the cached latents
+        (``w_uk [H * nope, kv_rank]``, ``w_uv [H * value_dim, kv_rank]``), or ``None``: this step is better served in the
+        latent's space (too few queries a key, sizes the kernel is not compiled for, float32)."""
+        n, H, dq = q.shape
+        r = latent_pages.shape[2]
+        dr, dv = dq - nope_dim, w_uv.shape[0] // H
+        if (q.dtype != torch.bfloat16 or latent_pages.dtype != torch.bfloat16 or w_uk.dtype != torch.bfloat16
+                or (meta is not None and meta.decode_bucket is not None)
+                or not self._query("jle_latent_expanded_supported", r, nope_dim, dr, dv, q.stride(0))):
+            return None
+        w = 0 if window is None else int(window)
+        key = f"latent_expanded_{w}"
+        plan = meta.meta.get(key) if meta is not None else None
+        if plan is None:
+            spans, blocks, rows, pairs = self.expanded_plan(*self._segments(meta, token_segment, positions), w)
+            if (rows > self.LATENT_EXPAND_ROWS * n and pairs < self.LATENT_EXPAND_PAIRS * rows
+                    or rows * H * (nope_dim + dv) * 2 > self.LATENT_EXPAND_BYTES):
+                plan = (None, 0, 0)
+            else:
+                plan = (torch.tensor(spans + blocks, dtype=torch.int32).to(q.device), len(spans), rows)
+            if meta is not None:
+                meta.meta[key] = plan
+        table, ns, rows = plan
+        if table is None:
+            return None
+        np_, ps = latent_pages.shape[0], latent_pages.shape[1]
+        if q.stride(2) != 1 or q.stride(1) != dq:
+            raise KernelError("the heads' queries must lie side by side at the start of contiguous rows")
+        self._chk(latent_pages, torch.bfloat16, (np_, ps, r), "latent pages")
+        self._chk(rope_pages, torch.bfloat16, (np_, ps, dr), "rotated key pages")
+        self._chk(block_table, torch.int32, None, "block table")
+        self._chk(positions, torch.int32, (n,), "positions")
+        self._chk(w_uk, torch.bfloat16, (H * nope_dim, r), "key matrix")
+        self._chk(w_uv, torch.bfloat16, (H * dv, r), "value matrix")
+        if sink is not None:
+            self._chk(sink, torch.float32, (H,), "sinks")
+        c = torch.empty(rows, r, dtype=q.dtype, device=q.device)
+        kr = torch.empty(rows, dr, dtype=q.dtype, device=q.device)
+        self._call("jle_latent_expanded_gather", _p(latent_pages), _p(rope_pages), _p(block_table), block_table.shape[1],
+                   _p(table), ns // 4, _p(c), _p(kr), r, dr, ps)
+        kn = torch.matmul(c, w_uk.t())  # [rows, H * nope]
+        vt = torch.matmul(w_uv, c.t())  # [H * value_dim, rows]
+        out = torch.empty(n, H * dv, dtype=q.dtype, device=q.device)
+        self._call("jle_latent_expanded_attention", _p(q), q.stride(0), _p(kn), _p(kr), _p(vt), rows, _p(out),
+                   _p(positions), _p(table[ns:]), (table.numel() - ns) // 4, w, float(scale), H, _p(sink))
         return out
 
     def scaled_add_norm(self, x, delta, weight, eps: float, out_dtype, want32: bool = False, norm: bool = True):

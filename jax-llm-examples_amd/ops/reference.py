@@ -629,6 +629,10 @@ class ReferenceOps:
             out[i] = (pr @ c).to(out.dtype)
         return out
 
+    def latent_attention_expanded(self, *args, **kw):
+        """``None``: the plain ops stay in the latent's space (:meth:`latent_attention`)."""
+        return None
+
     # ------------------------------------------------------------------ attention
     def qk_prepare_kv_write(self, qkv, num_heads: int, num_kv_heads: int, head_dim: int, positions, prep,
                             kv_cache: Optional[torch.Tensor], slot_mapping: Optional[torch.Tensor]):

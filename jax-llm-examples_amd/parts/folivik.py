@@ -25,7 +25,8 @@ from ..weights.bindings import TensorBinding
 class FolivikArchitecture:
     names = ("Folivik", "folivik")
     # what of csrc/ a model of this design calls (a first run on a machine without a built library compiles these)
-    kernel_sources = ("elementwise.hip", "mamba2.hip", "attention_latent.hip", "attention_heads.hip", "attention_conv.hip",
+    kernel_sources = ("elementwise.hip", "mamba2.hip", "attention_latent.hip",
+                      "attention_expanded.hip", "attention_heads.hip", "attention_conv.hip",
                       "attention_generic.hip", "attention_mfma.hip", "attention_f32.hip", "attention_prep.hip",
                       "moe_route.hip", "moe_choose.hip", "gemm_skinny.hip", "gemm_stream.hip", "gemm_grouped.hip",
                       "gemm_generic.hip", "gemm_f32.hip", "parallel.hip", "sampling.hip")

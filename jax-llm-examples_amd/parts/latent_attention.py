@@ -6,11 +6,12 @@ value ``W_uv c``; its query ``[q_n, q_r]`` (``nope_dim`` unrotated and ``rope_di
 
     score = (q_n . W_uk c + q_r . k_r) * softmax_scale.
 
-Neither keys nor values are ever formed.  ``q_n . W_uk c = (W_uk^T q_n) . c``, so the query is taken into the
-latent's space (one batched product per step), the attention kernel runs over the cached ``[c, k_r]`` rows
+With few queries a key neither keys nor values are formed.  ``q_n . W_uk c = (W_uk^T q_n) . c``, so the query is taken
+into the latent's space (one batched product per step), the attention kernel runs over the cached ``[c, k_r]`` rows
 with all heads sharing them and sums the latents with the softmax weights, and ``W_uv`` is applied to that sum
-(a second batched product).  Prefill and decode are the same computation, so a token's result does not depend
-on how its request was cut into steps.
+(a second batched product).  A step with many queries a key forms every head's keys and values of the visible tokens
+once and attends to those, a third of the operations per query and key; the two differ by the rounding of what lies
+between (``W_uk^T q`` and the summed latents there, keys and values here).
 
 Options as data: ``window`` (a query sees itself and the ``window - 1`` tokens before it; ``None``: all),
 ``retention`` (what the cache keeps: at least the window of every run that reads it), ``own_latent`` (False: the
@@ -152,14 +153,19 @@ class LatentAttention(Mixer):
             q = ops.linear(cq, self.params["w_uq"])
             ops.rotate_heads_(q, H, dn, dr, ctx.positions, self.rotation)
             q = q.view(n, H, dn + dr)
-        # queries into the latent's space: [H, N, dn] x [H, dn, r]
-        q_lat = ops.batched_linear(q[:, :, :dn].transpose(0, 1), self.params["w_uk"].view(H, dn, r))
-        o_lat = ops.latent_attention(q_lat, q, dn, cache.pages["latent"], cache.pages["rope_key"], cache.block_table,
-                                     ctx.positions, ctx.token_segment, self.window, self.softmax_scale,
-                                     cache.attn_meta, latent_t_pages=cache.pages.get("latent_t"),
-                                     sink=self.params.get("sink"))  # [N, H, r]
-        # the sums out of it: [H, N, r] x [H, r, dv], laid out [N, H * dv]
-        o = ops.batched_linear(o_lat.transpose(0, 1), self.w_out, tokens_first=True)
+        # a step of many tokens: every head's keys and values formed once, and attended to as such
+        o = ops.latent_attention_expanded(q, dn, self.params["w_uk"], self.params["w_uv"], cache.pages["latent"],
+                                          cache.pages["rope_key"], cache.block_table, ctx.positions, ctx.token_segment,
+                                          self.window, self.softmax_scale, cache.attn_meta, sink=self.params.get("sink"))
+        if o is None:
+            # queries into the latent's space: [H, N, dn] x [H, dn, r]
+            q_lat = ops.batched_linear(q[:, :, :dn].transpose(0, 1), self.params["w_uk"].view(H, dn, r))
+            o_lat = ops.latent_attention(q_lat, q, dn, cache.pages["latent"], cache.pages["rope_key"], cache.block_table,
+                                         ctx.positions, ctx.token_segment, self.window, self.softmax_scale,
+                                         cache.attn_meta, latent_t_pages=cache.pages.get("latent_t"),
+                                         sink=self.params.get("sink"))  # [N, H, r]
+            # the sums out of it: [H, N, r] x [H, r, dv], laid out [N, H * dv]
+            o = ops.batched_linear(o_lat.transpose(0, 1), self.w_out, tokens_first=True)
         o = o.view(n, H * dv)
         if self.output_gate:
             o = ops.sigmoid_mul(o, rows[:, self.gate_offset: self.gate_offset + H * dv])

@@ -1,0 +1,91 @@
+"""Attention over a cached latent with every head's keys and values formed from it (``csrc/attention_expanded.hip``)
+against its definition in 64 bits, and the layout of its work."""
+import pytest
+import torch
+
+from jax_llm_examples_amd.engine.batch import GroupContext
+from jax_llm_examples_amd.ops.hip import HipOps
+
+DN, DR, DV = 128, 64, 128
+
+CASES = [  # (segments: (tokens, position of the first), window, sink, heads, latent, page size)
+    ([(130, 0)], None, False, 3, 512, 16),                     # two blocks, the second of two tokens
+    ([(64, 0), (129, 0), (127, 5)], None, True, 2, 64, 16),    # a whole step of keys, one token over a block, one short
+    ([(33, 700), (200, 64), (96, 63)], None, False, 2, 96, 32),  # tokens cached before, at and beside a step's edge
+    ([(257, 1000)], 100, False, 2, 64, 16),                    # a window that begins within a step
+    ([(300, 0), (70, 333)], 64, True, 1, 40, 8),               # a window of one step; a latent of odd width
+    ([(128, 128)], 1, False, 2, 64, 16),                       # every token sees itself alone
+]
+
+
+@pytest.mark.parametrize("window", [0, 1, 63, 64, 500])
+def test_the_plan_covers_every_token_and_every_key_it_sees(window):
+    lens, starts = [1, 64, 129, 700, 5], [0, 63, 128, 1000, 777]
+    spans, blocks, rows, pairs = HipOps.expanded_plan(lens, starts, window)
+    assert len(spans) // 4 * 64 == rows
+    assert pairs == sum(min(p + 1, window or p + 1) for n, s in zip(lens, starts) for p in range(s, s + n))
+    where = [(i, s + t) for i, (n, s) in enumerate(zip(lens, starts)) for t in range(n)]
+    seen = []
+    for n0, n, off, _ in (blocks[i: i + 4] for i in range(0, len(blocks), 4)):
+        assert 0 < n <= 128
+        seg, pos = where[n0]
+        assert where[n0: n0 + n] == [(seg, pos + t) for t in range(n)]
+        seen += range(n0, n0 + n)
+        first = max(0, pos - window + 1) if window else 0
+        for kb in range(first // 64 * 64, pos + n, 64):
+            span = spans[4 * ((kb + off) // 64):][:4]
+            assert (kb + off) % 64 == 0 and span[:2] == [seg, kb] and span[2] <= first and span[3] >= pos + n
+    assert sorted(seen) == list(range(len(where)))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("segs, window, sink, H, R, ps", CASES)
+def test_against_the_definition(segs, window, sink, H, R, ps):
+    dev = "cuda:0"
+    ops = HipOps(dev)
+    ops.LATENT_EXPAND_PAIRS = 0  # (whatever the sizes)
+    g = torch.Generator().manual_seed(len(segs) + R)
+    bf = lambda *s, std=1.0: (torch.randn(*s, generator=g) * std).to(torch.bfloat16)
+    lens, starts = [n for n, _ in segs], [s for _, s in segs]
+    N, width = sum(lens), max(-(-(n + s) // ps) for n, s in segs)
+    need = [max(0, s - window + 1) if window else 0 for s in starts]
+    table = torch.full((len(segs), width), -1, dtype=torch.int32)
+    free = torch.randperm(len(segs) * width, generator=g).tolist()
+    for i, (n, s) in enumerate(segs):
+        for j in range(need[i] // ps, -(-(n + s) // ps)):  # (pages that no query sees were given back)
+            table[i, j] = free.pop()
+    latent, rope = bf(len(segs) * width, ps, R), bf(len(segs) * width, ps, DR)
+    for i, (n, s) in enumerate(segs):  # what lies behind a segment's end was never written
+        if (n + s) % ps:
+            latent[table[i, (n + s) // ps], (n + s) % ps:] = float("nan")
+            rope[table[i, (n + s) // ps], (n + s) % ps:] = float("nan")
+    q = bf(N, H * (DN + DR) + 8)
+    uk, uv = bf(H * DN, R, std=R ** -0.5), bf(H * DV, R, std=R ** -0.5)
+    sk = torch.randn(H, generator=g) if sink else None
+    pos = torch.tensor([s + t for n, s in segs for t in range(n)], dtype=torch.int32)
+    seg = torch.tensor([i for i, (n, _) in enumerate(segs) for _ in range(n)], dtype=torch.int32)
+    meta = GroupContext(block_table=None, slot_mapping=None, width=width, retention=("all",), seg_lens=lens, seg_starts=starts)
+    d = lambda t: None if t is None else t.to(dev)
+    scale = (DN + DR) ** -0.5
+    got = ops.latent_attention_expanded(d(q)[:, : H * (DN + DR)].view(N, H, DN + DR), DN, d(uk), d(uv), d(latent), d(rope),
+                                        d(table), d(pos), d(seg), window, scale, meta, sink=d(sk)).cpu().double()
+    o = 0
+    for i, (n, s) in enumerate(segs):
+        kpos = torch.arange(need[i], s + n)
+        c = latent[table[i][kpos // ps].long(), kpos % ps].double()
+        kr = rope[table[i][kpos // ps].long(), kpos % ps].double()
+        back = torch.arange(s, s + n)[:, None] - kpos[None]
+        seen = (back >= 0) & (back < (window or s + n + 1))
+        for h in range(H):
+            k = torch.cat([c @ uk[h * DN: (h + 1) * DN].double().T, kr], 1)
+            qh = q[o: o + n, h * (DN + DR): (h + 1) * (DN + DR)].double()
+            sc = (qh @ k.T * scale).masked_fill(~seen, float("-inf"))
+            if sink:  # one more key, without a value
+                sc = torch.cat([sc, sk[h].double().expand(n, 1)], 1)
+            v = c @ uv[h * DV: (h + 1) * DV].double().T
+            want = torch.softmax(sc, -1)[:, : len(kpos)] @ v
+            err = (got[o: o + n, h * DV: (h + 1) * DV] - want).norm() / want.norm()
+            # keys, values, probabilities and the result rounded to bfloat16 (2^-9 each at most, 2^-9 / sqrt(3) rms);
+            # a score of size 1 moves by the keys' rounding averaged over 128 terms, far below that
+            assert err < 4 * 2.0 ** -9, (i, h, float(err))
+        o += n
