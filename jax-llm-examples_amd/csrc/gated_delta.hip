@@ -1,12 +1,14 @@
 // The gated delta rule: a matrix memory S (dk x dv, float32) per head and request, written and read token by token,
 //     S <- g S;   u = beta (v - S^T k);   S <- S + k u^T;   o = S^T q
 // with q, k unit vectors per kv head (x / sqrt(sum(x^2) + floor), q times dk^(-1/2)), beta = sigmoid(b),
-// g = exp(-exp(A) softplus(a + dt)).  Three kernels:
+// g = exp(-exp(A) softplus(a + dt)).  Kernels:
 //   gdr_prepare_kernel   the unit vectors (float32), beta and the decay of every token of the step
 //   gdr_scan_kernel      the recurrence: a column of S depends on nothing but itself, k, q, v of its own place, beta
 //                        and g, so a wavefront takes 64 / KS columns of one head, KS neighbouring lanes share a
 //                        column (each holds R consecutive rows of it in registers), and the two dot products are
 //                        finished with log2(KS) lane swaps; the next tokens' rows are asked for before these are used
+//   gdr_chunk_kernel, gdr_carry_kernel   the same recurrence 64 tokens at a time on the float32 matrix instructions, for
+//                        segments of many tokens (below)
 //   gdr_out_kernel       o / sqrt(mean(o^2) + eps) * w * silu(gate), rounded to the run dtype
 // The memory lies [slot][half][H][dv][dk] (a column's rows together); a step reads the half `phase` and writes the other.  Every sum is formed
 // in an order that depends on the sizes alone, token after token: cutting a sequence into steps changes no bit.
@@ -92,7 +94,8 @@ __global__ __launch_bounds__(64) void gdr_scan_kernel(const T* __restrict__ rows
                                                       const int* __restrict__ cu_seqlens,
                                                       const int* __restrict__ state_slots,
                                                       const int* __restrict__ state_phase, float* __restrict__ o_raw,
-                                                      int H, int G, int dk, int dv) {
+                                                      int H, int G, int dk, int dv,
+                                                      int chunked_from /* longer segments go by chunks */) {
   using Shape = ScanShape<KS, R>;
   constexpr int TB = Shape::kTB, DKP = Shape::kDkp, NV = Shape::kVecs, cols = 64 / KS;
   __shared__ f32x4 sk[TB * DKP / 4], sq[TB * DKP / 4];
@@ -103,7 +106,7 @@ __global__ __launch_bounds__(64) void gdr_scan_kernel(const T* __restrict__ rows
   const int g = h / (H / G);
   const int C = 2 * G * dk + H * dv;
   const int t0 = cu_seqlens[seg], t1 = cu_seqlens[seg + 1];
-  if (t0 >= t1) return;
+  if (t0 >= t1 || t1 - t0 >= chunked_from) return;
   const size_t slot = (size_t)state_slots[seg];
   const int phase = state_phase[seg];
   const float* s_old = state + ((slot * 2 + phase) * H + h) * (size_t)dk * dv;
@@ -235,6 +238,374 @@ __global__ __launch_bounds__(64) void gdr_scan_kernel(const T* __restrict__ rows
   }
 }
 
+// ------------------------------------------------------------------ many tokens: 64 at a time
+// Within a chunk that starts with the memory S, let d(t, j) be the product of the decays behind token j up to token t, and
+// c(t) of those from the chunk's start up to t.  The writes follow from the memory before the chunk and from each other,
+//     u_t = beta_t (v_t - c(t) S^T k_t) - sum_{j < t} L_tj u_j,      L_tj = beta_t d(t, j) (k_t . k_j),
+// a unit lower triangular system.  With T = (I + L)^-1, per chunk and independent of S (gdr_chunk_kernel):
+//     U0 = T (beta V),   W = T (beta c K),   P_tj = d(t, j) (q_t . k_j) for j <= t;
+// then from chunk to chunk (gdr_carry_kernel):
+//     U = U0 - W S,   O = c Q S + P U,   S <- c(end) S + K^T (d(end, .) U).
+// Everything is float32 on the float32 matrix instructions, the decays' products formed by multiplying, as the scan does
+// (differences of summed logarithms would lose what a strong decay leaves of a later weak one).  One prompt of 2,048
+// tokens, 16 heads of 128 x 128 on 8 kv heads: 31 + 93 us instead of the scan's 726; a step's 25 prompts of 80 tokens
+// 51 + 88 instead of 165.
+// v_mfma_f32_16x16x4: lane (m = lane % 16, g = lane / 16) holds A[m][k] and B[k][m] of one k, and of the result the rows
+// 4 g .. 4 g + 3 of column m.  Taking k = 16 r + 4 g + i for the i-th product of tile r, A and B are 16-byte pieces of
+// rows, and a result's registers are the next product's B operand as they are.
+constexpr int kChunk = 64;
+
+__device__ __forceinline__ f32x4 mfma4(const f32x4& a, const f32x4& b, f32x4 c) {  // 16 of k: four products
+#pragma unroll
+  for (int i = 0; i < 4; ++i) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], b[i], c, 0, 0, 0);
+  return c;
+}
+
+// What goes from one kernel to the other lies as the operands that the second reads: a tile of 16 x 16 numbers is a
+// kilobyte, a lane's 16 bytes in the lanes' order.  (As plain matrices, 16 rows a load instruction, every lane's piece was
+// a request of its own to the first-level cache: 142 us instead of 93 for the second kernel, 2,048 tokens, 16 heads.)
+__device__ __forceinline__ int operand_at(int row, int col) {  // of an A operand's tile (rows its lanes, columns its k)
+  return (((col & 15) >> 2) * 16 + (row & 15)) * 4 + (col & 3);
+}
+
+// One block per (chunk, head).  ws: per (chunk, head) W (negated) [4][DK / 16] tiles, U0 [dv / 16][4] tiles as results, P
+// [4][4] tiles, and c(t), d(end, t) [2][64]; per (chunk, kv head) K^T [DK / 16][4] and Q [4][DK / 16] tiles.
+template <typename T, int DK>
+__global__ __launch_bounds__(256, 2) void gdr_chunk_kernel(const T* __restrict__ rows, const float* __restrict__ qn,
+                                                           const float* __restrict__ kn, const float* __restrict__ beta,
+                                                           const float* __restrict__ decay, const int* __restrict__ chunks,
+                                                           float* __restrict__ ws_w, float* __restrict__ ws_u,
+                                                           float* __restrict__ ws_p, float* __restrict__ ws_kt,
+                                                           float* __restrict__ ws_q, float* __restrict__ ws_s, int H, int G,
+                                                           int dv) {
+  constexpr int NT = DK / 16, KP = DK + 4, LP = kChunk + 4;
+  extern __shared__ __attribute__((aligned(16))) float smem[];
+  float* sk = smem;               // [64][KP]: the chunk's keys
+  float* sd = sk + kChunk * KP;   // [64][LP]: d(t, j), then T
+  float* sl = sd + kChunk * LP;   // [64][LP]: L
+  float* sb = sl + kChunk * LP;   // beta, decay, c(t)
+  float *sg = sb + kChunk, *sc = sg + kChunk;
+  const int tid = threadIdx.x, lane = tid & 63, c16 = lane & 15, g = lane >> 4;
+  const int w = wave_index();
+  const int c = blockIdx.x, h = blockIdx.y, kv = h / (H / G);
+  const int tok0 = chunks[3 * c + 1], nt = chunks[3 * c + 2];
+  const size_t at = (size_t)c * H + h;
+  // (places behind the segment's end: keys of zeros, no write, no decay)
+  for (int idx = tid; idx < kChunk * DK / 4; idx += 256) {
+    const int t = idx / (DK / 4), e = idx - t * (DK / 4);
+    f32x4 v = {0.f, 0.f, 0.f, 0.f};
+    if (t < nt) v = reinterpret_cast<const f32x4*>(kn + ((size_t)(tok0 + t) * G + kv) * DK)[e];
+    *reinterpret_cast<f32x4*>(sk + t * KP + 4 * e) = v;
+  }
+  if (tid < kChunk) {
+    sb[tid] = tid < nt ? beta[(size_t)(tok0 + tid) * H + h] : 0.f;
+    sg[tid] = tid < nt ? decay[(size_t)(tok0 + tid) * H + h] : 1.f;
+  }
+  __syncthreads();
+  if (w == 3) {  // a column of d a lane
+    float d = 0.f, p = 1.f, mine = 1.f;
+    for (int t = 0; t < kChunk; ++t) {
+      const float gt = sg[t];
+      d = t == lane ? 1.f : d * gt;
+      p *= gt;
+      mine = t == lane ? p : mine;
+      sd[t * LP + lane] = d;
+    }
+    sc[lane] = mine;
+  }
+  // the lower tiles (i, j) of K K^T and Q K^T, ten pairs for four wavefronts (the third and fourth: two each)
+  f32x4 kk[3], qk[3];
+#pragma unroll
+  for (int s = 0; s < 3; ++s) {
+    const int pair = w + 4 * s;
+    if (pair >= 10) break;
+    const int i = pair >= 6 ? 3 : pair >= 3 ? 2 : pair >= 1 ? 1 : 0, j = pair - i * (i + 1) / 2;
+    const int t = min(16 * i + c16, nt - 1);
+    const float* qrow = qn + ((size_t)(tok0 + t) * G + kv) * DK + 4 * g;
+    const float* krow = sk + (16 * i + c16) * KP + 4 * g;
+    const float* brow = sk + (16 * j + c16) * KP + 4 * g;
+    f32x4 qa[NT];
+#pragma unroll
+    for (int r = 0; r < NT; ++r) qa[r] = *reinterpret_cast<const f32x4*>(qrow + 16 * r);
+    kk[s] = qk[s] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int r = 0; r < NT; ++r) {
+      const f32x4 b = *reinterpret_cast<const f32x4*>(brow + 16 * r), a = *reinterpret_cast<const f32x4*>(krow + 16 * r);
+#pragma unroll
+      for (int x = 0; x < 4; ++x) {
+        kk[s] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[x], b[x], kk[s], 0, 0, 0);
+        qk[s] = __builtin_amdgcn_mfma_f32_16x16x4f32(qa[r][x], b[x], qk[s], 0, 0, 0);
+      }
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int s = 0; s < 3; ++s) {
+    const int pair = w + 4 * s;
+    if (pair >= 10) break;
+    const int i = pair >= 6 ? 3 : pair >= 3 ? 2 : pair >= 1 ? 1 : 0, j = pair - i * (i + 1) / 2;
+#pragma unroll
+    for (int x = 0; x < 4; ++x) {
+      const int t = 16 * i + 4 * g + x, u = 16 * j + c16;
+      const float d = sd[t * LP + u];
+      sl[t * LP + u] = u < t ? sb[t] * (d * kk[s][x]) : 0.f;
+      ws_p[(at * 16 + 4 * i + j) * 256 + operand_at(t, u)] = u <= t ? d * qk[s][x] : 0.f;
+    }
+  }
+  for (int idx = tid; idx < 6 * 256; idx += 256) {  // (the tiles above the diagonal)
+    const int pair = idx >> 8, j = pair >= 3 ? 3 : pair >= 1 ? 2 : 1, i = pair - j * (j - 1) / 2;
+    ws_p[(at * 16 + 4 * i + j) * 256 + tid] = 0.f;
+  }
+  if (tid < kChunk) {
+    ws_s[at * 2 * kChunk + tid] = sc[tid];
+    ws_s[at * 2 * kChunk + kChunk + tid] = sd[(kChunk - 1) * LP + tid];
+  }
+  if (h % (H / G) == 0) {  // (the head's keys are its group's)
+    f32x4* kt = reinterpret_cast<f32x4*>(ws_kt + ((size_t)c * G + kv) * DK * kChunk);
+    f32x4* qt = reinterpret_cast<f32x4*>(ws_q + ((size_t)c * G + kv) * DK * kChunk);
+    for (int idx = tid; idx < DK * kChunk / 4; idx += 256) {
+      const int tile = idx >> 6;  // (lane: idx % 64, as tid)
+      const float* src = sk + (16 * (tile & 3) + 4 * g) * KP + 16 * (tile >> 2) + c16;
+      kt[idx] = f32x4{src[0], src[KP], src[2 * KP], src[3 * KP]};
+      const int t = min(16 * (tile / NT) + c16, nt - 1);
+      qt[idx] = *reinterpret_cast<const f32x4*>(qn + ((size_t)(tok0 + t) * G + kv) * DK + 16 * (tile % NT) + 4 * g);
+    }
+  }
+  __syncthreads();
+  // T: the inverses of the four diagonal tiles, a column a lane, by forward substitution
+  if (lane < 16) {
+    const float* lt = sl + 16 * w * LP + 16 * w;
+    float x[16];
+#pragma unroll
+    for (int t = 0; t < 16; ++t) {
+      float v = t == lane ? 1.f : 0.f;
+#pragma unroll
+      for (int j = 0; j < t; ++j) v = __builtin_fmaf(-lt[t * LP + j], x[j], v);
+      x[t] = v;
+    }
+#pragma unroll
+    for (int t = 0; t < 16; ++t) sd[(16 * w + t) * LP + 16 * w + lane] = x[t];
+  }
+  __syncthreads();
+  // the tiles below them, a column of tiles a wavefront: T_ij = -T_ii sum_{j <= k < i} L_ik T_kj
+  if (w < 3) {
+    f32x4 col[4];
+#pragma unroll
+    for (int x = 0; x < 4; ++x) col[0][x] = sd[(16 * w + 4 * g + x) * LP + 16 * w + c16];
+#pragma unroll
+    for (int n = 1; n < 4; ++n) {
+      const int i = w + n;
+      if (i > 3) break;
+      f32x4 sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int k = 0; k < n; ++k)
+        sum = mfma4(*reinterpret_cast<const f32x4*>(sl + (16 * i + c16) * LP + 16 * (w + k) + 4 * g), col[k], sum);
+      const f32x4 t = mfma4(*reinterpret_cast<const f32x4*>(sd + (16 * i + c16) * LP + 16 * i + 4 * g), sum, f32x4{0.f, 0.f, 0.f, 0.f});
+      col[n] = -t;
+#pragma unroll
+      for (int x = 0; x < 4; ++x) sd[(16 * i + 4 * g + x) * LP + 16 * w + c16] = col[n][x];
+    }
+  }
+  __syncthreads();
+  // W and U0, a tile of 16 columns a wavefront and turn
+  const int C = 2 * G * DK + H * dv;
+  for (int ct = w; ct < NT + dv / 16; ct += 4) {
+    f32x4 b[4];
+    if (ct < NT) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int x = 0; x < 4; ++x) {
+          const int t = 16 * r + 4 * g + x;
+          b[r][x] = -(sb[t] * sc[t]) * sk[t * KP + 16 * ct + c16];
+        }
+    } else {
+      const T* v = rows + 2 * G * DK + (size_t)h * dv + 16 * (ct - NT) + c16;
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int x = 0; x < 4; ++x) {
+          const int t = 16 * r + 4 * g + x;
+          b[r][x] = sb[t] * Num<T>::load(v + (size_t)(tok0 + min(t, nt - 1)) * C);
+        }
+    }
+    f32x4 acc[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int i = r; i < 4; ++i)
+        acc[i] = mfma4(*reinterpret_cast<const f32x4*>(sd + (16 * i + c16) * LP + 16 * r + 4 * g), b[r], acc[i]);
+    if (ct < NT) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int x = 0; x < 4; ++x) ws_w[((at * 4 + i) * NT + ct) * 256 + operand_at(4 * g + x, c16)] = acc[i][x];
+    } else {
+      f32x4* dst = reinterpret_cast<f32x4*>(ws_u + at * kChunk * dv) + (size_t)(ct - NT) * 256 + lane;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) dst[64 * i] = acc[i];
+    }
+  }
+}
+
+// One block per (segment, head, 16 columns of the memory): four wavefronts, each with 16 of a chunk's tokens and a quarter
+// of the memory's rows; the writes and the memory go round through shared memory (two barriers a chunk), every operand
+// comes straight from the scratch arrays into registers and is asked for as soon as the chunk before has used its
+// registers.  A chunk is 112 matrix instructions a wavefront (DK = 128), 1.5 us of the 2.9 it takes at 2,048 tokens and 16
+// heads (128 blocks); without its loads it takes 2.3, so what the rest is made of is barriers and trips through shared
+// memory first, the 110 KB of operands second.
+template <int DK>
+__global__ __launch_bounds__(256, 2) void gdr_carry_kernel(const float* __restrict__ ws_q, const int* __restrict__ segs,
+                                                           const int* __restrict__ cu_seqlens,
+                                                           const int* __restrict__ state_slots,
+                                                           const int* __restrict__ state_phase, float* __restrict__ state,
+                                                           const float* __restrict__ ws_w, const float* __restrict__ ws_u,
+                                                           const float* __restrict__ ws_p, const float* __restrict__ ws_kt,
+                                                           const float* __restrict__ ws_s, float* __restrict__ o_raw, int N,
+                                                           int H, int G, int dv) {
+  constexpr int NT = DK / 16, OWN = NT / 4;
+  __shared__ f32x4 s_mem[NT][64], s_u[4][64], s_du[4][64];
+  const int lane = threadIdx.x & 63, c16 = lane & 15, g = lane >> 4;
+  const int w = wave_index();
+  const int h = blockIdx.x % H, kv = h / (H / G);
+  const int cb = blockIdx.x / H % (dv / 16), col = 16 * cb + c16;
+  const int* sgm = segs + 3 * (blockIdx.x / H / (dv / 16));
+  const int seg = sgm[0], c0 = sgm[1], c1 = c0 + sgm[2];
+  const size_t slot = (size_t)state_slots[seg];
+  const int phase = state_phase[seg];
+  const size_t own = (((slot * 2 + phase) * H + h) * (size_t)dv + col) * DK;
+  const size_t own_new = (((slot * 2 + (1 - phase)) * H + h) * (size_t)dv + col) * DK;
+  f32x4 S[NT];
+#pragma unroll
+  for (int r = 0; r < NT; ++r) S[r] = *reinterpret_cast<const f32x4*>(state + own + 16 * r + 4 * g);
+  f32x4 W[NT], Q[NT], P[4], KT[OWN][4], U0, cs, ds;
+  float cend;
+  const int tok0 = cu_seqlens[seg], len = cu_seqlens[seg + 1] - tok0;
+  int zero;  // (not known to be the same in all lanes: a load by it goes the vectors' way, in order with the others)
+  asm("v_mov_b32 %0, 0" : "=v"(zero));
+  auto ask_front = [&](int c) __attribute__((always_inline)) {
+    const f32x4* wr = reinterpret_cast<const f32x4*>(ws_w + (((size_t)c * H + h) * 4 + w) * DK * 16) + lane;
+    const f32x4* qr = reinterpret_cast<const f32x4*>(ws_q + (((size_t)c * G + kv) * 4 + w) * DK * 16) + lane;
+#pragma unroll
+    for (int r = 0; r < NT; ++r) {
+      W[r] = wr[64 * r];
+      Q[r] = qr[64 * r];
+    }
+    U0 = reinterpret_cast<const f32x4*>(ws_u + ((size_t)c * H + h) * kChunk * dv)[(4 * cb + w) * 64 + lane];
+  };
+  auto ask_back = [&](int c) __attribute__((always_inline)) {
+    const float* sr = ws_s + ((size_t)c * H + h) * 2 * kChunk;
+    cs = *reinterpret_cast<const f32x4*>(sr + 16 * w + 4 * g);
+    ds = *reinterpret_cast<const f32x4*>(sr + kChunk + 16 * w + 4 * g);
+    cend = sr[kChunk - 1 + zero];
+    const f32x4* pr = reinterpret_cast<const f32x4*>(ws_p + (((size_t)c * H + h) * 4 + w) * 1024) + lane;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) P[r] = pr[64 * r];
+    const f32x4* kr = reinterpret_cast<const f32x4*>(ws_kt + ((size_t)c * G + kv) * DK * kChunk) + (size_t)OWN * w * 256 + lane;
+#pragma unroll
+    for (int q = 0; q < OWN; ++q)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) KT[q][r] = kr[64 * (4 * q + r)];
+  };
+  const size_t behind = (size_t)N * H * dv;  // (64 places that nobody reads)
+  ask_front(c0);
+  __builtin_amdgcn_sched_barrier(0);
+  ask_back(c0);
+  __builtin_amdgcn_sched_barrier(0);
+  f32x4 mine[OWN];
+  for (int c = c0; c < c1; ++c) {
+    // (loads and stores without branches around them: the compiler then knows how many are on their way and waits for those
+    // it needs; with the last chunk's loads and the rows behind the segment's end under conditions it waited for all of
+    // them, the stores too, at every chunk's start)
+    const int next = min(c + 1, c1 - 1);
+    f32x4 u = U0, o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int r = 0; r < NT; ++r)
+#pragma unroll
+      for (int x = 0; x < 4; ++x) {
+        u = __builtin_amdgcn_mfma_f32_16x16x4f32(W[r][x], S[r][x], u, 0, 0, 0);
+        o = __builtin_amdgcn_mfma_f32_16x16x4f32(Q[r][x], S[r][x], o, 0, 0, 0);
+      }
+    s_u[w][lane] = u;
+    s_du[w][lane] = u * ds;
+    o *= cs;
+    ask_front(next);
+    __builtin_amdgcn_sched_barrier(0);
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < 4; ++r) o = mfma4(P[r], s_u[r][lane], o);
+#pragma unroll
+    for (int q = 0; q < OWN; ++q) {
+      // (the memory's tiles are all in registers; which of them are this wavefront's is known at run time only)
+      mine[q] = S[q];
+#pragma unroll
+      for (int n = 1; n < 4; ++n) mine[q] = w == n ? S[OWN * n + q] : mine[q];
+      mine[q] *= cend;
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const f32x4 du = s_du[r][lane];
+#pragma unroll
+      for (int x = 0; x < 4; ++x)
+#pragma unroll
+        for (int q = 0; q < OWN; ++q) mine[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(KT[q][r][x], du[x], mine[q], 0, 0, 0);
+    }
+#pragma unroll
+    for (int q = 0; q < OWN; ++q) s_mem[OWN * w + q][lane] = mine[q];
+    ask_back(next);
+    __builtin_amdgcn_sched_barrier(0);
+    const int t = kChunk * (c - c0) + 16 * w + 4 * g;
+#pragma unroll
+    for (int x = 0; x < 4; ++x) {
+      const size_t dst = ((size_t)(tok0 + t + x) * H + h) * dv + col;
+      o_raw[t + x < len ? dst : behind + lane] = o[x];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < NT; ++r) S[r] = s_mem[r][lane];
+  }
+#pragma unroll
+  for (int q = 0; q < OWN; ++q) *reinterpret_cast<f32x4*>(state + own_new + 16 * (OWN * w + q) + 4 * g) = mine[q];
+}
+
+// What the chunked form needs of a step: its chunks (segment, first token, tokens), the segments that go by chunks
+// (segment, first chunk, chunks) - those of `from` tokens and more -, whether others are left, and scratch.
+struct ByChunks {
+  const int *chunks, *segs;
+  int num_chunks, num_segs, from, others;
+  float* ws;
+};
+
+inline size_t chunk_floats(int H, int G, int dk, int dv) {  // scratch of one chunk
+  return (size_t)H * (kChunk * (dk + dv) + kChunk * kChunk + 2 * kChunk) + (size_t)2 * G * dk * kChunk;
+}
+
+template <typename T, int DK>
+int launch_chunks(const ByChunks& b, const T* rows, const float* qn, const float* kn, const float* beta, const float* decay,
+                  float* state, const int* cu_seqlens, const int* state_slots, const int* state_phase, float* o_raw, int N,
+                  int H, int G, int dv, hipStream_t s) {
+  const size_t n = (size_t)b.num_chunks * H;
+  float* ws_w = b.ws;
+  float* ws_u = ws_w + n * kChunk * DK;
+  float* ws_p = ws_u + n * kChunk * dv;
+  float* ws_s = ws_p + n * kChunk * kChunk;
+  float* ws_kt = ws_s + n * 2 * kChunk;
+  float* ws_q = ws_kt + (size_t)b.num_chunks * G * DK * kChunk;
+  constexpr int smem = (kChunk * (DK + 4) + 2 * kChunk * (kChunk + 4) + 3 * kChunk) * (int)sizeof(float);
+  static const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gdr_chunk_kernel<T, DK>),
+                                                  hipFuncAttributeMaxDynamicSharedMemorySize, smem);
+  if (e != hipSuccess) return (int)e;
+  hipLaunchKernelGGL((gdr_chunk_kernel<T, DK>), dim3(b.num_chunks, H), dim3(256), smem, s, rows, qn, kn, beta, decay,
+                     b.chunks, ws_w, ws_u, ws_p, ws_kt, ws_q, ws_s, H, G, dv);
+  JLE_LAUNCH_CHECK();
+  hipLaunchKernelGGL(gdr_carry_kernel<DK>, dim3((unsigned)(b.num_segs * H * (dv / 16))), dim3(256), 0, s, ws_q, b.segs,
+                     cu_seqlens, state_slots, state_phase, state, ws_w, ws_u, ws_p, ws_kt, ws_s, o_raw, N, H, G, dv);
+  JLE_LAUNCH_CHECK();
+  return 0;
+}
+
 template <typename T>
 __global__ __launch_bounds__(64) void gdr_out_kernel(const float* __restrict__ o_raw, const T* __restrict__ gate,
                                                      const float* __restrict__ w, T* __restrict__ out, float eps, int H,
@@ -257,7 +628,7 @@ template <typename T>
 int launch_gdr(const T* rows, const float* gates, const float* a_log, const float* dt_bias, const float* norm_w,
                const T* gate, float* state, const int* cu_seqlens, const int* state_slots, const int* state_phase,
                float* qn, float* kn, float* beta, float* decay, float* kq, float* o_raw, T* out, int N, int R_, int H,
-               int G, int dk, int dv, int dkp, float eps, float floor, hipStream_t s) {
+               int G, int dk, int dv, int dkp, float eps, float floor, const ByChunks& by_chunks, hipStream_t s) {
   // lanes a column: the fewest that leave a lane at most 16 rows of it (by the sizes alone)
   int KS = 1;
   while (KS < 64 && (dk + KS - 1) / KS > 16) KS <<= 1;
@@ -267,6 +638,13 @@ int launch_gdr(const T* rows, const float* gates, const float* a_log, const floa
   hipLaunchKernelGGL(gdr_prepare_kernel<T>, dim3(N, G + 1), dim3(64), 0, s, rows, gates, a_log, dt_bias, qn, kn, beta,
                      decay, kq, floor, H, G, dk, dv, dkp);
   JLE_LAUNCH_CHECK();
+  if (by_chunks.num_segs > 0) {
+    const int rc = dk == 128 ? launch_chunks<T, 128>(by_chunks, rows, qn, kn, beta, decay, state, cu_seqlens, state_slots,
+                                                     state_phase, o_raw, N, H, G, dv, s)
+                             : launch_chunks<T, 64>(by_chunks, rows, qn, kn, beta, decay, state, cu_seqlens, state_slots,
+                                                    state_phase, o_raw, N, H, G, dv, s);
+    if (rc != 0) return rc;
+  }
   // A step with few (segment, head) pairs leaves most of the machine idle, and what a token takes is the length of its
   // chain of dependent operations: then a column gets more lanes with fewer rows each (the row's width stays).
   int ks = KS, rr = RR;
@@ -278,7 +656,7 @@ int launch_gdr(const T* rows, const float* gates, const float* a_log, const floa
   const dim3 grid(R_, H, (dv + cols_ - 1) / cols_);
 #define JLE_SCAN(KS_, RR_)                                                                                          \
   hipLaunchKernelGGL((gdr_scan_kernel<T, KS_, RR_>), grid, dim3(64), 0, s, rows, qn, kn, beta, decay, kq, state, cu_seqlens, \
-                     state_slots, state_phase, o_raw, H, G, dk, dv)
+                     state_slots, state_phase, o_raw, H, G, dk, dv, by_chunks.from)
 #define JLE_SCAN_R(KS_)              \
   do {                               \
     if (rr == 4) JLE_SCAN(KS_, 4);   \
@@ -286,7 +664,7 @@ int launch_gdr(const T* rows, const float* gates, const float* a_log, const floa
     else if (rr == 16) JLE_SCAN(KS_, 16); \
     else JLE_SCAN(KS_, 32);          \
   } while (0)
-  switch (ks) {
+  if (by_chunks.others) switch (ks) {
     case 1: JLE_SCAN_R(1); break;
     case 2: JLE_SCAN_R(2); break;
     case 4: JLE_SCAN_R(4); break;
@@ -314,16 +692,35 @@ JLE_API int jle_gated_delta_padded(int dk) {
   return KS * (per <= 4 ? 4 : per <= 8 ? 8 : per <= 16 ? 16 : 32);
 }
 
+// The chunked form's scratch of one chunk of 64 tokens in KiB; -1: sizes that it is not compiled for.
+JLE_API int jle_gated_delta_chunk_kib(int H, int G, int dk, int dv) {
+  if ((dk != 64 && dk != 128) || dv <= 0 || dv % 16 || H <= 0 || G <= 0 || H % G || H > 65535) return -1;
+  return (int)((chunk_floats(H, G, dk, dv) * sizeof(float) + 1023) / 1024);
+}
+
 // rows [N, 2 G dk + H dv] (q | k | v behind convolution and activation) and gate [N, H dv] in the run dtype; gates
 // float32 [N, 2 H] (write strengths, then decays, before their biases and squashing); state float32 [slots, 2, H, dv,
-// dk]; qn, kn [N, G, dkp] (dkp = jle_gated_delta_padded(dk), 16-byte aligned), beta, decay [N, H], o_raw [N, H, dv]:
-// float32 scratch; out [N, H dv] in the run dtype.
+// dk]; qn, kn [N, G, dkp] (dkp = jle_gated_delta_padded(dk), 16-byte aligned), beta, decay [N, H], o_raw [N, H, dv]
+// and 64 floats behind it: float32 scratch; out [N, H dv] in the run dtype.
+// Segments of `from` tokens and more go 64 tokens at a time (num_segs of them, their num_chunks chunks; sizes as
+// jle_gated_delta_chunk_kib says; scratch of num_chunks times that many KiB, 16-byte aligned); others: whether shorter
+// ones are left.  num_segs = 0: none does.
 JLE_API int jle_gated_delta(const void* rows, int is_bf16, const float* gates, const float* a_log, const float* dt_bias,
                             const float* norm_w, const void* gate, float* state, const int* cu_seqlens,
                             const int* state_slots, const int* state_phase, float* qn, float* kn, float* beta,
                             float* decay, float* kq, float* o_raw, void* out, int N, int R, int H, int G, int dk, int dv,
-                            float eps, float floor, hipStream_t s) {
+                            float eps, float floor, const int* chunks, int num_chunks, const int* segs, int num_segs,
+                            int from, int others, float* ws, hipStream_t s) {
   if (N <= 0) return 0;
+  ByChunks b = {chunks, segs, num_chunks, num_segs, 0x7fffffff, 1, ws};
+  if (num_segs > 0) {
+    if ((dk != 64 && dk != 128) || dv % 16 || chunks == nullptr || segs == nullptr || ws == nullptr || from < 1 ||
+        num_chunks < num_segs || num_segs > R || ((uintptr_t)ws | (uintptr_t)state) % 16 ||
+        (long long)num_segs * H * (dv / 16) > (1ll << 31) - 1)
+      return JLE_BAD_ARG;
+    b.from = from;
+    b.others = others;
+  }
   const int dkp = jle_gated_delta_padded(dk);
   if (dkp <= 0 || ((uintptr_t)qn | (uintptr_t)kn) % 16) return JLE_BAD_ARG;
   if (R <= 0 || H <= 0 || G <= 0 || H % G || dk <= 0 || dk > 2048 || dv <= 0 || H > 65535 || G + 1 > 65535 ||
@@ -332,8 +729,8 @@ JLE_API int jle_gated_delta(const void* rows, int is_bf16, const float* gates, c
   if (is_bf16)
     return launch_gdr<bf16_t>((const bf16_t*)rows, gates, a_log, dt_bias, norm_w, (const bf16_t*)gate, state, cu_seqlens,
                               state_slots, state_phase, qn, kn, beta, decay, kq, o_raw, (bf16_t*)out, N, R, H, G, dk, dv, dkp,
-                              eps, floor, s);
+                              eps, floor, b, s);
   return launch_gdr<float>((const float*)rows, gates, a_log, dt_bias, norm_w, (const float*)gate, state, cu_seqlens,
                            state_slots, state_phase, qn, kn, beta, decay, kq, o_raw, (float*)out, N, R, H, G, dk, dv, dkp, eps,
-                           floor, s);
+                           floor, b, s);
 }

@@ -101,7 +101,7 @@ _SIGNATURES = {
                           _i, _vp],
     "jle_diff_combine": [_vp, _vp, _vp, _f, _f, _f, _i, _i, _i, _i, _i, _i, _vp],
     "jle_gated_delta": [_vp, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i,
-                        _i, _i, _i, _i, _f, _f, _vp],
+                        _i, _i, _i, _i, _f, _f, _vp, _i, _vp, _i, _i, _i, _vp, _vp],
     "jle_moe_choose": [_vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _f, _f, _i, _vp, _vp, _vp, _vp, _i, _i, _vp],
     "jle_moe_choose_groups": [_i, _i, _i, _i],
     "jle_mamba2": [_vp, _i, _vp, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _f, _i,
@@ -181,7 +181,7 @@ def _bind(path: str):
                        ("jle_latent_attention_mfma_supported", [_i, _i, _i, _i, _i]),
                        ("jle_latent_expanded_supported", [_i, _i, _i, _i, _i]), ("jle_attention_group_waves", []),
                        ("jle_mlstm_chunked_supported", [_i, _i]), ("jle_mlstm_chunk_tokens", []),
-                       ("jle_gated_delta_padded", [_i]), ("jle_gated_unit_chunk_tokens", []),
+                       ("jle_gated_delta_padded", [_i]), ("jle_gated_delta_chunk_kib", [_i, _i, _i, _i]), ("jle_gated_unit_chunk_tokens", []),
                        ("jle_retention_chunk_tokens", []), ("jle_retention_chunked_supported", [_i, _i]),
                        ("jle_retention_workspace_kib", [_i, _i, _i, _i])):
         fn = getattr(lib, name, None)
@@ -1144,6 +1144,41 @@ class HipOps:
                    self._is_bf16(o), n, num_heads, num_kv_heads, page_dim, value_dim)
         return out
 
+    # Segments of DELTA_CHUNKS_FROM tokens and more go by chunks (gated_delta.hip), if one has DELTA_CHUNKS_LONG tokens or
+    # all of them together DELTA_CHUNKS_WORK (token, head) pairs: the first of the two kernels takes 19 us however little
+    # it has to do.  Scan | chunks, microseconds, 16 heads of 128 x 128: one prompt of 64 tokens 21 | 26, 96 30 | 29, 128
+    # 39 | 29, 512 144 | 50, 2,048 726 | 124; 8 prompts of 80 45 | 54, 25 of 80 166 | 139, 50 of 40 177 | 155.
+    DELTA_CHUNK = 64
+    DELTA_CHUNKS_FROM = 32
+    DELTA_CHUNKS_LONG = 96
+    DELTA_CHUNKS_WORK = 16384
+    DELTA_CHUNK_BYTES = 2 << 30  # scratch of a step's chunks at most
+
+    def _delta_chunks(self, ctx, H: int, G: int, dk: int, dv: int, device):
+        """The chunks of the step's long segments ``(segment, first token, tokens)``, those segments ``(segment, first chunk,
+        chunks)``, and whether there are others; ``None``: no segment goes by chunks."""
+        long = [ln for ln in ctx.seg_lens if ln >= self.DELTA_CHUNKS_FROM]
+        if not long or max(long) < self.DELTA_CHUNKS_LONG and sum(long) * H < self.DELTA_CHUNKS_WORK:
+            return None
+        kib = self._query("jle_gated_delta_chunk_kib", H, G, dk, dv)
+        if kib < 0:
+            return None
+        made = ctx.scratch.get("delta_chunks")
+        if made is None:
+            chunks, segs, o, per = [], [], 0, self.DELTA_CHUNK
+            for i, ln in enumerate(ctx.seg_lens):
+                if ln >= self.DELTA_CHUNKS_FROM:
+                    segs += [i, len(chunks) // 3, -(-ln // per)]
+                    for t in range(0, ln, per):
+                        chunks += [i, o + t, min(per, ln - t)]
+                o += ln
+            both = torch.tensor(chunks + segs, dtype=torch.int32).to(device)
+            made = ctx.scratch["delta_chunks"] = (both[: len(chunks)], both[len(chunks):], len(chunks) // 3, len(segs) // 3)
+        nc = made[2]
+        if nc * kib * 1024 > self.DELTA_CHUNK_BYTES:
+            return None
+        return made, torch.empty(nc * kib * 256, dtype=torch.float32, device=device)
+
     def gated_delta(self, rows, gates, a_log, dt_bias, norm_weight, out_gate, num_heads: int, num_kv_heads: int,
                     head_dim: int, value_dim: int, eps: float, floor: float, state, ctx):
         """See ``gated_delta.hip``: unit vectors, write strengths and decays of the step's tokens, the recurrence
@@ -1164,16 +1199,18 @@ class HipOps:
         dkp = self._query("jle_gated_delta_padded", dk)  # (the unit vectors' rows, filled up to what the scan's lanes hold)
         if dkp < dk:
             raise KernelError(f"the gated delta rule's kernels take keys of up to 2048 elements, not {dk}")
-        scratch = torch.empty(n * (2 * G * dkp + 2 * H + G + H * dv), dtype=torch.float32, device=dev)
+        scratch = torch.empty(n * (2 * G * dkp + 2 * H + G + H * dv) + 64, dtype=torch.float32, device=dev)
         qn, kn = scratch[: n * G * dkp], scratch[n * G * dkp: 2 * n * G * dkp]
         o = 2 * n * G * dkp
         beta, decay, kq = scratch[o: o + n * H], scratch[o + n * H: o + 2 * n * H], scratch[o + 2 * n * H: o + 2 * n * H + n * G]
         o_raw = scratch[o + 2 * n * H + n * G:]
         out = torch.empty(n, H * dv, dtype=rows.dtype, device=dev)
+        by_chunks = self._delta_chunks(ctx, H, G, dk, dv, dev)
+        (chunks, segs, nc, ns), ws = by_chunks if by_chunks is not None else ((None, None, 0, 0), None)
         self._call("jle_gated_delta", _p(rows), self._is_bf16(rows), _p(gates), _p(a_log), _p(dt_bias), _p(norm_weight),
                    _p(out_gate), _p(state), _p(ctx.cu_seqlens), _p(ctx.state_slots), _p(ctx.state_phase), _p(qn), _p(kn),
                    _p(beta), _p(decay), _p(kq), _p(o_raw), _p(out), n, ctx.num_segments, H, G, dk, dv, float(eps),
-                   float(floor))
+                   float(floor), _p(chunks), nc, _p(segs), ns, self.DELTA_CHUNKS_FROM, int(ns < ctx.num_segments), _p(ws))
         return out
 
     def gated_unit(self, u, y, y_bias, w_ra, b_ra, w_ri, b_ri, lam, rate: float, state, ctx):
