@@ -9,6 +9,7 @@
 //                        finished with log2(KS) lane swaps; the next tokens' rows are asked for before these are used
 //   gdr_chunk_kernel, gdr_carry_kernel   the same recurrence 64 tokens at a time on the float32 matrix instructions, for
 //                        segments of many tokens (below)
+//   gdr_single_kernel    all of it in one launch, for steps of single tokens
 //   gdr_out_kernel       o / sqrt(mean(o^2) + eps) * w * silu(gate), rounded to the run dtype
 // The memory lies [slot][half][H][dv][dk] (a column's rows together); a step reads the half `phase` and writes the other.  Every sum is formed
 // in an order that depends on the sizes alone, token after token: cutting a sequence into steps changes no bit.
@@ -624,6 +625,136 @@ __global__ __launch_bounds__(64) void gdr_out_kernel(const float* __restrict__ o
   }
 }
 
+// ------------------------------------------------------------------ a step of single tokens
+// One block per (request, head) does all of a token: unit vectors, write strength and decay (as gdr_prepare_kernel forms
+// them), the memory's step, norm and gate (as gdr_out_kernel).  Eight lanes share a column of the memory and read its rows
+// 128 bytes at a time, 64 columns a turn of the block's eight wavefronts; a lane has asked for all its pieces of CP turns
+// before the first barrier, so the memory is on its way while the vectors are normed.  Bound by the memory's bytes, read
+// once and written once: 64 requests with 16 heads of 128 x 128 23 us (134 MB, 5.8 TB/s), 8 requests 5.5, where the three
+// launches, whose scan lays out 16 tokens' vectors for one, took 67 and 18.
+template <typename T, int DK, int CP>
+__global__ __launch_bounds__(512) void gdr_single_kernel(const T* __restrict__ rows, const float* __restrict__ gates,
+                                                         const float* __restrict__ a_log, const float* __restrict__ dt_bias,
+                                                         const float* __restrict__ norm_w, const T* __restrict__ gate,
+                                                         float* __restrict__ state, const int* __restrict__ state_slots,
+                                                         const int* __restrict__ state_phase, T* __restrict__ out, float eps,
+                                                         float floor, int H, int G, int dv) {
+  constexpr int PC = DK / 32;  // 16-byte pieces of a column in a lane
+  __shared__ f32x4 sk[DK / 4], sq[DK / 4];
+  __shared__ float so[64 * CP], s_beta, s_decay, s_kq;
+  const int n = blockIdx.x, h = blockIdx.y, kv = h / (H / G);
+  const int tid = threadIdx.x, lane = tid & 63, ks = tid & 7, c0 = tid >> 3;
+  const int w = wave_index();
+  const int C = 2 * G * DK + H * dv;
+  const size_t slot = (size_t)state_slots[n];
+  const int phase = state_phase[n];
+  const float* s_old = state + ((slot * 2 + phase) * H + h) * (size_t)dv * DK + 4 * ks;
+  float* s_new = state + ((slot * 2 + (1 - phase)) * H + h) * (size_t)dv * DK + 4 * ks;
+  f32x4 S[CP][PC];
+  float v[CP];
+#pragma unroll
+  for (int p = 0; p < CP; ++p) {
+    const int c = min(c0 + 64 * p, dv - 1);
+#pragma unroll
+    for (int j = 0; j < PC; ++j)
+      S[p][j] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(s_old + (size_t)c * DK + 32 * j));
+    v[p] = Num<T>::load(rows + (size_t)n * C + 2 * G * DK + (size_t)h * dv + c);
+  }
+  if (w == 0) {
+    float* dst[2] = {reinterpret_cast<float*>(sq), reinterpret_cast<float*>(sk)};
+    float x[2][DK / 64];
+#pragma unroll
+    for (int which = 0; which < 2; ++which) {
+      const T* src = rows + (size_t)n * C + (size_t)(which * G + kv) * DK;
+      float ss = 0.f;
+#pragma unroll
+      for (int e = 0; e < DK / 64; ++e) {
+        x[which][e] = Num<T>::load(src + lane + 64 * e);
+        ss = __builtin_fmaf(x[which][e], x[which][e], ss);
+      }
+      float inv = 1.0f / sqrtf(wave_sum(ss) + floor);
+      if (which == 0) inv *= 1.0f / sqrtf((float)DK);
+#pragma unroll
+      for (int e = 0; e < DK / 64; ++e) {
+        x[which][e] *= inv;
+        dst[which][lane + 64 * e] = x[which][e];
+      }
+    }
+    float d = 0.f;
+#pragma unroll
+    for (int e = 0; e < DK / 64; ++e) d = __builtin_fmaf(x[0][e], x[1][e], d);
+    d = wave_sum(d);
+    if (lane == 0) s_kq = d;
+  }
+  if (tid == 64) {
+    const float b = gates[(size_t)n * 2 * H + h], a = gates[(size_t)n * 2 * H + H + h] + dt_bias[h];
+    s_beta = 1.0f / (1.0f + expf(-b));
+    const float sp = a > 20.f ? a : log1pf(expf(a));
+    s_decay = expf(-expf(a_log[h]) * sp);
+  }
+  __syncthreads();
+  const float gc = s_decay, bc = s_beta, kqc = s_kq;
+  f32x4 k[PC], q[PC];
+#pragma unroll
+  for (int j = 0; j < PC; ++j) {
+    k[j] = sk[ks + 8 * j];
+    q[j] = sq[ks + 8 * j];
+  }
+#pragma unroll
+  for (int p = 0; p < CP; ++p) {
+    f32x4 d4 = {0.f, 0.f, 0.f, 0.f}, o4 = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < PC; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        d4[i] = __builtin_fmaf(S[p][j][i], k[j][i], d4[i]);
+        o4[i] = __builtin_fmaf(S[p][j][i], q[j][i], o4[i]);
+      }
+    const float dot = column_lanes_sum<8>((d4[0] + d4[1]) + (d4[2] + d4[3]));
+    const float oq = column_lanes_sum<8>((o4[0] + o4[1]) + (o4[2] + o4[3]));
+    const float u = bc * (v[p] - gc * dot);
+    const int c = c0 + 64 * p;
+    if (c < dv) {
+#pragma unroll
+      for (int j = 0; j < PC; ++j) {
+        f32x4 t;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) t[i] = __builtin_fmaf(k[j][i], u, gc * S[p][j][i]);
+        __builtin_nontemporal_store(t, reinterpret_cast<f32x4*>(s_new + (size_t)c * DK + 32 * j));
+      }
+      if (ks == 0) so[c] = __builtin_fmaf(kqc, u, gc * oq);
+    }
+  }
+  __syncthreads();
+  float ss = 0.f;
+  for (int e = lane; e < dv; e += 64) ss = __builtin_fmaf(so[e], so[e], ss);
+  const float inv = 1.0f / sqrtf(wave_sum(ss) / (float)dv + eps);
+  for (int e = tid; e < dv; e += 512) {
+    const size_t at = ((size_t)n * H + h) * dv + e;
+    const float z = Num<T>::load(gate + at);
+    Num<T>::store(out + at, so[e] * inv * norm_w[e] * (z / (1.0f + expf(-z))));
+  }
+}
+
+template <typename T>
+int launch_single(const T* rows, const float* gates, const float* a_log, const float* dt_bias, const float* norm_w,
+                  const T* gate, float* state, const int* state_slots, const int* state_phase, T* out, int R, int H, int G,
+                  int dk, int dv, float eps, float floor, hipStream_t s) {
+#define JLE_SINGLE(DK_, CP_)                                                                                            hipLaunchKernelGGL((gdr_single_kernel<T, DK_, CP_>), dim3(R, H), dim3(512), 0, s, rows, gates, a_log, dt_bias, norm_w,                      gate, state, state_slots, state_phase, out, eps, floor, H, G, dv)
+  if (dk == 128) {
+    if (dv <= 64) JLE_SINGLE(128, 1);
+    else if (dv <= 128) JLE_SINGLE(128, 2);
+    else JLE_SINGLE(128, 4);
+  } else {
+    if (dv <= 64) JLE_SINGLE(64, 1);
+    else if (dv <= 128) JLE_SINGLE(64, 2);
+    else JLE_SINGLE(64, 4);
+  }
+#undef JLE_SINGLE
+  JLE_LAUNCH_CHECK();
+  return 0;
+}
+
 template <typename T>
 int launch_gdr(const T* rows, const float* gates, const float* a_log, const float* dt_bias, const float* norm_w,
                const T* gate, float* state, const int* cu_seqlens, const int* state_slots, const int* state_phase,
@@ -733,4 +864,25 @@ JLE_API int jle_gated_delta(const void* rows, int is_bf16, const float* gates, c
   return launch_gdr<float>((const float*)rows, gates, a_log, dt_bias, norm_w, (const float*)gate, state, cu_seqlens,
                            state_slots, state_phase, qn, kn, beta, decay, kq, o_raw, (float*)out, N, R, H, G, dk, dv, dkp, eps,
                            floor, b, s);
+}
+
+// The sizes at which a step of single tokens is one launch.
+JLE_API int jle_gated_delta_single_supported(int H, int G, int dk, int dv) {
+  return (dk == 64 || dk == 128) && dv > 0 && dv <= 256 && H > 0 && G > 0 && H % G == 0 && H <= 65535;
+}
+
+// jle_gated_delta for a step whose every request has one token (token i is request i's): no scratch.
+JLE_API int jle_gated_delta_single(const void* rows, int is_bf16, const float* gates, const float* a_log,
+                                   const float* dt_bias, const float* norm_w, const void* gate, float* state,
+                                   const int* state_slots, const int* state_phase, void* out, int R, int H, int G, int dk,
+                                   int dv, float eps, float floor, hipStream_t s) {
+  if (R <= 0) return 0;
+  if (!jle_gated_delta_single_supported(H, G, dk, dv) || (uintptr_t)state % 16 || rows == nullptr || gates == nullptr ||
+      state == nullptr || out == nullptr || gate == nullptr)
+    return JLE_BAD_ARG;
+  if (is_bf16)
+    return launch_single<bf16_t>((const bf16_t*)rows, gates, a_log, dt_bias, norm_w, (const bf16_t*)gate, state, state_slots,
+                                 state_phase, (bf16_t*)out, R, H, G, dk, dv, eps, floor, s);
+  return launch_single<float>((const float*)rows, gates, a_log, dt_bias, norm_w, (const float*)gate, state, state_slots,
+                              state_phase, (float*)out, R, H, G, dk, dv, eps, floor, s);
 }

@@ -102,6 +102,7 @@ _SIGNATURES = {
     "jle_diff_combine": [_vp, _vp, _vp, _f, _f, _f, _i, _i, _i, _i, _i, _i, _vp],
     "jle_gated_delta": [_vp, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i,
                         _i, _i, _i, _i, _f, _f, _vp, _i, _vp, _i, _i, _i, _vp, _vp],
+    "jle_gated_delta_single": [_vp, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _f, _f, _vp],
     "jle_moe_choose": [_vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _f, _f, _i, _vp, _vp, _vp, _vp, _i, _i, _vp],
     "jle_moe_choose_groups": [_i, _i, _i, _i],
     "jle_mamba2": [_vp, _i, _vp, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _f, _i,
@@ -181,7 +182,8 @@ def _bind(path: str):
                        ("jle_latent_attention_mfma_supported", [_i, _i, _i, _i, _i]),
                        ("jle_latent_expanded_supported", [_i, _i, _i, _i, _i]), ("jle_attention_group_waves", []),
                        ("jle_mlstm_chunked_supported", [_i, _i]), ("jle_mlstm_chunk_tokens", []),
-                       ("jle_gated_delta_padded", [_i]), ("jle_gated_delta_chunk_kib", [_i, _i, _i, _i]), ("jle_gated_unit_chunk_tokens", []),
+                       ("jle_gated_delta_padded", [_i]), ("jle_gated_delta_chunk_kib", [_i, _i, _i, _i]),
+                       ("jle_gated_delta_single_supported", [_i, _i, _i, _i]), ("jle_gated_unit_chunk_tokens", []),
                        ("jle_retention_chunk_tokens", []), ("jle_retention_chunked_supported", [_i, _i]),
                        ("jle_retention_workspace_kib", [_i, _i, _i, _i])):
         fn = getattr(lib, name, None)
@@ -1196,6 +1198,12 @@ class HipOps:
                                (ctx.state_phase, "state phases", (ctx.num_segments,))):
             self._chk(t, torch.int32, shape, what)
         dev = rows.device
+        if ctx.max_seg_len == 1 and self._query("jle_gated_delta_single_supported", H, G, dk, dv):
+            out = torch.empty(n, H * dv, dtype=rows.dtype, device=dev)
+            self._call("jle_gated_delta_single", _p(rows), self._is_bf16(rows), _p(gates), _p(a_log), _p(dt_bias),
+                       _p(norm_weight), _p(out_gate), _p(state), _p(ctx.state_slots), _p(ctx.state_phase), _p(out), n, H, G,
+                       dk, dv, float(eps), float(floor))
+            return out
         dkp = self._query("jle_gated_delta_padded", dk)  # (the unit vectors' rows, filled up to what the scan's lanes hold)
         if dkp < dk:
             raise KernelError(f"the gated delta rule's kernels take keys of up to 2048 elements, not {dk}")

@@ -1,5 +1,5 @@
-"""The gated delta rule 64 tokens at a time (``csrc/gated_delta.hip``) against its recurrence in 64 bits, beside the
-token-by-token kernel on the same inputs."""
+"""The gated delta rule 64 tokens at a time, and of a step of single tokens in one launch (``csrc/gated_delta.hip``),
+against its recurrence in 64 bits, beside the token-by-token kernel on the same inputs."""
 import types
 
 import pytest
@@ -16,6 +16,9 @@ CASES = [  # (segment lengths, H, G, dk, dv, what is special)
     ([129, 63], 3, 1, 64, 16, ""),                         # the other key size, one tile of values
     ([300], 2, 1, 128, 256, "strong decays"),              # products of decays underflow within a chunk, weak ones after
     ([257], 2, 2, 128, 128, "one key again and again"),    # L is full: every token writes over what the last one wrote
+    ([1] * 5, 4, 2, 128, 128, ""),                         # single tokens
+    ([1], 3, 3, 64, 40, ""),                               # values that fill no turn of the block's columns
+    ([1] * 3, 2, 1, 64, 256, "strong decays"),
 ]
 
 
@@ -57,7 +60,7 @@ def test_chunks_against_the_recurrence(lens, H, G, dk, dv, special, dtype):
     state = rn(R + 1, 2, H, dv, dk)
     cu = torch.tensor([0] + lens).cumsum(0).int()
     got = {}
-    for way, first in (("chunks", 32), ("scan", 1 << 30)):
+    for way, first in (("chunks", 32), ("scan", 1 << 30)):  # ("chunks": or, of single tokens, the one launch)
         ops.DELTA_CHUNKS_FROM, ops.DELTA_CHUNKS_LONG = first, 1
         ctx = types.SimpleNamespace(seg_lens=lens, num_segments=R, cu_seqlens=cu.to(DEV), state_slots=slots.to(DEV),
                                     state_phase=phase.to(DEV), scratch={},
