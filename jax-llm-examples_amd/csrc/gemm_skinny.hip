@@ -404,7 +404,9 @@ JLE_API int jle_gemm_skinny(const void* X, const void* W, void* Y, const int* of
   if (K <= 0 || K % 8 || G < 1 || G > 65535 || (swiglu && Nout % 2)) return JLE_BAD_ARG;
   if (tiled && (K % 32 || Nout % 16 || (swiglu && (Nout / 2) % 16))) return JLE_BAD_ARG;
   if (max_rows <= 0 || max_rows > M) max_rows = M;
-  const int mt = (offsets == nullptr && max_rows > 32) ? 4 : (offsets == nullptr && max_rows > 16) ? 2 : 1;
+  // Groups of eight rows and more on average: some have over 16, and a second block would read their weights again.
+  const bool fuller = offsets != nullptr && M >= 8 * G;
+  const int mt = (offsets == nullptr && max_rows > 32) ? 4 : (fuller || (offsets == nullptr && max_rows > 16)) ? 2 : 1;
   const int ytiles = (max_rows + 16 * mt - 1) / (16 * mt);
   if (ytiles > 65535) return JLE_BAD_ARG;
   const int xrows = swiglu ? Nout / 2 : Nout;  // output columns to cover
@@ -414,6 +416,12 @@ JLE_API int jle_gemm_skinny(const void* X, const void* W, void* Y, const int* of
     const long long pair_tiles = (long long)((xrows + (swiglu ? 15 : 31)) / (swiglu ? 16 : 32)) * groups;
     if (swiglu) variant = 20408;
     else if (pair_tiles >= 4096) variant = 20408;  // very many rows of W (the output head)
+    // fuller groups: what a block reads of X is as much as its weights with 16 of their rows, so it takes 32 where that
+    // leaves four blocks a compute unit (one row tile, 16 rows of X a block | 32 rows of X | and two row tiles, in
+    // microseconds: 8 groups of 4,096 x 2,048 with 128 rows 36 | 32 | 27, with 64 24 | 24 | 24; of 7,168 x 4,096 with 128
+    // 127 | 108 | 83, with 64 79 | 78 | 73; of 2,048 x 4,096 with 128 39 | 35 | 36; 16 of 5,120 x 8,192 with 128
+    // 221 | 224 | 203; gate and up of 8 of 8,192 x 2,048 with 128 61 | 49)
+    else if (fuller && pair_tiles >= 1024) variant = 20408;
     else variant = 10408;  // one row tile per block: more blocks in flight
     if (split_tiles > 0) variant = 10804;  // cut tiles: eight wavefronts a block (measured: 12.5 against 14.0 us for 5120 x 5120)
   } else if (variant < 0) {  // (tuning: this variant, with the cut tiles)

@@ -1056,6 +1056,35 @@ def test_weight_streaming_product_grouped_with_swiglu(ops, ref, n, d, f, e, k):
     assert float((plain - gu).abs().max() / gu.abs().max()) <= 2e-5
 
 
+@pytest.mark.parametrize("tiled", [False, True])
+@pytest.mark.parametrize("counts,nout,k", [([17, 0, 32, 33, 1], 96, 160), ([24], 4096 * 16, 64), ([40, 8], 80, 72),
+                                           ([16, 15, 64, 9], 8192, 96)])
+def test_weight_streaming_product_of_fuller_groups(ops, counts, nout, k, tiled):
+    """Groups of eight rows and more on average take 32 rows a block, and with many rows of W two row tiles: groups that
+    end at, before and behind 16 and 32 rows, empty ones between."""
+    if tiled and (k % 32 or nout % 32):
+        pytest.skip("no whole tiles")
+    m, e = sum(counts), len(counts)
+    x, w = _rand(m, k, dt=torch.bfloat16, seed=1), _rand(e, nout, k, dt=torch.bfloat16, scale=0.1, seed=2)
+    off = torch.tensor([0] + counts).cumsum(0).int().to(DEV)
+    stored = w
+    if tiled:
+        from jax_llm_examples_amd.ops.layout import tile_
+        stored = w.clone()
+        tile_(stored)
+    got = ops.gemm_skinny(x, stored, offsets=off, out_f32=True, tiled=tiled)
+    act = ops.gemm_skinny(x, stored, offsets=off, swiglu=True, tiled=tiled)
+    o = 0
+    for c, we in zip(counts, w):
+        want = x[o: o + c].double() @ we.double().T
+        if c:
+            # float32 sums of k products of bfloat16 numbers: sqrt(k) 2^-24 of the terms' size, with room
+            assert float((got[o: o + c].double() - want).norm() / want.norm()) <= 2e-6
+            want = torch.nn.functional.silu(want[:, : nout // 2]) * want[:, nout // 2:]
+            assert float((act[o: o + c].double() - want).norm() / want.norm()) <= 2.0 ** -8  # (rounded to bfloat16)
+        o += c
+
+
 @pytest.mark.parametrize("n,d,f,e,k", [(300, 128, 48, 16, 1), (700, 264, 72, 3, 2), (2048, 512, 256, 16, 1),
                                        (150, 64, 40, 128, 1)])
 def test_grouped_product_for_many_rows(ops, ref, n, d, f, e, k):
