@@ -7,10 +7,11 @@
 //     h  = x' / sqrt(mean(x'^2) + eps) * w                          the next branch's input
 //     hs = h + (h_prev - h) * shift                                 h_prev: the float32 h of the token before
 // h_prev of a segment's first row comes from the request's state (zeros at position 0); the h of a segment's last
-// row goes into the state's other half.  A block takes `rows_per_block` consecutive rows one after the other and
-// keeps the last h in registers; if its first row is not a segment's first, it forms the h of the row before
-// anew (which is why the sum is not written in place).  Every row's arithmetic is the same whatever block it
-// is in, so a token's result does not depend on how its request was cut into steps or batched.
+// row goes into the state's other half.  With few rows a block forms its row and, if that is not a segment's first,
+// the h of the row before anew (which is why the sum is not written in place).  With many rows that is twice the
+// reading and two more reductions a row, so the first kernel leaves x' and 1 / sqrt(mean(x'^2) + eps) only, and
+// shift_rows_kernel streams down the columns of x' with the last row's h in registers.  Every row's arithmetic is the
+// same in both, so a token's result does not depend on how its request was cut into steps or batched.
 #include "common.h"
 #include "rows.h"
 
@@ -22,20 +23,45 @@ constexpr int kThreads = 256;
 
 template <typename T, int VEC>
 __device__ __forceinline__ void load_piece(const T* p, float (&o)[VEC]) {
-  if constexpr (VEC == 4) {
-    const f32x4_t r = load4<T>(p);
+  if constexpr (VEC == 8 && sizeof(T) == 2) {
+    typedef __attribute__((ext_vector_type(4))) unsigned u32x4;
+    const u32x4 r = *reinterpret_cast<const u32x4*>(p);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) o[e] = r[e];
+    for (int e = 0; e < 4; ++e) {
+      o[2 * e] = __uint_as_float(r[e] << 16);
+      o[2 * e + 1] = __uint_as_float(r[e] & 0xffff0000u);
+    }
+  } else if constexpr (VEC >= 4) {
+#pragma unroll
+    for (int e = 0; e < VEC; e += 4) {
+      const f32x4_t r = load4<T>(p + e);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) o[e + i] = r[i];
+    }
   } else {
     o[0] = Num<T>::load(p);
   }
 }
 template <typename T, int VEC>
 __device__ __forceinline__ void store_piece(T* p, const float (&o)[VEC]) {
-  if constexpr (VEC == 4) {
-    store4<T>(p, f32x4_t{o[0], o[1], o[2], o[3]});
+  if constexpr (VEC == 8 && sizeof(T) == 2) {
+    typedef __attribute__((ext_vector_type(4))) unsigned u32x4;
+    *reinterpret_cast<u32x4*>(p) = u32x4{pack_bf16(o[0], o[1]), pack_bf16(o[2], o[3]), pack_bf16(o[4], o[5]), pack_bf16(o[6], o[7])};
+  } else if constexpr (VEC >= 4) {
+#pragma unroll
+    for (int e = 0; e < VEC; e += 4) store4<T>(p + e, f32x4_t{o[e], o[e + 1], o[e + 2], o[e + 3]});
   } else {
     Num<T>::store(p, o[0]);
+  }
+}
+// a vector of weights, or `fill` where there is none or the row has ended
+template <int VEC>
+__device__ __forceinline__ void load_weights(const float* p, int d, bool in, float fill, float (&o)[VEC]) {
+  if (p != nullptr && in) {
+    load_piece<float, VEC>(p + d, o);
+  } else {
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) o[e] = fill;
   }
 }
 
@@ -61,88 +87,102 @@ struct SandwichArgs {
   const int* cu_seqlens;
   const int* state_slots;
   const int* state_phase;
-  int N, D, rows_per_block;
+  float* stats;          // [N] or null: 1 / sqrt(mean(x'^2) + eps) and no rows
+  int N, D;
 };
 
-template <typename T, int CPT, int VEC>
-__global__ __launch_bounds__(kThreads) void add_norm_shift_kernel(SandwichArgs a) {
-  __shared__ float red[kThreads / 64];
+// A block takes one row.  Everything it reads - the row's three arrays, the weights, the state - is asked for before the
+// first sum, where the registers allow it (a thread's 8 elements of rows of up to 8,192: as many threads as that takes):
+// each of the chain's stages would otherwise begin with a trip to memory.  8 rows of 2,048: 6.0 us, with the weights loaded
+// where they are used, an element at a time, 11.4; 2,048 rows of 4,096 without a shift 26 us (115 MB, 4.5 TB/s), before 36.
+template <typename T, int THREADS, int CPT, int VEC>
+__global__ __launch_bounds__(THREADS) void add_norm_shift_kernel(SandwichArgs a) {
+  __shared__ float red[THREADS / 64];
+  constexpr bool HOLD = CPT == 1;
   const int D = a.D;
-  const int r0 = blockIdx.x * a.rows_per_block;
-  const int r1 = min(a.N, r0 + a.rows_per_block);
+  const int row = blockIdx.x;
   const bool shift = a.shift_w != nullptr;
+  int first = 0, last = 0, slot = 0, phase = 0, pos = 0;
+  if (shift) {
+    const int seg = a.token_segment[row];
+    first = a.cu_seqlens[seg];
+    last = a.cu_seqlens[seg + 1] - 1;
+    slot = a.state_slots[seg];
+    phase = a.state_phase[seg];
+    pos = a.positions[row];
+  }
   float hprev[CPT][VEC];
+  float wy[HOLD ? CPT : 1][VEC], wg[HOLD ? CPT : 1][VEC], wp[HOLD ? CPT : 1][VEC], wn[HOLD ? CPT : 1][VEC],
+      ws[HOLD ? CPT : 1][VEC];
 #pragma unroll
-  for (int i = 0; i < CPT; ++i)
+  for (int i = 0; i < CPT; ++i) {
+    const int d = (threadIdx.x + THREADS * i) * VEC;
 #pragma unroll
     for (int e = 0; e < VEC; ++e) hprev[i][e] = 0.f;
-  int r = r0;
-  if (shift && r0 > 0 && a.cu_seqlens[a.token_segment[r0]] != r0) r = r0 - 1;  // the row before, formed anew
-  for (; r < r1; ++r) {
-    const bool write = r >= r0;
+    if (shift && row == first && pos != 0 && d < D)
+      load_piece<float, VEC>(a.state + ((size_t)slot * 2 + phase) * D + d, hprev[i]);
+    if constexpr (HOLD) {
+      load_weights<VEC>(a.y_bias, d, d < D, 0.f, wy[i]);
+      load_weights<VEC>(a.g_bias, d, d < D, 0.f, wg[i]);
+      load_weights<VEC>(a.post_w, d, d < D, 1.f, wp[i]);
+      load_weights<VEC>(a.w, d, d < D, 1.f, wn[i]);
+      load_weights<VEC>(a.shift_w, d, d < D, 0.f, ws[i]);
+    }
+  }
+  // (with a shift: the row before first, if it is the same segment's)
+  for (int r = shift && row > first ? row - 1 : row; r <= row; ++r) {
+    const bool write = r == row;
     const size_t base = (size_t)r * D;
-    float v[CPT][VEC];
+    float v[CPT][VEC], t[CPT][VEC], gg[CPT][VEC];
 #pragma unroll
     for (int i = 0; i < CPT; ++i) {
-      const int d = (threadIdx.x + kThreads * i) * VEC;
+      const int d = (threadIdx.x + THREADS * i) * VEC;
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) v[i][e] = t[i][e] = gg[i][e] = 0.f;
       if (d < D) {
         load_piece<float, VEC>(a.x + base + d, v[i]);
-      } else {
-#pragma unroll
-        for (int e = 0; e < VEC; ++e) v[i][e] = 0.f;
+        if (a.delta_kind != 0) load_piece<T, VEC>((const T*)a.y + base + d, t[i]);
+        if (a.delta_kind == 2) load_piece<T, VEC>((const T*)a.g + base + d, gg[i]);
       }
     }
     if (a.delta_kind == 1) {
 #pragma unroll
-      for (int i = 0; i < CPT; ++i) {
-        const int d = (threadIdx.x + kThreads * i) * VEC;
-        if (d < D) {
-          float t[VEC];
-          load_piece<T, VEC>((const T*)a.y + base + d, t);
+      for (int i = 0; i < CPT; ++i)
 #pragma unroll
-          for (int e = 0; e < VEC; ++e) v[i][e] += t[e];
-        }
-      }
+        for (int e = 0; e < VEC; ++e) v[i][e] += t[i][e];
     } else if (a.delta_kind == 2) {
-      float t[CPT][VEC];
       float ss = 0.f;
 #pragma unroll
       for (int i = 0; i < CPT; ++i) {
-        const int d = (threadIdx.x + kThreads * i) * VEC;
-#pragma unroll
-        for (int e = 0; e < VEC; ++e) t[i][e] = 0.f;
+        const int d = (threadIdx.x + THREADS * i) * VEC;
+        if constexpr (!HOLD) {
+          load_weights<VEC>(a.y_bias, d, d < D, 0.f, wy[0]);
+          load_weights<VEC>(a.g_bias, d, d < D, 0.f, wg[0]);
+        }
         if (d < D) {
-          float yy[VEC], gg[VEC];
-          load_piece<T, VEC>((const T*)a.y + base + d, yy);
-          load_piece<T, VEC>((const T*)a.g + base + d, gg);
 #pragma unroll
           for (int e = 0; e < VEC; ++e) {
-            const float yb = a.y_bias != nullptr ? yy[e] + a.y_bias[d + e] : yy[e];
-            const float gb = a.g_bias != nullptr ? gg[e] + a.g_bias[d + e] : gg[e];
+            const float yb = t[i][e] + wy[HOLD ? i : 0][e];
+            const float gb = gg[i][e] + wg[HOLD ? i : 0][e];
             t[i][e] = yb * (1.0f / (1.0f + expf(-gb)));
             ss = __builtin_fmaf(t[i][e], t[i][e], ss);
           }
         }
       }
-      const float tot = block_sum<kThreads>(ss, red);
+      const float tot = block_sum<THREADS>(ss, red);
       const float inv = 1.0f / sqrtf(tot / (float)D + a.post_eps);
 #pragma unroll
       for (int i = 0; i < CPT; ++i) {
-        const int d = (threadIdx.x + kThreads * i) * VEC;
-        if (d < D) {
+        const int d = (threadIdx.x + THREADS * i) * VEC;
+        if constexpr (!HOLD) load_weights<VEC>(a.post_w, d, d < D, 1.f, wp[0]);
 #pragma unroll
-          for (int e = 0; e < VEC; ++e) {
-            float u = t[i][e] * inv;
-            if (a.post_w != nullptr) u *= a.post_w[d + e];
-            v[i][e] += u;
-          }
-        }
+        for (int e = 0; e < VEC; ++e) v[i][e] += t[i][e] * inv * wp[HOLD ? i : 0][e];
       }
     }
     if (write && a.x_out != nullptr) {
 #pragma unroll
       for (int i = 0; i < CPT; ++i) {
-        const int d = (threadIdx.x + kThreads * i) * VEC;
+        const int d = (threadIdx.x + THREADS * i) * VEC;
         if (d < D) store_piece<float, VEC>(a.x_out + base + d, v[i]);
       }
     }
@@ -152,85 +192,118 @@ __global__ __launch_bounds__(kThreads) void add_norm_shift_kernel(SandwichArgs a
     for (int i = 0; i < CPT; ++i)
 #pragma unroll
       for (int e = 0; e < VEC; ++e) ss = __builtin_fmaf(v[i][e], v[i][e], ss);
-    const float tot = block_sum<kThreads>(ss, red);
+    const float tot = block_sum<THREADS>(ss, red);
     const float inv = 1.0f / sqrtf(tot / (float)D + a.eps);
-    int seg = 0, first = 0, last = 0, slot = 0, phase = 0, pos = 0;
-    if (shift && write) {
-      seg = a.token_segment[r];
-      first = a.cu_seqlens[seg];
-      last = a.cu_seqlens[seg + 1] - 1;
-      slot = a.state_slots[seg];
-      phase = a.state_phase[seg];
-      pos = a.positions[r];
+    if (a.stats != nullptr) {
+      if (threadIdx.x == 0) a.stats[r] = inv;
+      continue;
     }
 #pragma unroll
     for (int i = 0; i < CPT; ++i) {
-      const int d = (threadIdx.x + kThreads * i) * VEC;
-      if (d < D) {
-        float h[VEC];
+      const int d = (threadIdx.x + THREADS * i) * VEC;
+      if (d >= D) continue;
+      if constexpr (!HOLD) load_weights<VEC>(a.w, d, true, 1.f, wn[0]);
+      float h[VEC];
 #pragma unroll
-        for (int e = 0; e < VEC; ++e) {
-          h[e] = v[i][e] * inv;
-          if (a.w != nullptr) h[e] *= a.w[d + e];
+      for (int e = 0; e < VEC; ++e) h[e] = v[i][e] * inv * wn[HOLD ? i : 0][e];
+      if (write) {
+        if (a.h_out != nullptr) store_piece<T, VEC>((T*)a.h_out + base + d, h);
+        if (shift) {
+          if constexpr (!HOLD) load_weights<VEC>(a.shift_w, d, true, 0.f, ws[0]);
+          float hs[VEC];
+#pragma unroll
+          for (int e = 0; e < VEC; ++e) hs[e] = h[e] + (hprev[i][e] - h[e]) * ws[HOLD ? i : 0][e];
+          store_piece<T, VEC>((T*)a.hs_out + base + d, hs);
+          if (r == last) store_piece<float, VEC>(a.state + ((size_t)slot * 2 + (1 - phase)) * D + d, h);
         }
-        if (write) {
-          if (a.h_out != nullptr) store_piece<T, VEC>((T*)a.h_out + base + d, h);
-          if (shift) {
-            if (r == first) {
-              if (pos == 0) {
+      }
 #pragma unroll
-                for (int e = 0; e < VEC; ++e) hprev[i][e] = 0.f;
-              } else {
-                load_piece<float, VEC>(a.state + ((size_t)slot * 2 + phase) * D + d, hprev[i]);
-              }
-            }
-            float hs[VEC];
+      for (int e = 0; e < VEC; ++e) hprev[i][e] = h[e];
+    }
+  }
+}
+
+// The rows from the sums and their statistics: a block takes kShiftRows rows of kThreads * VEC columns, all of whose
+// values are asked for before the first is used.  Bound by its bytes (a row of 4,096: 16 KB read, 16 KB written): 2,048 rows
+// of 4,096 16 us behind 26 for the sums and statistics, where blocks of four rows and the one before took 90.
+constexpr int kShiftRows = 8;
+template <typename T, int VEC>
+__global__ __launch_bounds__(kThreads) void shift_rows_kernel(SandwichArgs a) {
+  const int D = a.D, r0 = blockIdx.x * kShiftRows, r1 = min(a.N, r0 + kShiftRows);
+  const int d = (blockIdx.y * kThreads + threadIdx.x) * VEC;
+  if (d >= D) return;
+  const float* x = a.x_out != nullptr ? a.x_out : a.x;
+  float v[kShiftRows + 1][VEC], inv[kShiftRows + 1], w[VEC], sw[VEC], hprev[VEC];
 #pragma unroll
-            for (int e = 0; e < VEC; ++e) hs[e] = h[e] + (hprev[i][e] - h[e]) * a.shift_w[d + e];
-            store_piece<T, VEC>((T*)a.hs_out + base + d, hs);
-            if (r == last) store_piece<float, VEC>(a.state + ((size_t)slot * 2 + (1 - phase)) * D + d, h);
-          }
-        }
+  for (int j = 0; j <= kShiftRows; ++j) {  // (place 0: the row before the block's)
+    const int r = max(0, min(r0 - 1 + j, r1 - 1));
+    load_piece<float, VEC>(x + (size_t)r * D + d, v[j]);
+    inv[j] = a.stats[r];
+  }
+  load_weights<VEC>(a.w, d, true, 1.f, w);
+  load_weights<VEC>(a.shift_w, d, true, 0.f, sw);
 #pragma unroll
-        for (int e = 0; e < VEC; ++e) hprev[i][e] = h[e];
+  for (int e = 0; e < VEC; ++e) hprev[e] = v[0][e] * inv[0] * w[e];
+#pragma unroll
+  for (int j = 1; j <= kShiftRows; ++j) {
+    const int r = r0 - 1 + j;
+    if (r >= r1) break;
+    const int seg = a.token_segment[r];
+    if (r == a.cu_seqlens[seg]) {
+      if (a.positions[r] == 0) {
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) hprev[e] = 0.f;
+      } else {
+        load_piece<float, VEC>(a.state + ((size_t)a.state_slots[seg] * 2 + a.state_phase[seg]) * D + d, hprev);
       }
     }
+    float h[VEC], hs[VEC];
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) {
+      h[e] = v[j][e] * inv[j] * w[e];
+      hs[e] = h[e] + (hprev[e] - h[e]) * sw[e];
+      hprev[e] = h[e];
+    }
+    if (a.h_out != nullptr) store_piece<T, VEC>((T*)a.h_out + (size_t)r * D + d, h);
+    store_piece<T, VEC>((T*)a.hs_out + (size_t)r * D + d, hs);
+    if (r == a.cu_seqlens[seg + 1] - 1)
+      store_piece<float, VEC>(a.state + ((size_t)a.state_slots[seg] * 2 + (1 - a.state_phase[seg])) * D + d, h);
   }
 }
 
 template <typename T, int VEC>
-int launch_sandwich(const SandwichArgs& a, hipStream_t s) {
-  const int pieces = (a.D + VEC - 1) / VEC;
-  const int cpt = (pieces + kThreads - 1) / kThreads;
-  dim3 g((unsigned)((a.N + a.rows_per_block - 1) / a.rows_per_block)), b(kThreads);
-#define JLE_SANDWICH_CASE(C)                                                                   \
-  if (cpt <= C) {                                                                              \
-    hipLaunchKernelGGL((add_norm_shift_kernel<T, C, VEC>), g, b, 0, s, a);                     \
-    return 0;                                                                                  \
-  }
-  JLE_SANDWICH_CASE(1)
-  JLE_SANDWICH_CASE(2)
-  JLE_SANDWICH_CASE(4)
-  JLE_SANDWICH_CASE(8)
-  if (VEC == 1) {
-    JLE_SANDWICH_CASE(16)
-    JLE_SANDWICH_CASE(32)
-  }
+int launch_sandwich(const SandwichArgs& args, hipStream_t s) {
+  const int strips = (args.D + kThreads * VEC - 1) / (kThreads * VEC);
+  SandwichArgs a = args;
+  if (a.stats != nullptr) a.shift_w = nullptr;  // (the first kernel: sums and statistics)
+  const dim3 g((unsigned)a.N);
+#define JLE_SANDWICH_CASE(TH, C) \
+  else if (a.D <= TH * C * VEC) hipLaunchKernelGGL((add_norm_shift_kernel<T, TH, C, VEC>), g, dim3(TH), 0, s, a)
+  if (a.D <= 256 * VEC) hipLaunchKernelGGL((add_norm_shift_kernel<T, 256, 1, VEC>), g, dim3(256), 0, s, a);
+  JLE_SANDWICH_CASE(512, 1);
+  JLE_SANDWICH_CASE(1024, 1);
+  else if constexpr (VEC > 1) return JLE_BAD_ARG;  // (such rows go an element a thread)
+  JLE_SANDWICH_CASE(1024, 8);
+  else return JLE_BAD_ARG;
 #undef JLE_SANDWICH_CASE
-  return JLE_BAD_ARG;
+  if (args.stats != nullptr)
+    hipLaunchKernelGGL((shift_rows_kernel<T, VEC>), dim3((unsigned)((a.N + kShiftRows - 1) / kShiftRows), (unsigned)strips), dim3(kThreads),
+                       0, s, args);
+  return 0;
 }
 
 // ------------------------------------------------------------------ polynomial activation
 // out = c0 N(u) + c1 N(u^2) + c2 N(u^3) + c3,  u = z + bias,  N(v) = v / sqrt(mean(v^2) + eps) over the row.
-// PIECES > 0: the row (up to kThreads * VEC * PIECES wide) stays in registers between the sums and the polynomial;
+// PIECES > 0: the row (up to THREADS * VEC * PIECES wide) stays in registers between the sums and the polynomial;
 // PIECES == 0: any width, the row is read twice.
-template <typename T, int VEC, int PIECES>
-__global__ __launch_bounds__(kThreads) void polynorm_kernel(const T* __restrict__ z, int ldz,
+template <typename T, int THREADS, int VEC, int PIECES>
+__global__ __launch_bounds__(THREADS) void polynorm_kernel(const T* __restrict__ z, int ldz,
                                                             const float* __restrict__ bias,
                                                             const float* __restrict__ coef, float eps,
                                                             T* __restrict__ out, int F) {
-  __shared__ float red[kThreads / 64];
+  __shared__ float red[3][THREADS / 64];
   const size_t row = blockIdx.x;
+  const float c0 = coef[0], c1 = coef[1], c2 = coef[2], c3 = coef[3];
   const T* zr = z + row * ldz;
   T* o = out + row * F;
   float s1 = 0.f, s2 = 0.f, s3 = 0.f;
@@ -246,8 +319,10 @@ __global__ __launch_bounds__(kThreads) void polynorm_kernel(const T* __restrict_
   auto fetch = [&](int d, float (&u)[VEC]) {
     load_piece<T, VEC>(zr + d, u);
     if (bias != nullptr) {
+      float b[VEC];
+      load_piece<float, VEC>(bias + d, b);
 #pragma unroll
-      for (int e = 0; e < VEC; ++e) u[e] += bias[d + e];
+      for (int e = 0; e < VEC; ++e) u[e] += b[e];
     }
   };
   constexpr int P = PIECES > 0 ? PIECES : 1;
@@ -255,7 +330,7 @@ __global__ __launch_bounds__(kThreads) void polynorm_kernel(const T* __restrict_
   if constexpr (PIECES > 0) {
 #pragma unroll
     for (int i = 0; i < PIECES; ++i) {
-      const int d = (threadIdx.x + kThreads * i) * VEC;
+      const int d = (threadIdx.x + THREADS * i) * VEC;
 #pragma unroll
       for (int e = 0; e < VEC; ++e) kept[i][e] = 0.f;
       if (d < F) fetch(d, kept[i]);
@@ -263,19 +338,30 @@ __global__ __launch_bounds__(kThreads) void polynorm_kernel(const T* __restrict_
 #pragma unroll
     for (int i = 0; i < PIECES; ++i) sums(kept[i]);  // (zeros beyond the row's end add nothing)
   } else {
-    for (int d = threadIdx.x * VEC; d < F; d += kThreads * VEC) {
+    for (int d = threadIdx.x * VEC; d < F; d += THREADS * VEC) {
       float u[VEC];
       fetch(d, u);
       sums(u);
     }
   }
-  const float t1 = block_sum<kThreads>(s1, red);
-  const float t2 = block_sum<kThreads>(s2, red);
-  const float t3 = block_sum<kThreads>(s3, red);
-  const float i1 = coef[0] / sqrtf(t1 / (float)F + eps);
-  const float i2 = coef[1] / sqrtf(t2 / (float)F + eps);
-  const float i3 = coef[2] / sqrtf(t3 / (float)F + eps);
-  const float c3 = coef[3];
+  // (the three sums together: one barrier instead of six)
+  s1 = wave_sum(s1);
+  s2 = wave_sum(s2);
+  s3 = wave_sum(s3);
+  if ((threadIdx.x & 63) == 0) {
+    red[0][threadIdx.x >> 6] = s1;
+    red[1][threadIdx.x >> 6] = s2;
+    red[2][threadIdx.x >> 6] = s3;
+  }
+  __syncthreads();
+  float t[3] = {0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < THREADS / 64; ++i)
+#pragma unroll
+    for (int j = 0; j < 3; ++j) t[j] += red[j][i];
+  const float i1 = c0 / sqrtf(t[0] / (float)F + eps);
+  const float i2 = c1 / sqrtf(t[1] / (float)F + eps);
+  const float i3 = c2 / sqrtf(t[2] / (float)F + eps);
   auto poly = [&](const float (&u)[VEC], float (&v)[VEC]) {
 #pragma unroll
     for (int e = 0; e < VEC; ++e) {
@@ -286,7 +372,7 @@ __global__ __launch_bounds__(kThreads) void polynorm_kernel(const T* __restrict_
   if constexpr (PIECES > 0) {
 #pragma unroll
     for (int i = 0; i < PIECES; ++i) {
-      const int d = (threadIdx.x + kThreads * i) * VEC;
+      const int d = (threadIdx.x + THREADS * i) * VEC;
       if (d < F) {
         float v[VEC];
         poly(kept[i], v);
@@ -294,7 +380,7 @@ __global__ __launch_bounds__(kThreads) void polynorm_kernel(const T* __restrict_
       }
     }
   } else {
-    for (int d = threadIdx.x * VEC; d < F; d += kThreads * VEC) {
+    for (int d = threadIdx.x * VEC; d < F; d += THREADS * VEC) {
       float u[VEC], v[VEC];
       fetch(d, u);
       poly(u, v);
@@ -305,47 +391,50 @@ __global__ __launch_bounds__(kThreads) void polynorm_kernel(const T* __restrict_
 
 template <typename T>
 void launch_polynorm(const T* z, int ldz, const float* bias, const float* coef, float eps, T* out, int N, int F,
-                     bool vec, hipStream_t s) {
-  // (which form runs depends on the width and on where the arrays lie, not on the step; the sums of a row are
-  // formed in the same order in the forms that keep the row and in the one that reads it twice)
-  dim3 g(N), b(kThreads);
-  if (vec && F <= kThreads * 4 * 4)
-    hipLaunchKernelGGL((polynorm_kernel<T, 4, 4>), g, b, 0, s, z, ldz, bias, coef, eps, out, F);
-  else if (vec && F <= kThreads * 4 * 16)
-    hipLaunchKernelGGL((polynorm_kernel<T, 4, 16>), g, b, 0, s, z, ldz, bias, coef, eps, out, F);
-  else if (vec)
-    hipLaunchKernelGGL((polynorm_kernel<T, 4, 0>), g, b, 0, s, z, ldz, bias, coef, eps, out, F);
-  else
-    hipLaunchKernelGGL((polynorm_kernel<T, 1, 0>), g, b, 0, s, z, ldz, bias, coef, eps, out, F);
+                     int vec, hipStream_t s) {
+  // (which form runs depends on the width and on where the arrays lie, not on the step; 2,048 rows of 14,336 in 16-byte
+  // pieces, the three sums behind one barrier: 34 us, 3.4 TB/s; in pieces of four with a barrier pair a sum 66; 8 rows of
+  // 8,192 7.1 and 12.6)
+#define JLE_POLYNORM(TH, V, P) \
+  hipLaunchKernelGGL((polynorm_kernel<T, TH, V, P>), dim3(N), dim3(TH), 0, s, z, ldz, bias, coef, eps, out, F)
+  if (vec == 8 && F <= 256 * 8 * 2) JLE_POLYNORM(256, 8, 2);
+  else if (vec == 8 && F <= 512 * 8 * 4) JLE_POLYNORM(512, 8, 4);
+  else if (vec == 8) JLE_POLYNORM(256, 8, 0);
+  else if (vec == 4) JLE_POLYNORM(256, 4, 0);
+  else JLE_POLYNORM(256, 1, 0);
+#undef JLE_POLYNORM
 }
 
 }  // namespace
 
+// stats: null, or N floats of scratch: with a shift, the rows are formed by a second kernel (for many rows).
 JLE_API int jle_add_norm_shift(const float* x, float* x_out, int delta_kind, const void* y, const float* y_bias,
                                const void* g, const float* g_bias, const float* post_w, float post_eps, int do_norm,
                                const float* w, float eps, void* h_out, const float* shift_w, void* hs_out,
                                float* state, const int* positions, const int* token_segment, const int* cu_seqlens,
-                               const int* state_slots, const int* state_phase, int is_bf16, int N, int D,
-                               int rows_per_block, hipStream_t s) {
+                               const int* state_slots, const int* state_phase, int is_bf16, int N, int D, float* stats,
+                               hipStream_t s) {
   if (N <= 0) return 0;
-  if (D <= 0 || rows_per_block < 1 || delta_kind < 0 || delta_kind > 2) return JLE_BAD_ARG;
+  if (D <= 0 || delta_kind < 0 || delta_kind > 2) return JLE_BAD_ARG;
   if (delta_kind != 0 && (y == nullptr || x_out == nullptr)) return JLE_BAD_ARG;
   if (delta_kind == 2 && g == nullptr) return JLE_BAD_ARG;
   if (shift_w != nullptr && (!do_norm || hs_out == nullptr || state == nullptr || positions == nullptr ||
                              token_segment == nullptr || cu_seqlens == nullptr || state_slots == nullptr ||
                              state_phase == nullptr))
     return JLE_BAD_ARG;
+  if (stats != nullptr && shift_w == nullptr) return JLE_BAD_ARG;
   SandwichArgs a{x, x_out, delta_kind, y, y_bias, g, g_bias, post_w, post_eps, do_norm, w, eps, h_out, shift_w,
-                 hs_out, state, positions, token_segment, cu_seqlens, state_slots, state_phase, N, D,
-                 shift_w != nullptr ? rows_per_block : 1};
-  auto aligned = [](const void* p) { return p == nullptr || ((uintptr_t)p % 16) == 0; };
-  const bool vec = D % 4 == 0 && aligned(x) && aligned(x_out) && aligned(y) && aligned(g) && aligned(h_out) &&
-                   aligned(hs_out) && aligned(state) && D <= kThreads * 8 * 4;
+                 hs_out, state, positions, token_segment, cu_seqlens, state_slots, state_phase, stats, N, D};
+  uintptr_t all = 0;
+  for (const void* p : {(const void*)x, (const void*)x_out, y, (const void*)y_bias, g, (const void*)g_bias, (const void*)post_w,
+                        (const void*)w, (const void*)h_out, (const void*)shift_w, (const void*)hs_out, (const void*)state})
+    all |= (uintptr_t)p;
+  const int vec = all % 16 ? 1 : D % 8 == 0 && D <= 1024 * 8 ? 8 : D % 4 == 0 && D <= 1024 * 4 ? 4 : 1;
   int rc;
   if (is_bf16)
-    rc = vec ? launch_sandwich<bf16_t, 4>(a, s) : launch_sandwich<bf16_t, 1>(a, s);
+    rc = vec == 8 ? launch_sandwich<bf16_t, 8>(a, s) : vec == 4 ? launch_sandwich<bf16_t, 4>(a, s) : launch_sandwich<bf16_t, 1>(a, s);
   else
-    rc = vec ? launch_sandwich<float, 4>(a, s) : launch_sandwich<float, 1>(a, s);
+    rc = vec == 8 ? launch_sandwich<float, 8>(a, s) : vec == 4 ? launch_sandwich<float, 4>(a, s) : launch_sandwich<float, 1>(a, s);
   if (rc != 0) return rc;
   JLE_LAUNCH_CHECK();
   return 0;
@@ -355,7 +444,8 @@ JLE_API int jle_polynorm(const void* z, int ldz, const float* bias, const float*
                          int is_bf16, int N, int F, hipStream_t s) {
   if (N <= 0) return 0;
   if (F <= 0 || ldz < F || coef == nullptr) return JLE_BAD_ARG;
-  const bool vec = F % 4 == 0 && ldz % 4 == 0 && (uintptr_t)z % 16 == 0 && (uintptr_t)out % 16 == 0;
+  const bool aligned = ((uintptr_t)z | (uintptr_t)out | (uintptr_t)bias) % 16 == 0;
+  const int vec = !aligned ? 1 : F % 8 == 0 && ldz % 8 == 0 ? 8 : F % 4 == 0 && ldz % 4 == 0 ? 4 : 1;
   if (is_bf16)
     launch_polynorm<bf16_t>((const bf16_t*)z, ldz, bias, coef, eps, (bf16_t*)out, N, F, vec, s);
   else

@@ -61,7 +61,7 @@ _SIGNATURES = {
     "jle_gemm_skinny": [_vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _i, _i, _vp, _i, _i, _i, _i, _vp, _vp,
                         _vp],
     "jle_add_norm_shift": [_vp, _vp, _i, _vp, _vp, _vp, _vp, _vp, _f, _i, _vp, _f, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp,
-                           _vp, _i, _i, _i, _i, _vp],
+                           _vp, _i, _i, _i, _vp, _vp],
     "jle_polynorm": [_vp, _i, _vp, _vp, _f, _vp, _i, _i, _i, _vp],
     "jle_latent_prepare": [_vp, _i, _i, _i, _i, _i, _vp, _vp, _i, _i, _f, _vp, _f, _vp, _vp, _vp, _i, _vp, _i, _i, _i,
                            _vp],
@@ -438,8 +438,8 @@ class HipOps:
                    _p(h_a), _p(h_b), 1 if out_dtype == torch.bfloat16 else 0, n, d)
         return h_a, h_b
 
-    SHIFT_ROWS_PER_BLOCK = 4  # a block of the norm-and-shift kernel takes so many rows in a step of many tokens
-    # (it forms the row before its first anew: with one row a block every row is formed twice)
+    SHIFT_APART_ROWS = 256  # from so many rows on (a row a compute unit) the shift is a kernel of its own behind sums and
+    # statistics: with one kernel every row is formed twice (see sandwich.hip)
 
     def add_norm_shift(self, x, delta, weight, eps: float, out_dtype, shift, ctx, do_norm: bool = True):
         """``x' = x + delta`` into a new tensor (``delta``: ``None``, a tensor, or a gated branch
@@ -465,14 +465,14 @@ class HipOps:
             self._chk(weight, torch.float32, (d,), "norm weight")
         x_out = torch.empty_like(x) if kind else None
         h = torch.empty(n, d, dtype=out_dtype, device=x.device) if do_norm else None
-        hs = sw = state = None
-        rows = 1
+        hs = sw = state = stats = None
         if shift is not None:
             sw, state = shift
             self._chk(sw, torch.float32, (d,), "shift weight")
             self._chk(state, torch.float32, (state.shape[0], 2, d), "shift state")
             hs = torch.empty(n, d, dtype=out_dtype, device=x.device)
-            rows = self.SHIFT_ROWS_PER_BLOCK if n >= self._compute_units * self.SHIFT_ROWS_PER_BLOCK else 1
+            if n >= self.SHIFT_APART_ROWS:
+                stats = torch.empty(n, dtype=torch.float32, device=x.device)
         is_bf16 = 1 if out_dtype == torch.bfloat16 else 0
         self._call("jle_add_norm_shift", _p(x), _p(x_out), kind, _p(y), _p(yb), _p(g), _p(gb), _p(pw), float(peps),
                    int(do_norm), _p(weight), float(eps), _p(h), _p(sw), _p(hs), _p(state),
@@ -480,7 +480,7 @@ class HipOps:
                    _p(ctx.token_segment) if shift is not None else None,
                    _p(ctx.cu_seqlens) if shift is not None else None,
                    _p(ctx.state_slots) if shift is not None else None,
-                   _p(ctx.state_phase) if shift is not None else None, is_bf16, n, d, rows)
+                   _p(ctx.state_phase) if shift is not None else None, is_bf16, n, d, _p(stats))
         return (x_out if kind else x), h, hs
 
     def polynorm(self, z, bias, coef, eps: float):

@@ -1085,6 +1085,32 @@ def test_weight_streaming_product_of_fuller_groups(ops, counts, nout, k, tiled):
         o += c
 
 
+@pytest.mark.parametrize("dt", DT)
+@pytest.mark.parametrize("d", [48, 50, 2048, 4104, 8192])
+def test_shift_apart_from_its_norm(ops, dt, d):
+    """With many rows the shift is a kernel of its own behind the sums: the bits of the kernel that does both, at segments
+    that begin and end within, at and across its blocks, with and without a branch output."""
+    import types
+    from jax_llm_examples_amd.parts.residual import GatedBranch
+    lens, starts = [1, 7, 8, 30, 3, 17], [5, 0, 3, 0, 0, 9]
+    n, cu = sum(lens), torch.tensor([0] + lens).cumsum(0)
+    i32 = lambda v: torch.as_tensor(v, dtype=torch.int32).to(DEV)
+    ctx = types.SimpleNamespace(positions=i32([s + t for s, k in zip(starts, lens) for t in range(k)]),
+                                token_segment=i32([i for i, k in enumerate(lens) for _ in range(k)]), cu_seqlens=i32(cu),
+                                state_slots=i32([3, 0, 5, 1, 2, 4]), state_phase=i32([0, 1, 1, 0, 0, 1]))
+    x, y, g = _rand(n, d, seed=1), _rand(n, d, dt=dt, seed=2), _rand(n, d, dt=dt, seed=3)
+    v = [_rand(d, seed=4 + i) for i in range(5)]
+    for delta in (None, y, GatedBranch(y, v[0], g, v[1], v[2], 1e-3)):
+        got = []
+        for apart in (1 << 30, 1):
+            ops.SHIFT_APART_ROWS = apart
+            state = _rand(6, 2, d, seed=9)
+            got.append((*ops.add_norm_shift(x.clone(), delta, v[3], 1e-5, dt, (v[4], state), ctx), state))
+        del ops.SHIFT_APART_ROWS
+        for a, b, what in zip(*got, ("sums", "normed rows", "shifted rows", "state")):
+            assert torch.equal(a, b), (what, float((a - b).abs().max()))
+
+
 @pytest.mark.parametrize("n,d,f,e,k", [(300, 128, 48, 16, 1), (700, 264, 72, 3, 2), (2048, 512, 256, 16, 1),
                                        (150, 64, 40, 128, 1)])
 def test_grouped_product_for_many_rows(ops, ref, n, d, f, e, k):
