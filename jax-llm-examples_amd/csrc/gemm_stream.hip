@@ -228,6 +228,221 @@ __global__ __launch_bounds__(WAVES * 64, 2) void gemm_stream_kernel(const bf16_t
 #undef GO
 }
 
+// ------------------------------------------------------------------ groups of many rows
+// A block of four wavefronts, one a SIMD, takes 256 rows of W (SWIGLU: 128 gate rows and their up rows) and up to 256 rows
+// of a group; a wavefront 64 of those rows of W, four tiles, and all the rows of X: 4 x NT tiles of accumulators.  Its
+// weights go from memory straight into the A operand (no other wavefront of the block wants them), four stages of 64 k in
+// registers; X comes through shared memory, brought by the load unit itself (a kilobyte an instruction in the lanes' order,
+// the rows' 16-byte pieces swizzled by which piece a lane fetches) into a ring of three stages.  A byte read from shared
+// memory serves 64 operations.  With one wavefront a SIMD nothing hides a wait, so there is none: a B operand is asked for
+// four products of tiles before its use, the barrier that says that the next stage's rows have come (and that the ring's
+// oldest place is free) stands in the middle of a stage, and the next stage's first operands are read at this one's end.
+// 16 groups of 16,384 x 5,120 (gate and up) with 410 rows each: 1,023 us (1.08 PFLOP/s) against 1,508 in passes of 192; 8 of
+// 4,096 x 7,168 163 (1.18) against 275.  (With eight wavefronts of 64 x half the rows and the weights through shared memory
+// too 422 and 188 at 8 groups: reading and bringing in together took shared memory as long as the products.)
+// Work items: a group's rows in tiles of at most 256, as even as multiples of 32 allow; item = ((row block / 8) * tiles +
+// tile) * 8 + row block % 8 within a group, so that the tiles that read the same weights run on one chiplet.
+constexpr int kWideRows = 256;
+constexpr int kWideStage = kWideRows * BK * 2, kWideLds = 3 * kWideStage;  // bytes of a stage's rows, and of the ring
+
+__device__ __forceinline__ void load_to_lds16(const void* base, uint32_t byte_off, uint32_t lds_addr) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1\n" ::"v"(byte_off), "s"(base), "s"(lds_addr) : "memory");
+}
+
+template <bool SWIGLU, int NT>
+__device__ __forceinline__ void wide_block(const bf16_t* __restrict__ X, const bf16_t* __restrict__ We,
+                                           bf16_t* __restrict__ Y, const int* __restrict__ a_rows,
+                                           const float* __restrict__ scale, unsigned char* smem, int tok0, int live, int K,
+                                           int Nout, int nb) {
+  static_assert(NT % 2 == 0 && NT >= 4, "a wavefront brings NT / 2 kilobytes of a stage's rows");
+  constexpr int PF = 4;  // operands asked for ahead
+  const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+  const int wave = wave_index();
+  const uint32_t lds0 = (uint32_t)(uintptr_t)smem;
+  const int half = Nout >> 1, ntile = (SWIGLU ? half : Nout) >> 4;
+  const int nstage = K / BK;  // a multiple of 4
+  // this wavefront's tiles of W (SWIGLU: two of the gate, two of up); those behind the end: the last one, not stored
+  const bf16_t* w_src[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int tile = SWIGLU ? min(nb * 8 + wave * 2 + (i & 1), ntile - 1) + (i >= 2 ? half >> 4 : 0)
+                            : min(nb * 16 + wave * 4 + i, ntile - 1);
+    w_src[i] = We + (size_t)tile * 16 * K + lane * 8;
+  }
+  uint32_t x_src[NT / 2];
+#pragma unroll
+  for (int i = 0; i < NT / 2; ++i) {
+    const int t = tok0 + min(8 * (wave + 4 * i) + (lane >> 3), live - 1);
+    x_src[i] = (uint32_t)(a_rows != nullptr ? a_rows[t] : t) * (uint32_t)(K * 2) + (uint32_t)(((lane & 7) ^ (lane >> 3)) * 16);
+  }
+  auto ask_rows = [&](int s, uint32_t place) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < NT / 2; ++i)
+      load_to_lds16(X + (size_t)s * BK, x_src[i], lds0 + place + (uint32_t)((wave + 4 * i) * 1024));
+  };
+  auto ask_weights = [&](u32x4 (&w)[2][4], int s) __attribute__((always_inline)) {
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) w[ks][i] = *reinterpret_cast<const u32x4*>(w_src[i] + (size_t)(2 * s + ks) * 512);
+  };
+  const uint32_t b_rd = (uint32_t)(r * 128 + ((g ^ (r & 7)) * 16));  // (k step 1: bit 6 the other way)
+  auto operand = [&](uint32_t place, int j) __attribute__((always_inline)) {
+    return *reinterpret_cast<const bf16x8*>(smem + place + (b_rd ^ (j >= NT ? 64 : 0)) + (j % NT) * 2048);
+  };
+  f32x4 acc[4][NT];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int n = 0; n < NT; ++n) acc[i][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+  u32x4 wa[2][4], wb[2][4], wc[2][4], wd[2][4];
+  bf16x8 ahead[PF];
+  uint32_t here = 0, next = kWideStage, free_ = 2 * kWideStage;  // the ring: this stage's rows, the next one's, the one after
+
+  // rows_next: how many of the loads on their way are younger than the next stage's rows (-1: there is no next stage)
+#define WIDE_STAGE(w_, s_, rows_next, ASKX, ASKW)                                                       \
+  do {                                                                                                  \
+    bf16x8 b_[2 * NT + PF];                                                                             \
+    _Pragma("unroll") for (int p = 0; p < PF; ++p) b_[p] = ahead[p];                                    \
+    _Pragma("unroll") for (int j = 0; j < 2 * NT; ++j) {                                                \
+      if (j == NT && rows_next >= 0) {                                                                  \
+        if (rows_next > 0) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");                             \
+        else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                                           \
+        __syncthreads();                                                                                \
+        if (ASKX) ask_rows((s_) + 2, free_);                                                            \
+      }                                                                                                 \
+      if (j + PF < 2 * NT) b_[j + PF] = operand(here, j + PF);                                          \
+      else if (rows_next >= 0) b_[j + PF] = operand(next, j + PF - 2 * NT);                             \
+      _Pragma("unroll") for (int i = 0; i < 4; ++i) {                                                   \
+        acc[i][j % NT] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, w_[j / NT][i]), b_[j], \
+                                                                 acc[i][j % NT], 0, 0, 0);              \
+      }                                                                                                 \
+      __builtin_amdgcn_sched_barrier(0);                                                                \
+    }                                                                                                   \
+    if (rows_next >= 0) {                                                                               \
+      _Pragma("unroll") for (int p = 0; p < PF; ++p) ahead[p] = b_[2 * NT + p];                         \
+    }                                                                                                   \
+    if (ASKW) ask_weights(w_, (s_) + WAHEAD);                                                           \
+    const uint32_t t_ = here;                                                                           \
+    here = next;                                                                                        \
+    next = free_;                                                                                       \
+    free_ = t_;                                                                                         \
+  } while (0)
+
+  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the rows' numbers have come; from here on only the stages' loads count
+  asm volatile("" ::: "memory");
+  ask_rows(0, 0);
+  ask_rows(1, kWideStage);
+  ask_weights(wa, 0);
+  ask_weights(wb, 1);
+  ask_weights(wc, 2);
+  ask_weights(wd, 3);
+  asm volatile("s_waitcnt vmcnt(24)" ::: "memory");
+  __syncthreads();
+#pragma unroll
+  for (int p = 0; p < PF; ++p) ahead[p] = operand(0, p);
+  int s = 0;
+  for (; s < nstage - WAHEAD; s += WAHEAD) {
+    WIDE_STAGE(wa, s, 8, true, true);
+    WIDE_STAGE(wb, s + 1, 8, true, true);
+    WIDE_STAGE(wc, s + 2, 8, true, true);
+    WIDE_STAGE(wd, s + 3, 8, true, true);
+  }
+  WIDE_STAGE(wa, s, 8, true, false);
+  WIDE_STAGE(wb, s + 1, 0, true, false);
+  WIDE_STAGE(wc, s + 2, 0, false, false);
+  WIDE_STAGE(wd, s + 3, -1, false, false);
+#undef WIDE_STAGE
+#pragma unroll
+  for (int n = 0; n < NT; ++n) {
+    const int row = n * 16 + r;
+    if (row >= live) continue;
+    const int t = tok0 + row;
+    const float sc = scale != nullptr ? scale[t] : 1.f;
+#pragma unroll
+    for (int i = 0; i < (SWIGLU ? 2 : 4); ++i) {
+      const int tile = SWIGLU ? nb * 8 + wave * 2 + i : nb * 16 + wave * 4 + i;
+      if (tile >= ntile) continue;
+      float y[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        if (SWIGLU) {
+          const float gate = acc[i][n][e] * sc, up = acc[i + 2][n][e] * sc;
+          y[e] = gate / (1.0f + expf(-gate)) * up;
+        } else {
+          y[e] = acc[i][n][e] * sc;
+        }
+      }
+      store4<bf16_t>(Y + (size_t)t * (SWIGLU ? half : Nout) + tile * 16 + 4 * g, y[0], y[1], y[2], y[3]);
+    }
+  }
+}
+
+template <bool SWIGLU>
+__global__ __launch_bounds__(256, 1) void wide_kernel(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W,
+                                                      bf16_t* __restrict__ Y, const int* __restrict__ offsets,
+                                                      const int* __restrict__ a_rows, const float* __restrict__ scale,
+                                                      int Nout, int K, int G, int nblk8) {
+  extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
+  // this block's group: 64 groups a look, the items before each by a sum over the lanes
+  const int lane = threadIdx.x & 63;
+  int left = blockIdx.x, e = -1, tiles = 0;
+  for (int g0 = 0; g0 < G && e < 0; g0 += 64) {
+    const int gi = g0 + lane;
+    const int rows = gi < G ? offsets[gi + 1] - offsets[gi] : 0;
+    const int mine = (rows + kWideRows - 1) / kWideRows;
+    int upto = mine * nblk8;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int v = __shfl_up(upto, o, 64);
+      if (lane >= o) upto += v;
+    }
+    const unsigned long long mask = __ballot(left < upto);
+    if (mask != 0) {
+      const int at = __ffsll((long long)mask) - 1;
+      e = g0 + at;
+      tiles = __shfl(mine, at, 64);
+      left -= __shfl(upto, at, 64) - tiles * nblk8;
+    } else {
+      left -= __shfl(upto, 63, 64);
+    }
+  }
+  if (e < 0) return;  // (the grid is laid out for the most tiles that so many rows can make)
+  e = __builtin_amdgcn_readfirstlane(e);
+  left = __builtin_amdgcn_readfirstlane(left);
+  tiles = __builtin_amdgcn_readfirstlane(tiles);
+  const int nb = left / (8 * tiles) * 8 + (left & 7), tile = (left >> 3) % tiles;
+  if (nb * (SWIGLU ? 128 : 256) >= (SWIGLU ? Nout / 2 : Nout)) return;
+  const int lo = offsets[e], rows = offsets[e + 1] - lo;
+  const int per = ((rows + tiles - 1) / tiles + 31) / 32 * 32;
+  const int tok0 = lo + tile * per, live = min(per, rows - tile * per);
+  if (live <= 0) return;
+  const bf16_t* We = W + (size_t)e * Nout * K;
+#define GO(NT_) wide_block<SWIGLU, NT_>(X, We, Y, a_rows, scale, smem, tok0, live, K, Nout, nb)
+  if (live <= 64) GO(4);
+  else if (live <= 128) GO(8);
+  else if (live <= 160) GO(10);
+  else if (live <= 192) GO(12);
+  else if (live <= 224) GO(14);
+  else GO(16);
+#undef GO
+}
+
+template <bool SW>
+int launch_wide(hipStream_t s, const void* X, const void* W, void* Y, const int* offsets, const int* a_rows,
+                const float* scale, int M, int Nout, int K, int G) {
+  static const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&wide_kernel<SW>),
+                                                  hipFuncAttributeMaxDynamicSharedMemorySize, kWideLds);
+  if (e != hipSuccess) return (int)e;
+  const int nblk8 = ((SW ? Nout / 2 : Nout) + (SW ? 1024 : 2048) - 1) / (SW ? 1024 : 2048) * 8;
+  const long long items = ((long long)M / kWideRows + G) * nblk8;
+  if (items > (1ll << 30)) return JLE_BAD_ARG;
+  hipLaunchKernelGGL(wide_kernel<SW>, dim3((unsigned)items), dim3(256), kWideLds, s, (const bf16_t*)X, (const bf16_t*)W,
+                     (bf16_t*)Y, offsets, a_rows, scale, Nout, K, G, nblk8);
+  JLE_LAUNCH_CHECK();
+  return 0;
+}
+
 template <bool SW, typename OT, int WV>
 void launch_stream(int nblk, int passes, int G, hipStream_t s, const void* X, const void* W, void* Y,
                    const int* offsets, const int* a_rows, const float* scale, int M, int Nout, int K) {
@@ -245,13 +460,20 @@ JLE_API int jle_gemm_stream_supported(int Nout, int K, int swiglu) {
 }
 
 // X [*, K] bf16, W [G, Nout, K] bf16 in the streaming layout, Y [M, Nout] (or [M, Nout / 2] with swiglu) bf16 or
-// float32; X must have fewer than 2^32 elements.  max_rows: the most rows any group can have (M if unknown).
+// float32; X must have fewer than 2^32 elements (wide: 2^32 bytes).  wide: wide_kernel (groups, bfloat16 out).  max_rows: the most rows any group can have (M if unknown).
 // Blocks are 8 wavefronts (two per SIMD, one block per compute unit): measured against 4, 5 and 6 on expert
 // shapes with even and with skewed numbers of rows per expert.
 JLE_API int jle_gemm_stream(const void* X, const void* W, void* Y, const int* offsets, const int* a_rows,
                             const float* scale, int swiglu, int out_f32, int M, int Nout, int K, int G, int max_rows,
-                            hipStream_t s) {
+                            int wide, hipStream_t s) {
   if (M <= 0 || Nout <= 0) return 0;
+  if (wide) {
+    if (offsets == nullptr || out_f32 || G < 1 || G > 65535 || !jle_gemm_stream_supported(Nout, K, swiglu) ||
+        ((uintptr_t)X | (uintptr_t)W | (uintptr_t)Y) % 16)
+      return JLE_BAD_ARG;
+    return swiglu ? launch_wide<true>(s, X, W, Y, offsets, a_rows, scale, M, Nout, K, G)
+                  : launch_wide<false>(s, X, W, Y, offsets, a_rows, scale, M, Nout, K, G);
+  }
   if (G < 1 || G > 65535 || !jle_gemm_stream_supported(Nout, K, swiglu)) return JLE_BAD_ARG;
   if (max_rows <= 0 || max_rows > M) max_rows = M;
   constexpr int kWaves = 8;

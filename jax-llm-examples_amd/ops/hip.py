@@ -7,6 +7,7 @@ fallback: if the library cannot be built or loaded, constructing :class:`HipOps`
 from __future__ import annotations
 
 import ctypes
+import functools
 from typing import Optional
 
 import torch
@@ -80,7 +81,7 @@ _SIGNATURES = {
     "jle_conv_rows": [_vp, _i, _i, _vp, _vp, _vp, _i, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _vp],
     "jle_conv_qk_prepare": [_vp, _i, _vp, _vp, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _f, _f, _vp, _vp, _i, _i,
                             _i, _i, _i, _i, _i, _i, _i, _vp],
-    "jle_gemm_stream": [_vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _vp],
+    "jle_gemm_stream": [_vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _i, _vp],
     "jle_streams_mix_norm": [_vp, _i, _vp, _vp, _vp, _i, _vp, _i, _vp, _vp, _vp, _vp, _f, _vp, _i, _vp, _i, _i, _i, _i,
                              _vp],
     "jle_embed_sinusoid": [_vp, _vp, _vp, _i, _f, _vp, _vp, _i, _i, _i, _vp],
@@ -1528,6 +1529,31 @@ class HipOps:
     def stream_supported(self, nout: int, k: int, swiglu: bool) -> bool:
         return bool(self._query("jle_gemm_stream_supported", nout, k, int(swiglu)))
 
+    WIDE_GROUP_ROWS = 176  # fewer rows a group on average: the weights' bytes take the time, each read once
+
+    @staticmethod
+    @functools.lru_cache(maxsize=4096)
+    def stream_wide(rows: int, groups: int, row_blocks: int) -> bool:
+        """Which of ``gemm_stream.hip``'s kernels takes ``rows`` rows in ``groups`` groups (``row_blocks`` blocks of 256 rows
+        of W a group): passes of 192 rows or wide tiles of 256.  A block fills a compute unit, so what counts is how many
+        rounds of blocks there are and how long one takes; measured per stage of 64 k, microseconds: passes 0.9 + 0.0037 a
+        row, tiles 0.95 + 0.003.  A group's rows scatter about their mean by its root.  Both sides measured (passes | tiles,
+        us): 8 groups of 14,336 x 4,096 gate and up with 192 rows each 286 | 226, 256 368 | 309, 410 529 | 401, 700
+        743 | 643; of 4,096 x 7,168 with 192 152 | 154, 410 275 | 163, 512 281 | 298, 700 302 | 329; of 8,192 x 2,048 gate
+        and up with 410 152 | 121, 512 152 | 167; 16 of 16,384 x 5,120 with 160 523 | 541, 410 1,508 | 1,023, 700
+        1,920 | 1,709."""
+        mean = rows / groups
+        if mean < HipOps.WIDE_GROUP_ROWS:
+            return False
+
+        def cost(most, start, a_row):
+            tiles = sum(-(-max(1.0, mean + d * mean ** 0.5) // most) for d in (-1, 0, 1)) / 3
+            blocks = row_blocks * groups * tiles
+            rounds = -(-blocks // 256) if blocks < 1024 else blocks / 256 + 0.5
+            return rounds * (start + a_row * mean / tiles)
+
+        return cost(256, 0.95, 0.003) < cost(192, 0.9, 0.0037)
+
     def gemm_stream(self, a, b, *, offsets=None, a_rows=None, scale=None, swiglu=False, out_f32=False, rows=None):
         """bfloat16 product on MFMA for about a hundred rows per group, weights in the streaming layout and
         read once per 192 rows of a group (see ``gemm_stream.hip``)."""
@@ -1546,8 +1572,10 @@ class HipOps:
                               f"whole tiles of 16 weight rows (32 with the fused activation), got {nout} x {k}")
         out = torch.empty(m, nout // 2 if swiglu else nout, dtype=torch.float32 if out_f32 else torch.bfloat16,
                           device=a.device)
+        wide = (offsets is not None and not out_f32 and a.numel() < 2 ** 31
+                and self.stream_wide(m, g, -(-nout // 256)))
         self._call("jle_gemm_stream", _p(a), _p(b), _p(out), _p(offsets), _p(a_rows), _p(scale), int(swiglu),
-                   int(out_f32), m, nout, k, g, m)
+                   int(out_f32), m, nout, k, g, m, int(wide))
         return out
 
     def lm_head(self, h, w, tiled: bool = False):

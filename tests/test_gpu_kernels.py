@@ -1085,6 +1085,30 @@ def test_weight_streaming_product_of_fuller_groups(ops, counts, nout, k, tiled):
         o += c
 
 
+@pytest.mark.parametrize("counts,nout,k,swiglu", [
+    ([1, 0, 31, 32, 33, 64, 65], 96, 256, False),           # few rows, whole rounds of stages only at the end
+    ([128, 129, 160, 161, 192, 193], 528, 512, False),      # every number of row tiles; a second block of W of one tile
+    ([224, 225, 256, 257, 512, 513, 700], 544, 768, True),  # one, two and three tiles of rows; gate and up
+    ([3, 0, 280] * 50, 64, 256, False),                     # more groups than a look takes
+    ([256], 2304, 256, True)])                              # more than eight blocks of W
+def test_wide_tiles_of_the_weight_streaming_product(ops, counts, nout, k, swiglu):
+    """The kernel for many rows a group gives the bits of the one that takes them in passes (the same sums in the same
+    order), with the rows gathered and scaled; that one is tested against the general product elsewhere."""
+    from jax_llm_examples_amd.ops.layout import tile_
+    m, e = sum(counts), len(counts)
+    x, w = _rand(m + 3, k, dt=torch.bfloat16, seed=1), _rand(e, nout, k, dt=torch.bfloat16, scale=0.1, seed=2)
+    tile_(w)
+    off = torch.tensor([0] + counts).cumsum(0).int().to(DEV)
+    rows = torch.randperm(m + 3, generator=torch.Generator().manual_seed(3))[:m].int().to(DEV)
+    scale = _rand(m, seed=4)
+    got = []
+    for wide in (False, True):
+        ops.stream_wide = lambda *a, wide=wide: wide
+        got.append(ops.gemm_stream(x, w, offsets=off, a_rows=rows, scale=scale, swiglu=swiglu, rows=m))
+    del ops.stream_wide
+    assert torch.equal(*got)
+
+
 @pytest.mark.parametrize("dt", DT)
 @pytest.mark.parametrize("d", [48, 50, 2048, 4104, 8192])
 def test_shift_apart_from_its_norm(ops, dt, d):
