@@ -1,5 +1,6 @@
 // Embedding gather, residual add + RMS norm, SiLU*up, row gather, expert output combine.
 #include "common.h"
+#include "gate_act.h"
 #include "rows.h"
 
 using namespace jle;
@@ -277,14 +278,7 @@ JLE_API int jle_gather_rows(const void* src, const int* idx, void* out, int M, i
 }
 
 // ------------------------------------------------------------------ act(gate) * up
-// in: [N, 2F] (gate columns, then up columns); out: [N, F].  ACT 0: silu, z / (1 + exp(-z)); 1: the tanh form of
-// gelu, 0.5 z (1 + tanh(sqrt(2 / pi) (z + 0.044715 z^3))).
-template <int ACT>
-__device__ __forceinline__ float gate_act(float g) {
-  if (ACT == 1) return 0.5f * g * (1.0f + tanhf(0.7978845608028654f * (g + 0.044715f * g * g * g)));
-  return g / (1.0f + expf(-g));
-}
-
+// in: [N, 2F] (gate columns, then up columns); out: [N, F].
 template <typename T, int ACT>
 __global__ void silu_mul_kernel(const T* __restrict__ in, T* __restrict__ out, int F) {
   const size_t row = blockIdx.y;

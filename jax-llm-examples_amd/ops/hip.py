@@ -49,6 +49,8 @@ _SIGNATURES = {
     "jle_moe_route_align": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _vp],
     "jle_gemm_generic": [_vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _vp],
     "jle_gemm_f32_skinny": [_vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _vp],
+    "jle_gemm_f32_rows": [_vp, _vp, _vp, _i, _i, _i, _i, _vp],
+    "jle_gemm_f32_split": [_vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _vp],
     "jle_gemm_f32_stream": [_vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _vp],
     "jle_sample": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _vp],
     "jle_attention_mfma_supported": [_i, _i, _i, _i],
@@ -973,10 +975,34 @@ class HipOps:
         return out
 
     # ------------------------------------------------------------------ matrix products
+    def _dense_float32(self, h, w, act: int = -1):
+        """The float32 products with kernels of their own (see ``gemm_f32_dense.hip``), or None: the library's.
+
+        Up to 4 rows the product is a stream of the weights, which the kernel reads at 6.0 to 6.7 TB/s where the
+        library's reads them at 4.0 to 5.2 (16384 x 2048 33 -> 21 us, 2048 x 8192 23 -> 13, 2048 x 2048 11.5 -> 5.3, 64 x
+        36 5.6 -> 2.5); up to 8 rows while the weights are no more than 2^25 numbers (33 -> 29.5 us there; 14336 x 4096 at
+        8 rows is 50 us against the library's 45).  Many rows: see :meth:`split_ranges`.  In between neither gains."""
+        if h.dtype != torch.float32 or w.dtype != torch.float32 or h.dim() != 2 or w.dim() != 2:
+            return None
+        rows, k = h.shape
+        n = w.shape[0]
+        if (rows == 0 or w.shape[1] != k or k % 4 or not (h.is_cuda and w.is_cuda and h.is_contiguous() and w.is_contiguous())
+                or h.data_ptr() % 16 or w.data_ptr() % 16 or n % (2 if act >= 0 else 1) or n == 0 or k == 0):
+            return None
+        if rows <= 4 or (rows <= 8 and n * k <= 1 << 25):
+            return self.gemm_f32_rows(h, w, act)
+        ranges = self.split_ranges(rows, n, k, act >= 0, self._compute_units)
+        if ranges:
+            return self.gemm_f32_split(h, w, act, ranges)
+        return None
+
     def linear(self, h, w, out_dtype=None):
-        """``h @ w.T``: through the BLAS library (float32: true float32); a few bfloat16 rows through the
-        weight-streaming kernel, which is as fast there or faster and much cheaper to launch."""
+        """``h @ w.T``: through the BLAS library; a few bfloat16 rows through the weight-streaming kernel, which is as
+        fast there or faster and much cheaper to launch, and few or many float32 rows through kernels of their own."""
         h = self._rows(h)
+        out = self._dense_float32(h, w)
+        if out is not None:
+            return out if out_dtype is None or out_dtype == out.dtype else out.to(out_dtype)
         if (h.dtype == torch.bfloat16 and h.shape[0] <= self.SKINNY_LINEAR_ROWS and w.dim() == 2
                 and w.dtype == torch.bfloat16 and w.shape[1] % 8 == 0 and h.is_contiguous() and w.is_contiguous()):
             out = self.gemm_skinny(h, w)
@@ -1013,7 +1039,8 @@ class HipOps:
         act = self._ACTS[activation]
         if h.dtype == torch.bfloat16 and h.shape[0] <= self.SKINNY_DENSE_ROWS and h.shape[1] % 8 == 0:
             return self.gemm_skinny(h, w_gate_up, swiglu=1 + act)  # (the activation in the product's epilogue)
-        return self.silu_mul(torch.matmul(h, w_gate_up.t()), activation)
+        out = self._dense_float32(h, w_gate_up, act)
+        return self.silu_mul(torch.matmul(h, w_gate_up.t()), activation) if out is None else out
 
     def sigmoid_mul(self, o, gate):
         """``o * sigmoid(gate)``; ``gate`` may be a slice of wider rows (its last axis contiguous), and narrower than ``o``:
@@ -1413,6 +1440,53 @@ class HipOps:
                    nout, k, g, m, slots)
         return out
 
+    @staticmethod
+    @functools.lru_cache(maxsize=4096)
+    def split_ranges(rows: int, nout: int, k: int, gated: bool, cus: int) -> int:
+        """How many ranges of k the kernel of operands in parts shares a product out over, or 0: the library's is faster.
+
+        A compute unit runs two blocks (tiles of 128 x 128) together; measured, a stage of 32 k takes 1.75 us of one block
+        alone and 2.75 of two, a launch 6 us beside, the ranges' sums 4 and their bytes.  The library reaches 75 to 150
+        TFLOP/s here, taken as 115 (its tiles fit some sizes better than others), and a pass of its own for the gate.
+        Both sides measured, library | parts, us: 777 rows of 16,384 x 2,048 470 | 354, 1,554 802 | 619, 4,096 of 4,096 x
+        2,048 474 | 369, 256 of 7,168 x 5,120 171 | 138, 777 of 5,120 x 5,120 328 | 294, 1,554 of 2,048 x 8,192 462 | 349;
+        left to the library: 140 of 16,384 x 2,048 96 | 112, 256 of 2,048 x 2,048 24 | 32, 64 of 7,168 x 5,120 50 | 66."""
+        if rows < 96 or k % 32 or nout % 8:
+            return 0
+        tiles, stages = -(-rows // 128) * -(-nout // 128), k // 32
+
+        def cost(ranges):
+            blocks = -(-tiles * ranges // cus)
+            sums = 4 + (2 * ranges + 1) * rows * nout * 4 / 5e6 if ranges > 1 else 0
+            return (blocks // 2 * 2.75 + blocks % 2 * 1.75) * -(-stages // ranges) + 6 + sums
+
+        best = min(range(1, 2 if gated else max(1, min(8, stages // 4)) + 1), key=cost)
+        library = 2 * rows * nout * k / 115e6 + 6 + (3 + rows * nout * 6 / 5e6 if gated else 0)
+        return best if cost(best) < library else 0
+
+    def gemm_f32_split(self, a, b, act: int = -1, ranges: int = 1):
+        """The dense float32 product for many rows: every operand as three bfloat16 numbers (see
+        ``gemm_f32_dense.hip``).  ``act``: -1 none, 0 silu, 1 gelu (tanh form) of the first half of ``b``'s rows times
+        the second; ``ranges``: of k, added up by blocks of their own (without ``act``)."""
+        nout, k = b.shape
+        m = a.shape[0]
+        self._chk(a, torch.float32, (m, k), "A")
+        self._chk(b, torch.float32, None, "B")
+        out = torch.empty(m, nout // 2 if act >= 0 else nout, dtype=torch.float32, device=a.device)
+        parts = torch.empty(ranges, m, nout, dtype=torch.float32, device=a.device) if ranges > 1 else None
+        self._call("jle_gemm_f32_split", _p(a), _p(b), _p(out), _p(parts), act, m, nout, k, ranges)
+        return out
+
+    def gemm_f32_rows(self, a, b, act: int = -1):
+        """The dense float32 product for up to eight rows: reads the weights once (see ``gemm_f32_dense.hip``)."""
+        nout, k = b.shape
+        m = a.shape[0]
+        self._chk(a, torch.float32, (m, k), "A")
+        self._chk(b, torch.float32, None, "B")
+        out = torch.empty(m, nout // 2 if act >= 0 else nout, dtype=torch.float32, device=a.device)
+        self._call("jle_gemm_f32_rows", _p(a), _p(b), _p(out), act, m, nout, k)
+        return out
+
     def f32_stream_supported(self, nout: int, k: int, swiglu: bool) -> bool:
         return bool(self._query("jle_gemm_f32_stream_supported", nout, k, int(swiglu)))
 
@@ -1581,7 +1655,8 @@ class HipOps:
     def lm_head(self, h, w, tiled: bool = False):
         """float32 logits; ``tiled``: ``w`` is in the streaming layout (``ops/layout.py``)."""
         if h.dtype == torch.float32:
-            return torch.matmul(h, w.t())
+            out = self._dense_float32(h, w)
+            return torch.matmul(h, w.t()) if out is None else out
         if h.shape[1] % 8 == 0:
             streams = tiled and self.stream_supported(w.shape[0], w.shape[1], False)
             # measured on a 202048 x 5120 head: up to 16 rows the skinny kernel is at the speed of reading the

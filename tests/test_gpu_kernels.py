@@ -844,6 +844,51 @@ def test_float32_products_are_true_float32_at_serving_sizes(ops, rows, k):
         assert err < 2e-6, f"{name}: {err:.3g} of the sum of the terms' sizes"
 
 
+@pytest.mark.parametrize("rows,nout,k", [(1, 2, 4), (2, 513, 1000), (3, 64, 36), (4, 1030, 2044), (5, 6, 256), (8, 70, 1284),
+                                         (128, 2056, 4096), (512, 4096, 4096), (300, 136, 256), (1, 8, 32), (257, 264, 8224)])
+def test_dense_float32_products(ops, rows, nout, k):
+    """The kernels for up to eight rows and for many (tiles of 128 x 128, stages of 32 k, ranges of k), and with the
+    activation.  A sum of K products carries at most a rounding of 2^-24 of the terms' sizes per addition that follows
+    one; the kernel for few rows adds up K / 256 numbers and 30 more a number, the one in parts rounds 192
+    times at most in a stage of 32, then once a stage, and leaves out less than 2^-21 of a product."""
+    x, w = _rand(rows, k, seed=21), _rand(nout, k, seed=22)
+    want, size = x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t()
+    gate, up = want.chunk(2, -1) if nout % 2 == 0 else (None, None)
+    kernels = [(ops.gemm_f32_rows, k / 256 * 4 + 40, 0.0)] if rows <= 8 else []
+    if k % 32 == 0 and nout % 8 == 0:
+        kernels.append((ops.gemm_f32_split, k / 32 + 200, 2.0 ** -21))
+        kernels.append((lambda *a: ops.gemm_f32_split(*a, ranges=1 if len(a) > 2 else min(7, k // 32)), k / 32 + 200, 2.0 ** -21))
+    for fn, adds, left in kernels:
+        bound = size * (adds * 2.0 ** -24 + left)
+        assert bool(((fn(x, w).double() - want).abs() <= bound).all())
+        if gate is not None:
+            assert torch.allclose(fn(x, w, 0), ops.silu_mul(fn(x, w)), rtol=1e-3, atol=1e-5 * float(size.max()))
+            act = fn(x, w, 1).double()  # (|gelu'| < 1.13, and its tanh form differs from itself by float32 roundings only)
+            g = torch.nn.functional.gelu(gate, approximate="tanh")
+            b = 1.13 * bound[:, :nout // 2] * up.abs() + (g.abs() + 2.0 ** -19 * gate.abs()) * bound[:, nout // 2:]
+            assert bool(((act - g * up).abs() <= 1.01 * b + 2.0 ** -19 * (gate * up).abs() + 1e-30).all())
+    ranges = ops.split_ranges(rows, nout, k, False, ops._compute_units)
+    assert ranges or (rows, nout, k) != (512, 4096, 4096)
+    if rows <= 4 or ranges:  # (where the way leads here)
+        assert torch.equal(ops.linear(x, w), ops.gemm_f32_split(x, w, -1, ranges) if ranges else ops.gemm_f32_rows(x, w))
+
+
+def test_dense_float32_products_of_special_numbers(ops):
+    """Infinities, NaN and numbers beyond bfloat16's largest give what float32 gives; rows of very small numbers
+    lose nothing."""
+    x, w = _rand(200, 320, seed=23), _rand(136, 320, seed=24)
+    x[3, 7], x[190, 9], x[70, 5], x[131, 319] = float("inf"), float("nan"), 3.4e38, -float("inf")
+    w[135, 0], w[5, 100] = -float("inf"), 3.4e38
+    x[40] = 0.0
+    want = (x.cpu().double() @ w.cpu().double().t()).float()
+    got = ops.gemm_f32_split(x, w).cpu()
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())
+    assert torch.equal(got[got.isinf()], want[want.isinf()])
+    x, w = _rand(130, 320, seed=25) * 1e-36, _rand(136, 320, seed=26) * 1e12
+    want, size = x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t()
+    assert bool(((ops.gemm_f32_split(x, w).double() - want).abs() <= size * (320 / 4 + 40) * 2.0 ** -24).all())
+
+
 @pytest.mark.parametrize("n,d,f,e,k", [(1, 64, 32, 4, 1), (8, 5120, 96, 16, 1), (64, 260, 36, 128, 2), (100, 128, 64, 5, 1),
                                        (128, 512, 256, 16, 1), (50, 1028, 44, 3, 2), (129, 64, 16, 1, 1)])
 def test_float32_grouped_product_on_the_float32_matrix_instructions(ops, n, d, f, e, k):
