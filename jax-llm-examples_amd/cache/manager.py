@@ -246,11 +246,14 @@ class CacheManager:
         if rid in self.requests:
             raise KeyError(f"request {rid!r} is already live")
         slot = self.slots.alloc()
-        for t in self.state.values():
-            t[slot].zero_()
-        for named in list(self.run_state.values()) + list(self.named_state.values()):
+        # The slot's state in all layers, a launch for each of their types (one for each tensor was seven a request of
+        # Sudilorn's, 448 where 64 start together: 5 us of host time and 3 of the GPU's each).
+        fresh = {}
+        for named in (self.state, *self.run_state.values(), *self.named_state.values()):
             for t in named.values():
-                t[slot].zero_()
+                fresh.setdefault(t.dtype, []).append(t[slot])
+        for rows in fresh.values():
+            torch._foreach_zero_(rows)
         self._lives += 1
         e = RequestEntry(slot=slot, tables=[[] for _ in self.groups], versions=[0 for _ in self.groups],
                          serial=self._lives, freed_upto=[0 for _ in self.groups])
