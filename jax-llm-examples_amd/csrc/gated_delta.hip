@@ -457,7 +457,11 @@ __global__ __launch_bounds__(256, 2) void gdr_chunk_kernel(const T* __restrict__
 // registers.  A chunk is 112 matrix instructions a wavefront (DK = 128), 1.5 us of the 2.9 it takes at 2,048 tokens and 16
 // heads (128 blocks); without its loads it takes 2.3, so what the rest is made of is barriers and trips through shared
 // memory first, the 110 KB of operands second.
-template <int DK>
+// In a chunk the zeros above the diagonals of T and P meet what later tokens write, and zero times an infinity or NaN is
+// NaN: one in a token's value, key or gates would reach the tokens before it.  It stays in the memory's column, so a column
+// that is not finite at the segment's end is worked out again token by token, in the order of gdr_scan_kernel with 16 lanes
+// a column, from the memory before the segment (which this step leaves as it is).
+template <typename T, int DK>
 __global__ __launch_bounds__(256, 2) void gdr_carry_kernel(const float* __restrict__ ws_q, const int* __restrict__ segs,
                                                            const int* __restrict__ cu_seqlens,
                                                            const int* __restrict__ state_slots,
@@ -465,9 +469,13 @@ __global__ __launch_bounds__(256, 2) void gdr_carry_kernel(const float* __restri
                                                            const float* __restrict__ ws_w, const float* __restrict__ ws_u,
                                                            const float* __restrict__ ws_p, const float* __restrict__ ws_kt,
                                                            const float* __restrict__ ws_s, float* __restrict__ o_raw, int N,
-                                                           int H, int G, int dv) {
+                                                           int H, int G, int dv, const T* __restrict__ rows,
+                                                           const float* __restrict__ qn, const float* __restrict__ kn,
+                                                           const float* __restrict__ beta, const float* __restrict__ decay,
+                                                           const float* __restrict__ kq) {
   constexpr int NT = DK / 16, OWN = NT / 4;
   __shared__ f32x4 s_mem[NT][64], s_u[4][64], s_du[4][64];
+  __shared__ int s_bad[4];
   const int lane = threadIdx.x & 63, c16 = lane & 15, g = lane >> 4;
   const int w = wave_index();
   const int h = blockIdx.x % H, kv = h / (H / G);
@@ -567,8 +575,55 @@ __global__ __launch_bounds__(256, 2) void gdr_carry_kernel(const float* __restri
 #pragma unroll
     for (int r = 0; r < NT; ++r) S[r] = s_mem[r][lane];
   }
+  bool bad = false;
 #pragma unroll
-  for (int q = 0; q < OWN; ++q) *reinterpret_cast<f32x4*>(state + own_new + 16 * (OWN * w + q) + 4 * g) = mine[q];
+  for (int q = 0; q < OWN; ++q)
+#pragma unroll
+    for (int x = 0; x < 4; ++x) bad |= !(fabsf(mine[q][x]) <= 3.402823466e38f);
+  unsigned long long mask = __ballot(bad);
+  mask |= mask >> 32;
+  mask |= mask >> 16;
+  if (lane == 0) s_bad[w] = (int)(mask & 0xffff);
+  __syncthreads();
+  const int bad_cols = s_bad[0] | s_bad[1] | s_bad[2] | s_bad[3];
+  if (!(bad_cols >> c16 & 1)) {
+#pragma unroll
+    for (int q = 0; q < OWN; ++q) *reinterpret_cast<f32x4*>(state + own_new + 16 * (OWN * w + q) + 4 * g) = mine[q];
+  }
+  if (bad_cols == 0) return;
+  constexpr int R = DK / 16;  // rows of a column in each of its 16 lanes
+  const int mc = threadIdx.x >> 4, ks = threadIdx.x & 15;
+  const bool redo = bad_cols >> mc & 1;
+  if (!__any(redo)) return;
+  const size_t at = (size_t)(16 * cb + mc) * DK + R * ks;
+  const float* s_old = state + ((slot * 2 + phase) * H + h) * (size_t)dv * DK + at;
+  float* s_new = state + ((slot * 2 + (1 - phase)) * H + h) * (size_t)dv * DK + at;
+  float M[R];
+#pragma unroll
+  for (int i = 0; i < R; ++i) M[i] = s_old[i];
+  const int C = 2 * G * DK + H * dv;
+  for (int t = tok0; t < tok0 + len; ++t) {
+    const float* kr = kn + ((size_t)t * G + kv) * DK + R * ks;
+    const float* qr = qn + ((size_t)t * G + kv) * DK + R * ks;
+    const float v = Num<T>::load(rows + (size_t)t * C + 2 * G * DK + (size_t)h * dv + 16 * cb + mc);
+    const float gc = decay[(size_t)t * H + h], bc = beta[(size_t)t * H + h], kqc = kq[(size_t)t * G + kv];
+    float d4[4] = {0.f, 0.f, 0.f, 0.f}, o4[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+      d4[i & 3] = __builtin_fmaf(M[i], kr[i], d4[i & 3]);
+      o4[i & 3] = __builtin_fmaf(M[i], qr[i], o4[i & 3]);
+    }
+    const float dot = column_lanes_sum<16>((d4[0] + d4[1]) + (d4[2] + d4[3]));
+    const float oq = column_lanes_sum<16>((o4[0] + o4[1]) + (o4[2] + o4[3]));
+    const float u = bc * (v - gc * dot);
+#pragma unroll
+    for (int i = 0; i < R; ++i) M[i] = __builtin_fmaf(kr[i], u, gc * M[i]);
+    if (redo && ks == 0) o_raw[((size_t)t * H + h) * dv + 16 * cb + mc] = __builtin_fmaf(kqc, u, gc * oq);
+  }
+  if (redo) {
+#pragma unroll
+    for (int i = 0; i < R; ++i) s_new[i] = M[i];
+  }
 }
 
 // What the chunked form needs of a step: its chunks (segment, first token, tokens), the segments that go by chunks
@@ -585,7 +640,7 @@ inline size_t chunk_floats(int H, int G, int dk, int dv) {  // scratch of one ch
 
 template <typename T, int DK>
 int launch_chunks(const ByChunks& b, const T* rows, const float* qn, const float* kn, const float* beta, const float* decay,
-                  float* state, const int* cu_seqlens, const int* state_slots, const int* state_phase, float* o_raw, int N,
+                  const float* kq, float* state, const int* cu_seqlens, const int* state_slots, const int* state_phase, float* o_raw, int N,
                   int H, int G, int dv, hipStream_t s) {
   const size_t n = (size_t)b.num_chunks * H;
   float* ws_w = b.ws;
@@ -601,8 +656,9 @@ int launch_chunks(const ByChunks& b, const T* rows, const float* qn, const float
   hipLaunchKernelGGL((gdr_chunk_kernel<T, DK>), dim3(b.num_chunks, H), dim3(256), smem, s, rows, qn, kn, beta, decay,
                      b.chunks, ws_w, ws_u, ws_p, ws_kt, ws_q, ws_s, H, G, dv);
   JLE_LAUNCH_CHECK();
-  hipLaunchKernelGGL(gdr_carry_kernel<DK>, dim3((unsigned)(b.num_segs * H * (dv / 16))), dim3(256), 0, s, ws_q, b.segs,
-                     cu_seqlens, state_slots, state_phase, state, ws_w, ws_u, ws_p, ws_kt, ws_s, o_raw, N, H, G, dv);
+  hipLaunchKernelGGL((gdr_carry_kernel<T, DK>), dim3((unsigned)(b.num_segs * H * (dv / 16))), dim3(256), 0, s, ws_q, b.segs,
+                     cu_seqlens, state_slots, state_phase, state, ws_w, ws_u, ws_p, ws_kt, ws_s, o_raw, N, H, G, dv, rows, qn,
+                     kn, beta, decay, kq);
   JLE_LAUNCH_CHECK();
   return 0;
 }
@@ -770,9 +826,9 @@ int launch_gdr(const T* rows, const float* gates, const float* a_log, const floa
                      decay, kq, floor, H, G, dk, dv, dkp);
   JLE_LAUNCH_CHECK();
   if (by_chunks.num_segs > 0) {
-    const int rc = dk == 128 ? launch_chunks<T, 128>(by_chunks, rows, qn, kn, beta, decay, state, cu_seqlens, state_slots,
+    const int rc = dk == 128 ? launch_chunks<T, 128>(by_chunks, rows, qn, kn, beta, decay, kq, state, cu_seqlens, state_slots,
                                                      state_phase, o_raw, N, H, G, dv, s)
-                             : launch_chunks<T, 64>(by_chunks, rows, qn, kn, beta, decay, state, cu_seqlens, state_slots,
+                             : launch_chunks<T, 64>(by_chunks, rows, qn, kn, beta, decay, kq, state, cu_seqlens, state_slots,
                                                     state_phase, o_raw, N, H, G, dv, s);
     if (rc != 0) return rc;
   }

@@ -84,3 +84,40 @@ def test_chunks_against_the_recurrence(lens, H, G, dk, dv, special, dtype):
     for a, b in zip(err["chunks"], err["scan"]):
         assert a < 2 * b + 2e-7, err
     assert err["chunks"][1] < 2e-6 and err["chunks"][0] < (2e-6 if dtype == torch.float32 else 3e-3), err
+
+
+@pytest.mark.parametrize("where", ["value", "key", "query", "write strength", "decay", "memory"])
+@pytest.mark.parametrize("what", [float("nan"), float("inf"), -float("inf")])
+def test_what_is_not_finite_reaches_no_token_before_it(where, what):
+    """An infinity or NaN within a chunk gives what the recurrence token by token gives: the tokens before it, other heads
+    and other columns of the memory keep their numbers."""
+    from jax_llm_examples_amd.engine import get_ops
+    ops = get_ops(DEV)
+    lens, H, G, dk, dv, bad = [150, 70], 2, 1, 128, 48, 100  # (in the first segment's second chunk)
+    g = torch.Generator().manual_seed(5)
+    N, R = sum(lens), len(lens)
+    rn = lambda *s: torch.randn(*s, generator=g)
+    rows, gates, state = rn(N, 2 * G * dk + H * dv), rn(N, 2 * H), rn(R, 2, H, dv, dk)
+    a_log, dt_bias, norm, gate = rn(H) - 1.0, rn(H), torch.rand(dv, generator=g) + 0.5, rn(N, H * dv)
+    if where == "memory":
+        state[0, 0, 1, 17, 5] = what
+    elif where in ("write strength", "decay"):
+        gates[bad, {"write strength": 0, "decay": H}[where] + 1] = what
+    else:
+        rows[bad, {"query": 3, "key": G * dk + 3, "value": 2 * G * dk + dv + 20}[where]] = what
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)
+    got = {}
+    for way, first in (("chunks", 32), ("scan", 1 << 30)):
+        ops.DELTA_CHUNKS_FROM, ops.DELTA_CHUNKS_LONG = first, 1
+        ctx = types.SimpleNamespace(seg_lens=lens, num_segments=R, cu_seqlens=i32([0, 150, 220]), state_slots=i32([0, 1]),
+                                    state_phase=i32([0, 1]), scratch={}, max_seg_len=max(lens))
+        st = state.to(DEV)
+        o = ops.gated_delta(*(x.to(DEV) for x in (rows, gates, a_log, dt_bias, norm, gate)), H, G, dk, dv, EPS, FLOOR, st, ctx)
+        got[way] = o.cpu(), st.cpu()
+    for a, b in zip(got["chunks"], got["scan"]):
+        for test in (torch.isnan, torch.isposinf, torch.isneginf):
+            assert torch.equal(test(a), test(b)), (where, what, int((test(a) != test(b)).sum()))
+        f = torch.isfinite(b)
+        assert float((a[f] - b[f]).norm() / b[f].norm()) < 2e-6  # (the same sums of float32 numbers in another order)
+    if where != "memory":
+        assert bool(torch.isfinite(got["chunks"][0][:bad]).all())
