@@ -5,15 +5,17 @@
 //   Y[t, f] = act(gate) * up, gate / up = rows f and F + f of W                    (ACT: silu or the tanh form of gelu)
 //
 // The float32 matrix instruction does 256 operations a cycle of a compute unit, the bfloat16 one 4,096.  A float32
-// number is the sum of three bfloat16 numbers, x = h + m + l, without any loss: h holds its upper 8 significant bits
-// (the upper half of the word as it stands), m the next 8, l the rest; both differences are exact.  Of the nine
-// products the six largest are formed (smallest first: h l, l h, m m, h m, m h, h h); the three others are on the average
-// 2^-25 of the whole, half of a float32's last bit.  A stage's six products are summed by themselves and added to the
-// whole once: 1 rounding of the whole for 32 k, where the float32 instruction has one for every 4 (with all six added
-// to the whole one after the other the error was four times as large, 7.0e-7 at K = 2048, and the logits of a model of two
-// layers 5,120 wide were further from 64 bits than with the library's products, 6.6e-6 against 4.6e-6; this way
-// 2.4e-6).  Against 64 bits, of the result's norm: 1.7e-7 where the library's float32 product has 8.1e-7 (K = 2048), 2.5e-7
-// and 1.3e-6 (5120), 3.1e-7 and 1.6e-6 (8192).
+// number is the sum of three bfloat16 numbers, x = h + m + l, without any loss: h is x rounded to the nearest, m what is
+// left rounded to the nearest, l the rest; both differences are exact.  Of the nine products the six largest are formed
+// (smallest first: h l, l h, m m, h m, m h, then h h); the three others are at most 2^-24 of a product, of either sign,
+// and 2^-27 of it in the mean square.  (Cut off instead of rounded, the parts carry the number's sign: up to 2^-21 left out,
+// always towards zero.)  The bfloat16 instruction's sums are not rounded to the nearest: what it drops is below the last
+// place of its largest addend, always downwards.  So h h, whose products are exact, has a sum of its own beside the five
+// small ones', and both are added to the whole on the vector units, once a stage: 1 rounding of the whole for 32 k, where
+// the float32 instruction has one for every 4.  Against 64 bits, of the result's norm, here | the library's float32 product:
+// sums of like terms 1.5e-7 | 4.1e-7 (K = 2048), 2.3e-7 | 6.4e-7 (5120), 2.9e-7 | 8.1e-7 (8192); a single term 2.6e-8 |
+// 2.5e-8, at most 1.6 * 2^-24 of it | 2^-24.  (All six in one sum: a single term 3.4e-8 and a shift of 2^-26 downwards, 4 %
+// faster; the parts cut off: 6.6e-8, at most 8.2 * 2^-24.)
 //
 // Six instructions of 16 times the rate: at best 2.7 times the float32 peak of 157 TFLOP/s.  Reached: 170 to 186 where the
 // library reaches 110 to 150.  What bounds it: the matrix cores are busy about half the time; splitting (24 operations for
@@ -47,16 +49,17 @@ constexpr int kStage = 32;              // k a stage
 constexpr int kPart = kTile * kStage;   // bfloat16 numbers of a part of an operand
 constexpr int kPanel = 8;               // tiles of W whose blocks run together
 
-// four float32 numbers as three times four bfloat16 numbers
+// four float32 numbers as three times four bfloat16 numbers, each what is left rounded to the nearest
 __device__ __forceinline__ void split4(f32x4 x, u32x2 (&p)[3]) {
 #pragma unroll
   for (int i = 0; i < 3; ++i) {
 #pragma unroll
-    for (int j = 0; j < 2; ++j)  // the upper halves of two numbers
-      p[i][j] = __builtin_amdgcn_perm(__float_as_uint(x[2 * j + 1]), __float_as_uint(x[2 * j]), 0x07060302u);
-    if (i < 2) {
-#pragma unroll
-      for (int j = 0; j < 4; ++j) x[j] -= __uint_as_float(__float_as_uint(x[j]) & 0xffff0000u);
+    for (int j = 0; j < 2; ++j) {
+      p[i][j] = pack_bf16(x[2 * j], x[2 * j + 1]);
+      if (i < 2) {
+        x[2 * j] -= __uint_as_float(p[i][j] << 16);
+        x[2 * j + 1] -= __uint_as_float(p[i][j] & 0xffff0000u);
+      }
     }
   }
 }
@@ -131,27 +134,31 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_split_kernel(const float* __r
     for (int n = 0; n < 4; ++n)
 #pragma unroll
       for (int j = 0; j < 3; ++j) b[n][j] = *reinterpret_cast<const bf16x8*>(b_at + j * kPart + n * 512);
-    f32x4 sum[2][4];  // of the stage alone: added to the whole once, not six times, while the next tile's products run
+    f32x4 sum[2][4], top[2][4];  // of the stage alone, the largest products apart from the others: added to the whole once,
+                                 // not six times, while the next tile's products run
 #pragma unroll
     for (int m = 0; m < 4; ++m) {
       bf16x8 a[3];
 #pragma unroll
       for (int j = 0; j < 3; ++j) a[j] = *reinterpret_cast<const bf16x8*>(a_at + j * kPart + m * 512);
-      constexpr int kOfA[6] = {0, 2, 1, 0, 1, 0}, kOfB[6] = {2, 0, 1, 1, 0, 0};  // smallest first
+      constexpr int kOfA[5] = {0, 2, 1, 0, 1}, kOfB[5] = {2, 0, 1, 1, 0};  // smallest first
 #pragma unroll
-      for (int n = 0; n < 4; ++n) sum[m & 1][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int n = 0; n < 4; ++n) sum[m & 1][n] = top[m & 1][n] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int q = 0; q < 6; ++q)
+      for (int q = 0; q < 5; ++q)
 #pragma unroll
         for (int n = 0; n < 4; ++n)
           sum[m & 1][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[kOfA[q]], b[n][kOfB[q]], sum[m & 1][n], 0, 0, 0);
+#pragma unroll
+      for (int n = 0; n < 4; ++n)
+        top[m & 1][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[0], b[n][0], top[m & 1][n], 0, 0, 0);
       if (m > 0)
 #pragma unroll
-        for (int n = 0; n < 4; ++n) acc[m - 1][n] += sum[(m - 1) & 1][n];
+        for (int n = 0; n < 4; ++n) acc[m - 1][n] += top[(m - 1) & 1][n] + sum[(m - 1) & 1][n];
       __builtin_amdgcn_sched_barrier(0);
     }
 #pragma unroll
-    for (int n = 0; n < 4; ++n) acc[3][n] += sum[1][n];
+    for (int n = 0; n < 4; ++n) acc[3][n] += top[1][n] + sum[1][n];
   }
   // element i of acc[m][n] in lane (g, r): row 4 g + i of W's tile m, row r of X's tile n
   auto store = [&](int m, int row, f32x4 y) {

@@ -873,6 +873,51 @@ def test_dense_float32_products(ops, rows, nout, k):
         assert torch.equal(ops.linear(x, w), ops.gemm_f32_split(x, w, -1, ranges) if ranges else ops.gemm_f32_rows(x, w))
 
 
+@pytest.mark.parametrize("k", [32, 256, 2080, 8192])
+def test_dense_float32_products_in_parts_lose_no_part(ops, k):
+    """The product of operands in three bfloat16 parts each is a float32 product: of sums of like terms, of a single
+    term, and with the leading parts cancelled so that each of the six partial products is all that is left."""
+    x, w = _rand(130, k, seed=31), _rand(136, k, seed=32)
+    want = x.double() @ w.double().t()
+    # a rounding of the whole per stage of 32 k and a few beside; one partial product left out alone is 2e-6
+    assert float((ops.gemm_f32_split(x, w).double() - want).norm() / want.norm()) < 2.0 ** -24 * (k / 32 + 4) ** 0.5
+    one = torch.arange(k, device=DEV)[None] == (torch.arange(130, device=DEV) % k)[:, None]
+    for ranges in (1, min(3, k // 32)):
+        want = torch.where(one, x, 0.0).double() @ w.double().t()
+        got = ops.gemm_f32_split(torch.where(one, x, 0.0), w, -1, ranges).double()
+        # left out 2^-24 at most, the sum of what is kept rounded once (and its small terms a little)
+        assert float(((got - want).abs() / want.abs()).max()) < 1.02 * 2.0 ** -23
+    m, l = 2.0 ** -9, 2.0 ** -18  # 1 + m + l: its three parts
+    for a, b, less in ((1 + m + l, 1.0, 1.0), (1.0, 1 + m + l, 1.0), (1 + l, 1.0, 1.0), (1.0, 1 + l, 1.0),
+                       (1 + m, 1 + m, 1 + 2 * m), (1 + 2.0 ** -23, 1.0, 1.0), (1.0, 1 + 2.0 ** -23, 1.0)):
+        x, w = torch.zeros(4, k, device=DEV), torch.zeros(8, k, device=DEV)
+        x[:, 5], w[:, 5], x[:, 17], w[:, 17] = a, b, -less, 1.0
+        assert torch.equal(ops.gemm_f32_split(x, w), torch.full((4, 8), a * b - less, device=DEV)), (a, b, less)
+
+
+@pytest.mark.parametrize("act", [0, 1])
+def test_dense_float32_products_of_special_numbers_with_the_activation(ops, act):
+    """Infinities and NaN in some rows of either operand, and rows of very small numbers, behind the fused activation."""
+    x, w = _rand(200, 320, seed=33), _rand(272, 320, seed=34, scale=0.1)
+    x[3, 7], x[190, 9] = float("inf"), float("nan")
+    w[135, 0], w[140, 100] = -float("inf"), float("nan")
+    x[50] *= 1e-36
+    gate, up = (x.double() @ w.double().t()).float().double().chunk(2, -1)
+    f = torch.nn.functional.silu if act == 0 else lambda z: torch.nn.functional.gelu(z, approximate="tanh")
+    want, got = f(gate) * up, ops.gemm_f32_split(x, w, act).double()
+    z = gate / (1 + torch.exp(-gate)) if act == 0 else want / up  # (silu as the kernels form it: -inf / inf is NaN)
+    nan = (z * up).isnan()
+    ok = torch.isfinite(want) & ~nan
+    assert bool(torch.isfinite(got[ok]).all()) and not bool(torch.isfinite(got[~ok]).any())
+    size = x.double().abs() @ w.double().abs().t()
+    size = torch.where(torch.isfinite(size), size, 0.0)
+    s_gate, s_up = size.chunk(2, -1)
+    # each sum as in test_dense_float32_products; |f'| < 1.13, f itself to a few roundings
+    e_gate, e_up = ((320 / 32 + 200) * 2.0 ** -24 * s for s in (s_gate, s_up))
+    bound = 1.13 * e_gate * up.abs() + (f(gate).abs() + 2.0 ** -19 * gate.abs()) * e_up + 2.0 ** -19 * (gate * up).abs()
+    assert bool(((got - want).abs()[ok] <= 1.01 * bound[ok] + 1e-44).all())
+
+
 def test_dense_float32_products_of_special_numbers(ops):
     """Infinities, NaN and numbers beyond bfloat16's largest give what float32 gives; rows of very small numbers
     lose nothing."""
