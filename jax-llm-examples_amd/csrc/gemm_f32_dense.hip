@@ -17,12 +17,13 @@
 // 2.5e-8, at most 1.6 * 2^-24 of it | 2^-24.  (All six in one sum: a single term 3.4e-8 and a shift of 2^-26 downwards, 4 %
 // faster; the parts cut off: 6.6e-8, at most 8.2 * 2^-24.)
 //
-// Six instructions of 16 times the rate: at best 2.7 times the float32 peak of 157 TFLOP/s.  Reached: 170 to 186 where the
-// library reaches 110 to 150.  What bounds it: the matrix cores are busy about half the time; splitting (24 operations for
+// Six instructions of 16 times the rate: at best 2.7 times the float32 peak of 157 TFLOP/s.  Reached: 137 to 182 where the
+// library reaches 107 to 150.  What bounds it: the matrix cores are busy about half the time; splitting (22 operations for
 // 4 numbers) and the way through shared memory run beside them only as far as the other block's phases fall in between.
 //
-// What the parts cannot hold - infinities and NaN - shows as a sum that is not finite: the wavefront then forms its tile
-// again with float32 instructions straight from memory, and the result is what float32 arithmetic gives.
+// What the parts cannot hold - infinities, NaN, numbers and partial products below 2^-126 - shows as a sum that is not
+// finite, or as one too small for what may have been lost: the wavefront then forms its tile again with float32
+// instructions straight from memory, and the result is what float32 arithmetic gives.
 //
 // A block is 128 rows of W by 128 of X, four wavefronts of 64 x 64 (a wavefront reads 24 KB of shared memory for 96
 // instructions of 16 cycles: half of what shared memory gives).  32 k at a time: every thread has its 32 numbers of the next
@@ -70,6 +71,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_split_kernel(const float* __r
                                                                 float* __restrict__ Y, int M, int Nout, int ld, int nb,
                                                                 int mb, int ranges, int per) {
   __shared__ __attribute__((aligned(16))) uint16_t parts[2][3][kPart];  // [W, X][part]
+  __shared__ __attribute__((aligned(16))) float largest[2][kTile];      // of the rows, without their signs
   constexpr bool GATED = ACT >= 0;
   // A die's blocks are neighbours: panels of kPanel tiles of W, in a panel all tiles of X one after the other.  The
   // 64 blocks that a die runs at a time read 16 tiles instead of 128.
@@ -111,7 +113,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_split_kernel(const float* __r
 #pragma unroll
     for (int n = 0; n < 4; ++n) acc[m][n] = f32x4{0.f, 0.f, 0.f, 0.f};
   f32x4 x[8];  // on their way: the numbers of the next stage
-  uint32_t bits[8] = {0, 0, 0, 0, 0, 0, 0, 0};  // all bits that are set in this thread's pieces of the rows
+  float most[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};  // the largest number in this thread's pieces of the rows
 #pragma unroll
   for (int i = 0; i < 8; ++i) x[i] = *reinterpret_cast<const f32x4*>(src[i]);
   for (int k = 0; k < K; k += kStage) {
@@ -120,7 +122,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_split_kernel(const float* __r
     for (int i = 0; i < 8; ++i) {
       u32x2 p[3];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) bits[i] |= __float_as_uint(x[i][j]);
+      for (int j = 0; j < 4; ++j) most[i] = fmaxf(most[i], fabsf(x[i][j]));
       split4(x[i], p);
 #pragma unroll
       for (int j = 0; j < 3; ++j) *reinterpret_cast<u32x2*>(&parts[i >> 2][j][dst[i & 3]]) = p[j];
@@ -171,23 +173,32 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_split_kernel(const float* __r
     for (int i = 0; i < 4; ++i) y[i] = gate_act<GATED ? ACT : 0>(gate[i]) * up[i];
     return y;
   };
-  // A row whose numbers are all below 2^-95 (none has one of the exponent's upper three bits) has parts that bfloat16
-  // cannot hold: below 2^-126 they are lost, up to there that is less than 2^-31 of the row's largest number.
-  bool odd = false;
+  // What float32 holds and the parts do not: parts and products of parts below 2^-126 are lost, in all no more than
+  // K 2^-122 times the largest number of the two rows (or 1).  A sum that is 2^24 times as large has lost nothing; one that
+  // is not, and is no sum of zeros because one of the rows is all zeros, is formed again, like one that is not finite.
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
-    uint32_t all = bits[i];
 #pragma unroll
-    for (int step = 1; step < 8; step <<= 1) all |= (uint32_t)__shfl_xor((int)all, step);
-    odd |= (all & 0x7fffffffu) != 0 && (all & 0x70000000u) == 0;
+    for (int step = 1; step < 8; step <<= 1) most[i] = fmaxf(most[i], __shfl_xor(most[i], step));
+    if (lc == 0) largest[i >> 2][32 * wave + 8 * (i & 3) + lr] = most[i];
   }
-  odd = __syncthreads_or(odd);
+  __syncthreads();
+  const float lost = (float)K * 0x1p-98f;
+  bool odd = false;
 #pragma unroll
-  for (int m = 0; m < 4; ++m)
+  for (int n = 0; n < 4; ++n) {
+    const float of_x = largest[1][wn * 64 + n * 16 + r];
 #pragma unroll
-    for (int n = 0; n < 4; ++n)
+    for (int m = 0; m < 4; ++m) {
+      const f32x4 of_w = *reinterpret_cast<const f32x4*>(&largest[0][wm * 64 + m * 16 + 4 * g]);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) odd |= !(fabsf(acc[m][n][i]) <= 3.402823466e38f);
+      for (int i = 0; i < 4; ++i) {
+        const float y = fabsf(acc[m][n][i]);
+        const bool small = y < lost * fmaxf(fmaxf(of_x, of_w[i]), 1.f) && of_x != 0.f && of_w[i] != 0.f;
+        odd |= small || !(y <= 3.402823466e38f);
+      }
+    }
+  }
   if (__any(odd)) {
     for (int n = 0; n < 4; ++n) {
       const int row = row0 + wn * 64 + n * 16 + r;

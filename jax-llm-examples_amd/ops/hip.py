@@ -1445,12 +1445,12 @@ class HipOps:
     def split_ranges(rows: int, nout: int, k: int, gated: bool, cus: int) -> int:
         """How many ranges of k the kernel of operands in parts shares a product out over, or 0: the library's is faster.
 
-        A compute unit runs two blocks (tiles of 128 x 128) together; measured, a stage of 32 k takes 1.75 us of one block
-        alone and 2.75 of two, a launch 6 us beside, the ranges' sums 4 and their bytes.  The library reaches 75 to 150
+        A compute unit runs two blocks (tiles of 128 x 128) together; measured, a stage of 32 k takes 1.85 us of one block
+        alone and 2.9 of two, a launch 6 us beside, the ranges' sums 4 and their bytes.  The library reaches 75 to 150
         TFLOP/s here, taken as 115 (its tiles fit some sizes better than others), and a pass of its own for the gate.
-        Both sides measured, library | parts, us: 777 rows of 16,384 x 2,048 470 | 354, 1,554 802 | 619, 4,096 of 4,096 x
-        2,048 474 | 369, 256 of 7,168 x 5,120 171 | 138, 777 of 5,120 x 5,120 328 | 294, 1,554 of 2,048 x 8,192 462 | 349;
-        left to the library: 140 of 16,384 x 2,048 96 | 112, 256 of 2,048 x 2,048 24 | 32, 64 of 7,168 x 5,120 50 | 66."""
+        Both sides measured, library | parts, us: 777 rows of 16,384 x 2,048 488 | 366, 1,554 785 | 631, 4,096 of 4,096 x
+        2,048 460 | 378, 256 of 7,168 x 5,120 148 | 128, 777 of 5,120 x 5,120 323 | 297, 1,554 of 2,048 x 8,192 428 | 335;
+        left to the library: 140 of 16,384 x 2,048 118 | 139, 256 of 2,048 x 2,048 22 | 35, 64 of 7,168 x 5,120 49 | 76."""
         if rows < 96 or k % 32 or nout % 8:
             return 0
         tiles, stages = -(-rows // 128) * -(-nout // 128), k // 32
@@ -1458,7 +1458,7 @@ class HipOps:
         def cost(ranges):
             blocks = -(-tiles * ranges // cus)
             sums = 4 + (2 * ranges + 1) * rows * nout * 4 / 5e6 if ranges > 1 else 0
-            return (blocks // 2 * 2.75 + blocks % 2 * 1.75) * -(-stages // ranges) + 6 + sums
+            return (blocks // 2 * 2.9 + blocks % 2 * 1.85) * -(-stages // ranges) + 6 + sums
 
         best = min(range(1, 2 if gated else max(1, min(8, stages // 4)) + 1), key=cost)
         library = 2 * rows * nout * k / 115e6 + 6 + (3 + rows * nout * 6 / 5e6 if gated else 0)

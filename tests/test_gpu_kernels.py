@@ -895,6 +895,20 @@ def test_dense_float32_products_in_parts_lose_no_part(ops, k):
         assert torch.equal(ops.gemm_f32_split(x, w), torch.full((4, 8), a * b - less, device=DEV)), (a, b, less)
 
 
+def test_dense_float32_products_of_small_numbers_beside_large_ones(ops):
+    """Numbers whose parts are too small for bfloat16, in rows that hold large ones (which meet a zero), and products whose
+    partial products are too small: what float32 holds is not lost.  Rows of zeros stay zeros."""
+    x, w = _rand(132, 320, seed=35) * 1e-36, _rand(136, 320, seed=36) * 1e12
+    x[:, 3], w[:, 3] = 1.0, 0.0
+    x[70] = 0.0
+    y, v = _rand(132, 320, seed=37) * 2.0 ** -59, _rand(136, 320, seed=38) * 2.0 ** -59
+    for a, b in ((x, w), (w, x), (y, v)):
+        want, size = a.double() @ b.double().t(), a.double().abs() @ b.double().abs().t()
+        for ranges in (1, 4):
+            got = ops.gemm_f32_split(a, b, -1, ranges).double()
+            assert bool(((got - want).abs() <= size * (320 / 4 + 40) * 2.0 ** -24).all())  # (a rounding per float32 sum of 4)
+
+
 @pytest.mark.parametrize("act", [0, 1])
 def test_dense_float32_products_of_special_numbers_with_the_activation(ops, act):
     """Infinities and NaN in some rows of either operand, and rows of very small numbers, behind the fused activation."""
@@ -905,9 +919,8 @@ def test_dense_float32_products_of_special_numbers_with_the_activation(ops, act)
     gate, up = (x.double() @ w.double().t()).float().double().chunk(2, -1)
     f = torch.nn.functional.silu if act == 0 else lambda z: torch.nn.functional.gelu(z, approximate="tanh")
     want, got = f(gate) * up, ops.gemm_f32_split(x, w, act).double()
-    z = gate / (1 + torch.exp(-gate)) if act == 0 else want / up  # (silu as the kernels form it: -inf / inf is NaN)
-    nan = (z * up).isnan()
-    ok = torch.isfinite(want) & ~nan
+    # (silu as the kernels form it: -inf / inf is NaN)
+    ok = torch.isfinite(want) & ~((gate / (1 + torch.exp(-gate)) * up).isnan() if act == 0 else want.isnan())
     assert bool(torch.isfinite(got[ok]).all()) and not bool(torch.isfinite(got[~ok]).any())
     size = x.double().abs() @ w.double().abs().t()
     size = torch.where(torch.isfinite(size), size, 0.0)
