@@ -125,6 +125,34 @@ __device__ __forceinline__ void softmax_step(bool masked, f32x4 (&st)[2][4], int
   }
 }
 
+// One token's outputs from the keys that it sees and no others, by a wavefront, with the maximum m and the factor inv that
+// the steps have found.  In a step's product the values of keys outside a token's range meet zero probabilities, and zero
+// times an infinity or NaN is NaN: a token whose outputs are not finite though its probabilities are takes this way.
+// off: the gathered row of position 0.
+__device__ __forceinline__ void attend_alone(const bf16_t* q, const bf16_t* kn, int kn_ld, const bf16_t* kr,
+                                             const bf16_t* vt, int S, int off, int lo, int hi, float scale_log2, float m,
+                                             float inv, bf16_t* out) {
+  const int lane = threadIdx.x & 63;
+  float o[2] = {0.f, 0.f};
+  for (int kb = lo; kb <= hi; kb += 64) {
+    const int count = min(64, hi - kb + 1);
+    const size_t row = (size_t)(kb + min(lane, count - 1) + off);  // (behind the last key: that one again, unused)
+    const bf16_t *a = kn + row * kn_ld, *b = kr + row * kDR;
+    float s = 0.f;
+    for (int e = 0; e < kDN; ++e) s = __builtin_fmaf(bf16_to_float(q[e]), bf16_to_float(a[e]), s);
+    for (int e = 0; e < kDR; ++e) s = __builtin_fmaf(bf16_to_float(q[kDN + e]), bf16_to_float(b[e]), s);
+    const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s, scale_log2, -m));
+    const bf16_t* v = vt + (size_t)lane * S + (kb + off);
+    for (int j = 0; j < count; ++j) {
+      const float pj = __shfl(p, j, 64);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) o[i] = __builtin_fmaf(pj, bf16_to_float(v[(size_t)(64 * i) * S + j]), o[i]);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i) out[lane + 64 * i] = float_to_bf16(o[i] * inv);
+}
+
 // A block takes up to 128 consecutive tokens of a segment and one head, a wavefront 32 of them; the keys in steps of 64
 // absolute positions, which the load unit brings into one of two buffers in shared memory while the other is worked on
 // (a wavefront a quarter of each of K, k_r and V^T), the score and value products transposed as in attention_mfma.hip.
@@ -256,15 +284,32 @@ __global__ __launch_bounds__(256, 2) void expanded_attention_kernel(
   for (int ct = 0; ct < 2; ++ct) {
     const int c = ct * 16 + c16;
     float sum = column_sum(l[ct]);
-    if (c >= nt) continue;
     if (sink != nullptr) sum += exp2f(sink[h] * kLog2e - m[ct]);
     const float inv = 1.0f / sum;
-    bf16_t* o = out + ((size_t)(n0 + c) * H + h) * kDV + 4 * g;
+    bool odd = false;
 #pragma unroll
-    for (int dt = 0; dt < kVT; ++dt) {
-      const u32x2 v = {pack_bf16(acc[ct][dt][0] * inv, acc[ct][dt][1] * inv),
-                       pack_bf16(acc[ct][dt][2] * inv, acc[ct][dt][3] * inv)};
-      *reinterpret_cast<u32x2*>(o + dt * 16) = v;
+    for (int dt = 0; dt < kVT; ++dt)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) odd |= !(fabsf(acc[ct][dt][i]) <= 3.402823466e38f);
+    // (a sum that is not finite is so because of a key that the token sees)
+    unsigned long long again = __ballot(odd && fabsf(sum) <= 3.402823466e38f && c < nt);
+    again |= again >> 32;
+    again |= again >> 16;
+    again &= 0xffff;
+    if (c < nt && !(again >> c16 & 1)) {
+      bf16_t* o = out + ((size_t)(n0 + c) * H + h) * kDV + 4 * g;
+#pragma unroll
+      for (int dt = 0; dt < kVT; ++dt) {
+        const u32x2 v = {pack_bf16(acc[ct][dt][0] * inv, acc[ct][dt][1] * inv),
+                         pack_bf16(acc[ct][dt][2] * inv, acc[ct][dt][3] * inv)};
+        *reinterpret_cast<u32x2*>(o + dt * 16) = v;
+      }
+    }
+    for (; again != 0; again &= again - 1) {
+      const int of = __ffsll((long long)again) - 1, n = n0 + ct * 16 + of;
+      attend_alone(q + (size_t)n * q_ld + (size_t)h * (kDN + kDR), kn + (size_t)h * kDN, H * kDN, kr,
+                   vt + (size_t)h * kDV * S, S, blk.z, __shfl(lo[ct], of, 64), __shfl(hi[ct], of, 64), scale_log2,
+                   __shfl(m[ct], of, 64), __shfl(inv, of, 64), out + ((size_t)n * H + h) * kDV);
     }
   }
 }

@@ -89,3 +89,33 @@ def test_against_the_definition(segs, window, sink, H, R, ps):
             # a score of size 1 moves by the keys' rounding averaged over 128 terms, far below that
             assert err < 4 * 2.0 ** -9, (i, h, float(err))
         o += n
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("window, seen_by", [(None, range(70, 300)), (64, range(70, 134)), (40, range(70, 110))])
+@pytest.mark.parametrize("what", [float("nan"), float("inf")])
+def test_a_latent_that_is_not_finite_reaches_only_the_tokens_that_see_it(window, seen_by, what):
+    """Tokens before its own, and those whose window has passed it, share its steps of 64 keys and keep their numbers."""
+    dev, n, H, R, ps = "cuda:0", 300, 2, 64, 16
+    ops = HipOps(dev)
+    ops.LATENT_EXPAND_PAIRS = 0
+    g = torch.Generator().manual_seed(11)
+    bf = lambda *s, std=1.0: (torch.randn(*s, generator=g) * std).to(torch.bfloat16).to(dev)
+    width = -(-n // ps)
+    table = torch.arange(width, dtype=torch.int32, device=dev).view(1, width)
+    latent, rope, q = bf(width, ps, R), bf(width, ps, DR), bf(n, H, DN + DR)
+    uk, uv = bf(H * DN, R, std=R ** -0.5), bf(H * DV, R, std=R ** -0.5)
+    pos, seg = torch.arange(n, dtype=torch.int32, device=dev), torch.zeros(n, dtype=torch.int32, device=dev)
+    got = []
+    for value in (None, what):
+        if value is not None:
+            latent[70 // ps, 70 % ps, 5] = value
+        meta = GroupContext(block_table=None, slot_mapping=None, width=width, retention=("all",), seg_lens=[n], seg_starts=[0])
+        got.append(ops.latent_attention_expanded(q, DN, uk, uv, latent, rope, table, pos, seg, window, (DN + DR) ** -0.5, meta))
+    clean, dirty = (x.view(n, H * DV).double() for x in got)
+    sees = torch.zeros(n, dtype=torch.bool, device=dev)
+    sees[list(seen_by)] = True
+    assert not bool(torch.isfinite(dirty[sees]).any())
+    # (probabilities not rounded to bfloat16 where a row is formed again, results rounded to it: 2^-9 each)
+    assert bool(torch.isfinite(dirty[~sees]).all())
+    assert float((dirty - clean)[~sees].norm() / clean[~sees].norm()) < 2.0 ** -8
