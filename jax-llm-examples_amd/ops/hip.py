@@ -716,7 +716,7 @@ class HipOps:
     # microseconds): one prompt of 512 tokens 129 | 59, of 2,048 837 | 107; 64 prompts of 20 107 | 74, of 40 196 | 80;
     # behind cached tokens: 128 behind 1,024 101 | 72, 64 behind 2,048 95 | 101 (63 pairs a key), 64 behind 8,192
     # 233 | 347, 512 behind 8,192 1,405 | 363, 256 behind 16,384 1,523 | 658 (254 pairs a key).
-    # The formed keys and values take no more than LATENT_EXPAND_BYTES.
+    # The gathered rows and the keys and values formed of them take no more than LATENT_EXPAND_BYTES.
     LATENT_EXPAND_ROWS = 8
     LATENT_EXPAND_PAIRS = 160
     LATENT_EXPAND_BYTES = 1 << 30
@@ -759,20 +759,19 @@ class HipOps:
                 or not self._query("jle_latent_expanded_supported", r, nope_dim, dr, dv, q.stride(0))):
             return None
         w = 0 if window is None else int(window)
+        # (the layout belongs to the step and the window; whether it pays, to the layer's heads and sizes too)
+        held = meta.meta if meta is not None else {}
         key = f"latent_expanded_{w}"
-        plan = meta.meta.get(key) if meta is not None else None
-        if plan is None:
-            spans, blocks, rows, pairs = self.expanded_plan(*self._segments(meta, token_segment, positions), w)
-            if (rows > self.LATENT_EXPAND_ROWS * n and pairs < self.LATENT_EXPAND_PAIRS * rows
-                    or rows * H * (nope_dim + dv) * 2 > self.LATENT_EXPAND_BYTES):
-                plan = (None, 0, 0)
-            else:
-                plan = (torch.tensor(spans + blocks, dtype=torch.int32).to(q.device), len(spans), rows)
-            if meta is not None:
-                meta.meta[key] = plan
-        table, ns, rows = plan
-        if table is None:
+        layout = held.get(key)
+        if layout is None:
+            layout = held[key] = self.expanded_plan(*self._segments(meta, token_segment, positions), w)
+        spans, blocks, rows, pairs = layout
+        if (rows > self.LATENT_EXPAND_ROWS * n and pairs < self.LATENT_EXPAND_PAIRS * rows
+                or rows * (H * (nope_dim + dv) + r + dr) * 2 > self.LATENT_EXPAND_BYTES):
             return None
+        table, ns = held.get(key + "_table"), len(spans)
+        if table is None:
+            table = held[key + "_table"] = torch.tensor(spans + blocks, dtype=torch.int32).to(q.device)
         np_, ps = latent_pages.shape[0], latent_pages.shape[1]
         if q.stride(2) != 1 or q.stride(1) != dq:
             raise KernelError("the heads' queries must lie side by side at the start of contiguous rows")

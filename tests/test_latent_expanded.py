@@ -119,3 +119,24 @@ def test_a_latent_that_is_not_finite_reaches_only_the_tokens_that_see_it(window,
     # (probabilities not rounded to bfloat16 where a row is formed again, results rounded to it: 2^-9 each)
     assert bool(torch.isfinite(dirty[~sees]).all())
     assert float((dirty - clean)[~sees].norm() / clean[~sees].norm()) < 2.0 ** -8
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("first, second", [(2, 8), (8, 2)])
+def test_layers_of_unlike_heads_in_one_step_are_judged_by_their_own_sizes(first, second):
+    """A step's layout is shared by its layers, what the keys and values take is not: a limit that two heads' keep and
+    eight heads' do not."""
+    dev, n, R, ps = "cuda:0", 128, 64, 16
+    ops = HipOps(dev)
+    ops.LATENT_EXPAND_PAIRS = 0
+    zeros = lambda *s: torch.zeros(*s, dtype=torch.bfloat16, device=dev)
+    table = torch.arange(n // ps, dtype=torch.int32, device=dev).view(1, -1)
+    pos, seg = torch.arange(n, dtype=torch.int32, device=dev), torch.zeros(n, dtype=torch.int32, device=dev)
+    meta = GroupContext(block_table=None, slot_mapping=None, width=n // ps, retention=("all",), seg_lens=[n], seg_starts=[0])
+    taken = lambda H: n * (H * (DN + DV) + R + DR) * 2
+    call = lambda H: ops.latent_attention_expanded(zeros(n, H, DN + DR), DN, zeros(H * DN, R), zeros(H * DV, R),
+                                                   zeros(n // ps, ps, R), zeros(n // ps, ps, DR), table, pos, seg, None, 0.1, meta)
+    ops.LATENT_EXPAND_BYTES = taken(2)
+    assert [call(H) is not None for H in (first, second)] == [first == 2, second == 2]
+    ops.LATENT_EXPAND_BYTES = taken(2) - 1
+    assert call(2) is None
