@@ -140,3 +140,17 @@ def test_layers_of_unlike_heads_in_one_step_are_judged_by_their_own_sizes(first,
     assert [call(H) is not None for H in (first, second)] == [first == 2, second == 2]
     ops.LATENT_EXPAND_BYTES = taken(2) - 1
     assert call(2) is None
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("scale", [0.1, 0.0, -0.1])
+def test_every_scale_has_a_way(scale):
+    """A scale of zero or below, which a configuration may name, stays in the latent's space."""
+    dev, n, H, R, ps = "cuda:0", 80, 2, 64, 16
+    ops = HipOps(dev)
+    zeros = lambda *s: torch.zeros(*s, dtype=torch.bfloat16, device=dev)
+    table = torch.arange(n // ps, dtype=torch.int32, device=dev).view(1, -1)
+    pos, seg = torch.arange(n, dtype=torch.int32, device=dev), torch.zeros(n, dtype=torch.int32, device=dev)
+    out = ops.latent_attention_expanded(zeros(n, H, DN + DR), DN, zeros(H * DN, R), zeros(H * DV, R), zeros(n // ps, ps, R),
+                                        zeros(n // ps, ps, DR), table, pos, seg, None, scale)
+    assert (out is not None) == (scale > 0)
