@@ -347,9 +347,7 @@ JLE_API int jle_latent_expanded_attention(const void* q, int q_ld, const void* k
       ((uintptr_t)q | (uintptr_t)kn | (uintptr_t)kr | (uintptr_t)vt | (uintptr_t)out | (uintptr_t)blocks) % 16)
     return JLE_BAD_ARG;
   constexpr int smem = 2 * kBuffer;
-  const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&expanded_attention_kernel),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, smem);
-  if (e != hipSuccess) return (int)e;
+  if (const int rc = allow_lds(expanded_attention_kernel, smem)) return rc;
   hipLaunchKernelGGL(expanded_attention_kernel, dim3((unsigned)(num_blocks * H)), dim3(256), smem, s, (const bf16_t*)q, q_ld,
                      (const bf16_t*)kn, (const bf16_t*)kr, (const bf16_t*)vt, S, (bf16_t*)out, positions,
                      (const int4*)blocks, window, scale * kLog2e, H, sink);

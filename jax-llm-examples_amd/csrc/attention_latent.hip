@@ -714,13 +714,7 @@ int launch_latent_lds(dim3 grid, size_t smem, hipStream_t s, const bf16_t* q_lat
                       int dr, const bf16_t* latent, const bf16_t* latent_t, const bf16_t* rope, bf16_t* out,
                       const int* positions, const int* token_segment, const int* block_table, int table_width,
                       int window, float scale, const int* blocks, int N, int H, int R, int ps, const float* sink) {
-  static size_t allowed = 0;  // (what this kernel has been given leave to use of the compute unit's shared memory)
-  if (smem > allowed) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&latent_attention_lds_kernel<NR>),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
-    if (e != hipSuccess) return (int)e;
-    allowed = smem;
-  }
+  if (const int rc = allow_lds(latent_attention_lds_kernel<NR>, smem)) return rc;
   hipLaunchKernelGGL(latent_attention_lds_kernel<NR>, grid, dim3(256), smem, s, q_lat, q, q_ld, dn, dr, latent,
                      latent_t, rope, out, positions, token_segment, block_table, table_width, window, scale, blocks, N,
                      H, R, ps, sink);

@@ -63,6 +63,14 @@ __device__ __forceinline__ float wave_max(float v) {
   return v;
 }
 
+// Leave for a kernel to use `bytes` of a compute unit's shared memory, on the current device.  Asked for at every launch: a
+// leave that the process remembers is the first device's alone.
+template <typename K>
+inline int allow_lds(K* kernel, size_t bytes) {
+  return (int)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  (int)bytes);
+}
+
 // Sum over a block of kThreads threads (a multiple of 64); every thread gets the result.
 // The order of additions is fixed, so the result depends on the inputs only.
 template <int kThreads>

@@ -650,9 +650,7 @@ int launch_chunks(const ByChunks& b, const T* rows, const float* qn, const float
   float* ws_kt = ws_s + n * 2 * kChunk;
   float* ws_q = ws_kt + (size_t)b.num_chunks * G * DK * kChunk;
   constexpr int smem = (kChunk * (DK + 4) + 2 * kChunk * (kChunk + 4) + 3 * kChunk) * (int)sizeof(float);
-  static const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gdr_chunk_kernel<T, DK>),
-                                                  hipFuncAttributeMaxDynamicSharedMemorySize, smem);
-  if (e != hipSuccess) return (int)e;
+  if (const int rc = allow_lds(gdr_chunk_kernel<T, DK>, smem)) return rc;
   hipLaunchKernelGGL((gdr_chunk_kernel<T, DK>), dim3(b.num_chunks, H), dim3(256), smem, s, rows, qn, kn, beta, decay,
                      b.chunks, ws_w, ws_u, ws_p, ws_kt, ws_q, ws_s, H, G, dv);
   JLE_LAUNCH_CHECK();

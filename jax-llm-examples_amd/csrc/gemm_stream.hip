@@ -431,9 +431,7 @@ __global__ __launch_bounds__(256, 1) void wide_kernel(const bf16_t* __restrict__
 template <bool SW>
 int launch_wide(hipStream_t s, const void* X, const void* W, void* Y, const int* offsets, const int* a_rows,
                 const float* scale, int M, int Nout, int K, int G) {
-  static const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&wide_kernel<SW>),
-                                                  hipFuncAttributeMaxDynamicSharedMemorySize, kWideLds);
-  if (e != hipSuccess) return (int)e;
+  if (const int rc = allow_lds(wide_kernel<SW>, kWideLds)) return rc;
   const int nblk8 = ((SW ? Nout / 2 : Nout) + (SW ? 1024 : 2048) - 1) / (SW ? 1024 : 2048) * 8;
   const long long items = ((long long)M / kWideRows + G) * nblk8;
   if (items > (1ll << 30)) return JLE_BAD_ARG;

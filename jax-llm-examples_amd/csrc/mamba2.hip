@@ -647,14 +647,8 @@ int launch_scan(const void* proj, const void* rows, const float* dt_bias, const 
 template <int NT, bool VEC>
 int launch_chunks(const bf16_t* proj, const bf16_t* rows, const float* dt_bias, const float* a_log, const float* skip,
                   const Memory& mem, float* y, const Sizes& z, int R, hipStream_t s) {
-  static bool allowed = false;
   constexpr size_t smem = chunk_lds<NT>();
-  if (!allowed) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&mamba2_chunk_kernel<NT, VEC>),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
-    if (e != hipSuccess) return (int)e;
-    allowed = true;
-  }
+  if (const int rc = allow_lds(mamba2_chunk_kernel<NT, VEC>, smem)) return rc;
   hipLaunchKernelGGL((mamba2_chunk_kernel<NT, VEC>), dim3(R, z.H, (z.P + kChunk - 1) / kChunk), dim3(kChunkThreads), smem, s, proj,
                      rows, dt_bias, a_log, skip, mem, y, z);
   JLE_LAUNCH_CHECK();

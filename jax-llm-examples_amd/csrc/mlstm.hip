@@ -545,19 +545,6 @@ __global__ __launch_bounds__(256) void mlstm_chunk_out_kernel(const T* __restric
   }
 }
 
-namespace {
-template <typename K>
-int allow_lds(K kernel, size_t smem, size_t& allowed) {
-  if (smem > allowed) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                       (int)smem);
-    if (e != hipSuccess) return (int)e;
-    allowed = smem;
-  }
-  return 0;
-}
-}  // namespace
-
 JLE_API int jle_mlstm_chunk_tokens() { return kChunk; }
 JLE_API int jle_mlstm_chunked_supported(int dk, int dv) { return dk >= 1 && dk <= 128 && dv >= 1; }
 
@@ -580,16 +567,15 @@ JLE_API int jle_mlstm_chunked(const void* rows, int is_bf16, float* gates, const
   const size_t smem_state = sizeof(float) * ((size_t)kChunk * KS + kChunk * VS + 5 * kChunk);
   const size_t smem_out = sizeof(float) * ((size_t)2 * kChunk * KS + 2 * kChunk * VS + (size_t)dkp * VS + dkp + 9 * kChunk);
   const float q_mul = 1.0f / sqrtf((float)dk);
-  static size_t allowed[4] = {0, 0, 0, 0};
   if (num_chunks > 0) {
     const dim3 grid(num_chunks, H, slices);
     int rc;
     if (is_bf16) {
-      if ((rc = allow_lds(&mlstm_chunk_state_kernel<bf16_t>, smem_state, allowed[0]))) return rc;
+      if ((rc = allow_lds(mlstm_chunk_state_kernel<bf16_t>, smem_state))) return rc;
       hipLaunchKernelGGL(mlstm_chunk_state_kernel<bf16_t>, grid, dim3(256), smem_state, s, (const bf16_t*)rows, gates,
                          chunks, ws_C, ws_n, ws_m, H, dk, dv);
     } else {
-      if ((rc = allow_lds(&mlstm_chunk_state_kernel<float>, smem_state, allowed[1]))) return rc;
+      if ((rc = allow_lds(mlstm_chunk_state_kernel<float>, smem_state))) return rc;
       hipLaunchKernelGGL(mlstm_chunk_state_kernel<float>, grid, dim3(256), smem_state, s, (const float*)rows, gates,
                          chunks, ws_C, ws_n, ws_m, H, dk, dv);
     }
@@ -602,11 +588,11 @@ JLE_API int jle_mlstm_chunked(const void* rows, int is_bf16, float* gates, const
     const dim3 grid(num_chunks, H, slices);
     int rc;
     if (is_bf16) {
-      if ((rc = allow_lds(&mlstm_chunk_out_kernel<bf16_t>, smem_out, allowed[2]))) return rc;
+      if ((rc = allow_lds(mlstm_chunk_out_kernel<bf16_t>, smem_out))) return rc;
       hipLaunchKernelGGL(mlstm_chunk_out_kernel<bf16_t>, grid, dim3(256), smem_out, s, (const bf16_t*)rows, gates, chunks,
                          ws_C, ws_n, ws_m0, o_raw, H, dk, dv, q_mul, floor_);
     } else {
-      if ((rc = allow_lds(&mlstm_chunk_out_kernel<float>, smem_out, allowed[3]))) return rc;
+      if ((rc = allow_lds(mlstm_chunk_out_kernel<float>, smem_out))) return rc;
       hipLaunchKernelGGL(mlstm_chunk_out_kernel<float>, grid, dim3(256), smem_out, s, (const float*)rows, gates, chunks,
                          ws_C, ws_n, ws_m0, o_raw, H, dk, dv, q_mul, floor_);
     }

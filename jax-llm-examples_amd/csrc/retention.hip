@@ -773,13 +773,7 @@ int launch_outputs(const bf16_t* rows, const Operands& o, const Heads& z, const 
                    bf16_t* out, float eps, hipStream_t s) {
   constexpr size_t lds = output_lds<DKS, DVT>();
   static_assert(lds <= 160 * 1024, "the two buffers fit a compute unit");
-  static bool allowed = false;
-  if (!allowed) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&retention_outputs_kernel<DKS, DVT, VEC>),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    if (e != hipSuccess) return (int)e;
-    allowed = true;
-  }
+  if (const int rc = allow_lds(retention_outputs_kernel<DKS, DVT, VEC>, lds)) return rc;
   hipLaunchKernelGGL((retention_outputs_kernel<DKS, DVT, VEC>), dim3(nc * z.H), dim3(kOutThreads), lds, s, rows, o, z, decays,
                      chunks, out, eps);
   JLE_LAUNCH_CHECK();
@@ -809,13 +803,7 @@ int run_chunks(const bf16_t* rows, const float2* angles, const Heads& z, const M
   const bool vec8 = z.dk % 8 == 0 && z.dv % 8 == 0 && (z.rd == 0 || z.half_pairs) && (z.rd / 2) % 8 == 0 &&
                     ((uintptr_t)rows | (uintptr_t)angles) % 16 == 0;  // (then a row's width is a multiple of 8 too)
   auto prepare = vec8 ? retention_prepare_kernel<true> : retention_prepare_kernel<false>;
-  static bool allowed[2] = {false, false};
-  if (!allowed[vec8]) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(prepare), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                       80 * 1024);
-    if (e != hipSuccess) return (int)e;
-    allowed[vec8] = true;
-  }
+  if (const int rc = allow_lds(prepare, 80 * 1024)) return rc;
   hipLaunchKernelGGL(prepare, dim3(nc, kChunk / kPrep, z.H), dim3(256), lds, s, rows, angles, z, mem.decays,
                      chunks, o);
   JLE_LAUNCH_CHECK();

@@ -31,3 +31,20 @@ def test_dense_float32_products_by_size():
                                   ("cuda:1", "cuda:1")])
 def test_matrices_elsewhere_are_left_to_the_library(rows, a, b):
     assert rule(tensor(rows, 4096, a), tensor(4096, 4096, b)) is None
+
+
+def test_leave_for_shared_memory_is_asked_for_on_the_device_of_the_launch():
+    """What a kernel may use of a compute unit's shared memory is an attribute of a device: a process with two must not
+    remember the first one's.  (One place asks for it, and no launcher keeps an answer.)"""
+    import glob
+    import os
+    from jax_llm_examples_amd.ops import build
+    asks = []
+    for path in glob.glob(os.path.join(build.CSRC, "*.h*")):
+        with open(path) as f:
+            for line in f:
+                if "hipFuncSetAttribute" in line:
+                    asks.append(os.path.basename(path))
+                kept = line.strip().startswith("static ") and ("allowed" in line or "hipError_t" in line)
+                assert not kept, (path, line)
+    assert asks == ["common.h"]
