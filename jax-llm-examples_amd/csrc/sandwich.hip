@@ -54,11 +54,22 @@ __device__ __forceinline__ void store_piece(T* p, const float (&o)[VEC]) {
     Num<T>::store(p, o[0]);
   }
 }
-// a vector of weights, or `fill` where there is none or the row has ended
+// a vector of weights, which may lie at any float (a slice of a longer vector: a load of four needs no more), or `fill`
+// where there is none or the row has ended
 template <int VEC>
 __device__ __forceinline__ void load_weights(const float* p, int d, bool in, float fill, float (&o)[VEC]) {
   if (p != nullptr && in) {
-    load_piece<float, VEC>(p + d, o);
+    typedef __attribute__((ext_vector_type(4), aligned(4))) float f32x4_anywhere;
+    if constexpr (VEC >= 4) {
+#pragma unroll
+      for (int e = 0; e < VEC; e += 4) {
+        const f32x4_t r = *reinterpret_cast<const f32x4_anywhere*>(p + d + e);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) o[e + i] = r[i];
+      }
+    } else {
+      o[0] = p[d];
+    }
   } else {
 #pragma unroll
     for (int e = 0; e < VEC; ++e) o[e] = fill;
@@ -277,13 +288,17 @@ int launch_sandwich(const SandwichArgs& args, hipStream_t s) {
   SandwichArgs a = args;
   if (a.stats != nullptr) a.shift_w = nullptr;  // (the first kernel: sums and statistics)
   const dim3 g((unsigned)a.N);
+  // (wider rows, up to 8,192: 2 x 4 elements a thread, or 8 or 16 single ones by fewer threads, which have the registers;
+  // sums and shift of 2,048 rows of 6,148 in pieces of four 69 us, in single elements 198; of 1,026 by 256 threads 23, by
+  // 1,024 that spill 96)
+  constexpr int T1 = VEC == 1 ? 256 : 1024, C1 = 8 / VEC, T2 = VEC == 1 ? 512 : T1, C2 = VEC == 1 ? 16 : C1;
 #define JLE_SANDWICH_CASE(TH, C) \
   else if (a.D <= TH * C * VEC) hipLaunchKernelGGL((add_norm_shift_kernel<T, TH, C, VEC>), g, dim3(TH), 0, s, a)
   if (a.D <= 256 * VEC) hipLaunchKernelGGL((add_norm_shift_kernel<T, 256, 1, VEC>), g, dim3(256), 0, s, a);
   JLE_SANDWICH_CASE(512, 1);
   JLE_SANDWICH_CASE(1024, 1);
-  else if constexpr (VEC > 1) return JLE_BAD_ARG;  // (such rows go an element a thread)
-  JLE_SANDWICH_CASE(1024, 8);
+  JLE_SANDWICH_CASE(T1, C1);
+  JLE_SANDWICH_CASE(T2, C2);
   else return JLE_BAD_ARG;
 #undef JLE_SANDWICH_CASE
   if (args.stats != nullptr)
@@ -318,12 +333,10 @@ __global__ __launch_bounds__(THREADS) void polynorm_kernel(const T* __restrict__
   };
   auto fetch = [&](int d, float (&u)[VEC]) {
     load_piece<T, VEC>(zr + d, u);
-    if (bias != nullptr) {
-      float b[VEC];
-      load_piece<float, VEC>(bias + d, b);
+    float b[VEC];
+    load_weights<VEC>(bias, d, true, 0.f, b);
 #pragma unroll
-      for (int e = 0; e < VEC; ++e) u[e] += b[e];
-    }
+    for (int e = 0; e < VEC; ++e) u[e] += b[e];
   };
   constexpr int P = PIECES > 0 ? PIECES : 1;
   float kept[P][VEC];
@@ -394,12 +407,14 @@ void launch_polynorm(const T* z, int ldz, const float* bias, const float* coef, 
                      int vec, hipStream_t s) {
   // (which form runs depends on the width and on where the arrays lie, not on the step; 2,048 rows of 14,336 in 16-byte
   // pieces, the three sums behind one barrier: 34 us, 3.4 TB/s; in pieces of four with a barrier pair a sum 66; 8 rows of
-  // 8,192 7.1 and 12.6)
+  // 8,192 7.1 and 12.6; 2,048 rows of 14,340 in pieces of four 28, with the row read twice 32)
 #define JLE_POLYNORM(TH, V, P) \
   hipLaunchKernelGGL((polynorm_kernel<T, TH, V, P>), dim3(N), dim3(TH), 0, s, z, ldz, bias, coef, eps, out, F)
   if (vec == 8 && F <= 256 * 8 * 2) JLE_POLYNORM(256, 8, 2);
   else if (vec == 8 && F <= 512 * 8 * 4) JLE_POLYNORM(512, 8, 4);
   else if (vec == 8) JLE_POLYNORM(256, 8, 0);
+  else if (vec == 4 && F <= 256 * 4 * 4) JLE_POLYNORM(256, 4, 4);
+  else if (vec == 4 && F <= 512 * 4 * 8) JLE_POLYNORM(512, 4, 8);
   else if (vec == 4) JLE_POLYNORM(256, 4, 0);
   else JLE_POLYNORM(256, 1, 0);
 #undef JLE_POLYNORM
@@ -426,10 +441,9 @@ JLE_API int jle_add_norm_shift(const float* x, float* x_out, int delta_kind, con
   SandwichArgs a{x, x_out, delta_kind, y, y_bias, g, g_bias, post_w, post_eps, do_norm, w, eps, h_out, shift_w,
                  hs_out, state, positions, token_segment, cu_seqlens, state_slots, state_phase, stats, N, D};
   uintptr_t all = 0;
-  for (const void* p : {(const void*)x, (const void*)x_out, y, (const void*)y_bias, g, (const void*)g_bias, (const void*)post_w,
-                        (const void*)w, (const void*)h_out, (const void*)shift_w, (const void*)hs_out, (const void*)state})
+  for (const void* p : {(const void*)x, (const void*)x_out, y, g, (const void*)h_out, (const void*)hs_out, (const void*)state})
     all |= (uintptr_t)p;
-  const int vec = all % 16 ? 1 : D % 8 == 0 && D <= 1024 * 8 ? 8 : D % 4 == 0 && D <= 1024 * 4 ? 4 : 1;
+  const int vec = all % 16 ? 1 : D % 8 == 0 ? 8 : D % 4 == 0 ? 4 : 1;
   int rc;
   if (is_bf16)
     rc = vec == 8 ? launch_sandwich<bf16_t, 8>(a, s) : vec == 4 ? launch_sandwich<bf16_t, 4>(a, s) : launch_sandwich<bf16_t, 1>(a, s);
@@ -444,7 +458,7 @@ JLE_API int jle_polynorm(const void* z, int ldz, const float* bias, const float*
                          int is_bf16, int N, int F, hipStream_t s) {
   if (N <= 0) return 0;
   if (F <= 0 || ldz < F || coef == nullptr) return JLE_BAD_ARG;
-  const bool aligned = ((uintptr_t)z | (uintptr_t)out | (uintptr_t)bias) % 16 == 0;
+  const bool aligned = ((uintptr_t)z | (uintptr_t)out) % 16 == 0;
   const int vec = !aligned ? 1 : F % 8 == 0 && ldz % 8 == 0 ? 8 : F % 4 == 0 && ldz % 4 == 0 ? 4 : 1;
   if (is_bf16)
     launch_polynorm<bf16_t>((const bf16_t*)z, ldz, bias, coef, eps, (bf16_t*)out, N, F, vec, s);

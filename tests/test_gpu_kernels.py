@@ -1238,6 +1238,54 @@ def test_shift_apart_from_its_norm(ops, dt, d):
             assert torch.equal(a, b), (what, float((a - b).abs().max()))
 
 
+@pytest.mark.parametrize("dt", DT)
+@pytest.mark.parametrize("off", [0, 1])
+@pytest.mark.parametrize("d", [100, 1026, 2050, 4092, 4098, 4100, 8188, 8190])
+def test_gated_branch_norm_and_shift_at_odd_widths(ops, dt, d, off):
+    """Every form of the sandwich arrangement's kernel against its definition in 64 bits: rows in pieces of four and of one,
+    one or several a thread, weights that lie at any float; with the shift in the same kernel and apart."""
+    import types
+    from jax_llm_examples_amd.parts.residual import GatedBranch
+    lens, starts = [1, 7, 12], [5, 0, 3]
+    n, cu = sum(lens), torch.tensor([0] + lens).cumsum(0)
+    i32 = lambda v: torch.as_tensor(v, dtype=torch.int32).to(DEV)
+    ctx = types.SimpleNamespace(positions=i32([s + t for s, k in zip(starts, lens) for t in range(k)]),
+                                token_segment=i32([i for i, k in enumerate(lens) for _ in range(k)]), cu_seqlens=i32(cu),
+                                state_slots=i32([2, 0, 1]), state_phase=i32([0, 1, 1]))
+    x, y, g = _rand(n, d, seed=1), _rand(n, d, dt=dt, seed=2), _rand(n, d, dt=dt, seed=3)
+    v = [_rand(d + off, seed=4 + i)[off:] for i in range(5)]
+    y64 = (y.double() + v[0].double()) * torch.sigmoid(g.double() + v[1].double())
+    sums = x.double() + y64 / torch.sqrt((y64 * y64).mean(-1, keepdim=True) + 1e-3) * v[2].double()
+    h = sums / torch.sqrt((sums * sums).mean(-1, keepdim=True) + 1e-5) * v[3].double()
+    old = _rand(3, 2, d, seed=9).double()
+    before = torch.cat([old[2, 0][None], torch.zeros(1, d, dtype=torch.float64, device=DEV), h[1:7], old[1, 1][None], h[8:19]])
+    new = old.clone()
+    new[2, 1], new[0, 0], new[1, 0] = h[0], h[7], h[19]
+    for apart in (1 << 30, 1):
+        ops.SHIFT_APART_ROWS = apart
+        state = _rand(3, 2, d, seed=9)
+        got = (*ops.add_norm_shift(x.clone(), GatedBranch(y, v[0], g, v[1], v[2], 1e-3), v[3], 1e-5, dt, (v[4], state), ctx), state)
+        del ops.SHIFT_APART_ROWS
+        for a, b, what in zip(got, (sums, h, h + (before - h) * v[4].double(), new), ("sums", "rows", "shifted", "state")):
+            # float32 arithmetic, some ten roundings and two sums; rows rounded to the run dtype
+            tol = 2e-6 if a.dtype == torch.float32 else 2.0 ** -8
+            assert float((a.double() - b).norm() / b.norm()) < tol, (what, apart)
+
+
+@pytest.mark.parametrize("dt", DT)
+@pytest.mark.parametrize("off", [0, 1])
+@pytest.mark.parametrize("f", [100, 4092, 4100, 8192, 14340, 16384, 16388, 1001])
+def test_polynomial_activation_at_odd_widths(ops, dt, f, off):
+    """Every form of the kernel (pieces of eight, four and one, the row kept or read twice), the bias at any float."""
+    z, b, c = _rand(5, f, dt=dt, seed=1), _rand(f + off, seed=2)[off:], _rand(4, seed=3)
+    u = z.double() + b.double()
+    norm = lambda t: t / torch.sqrt((t * t).mean(-1, keepdim=True) + 1e-4)
+    c64 = c.double()
+    want = c64[0] * norm(u) + c64[1] * norm(u ** 2) + c64[2] * norm(u ** 3) + c64[3]
+    got = ops.polynorm(z, b, c, 1e-4)
+    assert float((got.double() - want).norm() / want.norm()) < (2e-6 if dt == torch.float32 else 2.0 ** -8)
+
+
 @pytest.mark.parametrize("n,d,f,e,k", [(300, 128, 48, 16, 1), (700, 264, 72, 3, 2), (2048, 512, 256, 16, 1),
                                        (150, 64, 40, 128, 1)])
 def test_grouped_product_for_many_rows(ops, ref, n, d, f, e, k):
