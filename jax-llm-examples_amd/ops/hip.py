@@ -757,6 +757,7 @@ class HipOps:
         dr, dv = dq - nope_dim, w_uv.shape[0] // H
         if (q.dtype != torch.bfloat16 or latent_pages.dtype != torch.bfloat16 or w_uk.dtype != torch.bfloat16
                 or (meta is not None and meta.decode_bucket is not None) or not scale > 0
+                or (q.data_ptr() | latent_pages.data_ptr() | rope_pages.data_ptr()) % 16
                 or not self._query("jle_latent_expanded_supported", r, nope_dim, dr, dv, q.stride(0))):
             return None
         w = 0 if window is None else int(window)
@@ -1227,7 +1228,8 @@ class HipOps:
                                (ctx.state_phase, "state phases", (ctx.num_segments,))):
             self._chk(t, torch.int32, shape, what)
         dev = rows.device
-        if ctx.max_seg_len == 1 and self._query("jle_gated_delta_single_supported", H, G, dk, dv):
+        aligned = state.data_ptr() % 16 == 0  # (what the chunks and the single launch read 16 bytes at a time)
+        if ctx.max_seg_len == 1 and n == ctx.num_segments and aligned and self._query("jle_gated_delta_single_supported", H, G, dk, dv):
             out = torch.empty(n, H * dv, dtype=rows.dtype, device=dev)
             self._call("jle_gated_delta_single", _p(rows), self._is_bf16(rows), _p(gates), _p(a_log), _p(dt_bias),
                        _p(norm_weight), _p(out_gate), _p(state), _p(ctx.state_slots), _p(ctx.state_phase), _p(out), n, H, G,
@@ -1242,7 +1244,7 @@ class HipOps:
         beta, decay, kq = scratch[o: o + n * H], scratch[o + n * H: o + 2 * n * H], scratch[o + 2 * n * H: o + 2 * n * H + n * G]
         o_raw = scratch[o + 2 * n * H + n * G:]
         out = torch.empty(n, H * dv, dtype=rows.dtype, device=dev)
-        by_chunks = self._delta_chunks(ctx, H, G, dk, dv, dev)
+        by_chunks = self._delta_chunks(ctx, H, G, dk, dv, dev) if aligned else None
         (chunks, segs, nc, ns), ws = by_chunks if by_chunks is not None else ((None, None, 0, 0), None)
         self._call("jle_gated_delta", _p(rows), self._is_bf16(rows), _p(gates), _p(a_log), _p(dt_bias), _p(norm_weight),
                    _p(out_gate), _p(state), _p(ctx.cu_seqlens), _p(ctx.state_slots), _p(ctx.state_phase), _p(qn), _p(kn),
@@ -1647,7 +1649,7 @@ class HipOps:
                               f"whole tiles of 16 weight rows (32 with the fused activation), got {nout} x {k}")
         out = torch.empty(m, nout // 2 if swiglu else nout, dtype=torch.float32 if out_f32 else torch.bfloat16,
                           device=a.device)
-        wide = (offsets is not None and not out_f32 and a.numel() < 2 ** 31
+        wide = (offsets is not None and not out_f32 and a.numel() < 2 ** 31 and not (a.data_ptr() | b.data_ptr()) % 16
                 and self.stream_wide(m, g, -(-nout // 256)))
         self._call("jle_gemm_stream", _p(a), _p(b), _p(out), _p(offsets), _p(a_rows), _p(scale), int(swiglu),
                    int(out_f32), m, nout, k, g, m, int(wide))

@@ -121,3 +121,27 @@ def test_what_is_not_finite_reaches_no_token_before_it(where, what):
         assert float((a[f] - b[f]).norm() / b[f].norm()) < 2e-6  # (the same sums of float32 numbers in another order)
     if where != "memory":
         assert bool(torch.isfinite(got["chunks"][0][:bad]).all())
+
+
+@pytest.mark.parametrize("lens", [[100, 40], [1, 1, 1]])
+def test_a_memory_that_lies_off_its_16_bytes(lens):
+    """Goes token by token, as any memory did before there were chunks."""
+    from jax_llm_examples_amd.engine import get_ops
+    ops = get_ops(DEV)
+    ops.DELTA_CHUNKS_FROM, ops.DELTA_CHUNKS_LONG = 32, 1
+    H, G, dk, dv, R, N = 2, 1, 64, 32, len(lens), sum(lens)
+    g = torch.Generator(device=DEV).manual_seed(3)
+    rn = lambda *s: torch.randn(*s, generator=g, device=DEV)
+    args = [rn(N, 2 * G * dk + H * dv), rn(N, 2 * H), rn(H) - 1.0, rn(H), rn(dv), rn(N, H * dv)]
+    state = rn(R, 2, H, dv, dk)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)
+    got = []
+    for off in (0, 1):
+        ctx = types.SimpleNamespace(seg_lens=lens, num_segments=R, cu_seqlens=i32([0] + torch.tensor(lens).cumsum(0).tolist()),
+                                    state_slots=i32(list(range(R))), state_phase=i32([0] * R), scratch={}, max_seg_len=max(lens))
+        st = torch.empty(state.numel() + off, device=DEV)[off:].view(state.shape)
+        st.copy_(state)
+        o = ops.gated_delta(*args, H, G, dk, dv, EPS, FLOOR, st, ctx)
+        got.append((o, st))
+    for a, b in zip(*got):
+        assert float((a - b).norm() / b.norm()) < 2e-6  # (sums of float32 numbers in two orders)

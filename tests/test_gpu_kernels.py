@@ -1212,6 +1212,20 @@ def test_wide_tiles_of_the_weight_streaming_product(ops, counts, nout, k, swiglu
     assert torch.equal(*got)
 
 
+def test_rows_off_their_16_bytes_take_the_passes(ops):
+    """Rows that begin at 8 bytes, where the wide tiles want 16."""
+    from jax_llm_examples_amd.ops.layout import tile_
+    x, w = _rand(400, 256, dt=torch.bfloat16, seed=1), _rand(1, 64, 256, dt=torch.bfloat16, scale=0.1, seed=2)
+    tile_(w)
+    off = torch.tensor([0, 400], dtype=torch.int32, device=DEV)
+    elsewhere = torch.empty(400 * 256 + 4, dtype=torch.bfloat16, device=DEV)[4:].view(400, 256)
+    elsewhere.copy_(x)
+    ops.stream_wide = lambda *a: True
+    got = [ops.gemm_stream(t, w, offsets=off) for t in (x, elsewhere)]
+    del ops.stream_wide
+    assert torch.equal(*got)
+
+
 @pytest.mark.parametrize("dt", DT)
 @pytest.mark.parametrize("d", [48, 50, 2048, 4104, 8192])
 def test_shift_apart_from_its_norm(ops, dt, d):
