@@ -710,16 +710,29 @@ class HipOps:
         return out
 
     # Which steps form every head's keys and values (attention_expanded.hip) instead of staying in the latent's space
-    # (attention_latent.hip).  Forming a key's costs as much as about 160 (query, key) pairs save where the step's tokens
-    # alone do not fill the card; where a token has at most 8 gathered keys both take what their launches take or the
-    # expanded form less.  One call with all it launches, 32 heads, latent 512, page 16 (latent's space | expanded,
-    # microseconds): one prompt of 512 tokens 129 | 59, of 2,048 837 | 107; 64 prompts of 20 107 | 74, of 40 196 | 80;
-    # behind cached tokens: 128 behind 1,024 101 | 72, 64 behind 2,048 95 | 101 (63 pairs a key), 64 behind 8,192
-    # 233 | 347, 512 behind 8,192 1,405 | 363, 256 behind 16,384 1,523 | 658 (254 pairs a key).
+    # (attention_latent.hip).  From LATENT_EXPAND_PAIRS (query, key) pairs a gathered key on forming it gained at every size
+    # measured (between 80 and 160 it depends on how the latent's kernels fill the card).  With few gathered keys a token:
+    # up to LATENT_EXPAND_SMALL gathered keys times heads both take what their launches take or the expanded form less;
+    # beyond, forming the keys is what it takes, and pays with at most four a token or with LATENT_EXPAND_DENSE pairs a key.
+    # One call with all it launches, 32 heads, latent 512, page 16 (latent's space | expanded, microseconds): one prompt of
+    # 512 tokens 129 | 59, of 2,048 829 | 106; 64 prompts of 20 105 | 77, of 40 200 | 82; behind cached tokens, pairs a key
+    # in brackets: 128 behind 1,024 107 | 73 (121; 16 heads 79 | 65), 64 behind 2,048 96 | 100 (63), 128 behind 8,192
+    # 428 | 350 (127; 16 heads 239 | 296), 160 behind 8,192 829 | 352 (158), 512 behind 8,192 1,407 | 364 (497); 64 requests
+    # of 24 behind 168 189 | 176 (23), of 16 behind 48 89 | 78 (14), of 16 behind 112 111 | 124 (15); 200 of 8 behind 56
+    # 159 | 248 (8; 16 heads 93 | 162).
     # The gathered rows and the keys and values formed of them take no more than LATENT_EXPAND_BYTES.
     LATENT_EXPAND_ROWS = 8
+    LATENT_EXPAND_SMALL = 100_000
+    LATENT_EXPAND_DENSE = 20
     LATENT_EXPAND_PAIRS = 160
     LATENT_EXPAND_BYTES = 1 << 30
+
+    def expansion_pays(self, tokens: int, heads: int, rows: int, pairs: int) -> bool:
+        """Whether ``rows`` gathered keys with ``pairs`` (query, key) pairs are better formed than left in the latent."""
+        if pairs >= self.LATENT_EXPAND_PAIRS * rows:
+            return True
+        return rows <= self.LATENT_EXPAND_ROWS * tokens and (
+            rows * heads <= self.LATENT_EXPAND_SMALL or rows <= 4 * tokens or pairs >= self.LATENT_EXPAND_DENSE * rows)
 
     @staticmethod
     def expanded_plan(seg_lens, seg_starts, window: int):
@@ -768,7 +781,7 @@ class HipOps:
         if layout is None:
             layout = held[key] = self.expanded_plan(*self._segments(meta, token_segment, positions), w)
         spans, blocks, rows, pairs = layout
-        if (rows > self.LATENT_EXPAND_ROWS * n and pairs < self.LATENT_EXPAND_PAIRS * rows
+        if (not self.expansion_pays(n, H, rows, pairs)
                 or rows * (H * (nope_dim + dv) + r + dr) * 2 > self.LATENT_EXPAND_BYTES):
             return None
         table, ns = held.get(key + "_table"), len(spans)

@@ -48,3 +48,14 @@ def test_leave_for_shared_memory_is_asked_for_on_the_device_of_the_launch():
                 kept = line.strip().startswith("static ") and ("allowed" in line or "hipError_t" in line)
                 assert not kept, (path, line)
     assert asks == ["common.h"]
+
+
+@pytest.mark.parametrize("requests, tokens, behind, heads, formed", [
+    (1, 2048, 0, 32, True), (64, 20, 0, 32, True), (1, 512, 8192, 32, True), (64, 24, 168, 32, True), (64, 16, 48, 32, True),
+    (32, 8, 56, 16, True),                                                # (little of anything: the launches' time)
+    (200, 8, 56, 16, False), (200, 8, 56, 32, False), (128, 16, 112, 32, False),  # many short portions behind some context
+    (1, 64, 8192, 16, False), (8, 1, 2000, 16, False)])
+def test_which_steps_form_keys_and_values(requests, tokens, behind, heads, formed):
+    rows, pairs = HipOps.expanded_plan([tokens] * requests, [behind] * requests, 0)[2:]
+    ops = types.SimpleNamespace(**{k: v for k, v in vars(HipOps).items() if k.startswith("LATENT_EXPAND")})
+    assert HipOps.expansion_pays(ops, requests * tokens, heads, rows, pairs) == formed
