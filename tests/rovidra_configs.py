@@ -77,9 +77,25 @@ ROVIDRA_FAST = {
     },
 }
 
+# with the sizes that the kernels for keys and values formed once a step are made for (128 and 64 elements a key, 128 a
+# value): latents of two widths, readers of another layer's with other heads and a shorter and no window
+ROVIDRA_EXPANDED = {
+    "RE": {
+        "seed": 17, "architecture": "Rovidra", "vocab": 500, "width": 192, "embedding": {"scale": 13.0},
+        "norm": {"eps": 1e-5},
+        "layers": [
+            _layer(_mixer(2, 128, 64, 128, 64, 0.07, 50000.0, mask=90), ff=256),
+            _layer(_mixer(3, 128, 64, 128, 64, 0.08, 50000.0, mask=33, kv_from=0)),
+            _layer(_mixer(1, 128, 64, 128, 96, 0.06, 300.0, dims=32), ff=192),
+            _layer(_mixer(4, 128, 64, 128, 96, 0.07, 300.0, dims=32, mask=64, kv_from=2), ff=64),
+        ],
+    },
+}
+ALL = {**ROVIDRA, **ROVIDRA_FAST, **ROVIDRA_EXPANDED}
+
 
 def rovidra_config_json(name: str) -> dict:
-    return {k: v for k, v in {**ROVIDRA, **ROVIDRA_FAST}[name].items() if k != "seed"}
+    return {k: v for k, v in ALL[name].items() if k != "seed"}
 
 
 def write_rovidra(name: str, out_dir: str, dtype=torch.float32) -> str:
@@ -88,4 +104,4 @@ def write_rovidra(name: str, out_dir: str, dtype=torch.float32) -> str:
 
     top = rovidra_config_json(name)
     arch = get_architecture(top["architecture"])
-    return write_random_model(arch, arch.parse_config(top), out_dir, {**ROVIDRA, **ROVIDRA_FAST}[name]["seed"], dtype)
+    return write_random_model(arch, arch.parse_config(top), out_dir, ALL[name]["seed"], dtype)

@@ -309,6 +309,29 @@ def test_gpu_bfloat16_with_keys_shared_through_shared_memory(folders_bf16, monke
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("forced", [False, True])
+@pytest.mark.parametrize("mode", list(MODES))
+def test_gpu_bfloat16_with_keys_and_values_formed_once_a_step(tmp_path, monkeypatch, mode, forced):
+    """The sizes that steps of many tokens form every head's keys and values for: whole prompts over several blocks,
+    portions behind cached tokens, portions beside single tokens, latents borrowed from another layer, windows whose
+    pages were given back (and filled with NaN), by the rule and in every step that is not recorded."""
+    from jax_llm_examples_amd.ops.hip import HipOps
+
+    formed, inner = [], HipOps.latent_attention_expanded
+    def watched(self, *args, **kw):
+        out = inner(self, *args, **kw)
+        formed.append(out is not None)
+        return out
+    monkeypatch.setattr(HipOps, "latent_attention_expanded", watched)
+    if forced:
+        monkeypatch.setattr(HipOps, "LATENT_EXPAND_PAIRS", 0)
+    monkeypatch.setitem(LENGTHS, "RE", [300, 2, 141, 64, 97])
+    folder = write_rovidra("RE", str(tmp_path / "RE"), torch.bfloat16)
+    _check("RE", folder, "bfloat16", "cuda:0", mode, record=(mode != "tail"))
+    assert sum(formed) >= 4 and (all(formed) or not forced or mode in ("tail", "mixed"))
+
+
+@pytest.mark.gpu
 def test_gpu_float32_at_vector_sizes(tmp_path):
     folder = write_rovidra("RF", str(tmp_path / "RF"), torch.float32)
     for mode in ("portions", "mixed"):
