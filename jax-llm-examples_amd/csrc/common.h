@@ -52,6 +52,12 @@ struct Num<bf16_t> {
 // is computed from it stays in scalar registers and uniform loads take the scalar path).
 __device__ __forceinline__ int wave_index() { return __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)); }
 
+// 16 bytes a lane from base + byte_off straight into shared memory, a kilobyte from lds_addr on in the lanes' order (no
+// register waits for it: s_waitcnt vmcnt before it is read).
+__device__ __forceinline__ void load_to_lds16(const void* base, uint32_t byte_off, uint32_t lds_addr) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1\n" ::"v"(byte_off), "s"(base), "s"(lds_addr) : "memory");
+}
+
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);

@@ -11,8 +11,11 @@
 //                        segments of many tokens (below)
 //   gdr_single_kernel    all of it in one launch, for steps of single tokens
 //   gdr_out_kernel       o / sqrt(mean(o^2) + eps) * w * silu(gate), rounded to the run dtype
-// The memory lies [slot][half][H][dv][dk] (a column's rows together); a step reads the half `phase` and writes the other.  Every sum is formed
-// in an order that depends on the sizes alone, token after token: cutting a sequence into steps changes no bit.
+// The memory lies [slot][half][H][dv][dk] (a column's rows together); a step reads the half `phase` and writes the other.
+// What a token's result depends on beside its own sequence is rounding: the scan goes token after token, its sums over a
+// column in an order that follows from how many lanes share the column, which follows from the sizes and the number of
+// segments in the step; single tokens have a third order; and whether a segment goes by chunks, which begin at the step's
+// first token of it, is a question of its length and of the work of all such segments together.
 #include "common.h"
 
 using namespace jle;
@@ -794,7 +797,9 @@ template <typename T>
 int launch_single(const T* rows, const float* gates, const float* a_log, const float* dt_bias, const float* norm_w,
                   const T* gate, float* state, const int* state_slots, const int* state_phase, T* out, int R, int H, int G,
                   int dk, int dv, float eps, float floor, hipStream_t s) {
-#define JLE_SINGLE(DK_, CP_)                                                                                            hipLaunchKernelGGL((gdr_single_kernel<T, DK_, CP_>), dim3(R, H), dim3(512), 0, s, rows, gates, a_log, dt_bias, norm_w,                      gate, state, state_slots, state_phase, out, eps, floor, H, G, dv)
+#define JLE_SINGLE(DK_, CP_)                                                                                               \
+  hipLaunchKernelGGL((gdr_single_kernel<T, DK_, CP_>), dim3(R, H), dim3(512), 0, s, rows, gates, a_log, dt_bias, norm_w, \
+                     gate, state, state_slots, state_phase, out, eps, floor, H, G, dv)
   if (dk == 128) {
     if (dv <= 64) JLE_SINGLE(128, 1);
     else if (dv <= 128) JLE_SINGLE(128, 2);

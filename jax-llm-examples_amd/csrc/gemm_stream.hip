@@ -245,10 +245,6 @@ __global__ __launch_bounds__(WAVES * 64, 2) void gemm_stream_kernel(const bf16_t
 constexpr int kWideRows = 256;
 constexpr int kWideStage = kWideRows * BK * 2, kWideLds = 3 * kWideStage;  // bytes of a stage's rows, and of the ring
 
-__device__ __forceinline__ void load_to_lds16(const void* base, uint32_t byte_off, uint32_t lds_addr) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1\n" ::"v"(byte_off), "s"(base), "s"(lds_addr) : "memory");
-}
-
 template <bool SWIGLU, int NT>
 __device__ __forceinline__ void wide_block(const bf16_t* __restrict__ X, const bf16_t* __restrict__ We,
                                            bf16_t* __restrict__ Y, const int* __restrict__ a_rows,

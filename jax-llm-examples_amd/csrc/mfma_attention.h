@@ -1,5 +1,5 @@
-// What the attention kernels on the matrix cores share: operand types, sums over a column's lanes, loads straight into
-// shared memory.
+// What the attention kernels on the matrix cores share: operand types, sums over a column's lanes, where a page
+// tile's pieces lie in shared memory.
 #pragma once
 #include "common.h"
 
@@ -35,9 +35,5 @@ __device__ __forceinline__ float column_sum(float v) {
 // where piece p of key row r of a page tile lies: p ^ key_swizzle(r); the eight rows that eight neighbouring lanes read
 // (r % 4, r / 8 varying) then differ in the low three bits
 __device__ __forceinline__ int key_swizzle(int r) { return (r & 3) | ((r >> 3) << 2) | (((r >> 2) & 1) << 3); }
-
-__device__ __forceinline__ void load_to_lds16(const void* base, uint32_t byte_off, uint32_t lds_addr) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1\n" ::"v"(byte_off), "s"(base), "s"(lds_addr) : "memory");
-}
 
 }  // namespace jle

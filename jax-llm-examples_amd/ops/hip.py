@@ -1626,8 +1626,12 @@ class HipOps:
     def stream_wide(rows: int, groups: int, row_blocks: int) -> bool:
         """Which of ``gemm_stream.hip``'s kernels takes ``rows`` rows in ``groups`` groups (``row_blocks`` blocks of 256 rows
         of W a group): passes of 192 rows or wide tiles of 256.  A block fills a compute unit, so what counts is how many
-        rounds of blocks there are and how long one takes; measured per stage of 64 k, microseconds: passes 0.9 + 0.0037 a
-        row, tiles 0.95 + 0.003.  A group's rows scatter about their mean by its root.  Both sides measured (passes | tiles,
+        rounds of blocks there are on the 256 compute units and how long one takes; measured per stage of 64 k,
+        microseconds: passes 0.9 + 0.0037 a row, tiles 0.95 + 0.003.  A group's rows are taken to scatter about their mean by
+        its root: how they are shared out is known on the device only.  Over 99 sizes with even, so scattered and uneven
+        groups (0.3 to 1.7 of the mean; one with 40 % of the rows) the choice is 12 % faster than passes on the average and
+        2 % from the better of the two, at worst 25 % slower than passes (4 groups, one far fuller).  ``rows`` counts choices:
+        where some are of experts without rows, there are fewer.  Both sides measured (passes | tiles,
         us): 8 groups of 14,336 x 4,096 gate and up with 192 rows each 286 | 226, 256 368 | 309, 410 529 | 401, 700
         743 | 643; of 4,096 x 7,168 with 192 152 | 154, 410 275 | 163, 512 281 | 298, 700 302 | 329; of 8,192 x 2,048 gate
         and up with 410 152 | 121, 512 152 | 167; 16 of 16,384 x 5,120 with 160 523 | 541, 410 1,508 | 1,023, 700
@@ -1645,8 +1649,8 @@ class HipOps:
         return cost(256, 0.95, 0.003) < cost(192, 0.9, 0.0037)
 
     def gemm_stream(self, a, b, *, offsets=None, a_rows=None, scale=None, swiglu=False, out_f32=False, rows=None):
-        """bfloat16 product on MFMA for about a hundred rows per group, weights in the streaming layout and
-        read once per 192 rows of a group (see ``gemm_stream.hip``)."""
+        """bfloat16 product on MFMA for about a hundred rows per group and more, weights in the streaming layout and
+        read once per 192 rows of a group, or per tile of up to 256 (:meth:`stream_wide`; see ``gemm_stream.hip``)."""
         if b.dim() == 2:
             b = b.unsqueeze(0)
         g, nout, k = b.shape
@@ -2401,7 +2405,7 @@ class HipOps:
             routed = self.gemm_skinny(act, w_down, offsets=offsets, tiled=tiled)
         elif mfma and tiled and self.stream_supported(f2, d, True) and self.stream_supported(d, f2 // 2, False):
             # around a hundred rows per expert the cost is reading the weights, which this kernel reads once per
-            # 192 rows of an expert; with more rows it is still the faster one (measured up to 1024 per expert)
+            # 192 or 256 rows of an expert; with more rows it is still the faster one (measured up to 1024 per expert)
             act = self.gemm_stream(h, w_gate_up, offsets=offsets, a_rows=sorted_token, scale=sorted_gate, swiglu=True)
             routed = self.gemm_stream(act, w_down, offsets=offsets)
         elif mfma:
