@@ -1000,9 +1000,9 @@ class HipOps:
             return None
         rows, k = h.shape
         n = w.shape[0]
-        if (rows == 0 or w.shape[1] != k or k % 4 or not (h.is_cuda and w.is_cuda and h.is_contiguous() and w.is_contiguous())
-                or h.device.index != self._device_index or w.device.index != self._device_index
-                or h.data_ptr() % 16 or w.data_ptr() % 16 or n % (2 if act >= 0 else 1) or n == 0 or k == 0):
+        if (rows == 0 or n == 0 or k == 0 or w.shape[1] != k or k % 4 or n % (2 if act >= 0 else 1)
+                or not h.get_device() == w.get_device() == self._device_index
+                or not (h.is_contiguous() and w.is_contiguous()) or h.data_ptr() % 16 or w.data_ptr() % 16):
             return None
         if rows <= 4 or (rows <= 8 and n * k <= 1 << 25):
             return self.gemm_f32_rows(h, w, act)

@@ -9,8 +9,8 @@ from jax_llm_examples_amd.ops.hip import HipOps
 
 def tensor(rows, cols, device="cuda:0", dtype=torch.float32):
     """What the rule looks at of a matrix on a GPU."""
-    return types.SimpleNamespace(dtype=dtype, shape=(rows, cols), dim=lambda: 2, is_cuda=device.startswith("cuda"),
-                                 device=torch.device(device), is_contiguous=lambda: True, data_ptr=lambda: 4096)
+    return types.SimpleNamespace(dtype=dtype, shape=(rows, cols), dim=lambda: 2,
+                                 get_device=lambda: int(device[5:]) if device.startswith("cuda") else -1, is_contiguous=lambda: True, data_ptr=lambda: 4096)
 
 
 def rule(h, w, act=-1):
