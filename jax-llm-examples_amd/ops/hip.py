@@ -764,12 +764,13 @@ class HipOps:
         """The heads' outputs ``[N, H * value_dim]`` with every head's keys and values formed from the cached latents
         (``w_uk [H * nope, kv_rank]``, ``w_uv [H * value_dim, kv_rank]``), or ``None``: this step is better served in the
         latent's space (too few queries a key, sizes the kernel is not compiled for, float32, a scale that is not above
-        zero: this kernel scales a step's largest score, not its scores)."""
+        zero: this kernel scales a step's largest score, not its scores; pages that do not hold whole eights of tokens, of
+        which the latent's space has float32 probabilities)."""
         n, H, dq = q.shape
         r = latent_pages.shape[2]
         dr, dv = dq - nope_dim, w_uv.shape[0] // H
         if (q.dtype != torch.bfloat16 or latent_pages.dtype != torch.bfloat16 or w_uk.dtype != torch.bfloat16
-                or (meta is not None and meta.decode_bucket is not None) or not scale > 0
+                or (meta is not None and meta.decode_bucket is not None) or not scale > 0 or latent_pages.shape[1] % 8
                 or (q.data_ptr() | latent_pages.data_ptr() | rope_pages.data_ptr()) % 16
                 or not self._query("jle_latent_expanded_supported", r, nope_dim, dr, dv, q.stride(0))):
             return None

@@ -153,10 +153,13 @@ class LatentAttention(Mixer):
             q = ops.linear(cq, self.params["w_uq"])
             ops.rotate_heads_(q, H, dn, dr, ctx.positions, self.rotation)
             q = q.view(n, H, dn + dr)
-        # a step of many tokens: every head's keys and values formed once, and attended to as such
-        o = ops.latent_attention_expanded(q, dn, self.params["w_uk"], self.params["w_uv"], cache.pages["latent"],
-                                          cache.pages["rope_key"], cache.block_table, ctx.positions, ctx.token_segment,
-                                          self.window, self.softmax_scale, cache.attn_meta, sink=self.params.get("sink"))
+        # a step of many tokens: every head's keys and values formed once, and attended to as such (not at sizes whose
+        # attention has float32 probabilities: those formed keep them in bfloat16, like the matrix-core kernels)
+        o = None
+        if "latent_t" in cache.pages:
+            o = ops.latent_attention_expanded(q, dn, self.params["w_uk"], self.params["w_uv"], cache.pages["latent"],
+                                              cache.pages["rope_key"], cache.block_table, ctx.positions, ctx.token_segment,
+                                              self.window, self.softmax_scale, cache.attn_meta, sink=self.params.get("sink"))
         if o is None:
             # queries into the latent's space: [H, N, dn] x [H, dn, r]
             q_lat = ops.batched_linear(q[:, :, :dn].transpose(0, 1), self.params["w_uk"].view(H, dn, r))

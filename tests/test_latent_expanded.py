@@ -154,3 +154,39 @@ def test_every_scale_has_a_way(scale):
     out = ops.latent_attention_expanded(zeros(n, H, DN + DR), DN, zeros(H * DN, R), zeros(H * DV, R), zeros(n // ps, ps, R),
                                         zeros(n // ps, ps, DR), table, pos, seg, None, scale)
     assert (out is not None) == (scale > 0)
+
+
+@pytest.mark.parametrize("copies", [True, False])
+def test_a_mixer_without_the_transposed_latents_keeps_its_float32_probabilities(copies):
+    """At widths that the matrix-core kernels do not take (no transposed copies in the cache) attention over the latents is
+    float32 arithmetic; keys and values formed once a step are attended to with bfloat16 probabilities."""
+    import types
+    from jax_llm_examples_amd.parts.latent_attention import LatentAttention
+    calls, n = [], 3
+    named = lambda name, out=None: lambda *a, **k: (calls.append(name), out)[1]
+    ops = types.SimpleNamespace(
+        linear=lambda x, w: x @ w.T, batched_linear=lambda x, w, tokens_first=False: torch.zeros(n, 1, DV),
+        latent_prepare=named("prepare"), latent_attention=named("latent", torch.zeros(n, 1, 40)),
+        latent_attention_expanded=named("expanded", torch.zeros(n, DV)))
+    part = types.SimpleNamespace(
+        num_heads=1, nope_dim=DN, rope_dim=DR, value_dim=DV, kv_rank=40, own_latent=False, query_rank=None, rotation=None,
+        latent_norm_eps=0.0, q_rows=DN + DR, window=None, softmax_scale=1.0, output_gate=False, head_gate=False, w_out=None,
+        params={"w_in": torch.zeros(DN + DR, 8), "w_uk": torch.zeros(DN, 40), "w_uv": torch.zeros(DV, 40), "wo": torch.zeros(8, DV)})
+    pages = {"latent": None, "rope_key": None, **({"latent_t": None} if copies else {})}
+    cache = types.SimpleNamespace(pages=pages, writes=(), block_table=None, slot_mapping=None, attn_meta=None)
+    ctx = types.SimpleNamespace(ops=ops, positions=None, token_segment=None)
+    assert LatentAttention.forward(part, torch.zeros(n, 8), ctx, cache).shape == (n, 8)
+    assert calls == ["prepare", "expanded" if copies else "latent"]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("ps", [4, 8])
+def test_pages_that_the_matrix_cores_do_not_take_keep_their_float32_probabilities(ps):
+    dev, n, H, R = "cuda:0", 80, 2, 64
+    ops = HipOps(dev)
+    zeros = lambda *s: torch.zeros(*s, dtype=torch.bfloat16, device=dev)
+    table = torch.arange(n // ps, dtype=torch.int32, device=dev).view(1, -1)
+    pos, seg = torch.arange(n, dtype=torch.int32, device=dev), torch.zeros(n, dtype=torch.int32, device=dev)
+    out = ops.latent_attention_expanded(zeros(n, H, DN + DR), DN, zeros(H * DN, R), zeros(H * DV, R), zeros(n // ps, ps, R),
+                                        zeros(n // ps, ps, DR), table, pos, seg, None, 0.1)
+    assert (out is not None) == (ps == 8) == bool(ops._query("jle_latent_attention_mfma_supported", R, DN, DR, H * (DN + DR), ps))
