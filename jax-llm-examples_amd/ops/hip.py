@@ -1621,6 +1621,7 @@ class HipOps:
         return bool(self._query("jle_gemm_stream_supported", nout, k, int(swiglu)))
 
     WIDE_GROUP_ROWS = 176  # fewer rows a group on average: the weights' bytes take the time, each read once
+    WIDE_GROUPS = 8
 
     @staticmethod
     @functools.lru_cache(maxsize=4096)
@@ -1629,16 +1630,19 @@ class HipOps:
         of W a group): passes of 192 rows or wide tiles of 256.  A block fills a compute unit, so what counts is how many
         rounds of blocks there are on the 256 compute units and how long one takes; measured per stage of 64 k,
         microseconds: passes 0.9 + 0.0037 a row, tiles 0.95 + 0.003.  A group's rows are taken to scatter about their mean by
-        its root: how they are shared out is known on the device only.  Over 99 sizes with even, so scattered and uneven
-        groups (0.3 to 1.7 of the mean; one with 40 % of the rows) the choice is 12 % faster than passes on the average and
-        2 % from the better of the two, at worst 25 % slower than passes (4 groups, one far fuller).  ``rows`` counts choices:
+        its root: how they are shared out is known on the device only.  With fewer than WIDE_GROUPS groups one that is far
+        fuller than the others is what the launch takes, and is better cut in more pieces: 2 groups of 4,096 x 2,048 with 300
+        rows on average in even groups 43 | 38, with 90 and 510 42 | 53; 4 with 40 % of the rows in one 45 | 55.  Over 180
+        sizes of 8, 16 and 64 groups, even, from 0.3 to 1.7 of the mean, and one with 40 % of the rows, the choice is 15 %
+        faster than passes on the average and 2 % from the better of the two, at worst 13 % slower than passes (groups of
+        192 rows each, what a pass holds; beside that 8 %: one group far fuller at 192 on average).  ``rows`` counts choices:
         where some are of experts without rows, there are fewer.  Both sides measured (passes | tiles,
         us): 8 groups of 14,336 x 4,096 gate and up with 192 rows each 286 | 226, 256 368 | 309, 410 529 | 401, 700
         743 | 643; of 4,096 x 7,168 with 192 152 | 154, 410 275 | 163, 512 281 | 298, 700 302 | 329; of 8,192 x 2,048 gate
         and up with 410 152 | 121, 512 152 | 167; 16 of 16,384 x 5,120 with 160 523 | 541, 410 1,508 | 1,023, 700
         1,920 | 1,709."""
         mean = rows / groups
-        if mean < HipOps.WIDE_GROUP_ROWS:
+        if mean < HipOps.WIDE_GROUP_ROWS or groups < HipOps.WIDE_GROUPS:
             return False
 
         def cost(most, start, a_row):

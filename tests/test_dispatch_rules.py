@@ -59,3 +59,10 @@ def test_which_steps_form_keys_and_values(requests, tokens, behind, heads, forme
     rows, pairs = HipOps.expanded_plan([tokens] * requests, [behind] * requests, 0)[2:]
     ops = types.SimpleNamespace(**{k: v for k, v in vars(HipOps).items() if k.startswith("LATENT_EXPAND")})
     assert HipOps.expansion_pays(ops, requests * tokens, heads, rows, pairs) == formed
+
+
+@pytest.mark.parametrize("groups, rows, blocks, wide", [(8, 410, 56, True), (16, 410, 64, True), (8, 192, 56, True), (8, 170, 56, False),
+                                                        (2, 300, 32, False), (4, 300, 16, False), (4, 410, 56, False)])
+def test_few_groups_stay_with_passes(groups, rows, blocks, wide):
+    """Of few groups one may be far fuller than the others, and is then what the launch takes: it is cut in more pieces."""
+    assert HipOps.stream_wide(rows * groups, groups, blocks) == wide
