@@ -8,6 +8,7 @@ from __future__ import annotations
 
 import ctypes
 import functools
+import math
 from typing import Optional
 
 import torch
@@ -1191,20 +1192,39 @@ class HipOps:
         return out
 
     # Segments of DELTA_CHUNKS_FROM tokens and more go by chunks (gated_delta.hip), if one has DELTA_CHUNKS_LONG tokens or
-    # all of them together DELTA_CHUNKS_WORK (token, head) pairs: the first of the two kernels takes 19 us however little
-    # it has to do.  Scan | chunks, microseconds, 16 heads of 128 x 128: one prompt of 64 tokens 21 | 26, 96 30 | 29, 128
-    # 39 | 29, 512 144 | 50, 2,048 726 | 124; 8 prompts of 80 45 | 54, 25 of 80 166 | 139, 50 of 40 177 | 155.
+    # delta_chunks_pay expects less of it than of the scan.
     DELTA_CHUNK = 64
     DELTA_CHUNKS_FROM = 32
-    DELTA_CHUNKS_LONG = 96
-    DELTA_CHUNKS_WORK = 16384
+    DELTA_CHUNKS_LONG = 1024
     DELTA_CHUNK_BYTES = 2 << 30  # scratch of a step's chunks at most
+
+    @staticmethod
+    def delta_chunks_pay(lens, H: int, dk: int, dv: int) -> bool:
+        """Whether segments of these lengths are expected to take less by chunks than token after token.
+
+        The scan takes the longest segment's chain, 0.3 us a token, or, with many segments, what the (token, head) pairs of
+        all take together; chunks two launches and the longest segment's chain of chunks, and beside it (as the root of the
+        squares' sum: they overlap) what the segments' memories and the chunks take together, each chunk like a whole one of
+        64 tokens.  Over 235 sizes (2 to 64 heads, keys of 64 and 128, values of 16 to 256, equal, ragged and mixed lengths)
+        the choice takes 0.63 of the scan's time on the average, at worst 1.03, and 2.4 % more than the better of the two.
+        Scan | chunks, us, 16 heads of 128 x 128: one prompt of 64 tokens 30 | 36, 96 37 | 37, 128 47 | 38, 512 154 | 63,
+        2,048 754 | 149; 32 prompts of 32 103 | 122, 64 of 36 215 | 245, 50 of 40 201 | 195, 32 of 65 182 | 193, 16 of 80
+        111 | 106; 16 heads of 64 x 64: 128 of 32 132 | 203, 32 of 65 71 | 100, one of 2,048 612 | 104."""
+        longest, wide = max(lens), dv / 128
+        per = -(-longest // HipOps.DELTA_CHUNK)
+        chunks = sum(-(-ln // HipOps.DELTA_CHUNK) for ln in lens)
+        pairs = sum(lens) * H * wide
+        if dk > 64:
+            return (8 + math.hypot(28 + 2.6 * per, H * (len(lens) * 0.09 * wide + chunks * (0.02 + 0.12 * wide)))
+                    < max(10 + 0.33 * longest, 5 + 0.0054 * pairs))
+        return (8 + math.hypot(20 + 1.8 * per, H * (len(lens) * 0.05 * wide + chunks * (0.02 + 0.09 * wide)))
+                < max(10 + 0.29 * longest, 5 + 0.0031 * pairs))
 
     def _delta_chunks(self, ctx, H: int, G: int, dk: int, dv: int, device):
         """The chunks of the step's long segments ``(segment, first token, tokens)``, those segments ``(segment, first chunk,
         chunks)``, and whether there are others; ``None``: no segment goes by chunks."""
         long = [ln for ln in ctx.seg_lens if ln >= self.DELTA_CHUNKS_FROM]
-        if not long or max(long) < self.DELTA_CHUNKS_LONG and sum(long) * H < self.DELTA_CHUNKS_WORK:
+        if not long or max(long) < self.DELTA_CHUNKS_LONG and not self.delta_chunks_pay(long, H, dk, dv):
             return None
         kib = self._query("jle_gated_delta_chunk_kib", H, G, dk, dv)
         if kib < 0:

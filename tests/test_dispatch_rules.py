@@ -66,3 +66,13 @@ def test_which_steps_form_keys_and_values(requests, tokens, behind, heads, forme
 def test_few_groups_stay_with_passes(groups, rows, blocks, wide):
     """Of few groups one may be far fuller than the others, and is then what the launch takes: it is cut in more pieces."""
     assert HipOps.stream_wide(rows * groups, groups, blocks) == wide
+
+
+@pytest.mark.parametrize("lens, heads, dk, dv, pays", [
+    ([64], 16, 128, 128, False), ([256], 16, 128, 128, True), ([2048], 4, 64, 64, True), ([64] * 32, 16, 128, 128, True),
+    ([80] * 25, 16, 128, 128, True), ([32] * 64, 16, 128, 128, False), ([36] * 64, 64, 128, 128, False),
+    ([65] * 32, 16, 128, 128, False), ([32] * 128, 16, 64, 64, False), ([65] * 32, 32, 64, 128, False),
+    ([80] * 16, 32, 64, 128, False), ([36, 51, 53] * 20, 2, 128, 16, False), ([80] * 16, 8, 128, 256, True)])
+def test_which_segments_go_by_chunks(lens, heads, dk, dv, pays):
+    """A chunk of 64 places costs the same however many are filled: segments that fill theirs poorly stay with the scan."""
+    assert HipOps.delta_chunks_pay(lens, heads, dk, dv) == pays
