@@ -994,10 +994,13 @@ class HipOps:
     def _dense_float32(self, h, w, act: int = -1):
         """The float32 products with kernels of their own (see ``gemm_f32_dense.hip``), or None: the library's.
 
-        Up to 4 rows the product is a stream of the weights, which the kernel reads at 6.0 to 6.7 TB/s where the
-        library's reads them at 4.0 to 5.2 (16384 x 2048 33 -> 21 us, 2048 x 8192 23 -> 13, 2048 x 2048 11.5 -> 5.3, 64 x
-        36 5.6 -> 2.5); up to 8 rows while the weights are no more than 2^25 numbers (33 -> 29.5 us there; 14336 x 4096 at
-        8 rows is 50 us against the library's 45).  Many rows: see :meth:`split_ranges`.  In between neither gains."""
+        Up to 4 rows the product is a stream of the weights, which the kernel reads at 5.3 to 6.7 TB/s where the
+        library's reads them at 3.5 to 5.2 (one row, weights not in the caches: 16384 x 2048 33 -> 22 us, 2048 x 8192 23 -> 12,
+        2048 x 2048 12 -> 4.7, 36 x 64 5.2 -> 1.9; four rows 33 -> 26, 23 -> 13, 12 -> 5.5, 5.2 -> 2.4).  Of 5 to 8 rows it
+        takes weights of fewer than 2^24 numbers (8 rows of 2048 x 2048 12 -> 6.6), and of up to 2^25 with a k of 5,120 or
+        more (2048 x 8192 23 -> 16, 5120 x 5120 29 -> 25) or with the activation, which is a launch of its own behind the
+        library's; others it does not gain (8 rows of 8192 x 2048 15.8 against 17.6, 4096 x 4096 15.7 against 17.4).  Many
+        rows: see :meth:`split_ranges`.  In between neither gains."""
         if h.dtype != torch.float32 or w.dtype != torch.float32 or h.dim() != 2 or w.dim() != 2:
             return None
         rows, k = h.shape
@@ -1006,7 +1009,7 @@ class HipOps:
                 or not h.get_device() == w.get_device() == self._device_index
                 or not (h.is_contiguous() and w.is_contiguous()) or h.data_ptr() % 16 or w.data_ptr() % 16):
             return None
-        if rows <= 4 or (rows <= 8 and n * k <= 1 << 25):
+        if rows <= 4 or rows <= 8 and (n * k < 1 << 24 or n * k <= 1 << 25 and (k >= 5120 or act >= 0)):
             return self.gemm_f32_rows(h, w, act)
         ranges = self.split_ranges(rows, n, k, act >= 0, self._compute_units)
         if ranges:

@@ -76,3 +76,9 @@ def test_few_groups_stay_with_passes(groups, rows, blocks, wide):
 def test_which_segments_go_by_chunks(lens, heads, dk, dv, pays):
     """A chunk of 64 places costs the same however many are filled: segments that fill theirs poorly stay with the scan."""
     assert HipOps.delta_chunks_pay(lens, heads, dk, dv) == pays
+
+
+def test_few_rows_of_float32():
+    assert [rule(tensor(8, 2048), tensor(n, 2048)) for n in (2048, 8192)] == ["rows", None]
+    assert [rule(tensor(8, 4096), tensor(4096, 4096), act) for act in (-1, 0)] == [None, "rows"]
+    assert rule(tensor(5, 8192), tensor(2048, 8192)) == rule(tensor(4, 4096), tensor(14336, 4096)) == "rows"
