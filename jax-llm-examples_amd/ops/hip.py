@@ -1490,8 +1490,10 @@ class HipOps:
         TFLOP/s here, taken as 115 (its tiles fit some sizes better than others), and a pass of its own for the gate.
         Both sides measured, library | parts, us: 777 rows of 16,384 x 2,048 488 | 366, 1,554 785 | 631, 4,096 of 4,096 x
         2,048 460 | 378, 256 of 7,168 x 5,120 148 | 128, 777 of 5,120 x 5,120 323 | 297, 1,554 of 2,048 x 8,192 428 | 335;
-        left to the library: 140 of 16,384 x 2,048 118 | 139, 256 of 2,048 x 2,048 22 | 35, 64 of 7,168 x 5,120 49 | 76."""
-        if rows < 96 or k % 32 or nout % 8:
+        left to the library: 140 of 16,384 x 2,048 118 | 139, 256 of 2,048 x 2,048 22 | 35, 64 of 7,168 x 5,120 49 | 76, and
+        below 128 k without the gate, where the blocks' start and end are most of it: 777 of 16,384 x 96 30 | 33, 2,048 of
+        5,120 x 96 26 | 29 (gate and up of 1,024 of 7,168 x 96 35 | 18)."""
+        if rows < 96 or k % 32 or nout % 8 or (k < 128 and not gated):
             return 0
         tiles, stages = -(-rows // 128) * -(-nout // 128), k // 32
 

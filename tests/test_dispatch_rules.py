@@ -82,3 +82,9 @@ def test_few_rows_of_float32():
     assert [rule(tensor(8, 2048), tensor(n, 2048)) for n in (2048, 8192)] == ["rows", None]
     assert [rule(tensor(8, 4096), tensor(4096, 4096), act) for act in (-1, 0)] == [None, "rows"]
     assert rule(tensor(5, 8192), tensor(2048, 8192)) == rule(tensor(4, 4096), tensor(14336, 4096)) == "rows"
+
+
+def test_many_rows_of_float32_with_a_short_k():
+    sizes = [(777, 16384, 96), (2048, 5120, 96), (777, 16384, 2048), (1554, 2048, 8192), (512, 4096, 4096)]
+    assert [HipOps.split_ranges(*s, False, 256) > 0 for s in sizes] == [False, False, True, True, True]
+    assert HipOps.split_ranges(1024, 7168, 96, True, 256) == 1  # (the activation is a pass of its own behind the library's)
