@@ -239,18 +239,20 @@ __global__ __launch_bounds__(256) void latent_attention_kernel(
   }
 }
 
-// Merges the key ranges of a (token, head), 128 elements a wavefront, the ranges in their order; 16 ranges' pieces are
-// asked for before the first is added (a wavefront with all 512 elements and four ranges on their way: 16.4 us for 8
-// tokens of 16 heads and 33 ranges, 9.8 now).
-template <typename T>
+// Merges the key ranges of a (token, head), the ranges in their order: a wavefront 64 * E elements, U ranges' pieces asked
+// for before the first is added.  Many ranges come from few (token, head) pairs: E = 2, U = 16 (8 tokens of 16 heads and 33
+// ranges of 512 9.8 us, with E = 8, U = 4 16.4).  A few ranges come from many pairs or from short contexts: E = 8, U = 4 (64
+// tokens of 64 heads behind 60, attention and merge, 24.4 us, with E = 2, U = 16 31.5: pieces beyond the last range are
+// loaded too).
+template <typename T, int E, int U>
 __global__ __launch_bounds__(256) void latent_attention_merge_kernel(const float* __restrict__ ws_ml,
                                                                      const float* __restrict__ ws_o,
                                                                      T* __restrict__ out, int NH, int R, int splits,
                                                                      const float* __restrict__ sink, int H) {
   const int lane = threadIdx.x & 63;
-  const int parts = (R + 127) / 128;
+  const int parts = (R + 64 * E - 1) / (64 * E);
   const long long item = (long long)blockIdx.x * 4 + wave_index();
-  const int nh = (int)(item / parts), d0 = (int)(item % parts) * 128 + lane, d1 = d0 + 64;
+  const int nh = (int)(item / parts), d0 = (int)(item % parts) * 64 * E + lane;
   if (nh >= NH) return;
   const float* ml = ws_ml + (size_t)nh * splits * 2;
   float mx = -INFINITY;
@@ -268,18 +270,19 @@ __global__ __launch_bounds__(256) void latent_attention_merge_kernel(const float
     mx = fmaxf(mx, sk);
     l = expf(sk - mx);
   }
-  float acc0 = 0.f, acc1 = 0.f;
-  constexpr int U = 16;
+  float acc[E];
+#pragma unroll
+  for (int i = 0; i < E; ++i) acc[i] = 0.f;
   const float* rows = ws_o + (size_t)nh * splits * R;
   for (int s0 = 0; s0 < splits; s0 += U) {
-    float ms[U], ls[U], o0[U], o1[U];
+    float ms[U], ls[U], o[U][E];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int sp = min(s0 + u, splits - 1);  // (past the last: loaded again, not used)
       ms[u] = ml[sp * 2];
       ls[u] = ml[sp * 2 + 1];
-      o0[u] = d0 < R ? rows[(size_t)sp * R + d0] : 0.f;
-      o1[u] = d1 < R ? rows[(size_t)sp * R + d1] : 0.f;
+#pragma unroll
+      for (int i = 0; i < E; ++i) o[u][i] = d0 + 64 * i < R ? rows[(size_t)sp * R + d0 + 64 * i] : 0.f;
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
@@ -287,13 +290,26 @@ __global__ __launch_bounds__(256) void latent_attention_merge_kernel(const float
       if (ms[u] == -INFINITY || ms[u] != ms[u]) continue;  // a range without keys
       const float wgt = expf(ms[u] - mx);
       l += ls[u] * wgt;
-      acc0 = __builtin_fmaf(o0[u], wgt, acc0);
-      acc1 = __builtin_fmaf(o1[u], wgt, acc1);
+#pragma unroll
+      for (int i = 0; i < E; ++i) acc[i] = __builtin_fmaf(o[u][i], wgt, acc[i]);
     }
   }
   const float inv = bad ? __builtin_nanf("") : 1.0f / l;
-  if (d0 < R) Num<T>::store(out + (size_t)nh * R + d0, acc0 * inv);
-  if (d1 < R) Num<T>::store(out + (size_t)nh * R + d1, acc1 * inv);
+#pragma unroll
+  for (int i = 0; i < E; ++i)
+    if (d0 + 64 * i < R) Num<T>::store(out + (size_t)nh * R + d0 + 64 * i, acc[i] * inv);
+}
+
+template <typename T>
+void launch_latent_merge(hipStream_t s, const float* ws_ml, const float* ws_o, T* out, int NH, int R, int splits,
+                         const float* sink, int H) {
+  if (splits <= 8 && R > 128) {
+    hipLaunchKernelGGL((latent_attention_merge_kernel<T, 8, 4>), dim3((unsigned)(((long long)NH * ((R + 511) / 512) + 3) / 4)),
+                       dim3(256), 0, s, ws_ml, ws_o, out, NH, R, splits, sink, H);
+  } else {
+    hipLaunchKernelGGL((latent_attention_merge_kernel<T, 2, 16>), dim3((unsigned)(((long long)NH * ((R + 127) / 128) + 3) / 4)),
+                       dim3(256), 0, s, ws_ml, ws_o, out, NH, R, splits, sink, H);
+  }
 }
 
 // ------------------------------------------------------------------ on the matrix cores (bfloat16)
@@ -793,9 +809,7 @@ JLE_API int jle_latent_attention_mfma(const void* q_lat, const void* q, int q_ld
 #undef JLE_LATENT_MFMA
   JLE_LAUNCH_CHECK();
   if (splits > 1) {
-    dim3 gm((unsigned)(((long long)N * H * ((R + 127) / 128) + 3) / 4));
-    hipLaunchKernelGGL(latent_attention_merge_kernel<bf16_t>, gm, b, 0, s, ws_ml, ws_o, (bf16_t*)out, N * H, R, splits,
-                       sink, H);
+    launch_latent_merge(s, ws_ml, ws_o, (bf16_t*)out, N * H, R, splits, sink, H);
     JLE_LAUNCH_CHECK();
   }
   return 0;
@@ -888,7 +902,6 @@ JLE_API int jle_latent_attention(const void* q_lat, const void* q, int q_ld, int
   const long long items = (long long)N * H * splits;
   if (items > (1ll << 31) - 8) return JLE_BAD_ARG;
   dim3 g((unsigned)((items + 3) / 4)), b(256);
-  dim3 gm((unsigned)(((long long)N * H * ((R + 127) / 128) + 3) / 4));
   if (is_bf16) {
     hipLaunchKernelGGL(latent_attention_kernel<bf16_t>, g, b, 0, s, (const bf16_t*)q_lat, (const bf16_t*)q, q_ld, dn, dr,
                        (const bf16_t*)latent_pages, (const bf16_t*)rope_pages, (bf16_t*)out, positions, token_segment,
@@ -896,8 +909,7 @@ JLE_API int jle_latent_attention(const void* q_lat, const void* q, int q_ld, int
                        sink);
     JLE_LAUNCH_CHECK();
     if (splits > 1)
-      hipLaunchKernelGGL(latent_attention_merge_kernel<bf16_t>, gm, b, 0, s, ws_ml, ws_o, (bf16_t*)out, N * H, R,
-                         splits, sink, H);
+      launch_latent_merge(s, ws_ml, ws_o, (bf16_t*)out, N * H, R, splits, sink, H);
   } else {
     hipLaunchKernelGGL(latent_attention_kernel<float>, g, b, 0, s, (const float*)q_lat, (const float*)q, q_ld, dn, dr,
                        (const float*)latent_pages, (const float*)rope_pages, (float*)out, positions, token_segment,
@@ -905,8 +917,7 @@ JLE_API int jle_latent_attention(const void* q_lat, const void* q, int q_ld, int
                        sink);
     JLE_LAUNCH_CHECK();
     if (splits > 1)
-      hipLaunchKernelGGL(latent_attention_merge_kernel<float>, gm, b, 0, s, ws_ml, ws_o, (float*)out, N * H, R,
-                         splits, sink, H);
+      launch_latent_merge(s, ws_ml, ws_o, (float*)out, N * H, R, splits, sink, H);
   }
   JLE_LAUNCH_CHECK();
   return 0;
