@@ -404,12 +404,15 @@ JLE_API int jle_gemm_skinny(const void* X, const void* W, void* Y, const int* of
   if (K <= 0 || K % 8 || G < 1 || G > 65535 || (swiglu && Nout % 2)) return JLE_BAD_ARG;
   if (tiled && (K % 32 || Nout % 16 || (swiglu && (Nout / 2) % 16))) return JLE_BAD_ARG;
   if (max_rows <= 0 || max_rows > M) max_rows = M;
-  // Groups of eight rows and more on average: some have over 16, and a second block would read their weights again.
-  const bool fuller = offsets != nullptr && M >= 8 * G;
+  const int xrows = swiglu ? Nout / 2 : Nout;  // output columns to cover
+  // Groups of eight rows and more on average: some have over 16, and a second block would read their weights again.  Only
+  // where the row tiles alone are four blocks a compute unit: with fewer the second block runs beside the first (4 groups
+  // with 55 rows of 2,048 x 4,096, 512 tiles, 21.6 us with 16 rows of X a block, 26.7 with 32; with 132 of 2,048 x 2,048 16.9
+  // and 19.6; 8 groups with 121 of that, 1,024 tiles, 22 and 20).
+  const bool fuller = offsets != nullptr && M >= 8 * G && (long long)((xrows + 15) / 16) * G >= 1024;
   const int mt = (offsets == nullptr && max_rows > 32) ? 4 : (fuller || (offsets == nullptr && max_rows > 16)) ? 2 : 1;
   const int ytiles = (max_rows + 16 * mt - 1) / (16 * mt);
   if (ytiles > 65535) return JLE_BAD_ARG;
-  const int xrows = swiglu ? Nout / 2 : Nout;  // output columns to cover
   if (variant == 0) {
     // measured on MI355X at 1 to 64 rows (Scout's expert, attention and head shapes)
     const long long groups = offsets != nullptr ? (G < M ? G : M) : 1;

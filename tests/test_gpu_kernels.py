@@ -1161,10 +1161,11 @@ def test_weight_streaming_product_grouped_with_swiglu(ops, ref, n, d, f, e, k):
 
 @pytest.mark.parametrize("tiled", [False, True])
 @pytest.mark.parametrize("counts,nout,k", [([17, 0, 32, 33, 1], 96, 160), ([24], 4096 * 16, 64), ([40, 8], 80, 72),
-                                           ([16, 15, 64, 9], 8192, 96)])
+                                           ([16, 15, 64, 9], 8192, 96), ([40, 8] * 180, 80, 72),
+                                           ([17, 0, 32, 33, 1] * 70, 96, 160)])
 def test_weight_streaming_product_of_fuller_groups(ops, counts, nout, k, tiled):
-    """Groups of eight rows and more on average take 32 rows a block, and with many rows of W two row tiles: groups that
-    end at, before and behind 16 and 32 rows, empty ones between."""
+    """Groups of eight rows and more on average take 32 rows a block where the row tiles fill the card, and with many rows
+    of W two row tiles: groups that end at, before and behind 16 and 32 rows, empty ones between."""
     if tiled and (k % 32 or nout % 32):
         pytest.skip("no whole tiles")
     m, e = sum(counts), len(counts)
