@@ -711,29 +711,42 @@ class HipOps:
         return out
 
     # Which steps form every head's keys and values (attention_expanded.hip) instead of staying in the latent's space
-    # (attention_latent.hip).  From LATENT_EXPAND_PAIRS (query, key) pairs a gathered key on forming it gained at every size
-    # measured (between 80 and 160 it depends on how the latent's kernels fill the card).  With few gathered keys a token:
-    # up to LATENT_EXPAND_SMALL gathered keys times heads both take what their launches take or the expanded form less;
-    # beyond, forming the keys is what it takes, and pays with at most four a token or with LATENT_EXPAND_DENSE pairs a key.
-    # One call with all it launches, 32 heads, latent 512, page 16 (latent's space | expanded, microseconds): one prompt of
-    # 512 tokens 129 | 59, of 2,048 829 | 106; 64 prompts of 20 105 | 77, of 40 200 | 82; behind cached tokens, pairs a key
-    # in brackets: 128 behind 1,024 107 | 73 (121; 16 heads 79 | 65), 64 behind 2,048 96 | 100 (63), 128 behind 8,192
-    # 428 | 350 (127; 16 heads 239 | 296), 160 behind 8,192 829 | 352 (158), 512 behind 8,192 1,407 | 364 (497); 64 requests
-    # of 24 behind 168 189 | 176 (23), of 16 behind 48 89 | 78 (14), of 16 behind 112 111 | 124 (15); 200 of 8 behind 56
-    # 159 | 248 (8; 16 heads 93 | 162).
+    # (attention_latent.hip): those with LATENT_EXPAND_PAIRS (query, head) pairs a gathered key, where forming it gained by
+    # 40 % and more at every size measured, and those of which expansion_pays expects it.
     # The gathered rows and the keys and values formed of them take no more than LATENT_EXPAND_BYTES.
-    LATENT_EXPAND_ROWS = 8
-    LATENT_EXPAND_SMALL = 100_000
-    LATENT_EXPAND_DENSE = 20
-    LATENT_EXPAND_PAIRS = 160
+    LATENT_EXPAND_PAIRS = 40_000
     LATENT_EXPAND_BYTES = 1 << 30
 
-    def expansion_pays(self, tokens: int, heads: int, rows: int, pairs: int) -> bool:
-        """Whether ``rows`` gathered keys with ``pairs`` (query, key) pairs are better formed than left in the latent."""
-        if pairs >= self.LATENT_EXPAND_PAIRS * rows:
-            return True
-        return rows <= self.LATENT_EXPAND_ROWS * tokens and (
-            rows * heads <= self.LATENT_EXPAND_SMALL or rows <= 4 * tokens or pairs >= self.LATENT_EXPAND_DENSE * rows)
+    @staticmethod
+    def expansion_pays(tokens: int, heads: int, rank: int, rows: int, pairs: int, blocks: int, steps: int) -> bool:
+        """Whether ``rows`` gathered keys with ``pairs`` (query, key) pairs in ``blocks`` blocks, the longest of them ``steps``
+        steps of 64 keys, are expected to take less with every head's keys and values formed than in the latent's space.
+
+        The formed way costs its launches, the chain of the longest block's steps (1.46 us each), the pairs, and forming the
+        keys; the latent's way its launches and products (more with a wide latent), short chains only (its kernels share a long one
+        out), and pairs by the latent's width.  Fitted to 9,328 sizes of one call with all it launches (1 to 128 heads, latents
+        of 64 to 512, 1 to 128 portions of up to 4,096 tokens behind up to 8,000, windows, single tokens beside); what is
+        expected of the formed way is taken 10 % and 3 us longer.  The choice takes 0.69 of the latent's time on the average,
+        4 % more than the better of the two; in 16 of the sizes it is over 5 % slower than the latent's way, at worst 28 %.
+        Latent's space | formed, us, 32 heads, latent 512: one prompt of 512 tokens 129 | 59, of 2,048 829 | 106; 64 prompts of
+        20 105 | 77; 128 behind 8,192 428 | 350 (16 heads 239 | 296), 512 behind 8,192 1,407 | 364; 200 of 8 behind 56
+        159 | 248.  A head alone, latent 64: 174 behind 8,000 49 | 209."""
+        latent = (20 + rank / 32 + 1.2 * min(steps, 8) + 0.2 * steps + heads * pairs * (0.73 + 0.024 * rank) / 1e6
+                  + tokens * heads * (0.56 + 0.003 * rank) / 1e3)
+        formed = ((17 if heads >= 4 else 27)  # (the library's products of so few columns)
+                  + rank / 73 + 1.46 * steps + 0.23 * heads * pairs / 1e6 + heads * rows * (0.2 + 0.00044 * rank) / 1e3
+                  + heads * (0.19 * tokens + 0.8 * blocks) / 1e3)
+        return 1.1 * formed + 3 < latent
+
+    @staticmethod
+    def expanded_steps(seg_lens, seg_starts, window: int) -> int:
+        """The steps of 64 keys that the longest block of :meth:`expanded_plan` takes."""
+        most = 0
+        for ln, start in zip(seg_lens, seg_starts):
+            end = start + ln
+            first = max(0, start + (ln - 1) // 128 * 128 - window + 1) if window else 0  # (of the segment's last block)
+            most = max(most, (end - 1) // 64 - first // 64 + 1)
+        return most
 
     @staticmethod
     def expanded_plan(seg_lens, seg_starts, window: int):
@@ -781,9 +794,11 @@ class HipOps:
         key = f"latent_expanded_{w}"
         layout = held.get(key)
         if layout is None:
-            layout = held[key] = self.expanded_plan(*self._segments(meta, token_segment, positions), w)
-        spans, blocks, rows, pairs = layout
-        if (not self.expansion_pays(n, H, rows, pairs)
+            segments = self._segments(meta, token_segment, positions)
+            layout = held[key] = (*self.expanded_plan(*segments, w), self.expanded_steps(*segments, w))
+        spans, blocks, rows, pairs, steps = layout
+        if (pairs * H < self.LATENT_EXPAND_PAIRS * rows
+                and not self.expansion_pays(n, H, r, rows, pairs, len(blocks) // 4, steps)
                 or rows * (H * (nope_dim + dv) + r + dr) * 2 > self.LATENT_EXPAND_BYTES):
             return None
         table, ns = held.get(key + "_table"), len(spans)

@@ -50,15 +50,32 @@ def test_leave_for_shared_memory_is_asked_for_on_the_device_of_the_launch():
     assert asks == ["common.h"]
 
 
-@pytest.mark.parametrize("requests, tokens, behind, heads, formed", [
-    (1, 2048, 0, 32, True), (64, 20, 0, 32, True), (1, 512, 8192, 32, True), (64, 24, 168, 32, True), (64, 16, 48, 32, True),
-    (32, 8, 56, 16, True),                                                # (little of anything: the launches' time)
-    (200, 8, 56, 16, False), (200, 8, 56, 32, False), (128, 16, 112, 32, False),  # many short portions behind some context
-    (1, 64, 8192, 16, False), (8, 1, 2000, 16, False)])
-def test_which_steps_form_keys_and_values(requests, tokens, behind, heads, formed):
-    rows, pairs = HipOps.expanded_plan([tokens] * requests, [behind] * requests, 0)[2:]
-    ops = types.SimpleNamespace(**{k: v for k, v in vars(HipOps).items() if k.startswith("LATENT_EXPAND")})
-    assert HipOps.expansion_pays(ops, requests * tokens, heads, rows, pairs) == formed
+@pytest.mark.parametrize("requests, tokens, behind, heads, rank, formed", [
+    (1, 2048, 0, 32, 512, True), (64, 20, 0, 32, 512, True), (1, 512, 8192, 32, 512, True), (64, 24, 168, 32, 512, True),
+    (1, 2048, 0, 8, 256, True), (2, 954, 0, 8, 512, True),
+    (200, 8, 56, 16, 512, False), (200, 8, 56, 32, 512, False), (128, 16, 112, 32, 512, False),  # many short portions
+    (1, 64, 8192, 16, 512, False), (8, 1, 2000, 16, 512, False), (1, 128, 8192, 16, 512, False),
+    (1, 186, 4000, 2, 512, False), (1, 174, 8000, 1, 64, False), (1, 463, 8000, 1, 128, False),  # few heads: one long chain
+    (1, 88, 500, 32, 64, False), (2, 8, 0, 2, 256, False)])
+def test_which_steps_form_keys_and_values(requests, tokens, behind, heads, rank, formed):
+    segments = [tokens] * requests, [behind] * requests, 0
+    _, blocks, rows, pairs = HipOps.expanded_plan(*segments)
+    assert HipOps.expansion_pays(requests * tokens, heads, rank, rows, pairs, len(blocks) // 4,
+                                 HipOps.expanded_steps(*segments)) == formed
+
+
+@pytest.mark.parametrize("window", [0, 1, 63, 64, 500])
+def test_the_longest_block_of_a_step(window):
+    lens, starts = [1, 64, 129, 700, 5], [0, 63, 128, 1000, 777]
+    for one in [*zip(lens, starts), None]:
+        ln, st = ([one[0]], [one[1]]) if one else (lens, starts)
+        blocks, keys = HipOps.expanded_plan(ln, st, window)[1], []
+        for n0, nt in zip(blocks[::4], blocks[1::4]):
+            seg = next(i for i in range(len(ln)) if sum(ln[: i + 1]) > n0)
+            pos = st[seg] + n0 - sum(ln[:seg])
+            first = max(0, pos - window + 1) if window else 0
+            keys.append((pos + nt - 1) // 64 - first // 64 + 1)
+        assert max(keys) - 2 <= HipOps.expanded_steps(ln, st, window) <= max(keys)
 
 
 @pytest.mark.parametrize("groups, rows, blocks, wide", [(8, 410, 56, True), (16, 410, 64, True), (8, 192, 56, True), (8, 170, 56, False),

@@ -148,6 +148,7 @@ def test_every_scale_has_a_way(scale):
     """A scale of zero or below, which a configuration may name, stays in the latent's space."""
     dev, n, H, R, ps = "cuda:0", 80, 2, 64, 16
     ops = HipOps(dev)
+    ops.LATENT_EXPAND_PAIRS = 0
     zeros = lambda *s: torch.zeros(*s, dtype=torch.bfloat16, device=dev)
     table = torch.arange(n // ps, dtype=torch.int32, device=dev).view(1, -1)
     pos, seg = torch.arange(n, dtype=torch.int32, device=dev), torch.zeros(n, dtype=torch.int32, device=dev)
@@ -184,6 +185,7 @@ def test_a_mixer_without_the_transposed_latents_keeps_its_float32_probabilities(
 def test_pages_that_the_matrix_cores_do_not_take_keep_their_float32_probabilities(ps):
     dev, n, H, R = "cuda:0", 80, 2, 64
     ops = HipOps(dev)
+    ops.LATENT_EXPAND_PAIRS = 0
     zeros = lambda *s: torch.zeros(*s, dtype=torch.bfloat16, device=dev)
     table = torch.arange(n // ps, dtype=torch.int32, device=dev).view(1, -1)
     pos, seg = torch.arange(n, dtype=torch.int32, device=dev), torch.zeros(n, dtype=torch.int32, device=dev)

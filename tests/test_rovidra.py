@@ -314,7 +314,7 @@ def test_gpu_bfloat16_with_keys_shared_through_shared_memory(folders_bf16, monke
 def test_gpu_bfloat16_with_keys_and_values_formed_once_a_step(tmp_path, monkeypatch, mode, forced):
     """The sizes that steps of many tokens form every head's keys and values for: whole prompts over several blocks,
     portions behind cached tokens, portions beside single tokens, latents borrowed from another layer, windows whose
-    pages were given back (and filled with NaN), by the rule and in every step that is not recorded."""
+    pages were given back (and filled with NaN), where the rule says so and in every step that is not recorded."""
     from jax_llm_examples_amd.ops.hip import HipOps
 
     formed, inner = [], HipOps.latent_attention_expanded
@@ -328,7 +328,7 @@ def test_gpu_bfloat16_with_keys_and_values_formed_once_a_step(tmp_path, monkeypa
     monkeypatch.setitem(LENGTHS, "RE", [300, 2, 141, 64, 97])
     folder = write_rovidra("RE", str(tmp_path / "RE"), torch.bfloat16)
     _check("RE", folder, "bfloat16", "cuda:0", mode, record=(mode != "tail"))
-    assert sum(formed) >= 4 and (all(formed) or not forced or mode in ("tail", "mixed"))
+    assert not forced or sum(formed) >= 4 and (all(formed) or mode in ("tail", "mixed"))
 
 
 @pytest.mark.gpu
