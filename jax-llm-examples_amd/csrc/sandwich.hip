@@ -294,7 +294,10 @@ int launch_sandwich(const SandwichArgs& args, hipStream_t s) {
   constexpr int T1 = VEC == 1 ? 256 : 1024, C1 = 8 / VEC, T2 = VEC == 1 ? 512 : T1, C2 = VEC == 1 ? 16 : C1;
 #define JLE_SANDWICH_CASE(TH, C) \
   else if (a.D <= TH * C * VEC) hipLaunchKernelGGL((add_norm_shift_kernel<T, TH, C, VEC>), g, dim3(TH), 0, s, a)
-  if (a.D <= 256 * VEC) hipLaunchKernelGGL((add_norm_shift_kernel<T, 256, 1, VEC>), g, dim3(256), 0, s, a);
+  // (narrow rows by as few wavefronts: 4,096 rows of 192 with a gated branch and the shift by one 8.8 us, by four 15.8)
+  if (VEC < 8 && a.D <= 64 * VEC) hipLaunchKernelGGL((add_norm_shift_kernel<T, 64, 1, VEC < 8 ? VEC : 1>), g, dim3(64), 0, s, a);
+  else if (VEC < 8 && a.D <= 128 * VEC) hipLaunchKernelGGL((add_norm_shift_kernel<T, 128, 1, VEC < 8 ? VEC : 1>), g, dim3(128), 0, s, a);
+  JLE_SANDWICH_CASE(256, 1);
   JLE_SANDWICH_CASE(512, 1);
   JLE_SANDWICH_CASE(1024, 1);
   JLE_SANDWICH_CASE(T1, C1);
@@ -443,7 +446,9 @@ JLE_API int jle_add_norm_shift(const float* x, float* x_out, int delta_kind, con
   uintptr_t all = 0;
   for (const void* p : {(const void*)x, (const void*)x_out, y, g, (const void*)h_out, (const void*)hs_out, (const void*)state})
     all |= (uintptr_t)p;
-  const int vec = all % 16 ? 1 : D % 8 == 0 ? 8 : D % 4 == 0 ? 4 : 1;
+  // (pieces of eight leave narrow rows too few threads: 2,048 rows of 1,024, gated branch and shift, 18.9 us, of four 15.0;
+  // of float32 they are two loads: 256 rows of 2,048 8.3 and 7.6)
+  const int vec = all % 16 ? 1 : D % 8 == 0 && D > (is_bf16 ? 1024 : 2048) ? 8 : D % 4 == 0 ? 4 : 1;
   int rc;
   if (is_bf16)
     rc = vec == 8 ? launch_sandwich<bf16_t, 8>(a, s) : vec == 4 ? launch_sandwich<bf16_t, 4>(a, s) : launch_sandwich<bf16_t, 1>(a, s);

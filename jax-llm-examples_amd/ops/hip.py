@@ -442,8 +442,12 @@ class HipOps:
                    _p(h_a), _p(h_b), 1 if out_dtype == torch.bfloat16 else 0, n, d)
         return h_a, h_b
 
-    SHIFT_APART_ROWS = 256  # from so many rows on (a row a compute unit) the shift is a kernel of its own behind sums and
-    # statistics: with one kernel every row is formed twice (see sandwich.hip)
+    # From so many elements on, by what is added to the rows before (nothing, a tensor, a gated branch), the shift is a kernel
+    # of its own behind sums and statistics: with one kernel every row is formed twice (see sandwich.hip).  One kernel | two,
+    # us: gated, 256 rows of 4,096 9.8 | 14.5, 2,048 of 1,024 14.0 | 18.2, of 2,048 23.6 | 25.0, of 4,096 43.8 | 38.4, 4,096
+    # of 2,048 39.4 | 37.2; a tensor, 2,048 of 2,048 18.1 | 21.8, of 4,096 32.9 | 32.2; nothing, 4,096 of 2,048 21.7 | 24.2,
+    # of 6,148 87 | 73.
+    SHIFT_APART = (1 << 24, 1 << 23, 1 << 22)
 
     def add_norm_shift(self, x, delta, weight, eps: float, out_dtype, shift, ctx, do_norm: bool = True):
         """``x' = x + delta`` into a new tensor (``delta``: ``None``, a tensor, or a gated branch
@@ -475,7 +479,7 @@ class HipOps:
             self._chk(sw, torch.float32, (d,), "shift weight")
             self._chk(state, torch.float32, (state.shape[0], 2, d), "shift state")
             hs = torch.empty(n, d, dtype=out_dtype, device=x.device)
-            if n >= self.SHIFT_APART_ROWS:
+            if n * d >= self.SHIFT_APART[kind]:
                 stats = torch.empty(n, dtype=torch.float32, device=x.device)
         is_bf16 = 1 if out_dtype == torch.bfloat16 else 0
         self._call("jle_add_norm_shift", _p(x), _p(x_out), kind, _p(y), _p(yb), _p(g), _p(gb), _p(pw), float(peps),

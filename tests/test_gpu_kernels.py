@@ -1228,7 +1228,7 @@ def test_rows_off_their_16_bytes_take_the_passes(ops):
 
 
 @pytest.mark.parametrize("dt", DT)
-@pytest.mark.parametrize("d", [48, 50, 2048, 4104, 8192])
+@pytest.mark.parametrize("d", [48, 50, 320, 1024, 2048, 4104, 8192])
 def test_shift_apart_from_its_norm(ops, dt, d):
     """With many rows the shift is a kernel of its own behind the sums: the bits of the kernel that does both, at segments
     that begin and end within, at and across its blocks, with and without a branch output."""
@@ -1244,18 +1244,18 @@ def test_shift_apart_from_its_norm(ops, dt, d):
     v = [_rand(d, seed=4 + i) for i in range(5)]
     for delta in (None, y, GatedBranch(y, v[0], g, v[1], v[2], 1e-3)):
         got = []
-        for apart in (1 << 30, 1):
-            ops.SHIFT_APART_ROWS = apart
+        for apart in (1 << 62, 1):
+            ops.SHIFT_APART = (apart,) * 3
             state = _rand(6, 2, d, seed=9)
             got.append((*ops.add_norm_shift(x.clone(), delta, v[3], 1e-5, dt, (v[4], state), ctx), state))
-        del ops.SHIFT_APART_ROWS
+        del ops.SHIFT_APART
         for a, b, what in zip(*got, ("sums", "normed rows", "shifted rows", "state")):
             assert torch.equal(a, b), (what, float((a - b).abs().max()))
 
 
 @pytest.mark.parametrize("dt", DT)
 @pytest.mark.parametrize("off", [0, 1])
-@pytest.mark.parametrize("d", [100, 1026, 2050, 4092, 4098, 4100, 8188, 8190])
+@pytest.mark.parametrize("d", [63, 100, 126, 510, 512, 1000, 1026, 1032, 2050, 4092, 4098, 4100, 8188, 8190])
 def test_gated_branch_norm_and_shift_at_odd_widths(ops, dt, d, off):
     """Every form of the sandwich arrangement's kernel against its definition in 64 bits: rows in pieces of four and of one,
     one or several a thread, weights that lie at any float; with the shift in the same kernel and apart."""
@@ -1276,11 +1276,11 @@ def test_gated_branch_norm_and_shift_at_odd_widths(ops, dt, d, off):
     before = torch.cat([old[2, 0][None], torch.zeros(1, d, dtype=torch.float64, device=DEV), h[1:7], old[1, 1][None], h[8:19]])
     new = old.clone()
     new[2, 1], new[0, 0], new[1, 0] = h[0], h[7], h[19]
-    for apart in (1 << 30, 1):
-        ops.SHIFT_APART_ROWS = apart
+    for apart in (1 << 62, 1):
+        ops.SHIFT_APART = (apart,) * 3
         state = _rand(3, 2, d, seed=9)
         got = (*ops.add_norm_shift(x.clone(), GatedBranch(y, v[0], g, v[1], v[2], 1e-3), v[3], 1e-5, dt, (v[4], state), ctx), state)
-        del ops.SHIFT_APART_ROWS
+        del ops.SHIFT_APART
         for a, b, what in zip(got, (sums, h, h + (before - h) * v[4].double(), new), ("sums", "rows", "shifted", "state")):
             # float32 arithmetic, some ten roundings and two sums; rows rounded to the run dtype
             tol = 2e-6 if a.dtype == torch.float32 else 2.0 ** -8
