@@ -446,7 +446,7 @@ class HipOps:
     # of its own behind sums and statistics: with one kernel every row is formed twice (see sandwich.hip).  One kernel | two,
     # us: gated, 256 rows of 4,096 9.8 | 14.5, 2,048 of 1,024 14.0 | 18.2, of 2,048 23.6 | 25.0, of 4,096 43.8 | 38.4, 4,096
     # of 2,048 39.4 | 37.2; a tensor, 2,048 of 2,048 18.1 | 21.8, of 4,096 32.9 | 32.2; nothing, 4,096 of 2,048 21.7 | 24.2,
-    # of 6,148 87 | 73.
+    # of 4,096 41.3 | 41.6, of 6,148 89 | 77.
     SHIFT_APART = (1 << 24, 1 << 23, 1 << 22)
 
     def add_norm_shift(self, x, delta, weight, eps: float, out_dtype, shift, ctx, do_norm: bool = True):
