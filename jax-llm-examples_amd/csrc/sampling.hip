@@ -22,6 +22,8 @@ __device__ __forceinline__ float uniform_from_hash(uint32_t s, uint32_t c, uint3
   return ((float)(x >> 8) + 0.5f) * (1.0f / 16777216.0f);
 }
 
+typedef __attribute__((ext_vector_type(4))) float f32x4;
+
 struct Best {
   float v;
   int i;
@@ -194,7 +196,107 @@ JLE_API int jle_sample(const float* logits, const float* temperature, const int*
   return 0;
 }
 
-// ------------------------------------------------------------------ the same without a workspace argument
+// ------------------------------------------------------------------ greedy rows
+// The largest logit of every row (lowest index among equals) where no row samples: no temperatures, seeds and counters to
+// bring to the device first (three copies from the host and their waits, 100 us of a decode step of 640).  `copy`: the
+// logits are read anyway, so whoever must also keep them (the step's buffer is written again by the next step) has them
+// copied here and not by a launch of its own.  `out` may be host memory that the device reaches.
+//
+// What bounds it is latency, so everything a thread takes is on its way together (LOADS pieces of four).  A row of up to
+// kGreedyRow logits is one block's; a longer one is shared out over blocks of kGreedyChunk and finished by a second launch.
+// Microseconds with the copy: 64 rows of 32,000 8.6, 8 rows 7.6, one 6.3; one of 202,048 5.1 + 2.4, 8 6.0 + 3.3.  (The launches
+// for any kind of row, without a copy: 8.0 + 2.5, 8.0 + 2.9, 7.0 + 1.7, 8.2 + 3.0, 8.0 + 3.9.)
+constexpr int kGreedyThreads = 1024, kGreedyRow = kGreedyThreads * 32, kGreedyChunk = kGreedyThreads * 8;
+
+template <bool VEC, int LOADS>
+__global__ __launch_bounds__(kGreedyThreads) void greedy_kernel(const float* __restrict__ logits, float* __restrict__ copy,
+                                                                float* __restrict__ part_v, int* __restrict__ part_i,
+                                                                int* __restrict__ out, int V, int S) {
+  __shared__ Best smem[kGreedyThreads / 64];
+  const int row = blockIdx.y;
+  const float* x = logits + (size_t)row * V;
+  float* y = copy == nullptr ? nullptr : copy + (size_t)row * V;
+  constexpr int W = VEC ? 4 : 1, N = VEC ? LOADS : LOADS * 4;
+  const int first = blockIdx.x * (LOADS * 4 * kGreedyThreads) + (int)threadIdx.x * W;
+  float v[N][W];
+#pragma unroll
+  for (int u = 0; u < N; ++u) {
+    const int i = first + u * kGreedyThreads * W;
+    if (VEC) {
+      const f32x4 q = i < V ? *reinterpret_cast<const f32x4*>(x + i) : f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int j = 0; j < W; ++j) v[u][j] = q[j];
+    } else {
+      v[u][0] = i < V ? x[i] : 0.f;
+    }
+  }
+  Best b = {-INFINITY, 0x7fffffff};
+#pragma unroll
+  for (int u = 0; u < N; ++u) {
+    const int i = first + u * kGreedyThreads * W;
+    if (i >= V) continue;
+    if (y != nullptr) {
+      if (VEC) *reinterpret_cast<f32x4*>(y + i) = f32x4{v[u][0], v[u][W > 1 ? 1 : 0], v[u][W > 2 ? 2 : 0], v[u][W > 3 ? 3 : 0]};
+      else y[i] = v[u][0];
+    }
+#pragma unroll
+    for (int j = 0; j < W; ++j)
+      if (better(v[u][j], i + j, b.v, b.i)) b = {v[u][j], i + j};
+  }
+  b = block_best(b, smem);
+  if (threadIdx.x != 0) return;
+  if (S == 1) {
+    out[row] = b.i == 0x7fffffff ? 0 : b.i;
+  } else {
+    part_v[(size_t)row * S + blockIdx.x] = b.v;
+    part_i[(size_t)row * S + blockIdx.x] = b.i;
+  }
+}
+
+__global__ __launch_bounds__(64) void greedy_final_kernel(const float* __restrict__ part_v, const int* __restrict__ part_i,
+                                                          int* __restrict__ out, int S) {
+  __shared__ Best smem[1];
+  const int row = blockIdx.x;
+  Best b = {-INFINITY, 0x7fffffff};
+  for (int s = threadIdx.x; s < S; s += 64) {
+    const float v = part_v[(size_t)row * S + s];
+    const int i = part_i[(size_t)row * S + s];
+    if (better(v, i, b.v, b.i)) b = {v, i};
+  }
+  b = block_best(b, smem);
+  if (threadIdx.x == 0) out[row] = b.i == 0x7fffffff ? 0 : b.i;
+}
+
+// Blocks that share a row (0: bad sizes): the workspaces part_v and part_i hold M times as many entries (none for one).
+JLE_API int jle_greedy_blocks(int V) {
+  if (V <= 0) return 0;
+  return V <= kGreedyRow ? 1 : (V + kGreedyChunk - 1) / kGreedyChunk;
+}
+
+JLE_API int jle_greedy(const float* logits, float* copy, int* out, float* part_v, int* part_i, int M, int V, hipStream_t s) {
+  if (M <= 0) return 0;
+  if (V <= 0 || M > 65535) return JLE_BAD_ARG;
+  const int S = jle_greedy_blocks(V);
+  if (S > 1 && (part_v == nullptr || part_i == nullptr)) return JLE_BAD_ARG;
+  // (every row starts at 16 bytes if the arrays do and rows are whole pieces of four)
+  const bool vec = V % 4 == 0 && (((uintptr_t)logits | (uintptr_t)copy) & 15) == 0;
+#define GO(VEC, LOADS)                                                                                                       \
+  hipLaunchKernelGGL((greedy_kernel<VEC, LOADS>), dim3(S, M), dim3(kGreedyThreads), 0, s, logits, copy, part_v, part_i, out, V, S)
+  if (S > 1) {
+    if (vec) GO(true, 2); else GO(false, 2);
+  } else {
+    if (vec) GO(true, 8); else GO(false, 8);
+  }
+#undef GO
+  JLE_LAUNCH_CHECK();
+  if (S > 1) {
+    hipLaunchKernelGGL(greedy_final_kernel, dim3(M), dim3(64), 0, s, part_v, part_i, out, S);
+    JLE_LAUNCH_CHECK();
+  }
+  return 0;
+}
+
+// ------------------------------------------------------------------ jle_sample without a workspace argument
 // The blocks' choices of the two-stage kernels go into an array that is part of the loaded code object, so the
 // call allocates nothing (see jle.h).  Every GPU that runs this library holds its own copy of the array, at an
 // address of its own, until the process ends.

@@ -68,6 +68,7 @@ class StepContext:
     max_seg_len: int
     max_context_len: int
     page_size: int
+    every_row: bool = False  # logits_indices is known to be 0, 1, .. N - 1
     # ``tap(part, name, value)``: installed by whoever wants to watch a step (tests, benchmarks).  A part may
     # hand it named intermediate values; if the tap returns something, the part goes on with that instead.
     tap: Optional[Any] = None
@@ -182,9 +183,9 @@ def fill_step(layout: StepLayout, flat: np.ndarray, cache, entries: Sequence[Ste
 
 
 def context_over(layout: StepLayout, flat: torch.Tensor, cache, ops, dtype, device, *, seg_lens, seg_starts,
-                 max_context_len: int, bucket: Optional[int], tap=None) -> StepContext:
+                 max_context_len: int, bucket: Optional[int], tap=None, every_row: bool = False) -> StepContext:
     """The :class:`StepContext` whose arrays are views of ``flat`` (on the device the model runs on).
-    ``bucket``: see :class:`GroupContext`."""
+    ``bucket``: see :class:`GroupContext`; ``every_row``: see :class:`StepContext`."""
     R = layout.num_segments
     d = lambda name: layout.view(flat, name)
     groups = []
@@ -198,7 +199,7 @@ def context_over(layout: StepLayout, flat: torch.Tensor, cache, ops, dtype, devi
         cu_seqlens=d("cu_seqlens"), context_lens=d("context_lens"), state_slots=d("state_slots"),
         state_phase=d("state_phase"),
         logits_indices=d("logits_indices"), groups=groups, seg_lens=seg_lens, seg_starts=seg_starts,
-        max_seg_len=max(seg_lens), max_context_len=max_context_len, page_size=cache.page_size, tap=tap)
+        max_seg_len=max(seg_lens), max_context_len=max_context_len, page_size=cache.page_size, every_row=every_row, tap=tap)
 
 
 def build_context(ops, dtype, device, cache, entries: Sequence[StepEntry], vocab_size: int,
@@ -215,5 +216,5 @@ def build_context(ops, dtype, device, cache, entries: Sequence[StepEntry], vocab
     dev = host.to(device, non_blocking=False) if torch.device(device).type != "cpu" else host
     longest = max(s + n for s, n in zip(seg_starts, seg_lens))
     return context_over(layout, dev, cache, ops, dtype, device, seg_lens=seg_lens, seg_starts=seg_starts,
-                        max_context_len=longest, bucket=decode_bucket(longest) if max(seg_lens) == 1 else None,
-                        tap=tap)
+                        max_context_len=longest, bucket=decode_bucket(longest) if max(seg_lens) == 1 else None, tap=tap,
+                        every_row=all(len(e.tokens) == 1 and len(e.want) == 1 for e in entries))

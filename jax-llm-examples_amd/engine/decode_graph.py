@@ -44,7 +44,7 @@ class _Recording:
         self.turn = 0
         self.device_buf = torch.zeros(total, dtype=torch.int32, device=model.device)
         self.ctx = context_over(self.layout, self.device_buf, cache, ops, model.dtype, model.device,
-                                seg_lens=[1] * R, seg_starts=None, max_context_len=bucket, bucket=bucket)
+                                seg_lens=[1] * R, seg_starts=None, max_context_len=bucket, bucket=bucket, every_row=True)
         self.graph = None
         self.logits = None
 

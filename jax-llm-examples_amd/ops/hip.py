@@ -29,7 +29,7 @@ def _ret_mode(retention) -> int:
 _vp, _i, _f, _ll = ctypes.c_void_p, ctypes.c_int, ctypes.c_float, ctypes.c_longlong
 
 _SIGNATURES = {
-    "jle_embed": [_vp, _vp, _i, _vp, _i, _i, _vp],
+    "jle_embed": [_vp, _vp, _i, _f, _vp, _i, _i, _vp],
     "jle_add_rmsnorm": [_vp, _i, _vp, _vp, _vp, _i, _vp, _i, _vp, _f, _vp, _i, _vp, _i, _i, _vp, _vp, _i, _vp],
     "jle_add_residual": [_vp, _vp, _i, _ll, _vp],
     "jle_gather_rows": [_vp, _vp, _vp, _i, _i, _vp],
@@ -54,6 +54,7 @@ _SIGNATURES = {
     "jle_gemm_f32_split": [_vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _vp],
     "jle_gemm_f32_stream": [_vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _vp],
     "jle_sample": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _vp],
+    "jle_greedy": [_vp, _vp, _vp, _vp, _vp, _i, _i, _vp],
     "jle_attention_mfma_supported": [_i, _i, _i, _i],
     "jle_attention_prefill": [_vp, _vp, _vp, _vp, _vp, _vp, _i, _vp, _i, _i, _vp, _i, _i, _i, _f, _i, _i, _i, _i, _vp,
                               _i, _vp, _f, _vp],
@@ -139,6 +140,12 @@ class ExpertSum:
         self.shape = torch.Size((n, d))
         self.dtype = routed.dtype
 
+    def rows(self, ops, idx) -> "ExpertSum":
+        """The sum of the chosen rows only, still in pieces."""
+        own = None if self.own is None else tuple(ops.gather_rows(t, idx) for t in self.own)
+        return ExpertSum(self.routed, ops.gather_rows(self.inv[: self.shape[0] * self.k].view(-1, self.k), idx).view(-1), self.k,
+                         None if self.shared is None else ops.gather_rows(self.shared, idx), idx.numel(), self.shape[1], own)
+
 
 class PendingNorm:
     """The rows a norm will give, not computed yet: the residual, the branch output still to be added to it, the
@@ -182,7 +189,7 @@ def _bind(path: str):
             fn.argtypes = args
             fn.restype = ctypes.c_int
     for name, args in (("jle_attention_mfma_supported", [_i, _i, _i, _i]),  # queries, not launches: no stream
-                       ("jle_gemm_stream_supported", [_i, _i, _i]), ("jle_gemm_f32_stream_supported", [_i, _i, _i]),
+                       ("jle_greedy_blocks", [_i]), ("jle_gemm_stream_supported", [_i, _i, _i]), ("jle_gemm_f32_stream_supported", [_i, _i, _i]),
                        ("jle_latent_attention_mfma_supported", [_i, _i, _i, _i, _i]),
                        ("jle_latent_expanded_supported", [_i, _i, _i, _i, _i]), ("jle_attention_group_waves", []),
                        ("jle_mlstm_chunked_supported", [_i, _i]), ("jle_mlstm_chunk_tokens", []),
@@ -283,12 +290,13 @@ class HipOps:
         return t
 
     # ------------------------------------------------------------------ embedding, norms
-    def embed(self, token_ids, table):
+    def embed(self, token_ids, table, multiplier: float = 1.0):
+        """``table[token] * multiplier``, float32."""
         n, (v, d) = token_ids.numel(), table.shape
         self._chk(token_ids, torch.int32, (n,), "token ids")
         self._chk(table, None, (v, d), "embedding table")
         out = torch.empty(n, d, dtype=torch.float32, device=table.device)
-        self._call("jle_embed", _p(token_ids), _p(table), self._is_bf16(table), _p(out), n, d)
+        self._call("jle_embed", _p(token_ids), _p(table), self._is_bf16(table), float(multiplier), _p(out), n, d)
         return out
 
     def embed_pair(self, token_ids, prev_token_ids, table, pair_table, buckets: int, mul_prev: int, mul_cur: int):
@@ -2499,3 +2507,20 @@ class HipOps:
         self._call("jle_sample", _p(logits), _p(temperature), _p(top_k), _p(seeds), _p(counters), _p(out), _p(part_v),
                    _p(part_i), m, v, int(any_top_k))
         return out
+
+    def greedy(self, logits, copy: bool = False):
+        """The largest logit's id of every row (lowest among equals) as a list, where no row samples, and with ``copy`` the
+        logits once more.  Waits for the stream: the kernel writes the ids into host memory that this call allocates, so
+        they are there when it has run."""
+        m, v = logits.shape
+        self._chk(logits, torch.float32, None, "logits")
+        kept = torch.empty_like(logits) if copy else None
+        if m == 0:
+            return [], kept
+        out = torch.empty(m, dtype=torch.int32, pin_memory=True)
+        blocks = self._query("jle_greedy_blocks", v)
+        parts = (None, None) if blocks == 1 else (torch.empty(m * blocks, dtype=torch.float32, device=logits.device),
+                                                  torch.empty(m * blocks, dtype=torch.int32, device=logits.device))
+        self._call("jle_greedy", _p(logits), _p(kept), _p(out), _p(parts[0]), _p(parts[1]), m, v)
+        torch.cuda.current_stream(self._device_index).synchronize()
+        return out.tolist(), kept

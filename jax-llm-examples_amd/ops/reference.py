@@ -39,8 +39,9 @@ class ReferenceOps:
     name = "reference"
 
     # ------------------------------------------------------------------ embedding
-    def embed(self, token_ids: torch.Tensor, table: torch.Tensor) -> torch.Tensor:
-        return table[token_ids.long()].float()
+    def embed(self, token_ids: torch.Tensor, table: torch.Tensor, multiplier: float = 1.0) -> torch.Tensor:
+        """``table[token] * multiplier``, float32."""
+        return table[token_ids.long()].float() * float(multiplier)
 
     def embed_pair(self, token_ids, prev_token_ids, table, pair_table, buckets: int, mul_prev: int, mul_cur: int):
         """``table[token] + pair_table[(prev * mul_prev + token * mul_cur) mod buckets]``, and row ``buckets`` of the

@@ -47,10 +47,7 @@ class TokenEmbedding(Embedding):
         if self.sinusoid_base is not None:
             return ctx.ops.embed_sinusoid(token_ids, ctx.positions, self.params["weight"],
                                           1.0 if self.multiplier is None else self.multiplier, self.rates)
-        x = ctx.ops.embed(token_ids, self.params["weight"])
-        if self.multiplier is not None:
-            x.mul_(self.multiplier)
-        return x
+        return ctx.ops.embed(token_ids, self.params["weight"], 1.0 if self.multiplier is None else self.multiplier)
 
 
 @register_embedding("token_pair_embedding")

@@ -118,6 +118,7 @@ class DecoderModel:
         if ctx.logits_indices.numel() == 0:
             residual.value(ctx)
             return torch.empty(0, self.plan.vocab_size, dtype=torch.float32, device=ctx.device)
-        picked = residual.rows(ctx, ctx.logits_indices)
+        # (where every row is wanted, in its place, as in a step of single tokens, there is nothing to pick)
+        picked = residual if ctx.every_row else residual.rows(ctx, ctx.logits_indices)
         h, _ = self.final_norm.forward(picked, ctx)
         return self.lm_head.forward(h, ctx, self.embed)

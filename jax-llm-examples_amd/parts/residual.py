@@ -12,6 +12,11 @@ from __future__ import annotations
 import torch
 
 
+def pick_rows(ops, t, idx):
+    """The chosen rows of a branch output; one that is not formed yet stays in its pieces."""
+    return t.rows(ops, idx) if hasattr(t, "rows") else ops.gather_rows(t, idx)
+
+
 class GatedBranch:
     """A branch output that is not formed yet: ``rmsnorm((y + y_bias) * sigmoid(gate + gate_bias)) * weight``
     per row (statistics over the row, ``eps`` inside the root, float32).  ``y`` and ``gate`` are ``[N, hidden]``
@@ -36,7 +41,7 @@ class BranchSum:
         self.shape, self.dtype = a.shape, a.dtype
 
     def rows(self, ops, idx) -> "BranchSum":
-        return BranchSum(ops.gather_rows(self.a, idx), None if self.b is None else ops.gather_rows(self.b, idx))
+        return BranchSum(pick_rows(ops, self.a, idx), None if self.b is None else pick_rows(ops, self.b, idx))
 
 
 class ScaledSum:
@@ -69,7 +74,7 @@ class ScaledSum:
         return ScaledSum(self.terms + [(y, factor)])
 
     def rows(self, ops, idx) -> "ScaledSum":
-        return ScaledSum([(ops.gather_rows(t, idx), f) for t, f in self.terms], self.vector)
+        return ScaledSum([(pick_rows(ops, t, idx), f) for t, f in self.terms], self.vector)
 
 
 class Residual:
@@ -124,6 +129,10 @@ class Residual:
             p = ctx.ops.defer_norm(self.x, self.pending, weight, eps, ctx.dtype)
             self.pending, self._deferred = None, p
             return p, (p if want32 else None)
+        if hasattr(self.pending, "gate") and not want32:  # (the kernel that knows it writes the sum into a new array)
+            self._x, h, _ = ctx.ops.add_norm_shift(self.x, self.pending, weight, eps, ctx.dtype, None, ctx)
+            self.pending = None
+            return h, None
         h, h32 = ctx.ops.add_rmsnorm(self.x, self.pending, weight, eps, ctx.dtype, want32)
         self.pending = None
         return h, h32
@@ -166,10 +175,7 @@ class Residual:
         self._settle_injected(ctx)
         r = Residual(ctx.ops.gather_rows(self.x, idx))
         if self.pending is not None:
-            if hasattr(self.pending, "rows"):
-                r.pending = self.pending.rows(ctx.ops, idx)
-            else:
-                r.pending = ctx.ops.gather_rows(self.pending, idx)
+            r.pending = pick_rows(ctx.ops, self.pending, idx)
         return r
 
 
@@ -231,7 +237,7 @@ class StreamsResidual:
         r = StreamsResidual(ctx.ops.gather_rows(self.xs.view(n, s * d), idx).view(-1, s, d))
         if self.pending is not None:
             p = self.pending
-            r.pending = StreamUpdate(ctx.ops.gather_rows(p.y, idx), p.mix, p.outw)
+            r.pending = StreamUpdate(pick_rows(ctx.ops, p.y, idx), p.mix, p.outw)
         return r
 
 

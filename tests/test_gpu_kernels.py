@@ -1404,3 +1404,54 @@ def test_streaming_layout_gives_the_same_results_bit_for_bit(ops):
         w2t = w2.clone()
         tile_(w2t)
         assert torch.equal(ops.lm_head(h, w2), ops.lm_head(h, w2t, tiled=True))
+
+
+@pytest.mark.parametrize("m,v", [(1, 1), (3, 512), (2, 8191), (5, 8192), (64, 8200), (2, 32767), (3, 32768), (2, 32772), (2, 32773), (1, 202048)])
+@pytest.mark.parametrize("off", [0, 1])
+def test_greedy_rows_and_their_copy(ops, m, v, off):
+    """Edges of what a block takes of a long row (8,192) and of the longest row that one block takes alone (32,768), rows that do not start at 16
+    bytes; equal maxima, rows without any number and rows of the lowest value."""
+    g = torch.Generator().manual_seed(v)
+    flat = torch.empty(m * v + off, device=DEV)
+    logits = flat[off:].view(m, v)
+    logits.copy_(torch.randn(m, v, generator=g))
+    logits[0, v // 3] = logits[0, v - 1] = 9.0
+    if m > 1:
+        logits[1] = float("-inf")
+    if m > 2:
+        logits[2] = float("nan")
+        logits[2, v // 2] = -7.0
+    want = [v // 3] + [0] * (m > 1) + [v // 2] * (m > 2) + torch.argmax(logits[3:].cpu(), -1).tolist()
+    got, kept = ops.greedy(logits, copy=True)
+    assert got == want and torch.equal(kept.view(torch.int32), logits.contiguous().view(torch.int32))
+    assert ops.greedy(logits) == (want, None)
+
+
+@pytest.mark.parametrize("n,d", [(1, 64), (3, 2048), (2, 2056), (5, 100), (70, 5120)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_embedding_rows_times_a_number(ops, ref, n, d, dtype):
+    table = torch.randn(90, d, generator=torch.Generator().manual_seed(d)).to(DEV, dtype)
+    tok = torch.randint(0, 90, (n,), generator=torch.Generator().manual_seed(n)).int().to(DEV)
+    for mul in (1.0, 45.254834):
+        assert torch.equal(ops.embed(tok, table, mul), ref.embed(tok, table, mul))
+
+
+@pytest.mark.parametrize("k,shared,own", [(1, True, False), (2, False, False), (2, True, True), (6, True, False)])
+def test_chosen_rows_of_an_expert_sum_stay_in_pieces(ops, k, shared, own):
+    from jax_llm_examples_amd.ops.hip import ExpertSum
+
+    g = torch.Generator().manual_seed(k)
+    n, d = 9, 2048
+    bf = lambda *s: torch.randn(*s, generator=g).to(DEV, torch.bfloat16)
+    inv = torch.randperm(n * k, generator=g).int()
+    if own:
+        inv[::3] = -1
+    lazy = ExpertSum(bf(n * k, d), inv.to(DEV), k, bf(n, d) if shared else None, n, d,
+                     (bf(n, d), torch.rand(n, k, generator=g).to(DEV)) if own else None)
+    idx = torch.tensor([7, 0, 7, 3], dtype=torch.int32, device=DEV)
+    x = torch.randn(n, d, generator=g).to(DEV)
+    w = torch.rand(d, generator=g).to(DEV)
+    a, b = ops.gather_rows(x, idx), x.clone()
+    got, _ = ops.add_rmsnorm(a, lazy.rows(ops, idx), w, 1e-5, torch.bfloat16)
+    want, _ = ops.add_rmsnorm(b, lazy, w, 1e-5, torch.bfloat16)
+    assert torch.equal(a, b[idx.long()]) and torch.equal(got, want[idx.long()])
