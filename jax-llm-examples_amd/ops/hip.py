@@ -65,6 +65,7 @@ _SIGNATURES = {
     "jle_gemm_grouped": [_vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _vp],
     "jle_gemm_skinny": [_vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _i, _i, _vp, _i, _i, _i, _i, _vp, _vp,
                         _vp],
+    "jle_gemm_few": [_vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _i, _i, _vp, _i, _i, _i, _vp],
     "jle_add_norm_shift": [_vp, _vp, _i, _vp, _vp, _vp, _vp, _vp, _f, _i, _vp, _f, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp,
                            _vp, _i, _i, _i, _vp, _vp],
     "jle_polynorm": [_vp, _i, _vp, _vp, _f, _vp, _i, _i, _i, _vp],
@@ -1044,11 +1045,14 @@ class HipOps:
         return None
 
     def linear(self, h, w, out_dtype=None):
-        """``h @ w.T``: through the BLAS library; a few bfloat16 rows through the weight-streaming kernel, which is as
-        fast there or faster and much cheaper to launch, and few or many float32 rows through kernels of their own."""
+        """``h @ w.T``: through the BLAS library; up to a few tens of bfloat16 rows (:meth:`_few`), and few or many float32
+        rows, through kernels of their own."""
         h = self._rows(h)
         out = self._dense_float32(h, w)
         if out is not None:
+            return out if out_dtype is None or out_dtype == out.dtype else out.to(out_dtype)
+        if self._few(h, w):
+            out = self.gemm_few(h, w)
             return out if out_dtype is None or out_dtype == out.dtype else out.to(out_dtype)
         if (h.dtype == torch.bfloat16 and h.shape[0] <= self.SKINNY_LINEAR_ROWS and w.dim() == 2
                 and w.dtype == torch.bfloat16 and w.shape[1] % 8 == 0 and h.is_contiguous() and w.is_contiguous()):
@@ -1056,6 +1060,27 @@ class HipOps:
             return out if out_dtype is None or out_dtype == out.dtype else out.to(out_dtype)
         out = torch.matmul(h, w.t())
         return out if out_dtype is None or out_dtype == out.dtype else out.to(out_dtype)
+
+    FEW_ROWS = 64
+
+    def _few_fits(self, a, *weights) -> bool:
+        """Whether the sizes and addresses are ones that ``gemm_few.hip`` takes (weights ``[*, rows, K]``)."""
+        k = a.shape[1]
+        return (a.dtype == torch.bfloat16 and k > 0 and k % 64 == 0 and a.numel() < 2 ** 31 and a.data_ptr() % 16 == 0
+                and all(w.dtype == torch.bfloat16 and w.shape[-1] == k and w.shape[-2] * k < 2 ** 31 and w.data_ptr() % 16 == 0
+                        for w in weights))
+
+    def _few(self, h, w) -> bool:
+        """Whether ``h @ w.T`` goes through the kernel for a few rows: up to FEW_ROWS of them, wherever it takes the sizes.
+        The weight-streaming kernel, which cuts a long row of few weight rows into slices, keeps its up to 8 rows of those
+        (2,048 x 8,192, 8 rows: 10.7 against 12.3 us).  Of the library's it takes all: at worst 3 % behind (7,168 x 5,120, 64
+        rows: 23.9 against 23.3 us), else up to half of its time (figures: ``gemm_few.hip``)."""
+        if h.dim() != 2 or w.dim() != 2 or h.shape[0] > self.FEW_ROWS or not self._few_fits(h, w):
+            return False
+        if h.shape[0] <= self.SKINNY_LINEAR_ROWS and w.shape[1] >= 4 * w.shape[0]:
+            return False
+        return (h.is_contiguous() and w.is_contiguous() and h.get_device() == w.get_device() == self._device_index
+                and not (torch.is_grad_enabled() and (h.requires_grad or w.requires_grad)))
 
     def linear_float32(self, h, w):
         """``h @ w.T`` with the float32 sums as they are: a library product where there are many rows."""
@@ -1070,6 +1095,8 @@ class HipOps:
         h = self._rows(h)
         if bias is None:
             return self.linear(h, w), None
+        if self._few(h, w):
+            return self.gemm_few(h, w, out_f32=True), bias
         if (h.dtype == torch.bfloat16 and h.shape[0] <= self.SKINNY_LINEAR_ROWS and w.dtype == torch.bfloat16
                 and w.shape[1] % 8 == 0 and h.is_contiguous() and w.is_contiguous()):
             return self.gemm_skinny(h, w, out_f32=True), bias
@@ -1085,7 +1112,8 @@ class HipOps:
         h = self._rows(h)
         act = self._ACTS[activation]
         if h.dtype == torch.bfloat16 and h.shape[0] <= self.SKINNY_DENSE_ROWS and h.shape[1] % 8 == 0:
-            return self.gemm_skinny(h, w_gate_up, swiglu=1 + act)  # (the activation in the product's epilogue)
+            product = self.gemm_few if self._few(h, w_gate_up) else self.gemm_skinny
+            return product(h, w_gate_up, swiglu=1 + act)  # (the activation in the product's epilogue)
         out = self._dense_float32(h, w_gate_up, act)
         return self.silu_mul(torch.matmul(h, w_gate_up.t()), activation) if out is None else out
 
@@ -1649,6 +1677,38 @@ class HipOps:
                    split_tiles, split, _p(ws), _p(self._slice_tickets))
         return out
 
+    def gemm_few(self, a, b, *, offsets=None, a_rows=None, scale=None, swiglu=0, relu2=False, out_f32=False, rows=None,
+                 tiled=False, b_last=None, tiled_last=False, tiles=0):
+        """bfloat16 product on MFMA for up to a few tens of rows a group (see ``gemm_few.hip``).  ``swiglu`` 1 or 2: silu or
+        gelu_tanh of the gate times up; ``relu2``: of every rounded sum ``max(., 0)^2``.  ``b_last``: one more group behind
+        ``b``'s, its matrix a tensor of its own (``offsets`` then has an entry more)."""
+        if b.dim() == 2:
+            b = b.unsqueeze(0)
+        g, nout, k = b.shape
+        if b_last is not None:
+            self._chk(b_last, torch.bfloat16, (nout, k), "the last group's matrix")
+            if offsets is None or offsets.numel() != g + 2:
+                raise KernelError("a last group with a matrix of its own needs offsets for one group more")
+            g += 1
+        m = rows if rows is not None else (a_rows.numel() if a_rows is not None else a.shape[0])
+        self._chk(a, torch.bfloat16, None, "A")
+        self._chk(b, torch.bfloat16, None, "B")
+        if a.shape[1] != k:
+            raise KernelError(f"inner sizes differ: A {tuple(a.shape)}, B {tuple(b.shape)}")
+        if a.numel() >= 2 ** 31:
+            raise KernelError("the product of a few rows addresses its rows with 32 bits")
+        out = torch.empty(m, nout // 2 if swiglu else nout, dtype=torch.float32 if out_f32 else torch.bfloat16, device=a.device)
+        slots = m if offsets is not None and g > m and m <= self.SLOT_ROWS else 0  # (no more groups have rows than there are rows)
+        self._call("jle_gemm_few", _p(a), _p(b), _p(out), _p(offsets), _p(a_rows), _p(scale), int(swiglu), int(relu2),
+                   int(out_f32), m, nout, k, g, m, int(tiled), _p(b_last), int(tiled_last), slots, tiles)
+        return out
+
+    def _few_experts(self, a, b, *, b_last=None, **kw):
+        """The product of a step's few rows a group: the kernel for a few rows where it takes the sizes, else the
+        weight-streaming one."""
+        product = self.gemm_few if self._few_fits(a, b, *(() if b_last is None else (b_last,))) else self.gemm_skinny
+        return product(a, b, b_last=b_last, **kw)
+
     def gemm_grouped(self, a, b, *, offsets=None, a_rows=None, scale=None, swiglu=False, out_f32=False, rows=None,
                      tiled=False):
         """bfloat16 product on MFMA for many rows, grouped by ``offsets`` (see ``gemm_grouped.hip``)."""
@@ -1736,8 +1796,14 @@ class HipOps:
             return torch.matmul(h, w.t()) if out is None else out
         if h.shape[1] % 8 == 0:
             streams = tiled and self.stream_supported(w.shape[0], w.shape[1], False)
-            # measured on a 202048 x 5120 head: up to 16 rows the skinny kernel is at the speed of reading the
-            # weights; beyond, the kernel that shares the rows between wavefronts through shared memory
+            # (kernel for a few rows | the one it takes them from, us: 32,000 x 2,048, 1 row 23.1 | 23.5, 8 23.6 | 26.1,
+            # 16 24.2 | 34.8, 32 27.8 | 33.8, 64 32.5 | 34.1; 202,048 x 5,120, 1 row 305 | 310, 8 317 | 323, 16 336 | 383,
+            # 32 387 | 397, 64 463 | 400)
+            if (h.shape[0] <= (self.FEW_ROWS if w.numel() < 1 << 28 else 32) and h.is_contiguous() and w.is_contiguous()
+                    and self._few_fits(h, w) and (not tiled or w.shape[0] % 16 == 0)):
+                return self.gemm_few(h, w, out_f32=True, tiled=tiled)
+            # sizes that it does not take, and more rows: the skinny kernel up to 16; beyond, the kernel that shares the rows
+            # between wavefronts through shared memory
             if h.shape[0] <= (16 if streams else self.SKINNY_MAX_ROWS):
                 return self.gemm_skinny(h, w, out_f32=True, tiled=tiled)
             if streams:
@@ -2273,10 +2339,10 @@ class HipOps:
         offsets, sorted_token, sorted_weight, inv = grouping
         own = (h, weights.contiguous()) if identity else None
         if ride:  # (a token's row of the shared expert is noted in ``inv`` behind its choices')
-            act = self.gemm_skinny(h, w_up, offsets=offsets, a_rows=sorted_token, swiglu=True, tiled=tiled,
-                                   b_last=shared_weights[0], rows=m + n)
-            routed = self.gemm_skinny(act, w_down, offsets=offsets, scale=sorted_weight, tiled=tiled,
-                                      b_last=shared_weights[1])
+            act = self._few_experts(h, w_up, offsets=offsets, a_rows=sorted_token, swiglu=True, tiled=tiled,
+                                    b_last=shared_weights[0], rows=m + n)
+            routed = self._few_experts(act, w_down, offsets=offsets, scale=sorted_weight, tiled=tiled,
+                                       b_last=shared_weights[1])
             return ExpertSum(routed, inv, k + 1, None, n, d, own)
         shared = None
         if offsets.numel() == e + 2:  # (grouped with the shared expert's rows: they are the sum's last piece all the same)
@@ -2289,7 +2355,7 @@ class HipOps:
         def product(x, w, nout, kdim, fused=False, **kw):
             kw.update(offsets=offsets)
             if mfma and m <= 2 * self.SKINNY_MAX_ROWS:
-                return self.gemm_skinny(x, w, swiglu=fused, tiled=tiled, **kw)
+                return self._few_experts(x, w, swiglu=fused, tiled=tiled, **kw)
             if mfma and tiled and self.stream_supported(nout, kdim, fused):
                 return self.gemm_stream(x, w, swiglu=fused, **kw)
             if mfma:
@@ -2307,6 +2373,8 @@ class HipOps:
 
         if swiglu:
             act = product(h, w_up, 2 * f, d, fused=True, a_rows=sorted_token)
+        elif mfma and m <= 2 * self.SKINNY_MAX_ROWS and self._few_fits(h, w_up):  # (the activation of the rounded sums too)
+            act = self.gemm_few(h, w_up, offsets=offsets, a_rows=sorted_token, tiled=tiled, relu2=True)
         else:
             act = self.relu2(product(h, w_up, f, d, a_rows=sorted_token))
         routed = product(act, w_down, d, f, scale=sorted_weight)
@@ -2448,18 +2516,18 @@ class HipOps:
             grouping = self.moe_align(expert_ids.contiguous(), gates.contiguous(), e, extra_group=fuse)
         offsets, sorted_token, sorted_gate, inv = grouping
         if fuse:
-            act = self.gemm_skinny(h, w_gate_up, offsets=offsets, a_rows=sorted_token, scale=sorted_gate, swiglu=True,
-                                   tiled=tiled, b_last=shared_weights[0], rows=m + n)
-            both = self.gemm_skinny(act, w_down, offsets=offsets, tiled=tiled, b_last=shared_weights[1])
+            act = self._few_experts(h, w_gate_up, offsets=offsets, a_rows=sorted_token, scale=sorted_gate, swiglu=True,
+                                    tiled=tiled, b_last=shared_weights[0], rows=m + n)
+            both = self._few_experts(act, w_down, offsets=offsets, tiled=tiled, b_last=shared_weights[1])
             return ExpertSum(both[:m], inv, k, both[m:], n, d)
         if shared is None and shared_weights is not None:
             shared = self.linear(self.swiglu_linear(h, shared_weights[0]), shared_weights[1])
         if grouping[0].numel() != e + 1:  # (made with the extra group: the kernels below do not know of it)
             offsets, sorted_token, sorted_gate = offsets[: e + 1], sorted_token[:m], sorted_gate[:m]
         if mfma and m <= 2 * self.SKINNY_MAX_ROWS:  # few rows: the cost is streaming the chosen experts' weights
-            act = self.gemm_skinny(h, w_gate_up, offsets=offsets, a_rows=sorted_token, scale=sorted_gate, swiglu=True,
-                                   tiled=tiled)
-            routed = self.gemm_skinny(act, w_down, offsets=offsets, tiled=tiled)
+            act = self._few_experts(h, w_gate_up, offsets=offsets, a_rows=sorted_token, scale=sorted_gate, swiglu=True,
+                                    tiled=tiled)
+            routed = self._few_experts(act, w_down, offsets=offsets, tiled=tiled)
         elif mfma and tiled and self.stream_supported(f2, d, True) and self.stream_supported(d, f2 // 2, False):
             # around a hundred rows per expert the cost is reading the weights, which this kernel reads once per
             # 192 or 256 rows of an expert; with more rows it is still the faster one (measured up to 1024 per expert)

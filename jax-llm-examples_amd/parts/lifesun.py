@@ -25,7 +25,7 @@ class LifesunArchitecture:
     # what of csrc/ a model of this design calls (a first run on a machine without a built library compiles these)
     kernel_sources = ("elementwise.hip", "parallel.hip", "terms.hip", "retention.hip", "gated_unit.hip",
                       "attention_heads.hip", "attention_conv.hip", "attention_span.hip", "attention_generic.hip",
-                      "attention_mfma.hip", "attention_f32.hip", "gemm_skinny.hip", "gemm_stream.hip",
+                      "attention_mfma.hip", "attention_f32.hip", "gemm_skinny.hip", "gemm_few.hip", "gemm_stream.hip",
                       "gemm_grouped.hip", "gemm_generic.hip", "gemm_f32_dense.hip", "sampling.hip")
 
     def parse_config(self, top: Mapping[str, Any]) -> LifesunConfig:

@@ -22,7 +22,7 @@ class RovidraArchitecture:
     names = ("Rovidra", "rovidra")
     # what of csrc/ a model of this design calls (a first run on a machine without a built library compiles these)
     kernel_sources = ("elementwise.hip", "sandwich.hip", "attention_latent.hip",
-                      "attention_expanded.hip", "gemm_skinny.hip", "gemm_stream.hip",
+                      "attention_expanded.hip", "gemm_skinny.hip", "gemm_few.hip", "gemm_stream.hip",
                       "gemm_grouped.hip", "gemm_generic.hip", "gemm_f32_dense.hip", "sampling.hip")
 
     def parse_config(self, top: Mapping[str, Any]) -> RovidraConfig:

@@ -28,7 +28,8 @@ class SudilornArchitecture:
     # what of csrc/ a model of this design calls (a first run on a machine without a built library compiles these)
     kernel_sources = ("elementwise.hip", "scaled.hip", "gated_delta.hip", "attention_heads.hip", "attention_conv.hip",
                       "attention_generic.hip", "attention_mfma.hip", "attention_f32.hip", "attention_prep.hip",
-                      "moe_route.hip", "moe_choose.hip", "gemm_skinny.hip", "gemm_stream.hip", "gemm_grouped.hip",
+                      "moe_route.hip", "moe_choose.hip", "gemm_skinny.hip", "gemm_few.hip", "gemm_stream.hip",
+                      "gemm_grouped.hip",
                       "gemm_generic.hip", "gemm_f32.hip", "gemm_f32_dense.hip", "parallel.hip", "sampling.hip")
 
     def parse_config(self, top: Mapping[str, Any]) -> SudilornConfig:

@@ -1455,3 +1455,79 @@ def test_chosen_rows_of_an_expert_sum_stay_in_pieces(ops, k, shared, own):
     got, _ = ops.add_rmsnorm(a, lazy.rows(ops, idx), w, 1e-5, torch.bfloat16)
     want, _ = ops.add_rmsnorm(b, lazy, w, 1e-5, torch.bfloat16)
     assert torch.equal(a, b[idx.long()]) and torch.equal(got, want[idx.long()])
+
+
+def _few_bound(a, b):
+    """What float32 sums of exact products may be off by, a k of any order: (k + 2) roundings of 2^-24 of the sum of their sizes."""
+    return (a.shape[1] + 2) * 2.0 ** -24 * (a.double().abs() @ b.double().abs().t()) + 1e-30
+
+
+@pytest.mark.parametrize("m,nout,k", [(1, 64, 64), (8, 70, 192), (16, 33, 128), (17, 96, 320), (33, 500, 256), (64, 130, 5120),
+                                       (5, 1000, 8192), (3, 80, 1088), (64, 8192, 128), (24, 4112, 64), (63, 16, 448)])
+@pytest.mark.parametrize("tiles", [0, 11, 12, 14, 21, 22, 24, 41, 42, 44])
+def test_product_of_a_few_rows(ops, m, nout, k, tiles):
+    """Tiles with one row and one column over, lines fewer than wavefronts, every tile of the choice."""
+    from jax_llm_examples_amd.ops.layout import can_tile, tile_
+
+    g = torch.Generator().manual_seed(m + nout)
+    a = torch.randn(m, k, generator=g).to(DEV, torch.bfloat16)
+    b = torch.randn(nout, k, generator=g).to(DEV, torch.bfloat16)
+    want = a.double() @ b.double().t()
+    got = ops.gemm_few(a, b, out_f32=True, tiles=tiles)
+    assert ((got.double() - want).abs() <= _few_bound(a, b)).all()
+    assert torch.equal(ops.gemm_few(a, b, tiles=tiles), got.bfloat16())
+    # (a row's sums are formed in one order whatever the tiles, the other rows and the layout)
+    assert torch.equal(ops.gemm_few(a[m - 1:].contiguous(), b, out_f32=True)[0], got[m - 1])
+    if can_tile(b):
+        bt = b.clone()
+        tile_(bt)
+        assert torch.equal(ops.gemm_few(a, bt, out_f32=True, tiled=True, tiles=tiles), got)
+
+
+@pytest.mark.parametrize("sizes", [[0, 17, 1, 0, 16], [33, 0, 64, 2, 30], [1, 0, 0, 0, 0], [0, 0, 0, 0, 3], [2] * 70 + [0] * 5 + [9]])
+@pytest.mark.parametrize("tiled", [False, True])
+def test_product_of_a_few_rows_in_groups(ops, sizes, tiled):
+    """Groups without rows, group slots, the last group's matrix elsewhere and in the other layout, picked rows, a scale a row,
+    and both activations."""
+    from jax_llm_examples_amd.ops.layout import tile_
+
+    g = torch.Generator().manual_seed(len(sizes))
+    G, m, n, k, f = len(sizes), sum(sizes), 30, 256, 96
+    bf = lambda *s: torch.randn(*s, generator=g).to(DEV, torch.bfloat16)
+    w, last, x = bf(G - 1, 2 * f, k), bf(2 * f, k), bf(n, k)
+    off = torch.tensor([0] + sizes).cumsum(0).int().to(DEV)
+    rows = torch.randint(0, n, (m,), generator=g).int().to(DEV)
+    scale = torch.rand(m, generator=g).to(DEV)
+    group = torch.repeat_interleave(torch.arange(G), torch.tensor(sizes)).to(DEV)
+    every = torch.cat([w, last[None]]).double()
+    xs = x[rows.long()].double()
+    want = torch.einsum("mk,mnk->mn", xs, every[group]) * scale.double()[:, None]
+    bound = (k + 3) * 2.0 ** -24 * torch.einsum("mk,mnk->mn", xs.abs(), every[group].abs()) * scale.double()[:, None] + 1e-30
+    wt = w.clone()
+    if tiled:
+        tile_(wt)
+    kw = dict(offsets=off, a_rows=rows, scale=scale, tiled=tiled, b_last=last)
+    got = ops.gemm_few(x, wt, out_f32=True, **kw)
+    assert ((got.double() - want).abs() <= bound).all()
+    # (a factor of 2^-8 for the rounding to bfloat16, before and after the square)
+    y = ops.gemm_few(x, wt, relu2=True, **kw)
+    assert torch.equal(y, (got.bfloat16().float().clamp(min=0) ** 2).bfloat16())
+    for act in (1, 2):
+        y = ops.gemm_few(x, wt, swiglu=act, out_f32=True, **kw)
+        gate, up, of_gate, of_up = want[:, :f], want[:, f:], bound[:, :f], bound[:, f:]
+        ref_act = torch.nn.functional.silu(gate) if act == 1 else torch.nn.functional.gelu(gate, approximate="tanh")
+        # (the sums' own bounds, through slopes of up to 1.13; expf and tanhf within a few units of 2^-24 of 1 + |x|)
+        tol = 1.13 * of_gate * (up.abs() + of_up) + ref_act.abs() * of_up + 32 * 2.0 ** -24 * (1 + gate.abs()) * up.abs()
+        assert ((y.double() - ref_act * up).abs() <= tol + 1e-30).all()
+
+
+def test_product_of_a_few_rows_refuses_what_it_cannot_read(ops):
+    from jax_llm_examples_amd.ops.hip import KernelError
+
+    a, b = torch.zeros(4, 64, device=DEV, dtype=torch.bfloat16), torch.zeros(16, 64, device=DEV, dtype=torch.bfloat16)
+    odd = torch.zeros(4 * 64 + 1, device=DEV, dtype=torch.bfloat16)[1:].view(4, 64)
+    for x, w in ((a[:, :56].contiguous(), b[:, :56].contiguous()), (odd, b)):
+        assert not ops._few(x, w)
+        with pytest.raises(KernelError):
+            ops.gemm_few(x, w)
+    assert torch.equal(ops.linear(odd, b), torch.zeros(4, 16, device=DEV, dtype=torch.bfloat16))
