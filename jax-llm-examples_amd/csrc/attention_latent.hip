@@ -815,6 +815,279 @@ JLE_API int jle_latent_attention_mfma(const void* q_lat, const void* q, int q_ld
   return 0;
 }
 
+// ------------------------------------------------------------------ few rows: a block a tile of rows and a range of keys
+// The kernel above has a wavefront do everything for its keys, one trip to memory after the other (page numbers, 32 keys in
+// two halves, their transposed copies in two halves), and leave 16 rows of kv_rank sums behind for every 32 keys: 18 us for
+// 8 requests of 16 heads behind 1,100 tokens, and 9 for a merge that reads as much again.  Here the four wavefronts of a
+// block share a tile and 128 keys a step: the scores of 32 keys each, maxima, sums and probabilities through shared memory,
+// then a quarter of the latent's columns each over all 128.  Everything a step reads is asked for at its start (a wavefront a
+// SIMD: registers for 36 + 32 operands), and there is a fourth of the partial sums.
+// latent_values_kernel merges them and takes them out of the latent's space in the same launch (a head's matrix on the matrix
+// cores, asked for before the merge), laid out as the output projection reads them: merge, product and transposition were
+// 9.0 + 10.6 + 4.7 us.  All of it for 8 requests of 16 heads, latent 512, window 1,024: 39.2 -> 19.9 us (13.4 + 5.2); what is
+// left is the chain to a key (tile, position, table, page) and a compute unit's share of the reads.
+template <int NR>  // chunks of 32 latent elements: kv_rank <= 32 * NR
+__global__ __launch_bounds__(256, 1) void latent_decode_kernel(
+    const bf16_t* __restrict__ q_lat, const bf16_t* __restrict__ q, int q_ld, int dn, int dr,
+    const bf16_t* __restrict__ latent, const bf16_t* __restrict__ latent_t, const bf16_t* __restrict__ rope,
+    const int* __restrict__ positions, const int* __restrict__ token_segment, const int* __restrict__ block_table,
+    int table_width, int window, float scale, const int* __restrict__ tiles, int N, int H, int R, int ps, int splits,
+    int chunks_per_split, float* __restrict__ ws_ml, float* __restrict__ ws_o) {
+  constexpr int DT = NR / 2;  // tiles of 16 latent columns of a wavefront
+  __shared__ float s_max[4][16], s_sum[4][16];
+  __shared__ u32x4 s_p[4][64];
+  const int lane = threadIdx.x & 63, g = lane >> 4, r = lane & 15, wave = wave_index();
+  const int tile = blockIdx.x / splits, sp = blockIdx.x - tile * splits;
+  const int row0 = tiles[2 * tile], nrows = tiles[2 * tile + 1];
+  const bool row_ok = r < nrows;
+  const int row = row0 + (row_ok ? r : 0);
+  const int n = row / H, h = row - n * H;
+  const int pos = positions[n];
+  const int first = window > 0 ? max(0, pos - window + 1) : 0;
+  const int* table = block_table + (size_t)token_segment[__builtin_amdgcn_readfirstlane(row0 / H)] * table_width;
+  int lo = row_ok ? first : 0x7fffffff, hi = row_ok ? pos : -1;
+#pragma unroll
+  for (int o = 8; o > 0; o >>= 1) {
+    lo = min(lo, __shfl_xor(lo, o, 64));
+    hi = max(hi, __shfl_xor(hi, o, 64));
+  }
+  const u32x4 zero4 = {0u, 0u, 0u, 0u};
+  bf16x8 qb[NR + 2];  // the queries: B operands, column = this lane's row, 8 consecutive k a lane
+  {
+    const bf16_t* ql = q_lat + ((size_t)h * N + n) * R;
+#pragma unroll
+    for (int c = 0; c < NR; ++c) {
+      const int k0 = c * 32 + g * 8;
+      qb[c] = __builtin_bit_cast(bf16x8, k0 < R ? load16(ql + k0) : zero4);
+    }
+    const bf16_t* qr = q + (size_t)n * q_ld + (size_t)h * (dn + dr) + dn;
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      const int k0 = c * 32 + g * 8;
+      qb[NR + c] = __builtin_bit_cast(bf16x8, k0 < dr ? load16(qr + k0) : zero4);
+    }
+  }
+  float m = -INFINITY, l = 0.f;
+  f32x4 acc[DT];
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt) acc[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int t_lo = __builtin_amdgcn_readfirstlane((lo / 32) * 32 + sp * chunks_per_split * 128);
+  const int last = __builtin_amdgcn_readfirstlane(hi);
+  const int t_hi = min(last, t_lo + chunks_per_split * 128 - 1);
+  for (int t0 = t_lo; t0 <= t_hi; t0 += 128) {  // (the same for all wavefronts of the block)
+    // page numbers, then keys and transposed copies, all on their way together; what lies behind the last key is asked for
+    // from a place that exists and put to zero
+    int vpage[4];
+#pragma unroll
+    for (int kc = 0; kc < 4; ++kc) vpage[kc] = table[min(t0 + 32 * kc + 8 * g, last) / ps];
+    int kpage[2];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) kpage[t] = table[min(t0 + 32 * wave + 8 * (r >> 2) + 4 * t + (r & 3), last) / ps];
+    u32x4 ka[2][NR + 2], v[4][DT];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const int key = t0 + 32 * wave + 8 * (r >> 2) + 4 * t + (r & 3);
+      const size_t slot = (size_t)max(kpage[t], 0) * ps + key % ps;
+#pragma unroll
+      for (int c = 0; c < NR; ++c) ka[t][c] = load16(latent + slot * R + min(c * 32, R - 32) + g * 8);
+#pragma unroll
+      for (int c = 0; c < 2; ++c) ka[t][NR + c] = load16(rope + slot * dr + min(c * 32 + g * 8, dr - 8));
+    }
+#pragma unroll
+    for (int kc = 0; kc < 4; ++kc) {
+      const int key0 = t0 + 32 * kc + 8 * g;
+      const bf16_t* vbase = latent_t + ((size_t)max(vpage[kc], 0) * R + r) * ps + key0 % ps;
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) v[kc][dt] = load16(vbase + (size_t)min((wave * DT + dt) * 16, R - 16) * ps);
+    }
+    __builtin_amdgcn_sched_barrier(0);  // (every load above is asked for before the first product below)
+    f32x4 st[2];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      st[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+      const bool have = t0 + 32 * wave + 8 * (r >> 2) + 4 * t + (r & 3) <= last && kpage[t] >= 0;
+#pragma unroll
+      for (int c = 0; c < NR + 2; ++c) {
+        u32x4 k = ka[t][c];
+        if (!have || (c < NR ? c * 32 >= R : (c - NR) * 32 + g * 8 >= dr)) k = zero4;
+        st[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, k), qb[c], st[t], 0, 0, 0);
+      }
+    }
+    // this lane holds, for its row, the scores of keys t0 + 32 wave + 8 g .. + 7
+    float sv[8], mx = -INFINITY;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const int key = t0 + 32 * wave + 8 * g + e;
+      sv[e] = row_ok && key >= first && key <= pos && key <= t_hi ? st[e >> 2][e & 3] * scale : -INFINITY;
+      mx = fmaxf(mx, sv[e]);
+    }
+    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    if (g == 0) s_max[wave][r] = mx;
+    __syncthreads();
+    const float m_new = fmaxf(fmaxf(fmaxf(s_max[0][r], s_max[1][r]), fmaxf(s_max[2][r], s_max[3][r])), m);
+    const float corr = m_new == -INFINITY ? 1.f : expf(m - m_new);
+    float p[8], psum = 0.f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      p[e] = sv[e] == -INFINITY ? 0.f : expf(sv[e] - m_new);
+      psum += p[e];
+    }
+    psum += __shfl_xor(psum, 16, 64);
+    psum += __shfl_xor(psum, 32, 64);
+    if (g == 0) s_sum[wave][r] = psum;
+    s_p[wave][lane] = u32x4{pack_bf16(p[0], p[1]), pack_bf16(p[2], p[3]), pack_bf16(p[4], p[5]), pack_bf16(p[6], p[7])};
+    __syncthreads();
+    l = l * corr + ((s_sum[0][r] + s_sum[1][r]) + (s_sum[2][r] + s_sum[3][r]));
+    m = m_new;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) acc[dt] *= corr;
+#pragma unroll
+    for (int kc = 0; kc < 4; ++kc) {
+      const bf16x8 pb = __builtin_bit_cast(bf16x8, s_p[kc][lane]);
+      // tokens behind the rows' last position are not written yet: what lies there must not meet a zero weight
+      const int n_ok = last - (t0 + 32 * kc + 8 * g) + 1;
+      u32x4 keep;
+#pragma unroll
+      for (int w2 = 0; w2 < 4; ++w2)
+        keep[w2] = vpage[kc] < 0 ? 0u : (n_ok >= 2 * w2 + 2 ? 0xffffffffu : (n_ok == 2 * w2 + 1 ? 0x0000ffffu : 0u));
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt)
+        acc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, v[kc][dt] & keep), pb, acc[dt], 0, 0, 0);
+    }
+  }
+  if (!row_ok) return;
+  const size_t slot = (size_t)row * splits + sp;
+  if (wave == 0 && g == 0) {
+    ws_ml[slot * 2] = m;
+    ws_ml[slot * 2 + 1] = l;
+  }
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt)
+    if ((wave * DT + dt) * 16 < R) *reinterpret_cast<f32x4*>(ws_o + slot * R + (wave * DT + dt) * 16 + g * 4) = acc[dt];
+}
+
+// o[n, h dv + j] = sum_d w_uv[h dv + j, d] c[n, h, d], c the merged sums rounded to bfloat16.  Block: 64 rows of a head's matrix
+// (16 for each of the first four wavefronts), 16 tokens; a wavefront merges a token or two, every range's sums and
+// statistics on their way together (one trip to memory; with the statistics first, four wavefronts and two tokens one after
+// the other 9.7 us at 8 tokens).  The merge of a block's tokens is done by each of the head's dv / 64 blocks.
+template <int NR>
+__global__ __launch_bounds__(512) void latent_values_kernel(const float* __restrict__ ws_ml, const float* __restrict__ ws_o,
+                                                            const bf16_t* __restrict__ w_uv, bf16_t* __restrict__ out, int N,
+                                                            int H, int R, int dv, int splits, const float* __restrict__ sink) {
+  constexpr int U = 5, E = (NR * 32 + 255) / 256;  // ranges on their way; pieces of four elements a lane
+  constexpr int LD = NR * 32 + 8;                   // elements from token to token: 16 tokens' pieces do not collide
+  __shared__ __attribute__((aligned(16))) bf16_t c[16 * LD];
+  const int lane = threadIdx.x & 63, g = lane >> 4, r = lane & 15, wave = wave_index();
+  const int h = blockIdx.y, n0 = blockIdx.z * 16, j0 = blockIdx.x * 64 + wave * 16;
+  u32x4 w[NR];
+  if (wave < 4) {
+    const bf16_t* wr = w_uv + ((size_t)h * dv + min(j0 + r, dv - 1)) * R + g * 8;
+#pragma unroll
+    for (int k = 0; k < NR; ++k) w[k] = load16(wr + min(k * 32, R - 32));
+  }
+  for (int t = wave; t < 16; t += 8) {
+    const int n = n0 + t;
+    if (n >= N) break;
+    const size_t row = (size_t)n * H + h;
+    const float* ml = ws_ml + row * splits * 2;
+    const float* rows = ws_o + row * splits * R;
+    // (sums about the largest maximum so far, which starts as the sink's)
+    float mx = sink != nullptr ? sink[h] : -INFINITY, l = sink != nullptr ? 1.f : 0.f;
+    f32x4 acc[E];
+#pragma unroll
+    for (int i = 0; i < E; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int s0 = 0; s0 < splits; s0 += U) {
+      f32x4 o[U][E];
+      float ms[U], ls[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int sp = min(s0 + u, splits - 1);  // (past the last: loaded again, not used)
+        ms[u] = ml[sp * 2];
+        ls[u] = ml[sp * 2 + 1];
+#pragma unroll
+        for (int i = 0; i < E; ++i) {
+          const int d = (i * 64 + lane) * 4;
+          o[u][i] = d < R ? *reinterpret_cast<const f32x4*>(rows + (size_t)sp * R + d) : f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+      }
+      float top = mx;
+#pragma unroll
+      for (int u = 0; u < U; ++u) top = fmaxf(top, ms[u]);
+      if (top > mx) {
+        const float corr = expf(mx - top);
+        mx = top;
+        l *= corr;
+#pragma unroll
+        for (int i = 0; i < E; ++i) acc[i] *= corr;
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const float wgt = s0 + u < splits ? expf(ms[u] - mx) : 0.f;  // (a range without keys: 0 too)
+        l += ls[u] * wgt;
+#pragma unroll
+        for (int i = 0; i < E; ++i)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_fmaf(o[u][i][j], wgt, acc[i][j]);
+      }
+    }
+    const float inv = 1.0f / l;
+#pragma unroll
+    for (int i = 0; i < E; ++i) {
+      const int d = (i * 64 + lane) * 4;
+      if (d < R)
+        *reinterpret_cast<uint2*>(c + t * LD + d) = uint2{pack_bf16(acc[i][0] * inv, acc[i][1] * inv),
+                                                         pack_bf16(acc[i][2] * inv, acc[i][3] * inv)};
+    }
+  }
+  __syncthreads();
+  if (wave >= 4) return;
+  f32x4 y = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int k = 0; k < NR; ++k) {
+    const bf16x8 b = *reinterpret_cast<const bf16x8*>(c + r * LD + min(k * 32, R - 32) + g * 8);
+    if (k * 32 < R) y = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, w[k]), b, y, 0, 0, 0);
+  }
+  // element j of y: row 4 g + j of the wavefront's 16, token r
+  if (n0 + r >= N || j0 + 4 * g >= dv) return;
+  *reinterpret_cast<uint2*>(out + ((size_t)(n0 + r) * H + h) * dv + j0 + 4 * g) = uint2{pack_bf16(y[0], y[1]), pack_bf16(y[2], y[3])};
+}
+
+// Sizes that the two kernels take: those of the matrix-core kernel, the value width in whole pieces of four.
+JLE_API int jle_latent_values_supported(int R, int dn, int dr, int q_ld, int ps, int dv) {
+  return jle_latent_attention_mfma_supported(R, dn, dr, q_ld, ps) && dv > 0 && dv % 4 == 0;
+}
+
+// jle_latent_attention_mfma with the value matrices w_uv [H * dv, R] behind it: out [N, H * dv].  The keys from a tile's first
+// one on are shared out in splits ranges of chunks_per_split times 128.
+JLE_API int jle_latent_values(const void* q_lat, const void* q, int q_ld, int dn, int dr, const void* latent_pages,
+                              const void* latent_t_pages, const void* rope_pages, const void* w_uv, void* out,
+                              const int* positions, const int* token_segment, const int* block_table, int table_width,
+                              int window, float scale, const int* tiles, int num_tiles, int N, int H, int R, int dv, int ps,
+                              int splits, int chunks_per_split, float* ws_ml, float* ws_o, const float* sink, hipStream_t s) {
+  if (N <= 0 || num_tiles <= 0) return 0;
+  if (!jle_latent_values_supported(R, dn, dr, q_ld, ps, dv) || H <= 0 || H > 65535 || N > 65535 * 16 || window < 0 ||
+      q_ld < H * (dn + dr) || splits < 1 || chunks_per_split < 1 || (long long)num_tiles * splits > 0x7fffffff ||
+      (((uintptr_t)w_uv | (uintptr_t)out | (uintptr_t)ws_o) & 15))
+    return JLE_BAD_ARG;
+#define GO(NRV)                                                                                                              \
+  do {                                                                                                                       \
+    hipLaunchKernelGGL(latent_decode_kernel<NRV>, dim3(num_tiles * splits), dim3(256), 0, s, (const bf16_t*)q_lat,           \
+                       (const bf16_t*)q, q_ld, dn, dr, (const bf16_t*)latent_pages, (const bf16_t*)latent_t_pages,           \
+                       (const bf16_t*)rope_pages, positions, token_segment, block_table, table_width, window, scale, tiles,  \
+                       N, H, R, ps, splits, chunks_per_split, ws_ml, ws_o);                                                  \
+    JLE_LAUNCH_CHECK();                                                                                                      \
+    hipLaunchKernelGGL(latent_values_kernel<NRV>, dim3((dv + 63) / 64, H, (N + 15) / 16), dim3(512), 0, s, ws_ml, ws_o,      \
+                       (const bf16_t*)w_uv, (bf16_t*)out, N, H, R, dv, splits, sink);                                        \
+  } while (0)
+  if (R <= 128) GO(4);
+  else if (R <= 256) GO(8);
+  else GO(16);
+#undef GO
+  JLE_LAUNCH_CHECK();
+  return 0;
+}
+
 // out[b][a][:] = in[a][b][:] for rows of row_bytes bytes (a multiple of 4; of 16 where the arrays allow it).
 __global__ __launch_bounds__(256) void swap_leading_kernel(const uint32_t* __restrict__ in, uint32_t* __restrict__ out,
                                                            int A, int B, int words) {

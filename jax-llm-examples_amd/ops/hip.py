@@ -76,6 +76,8 @@ _SIGNATURES = {
                                  _i, _i, _vp, _vp],
     "jle_latent_attention_mfma": [_vp, _vp, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _f, _vp, _i, _i, _i,
                                   _i, _i, _i, _i, _vp, _vp, _vp, _vp],
+    "jle_latent_values": [_vp, _vp, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _f, _vp, _i, _i, _i, _i, _i, _i,
+                          _i, _i, _vp, _vp, _vp, _vp],
     "jle_latent_attention": [_vp, _vp, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _f, _i, _i, _i, _i, _i, _i, _i,
                              _vp, _vp, _vp, _vp],
     "jle_embed_pair": [_vp, _vp, _vp, _vp, _i, _vp, _i, _i, _i, _ll, _ll, _vp],
@@ -192,6 +194,7 @@ def _bind(path: str):
     for name, args in (("jle_attention_mfma_supported", [_i, _i, _i, _i]),  # queries, not launches: no stream
                        ("jle_greedy_blocks", [_i]), ("jle_gemm_stream_supported", [_i, _i, _i]), ("jle_gemm_f32_stream_supported", [_i, _i, _i]),
                        ("jle_latent_attention_mfma_supported", [_i, _i, _i, _i, _i]),
+                       ("jle_latent_values_supported", [_i] * 6),
                        ("jle_latent_expanded_supported", [_i, _i, _i, _i, _i]), ("jle_attention_group_waves", []),
                        ("jle_mlstm_chunked_supported", [_i, _i]), ("jle_mlstm_chunk_tokens", []),
                        ("jle_gated_delta_padded", [_i]), ("jle_gated_delta_chunk_kib", [_i, _i, _i, _i]),
@@ -632,12 +635,7 @@ class HipOps:
         splits, tiles_per_split, ws_ml, ws_o = 1, 0, None, None
         waves = n * H
         if waves < self.LATENT_SPLIT_BELOW:
-            if meta is not None and meta.decode_bucket is not None:
-                longest = meta.decode_bucket  # (a step of single tokens: laid out for the bound, see GroupContext)
-            elif meta is not None and meta.seg_starts is not None:
-                longest = max(s0 + ln for s0, ln in zip(meta.seg_starts, meta.seg_lens))
-            else:
-                longest = int(positions.max()) + 1
+            longest = self._longest(meta, positions)
             span = min(w, longest) if w else longest
             tiles = -(-span // 64) + 1
             want = min(tiles, -(-self.LATENT_SPLIT_BELOW // waves))
@@ -651,11 +649,66 @@ class HipOps:
                    self._is_bf16(q_lat), n, H, r, ps, splits, tiles_per_split, _p(ws_ml), _p(ws_o), _p(sink))
         return out
 
-    def _latent_attention_mfma(self, q_lat, q, q_ld, dn, dr, latent_pages, latent_t_pages, rope_pages, out,
-                               block_table, positions, token_segment, window, scale, meta, sink=None):
+    # Up to so many row tiles a block of latent_values' takes a tile and a range of keys (with more, tiles alone fill the
+    # compute units).  latent_attention, product and transposition | latent_values, us, latent 512: 1 request of 16 heads
+    # behind 300 33 | 17, of 32 behind 8,000 78 | 28; 16 of 16 behind 2,000 46 | 31; 64 87 | 62; 128 (128 tiles) 147 | 116,
+    # behind 300 60 | 41; 64 of 32 behind 2,000 124 | 104; latent 256, 32 of 16 behind 1,000 31 | 19.
+    LATENT_VALUES_TILES = 128
+
+    def latent_values(self, q_lat, q, nope_dim: int, latent_pages, rope_pages, block_table, positions, token_segment, window,
+                      scale: float, w_uv, meta=None, latent_t_pages=None, sink=None):
+        """:meth:`latent_attention` with the heads' value matrices ``w_uv [H * dv, kv_rank]`` behind it, for few rows in
+        bfloat16: ``[N, H * dv]``, or ``None`` where other kernels take the step."""
         H, n, r = q_lat.shape
-        ps = latent_pages.shape[1]
-        # row tiles: 16 consecutive (token, head) pairs of one segment
+        dr = q.shape[2] - nope_dim
+        np_, ps = latent_pages.shape[0], latent_pages.shape[1]
+        if (latent_t_pages is None or q_lat.dtype != torch.bfloat16 or q.dtype != torch.bfloat16 or n == 0 or H > 65535
+                or w_uv.dtype != torch.bfloat16 or not w_uv.is_contiguous() or w_uv.data_ptr() % 16 or w_uv.shape[0] % H
+                or n * H > 16 * self.LATENT_VALUES_TILES or q.stride(2) != 1 or q.stride(1) != q.shape[2]
+                or q.shape[:2] != (n, H) or w_uv.shape[1] != r):
+            return None
+        q_ld, dv = q.stride(0), w_uv.shape[0] // H
+        if not self._query("jle_latent_values_supported", r, nope_dim, dr, q_ld, ps, dv):
+            return None
+        plan = self._latent_tiles(meta, H, token_segment, positions, q_lat.device)
+        tiles = plan.numel() // 2
+        if tiles > self.LATENT_VALUES_TILES:
+            return None
+        self._chk(q_lat, torch.bfloat16, (H, n, r), "queries in the latent's space")
+        for pages, what in ((latent_pages, "latent pages"), (latent_t_pages, "transposed latent pages")):
+            self._chk(pages, torch.bfloat16, (np_, ps, r), what)
+        self._chk(rope_pages, torch.bfloat16, (np_, ps, dr), "rotated key pages")
+        self._chk(block_table, torch.int32, None, "block table")
+        self._chk(positions, torch.int32, (n,), "positions")
+        self._chk(token_segment, torch.int32, (n,), "token segments")
+        if sink is not None:
+            self._chk(sink, torch.float32, (H,), "sinks")
+        window = 0 if window is None else int(window)
+        longest = self._longest(meta, positions)
+        span = min(window, longest) if window else longest
+        spanned = -(-16 // H) + 1 if H < 16 else 1  # tokens whose rows may share a tile
+        chunks = -(-(span + spanned + 31) // 128)  # (a tile's first key is at most 31 behind a multiple of 32)
+        per = -(-chunks // max(1, min(chunks, 256 // tiles)))
+        splits = -(-chunks // per)
+        ws_ml = torch.empty(n * H * splits * 2, dtype=torch.float32, device=q_lat.device)
+        ws_o = torch.empty(n * H * splits * r, dtype=torch.float32, device=q_lat.device)
+        out = torch.empty(n, H * dv, dtype=torch.bfloat16, device=q_lat.device)
+        self._call("jle_latent_values", _p(q_lat), _p(q), q_ld, nope_dim, dr, _p(latent_pages), _p(latent_t_pages),
+                   _p(rope_pages), _p(w_uv), _p(out), _p(positions), _p(token_segment), _p(block_table), block_table.shape[1],
+                   window, float(scale), _p(plan), tiles, n, H, r, dv, ps, splits, per, _p(ws_ml), _p(ws_o), _p(sink))
+        return out
+
+    @staticmethod
+    def _longest(meta, positions) -> int:
+        """The context length that a step's key ranges are laid out for."""
+        if meta is not None and meta.decode_bucket is not None:
+            return meta.decode_bucket  # (a step of single tokens: laid out for the bound, see GroupContext)
+        if meta is not None and meta.seg_starts is not None:
+            return max(s0 + ln for s0, ln in zip(meta.seg_starts, meta.seg_lens))
+        return int(positions.max()) + 1
+
+    def _latent_tiles(self, meta, H: int, token_segment, positions, device):
+        """Row tiles: 16 consecutive (token, head) pairs of one segment, as (first row, rows)."""
         key = f"latent_tiles_{H}"
         plan = meta.meta.get(key) if meta is not None else None
         if plan is None:
@@ -667,9 +720,16 @@ class HipOps:
                 for t in range(0, rows, 16):
                     flat += [o * H + t, min(16, rows - t)]
                 o += ln
-            plan = torch.tensor(flat, dtype=torch.int32).to(q_lat.device)
+            plan = torch.tensor(flat, dtype=torch.int32).to(device)
             if meta is not None:
                 meta.meta[key] = plan
+        return plan
+
+    def _latent_attention_mfma(self, q_lat, q, q_ld, dn, dr, latent_pages, latent_t_pages, rope_pages, out,
+                               block_table, positions, token_segment, window, scale, meta, sink=None):
+        H, n, r = q_lat.shape
+        ps = latent_pages.shape[1]
+        plan = self._latent_tiles(meta, H, token_segment, positions, q_lat.device)
         tiles = plan.numel() // 2
         if tiles >= self.LATENT_LDS_TILES:
             # many rows: blocks of four neighbouring tiles that share their keys through shared memory
@@ -702,12 +762,7 @@ class HipOps:
             return out
         splits, steps_per_split, ws_ml, ws_o = 1, 0, None, None
         if tiles < self.LATENT_MFMA_ITEMS:
-            if meta is not None and meta.decode_bucket is not None:
-                longest = meta.decode_bucket  # (a step of single tokens: laid out for the bound, see GroupContext)
-            elif meta is not None and meta.seg_starts is not None:
-                longest = max(s0 + ln for s0, ln in zip(meta.seg_starts, meta.seg_lens))
-            else:
-                longest = int(positions.max()) + 1
+            longest = self._longest(meta, positions)
             span = min(window, longest) if window else longest
             spanned = -(-16 // H) + 1 if H < 16 else 1  # tokens whose rows may share a tile
             steps = -(-(span + spanned + 31) // 32)

@@ -630,6 +630,10 @@ class ReferenceOps:
             out[i] = (pr @ c).to(out.dtype)
         return out
 
+    def latent_values(self, *args, **kw):
+        """``None``: the plain ops take the sums out of the latent's space by a product of its own."""
+        return None
+
     def latent_attention_expanded(self, *args, **kw):
         """``None``: the plain ops stay in the latent's space (:meth:`latent_attention`)."""
         return None

@@ -163,12 +163,15 @@ class LatentAttention(Mixer):
         if o is None:
             # queries into the latent's space: [H, N, dn] x [H, dn, r]
             q_lat = ops.batched_linear(q[:, :, :dn].transpose(0, 1), self.params["w_uk"].view(H, dn, r))
-            o_lat = ops.latent_attention(q_lat, q, dn, cache.pages["latent"], cache.pages["rope_key"], cache.block_table,
-                                         ctx.positions, ctx.token_segment, self.window, self.softmax_scale,
-                                         cache.attn_meta, latent_t_pages=cache.pages.get("latent_t"),
-                                         sink=self.params.get("sink"))  # [N, H, r]
-            # the sums out of it: [H, N, r] x [H, r, dv], laid out [N, H * dv]
-            o = ops.batched_linear(o_lat.transpose(0, 1), self.w_out, tokens_first=True)
+            args = (q_lat, q, dn, cache.pages["latent"], cache.pages["rope_key"], cache.block_table, ctx.positions,
+                    ctx.token_segment, self.window, self.softmax_scale)
+            more = dict(meta=cache.attn_meta, latent_t_pages=cache.pages.get("latent_t"), sink=self.params.get("sink"))
+            if "latent_t" in cache.pages:  # (few rows: attention and the product out of the latent's space together)
+                o = ops.latent_values(*args, self.params["w_uv"], **more)
+            if o is None:
+                o_lat = ops.latent_attention(*args, **more)  # [N, H, r]
+                # the sums out of it: [H, N, r] x [H, r, dv], laid out [N, H * dv]
+                o = ops.batched_linear(o_lat.transpose(0, 1), self.w_out, tokens_first=True)
         o = o.view(n, H * dv)
         if self.output_gate:
             o = ops.sigmoid_mul(o, rows[:, self.gate_offset: self.gate_offset + H * dv])

@@ -192,3 +192,54 @@ def test_pages_that_the_matrix_cores_do_not_take_keep_their_float32_probabilitie
     out = ops.latent_attention_expanded(zeros(n, H, DN + DR), DN, zeros(H * DN, R), zeros(H * DV, R), zeros(n // ps, ps, R),
                                         zeros(n // ps, ps, DR), table, pos, seg, None, 0.1)
     assert (out is not None) == (ps == 8) == bool(ops._query("jle_latent_attention_mfma_supported", R, DN, DR, H * (DN + DR), ps))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("segs, window, sink, H, R, dv, ps", [
+    ([(1, 0)], None, False, 1, 32, 4, 8),                                   # one key, the smallest sizes
+    ([(1, 126), (1, 127), (1, 128), (1, 159)], None, False, 16, 512, 128, 16),  # beside the edge of a range of 128 keys
+    ([(1, 700), (1, 3), (1, 1029)], 128, True, 20, 512, 68, 16),            # windows of one range, tiles of 4 rows, odd widths
+    ([(1, 1060 + 50 * i) for i in range(8)], 1024, False, 16, 512, 128, 16),
+    ([(5, 100), (1, 31), (17, 64)], 40, False, 3, 160, 64, 32),             # tiles over several tokens, more than 16 tokens
+    ([(1, 2000 + i) for i in range(70)], None, True, 16, 256, 96, 16),      # several ranges a block
+])
+def test_few_rows_through_the_latent_and_out_of_it(segs, window, sink, H, R, dv, ps):
+    dev = "cuda:0"
+    ops = HipOps(dev)
+    g = torch.Generator().manual_seed(len(segs) + R)
+    bf = lambda *s, std=1.0: (torch.randn(*s, generator=g) * std).to(torch.bfloat16)
+    lens, starts = [n for n, _ in segs], [s for _, s in segs]
+    N, width = sum(lens), max(-(-(n + s) // ps) for n, s in segs)
+    need = [max(0, s - window + 1) if window else 0 for s in starts]
+    table = torch.full((len(segs), width), -1, dtype=torch.int32)
+    free = torch.randperm(len(segs) * width, generator=g).tolist()
+    latent, rope = bf(len(segs) * width, ps, R), bf(len(segs) * width, ps, DR)
+    for i, (n, s) in enumerate(segs):
+        for j in range(need[i] // ps, -(-(n + s) // ps)):  # (pages that no query sees were given back)
+            table[i, j] = free.pop()
+        if (n + s) % ps:  # what lies behind a segment's end was never written
+            latent[table[i, (n + s) // ps], (n + s) % ps:] = float("nan")
+            rope[table[i, (n + s) // ps], (n + s) % ps:] = float("nan")
+    q, q_lat, uv = bf(N, H * (DN + DR) + 8), bf(H, N, R, std=R ** -0.5 * DN ** 0.5), bf(H * dv, R, std=R ** -0.5)
+    sk = torch.randn(H, generator=g) if sink else None
+    pos = torch.tensor([s + t for n, s in segs for t in range(n)], dtype=torch.int32)
+    seg = torch.tensor([i for i, (n, _) in enumerate(segs) for _ in range(n)], dtype=torch.int32)
+    single = max(lens) == 1
+    meta = GroupContext(block_table=None, slot_mapping=None, width=width, retention=("all",), seg_lens=lens, seg_starts=starts,
+                        decode_bucket=-(-max(starts) // 1024) * 1024 + 1024 if single else None)
+    d = lambda t: None if t is None else t.to(dev)
+    scale = (DN + DR) ** -0.5
+    got = ops.latent_values(d(q_lat), d(q)[:, : H * (DN + DR)].view(N, H, DN + DR), DN, d(latent), d(rope), d(table), d(pos),
+                            d(seg), window, scale, d(uv), meta=meta, latent_t_pages=d(latent.transpose(1, 2).contiguous()).view(-1, ps, R),
+                            sink=d(sk)).cpu().double().view(N, H, dv)
+    for t in range(N):
+        p, i = int(pos[t]), int(seg[t])
+        kpos = torch.arange(max(0, p - window + 1) if window else 0, p + 1)
+        c, kr = (x[table[i][kpos // ps].long(), kpos % ps].double() for x in (latent, rope))
+        sc = (q_lat[:, t].double() @ c.T + q[t, : H * (DN + DR)].view(H, DN + DR)[:, DN:].double() @ kr.T) * scale
+        if sink:
+            sc = torch.cat([sc, sk.double()[:, None]], 1)
+        out = torch.softmax(sc, -1)[:, : len(kpos)] @ c
+        want = torch.einsum("hr,hvr->hv", out, uv.view(H, dv, R).double())
+        # probabilities, sums and the result rounded to bfloat16: 2^-9 each at most
+        assert (got[t] - want).norm() < 4 * 2.0 ** -9 * want.norm(), (t, float((got[t] - want).norm() / want.norm()))
