@@ -240,17 +240,24 @@ __global__ __launch_bounds__(WAVES * 64, 2) void gemm_stream_kernel(const bf16_t
 // 16 groups of 16,384 x 5,120 (gate and up) with 410 rows each: 1,023 us (1.08 PFLOP/s) against 1,508 in passes of 192; 8 of
 // 4,096 x 7,168 163 (1.18) against 275.  (With eight wavefronts of 64 x half the rows and the weights through shared memory
 // too 422 and 188 at 8 groups: reading and bringing in together took shared memory as long as the products.)
-// Work items: a group's rows in tiles of at most 256, as even as multiples of 32 allow; item = ((row block / 8) * tiles +
+// HALF (plain products): a block takes 128 rows of W and up to 288 of X, its wavefronts in twos by twos, 64 rows of W and half
+// of X each.  It reads twice as much for a product, but where blocks of 256 would fill a part of the compute units or of their
+// last round it is the faster: 8 groups of 2,048 x 4,096 with 512 rows 90 us in passes, 106 in wide tiles (128 blocks; a
+// group of more than 512 rows makes three tiles), 75 so.  (All of 288 rows in wide tiles spills registers: 10 times slower.)
+// Work items: a group's rows in tiles of at most 256 (288), as even as multiples of 32 allow; item = ((row block / 8) * tiles +
 // tile) * 8 + row block % 8 within a group, so that the tiles that read the same weights run on one chiplet.
-constexpr int kWideRows = 256;
-constexpr int kWideStage = kWideRows * BK * 2, kWideLds = 3 * kWideStage;  // bytes of a stage's rows, and of the ring
+constexpr int wide_rows(bool half) { return half ? 288 : 256; }                            // of X, of a block
+constexpr uint32_t wide_stage(bool half) { return (uint32_t)wide_rows(half) * BK * 2; }  // bytes of a stage's rows
 
-template <bool SWIGLU, int NT>
+template <bool SWIGLU, bool HALF, int NT>
 __device__ __forceinline__ void wide_block(const bf16_t* __restrict__ X, const bf16_t* __restrict__ We,
                                            bf16_t* __restrict__ Y, const int* __restrict__ a_rows,
                                            const float* __restrict__ scale, unsigned char* smem, int tok0, int live, int K,
                                            int Nout, int nb) {
-  static_assert(NT % 2 == 0 && NT >= 4, "a wavefront brings NT / 2 kilobytes of a stage's rows");
+  static_assert(NT % 2 == 0, "a wavefront brings NT / 2 kilobytes of a stage's rows");
+  static_assert(!HALF || !SWIGLU, "half a block of rows of W: plain products only");
+  constexpr int NW = HALF ? NT / 2 : NT;  // tiles of X a wavefront multiplies with
+  static_assert(NW >= 4, "a stage's first operands are read behind the barrier in the middle of the stage before");
   constexpr int PF = 4;  // operands asked for ahead
   const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
   const int wave = wave_index();
@@ -262,7 +269,7 @@ __device__ __forceinline__ void wide_block(const bf16_t* __restrict__ X, const b
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int tile = SWIGLU ? min(nb * 8 + wave * 2 + (i & 1), ntile - 1) + (i >= 2 ? half >> 4 : 0)
-                            : min(nb * 16 + wave * 4 + i, ntile - 1);
+                            : min(HALF ? nb * 8 + (wave & 1) * 4 + i : nb * 16 + wave * 4 + i, ntile - 1);
     w_src[i] = We + (size_t)tile * 16 * K + lane * 8;
   }
   uint32_t x_src[NT / 2];
@@ -282,41 +289,43 @@ __device__ __forceinline__ void wide_block(const bf16_t* __restrict__ X, const b
 #pragma unroll
       for (int i = 0; i < 4; ++i) w[ks][i] = *reinterpret_cast<const u32x4*>(w_src[i] + (size_t)(2 * s + ks) * 512);
   };
-  const uint32_t b_rd = (uint32_t)(r * 128 + ((g ^ (r & 7)) * 16));  // (k step 1: bit 6 the other way)
+  const int n0 = HALF ? (wave >> 1) * NW : 0;  // the first of its tiles of X
+  const uint32_t b_rd = (uint32_t)(n0 * 2048 + r * 128 + ((g ^ (r & 7)) * 16));  // (k step 1: bit 6 the other way)
   auto operand = [&](uint32_t place, int j) __attribute__((always_inline)) {
-    return *reinterpret_cast<const bf16x8*>(smem + place + (b_rd ^ (j >= NT ? 64 : 0)) + (j % NT) * 2048);
+    return *reinterpret_cast<const bf16x8*>(smem + place + (b_rd ^ (j >= NW ? 64 : 0)) + (j % NW) * 2048);
   };
-  f32x4 acc[4][NT];
+  f32x4 acc[4][NW];
 #pragma unroll
   for (int i = 0; i < 4; ++i)
 #pragma unroll
-    for (int n = 0; n < NT; ++n) acc[i][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int n = 0; n < NW; ++n) acc[i][n] = f32x4{0.f, 0.f, 0.f, 0.f};
   u32x4 wa[2][4], wb[2][4], wc[2][4], wd[2][4];
   bf16x8 ahead[PF];
-  uint32_t here = 0, next = kWideStage, free_ = 2 * kWideStage;  // the ring: this stage's rows, the next one's, the one after
+  constexpr uint32_t STAGE = wide_stage(HALF);
+  uint32_t here = 0, next = STAGE, free_ = 2 * STAGE;  // the ring: this stage's rows, the next one's, the one after
 
   // rows_next: how many of the loads on their way are younger than the next stage's rows (-1: there is no next stage)
 #define WIDE_STAGE(w_, s_, rows_next, ASKX, ASKW)                                                       \
   do {                                                                                                  \
-    bf16x8 b_[2 * NT + PF];                                                                             \
+    bf16x8 b_[2 * NW + PF];                                                                             \
     _Pragma("unroll") for (int p = 0; p < PF; ++p) b_[p] = ahead[p];                                    \
-    _Pragma("unroll") for (int j = 0; j < 2 * NT; ++j) {                                                \
-      if (j == NT && rows_next >= 0) {                                                                  \
+    _Pragma("unroll") for (int j = 0; j < 2 * NW; ++j) {                                                \
+      if (j == NW && rows_next >= 0) {                                                                  \
         if (rows_next > 0) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");                             \
         else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                                           \
         __syncthreads();                                                                                \
         if (ASKX) ask_rows((s_) + 2, free_);                                                            \
       }                                                                                                 \
-      if (j + PF < 2 * NT) b_[j + PF] = operand(here, j + PF);                                          \
-      else if (rows_next >= 0) b_[j + PF] = operand(next, j + PF - 2 * NT);                             \
+      if (j + PF < 2 * NW) b_[j + PF] = operand(here, j + PF);                                          \
+      else if (rows_next >= 0) b_[j + PF] = operand(next, j + PF - 2 * NW);                             \
       _Pragma("unroll") for (int i = 0; i < 4; ++i) {                                                   \
-        acc[i][j % NT] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, w_[j / NT][i]), b_[j], \
-                                                                 acc[i][j % NT], 0, 0, 0);              \
+        acc[i][j % NW] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, w_[j / NW][i]), b_[j], \
+                                                                 acc[i][j % NW], 0, 0, 0);              \
       }                                                                                                 \
       __builtin_amdgcn_sched_barrier(0);                                                                \
     }                                                                                                   \
     if (rows_next >= 0) {                                                                               \
-      _Pragma("unroll") for (int p = 0; p < PF; ++p) ahead[p] = b_[2 * NT + p];                         \
+      _Pragma("unroll") for (int p = 0; p < PF; ++p) ahead[p] = b_[2 * NW + p];                         \
     }                                                                                                   \
     if (ASKW) ask_weights(w_, (s_) + WAHEAD);                                                           \
     const uint32_t t_ = here;                                                                           \
@@ -328,7 +337,7 @@ __device__ __forceinline__ void wide_block(const bf16_t* __restrict__ X, const b
   __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the rows' numbers have come; from here on only the stages' loads count
   asm volatile("" ::: "memory");
   ask_rows(0, 0);
-  ask_rows(1, kWideStage);
+  ask_rows(1, STAGE);
   ask_weights(wa, 0);
   ask_weights(wb, 1);
   ask_weights(wc, 2);
@@ -350,14 +359,14 @@ __device__ __forceinline__ void wide_block(const bf16_t* __restrict__ X, const b
   WIDE_STAGE(wd, s + 3, -1, false, false);
 #undef WIDE_STAGE
 #pragma unroll
-  for (int n = 0; n < NT; ++n) {
-    const int row = n * 16 + r;
+  for (int n = 0; n < NW; ++n) {
+    const int row = (n0 + n) * 16 + r;
     if (row >= live) continue;
     const int t = tok0 + row;
     const float sc = scale != nullptr ? scale[t] : 1.f;
 #pragma unroll
     for (int i = 0; i < (SWIGLU ? 2 : 4); ++i) {
-      const int tile = SWIGLU ? nb * 8 + wave * 2 + i : nb * 16 + wave * 4 + i;
+      const int tile = SWIGLU ? nb * 8 + wave * 2 + i : HALF ? nb * 8 + (wave & 1) * 4 + i : nb * 16 + wave * 4 + i;
       if (tile >= ntile) continue;
       float y[4];
 #pragma unroll
@@ -374,12 +383,13 @@ __device__ __forceinline__ void wide_block(const bf16_t* __restrict__ X, const b
   }
 }
 
-template <bool SWIGLU>
+template <bool SWIGLU, bool HALF>
 __global__ __launch_bounds__(256, 1) void wide_kernel(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W,
                                                       bf16_t* __restrict__ Y, const int* __restrict__ offsets,
                                                       const int* __restrict__ a_rows, const float* __restrict__ scale,
                                                       int Nout, int K, int G, int nblk8) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
+  constexpr int kWideRows = wide_rows(HALF);
   // this block's group: 64 groups a look, the items before each by a sum over the lanes
   const int lane = threadIdx.x & 63;
   int left = blockIdx.x, e = -1, tiles = 0;
@@ -408,14 +418,20 @@ __global__ __launch_bounds__(256, 1) void wide_kernel(const bf16_t* __restrict__
   left = __builtin_amdgcn_readfirstlane(left);
   tiles = __builtin_amdgcn_readfirstlane(tiles);
   const int nb = left / (8 * tiles) * 8 + (left & 7), tile = (left >> 3) % tiles;
-  if (nb * (SWIGLU ? 128 : 256) >= (SWIGLU ? Nout / 2 : Nout)) return;
+  if (nb * (SWIGLU || HALF ? 128 : 256) >= (SWIGLU ? Nout / 2 : Nout)) return;
   const int lo = offsets[e], rows = offsets[e + 1] - lo;
   const int per = ((rows + tiles - 1) / tiles + 31) / 32 * 32;
   const int tok0 = lo + tile * per, live = min(per, rows - tile * per);
   if (live <= 0) return;
   const bf16_t* We = W + (size_t)e * Nout * K;
-#define GO(NT_) wide_block<SWIGLU, NT_>(X, We, Y, a_rows, scale, smem, tok0, live, K, Nout, nb)
-  if (live <= 64) GO(4);
+#define GO(NT_) wide_block<SWIGLU, HALF, NT_>(X, We, Y, a_rows, scale, smem, tok0, live, K, Nout, nb)
+  if constexpr (HALF) {
+    if (live > 256) {
+      GO(18);
+      return;
+    }
+  }
+  if (live <= 64) GO(HALF ? 8 : 4);
   else if (live <= 128) GO(8);
   else if (live <= 160) GO(10);
   else if (live <= 192) GO(12);
@@ -424,14 +440,16 @@ __global__ __launch_bounds__(256, 1) void wide_kernel(const bf16_t* __restrict__
 #undef GO
 }
 
-template <bool SW>
+template <bool SW, bool HALF>
 int launch_wide(hipStream_t s, const void* X, const void* W, void* Y, const int* offsets, const int* a_rows,
                 const float* scale, int M, int Nout, int K, int G) {
-  if (const int rc = allow_lds(wide_kernel<SW>, kWideLds)) return rc;
-  const int nblk8 = ((SW ? Nout / 2 : Nout) + (SW ? 1024 : 2048) - 1) / (SW ? 1024 : 2048) * 8;
-  const long long items = ((long long)M / kWideRows + G) * nblk8;
+  constexpr uint32_t lds = 3 * wide_stage(HALF);
+  if (const int rc = allow_lds(wide_kernel<SW, HALF>, lds)) return rc;
+  constexpr int of8 = SW || HALF ? 1024 : 2048;  // columns of Y of eight blocks
+  const int nblk8 = ((SW ? Nout / 2 : Nout) + of8 - 1) / of8 * 8;
+  const long long items = ((long long)M / wide_rows(HALF) + G) * nblk8;
   if (items > (1ll << 30)) return JLE_BAD_ARG;
-  hipLaunchKernelGGL(wide_kernel<SW>, dim3((unsigned)items), dim3(256), kWideLds, s, (const bf16_t*)X, (const bf16_t*)W,
+  hipLaunchKernelGGL((wide_kernel<SW, HALF>), dim3((unsigned)items), dim3(256), lds, s, (const bf16_t*)X, (const bf16_t*)W,
                      (bf16_t*)Y, offsets, a_rows, scale, Nout, K, G, nblk8);
   JLE_LAUNCH_CHECK();
   return 0;
@@ -454,7 +472,7 @@ JLE_API int jle_gemm_stream_supported(int Nout, int K, int swiglu) {
 }
 
 // X [*, K] bf16, W [G, Nout, K] bf16 in the streaming layout, Y [M, Nout] (or [M, Nout / 2] with swiglu) bf16 or
-// float32; X must have fewer than 2^32 elements (wide: 2^32 bytes).  wide: wide_kernel (groups, bfloat16 out).  max_rows: the most rows any group can have (M if unknown).
+// float32; X must have fewer than 2^32 elements (wide: 2^32 bytes).  wide: wide_kernel (groups, bfloat16 out), 2 (plain): HALF.  max_rows: the most rows any group can have (M if unknown).
 // Blocks are 8 wavefronts (two per SIMD, one block per compute unit): measured against 4, 5 and 6 on expert
 // shapes with even and with skewed numbers of rows per expert.
 JLE_API int jle_gemm_stream(const void* X, const void* W, void* Y, const int* offsets, const int* a_rows,
@@ -465,8 +483,9 @@ JLE_API int jle_gemm_stream(const void* X, const void* W, void* Y, const int* of
     if (offsets == nullptr || out_f32 || G < 1 || G > 65535 || !jle_gemm_stream_supported(Nout, K, swiglu) ||
         ((uintptr_t)X | (uintptr_t)W | (uintptr_t)Y) % 16)
       return JLE_BAD_ARG;
-    return swiglu ? launch_wide<true>(s, X, W, Y, offsets, a_rows, scale, M, Nout, K, G)
-                  : launch_wide<false>(s, X, W, Y, offsets, a_rows, scale, M, Nout, K, G);
+    if (swiglu) return launch_wide<true, false>(s, X, W, Y, offsets, a_rows, scale, M, Nout, K, G);
+    return wide == 2 ? launch_wide<false, true>(s, X, W, Y, offsets, a_rows, scale, M, Nout, K, G)
+                     : launch_wide<false, false>(s, X, W, Y, offsets, a_rows, scale, M, Nout, K, G);
   }
   if (G < 1 || G > 65535 || !jle_gemm_stream_supported(Nout, K, swiglu)) return JLE_BAD_ARG;
   if (max_rows <= 0 || max_rows > M) max_rows = M;

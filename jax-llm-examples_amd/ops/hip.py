@@ -1802,8 +1802,7 @@ class HipOps:
         rows on average in even groups 43 | 38, with 90 and 510 42 | 53; 4 with 40 % of the rows in one 45 | 55.  Over 180
         sizes of 8, 16 and 64 groups, even, from 0.3 to 1.7 of the mean, and one with 40 % of the rows, the choice is 15 %
         faster than passes on the average and 2 % from the better of the two, at worst 13 % slower than passes (groups of
-        192 rows each, what a pass holds; beside that 8 %: one group far fuller at 192 on average).  ``rows`` counts choices:
-        where some are of experts without rows, there are fewer.  Both sides measured (passes | tiles,
+        192 rows each, what a pass holds; beside that 8 %: one group far fuller at 192 on average).  Both sides measured (passes | tiles,
         us): 8 groups of 14,336 x 4,096 gate and up with 192 rows each 286 | 226, 256 368 | 309, 410 529 | 401, 700
         743 | 643; of 4,096 x 7,168 with 192 152 | 154, 410 275 | 163, 512 281 | 298, 700 302 | 329; of 8,192 x 2,048 gate
         and up with 410 152 | 121, 512 152 | 167; 16 of 16,384 x 5,120 with 160 523 | 541, 410 1,508 | 1,023, 700
@@ -1812,17 +1811,44 @@ class HipOps:
         if mean < HipOps.WIDE_GROUP_ROWS or groups < HipOps.WIDE_GROUPS:
             return False
 
-        def cost(most, start, a_row):
-            tiles = sum(-(-max(1.0, mean + d * mean ** 0.5) // most) for d in (-1, 0, 1)) / 3
-            blocks = row_blocks * groups * tiles
-            rounds = -(-blocks // 256) if blocks < 1024 else blocks / 256 + 0.5
-            return rounds * (start + a_row * mean / tiles)
+        cost = HipOps._stream_cost
+        return cost(mean, row_blocks * groups, 256, 0.95, 0.003) < cost(mean, row_blocks * groups, 192, 0.9, 0.0037)
 
-        return cost(256, 0.95, 0.003) < cost(192, 0.9, 0.0037)
+    @staticmethod
+    def _stream_cost(mean: float, blocks: int, most: int, start: float, a_row: float) -> float:
+        """Microseconds a stage of 64 k: ``blocks`` blocks of rows of W in all groups, their ``mean`` rows in tiles of up to
+        ``most``, a stage of a tile ``start + a_row`` a row."""
+        tiles = sum(-(-max(1.0, mean + d * mean ** 0.5) // most) for d in (-1, 0, 1)) / 3
+        blocks = blocks * tiles
+        rounds = -(-blocks // 256) if blocks < 1024 else blocks / 256 + 0.5
+        return rounds * (start + a_row * mean / tiles)
 
-    def gemm_stream(self, a, b, *, offsets=None, a_rows=None, scale=None, swiglu=False, out_f32=False, rows=None):
+    @staticmethod
+    @functools.lru_cache(maxsize=4096)
+    def stream_half(rows: int, groups: int, row_blocks: int) -> bool:
+        """Whether plain products take tiles of 128 rows of W (``row_blocks`` of them a group) by up to 288 of X: where a tile
+        of 256 leaves compute units without a block, or fills two rounds where these, half as long, fill two as well (a stage
+        measured at 0.55 + 0.0022 us a row).  Where the rounds are more than two, the wide tiles' better use of what they read
+        counts for more.  Few rows a group are the time of their weights' bytes: then only where these tiles are one round,
+        and with 112 rows on average, or half of one.  8 groups, passes | wide | these, us: 4,096 x 2,048 with 512 rows
+        101 | 113 | 87, 256 64 | 62 | 52, 330 60 | 55 | 67, 128 42 | 44 | 40, 64 31 | 36 | 37; 2,048 x 4,096 with 512
+        90 | 106 | 75, 410 85 | 93 | 66, 160 76 | 81 | 58, 64 52 | 58 | 45; 4,096 x 7,168 with 410 266 | 180 | 242, 190
+        140 | 165 | 135; 16 of 5,120 x 8,192 with 128 286 | 325 | 333, 256 530 | 435 | 458."""
+        mean, blocks = rows / groups, row_blocks * groups
+        if groups < HipOps.WIDE_GROUPS or mean < HipOps.WIDE_GROUP_ROWS and not (
+                mean >= 112 and blocks <= 256 or mean >= 48 and blocks <= 128):
+            return False
+        cost = HipOps._stream_cost
+        wide = -(-row_blocks // 2) * groups
+        half = cost(mean, blocks, 288, 0.55, 0.0022)
+        tiles = sum(-(-max(1.0, mean + d * mean ** 0.5) // 288) for d in (-1, 0, 1)) / 3
+        return blocks * tiles <= 512 and half < min(cost(mean, wide, 256, 0.95, 0.003), cost(mean, wide, 192, 0.9, 0.0037))
+
+    def gemm_stream(self, a, b, *, offsets=None, a_rows=None, scale=None, swiglu=False, out_f32=False, rows=None,
+                    expected=None):
         """bfloat16 product on MFMA for about a hundred rows per group and more, weights in the streaming layout and
-        read once per 192 rows of a group, or per tile of up to 256 (:meth:`stream_wide`; see ``gemm_stream.hip``)."""
+        read once per 192 rows of a group, or per tile of up to 256 or 288 (:meth:`stream_wide`, :meth:`stream_half`; see
+        ``gemm_stream.hip``).  ``expected``: how many of the rows are expected to belong to a group, if not all."""
         if b.dim() == 2:
             b = b.unsqueeze(0)
         g, nout, k = b.shape
@@ -1838,8 +1864,9 @@ class HipOps:
                               f"whole tiles of 16 weight rows (32 with the fused activation), got {nout} x {k}")
         out = torch.empty(m, nout // 2 if swiglu else nout, dtype=torch.float32 if out_f32 else torch.bfloat16,
                           device=a.device)
-        wide = (offsets is not None and not out_f32 and a.numel() < 2 ** 31 and not (a.data_ptr() | b.data_ptr()) % 16
-                and self.stream_wide(m, g, -(-nout // 256)))
+        wide, among = 0, m if expected is None else expected
+        if offsets is not None and not out_f32 and a.numel() < 2 ** 31 and not (a.data_ptr() | b.data_ptr()) % 16:
+            wide = 2 if not swiglu and self.stream_half(among, g, -(-nout // 128)) else self.stream_wide(among, g, -(-nout // 256))
         self._call("jle_gemm_stream", _p(a), _p(b), _p(out), _p(offsets), _p(a_rows), _p(scale), int(swiglu),
                    int(out_f32), m, nout, k, g, m, int(wide))
         return out
@@ -2369,12 +2396,12 @@ class HipOps:
         return y
 
     def moe_experts_scored(self, h, expert_ids, weights, w_up, w_down, activation: str = "relu2", tiled: bool = False,
-                           grouping=None, shared_weights=None, identity: bool = False):
+                           grouping=None, shared_weights=None, identity: int = 0):
         """``sum_j weights[j] * W_down[e_j] relu(W_up[e_j] h)^2``: the choices grouped by expert, the first product
         plain, the activation a kernel of its own, the weights the second product's row scale (applied to its float32
         sums); the sum over a token's choices stays in pieces (:class:`ExpertSum`).  ``activation = "swiglu"``: ``w_up`` holds
-        gate and up rows, the activation is part of the first product.  ``identity``: choices beyond the experts are identity
-        experts (they have no row; the sum adds the token's own).  ``shared_weights``: a SwiGLU expert of every token,
+        gate and up rows, the activation is part of the first product.  ``identity``: how many identity experts
+        choices beyond the experts name (they have no row; the sum adds the token's own).  ``shared_weights``: a SwiGLU expert of every token,
         unweighted; in steps of few tokens one more group of the two products."""
         if activation not in ("relu2", "swiglu"):
             raise KernelError(f"unknown activation {activation!r}")
@@ -2412,7 +2439,7 @@ class HipOps:
             if mfma and m <= 2 * self.SKINNY_MAX_ROWS:
                 return self._few_experts(x, w, swiglu=fused, tiled=tiled, **kw)
             if mfma and tiled and self.stream_supported(nout, kdim, fused):
-                return self.gemm_stream(x, w, swiglu=fused, **kw)
+                return self.gemm_stream(x, w, swiglu=fused, expected=m * e // (e + int(identity)), **kw)
             if mfma:
                 return self.gemm_grouped(x, w, swiglu=fused, tiled=tiled, **kw)
             if tiled:

@@ -852,7 +852,7 @@ class ReferenceOps:
         return ids.to(torch.int32), w * weight_scale, None
 
     def moe_experts_scored(self, h, expert_ids, weights, w_up, w_down, activation: str = "relu2", tiled: bool = False,
-                           grouping=None, shared_weights=None, identity: bool = False):
+                           grouping=None, shared_weights=None, identity: int = 0):
         """``sum_j weights[j] * W_down[e_j] act(W_up[e_j] h)`` per token, float32 result; ``w_up`` ``[E, F, D]``,
         ``w_down`` ``[E, D, F]``; ``act = relu2``: the square of relu.  ``swiglu``: ``w_up`` is ``[E, 2F, D]`` (gate
         rows, then up rows) and ``act`` gives ``silu(gate) * up``.  A choice ``e_j >= E`` is an identity expert: its

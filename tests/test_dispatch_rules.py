@@ -85,6 +85,13 @@ def test_few_groups_stay_with_passes(groups, rows, blocks, wide):
     assert HipOps.stream_wide(rows * groups, groups, blocks) == wide
 
 
+@pytest.mark.parametrize("groups, rows, blocks, half", [
+    (8, 512, 32, True), (8, 512, 16, True), (8, 410, 32, False), (8, 190, 32, True), (8, 330, 32, False), (8, 128, 32, True),
+    (8, 64, 32, False), (8, 64, 16, True), (16, 128, 40, False), (16, 256, 40, False), (4, 512, 16, False), (8, 700, 16, False)])
+def test_narrower_tiles_where_wide_ones_leave_compute_units_idle(groups, rows, blocks, half):
+    assert HipOps.stream_half(rows * groups, groups, blocks) == half
+
+
 @pytest.mark.parametrize("lens, heads, dk, dv, pays", [
     ([64], 16, 128, 128, False), ([256], 16, 128, 128, True), ([2048], 4, 64, 64, True), ([64] * 32, 16, 128, 128, True),
     ([80] * 25, 16, 128, 128, True), ([32] * 64, 16, 128, 128, False), ([36] * 64, 64, 128, 128, False),

@@ -1531,3 +1531,25 @@ def test_product_of_a_few_rows_refuses_what_it_cannot_read(ops):
         with pytest.raises(KernelError):
             ops.gemm_few(x, w)
     assert torch.equal(ops.linear(odd, b), torch.zeros(4, 16, device=DEV, dtype=torch.bfloat16))
+
+
+@pytest.mark.parametrize("counts,nout,k", [
+    ([1, 0, 63, 64, 65, 128, 129, 160], 96, 256),
+    ([287, 288, 289, 576, 577, 256, 257, 700, 1], 144, 512),  # one, two and three tiles of rows, a second block of W of one tile
+    ([3, 0, 300] * 50, 64, 256),                              # more groups than a look takes
+    ([192] * 8, 1168, 768)])                                  # more than eight blocks of W
+def test_narrower_tiles_of_the_weight_streaming_product(ops, counts, nout, k):
+    """The bits of the kernel that takes a group's rows in passes, rows gathered and scaled."""
+    from jax_llm_examples_amd.ops.layout import tile_
+    m, e = sum(counts), len(counts)
+    x, w = _rand(m + 3, k, dt=torch.bfloat16, seed=1), _rand(e, nout, k, dt=torch.bfloat16, scale=0.1, seed=2)
+    tile_(w)
+    off = torch.tensor([0] + counts).cumsum(0).int().to(DEV)
+    rows = torch.randperm(m + 3, generator=torch.Generator().manual_seed(3))[:m].int().to(DEV)
+    scale = _rand(m, seed=4)
+    got = []
+    for half in (False, True):
+        ops.stream_half, ops.stream_wide = (lambda *a, half=half: half), (lambda *a: False)
+        got.append(ops.gemm_stream(x, w, offsets=off, a_rows=rows, scale=scale, rows=m))
+    del ops.stream_half, ops.stream_wide
+    assert torch.equal(*got)
