@@ -291,6 +291,14 @@ class CacheManager:
         e = self.requests[rid]
         if e.reserved:
             raise AssertionError(f"request {rid!r} already has a reservation of {e.reserved} tokens")
+        if n_new == 1:  # (most decoded tokens: their page is there already)
+            j = e.num_tokens // self.page_size
+            for table in e.tables:
+                if j >= len(table) or table[j] < 0:
+                    break
+            else:
+                e.reserved = 1
+                return
         upto = e.num_tokens + n_new
         missing = [self._pages_missing(e, g, upto) for g in self.groups]
         for g, m in zip(self.groups, missing):
@@ -323,8 +331,10 @@ class CacheManager:
             keep_from = first_needed_position(g.retention, e.num_tokens)
             table = e.tables[g.index]
             # page j holds positions [j*ps, (j+1)*ps): free iff it lies wholly in [kept prefix, keep_from)
-            first = max(e.freed_upto[g.index], -(-kept_prefix(g.retention) // self.page_size))
             upto = min(len(table), keep_from // self.page_size)
+            if upto <= e.freed_upto[g.index]:
+                continue
+            first = max(e.freed_upto[g.index], -(-kept_prefix(g.retention) // self.page_size))
             gone = [j for j in range(first, upto) if table[j] >= 0]
             e.freed_upto[g.index] = max(e.freed_upto[g.index], upto)
             if gone:

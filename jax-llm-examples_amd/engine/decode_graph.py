@@ -40,6 +40,7 @@ class _Recording:
         self.stamps = [None] * R  # per row: the stamp of the block tables it holds (see fill_step)
         # two pinned staging buffers: the copy of one step may still be on its way when the next is laid out
         self.staging = [torch.empty(total, dtype=torch.int32, pin_memory=True) for _ in range(2)]
+        self.staging_np = [t.numpy() for t in self.staging]
         self.staged = [None, None]  # the event after each buffer's last copy
         self.turn = 0
         self.device_buf = torch.zeros(total, dtype=torch.int32, device=model.device)
@@ -51,17 +52,16 @@ class _Recording:
     def lay_out(self, cache, entries: Sequence[StepEntry], vocab_size: int) -> None:
         """This step's numbers into the mirror (every row's logits are computed; the caller picks the wanted
         ones), then one copy to the device."""
-        fill_step(self.layout, self.mirror, cache, [StepEntry(e.rid, e.tokens, (0,)) for e in entries], vocab_size,
-                  stamps=self.stamps)
+        fill_step(self.layout, self.mirror, cache, entries, vocab_size, stamps=self.stamps, every_row=True)
         b = self.turn
         self.turn ^= 1
-        if self.staged[b] is not None:
+        if self.staged[b] is None:
+            self.staged[b] = torch.cuda.Event()
+        else:
             self.staged[b].synchronize()
-        self.staging[b].numpy()[:] = self.mirror
+        self.staging_np[b][:] = self.mirror
         self.device_buf.copy_(self.staging[b], non_blocking=True)
-        ev = torch.cuda.Event()
-        ev.record()
-        self.staged[b] = ev
+        self.staged[b].record()
 
 
 class DecodeGraphs:

@@ -121,7 +121,7 @@ class Engine:
         if any(len(t) < 1 for t in prompts):
             raise ValueError("a prompt needs at least one token")
         done = [0] * len(prompts)
-        rows: dict = {}
+        kept, closed = [], []  # logits of the prompts that end in each step, and whose they are
         while any(d < len(t) for d, t in zip(done, prompts)):
             left, entries, closing = self.max_num_batched_tokens, [], []
             for j, t in enumerate(prompts):
@@ -135,11 +135,15 @@ class Engine:
                 done[j] += n
                 left -= n
             logits = self.runner.step(entries)
-            # (a step of single tokens hands out a buffer that the next such step writes again: what is kept
-            # and handed on is a copy)
-            for r, j in enumerate(closing):
-                rows[j] = logits[r].clone()
-        logits = torch.stack([rows[j] for j in range(len(prompts))])
+            if closing:
+                # (a step of single tokens hands out a buffer that the next such step writes again: what is kept
+                # and handed on is a copy)
+                kept.append(logits.clone() if all(len(e.tokens) == 1 for e in entries) else logits)
+                closed += closing
+        # (a step's tokens go to the prompts in their order, so they end in it)
+        if closed != list(range(len(prompts))):
+            raise AssertionError("prompts ended in another order than they were given")
+        logits = kept[0] if len(kept) == 1 else torch.cat(kept)
         return self._greedy(logits), logits, ids
 
     def decode_step(self, last_tokens: Sequence[int], ids: Sequence):

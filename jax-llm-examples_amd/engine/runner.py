@@ -48,11 +48,12 @@ class ModelRunner:
         graph (:mod:`.decode_graph`); its logits then lie in that recording's buffer, which the next
         step of the same shape writes again."""
         cache = self.cache
-        seen = set()
-        for e in entries:
-            if e.rid in seen:
-                raise ValueError(f"request {e.rid!r} appears twice in one step")
-            seen.add(e.rid)
+        if len({e.rid for e in entries}) != len(entries):
+            seen = set()
+            for e in entries:
+                if e.rid in seen:
+                    raise ValueError(f"request {e.rid!r} appears twice in one step")
+                seen.add(e.rid)
         added, reserved = [], []
         try:
             for e in entries:

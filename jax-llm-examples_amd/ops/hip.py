@@ -14,6 +14,7 @@ from typing import Optional
 import torch
 
 from . import build as _build
+from .transfer import to_device
 
 # the rules under which the attention kernels here read keys ("window_keep": the general kernel alone)
 _RET_MODES = {"all": 0, "chunk": 1, "window": 2, "window_keep": 2}
@@ -378,7 +379,7 @@ class HipOps:
                     flat += [i, o + t, min(per, ln - t)]
                 firsts.append(len(flat) // 3)
                 o += ln
-            both = torch.tensor(flat + firsts, dtype=torch.int32).to(device)
+            both = to_device(torch.tensor(flat + firsts, dtype=torch.int32), device)
             table = ctx.scratch[key] = (both[: len(flat)], both[len(flat):], len(flat) // 3)
         return table
 
@@ -720,7 +721,7 @@ class HipOps:
                 for t in range(0, rows, 16):
                     flat += [o * H + t, min(16, rows - t)]
                 o += ln
-            plan = torch.tensor(flat, dtype=torch.int32).to(device)
+            plan = to_device(torch.tensor(flat, dtype=torch.int32), device)
             if meta is not None:
                 meta.meta[key] = plan
         return plan
@@ -752,7 +753,7 @@ class HipOps:
                     o += ln
                 keyed.sort()
                 flat = [v for _, _, row0, nrows in keyed for v in (row0, nrows)]
-                blocks = torch.tensor(flat, dtype=torch.int32).to(q_lat.device)
+                blocks = to_device(torch.tensor(flat, dtype=torch.int32), q_lat.device)
                 if meta is not None:
                     meta.meta[key] = blocks
             self._call("jle_latent_attention_lds", _p(q_lat), _p(q), q_ld, dn, dr, _p(latent_pages),
@@ -871,7 +872,7 @@ class HipOps:
             return None
         table, ns = held.get(key + "_table"), len(spans)
         if table is None:
-            table = held[key + "_table"] = torch.tensor(spans + blocks, dtype=torch.int32).to(q.device)
+            table = held[key + "_table"] = to_device(torch.tensor(spans + blocks, dtype=torch.int32), q.device)
         np_, ps = latent_pages.shape[0], latent_pages.shape[1]
         if q.stride(2) != 1 or q.stride(1) != dq:
             raise KernelError("the heads' queries must lie side by side at the start of contiguous rows")
@@ -1351,7 +1352,7 @@ class HipOps:
                     for t in range(0, ln, per):
                         chunks += [i, o + t, min(per, ln - t)]
                 o += ln
-            both = torch.tensor(chunks + segs, dtype=torch.int32).to(device)
+            both = to_device(torch.tensor(chunks + segs, dtype=torch.int32), device)
             made = ctx.scratch["delta_chunks"] = (both[: len(chunks)], both[len(chunks):], len(chunks) // 3, len(segs) // 3)
         nc = made[2]
         if nc * kib * 1024 > self.DELTA_CHUNK_BYTES:
@@ -2120,7 +2121,7 @@ class HipOps:
             keyed.sort()
             groups = [v for _, _, quad in keyed for v in quad]
         flat = dec + tiles + groups
-        flat = torch.tensor(flat, dtype=torch.int32).to(device) if flat else None
+        flat = to_device(torch.tensor(flat, dtype=torch.int32), device) if flat else None
         nd, nt = len(dec), len(tiles)
         return {"num_dec": nd, "num_tiles": nt // 2, "max_splits": max_splits, "split": split,
                 "dec": flat[:nd] if dec else None, "tiles": flat[nd: nd + nt] if tiles else None,
@@ -2221,7 +2222,7 @@ class HipOps:
                     for t in range(0, ln, self.F32_TILE):
                         flat += [o + t, min(self.F32_TILE, ln - t)]
                     o += ln
-                tiles = torch.tensor(flat, dtype=torch.int32).to(q.device)
+                tiles = to_device(torch.tensor(flat, dtype=torch.int32), q.device)
                 if meta is not None:
                     meta.meta["f32_tiles"] = tiles
             self._call("jle_attention_f32_tiles", _p(q), _p(kv_cache), _p(out), _p(positions), _p(token_segment),
@@ -2305,7 +2306,7 @@ class HipOps:
                         for t in range(0, ln, self.PREFILL_TILE):
                             flat += [o + t, min(self.PREFILL_TILE, ln - t)]
                         o += ln
-                    tiles = torch.tensor(flat, dtype=torch.int32).to(q.device)
+                    tiles = to_device(torch.tensor(flat, dtype=torch.int32), q.device)
                     if meta is not None:
                         meta.meta["kept_tiles"] = tiles
                 self._call("jle_attention_prefill_kept", _p(q), _p(kv_cache), _p(out), _p(positions),

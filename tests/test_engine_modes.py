@@ -282,3 +282,51 @@ def test_gpu_bfloat16_expert_choices_differ_only_at_near_ties(model_dirs_bf16, n
                 margin = (torch.gather(scores, 1, want) - torch.gather(scores, 1, got)).abs().max(-1).values
                 assert (margin[diff] < 0.05 * scores.std()).all(), f"{rid} layer {li}: a clear choice went wrong"
     assert flips <= 0.05 * total
+
+
+def test_single_tokens_are_laid_out_like_the_tokens_of_any_step():
+    """The lists that a step of single tokens is gathered in give what the general way writes for the same entries (with an
+    entry of two tokens behind them), with and without block tables kept from the step before."""
+    import numpy as np
+    from jax_llm_examples_amd.cache.manager import CacheManager
+    from jax_llm_examples_amd.engine.batch import StepEntry, StepLayout, fill_step
+    from jax_llm_examples_amd.parts.base import CacheNeed
+
+    needs = {0: CacheNeed(kv=(1, 4), retention=("all",)), 1: CacheNeed(kv=(2, 4), retention=("window", 5))}
+    cache = CacheManager(needs, page_size=4, num_pages=64, max_requests=8, dtype=torch.float32, device="cpu")
+    lens = [1, 3, 4, 9, 17]
+    for i, n in enumerate(lens):
+        cache.add_request(i)
+        cache.reserve(i, n)
+        cache.commit(i, last_token=100 + i)
+    cache.add_request("two")
+    stamps = [None] * len(lens)
+    kept = None
+    for step in range(6):
+        entries = [StepEntry(i, [7 * i + step], [0] if (i + step) % 2 else []) for i in range(len(lens))]
+        for e in entries:
+            cache.reserve(e.rid, 1)
+        cache.reserve("two", 2)
+        widths = [8, 8]
+        wanted = sum(len(e.want) for e in entries)
+        one, more = StepLayout(5, 5, wanted, widths), StepLayout(7, 6, wanted, widths)
+        flat, general = np.full(one.size, -9, np.int32), np.full(more.size, -9, np.int32)
+        seg = fill_step(one, flat, cache, entries, 1000)
+        fill_step(more, general, cache, [*entries, StepEntry("two", [1, 2], [])], 1000)
+        for name, (lo, hi) in one.bounds.items():
+            assert flat[lo:hi].tolist() == more.view(general, name)[: hi - lo].tolist(), name
+        assert seg == ([1] * 5, [cache.num_tokens(i) for i in range(5)])
+        every = StepLayout(5, 5, 5, widths)
+        kept = np.full(every.size, -9, np.int32) if kept is None else kept
+        fill_step(every, kept, cache, entries, 1000, stamps=stamps, every_row=True)
+        assert every.view(kept, "logits_indices").tolist() == list(range(5))
+        for name in one.bounds:
+            assert name == "logits_indices" or every.view(kept, name).tolist() == one.view(flat, name).tolist(), name
+        with pytest.raises(ValueError):
+            fill_step(one, flat.copy(), cache, [StepEntry(0, [1000], []), *entries[1:]], 1000)
+        with pytest.raises(ValueError):
+            fill_step(one, flat.copy(), cache, [StepEntry(0, [1], [1]), *entries[1:]], 1000)
+        cache.cancel("two")
+        for e in entries:
+            cache.commit(e.rid, last_token=e.tokens[0])
+        cache.check()
