@@ -123,7 +123,9 @@ __global__ __launch_bounds__(THREADS) void add_rmsnorm_reg_kernel(float* __restr
 }
 
 // Rows whose width is a multiple of 8 (and 16-byte aligned arrays): a thread takes CPT pieces of 4
-// neighbouring elements, piece = thread, thread + THREADS, ...; up to THREADS * CPT * 4 wide.
+// neighbouring elements, piece = thread, thread + THREADS, ...; up to THREADS * CPT * 4 wide.  A step of few tokens waits for
+// the kernel's code too, which is fetched and run through once: pieces past the row's end cost as much as the others (16 rows
+// of 2,048: 7.0 us with the eight pieces of the widest row, 5.8 with its two; one of 5,120 6.6 with eight, 6.3 with six).
 template <typename DT, typename OT, int THREADS, int CPT, bool STREAM>
 __global__ __launch_bounds__(THREADS, 4) void add_rmsnorm_vec_kernel(float* __restrict__ x, Delta<DT> delta,
                                                                   const float* __restrict__ w, float eps,
@@ -219,13 +221,23 @@ static void launch_add_rmsnorm(float* x, Delta<DT> delta, const float* w, float 
   const uintptr_t all = (uintptr_t)x | (uintptr_t)delta.plain | (uintptr_t)delta.routed | (uintptr_t)delta.shared |
                         (uintptr_t)delta.self | (uintptr_t)w | (uintptr_t)out | (uintptr_t)out32;
   if (D % 8 == 0 && (all & 15) == 0 && D > 1024 && D <= 8192) {  // (rows of any of the arrays then start 16-byte aligned)
-    // (the same arithmetic either way: only where the data are kept differs)
-    if ((size_t)N * D >= ((size_t)4 << 20))
-      hipLaunchKernelGGL((add_rmsnorm_vec_kernel<DT, OT, 256, 8, true>), g, dim3(256), 0, s, x, delta, w, eps,
-                         (OT*)out, out32, D);
-    else
-      hipLaunchKernelGGL((add_rmsnorm_vec_kernel<DT, OT, 256, 8, false>), g, dim3(256), 0, s, x, delta, w, eps,
-                         (OT*)out, out32, D);
+    // (the same arithmetic either way: only where the data are kept differs, and how many pieces past the row's end are
+    // left out, see add_rmsnorm_vec_kernel)
+    const bool stream = (size_t)N * D >= ((size_t)4 << 20);
+#define GO(CPT)                                                                                                          \
+  do {                                                                                                                   \
+    if (stream)                                                                                                          \
+      hipLaunchKernelGGL((add_rmsnorm_vec_kernel<DT, OT, 256, CPT, true>), g, dim3(256), 0, s, x, delta, w, eps, (OT*)out, \
+                         out32, D);                                                                                      \
+    else                                                                                                                 \
+      hipLaunchKernelGGL((add_rmsnorm_vec_kernel<DT, OT, 256, CPT, false>), g, dim3(256), 0, s, x, delta, w, eps,        \
+                         (OT*)out, out32, D);                                                                            \
+  } while (0)
+    if (D <= 2048) GO(2);
+    else if (D <= 4096) GO(4);
+    else if (D <= 6144) GO(6);
+    else GO(8);
+#undef GO
   }
   else if (D <= 1024)
     hipLaunchKernelGGL((add_rmsnorm_reg_kernel<DT, OT, 256, 4>), g, dim3(256), 0, s, x, delta, w, eps, (OT*)out, out32,
