@@ -7,6 +7,7 @@
 // channel, and whose mixer may be two mixers side by side with a weight each.  One block per row, the row in
 // registers (wider rows are read again); every sum in an order that depends on the width alone.
 #include "common.h"
+#include "rows.h"
 
 using namespace jle;
 
@@ -162,6 +163,90 @@ __global__ __launch_bounds__(THREADS) void scaled_add_norm_kernel(ScaledArgs p) 
   }
 }
 
+// Rows whose width is a multiple of 4, all arrays at 16 bytes: a thread takes PIECES pieces of four neighbours.  A step of few
+// tokens waits for the kernel's code, which is fetched and run through once (asking for everything up front, element by
+// element, gained nothing): a
+// fourth of the loads and tests.  64 rows of 2,048 with two pieces of an expert sum 9.9 -> 5.9 us, 2,048 rows 15.6 -> 12.1.
+template <int PIECES, typename AT, typename BT>
+__global__ __launch_bounds__(256) void scaled_add_norm_vec_kernel(ScaledArgs p) {
+  __shared__ float red[4];
+  const size_t base = (size_t)blockIdx.x * p.D;
+  const int D = p.D;
+  const AT* __restrict__ pa = (const AT*)p.a;
+  const BT* __restrict__ pb = (const BT*)p.b;
+  const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
+  f32x4_t v[PIECES], t[PIECES], w[PIECES];
+  auto at = [&](int i) { return ((int)threadIdx.x + 256 * i) * 4; };
+#pragma unroll
+  for (int i = 0; i < PIECES; ++i) {
+    v[i] = at(i) < D ? load4<float>(p.x + base + at(i)) : zero;
+    w[i] = (p.w != nullptr && at(i) < D) ? load4<float>(p.w + at(i)) : f32x4_t{1.f, 1.f, 1.f, 1.f};
+    t[i] = zero;
+  }
+  if (pa != nullptr) {
+    if (p.a_inv != nullptr) {  // (the pieces of an expert sum, added up in their order from zero, two on their way)
+      const int* rows = p.a_inv + (size_t)blockIdx.x * p.a_k;
+      for (int j = 0; j < p.a_k; j += 2) {
+        const bool two = j + 1 < p.a_k;
+        const AT* a0 = pa + (size_t)rows[j] * D;
+        const AT* a1 = pa + (size_t)rows[two ? j + 1 : j] * D;
+        f32x4_t q0[PIECES], q1[PIECES];
+#pragma unroll
+        for (int i = 0; i < PIECES; ++i) {
+          q0[i] = at(i) < D ? load4<AT>(a0 + at(i)) : zero;
+          q1[i] = at(i) < D ? load4<AT>(a1 + at(i)) : zero;
+        }
+#pragma unroll
+        for (int i = 0; i < PIECES; ++i) {
+          t[i] += q0[i];
+          if (two) t[i] += q1[i];
+        }
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < PIECES; ++i) t[i] = at(i) < D ? load4<AT>(pa + base + at(i)) : zero;
+    }
+#pragma unroll
+    for (int i = 0; i < PIECES; ++i) t[i] *= p.fa;
+    if (pb != nullptr) {
+#pragma unroll
+      for (int i = 0; i < PIECES; ++i) {
+        const f32x4_t u = at(i) < D ? load4<BT>(pb + base + at(i)) : zero;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) t[i][e] = __builtin_fmaf(p.fb, u[e], t[i][e]);
+      }
+    }
+    if (p.vec != nullptr) {
+#pragma unroll
+      for (int i = 0; i < PIECES; ++i) {
+        const f32x4_t u = at(i) < D ? load4<float>(p.vec + at(i)) : zero;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[i][e] = __builtin_fmaf(u[e], t[i][e], v[i][e]);
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < PIECES; ++i) v[i] += t[i];
+    }
+#pragma unroll
+    for (int i = 0; i < PIECES; ++i)
+      if (at(i) < D) store4<float>(p.x + base + at(i), v[i]);
+  }
+  if (p.h == nullptr) return;
+  float ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < PIECES; ++i) ss = add_squares4(ss, v[i]);
+  const float inv = 1.0f / sqrtf(block_sum<256>(ss, red) / (float)D + p.eps);
+#pragma unroll
+  for (int i = 0; i < PIECES; ++i) {
+    if (at(i) >= D) continue;
+    f32x4_t h = v[i] * inv;
+    if (p.w != nullptr) h *= w[i];
+    if (p.h_bf16) store4<bf16_t>((bf16_t*)p.h + base + at(i), h);
+    else store4<float>((float*)p.h + base + at(i), h);
+    if (p.h32 != nullptr) store4<float>(p.h32 + base + at(i), h);
+  }
+}
+
 template <int THREADS>
 __global__ __launch_bounds__(THREADS) void scaled_add_norm_wide_kernel(ScaledArgs p) {
   __shared__ float red[THREADS / 64];
@@ -194,10 +279,16 @@ JLE_API int jle_scaled_add_norm(float* x, const void* a, int a_kind, float fa, c
       (b != nullptr && a == nullptr) || (h == nullptr && h32 != nullptr) || (a_inv != nullptr && (a == nullptr || a_k < 1)))
     return JLE_BAD_ARG;
   ScaledArgs p{x, a, b, vec, w, h, h32, fa, fb, eps, a_kind == 1, b_kind == 1, h_bf16, D, a_inv, a_k};
-  // (which kernel: by the width and the terms' types alone, never by the step's size)
+  // (which kernel: by the width, the arrays' alignment and the terms' types alone, never by the step's size)
+  const bool vec4 = D % 4 == 0 && D > 256 && D <= 8192 &&
+                    (((uintptr_t)x | (uintptr_t)a | (uintptr_t)b | (uintptr_t)vec | (uintptr_t)w | (uintptr_t)h | (uintptr_t)h32) & 15) == 0;
 #define JLE_SCALED(AT, BT)                                                                                \
   do {                                                                                                    \
-    if (D <= 256) hipLaunchKernelGGL((scaled_add_norm_kernel<64, 4, AT, BT>), dim3(N), dim3(64), 0, s, p);  \
+    if (vec4 && D <= 1024) hipLaunchKernelGGL((scaled_add_norm_vec_kernel<1, AT, BT>), dim3(N), dim3(256), 0, s, p); \
+    else if (vec4 && D <= 2048) hipLaunchKernelGGL((scaled_add_norm_vec_kernel<2, AT, BT>), dim3(N), dim3(256), 0, s, p); \
+    else if (vec4 && D <= 4096) hipLaunchKernelGGL((scaled_add_norm_vec_kernel<4, AT, BT>), dim3(N), dim3(256), 0, s, p); \
+    else if (vec4) hipLaunchKernelGGL((scaled_add_norm_vec_kernel<8, AT, BT>), dim3(N), dim3(256), 0, s, p); \
+    else if (D <= 256) hipLaunchKernelGGL((scaled_add_norm_kernel<64, 4, AT, BT>), dim3(N), dim3(64), 0, s, p);  \
     else if (D <= 1024) hipLaunchKernelGGL((scaled_add_norm_kernel<256, 4, AT, BT>), dim3(N), dim3(256), 0, s, p); \
     else if (D <= 2048) hipLaunchKernelGGL((scaled_add_norm_kernel<256, 8, AT, BT>), dim3(N), dim3(256), 0, s, p); \
     else if (D <= 4096) hipLaunchKernelGGL((scaled_add_norm_kernel<256, 16, AT, BT>), dim3(N), dim3(256), 0, s, p); \
