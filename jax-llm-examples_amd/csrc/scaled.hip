@@ -165,8 +165,8 @@ __global__ __launch_bounds__(THREADS) void scaled_add_norm_kernel(ScaledArgs p) 
 
 // Rows whose width is a multiple of 4, all arrays at 16 bytes: a thread takes PIECES pieces of four neighbours.  A step of few
 // tokens waits for the kernel's code, which is fetched and run through once (asking for everything up front, element by
-// element, gained nothing): a
-// fourth of the loads and tests.  64 rows of 2,048 with two pieces of an expert sum 9.9 -> 5.9 us, 2,048 rows 15.6 -> 12.1.
+// element, gained nothing): a fourth of the loads and tests.
+// 64 rows of 2,048 with two pieces of an expert sum 9.9 -> 5.9 us, 2,048 rows 15.6 -> 12.1.
 template <int PIECES, typename AT, typename BT>
 __global__ __launch_bounds__(256) void scaled_add_norm_vec_kernel(ScaledArgs p) {
   __shared__ float red[4];

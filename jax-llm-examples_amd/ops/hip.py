@@ -1665,9 +1665,9 @@ class HipOps:
                    nout, k, g, m)
         return out
 
-    SKINNY_MAX_ROWS = 64  # up to here a product is a stream of the weights: the MFMA weight-streaming kernel
+    SKINNY_MAX_ROWS = 64  # up to here (twice that many choices of experts) a product is a stream of the weights
     SKINNY_DENSE_ROWS = 16  # the fused gate|up projection of a dense feed-forward: beyond this the BLAS library
-    SKINNY_LINEAR_ROWS = 8  # plain projections (q|k|v, o, down)
+    SKINNY_LINEAR_ROWS = 8  # plain projections (q|k|v, o, down) that gemm_few.hip does not take
     SHARED_RIDES_ROWS = 16  # a shared expert's two products ride in the routed experts' launches as one more group
 
     SLICE_TICKETS = 1 << 14
