@@ -1553,3 +1553,32 @@ def test_narrower_tiles_of_the_weight_streaming_product(ops, counts, nout, k):
         got.append(ops.gemm_stream(x, w, offsets=off, a_rows=rows, scale=scale, rows=m))
     del ops.stream_half, ops.stream_wide
     assert torch.equal(*got)
+
+
+@pytest.mark.parametrize("d", [256, 260, 1024, 1028, 2048, 2052, 4096, 4100, 8192, 8196, 2050])
+@pytest.mark.parametrize("k", [0, 1, 2, 3])
+def test_sum_with_factors_by_pieces_of_four(ops, d, k):
+    """Widths at the edges of the pieces a thread takes, and those that go element by element; a plain term (k = 0) or one to
+    three pieces of an expert sum, a second term, a scale a channel."""
+    from jax_llm_examples_amd.ops.hip import ExpertSum
+    from jax_llm_examples_amd.parts.residual import ScaledSum
+
+    g = torch.Generator().manual_seed(d + k)
+    n = 5
+    bf = lambda *s: torch.randn(*s, generator=g).to(DEV, torch.bfloat16)
+    x, b = torch.randn(n, d, generator=g).to(DEV), bf(n, d)
+    vec, w = (torch.rand(d, generator=g).to(DEV) + 0.5 for _ in range(2))
+    if k:
+        inv, rows = torch.randperm(n * k, generator=g).int().to(DEV), bf(n * k, d)
+        a, plain = ExpertSum(rows, inv, k, None, n, d), rows.double()[inv.long()].view(n, k, d).sum(1)
+    else:
+        a = bf(n, d)
+        plain = a.double()
+    want = x.double() + vec.double() * (0.7 * plain + 1.3 * b.double())
+    h, h32 = ops.scaled_add_norm(x, ScaledSum([(a, 0.7), (b, 1.3)], vec), w, 1e-5, torch.bfloat16, want32=True)
+    normed = want / torch.sqrt((want ** 2).mean(-1, keepdim=True) + 1e-5) * w.double()
+    # (a few roundings of 2^-24 of what is added up; the row's statistics another few)
+    size = x.double().abs() + want.abs() + vec.double() * (0.7 * plain.abs() + 1.3 * b.double().abs()) + 4
+    assert ((x.double() - want).abs() <= 8 * 2.0 ** -24 * size).all()
+    assert ((h32.double() - normed).abs() <= 32 * 2.0 ** -24 * (size + normed.abs())).all()
+    assert torch.equal(h, h32.bfloat16())
