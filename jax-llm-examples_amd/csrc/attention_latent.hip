@@ -1023,7 +1023,8 @@ __global__ __launch_bounds__(512) void latent_values_kernel(const float* __restr
       }
 #pragma unroll
       for (int u = 0; u < U; ++u) {
-        const float wgt = s0 + u < splits ? expf(ms[u] - mx) : 0.f;  // (a range without keys: 0 too)
+        // (a range without keys, or whose scores are all -inf: 0 too, also while there is no finite maximum yet)
+        const float wgt = s0 + u < splits && ms[u] != -INFINITY ? expf(ms[u] - mx) : 0.f;
         l += ls[u] * wgt;
 #pragma unroll
         for (int i = 0; i < E; ++i)

@@ -243,3 +243,29 @@ def test_few_rows_through_the_latent_and_out_of_it(segs, window, sink, H, R, dv,
         want = torch.einsum("hr,hvr->hv", out, uv.view(H, dv, R).double())
         # probabilities, sums and the result rounded to bfloat16: 2^-9 each at most
         assert (got[t] - want).norm() < 4 * 2.0 ** -9 * want.norm(), (t, float((got[t] - want).norm() / want.norm()))
+
+
+@pytest.mark.gpu
+def test_ranges_whose_scores_are_all_minus_infinity_add_nothing():
+    """The first 640 keys' scores overflow to minus infinity: five ranges of 128, as many as the merge takes at a time, have
+    no finite maximum before the first that has one."""
+    dev, H, R, dv, ps, pos, low = "cuda:0", 16, 64, 32, 16, 1000, 640
+    ops = HipOps(dev)
+    g = torch.Generator().manual_seed(5)
+    bf = lambda *s, std=1.0: (torch.randn(*s, generator=g) * std).to(torch.bfloat16)
+    latent, rope = bf(64, ps, R), bf(64, ps, DR)
+    q, q_lat, uv = bf(1, H, DN + DR), bf(H, 1, R), bf(H * dv, R, std=R ** -0.5)
+    latent[:, :, 0], q_lat[:, :, 0] = 0.0, 1e30
+    latent[: low // ps, :, 0] = -1e30
+    table, one = torch.arange(64, dtype=torch.int32).view(1, -1), torch.zeros(1, dtype=torch.int32)
+    meta = GroupContext(block_table=None, slot_mapping=None, width=64, retention=("all",), seg_lens=[1], seg_starts=[pos],
+                        decode_bucket=1024)
+    scale = (DN + DR) ** -0.5
+    d = lambda t: t.to(dev)
+    got = ops.latent_values(d(q_lat), d(q), DN, d(latent), d(rope), d(table), d(one + pos), d(one), None, scale, d(uv), meta=meta,
+                            latent_t_pages=d(latent.transpose(1, 2).contiguous()).view(-1, ps, R)).cpu().double().view(H, dv)
+    c, kr = latent.view(-1, R)[low: pos + 1].double(), rope.view(-1, DR)[low: pos + 1].double()
+    out = torch.softmax((q_lat[:, 0].double() @ c.T + q[0, :, DN:].double() @ kr.T) * scale, -1) @ c
+    want = torch.einsum("hr,hvr->hv", out, uv.view(H, dv, R).double())
+    # probabilities, sums and the result rounded to bfloat16: 2^-9 each at most
+    assert (got - want).norm() < 4 * 2.0 ** -9 * want.norm()
