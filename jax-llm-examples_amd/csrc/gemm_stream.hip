@@ -242,8 +242,8 @@ __global__ __launch_bounds__(WAVES * 64, 2) void gemm_stream_kernel(const bf16_t
 // too 422 and 188 at 8 groups: reading and bringing in together took shared memory as long as the products.)
 // HALF (plain products): a block takes 128 rows of W and up to 288 of X, its wavefronts in twos by twos, 64 rows of W and half
 // of X each.  It reads twice as much for a product, but where blocks of 256 would fill a part of the compute units or of their
-// last round it is the faster: 8 groups of 2,048 x 4,096 with 512 rows 90 us in passes, 106 in wide tiles (128 blocks; a
-// group of more than 512 rows makes three tiles), 75 so.  (All of 288 rows in wide tiles spills registers: 10 times slower.)
+// last round it is the faster: 8 groups of 2,048 x 4,096 with 300 rows 84 us in passes, 80 in wide tiles (128
+// blocks, two tiles a group), 64 so.  (All of 288 rows in wide tiles spills registers: 10 times slower.)
 // Work items: a group's rows in tiles of at most 256 (288), as even as multiples of 32 allow; item = ((row block / 8) * tiles +
 // tile) * 8 + row block % 8 within a group, so that the tiles that read the same weights run on one chiplet.
 constexpr int wide_rows(bool half) { return half ? 288 : 256; }                            // of X, of a block

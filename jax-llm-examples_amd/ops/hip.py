@@ -1812,38 +1812,35 @@ class HipOps:
         if mean < HipOps.WIDE_GROUP_ROWS or groups < HipOps.WIDE_GROUPS:
             return False
 
-        cost = HipOps._stream_cost
-        return cost(mean, row_blocks * groups, 256, 0.95, 0.003) < cost(mean, row_blocks * groups, 192, 0.9, 0.0037)
+        def cost(most, start, a_row):
+            tiles = sum(-(-max(1.0, mean + d * mean ** 0.5) // most) for d in (-1, 0, 1)) / 3
+            blocks = row_blocks * groups * tiles
+            rounds = -(-blocks // 256) if blocks < 1024 else blocks / 256 + 0.5
+            return rounds * (start + a_row * mean / tiles)
 
-    @staticmethod
-    def _stream_cost(mean: float, blocks: int, most: int, start: float, a_row: float) -> float:
-        """Microseconds a stage of 64 k: ``blocks`` blocks of rows of W in all groups, their ``mean`` rows in tiles of up to
-        ``most``, a stage of a tile ``start + a_row`` a row."""
-        tiles = sum(-(-max(1.0, mean + d * mean ** 0.5) // most) for d in (-1, 0, 1)) / 3
-        blocks = blocks * tiles
-        rounds = -(-blocks // 256) if blocks < 1024 else blocks / 256 + 0.5
-        return rounds * (start + a_row * mean / tiles)
+        return cost(256, 0.95, 0.003) < cost(192, 0.9, 0.0037)
 
     @staticmethod
     @functools.lru_cache(maxsize=4096)
     def stream_half(rows: int, groups: int, row_blocks: int) -> bool:
-        """Whether plain products take tiles of 128 rows of W (``row_blocks`` of them a group) by up to 288 of X: where a tile
-        of 256 leaves compute units without a block, or fills two rounds where these, half as long, fill two as well (a stage
-        measured at 0.55 + 0.0022 us a row).  Where the rounds are more than two, the wide tiles' better use of what they read
-        counts for more.  Few rows a group are the time of their weights' bytes: then only where these tiles are one round,
-        and with 112 rows on average, or half of one.  8 groups, passes | wide | these, us: 4,096 x 2,048 with 512 rows
-        101 | 113 | 87, 256 64 | 62 | 52, 330 60 | 55 | 67, 128 42 | 44 | 40, 64 31 | 36 | 37; 2,048 x 4,096 with 512
-        90 | 106 | 75, 410 85 | 93 | 66, 160 76 | 81 | 58, 64 52 | 58 | 45; 4,096 x 7,168 with 410 266 | 180 | 242, 190
-        140 | 165 | 135; 16 of 5,120 x 8,192 with 128 286 | 325 | 333, 256 530 | 435 | 458."""
-        mean, blocks = rows / groups, row_blocks * groups
-        if groups < HipOps.WIDE_GROUPS or mean < HipOps.WIDE_GROUP_ROWS and not (
-                mean >= 112 and blocks <= 256 or mean >= 48 and blocks <= 128):
-            return False
-        cost = HipOps._stream_cost
-        wide = -(-row_blocks // 2) * groups
-        half = cost(mean, blocks, 288, 0.55, 0.0022)
-        tiles = sum(-(-max(1.0, mean + d * mean ** 0.5) // 288) for d in (-1, 0, 1)) / 3
-        return blocks * tiles <= 512 and half < min(cost(mean, wide, 256, 0.95, 0.003), cost(mean, wide, 192, 0.9, 0.0037))
+        """Whether plain products take tiles of 128 rows of W (``row_blocks`` of them a group) by up to 288 of X.  They are for
+        launches whose wide tiles or passes would leave compute units without a block: a block takes half as long, which pays
+        if all of them start together and is lost if one is left over.  So they have to fit one round of the 256 compute units
+        however the rows are shared out, which is known on the device only: a group is taken to have half a tile more than its
+        rows fill, and an eighth of the round stays free.  Row blocks count in eights, as they are dealt to the eight chiplets
+        (of groups of 256 rows of W all blocks are on two of them: 64 such groups up to 2.1 times the time of passes).  Few rows a group are
+        the time of their weights' bytes.
+
+        Measured over 22 matrices, 8 to 128 groups and 24 means from 48 to 800 rows, each even, drawn, uneven by a quarter,
+        from 0.3 to 1.7 of the mean and with 40 % of the rows in one group: where these tiles are taken they are 12 % faster
+        than what else would be on the average, at worst 16 % slower (24 groups of 1,024 x 4,096 with 145 rows, 40 % in one).
+        Taken wherever even groups would fill one round or two, they were up to 67 % slower (8 of 4,096 x 7,168 with 256 rows:
+        even 199 | 168 us, 40 % in one 154 | 257).  What else would be | these, us, even and with 40 % in one: 8 of 2,048 x 4,096
+        with 128 rows 62 | 59 and 79 | 67, 230 84 | 74 and 79 | 72, 300 80 | 64 and 100 | 73; 8 of 1,024 x 8,192 with 512
+        152 | 133 and 151 | 147."""
+        slots = -(-row_blocks // 8) * 8 * groups
+        mean = rows / groups
+        return groups >= HipOps.WIDE_GROUPS and mean >= 90 and slots <= 192 and slots * (mean / 288 + 0.5) <= 224
 
     def gemm_stream(self, a, b, *, offsets=None, a_rows=None, scale=None, swiglu=False, out_f32=False, rows=None,
                     expected=None):

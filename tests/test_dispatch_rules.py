@@ -86,10 +86,29 @@ def test_few_groups_stay_with_passes(groups, rows, blocks, wide):
 
 
 @pytest.mark.parametrize("groups, rows, blocks, half", [
-    (8, 512, 32, True), (8, 512, 16, True), (8, 410, 32, False), (8, 190, 32, True), (8, 330, 32, False), (8, 128, 32, True),
-    (8, 64, 32, False), (8, 64, 16, True), (16, 128, 40, False), (16, 256, 40, False), (4, 512, 16, False), (8, 700, 16, False)])
+    (8, 512, 32, False), (8, 512, 16, False), (8, 410, 32, False), (8, 190, 32, False), (8, 330, 32, False), (8, 128, 32, False),
+    (8, 64, 32, False), (8, 64, 16, False), (16, 128, 40, False), (16, 256, 40, False), (4, 512, 16, False), (8, 700, 16, False),
+    (8, 128, 16, True), (8, 300, 16, True), (8, 512, 8, True), (16, 160, 8, True), (8, 160, 24, True), (64, 190, 2, False)])
 def test_narrower_tiles_where_wide_ones_leave_compute_units_idle(groups, rows, blocks, half):
     assert HipOps.stream_half(rows * groups, groups, blocks) == half
+
+
+@pytest.mark.parametrize("groups", [8, 10, 12, 16, 20, 24])
+def test_narrower_tiles_are_one_round_however_the_rows_are_shared_out(groups):
+    """The tiles of a group as the kernel cuts them, its row blocks dealt to the eight chiplets in turn: none gets more than
+    its 32 compute units, with even groups, uneven ones, from 0.3 to 1.7 of the mean, and 40 % of the rows in one."""
+    g = torch.Generator().manual_seed(groups)
+    taken = 0
+    for blocks in range(1, 49):
+        for mean in range(90, 900, 20):
+            if not HipOps.stream_half(mean * groups, groups, blocks):
+                continue
+            taken += 1
+            weight = torch.exp(0.25 * torch.randn(groups, generator=g))
+            for part in (torch.ones(groups), weight, torch.linspace(0.3, 1.7, groups), torch.tensor([0.4 * groups] + [0.6 * groups / (groups - 1)] * (groups - 1))):
+                rows = (part / part.sum() * mean * groups).int()
+                assert -(-blocks // 8) * int(((rows + 287) // 288).sum()) <= 32, (blocks, mean, rows.tolist())
+    assert taken
 
 
 @pytest.mark.parametrize("lens, heads, dk, dv, pays", [
