@@ -239,15 +239,23 @@ __global__ __launch_bounds__(kWaves * 64) void gemm_few_kernel(FewArgs p) {
 
 // The tiles of a block.  What a compute unit reads of W and X together sets the time: rounds of blocks on the 256 compute
 // units times the tiles that a block reads (2,048 x 2,048, 64 rows: 1 of W with 2 of X, 256 blocks, 6.0 us; 2 with 2 7.1,
-// 1 with 4 7.7, 1 with 1 in two rounds 6.9; 8,192 x 2,048: 2 with 4 11.1, 4 with 2 11.2, 2 with 2 13.9, 1 with 2 17.2).  In
-// groups the rows of W are many rounds anyway: two of W, so that two blocks fit a compute unit and one's end hides behind
-// the other (8 groups of 4,096 x 2,048 with 128 rows: 2 with 2 24.5 us, 4 with 2 27.3, 2 with 1 30.5), and tiles of X that
-// hold a group's rows, taken to scatter about their mean by its root (a second tile reads the weights again).
+// 1 with 4 7.7, 1 with 1 in two rounds 6.9; 8,192 x 2,048: 2 with 4 11.1, 4 with 2 11.2, 2 with 2 13.9, 1 with 2 17.2).
+// Where there are many rounds anyway (an output head) and one tile of X, two of W, so that two blocks fit a compute unit and
+// one's end hides behind the other: a tiled head of 50,000 x 3,072, 1 row 57 us with four, 52 with two (gemm_skinny 49), 8 rows
+// 57 and 52 (55); 32,000 x 2,048, 1 row 25.2 and 23.2 (23.2).  Row-major matrices of up to two rounds are as fast with four.
+// In groups likewise: two of W (8 groups of 4,096 x 2,048 with 128 rows: 2 with 2 24.5 us, 4 with 2 27.3, 2 with 1 30.5), and
+// tiles of X that hold a group's rows, taken to scatter about their mean by its root (a second tile reads the weights again);
+// four of W only beside four of X, where a block has the compute unit to itself either way (4 groups of 16,384 x 5,120, gate and
+// up, with 128 rows 124 us, with two of W 153).  Up to a few rows a group one of W, three blocks a compute unit (us, one
+// | two | gemm_skinny: a token's expert and the shared one of 5,120 x 8,192 32.6 | 36.1 | 33.6; 2 tokens, top 2, and the shared
+// expert of 3,072 x 4,096 21.5 | 22.4 | 21.3, of 2,048 x 4,096 16.2 | 17.0 | 15.8); not where rows of W are short, whose blocks
+// are over too soon (64 groups of 4,096 x 1,408, 16 choices 33.7 | 33.0), and not with more rows (16 groups of 7,168 x 2,048, 128
+// choices 84.8 | 77.8).
 struct Tiles {
   int mt, rt;
 };
 
-Tiles few_tiles(int M, int width, bool swiglu, int G, bool grouped) {
+Tiles few_tiles(int M, int width, int K, bool swiglu, int G, bool grouped, bool tiled) {
   const int tiles = (width + 15) / 16 * (swiglu ? 2 : 1);  // of W's rows
   const int least = swiglu ? 2 : 1;
   if (grouped) {
@@ -255,6 +263,7 @@ Tiles few_tiles(int M, int width, bool swiglu, int G, bool grouped) {
     const float mean = (float)M / (float)used, most = mean + sqrtf(mean);
     const int mt = most <= 16.f ? 1 : most <= 32.f ? 2 : 4;
     const long long pairs = (long long)((tiles + 1) / 2) * used;
+    if (mt == 1 && !swiglu && K >= 2048 && mean < 6.f) return {1, 1};
     return {mt, mt == 4 && pairs >= 512 ? 4 : pairs >= 256 ? 2 : least};
   }
   Tiles best = {0, 0};
@@ -262,6 +271,7 @@ Tiles few_tiles(int M, int width, bool swiglu, int G, bool grouped) {
   for (int mt = 1; mt <= 4; mt *= 2) {
     if (mt > 1 && M <= 8 * mt) break;
     for (int rt = least; rt <= 4; rt *= 2) {
+      if (mt == 1 && rt == 4 && !swiglu && (tiled || tiles > 4 * 512)) break;
       const long long blocks = (long long)((tiles + rt - 1) / rt) * ((M + 16 * mt - 1) / (16 * mt));
       const long long cost = (blocks + 255) / 256 * (mt + rt);
       if (best.mt == 0 || cost < least_cost || (cost == least_cost && mt > best.mt)) {
@@ -306,6 +316,12 @@ int pick_few(const FewArgs& p, Tiles t, int max_rows, int zdim, hipStream_t s) {
 
 }  // namespace
 
+// The tiles that jle_gemm_few takes by itself: row tiles of X * 10 + of W.
+JLE_API int jle_gemm_few_tiles(int M, int Nout, int K, int G, int swiglu, int grouped, int tiled) {
+  const Tiles t = few_tiles(M, swiglu ? Nout / 2 : Nout, K, swiglu != 0, G, grouped != 0, tiled != 0);
+  return t.mt * 10 + t.rt;
+}
+
 // X [*, K] bf16, W [G, Nout, K] bf16 (row-major, or in the streaming layout: tiled), Y [M, Nout] (or [M, Nout / 2] with
 // swiglu) bf16 or float32.  swiglu 0: plain, with act 1 max(., 0)^2; 1: silu(gate) * up; 2: gelu_tanh(gate) * up.
 // max_rows: the most rows a group can have (M if unknown).  W_last, tiled_last: the last of the G groups' matrix, if it lies
@@ -323,7 +339,7 @@ JLE_API int jle_gemm_few(const void* X, const void* W, void* Y, const int* offse
   if (max_rows <= 0 || max_rows > M) max_rows = M;
   const FewArgs p = {(const bf16_t*)X, (const bf16_t*)W, Y, offsets, a_rows, scale, (const bf16_t*)W_last, M, Nout, K, G,
                      tiled, tiled_last, slots, swiglu ? swiglu - 1 : act};
-  const Tiles t = tiles ? Tiles{tiles / 10, tiles % 10} : few_tiles(M, swiglu ? Nout / 2 : Nout, swiglu != 0, G, offsets != nullptr);
+  const Tiles t = tiles ? Tiles{tiles / 10, tiles % 10} : few_tiles(M, swiglu ? Nout / 2 : Nout, K, swiglu != 0, G, offsets != nullptr, tiled);
   const int zdim = slots > 0 ? slots : G;
   if (swiglu) return out_f32 ? pick_few<true, float>(p, t, max_rows, zdim, s) : pick_few<true, bf16_t>(p, t, max_rows, zdim, s);
   return out_f32 ? pick_few<false, float>(p, t, max_rows, zdim, s) : pick_few<false, bf16_t>(p, t, max_rows, zdim, s);

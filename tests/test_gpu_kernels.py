@@ -1521,6 +1521,16 @@ def test_product_of_a_few_rows_in_groups(ops, sizes, tiled):
         assert ((y.double() - ref_act * up).abs() <= tol + 1e-30).all()
 
 
+@pytest.mark.parametrize("m,nout,k,groups,swiglu,grouped,tiled,tiles", [
+    (2, 5120, 8192, 17, 0, 1, 1, 11), (6, 2048, 4096, 9, 0, 1, 1, 11), (30, 5120, 8192, 17, 0, 1, 1, 11),  # a few rows a group
+    (16, 4096, 1408, 64, 0, 1, 1, 12), (128, 7168, 2048, 16, 0, 1, 1, 12), (128, 4096, 2048, 8, 0, 1, 1, 22),
+    (2, 16384, 5120, 17, 1, 1, 1, 12), (1, 16384, 5120, 1, 1, 0, 0, 14),
+    (1, 50000, 3072, 1, 0, 0, 1, 12), (8, 16000, 2048, 1, 0, 0, 1, 12), (1, 202048, 5120, 1, 0, 0, 0, 12),  # many rounds
+    (1, 32000, 2048, 1, 0, 0, 0, 14), (1, 2048, 2048, 1, 0, 0, 0, 11), (64, 202048, 5120, 1, 0, 0, 1, 44)])
+def test_tiles_of_a_product_of_a_few_rows(ops, m, nout, k, groups, swiglu, grouped, tiled, tiles):
+    assert ops._query("jle_gemm_few_tiles", m, nout, k, groups, swiglu, grouped, tiled) == tiles
+
+
 def test_product_of_a_few_rows_refuses_what_it_cannot_read(ops):
     from jax_llm_examples_amd.ops.hip import KernelError
 
