@@ -1760,11 +1760,25 @@ class HipOps:
                    int(out_f32), m, nout, k, g, m, int(tiled), _p(b_last), int(tiled_last), slots, tiles)
         return out
 
-    def _few_experts(self, a, b, *, b_last=None, **kw):
-        """The product of a step's few rows a group: the kernel for a few rows where it takes the sizes, else the
-        weight-streaming one."""
-        product = self.gemm_few if self._few_fits(a, b, *(() if b_last is None else (b_last,))) else self.gemm_skinny
-        return product(a, b, b_last=b_last, **kw)
+    @staticmethod
+    def few_pays(k: int, rows: int, groups: int, swiglu) -> bool:
+        """Whether the products of ``rows`` rows in groups go through the kernel for a few rows and not the weight-streaming
+        one.  With rows of W of up to 1,024 a wavefront of it has four lines of them or fewer: filling its ring and adding up
+        four wavefronts' sums is what takes the time, a tenth to a fifth more than the other kernel (this | the other, us:
+        128 groups of 2,048 x 768, 128 choices 56 | 47; 16 of 2,048 x 1,024, 16 choices 11.0 | 9.7; gate and up of 32 of
+        2,048 x 1,024 24.2 | 20.6).  It keeps the calls whose matrices the other one would cut (two groups at most: of
+        2,048 x 1,024 4.9 | 7.7), and groups of a dozen rows, of which the other one reads the weights twice where they are
+        over sixteen (8 of 2,048 x 1,024, 128 choices 9.2 | 11.7)."""
+        return k > 1024 or rows >= 12 * groups or (rows <= HipOps.CUT_SLOTS and not swiglu)
+
+    def _few_experts(self, a, b, *, b_last=None, swiglu=0, **kw):
+        """The product of a step's few rows a group: the kernel for a few rows where it takes the sizes and pays
+        (:meth:`few_pays`), else the weight-streaming one."""
+        picked = kw.get("a_rows")
+        rows = kw.get("rows") or (a.shape[0] if picked is None else picked.numel())
+        few = (self._few_fits(a, b, *(() if b_last is None else (b_last,)))
+               and self.few_pays(b.shape[2], rows, b.shape[0] + (b_last is not None), swiglu))
+        return (self.gemm_few if few else self.gemm_skinny)(a, b, b_last=b_last, swiglu=swiglu, **kw)
 
     def gemm_grouped(self, a, b, *, offsets=None, a_rows=None, scale=None, swiglu=False, out_f32=False, rows=None,
                      tiled=False):

@@ -111,6 +111,27 @@ def test_narrower_tiles_are_one_round_however_the_rows_are_shared_out(groups):
     assert taken
 
 
+@pytest.mark.parametrize("k, rows, groups, swiglu, pays", [
+    (2048, 16, 8, True, True), (1088, 128, 64, False, True), (1024, 16, 32, True, False), (768, 128, 128, False, False),
+    (1024, 2, 16, False, True), (1024, 2, 16, True, False), (1024, 3, 16, False, False), (1024, 96, 8, True, True), (1024, 95, 8, True, False),
+    (64, 1, 4, False, True)])
+def test_short_rows_of_weights_stay_with_the_weight_streaming_product(k, rows, groups, swiglu, pays):
+    assert HipOps.few_pays(k, rows, groups, swiglu) == pays
+
+
+@pytest.mark.parametrize("k, rows, last, product", [(2048, 4, False, "few"), (1024, 4, False, "skinny"), (1024, 2, False, "few"),
+                                                     (1024, 48, False, "few"), (1024, 48, True, "skinny"), (72, 4, False, "skinny")])
+def test_experts_products_go_where_they_pay(k, rows, last, product):
+    """Four groups, and with the shared expert's one more; rows that are picked count, not those they are picked from."""
+    at = lambda *shape: types.SimpleNamespace(dtype=torch.bfloat16, shape=shape, data_ptr=lambda: 4096, numel=lambda: shape[0] * shape[1])
+    ops = types.SimpleNamespace(gemm_few=lambda *a, **kw: "few", gemm_skinny=lambda *a, **kw: "skinny", few_pays=HipOps.few_pays)
+    ops._few_fits = lambda *a: HipOps._few_fits(ops, *a)
+    b, more = at(4, 256, k), dict(b_last=at(256, k)) if last else {}
+    assert HipOps._few_experts(ops, at(rows, k), b, **more) == product
+    assert HipOps._few_experts(ops, at(200, k), b, a_rows=types.SimpleNamespace(numel=lambda: rows), **more) == product
+    assert HipOps._few_experts(ops, at(200, k), b, a_rows=types.SimpleNamespace(numel=lambda: 999), rows=rows, **more) == product
+
+
 @pytest.mark.parametrize("lens, heads, dk, dv, pays", [
     ([64], 16, 128, 128, False), ([256], 16, 128, 128, True), ([2048], 4, 64, 64, True), ([64] * 32, 16, 128, 128, True),
     ([80] * 25, 16, 128, 128, True), ([32] * 64, 16, 128, 128, False), ([36] * 64, 64, 128, 128, False),
