@@ -1884,6 +1884,28 @@ class HipOps:
                    int(out_f32), m, nout, k, g, m, int(wide))
         return out
 
+    @staticmethod
+    def head_few(rows: int, n: int, k: int, tiled: bool, streams: bool) -> bool:
+        """Whether an output head ``[n, k]`` of ``rows`` rows goes through the kernel for a few rows.  In the streaming layout
+        up to 4 are as fast or faster in the skinny kernel, which needs no shared memory for so few, and from 17 on there
+        is the weight-streaming kernel (``streams``), whose blocks take 256 rows of W: it is the faster one unless it
+        leaves half of the compute units without a block (n up to 32,768; with more than 32 rows 28,672), or the matrix is so
+        large that up to 24 rows are the time of its bytes.  A row-major head has the skinny kernel beside it, which reads
+        its rows again for every 16.  This | the other, us, weights not in the caches; in the streaming layout:
+          28,672 x 4,096   4 rows 40.9 | 38.5    8 41.4 | 42.5    16 42.3 | 53.3    32 47.6 | 58.2    64 56.7 | 57.9
+          32,000 x 2,048   4 rows 23.6 | 23.5    8 23.7 | 25.6    16 24.6 | 32.6    32 28.9 | 31.1    64 32.7 | 31.8
+          50,000 x 3,072   4 rows 51.4 | 50.1    8 51.6 | 55.4    16 54.3 | 72.4    24 65.8 | 54.2    64 82.1 | 54.8
+          65,536 x 2,048   4 rows 45.1 | 44.8    8 46.3 | 49.3    16 47.9 | 64.3    24 55.0 | 52.4    64 65.8 | 54.4
+          202,048 x 5,120  1 row 308 | 309       8 308 | 313      16 331 | 369      24 365 | 387      64 456 | 400
+        row-major:
+          32,000 x 2,048   1 row 22.8 | 23.6     16 23.2 | 31.7   64 32.8 | 83.1
+          202,048 x 5,120  1 row 307 | 311       16 339 | 375     64 479 | 776"""
+        if tiled and rows <= 4:
+            return False
+        if not streams:
+            return rows <= HipOps.FEW_ROWS
+        return rows <= (HipOps.FEW_ROWS if n <= 28672 else 32 if n <= 32768 else 24 if n * k >= 1 << 28 else 16)
+
     def lm_head(self, h, w, tiled: bool = False):
         """float32 logits; ``tiled``: ``w`` is in the streaming layout (``ops/layout.py``)."""
         if h.dtype == torch.float32:
@@ -1891,14 +1913,11 @@ class HipOps:
             return torch.matmul(h, w.t()) if out is None else out
         if h.shape[1] % 8 == 0:
             streams = tiled and self.stream_supported(w.shape[0], w.shape[1], False)
-            # (kernel for a few rows | the one it takes them from, us: 32,000 x 2,048, 1 row 23.1 | 23.5, 8 23.6 | 26.1,
-            # 16 24.2 | 34.8, 32 27.8 | 33.8, 64 32.5 | 34.1; 202,048 x 5,120, 1 row 305 | 310, 8 317 | 323, 16 336 | 383,
-            # 32 387 | 397, 64 463 | 400)
-            if (h.shape[0] <= (self.FEW_ROWS if w.numel() < 1 << 28 else 32) and h.is_contiguous() and w.is_contiguous()
+            if (self.head_few(h.shape[0], *w.shape, tiled, streams) and h.is_contiguous() and w.is_contiguous()
                     and self._few_fits(h, w) and (not tiled or w.shape[0] % 16 == 0)):
                 return self.gemm_few(h, w, out_f32=True, tiled=tiled)
-            # sizes that it does not take, and more rows: the skinny kernel up to 16; beyond, the kernel that shares the rows
-            # between wavefronts through shared memory
+            # the others: the skinny kernel up to 16 rows; beyond, the kernel that shares the rows between wavefronts through
+            # shared memory
             if h.shape[0] <= (16 if streams else self.SKINNY_MAX_ROWS):
                 return self.gemm_skinny(h, w, out_f32=True, tiled=tiled)
             if streams:

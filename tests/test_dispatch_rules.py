@@ -111,6 +111,16 @@ def test_narrower_tiles_are_one_round_however_the_rows_are_shared_out(groups):
     assert taken
 
 
+@pytest.mark.parametrize("n, k, least, most", [(16000, 2048, 5, 64), (28672, 4096, 5, 64), (28688, 4096, 5, 32), (32768, 2048, 5, 32),
+                                                 (32784, 2048, 5, 16), (50000, 3072, 5, 16), (65536, 4096, 5, 24), (202048, 5120, 5, 24)])
+def test_output_heads_by_size(n, k, least, most):
+    """In the streaming layout, where that layout has no kernel of its own for many rows, and row-major."""
+    few = lambda tiled, streams: [r for r in range(1, 130) if HipOps.head_few(r, n, k, tiled, streams)]
+    assert few(True, True) == list(range(least, most + 1))
+    assert few(True, False) == list(range(least, 65))
+    assert few(False, False) == list(range(1, 65))
+
+
 @pytest.mark.parametrize("k, rows, groups, swiglu, pays", [
     (2048, 16, 8, True, True), (1088, 128, 64, False, True), (1024, 16, 32, True, False), (768, 128, 128, False, False),
     (1024, 2, 16, False, True), (1024, 2, 16, True, False), (1024, 3, 16, False, False), (1024, 96, 8, True, True), (1024, 95, 8, True, False),
