@@ -64,6 +64,39 @@ def test_add_rmsnorm(ops, ref, dt, d):
             assert h32_1.dtype == torch.float32
 
 
+_PIECE_EDGES = [1032, 2048, 2056, 4096, 4104, 6144, 6152, 8192]  # first and last width of two, four, six and eight pieces
+
+
+@pytest.mark.parametrize("many", [False, True])
+@pytest.mark.parametrize("d", _PIECE_EDGES)
+def test_add_rmsnorm_at_the_edges_of_its_pieces(ops, d, many):
+    """Few rows, and as many as are stored past the caches, against 64 bits."""
+    n = -(-(4 << 20) // d) if many else 7
+    x, delta, w = _rand(n, d, seed=1), _rand(n, d, dt=torch.bfloat16, seed=2), _rand(d, seed=3)
+    want = x.double() + delta.double()
+    h, h32 = ops.add_rmsnorm(x, delta, w, 1e-3, torch.bfloat16, True)
+    normed = want / torch.sqrt((want ** 2).mean(-1, keepdim=True) + 1e-3) * w.double()
+    assert ((x.double() - want).abs() <= 2.0 ** -24 * want.abs()).all()
+    # (a thread's up to 32 squares, 8 levels of the sum, root, quotient and products: not 50 roundings of 2^-24)
+    assert ((h32.double() - normed).abs() <= 50 * 2.0 ** -24 * normed.abs() + 1e-30).all()
+    assert torch.equal(h, h32.bfloat16())
+
+
+@pytest.mark.parametrize("d", _PIECE_EDGES)
+def test_norm_and_router_in_one_launch_at_the_edges_of_its_pieces(ops, d):
+    x, delta, w = _rand(5, d, seed=1), _rand(5, d, dt=torch.bfloat16, seed=2), _rand(d, seed=3) + 1.0
+    router = _rand(8, d, scale=0.05, seed=4)
+    pending = ops.defer_norm(x.clone(), delta, w, 1e-5, torch.bfloat16)
+    ids, gates, logits, _ = ops.moe_route(pending, router, 2, want_logits=True, group=True)
+    y = x.clone()
+    h, h32 = ops.add_rmsnorm(y, delta, w, 1e-5, torch.bfloat16, want32=True)
+    assert torch.equal(pending.residual(), y) and torch.equal(pending.rows(), h)
+    # (d products of float32 rows, a k of any order, are off by no more than (d + 2) roundings of their sizes' sum)
+    want = h32.double() @ router.double().t()
+    assert ((logits.double() - want).abs() <= (d + 2) * 2.0 ** -24 * (h32.double().abs() @ router.double().abs().t())).all()
+    assert torch.equal(ids.sort(1).values.long(), logits.topk(2, 1).indices.sort(1).values)
+
+
 def test_rmsnorm_eps_is_inside_the_root(ops):
     x = torch.full((1, 64), 1e-3, device=DEV)
     h, _ = ops.add_rmsnorm(x, None, None, 1e-2, torch.float32)
@@ -1521,6 +1554,52 @@ def test_product_of_a_few_rows_in_groups(ops, sizes, tiled):
         assert ((y.double() - ref_act * up).abs() <= tol + 1e-30).all()
 
 
+@pytest.mark.parametrize("tiles", [12, 14, 22, 24, 42, 44])
+@pytest.mark.parametrize("sizes", [None, [0, 17, 64, 1, 33]])
+@pytest.mark.parametrize("f,tiled", [(48, False), (48, True), (80, True), (88, False)])
+def test_gate_and_up_of_a_few_rows_with_every_tile(ops, f, tiled, sizes, tiles):
+    """The last block part of its tiles of gate rows and of up rows, whole tiles and half of one; one matrix, or groups of
+    which one fills the largest tile of rows."""
+    from jax_llm_examples_amd.ops.layout import tile_
+
+    g = torch.Generator().manual_seed(f)
+    G, m, k = len(sizes or [1]), sum(sizes or [50]), 192
+    w, x = (torch.randn(*s, generator=g).to(DEV, torch.bfloat16) for s in ((G, 2 * f, k), (m, k)))
+    group = torch.repeat_interleave(torch.arange(G), torch.tensor(sizes or [m])).to(DEV)
+    want = torch.stack([x[t].double() @ w[group[t]].double().t() for t in range(m)])
+    bound = torch.stack([(k + 3) * 2.0 ** -24 * (x[t].double().abs() @ w[group[t]].double().abs().t()) for t in range(m)])
+    wt = w.clone()
+    if tiled:
+        tile_(wt)
+    kw = dict(tiled=tiled, tiles=tiles, offsets=None if sizes is None else torch.tensor([0] + sizes).cumsum(0).int().to(DEV))
+    for act in (1, 2):
+        y = ops.gemm_few(x, wt if sizes else wt[0], swiglu=act, out_f32=True, **kw)
+        gate, up, of_gate, of_up = want[:, :f], want[:, f:], bound[:, :f], bound[:, f:]
+        ref_act = torch.nn.functional.silu(gate) if act == 1 else torch.nn.functional.gelu(gate, approximate="tanh")
+        # (the sums' own bounds, through slopes of up to 1.13; expf and tanhf within a few units of 2^-24 of 1 + |x|)
+        tol = 1.13 * of_gate * (up.abs() + of_up) + ref_act.abs() * of_up + 32 * 2.0 ** -24 * (1 + gate.abs()) * up.abs()
+        assert ((y.double() - ref_act * up).abs() <= tol + 1e-30).all()
+
+
+@pytest.mark.parametrize("tiles", [11, 12, 14, 21, 22, 24, 41, 42, 44])
+@pytest.mark.parametrize("nout,tiled", [(80, True), (70, False)])
+def test_grouped_product_of_a_few_rows_with_every_tile(ops, nout, tiled, tiles):
+    from jax_llm_examples_amd.ops.layout import tile_
+
+    g = torch.Generator().manual_seed(nout)
+    sizes, k = [0, 17, 64, 1, 33, 65], 320
+    m = sum(sizes)
+    w, x = (torch.randn(*s, generator=g).to(DEV, torch.bfloat16) for s in ((len(sizes), nout, k), (m, k)))
+    off = torch.tensor([0] + sizes).cumsum(0).int().to(DEV)
+    wt = w.clone()
+    if tiled:
+        tile_(wt)
+    got = ops.gemm_few(x, wt, offsets=off, tiled=tiled, tiles=tiles, out_f32=True)
+    for e, (lo, hi) in enumerate(zip(off[:-1].tolist(), off[1:].tolist())):
+        want = x[lo:hi].double() @ w[e].double().t()
+        assert ((got[lo:hi].double() - want).abs() <= _few_bound(x[lo:hi], w[e])).all()
+
+
 @pytest.mark.parametrize("m,nout,k,groups,swiglu,grouped,tiled,tiles", [
     (2, 5120, 8192, 17, 0, 1, 1, 11), (6, 2048, 4096, 9, 0, 1, 1, 11), (30, 5120, 8192, 17, 0, 1, 1, 11),  # a few rows a group
     (16, 4096, 1408, 64, 0, 1, 1, 12), (128, 7168, 2048, 16, 0, 1, 1, 12), (128, 4096, 2048, 8, 0, 1, 1, 22),
@@ -1548,7 +1627,7 @@ def test_product_of_a_few_rows_refuses_what_it_cannot_read(ops):
     ([287, 288, 289, 576, 577, 256, 257, 700, 1], 144, 512),  # one, two and three tiles of rows, a second block of W of one tile
     ([3, 0, 300] * 50, 64, 256),                              # more groups than a look takes
     ([192] * 8, 1168, 768)])                                  # more than eight blocks of W
-def test_narrower_tiles_of_the_weight_streaming_product(ops, counts, nout, k):
+def test_narrower_tiles_of_the_weight_streaming_product(ops, monkeypatch, counts, nout, k):
     """The bits of the kernel that takes a group's rows in passes, rows gathered and scaled."""
     from jax_llm_examples_amd.ops.layout import tile_
     m, e = sum(counts), len(counts)
@@ -1559,9 +1638,9 @@ def test_narrower_tiles_of_the_weight_streaming_product(ops, counts, nout, k):
     scale = _rand(m, seed=4)
     got = []
     for half in (False, True):
-        ops.stream_half, ops.stream_wide = (lambda *a, half=half: half), (lambda *a: False)
+        monkeypatch.setattr(ops, "stream_half", lambda *a, half=half: half, raising=False)
+        monkeypatch.setattr(ops, "stream_wide", lambda *a: False, raising=False)
         got.append(ops.gemm_stream(x, w, offsets=off, a_rows=rows, scale=scale, rows=m))
-    del ops.stream_half, ops.stream_wide
     assert torch.equal(*got)
 
 
@@ -1589,6 +1668,34 @@ def test_sum_with_factors_by_pieces_of_four(ops, d, k):
     normed = want / torch.sqrt((want ** 2).mean(-1, keepdim=True) + 1e-5) * w.double()
     # (a few roundings of 2^-24 of what is added up; the row's statistics another few)
     size = x.double().abs() + want.abs() + vec.double() * (0.7 * plain.abs() + 1.3 * b.double().abs()) + 4
+    assert ((x.double() - want).abs() <= 8 * 2.0 ** -24 * size).all()
+    assert ((h32.double() - normed).abs() <= 32 * 2.0 ** -24 * (size + normed.abs())).all()
+    assert torch.equal(h, h32.bfloat16())
+
+
+@pytest.mark.parametrize("d", [1024, 2048, 4096, 8192])
+@pytest.mark.parametrize("k", [0, 2])
+def test_sum_with_factors_of_rows_off_their_16_bytes(ops, d, k):
+    """Widths of each number of pieces, a term that starts 8 bytes on: element by element, to the same bounds."""
+    from jax_llm_examples_amd.ops.hip import ExpertSum
+    from jax_llm_examples_amd.parts.residual import ScaledSum
+
+    g = torch.Generator().manual_seed(d + k)
+    n = 5
+    off = lambda *s: torch.randn(math.prod(s) + 4, generator=g).to(DEV, torch.bfloat16)[4:].view(*s)
+    x, b = torch.randn(n, d, generator=g).to(DEV), off(n, d)
+    vec, w = (torch.rand(d, generator=g).to(DEV) + 0.5 for _ in range(2))
+    if k:
+        inv, rows = torch.randperm(n * k, generator=g).int().to(DEV), off(n * k, d)
+        a, plain = ExpertSum(rows, inv, k, None, n, d), rows.double()[inv.long()].view(n, k, d).sum(1)
+    else:
+        a = off(n, d)
+        plain = a.double()
+    want = x.double() + vec.double() * (0.7 * plain + 1.3 * b.double())
+    size = x.double().abs() + want.abs() + vec.double() * (0.7 * plain.abs() + 1.3 * b.double().abs()) + 4
+    h, h32 = ops.scaled_add_norm(x, ScaledSum([(a, 0.7), (b, 1.3)], vec), w, 1e-5, torch.bfloat16, want32=True)
+    normed = want / torch.sqrt((want ** 2).mean(-1, keepdim=True) + 1e-5) * w.double()
+    # (a few roundings of 2^-24 of what is added up; the row's statistics another few)
     assert ((x.double() - want).abs() <= 8 * 2.0 ** -24 * size).all()
     assert ((h32.double() - normed).abs() <= 32 * 2.0 ** -24 * (size + normed.abs())).all()
     assert torch.equal(h, h32.bfloat16())
