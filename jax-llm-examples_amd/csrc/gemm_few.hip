@@ -1,4 +1,4 @@
-// Matrix product of a few tens of rows (a decode step of 9 to 64 requests, the experts of such a step): bfloat16 in, float32
+// Matrix product of up to a few tens of rows (a decode step of up to 64 requests, the experts of such a step): bfloat16 in, float32
 // accumulate on MFMA.
 //
 //   Y[t, n] = scale[t] * sum_k X[arow(t), k] * W[g(t)][n, k]     (plain; optionally max(., 0)^2 of the rounded sum)
@@ -9,15 +9,19 @@
 // 6.5 us, with 64 13.1).  Here both come through shared memory, brought by the load unit itself in whole lines of 128 bytes
 // (a kilobyte an instruction, no register waits for it): a wavefront has a ring of its own, of stages of 64 k of its block's
 // rows of W and X, and takes every fourth stage of k.  No wavefront waits for another until the four add up their sums, so
-// the only thing that bounds it is how much is on its way: 48 to 96 KiB of rings a block.  Weights are asked for with loads
+// the only thing that bounds it is how much is on its way: 48 to 128 KiB of rings a block.  Weights are asked for with loads
 // that the caches need not keep.  Either layout of W (row-major, or tiles of 16 rows x 32 k of a kilobyte) is read by whole
 // lines; sums and their order are the same.
-// In microseconds, weights not in the caches (library | gemm_skinny | this):
-//   2,048 x 2,048    8 rows 11.1 | 6.5 | 4.6   16 rows 11.0 | 6.7 | 4.9    64 rows 11.7 | 13.1 | 6.0
-//   2,048 x 4,096    8 rows 14.8 | 7.7 | 6.8   16 rows 14.9 | 8.1 | 7.4    64 rows 14.0 | 22.8 | 9.2
-//   10,304 x 2,048   8 rows 16.4 | 12.0 | 10.6  32 rows 14.7 | 19.6 | 11.9  64 rows 15.9 | 32.7 | 14.7
-//   14,336 x 4,096   8 rows 30.6 | 24.5 | 21.8  32 rows 26.8 | 45.4 | 23.4  64 rows 28.8 | 77.6 | 27.1
-//   5,120 x 5,120    8 rows 16.1 | 13.3 | 14.4  32 rows 18.8 | 31.4 | 17.8  64 rows 22.2 | 53.5 | 22.8
+// In microseconds, weights not in the caches (gigabytes of other reads between two of the same W), this and what it is taken
+// instead of: gemm_skinny up to 8 rows, the library from 9 on:
+//   2,048 x 2,048    1 row 4.8 | 6.6     8 rows 4.9 | 6.8     16 rows 5.2 | 11.9    32 rows 5.2 | 12.0    64 rows 6.2 | 12.4
+//   2,048 x 4,096    1 row 7.0 | 7.8     8 rows 7.2 | 8.1     16 rows 7.7 | 15.5    32 rows 7.6 | 13.1    64 rows 9.5 | 15.0
+//   4,096 x 4,096    1 row 7.9 | 10.0    8 rows 8.0 | 10.6    16 rows 8.5 | 16.9    32 rows 10.5 | 14.9   64 rows 12.5 | 16.8
+//   4,096 x 14,336   1 row 22.8 | 31.3   8 rows 22.3 | 31.1   16 rows 24.7 | 38.1   32 rows 31.6 | 41.3   64 rows 38.9 | 51.5
+//   5,120 x 5,120    1 row 12.3 | 13.0   8 rows 13.3 | 13.5   16 rows 14.6 | 19.6   32 rows 17.8 | 21.7   64 rows 23.8 | 24.7
+//   7,168 x 5,120    1 row 14.3 | 15.3   8 rows 14.9 | 17.7   16 rows 16.0 | 23.6   32 rows 19.3 | 24.8   64 rows 25.1 | 27.2
+//   10,304 x 2,048   1 row 10.0 | 10.3   8 rows 10.2 | 11.7   16 rows 10.8 | 18.0   32 rows 12.3 | 18.0   64 rows 15.0 | 18.9
+//   14,336 x 4,096   1 row 21.9 | 22.7   8 rows 21.9 | 24.3   16 rows 22.1 | 38.9   32 rows 23.4 | 37.6   64 rows 27.7 | 37.1
 // 8 groups of 4,096 x 2,048 with 128 rows 29.0 -> 24.6, of 2,048 x 4,096 37.7 -> 26.1, of 4,096 x 7,168 89.7 -> 79.7; gate
 // and up of 4,096 x 2,048, 9 groups with 42 rows 47.5 -> 44.8, 8 with 128 51.4 -> 43.4 (gemm_skinny -> this).
 #include "common.h"

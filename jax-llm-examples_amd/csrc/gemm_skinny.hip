@@ -1,6 +1,7 @@
-// Weight-streaming matrix product for few rows (decode): bfloat16 in, float32 accumulate on MFMA.  gemm_few.hip is the faster
-// one and takes what it can; left are inner sizes that are no multiple of 64, rows off their 16 bytes, and up to 8 rows of
-// matrices four times as long as they are high, which are cut along K here.
+// Weight-streaming matrix product for few rows (decode): bfloat16 in, float32 accumulate on MFMA.  gemm_few.hip takes most
+// of what it can; left are inner sizes that are no multiple of 64, rows off their 16 bytes, up to 8 rows of matrices four times
+// as long as they are high, which are cut along K here, experts' products with rows of weights of up to 1,024, and up to 4 rows
+// of an output head in the streaming layout.
 //
 //   Y[t, n] = scale[t] * sum_k X[arow(t), k] * W[g(t)][n, k]          (plain)
 //   Y[t, f] = silu(s * gate) * (s * up),  gate/up = rows f and F + f of W[g(t)]   (SWIGLU, s = scale[t])

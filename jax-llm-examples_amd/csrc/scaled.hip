@@ -5,7 +5,8 @@
 // and the same launch forms the next norm's rows, h = x / sqrt(mean(x^2) + eps) * w, in the run dtype (and in float32
 // for a router).  It is what a layer leaves pending whose branches have a multiplier and a learned scale per
 // channel, and whose mixer may be two mixers side by side with a weight each.  One block per row, the row in
-// registers (wider rows are read again); every sum in an order that depends on the width alone.
+// registers (wider rows are read again); every sum in an order that depends on the width, and on whether all arrays start at 16
+// bytes, alone.
 #include "common.h"
 #include "rows.h"
 

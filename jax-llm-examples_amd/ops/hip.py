@@ -1129,9 +1129,10 @@ class HipOps:
 
     def _few(self, h, w) -> bool:
         """Whether ``h @ w.T`` goes through the kernel for a few rows: up to FEW_ROWS of them, wherever it takes the sizes.
-        The weight-streaming kernel, which cuts a long row of few weight rows into slices, keeps its up to 8 rows of those
-        (2,048 x 8,192, 8 rows: 10.7 against 12.3 us).  Of the library's it takes all: at worst 3 % behind (7,168 x 5,120, 64
-        rows: 23.9 against 23.3 us), else up to half of its time (figures: ``gemm_few.hip``)."""
+        The weight-streaming kernel, which cuts a long row of few weight rows into slices, keeps its up to 8 rows of those: it
+        is ahead from an inner size of 8,192 on (it | this one, 4 rows, us: 2,048 x 8,192 10.8 | 10.7, 1,024 x 8,192 8.8 | 10.0,
+        2,048 x 16,384 15.5 | 18.8, 512 x 16,384 9.7 | 16.8) and behind with shorter ones (1,024 x 4,096 7.7 | 6.6).  Of the
+        library's it takes all: 1.02 to 3.4 times as fast over fifty sizes and 9 to 64 rows (figures: ``gemm_few.hip``)."""
         if h.dim() != 2 or w.dim() != 2 or h.shape[0] > self.FEW_ROWS or not self._few_fits(h, w):
             return False
         if h.shape[0] <= self.SKINNY_LINEAR_ROWS and w.shape[1] >= 4 * w.shape[0]:
