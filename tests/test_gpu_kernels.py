@@ -1469,6 +1469,13 @@ def test_embedding_rows_times_a_number(ops, ref, n, d, dtype):
         assert torch.equal(ops.embed(tok, table, mul), ref.embed(tok, table, mul))
 
 
+@pytest.mark.parametrize("n,d", [(1, 8), (257, 8), (300, 264), (31, 2048), (513, 2056)])
+def test_embedding_rows_end_within_a_block(ops, ref, n, d):
+    table = torch.randn(600, d, generator=torch.Generator().manual_seed(d)).to(DEV, torch.bfloat16)
+    tok = torch.randint(0, 600, (n,), generator=torch.Generator().manual_seed(n)).int().to(DEV)
+    assert torch.equal(ops.embed(tok, table, 1.5), ref.embed(tok, table, 1.5))
+
+
 @pytest.mark.parametrize("k,shared,own", [(1, True, False), (2, False, False), (2, True, True), (6, True, False)])
 def test_chosen_rows_of_an_expert_sum_stay_in_pieces(ops, k, shared, own):
     from jax_llm_examples_amd.ops.hip import ExpertSum
