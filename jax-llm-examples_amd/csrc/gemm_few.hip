@@ -248,7 +248,8 @@ __global__ __launch_bounds__(kWaves * 64) void gemm_few_kernel(FewArgs p) {
 // one's end hides behind the other: a tiled head of 50,000 x 3,072, 1 row 57 us with four, 52 with two (gemm_skinny 49), 8 rows
 // 57 and 52 (55); 32,000 x 2,048, 1 row 25.2 and 23.2 (23.2).  Row-major matrices of up to two rounds are as fast with four.
 // In groups likewise: two of W (8 groups of 4,096 x 2,048 with 128 rows: 2 with 2 24.5 us, 4 with 2 27.3, 2 with 1 30.5), and
-// tiles of X that hold a group's rows, taken to scatter about their mean by its root (a second tile reads the weights again);
+// tiles of X that hold a group's rows, which scatter about their mean by its root or more (a second tile reads the weights
+// again: gate and up of 8 of 14,336 x 4,096 with a dozen rows a group 160 us with one, 145 with two, 152 in gemm_skinny);
 // four of W only beside four of X, where a block has the compute unit to itself either way (4 groups of 16,384 x 5,120, gate and
 // up, with 128 rows 124 us, with two of W 153).  Up to a few rows a group one of W, three blocks a compute unit (us, one
 // | two | gemm_skinny: a token's expert and the shared one of 5,120 x 8,192 32.6 | 36.1 | 33.6; 2 tokens, top 2, and the shared
@@ -264,8 +265,8 @@ Tiles few_tiles(int M, int width, int K, bool swiglu, int G, bool grouped, bool 
   const int least = swiglu ? 2 : 1;
   if (grouped) {
     const int used = G < M ? G : M;
-    const float mean = (float)M / (float)used, most = mean + sqrtf(mean);
-    const int mt = most <= 16.f ? 1 : most <= 32.f ? 2 : 4;
+    const float mean = (float)M / (float)used;
+    const int mt = mean < 12.f ? 1 : mean + sqrtf(mean) <= 32.f ? 2 : 4;
     const long long pairs = (long long)((tiles + 1) / 2) * used;
     if (mt == 1 && !swiglu && K >= 2048 && mean < 6.f) return {1, 1};
     return {mt, mt == 4 && pairs >= 512 ? 4 : pairs >= 256 ? 2 : least};

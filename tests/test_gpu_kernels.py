@@ -1610,6 +1610,7 @@ def test_grouped_product_of_a_few_rows_with_every_tile(ops, nout, tiled, tiles):
 @pytest.mark.parametrize("m,nout,k,groups,swiglu,grouped,tiled,tiles", [
     (2, 5120, 8192, 17, 0, 1, 1, 11), (6, 2048, 4096, 9, 0, 1, 1, 11), (30, 5120, 8192, 17, 0, 1, 1, 11),  # a few rows a group
     (16, 4096, 1408, 64, 0, 1, 1, 12), (128, 7168, 2048, 16, 0, 1, 1, 12), (128, 4096, 2048, 8, 0, 1, 1, 22),
+    (95, 14336, 4096, 8, 1, 1, 1, 12), (96, 14336, 4096, 8, 1, 1, 1, 22), (106, 14336, 4096, 4, 1, 1, 1, 22), (108, 14336, 4096, 4, 1, 1, 1, 44),
     (2, 16384, 5120, 17, 1, 1, 1, 12), (1, 16384, 5120, 1, 1, 0, 0, 14),
     (1, 50000, 3072, 1, 0, 0, 1, 12), (8, 16000, 2048, 1, 0, 0, 1, 12), (1, 202048, 5120, 1, 0, 0, 0, 12),  # many rounds
     (1, 32000, 2048, 1, 0, 0, 0, 14), (1, 2048, 2048, 1, 0, 0, 0, 11), (64, 202048, 5120, 1, 0, 0, 1, 44)])
