@@ -16,8 +16,15 @@
 // four stages.  Groups with more than 192 rows are done in passes (each reads the weights again).
 //
 // Work items are (group, pass, block of WAVES * 32 weight rows), the last fastest, so the blocks of a group
-// are dealt to all dies in turn and a group with many rows slows all of them alike.  Items without rows
-// leave at once.
+// are dealt to all dies in turn and a group with many rows slows all of them alike.  How many there are is known on the
+// device only (Items): every block counts the groups' passes itself, so that items are those with rows and nothing else.
+// (The grid once had an item for every pass that any group could have: those without rows lay between those with, and where
+// their number was even only some of the chiplets got work: 64 groups of 256 x 2,048 with 190 rows 328 us, counted 48; 32 of
+// 1,536 x 2,048, gate and up, with 48 rows 78 -> 41; 12 of 2,560 x 6,144 with 250 237 -> 108.)
+// A block has a compute unit to itself, and those left over behind the last full round would keep a few of them busy for a
+// round's time: they are cut along k into as many pieces as the round has places (Cut), whose float32 sums add_pieces_kernel
+// adds up in their order and finishes.  16 groups of 5,120 x 8,192 with 128 rows, 320 blocks: 297 -> 269 us, what reading the
+// weights alone takes in this arrangement 234.
 #include "common.h"
 
 using namespace jle;
@@ -44,6 +51,112 @@ __device__ __forceinline__ void store4<bf16_t>(bf16_t* p, float a, float b, floa
   *reinterpret_cast<uint2*>(p) = uint2{pack_bf16(a, b), pack_bf16(c, d)};
 }
 
+// The work items of a launch, found by every wavefront for itself: each group has its rows in tiles of at most `most`, times
+// nblk blocks of its weights.  64 groups a look, the items before each by a sum over the lanes.
+struct Items {
+  const int* offsets;  // null: one group of M rows
+  int M, G, nblk, most;
+
+  __device__ __forceinline__ int rows_of(int g) const {
+    return offsets == nullptr ? (g == 0 ? M : 0) : g < G ? offsets[g + 1] - offsets[g] : 0;
+  }
+  __device__ __forceinline__ int count() const {
+    const int lane = threadIdx.x & 63;
+    int n = 0;
+    for (int g0 = 0; g0 < G; g0 += 64) n += (rows_of(g0 + lane) + most - 1) / most;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) n += __shfl_xor(n, o, 64);
+    return __builtin_amdgcn_readfirstlane(n) * nblk;
+  }
+  // Item `left`'s group (-1: no such item), how many tiles the group has, and which of the group's items it is.
+  __device__ __forceinline__ int find(int& left, int& tiles) const {
+    const int lane = threadIdx.x & 63;
+    for (int g0 = 0; g0 < G; g0 += 64) {
+      const int mine = (rows_of(g0 + lane) + most - 1) / most;
+      int upto = mine * nblk;
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const int v = __shfl_up(upto, o, 64);
+        if (lane >= o) upto += v;
+      }
+      const unsigned long long mask = __ballot(left < upto);
+      if (mask != 0) {
+        const int at = __ffsll((long long)mask) - 1;
+        tiles = __builtin_amdgcn_readfirstlane(__shfl(mine, at, 64));
+        left = __builtin_amdgcn_readfirstlane(left - __shfl(upto, at, 64) + tiles * nblk);
+        return __builtin_amdgcn_readfirstlane(g0 + at);
+      }
+      left -= __shfl(upto, 63, 64);
+    }
+    return -1;
+  }
+  // Up to 64 groups whose numbers of tiles differ from the first one's by one at most.
+  __device__ __forceinline__ bool even() const {
+    const int mine = (rows_of(threadIdx.x & 63) + most - 1) / most, of = __builtin_amdgcn_readfirstlane(mine);
+    return G <= 64 && __ballot((int)(threadIdx.x & 63) < G && (mine > of + 1 || mine < of - 1)) == 0;
+  }
+  // find() of such groups with every group's first tile before all second ones: with a round or two of blocks in all the last
+  // ones are then those with the fewest rows (8 groups of 4,096 x 2,048 with 512 rows, three passes of 192, 192 and 128: 106
+  // us group after group, 94 so; where one group has most of the rows its last tiles would come last: 16 of 5,120 x 8,192
+  // with 128, 40 % in one, 287 | 352).
+  __device__ __forceinline__ int find_by_tile(int& left, int& tiles) const {
+    const int mine = (rows_of(threadIdx.x & 63) + most - 1) / most;
+    for (int t = 0;; ++t) {
+      unsigned long long mask = __ballot(mine > t);
+      const int n = __popcll(mask);
+      if (n == 0) return -1;
+      if (left < n * nblk) {
+        for (int j = left / nblk; j > 0; --j) mask &= mask - 1;  // drop the lower set bits
+        const int g = __ffsll((long long)mask) - 1;
+        tiles = __builtin_amdgcn_readfirstlane(__shfl(mine, g, 64));
+        left = __builtin_amdgcn_readfirstlane(left % nblk + t * nblk);
+        return __builtin_amdgcn_readfirstlane(g);
+      }
+      left -= n * nblk;
+    }
+  }
+};
+
+// How the items of the last, partly filled round are cut along k: into `pieces` each, one for every compute unit at most, none
+// shorter than kLeastStages.
+constexpr int kLeastStages = 16, kMostPieces = 8, kMostCutGroups = 1024;
+struct Cut {
+  int whole, tail, pieces;  // items taken whole, items behind them, pieces of each of those
+
+  __device__ __forceinline__ Cut(int items, int units, int nstage) {
+    tail = items % units;
+    pieces = tail > 0 ? min(min(units / tail, kMostPieces), nstage / kLeastStages) : 1;
+    if (pieces < 2) tail = 0;
+    whole = items - tail;
+  }
+  // the stages that a piece begins at: whole rounds of four
+  static __device__ __forceinline__ int stage(int piece, int pieces, int nstage) {
+    return (int)((long long)(nstage / WAHEAD) * piece / pieces) * WAHEAD;
+  }
+};
+
+// Rows of a tile: a group's rows as even as multiples of 32 allow.
+__device__ __forceinline__ int rows_a_tile(int rows, int tiles) { return ((rows + tiles - 1) / tiles + 31) / 32 * 32; }
+
+// A lane's sums of a row, four neighbouring rows of two tiles of W, scaled and stored.
+template <bool SWIGLU, typename OutT>
+__device__ __forceinline__ void finish_pair(OutT* __restrict__ Y, int t, const float* __restrict__ scale, f32x4 a0, f32x4 a1,
+                                            int Nout, int t0, int t1, int g) {
+  const float sc = scale != nullptr ? scale[t] : 1.f;
+  if (SWIGLU) {
+    float y[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float gate = a0[i] * sc, up = a1[i] * sc;
+      y[i] = gate / (1.0f + expf(-gate)) * up;
+    }
+    store4<OutT>(Y + (size_t)t * (Nout >> 1) + t0 * 16 + 4 * g, y[0], y[1], y[2], y[3]);
+  } else {
+    store4<OutT>(Y + (size_t)t * Nout + t0 * 16 + 4 * g, a0[0] * sc, a0[1] * sc, a0[2] * sc, a0[3] * sc);
+    if (t1 != t0) store4<OutT>(Y + (size_t)t * Nout + t1 * 16 + 4 * g, a1[0] * sc, a1[1] * sc, a1[2] * sc, a1[3] * sc);
+  }
+}
+
 // The work of one block once it knows its rows and tiles; NTL = B tiles (of 16 rows) that hold live rows, even
 // (the rows are brought in by whole rounds of the block's threads, 64 rows each: a round's rows past the live
 // tiles land in tiles that nobody reads).  The main loop has no branch but its own: every load is asked for unconditionally (rows past
@@ -54,14 +167,15 @@ __device__ __forceinline__ void stream_block(const bf16_t* __restrict__ X, const
                                              const bf16_t* __restrict__ w1, OutT* __restrict__ Y,
                                              const int* __restrict__ a_rows, const float* __restrict__ scale,
                                              bf16_t (&sX)[2][kRows * BK], int tok0, int live, int K, int Nout, int t0,
-                                             int t1, bool wave_ok) {
+                                             int t1, bool wave_ok, int first, int nstage, f32x4* __restrict__ piece) {
   constexpr int THREADS = WAVES * 64;
   constexpr int CHUNKS = NTL * 16 * (BK / 8);            // 16-byte pieces of X per stage
   constexpr int CPT = (CHUNKS + THREADS - 1) / THREADS;  // per thread
   const int lane = threadIdx.x & 63;
   const int r = lane & 15, g = lane >> 4;
-  const int nstage = K / BK;  // a multiple of 4
-  const int half = Nout >> 1;
+  X += (size_t)first * BK;  // (this block's stages: nstage of them, a multiple of 4)
+  w0 += (size_t)first * 1024;
+  w1 += (size_t)first * 1024;
 
   // who brings which pieces of X: piece c is 8 k of row c / 8, 8 consecutive threads a row's 128 bytes
   uint32_t xsrc[CPT];  // elements from X (the host checks that X has fewer than 2^32)
@@ -151,74 +265,97 @@ __device__ __forceinline__ void stream_block(const bf16_t* __restrict__ X, const
   STAGE(xb, wd, 1, s + 3, false, false);
 #undef STAGE
   if (!wave_ok) return;
+  if (piece != nullptr) {  // a piece of k: its sums as they are
+#pragma unroll
+    for (int nt = 0; nt < NTL; ++nt) {
+      piece[(nt * WAVES * 2 + (threadIdx.x >> 6) * 2) * 64 + lane] = acc0[nt];
+      piece[(nt * WAVES * 2 + (threadIdx.x >> 6) * 2 + 1) * 64 + lane] = acc1[nt];
+    }
+    return;
+  }
 
   // accumulators: element i of tile nt in lane (g, r) = weight row 4 g + i of the tile, row 16 nt + r of the pass
 #pragma unroll
   for (int nt = 0; nt < NTL; ++nt) {
     const int row = nt * 16 + r;
     if (row >= live) continue;
-    const int t = tok0 + row;
-    const float sc = scale != nullptr ? scale[t] : 1.f;
-    if (SWIGLU) {
-      float y[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float gate = acc0[nt][i] * sc, up = acc1[nt][i] * sc;
-        y[i] = gate / (1.0f + expf(-gate)) * up;
-      }
-      store4<OutT>(Y + (size_t)t * half + t0 * 16 + 4 * g, y[0], y[1], y[2], y[3]);
-    } else {
-      store4<OutT>(Y + (size_t)t * Nout + t0 * 16 + 4 * g, acc0[nt][0] * sc, acc0[nt][1] * sc, acc0[nt][2] * sc,
-                   acc0[nt][3] * sc);
-      if (t1 != t0)
-        store4<OutT>(Y + (size_t)t * Nout + t1 * 16 + 4 * g, acc1[nt][0] * sc, acc1[nt][1] * sc, acc1[nt][2] * sc,
-                     acc1[nt][3] * sc);
-    }
+    finish_pair<SWIGLU>(Y, tok0 + row, scale, acc0[nt], acc1[nt], Nout, t0, t1, g);
   }
 }
 
-template <bool SWIGLU, typename OutT, int WAVES>
-__global__ __launch_bounds__(WAVES * 64, 2) void gemm_stream_kernel(const bf16_t* __restrict__ X,
-                                                                 const bf16_t* __restrict__ W, OutT* __restrict__ Y,
-                                                                 const int* __restrict__ offsets,
-                                                                 const int* __restrict__ a_rows,
-                                                                 const float* __restrict__ scale, int M, int Nout,
-                                                                 int K, int nblk, int passes) {
-  __shared__ __attribute__((aligned(16))) bf16_t sX[2][kRows * BK];
-  const int item = blockIdx.x;
-  const int nb = item % nblk, pass = (item / nblk) % passes, e = item / (nblk * passes);
-  int row_lo = 0, row_hi = M;
-  if (offsets != nullptr) {
-    row_lo = offsets[e];
-    row_hi = offsets[e + 1];
-  }
-  const int tok0 = row_lo + pass * kRows;
-  if (tok0 >= row_hi) return;  // the whole block
-  const int live = min(kRows, row_hi - tok0);  // rows of this pass
+struct StreamArgs {
+  const bf16_t* X;
+  const bf16_t* W;
+  void* Y;
+  const int* a_rows;
+  const float* scale;
+  Items items;
+  f32x4* pieces;     // null: nothing is cut
+  size_t a_piece;    // f32x4 of a piece
+  int Nout, K, units;
+};
 
+// Item `left`'s group, how many passes the group has, and which of the group's items it is; `items` there are.
+__device__ __forceinline__ int locate(const StreamArgs& p, int items, int& left, int& passes) {
+  if (left >= items) return -1;
+  return items <= 2 * p.units && p.items.even() ? p.items.find_by_tile(left, passes) : p.items.find(left, passes);
+}
+
+// The rows of item `left` of a group with `tiles` passes, the first of its block's pairs of tiles of W
+struct Pass {
+  int tok0, live, nb;
+
+  __device__ __forceinline__ Pass(const Items& it, int e, int left, int tiles) {
+    nb = left % it.nblk;
+    const int lo = it.offsets == nullptr ? 0 : it.offsets[e], rows = it.rows_of(e), per = rows_a_tile(rows, tiles);
+    tok0 = lo + left / it.nblk * per;
+    live = min(per, rows - left / it.nblk * per);
+  }
+};
+
+// The two tiles of W of wavefront `wave` of block nb; false: behind the last one.
+template <bool SWIGLU, int WAVES>
+__device__ __forceinline__ bool tiles_of(int nb, int wave, int Nout, int& t0, int& t1) {
+  const int ntile = (SWIGLU ? Nout >> 1 : Nout) >> 4;
+  const int ft = SWIGLU ? nb * WAVES + wave : (nb * WAVES + wave) * 2;
+  t0 = ft < ntile ? ft : 0;
+  t1 = SWIGLU ? ntile + t0 : min(t0 + 1, ntile - 1);
+  return ft < ntile;
+}
+
+template <bool SWIGLU, typename OutT, int WAVES>
+__global__ __launch_bounds__(WAVES * 64, 2) void gemm_stream_kernel(StreamArgs p) {
+  __shared__ __attribute__((aligned(16))) bf16_t sX[2][kRows * BK];
+  const int K = p.K, Nout = p.Nout;
+  const int items = p.items.count(), all = K / BK;
+  int left = blockIdx.x, first = 0, stages = all;
+  f32x4* piece = nullptr;
+  if (p.pieces != nullptr) {
+    const Cut c(items, p.units, all);
+    const int slot = left - c.whole;
+    if (slot >= c.tail * c.pieces) return;
+    if (slot >= 0) {
+      left = c.whole + slot % c.tail;
+      first = Cut::stage(slot / c.tail, c.pieces, all);
+      stages = Cut::stage(slot / c.tail + 1, c.pieces, all) - first;
+      piece = p.pieces + (size_t)slot * p.a_piece;
+    }
+  }
+  int passes;
+  const int e = locate(p, items, left, passes);
+  if (e < 0) return;  // (the grid is laid out for the most items that so many rows can make)
+  const Pass at(p.items, e, left, passes);
+  const int tok0 = at.tok0, live = at.live, nb = at.nb;
   const int lane = threadIdx.x & 63, wave = wave_index();
   const int nkb = K >> 5;
-  const int half = Nout >> 1;
-  const bf16_t* We = W + (size_t)e * Nout * K;
-  // the wavefront's two weight tiles
-  const int ntile = (SWIGLU ? half : Nout) >> 4;
+  const bf16_t* We = p.W + (size_t)e * Nout * K;
   int t0, t1;
-  bool wave_ok;
-  if (SWIGLU) {
-    const int ft = nb * WAVES + wave;
-    wave_ok = ft < ntile;
-    t0 = wave_ok ? ft : 0;
-    t1 = (half >> 4) + t0;
-  } else {
-    const int ft = (nb * WAVES + wave) * 2;
-    wave_ok = ft < ntile;
-    t0 = wave_ok ? ft : 0;
-    t1 = min(t0 + 1, ntile - 1);
-  }
+  const bool wave_ok = tiles_of<SWIGLU, WAVES>(nb, wave, Nout, t0, t1);
   const bf16_t* w0 = We + (size_t)t0 * nkb * 512 + lane * 8;
   const bf16_t* w1 = We + (size_t)t1 * nkb * 512 + lane * 8;
 #define GO(NTL_) \
-  stream_block<SWIGLU, OutT, WAVES, NTL_>(X, w0, w1, Y, a_rows, scale, sX, tok0, live, K, Nout, t0, t1, wave_ok)
+  stream_block<SWIGLU, OutT, WAVES, NTL_>(p.X, w0, w1, (OutT*)p.Y, p.a_rows, p.scale, sX, tok0, live, K, Nout, t0, t1, \
+                                          wave_ok, first, stages, piece)
   if (live <= 32) GO(2);
   else if (live <= 64) GO(4);
   else if (live <= 96) GO(6);
@@ -226,6 +363,33 @@ __global__ __launch_bounds__(WAVES * 64, 2) void gemm_stream_kernel(const bf16_t
   else if (live <= 160) GO(10);
   else GO(12);
 #undef GO
+}
+
+// The cut items' pieces, added up in their order and finished: blockIdx.x is the item behind the whole ones, blockIdx.y
+// which of its tiles of rows.
+template <bool SWIGLU, typename OutT, int WAVES>
+__global__ __launch_bounds__(WAVES * 64) void add_pieces_kernel(StreamArgs p) {
+  const int items = p.items.count();
+  const Cut c(items, p.units, p.K / BK);
+  if ((int)blockIdx.x >= c.tail) return;
+  int left = c.whole + blockIdx.x, passes;
+  const int e = locate(p, items, left, passes);
+  if (e < 0) return;
+  const Pass at(p.items, e, left, passes);
+  const int lane = threadIdx.x & 63, r = lane & 15, wave = wave_index();
+  int t0, t1;
+  if (!tiles_of<SWIGLU, WAVES>(at.nb, wave, p.Nout, t0, t1)) return;
+  for (int nt = blockIdx.y; nt * 16 < at.live; nt += gridDim.y) {
+    const f32x4* from = p.pieces + (size_t)blockIdx.x * p.a_piece + (nt * WAVES * 2 + wave * 2) * 64 + lane;
+    f32x4 a0 = from[0], a1 = from[64];
+    for (int i = 1; i < c.pieces; ++i) {
+      from += (size_t)c.tail * p.a_piece;
+      a0 += from[0];
+      a1 += from[64];
+    }
+    if (nt * 16 + r < at.live)
+      finish_pair<SWIGLU>((OutT*)p.Y, at.tok0 + nt * 16 + r, p.scale, a0, a1, p.Nout, t0, t1, lane >> 4);
+  }
 }
 
 // ------------------------------------------------------------------ groups of many rows
@@ -390,37 +554,14 @@ __global__ __launch_bounds__(256, 1) void wide_kernel(const bf16_t* __restrict__
                                                       int Nout, int K, int G, int nblk8) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
   constexpr int kWideRows = wide_rows(HALF);
-  // this block's group: 64 groups a look, the items before each by a sum over the lanes
-  const int lane = threadIdx.x & 63;
-  int left = blockIdx.x, e = -1, tiles = 0;
-  for (int g0 = 0; g0 < G && e < 0; g0 += 64) {
-    const int gi = g0 + lane;
-    const int rows = gi < G ? offsets[gi + 1] - offsets[gi] : 0;
-    const int mine = (rows + kWideRows - 1) / kWideRows;
-    int upto = mine * nblk8;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const int v = __shfl_up(upto, o, 64);
-      if (lane >= o) upto += v;
-    }
-    const unsigned long long mask = __ballot(left < upto);
-    if (mask != 0) {
-      const int at = __ffsll((long long)mask) - 1;
-      e = g0 + at;
-      tiles = __shfl(mine, at, 64);
-      left -= __shfl(upto, at, 64) - tiles * nblk8;
-    } else {
-      left -= __shfl(upto, 63, 64);
-    }
-  }
+  const Items items = {offsets, 0, G, nblk8, kWideRows};
+  int left = blockIdx.x, tiles;
+  const int e = items.find(left, tiles);
   if (e < 0) return;  // (the grid is laid out for the most tiles that so many rows can make)
-  e = __builtin_amdgcn_readfirstlane(e);
-  left = __builtin_amdgcn_readfirstlane(left);
-  tiles = __builtin_amdgcn_readfirstlane(tiles);
   const int nb = left / (8 * tiles) * 8 + (left & 7), tile = (left >> 3) % tiles;
   if (nb * (SWIGLU || HALF ? 128 : 256) >= (SWIGLU ? Nout / 2 : Nout)) return;
   const int lo = offsets[e], rows = offsets[e + 1] - lo;
-  const int per = ((rows + tiles - 1) / tiles + 31) / 32 * 32;
+  const int per = rows_a_tile(rows, tiles);
   const int tok0 = lo + tile * per, live = min(per, rows - tile * per);
   if (live <= 0) return;
   const bf16_t* We = W + (size_t)e * Nout * K;
@@ -456,10 +597,13 @@ int launch_wide(hipStream_t s, const void* X, const void* W, void* Y, const int*
 }
 
 template <bool SW, typename OT, int WV>
-void launch_stream(int nblk, int passes, int G, hipStream_t s, const void* X, const void* W, void* Y,
-                   const int* offsets, const int* a_rows, const float* scale, int M, int Nout, int K) {
-  hipLaunchKernelGGL((gemm_stream_kernel<SW, OT, WV>), dim3(nblk * passes * G), dim3(WV * 64), 0, s,
-                     (const bf16_t*)X, (const bf16_t*)W, (OT*)Y, offsets, a_rows, scale, M, Nout, K, nblk, passes);
+int launch_stream(const StreamArgs& p, long long items, hipStream_t s) {
+  hipLaunchKernelGGL((gemm_stream_kernel<SW, OT, WV>), dim3((unsigned)items), dim3(WV * 64), 0, s, p);
+  JLE_LAUNCH_CHECK();
+  if (p.pieces == nullptr) return 0;
+  hipLaunchKernelGGL((add_pieces_kernel<SW, OT, WV>), dim3(p.units / 2, 4), dim3(WV * 64), 0, s, p);
+  JLE_LAUNCH_CHECK();
+  return 0;
 }
 
 }  // namespace
@@ -471,13 +615,17 @@ JLE_API int jle_gemm_stream_supported(int Nout, int K, int swiglu) {
   return Nout > 0 && Nout % 16 == 0;
 }
 
+// Bytes that a piece's sums take, of the most rows that an item of M rows can have.
+JLE_API int jle_gemm_stream_piece(int M) { return (M < kRows ? (M + 31) / 32 * 32 : kRows) * 256 * 4; }
+
 // X [*, K] bf16, W [G, Nout, K] bf16 in the streaming layout, Y [M, Nout] (or [M, Nout / 2] with swiglu) bf16 or
-// float32; X must have fewer than 2^32 elements (wide: 2^32 bytes).  wide: wide_kernel (groups, bfloat16 out), 2 (plain): HALF.  max_rows: the most rows any group can have (M if unknown).
+// float32; X must have fewer than 2^32 elements (wide: 2^32 bytes).  wide: wide_kernel (groups, bfloat16 out), 2 (plain): HALF.
+// pieces: null, or room for `units` pieces (the compute units), and the items of the last, partly filled round are cut.
 // Blocks are 8 wavefronts (two per SIMD, one block per compute unit): measured against 4, 5 and 6 on expert
 // shapes with even and with skewed numbers of rows per expert.
 JLE_API int jle_gemm_stream(const void* X, const void* W, void* Y, const int* offsets, const int* a_rows,
-                            const float* scale, int swiglu, int out_f32, int M, int Nout, int K, int G, int max_rows,
-                            int wide, hipStream_t s) {
+                            const float* scale, int swiglu, int out_f32, int M, int Nout, int K, int G,
+                            int wide, void* pieces, int units, hipStream_t s) {
   if (M <= 0 || Nout <= 0) return 0;
   if (wide) {
     if (offsets == nullptr || out_f32 || G < 1 || G > 65535 || !jle_gemm_stream_supported(Nout, K, swiglu) ||
@@ -487,20 +635,20 @@ JLE_API int jle_gemm_stream(const void* X, const void* W, void* Y, const int* of
     return wide == 2 ? launch_wide<false, true>(s, X, W, Y, offsets, a_rows, scale, M, Nout, K, G)
                      : launch_wide<false, false>(s, X, W, Y, offsets, a_rows, scale, M, Nout, K, G);
   }
-  if (G < 1 || G > 65535 || !jle_gemm_stream_supported(Nout, K, swiglu)) return JLE_BAD_ARG;
-  if (max_rows <= 0 || max_rows > M) max_rows = M;
+  if (G < 1 || G > 65535 || (offsets == nullptr && G != 1) || !jle_gemm_stream_supported(Nout, K, swiglu)) return JLE_BAD_ARG;
   constexpr int kWaves = 8;
-  const int passes = (max_rows + kRows - 1) / kRows;
   const int pairs = swiglu ? Nout / 32 : (Nout / 16 + 1) / 2;  // pairs of weight tiles = wavefronts needed per group
   const int nblk = (pairs + kWaves - 1) / kWaves;
-  if ((long long)nblk * passes * G > (1ll << 30)) return JLE_BAD_ARG;
-  if (swiglu) {
-    if (out_f32) launch_stream<true, float, kWaves>(nblk, passes, G, s, X, W, Y, offsets, a_rows, scale, M, Nout, K);
-    else launch_stream<true, bf16_t, kWaves>(nblk, passes, G, s, X, W, Y, offsets, a_rows, scale, M, Nout, K);
-  } else {
-    if (out_f32) launch_stream<false, float, kWaves>(nblk, passes, G, s, X, W, Y, offsets, a_rows, scale, M, Nout, K);
-    else launch_stream<false, bf16_t, kWaves>(nblk, passes, G, s, X, W, Y, offsets, a_rows, scale, M, Nout, K);
+  long long items = ((long long)M / kRows + (offsets == nullptr ? 1 : G)) * nblk;
+  if (pieces != nullptr) {
+    if (units < 2 || units > 65535 || K / BK < 2 * kLeastStages || G > kMostCutGroups ||
+        (uintptr_t)pieces % 16)
+      return JLE_BAD_ARG;
+    items += units;
   }
-  JLE_LAUNCH_CHECK();
-  return 0;
+  if (items > (1ll << 30)) return JLE_BAD_ARG;
+  const StreamArgs p = {(const bf16_t*)X, (const bf16_t*)W, Y, a_rows, scale, {offsets, M, G, nblk, kRows}, (f32x4*)pieces,
+                        (size_t)jle_gemm_stream_piece(M) / 16, Nout, K, units};
+  if (swiglu) return out_f32 ? launch_stream<true, float, kWaves>(p, items, s) : launch_stream<true, bf16_t, kWaves>(p, items, s);
+  return out_f32 ? launch_stream<false, float, kWaves>(p, items, s) : launch_stream<false, bf16_t, kWaves>(p, items, s);
 }

@@ -89,7 +89,7 @@ _SIGNATURES = {
     "jle_conv_rows": [_vp, _i, _i, _vp, _vp, _vp, _i, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _vp],
     "jle_conv_qk_prepare": [_vp, _i, _vp, _vp, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _f, _f, _vp, _vp, _i, _i,
                             _i, _i, _i, _i, _i, _i, _i, _vp],
-    "jle_gemm_stream": [_vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _i, _vp],
+    "jle_gemm_stream": [_vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _vp, _i, _vp],
     "jle_streams_mix_norm": [_vp, _i, _vp, _vp, _vp, _i, _vp, _i, _vp, _vp, _vp, _vp, _f, _vp, _i, _vp, _i, _i, _i, _i,
                              _vp],
     "jle_embed_sinusoid": [_vp, _vp, _vp, _i, _f, _vp, _vp, _i, _i, _i, _vp],
@@ -193,7 +193,7 @@ def _bind(path: str):
             fn.argtypes = args
             fn.restype = ctypes.c_int
     for name, args in (("jle_attention_mfma_supported", [_i, _i, _i, _i]),  # queries, not launches: no stream
-                       ("jle_greedy_blocks", [_i]), ("jle_gemm_stream_supported", [_i, _i, _i]), ("jle_gemm_f32_stream_supported", [_i, _i, _i]),
+                       ("jle_greedy_blocks", [_i]), ("jle_gemm_stream_supported", [_i, _i, _i]), ("jle_gemm_stream_piece", [_i]), ("jle_gemm_f32_stream_supported", [_i, _i, _i]),
                        ("jle_gemm_few_tiles", [_i] * 7),
                        ("jle_latent_attention_mfma_supported", [_i, _i, _i, _i, _i]),
                        ("jle_latent_values_supported", [_i] * 6),
@@ -1858,6 +1858,28 @@ class HipOps:
         mean = rows / groups
         return groups >= HipOps.WIDE_GROUPS and mean >= 90 and slots <= 192 and slots * (mean / 288 + 0.5) <= 224
 
+    CUT_STAGES = 64  # stages of 64 k from which on it pays
+
+    @staticmethod
+    @functools.lru_cache(maxsize=4096)
+    def stream_cuts(rows: int, groups: int, row_blocks: int, k: int, units: int) -> bool:
+        """Whether the products in passes cut the blocks left over behind the last full round of ``units`` compute units along
+        k (``row_blocks`` blocks of 256 rows of W a group; see ``gemm_stream.hip``).  How many are left over is known on the
+        device only, where nothing is cut if they fill more than half of the round; the launch that adds the pieces up is made
+        all the same, so this asks whether groups whose sizes scatter about their mean by twice its root can leave such a
+        rest.  Writing and adding up the pieces takes about 12 us, more than the round is shorter by with a short k.  Whole |
+        cut, us: 16 groups of 5,120 x 8,192 (320 blocks) with 64 rows 285 | 254, 128 309 | 276, 192 356 | 300; 8 of
+        4,096 x 7,168 (128) with 64 101 | 90, 190 140 | 117; 8 of 2,048 x 4,096 (64) with 64 55 | 42; an output head of
+        32,000 x 4,096 (125), 64 rows 67 | 61; but 16 of 2,048 x 3,072 (128) with 128 57 | 68, 8 of 4,096 x 2,048 (128) with
+        64 30 | 39."""
+        if k // 64 < HipOps.CUT_STAGES or groups > 1024:
+            return False
+        mean = rows / groups
+        spread = 2 * mean ** 0.5 if groups > 1 else 0.0
+        passes = [max(1, -(-int(mean + d) // 192)) for d in (-spread, spread)]
+        tail = groups * row_blocks * passes[0] % units
+        return passes[0] != passes[1] or 0 < tail <= units // 2
+
     def gemm_stream(self, a, b, *, offsets=None, a_rows=None, scale=None, swiglu=False, out_f32=False, rows=None,
                     expected=None):
         """bfloat16 product on MFMA for about a hundred rows per group and more, weights in the streaming layout and
@@ -1881,8 +1903,12 @@ class HipOps:
         wide, among = 0, m if expected is None else expected
         if offsets is not None and not out_f32 and a.numel() < 2 ** 31 and not (a.data_ptr() | b.data_ptr()) % 16:
             wide = 2 if not swiglu and self.stream_half(among, g, -(-nout // 128)) else self.stream_wide(among, g, -(-nout // 256))
+        pieces = None  # (sums of the pieces: 192 KiB each at most)
+        if not wide and self.stream_cuts(among, g, -(-nout // 256), k, self._compute_units):
+            room = self._query("jle_gemm_stream_piece", m) * self._compute_units
+            pieces = torch.empty(room, dtype=torch.uint8, device=a.device)
         self._call("jle_gemm_stream", _p(a), _p(b), _p(out), _p(offsets), _p(a_rows), _p(scale), int(swiglu),
-                   int(out_f32), m, nout, k, g, m, int(wide))
+                   int(out_f32), m, nout, k, g, int(wide), _p(pieces), self._compute_units)
         return out
 
     @staticmethod

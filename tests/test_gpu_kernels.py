@@ -1246,6 +1246,40 @@ def test_wide_tiles_of_the_weight_streaming_product(ops, counts, nout, k, swiglu
     assert torch.equal(*got)
 
 
+@pytest.mark.parametrize("counts,nout,k,swiglu", [
+    ([5, 0, 192, 193, 31, 385], 272, 4096, False),   # several passes, two blocks of W, the second of one tile
+    ([100, 33, 64], 544, 4352, True),                # pieces of unequal length
+    ([3] * 256, 64, 4096, False),                    # exactly a round of blocks: nothing to cut
+    ([3] * 257, 64, 4096, False),                    # one left over, in as many pieces as its stages allow
+    ([200] * 65, 512, 4096, True),                   # more groups than a look takes, blocks left over that stay whole
+    ([77], 2048, 16384, False)])                     # one group: all of it is cut
+def test_blocks_cut_along_k_of_the_weight_streaming_product(ops, counts, nout, k, swiglu):
+    from jax_llm_examples_amd.ops.layout import tile_
+    m, e = sum(counts), len(counts)
+    x, w = _rand(m + 3, k, dt=torch.bfloat16, seed=1), _rand(e, nout, k, dt=torch.bfloat16, scale=0.02, seed=2)
+    stored = w.clone()
+    tile_(stored)
+    off = torch.tensor([0] + counts).cumsum(0).int().to(DEV)
+    rows = torch.randperm(m + 3, generator=torch.Generator().manual_seed(3))[:m].int().to(DEV)
+    scale = _rand(m, seed=4)
+    ops.stream_wide, ops.stream_half, ops.stream_cuts = (lambda *a: False), (lambda *a: False), (lambda *a: True)
+    got = [ops.gemm_stream(x, stored, offsets=off, a_rows=rows, scale=scale, swiglu=swiglu, rows=m, out_f32=True) for _ in range(2)]
+    if e == 1:
+        got.append(ops.gemm_stream(x[rows.long()], stored[0], out_f32=True) * scale[:, None])  # (no offsets)
+    del ops.stream_wide, ops.stream_half, ops.stream_cuts
+    assert torch.equal(got[0], got[1]) and torch.equal(got[0], got[-1])
+    o = 0
+    for c, we in zip(counts, w):
+        want = x[rows[o: o + c].long()].double() @ we.double().T * scale[o: o + c, None].double()
+        if swiglu:
+            want = torch.nn.functional.silu(want[:, : nout // 2]) * want[:, nout // 2:]
+        if c:
+            # float32 sums of k products of bfloat16 numbers: sqrt(k) 2^-24 of the terms' size is 4e-6 at 4,096 in the worst
+            # order and a tenth of that as the matrix units add up; the activation doubles it
+            assert float((got[0][o: o + c].double() - want).norm() / want.norm()) <= 4e-6
+        o += c
+
+
 def test_rows_off_their_16_bytes_take_the_passes(ops):
     """Rows that begin at 8 bytes, where the wide tiles want 16."""
     from jax_llm_examples_amd.ops.layout import tile_
