@@ -1,7 +1,7 @@
 // Weight-streaming grouped matrix product for a moderate number of rows per group (prefill through
 // experts: around a hundred tokens per expert): bfloat16 in, float32 accumulate on MFMA.
 //
-//   Y[t, n] = scale[t] * sum_k X[arow(t), k] * W[g(t)][n, k]          (plain)
+//   Y[t, n] = scale[t] * sum_k X[arow(t), k] * W[g(t)][n, k]          (plain; optionally max(., 0)^2 of the rounded sum)
 //   Y[t, f] = silu(s * gate) * (s * up),  gate/up = rows f and F + f of W[g(t)]   (SWIGLU, s = scale[t])
 //
 // With so few rows the cost is reading W, and every element of W is needed by one wavefront only if
@@ -138,22 +138,35 @@ struct Cut {
 // Rows of a tile: a group's rows as even as multiples of 32 allow.
 __device__ __forceinline__ int rows_a_tile(int rows, int tiles) { return ((rows + tiles - 1) / tiles + 31) / 32 * 32; }
 
+// max(., 0)^2 of a sum as it would be stored
+template <typename OutT>
+__device__ __forceinline__ float relu2(float v) {
+  const float u = fmaxf(Num<OutT>::round(v), 0.f);
+  return u * u;
+}
+
 // A lane's sums of a row, four neighbouring rows of two tiles of W, scaled and stored.
 template <bool SWIGLU, typename OutT>
-__device__ __forceinline__ void finish_pair(OutT* __restrict__ Y, int t, const float* __restrict__ scale, f32x4 a0, f32x4 a1,
-                                            int Nout, int t0, int t1, int g) {
+__device__ __forceinline__ void finish_pair(OutT* __restrict__ Y, int t, const float* __restrict__ scale, int act, f32x4 a0,
+                                            f32x4 a1, int Nout, int t0, int t1, int g) {
   const float sc = scale != nullptr ? scale[t] : 1.f;
+  a0 *= sc;
+  a1 *= sc;
   if (SWIGLU) {
     float y[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const float gate = a0[i] * sc, up = a1[i] * sc;
-      y[i] = gate / (1.0f + expf(-gate)) * up;
-    }
+    for (int i = 0; i < 4; ++i) y[i] = a0[i] / (1.0f + expf(-a0[i])) * a1[i];
     store4<OutT>(Y + (size_t)t * (Nout >> 1) + t0 * 16 + 4 * g, y[0], y[1], y[2], y[3]);
   } else {
-    store4<OutT>(Y + (size_t)t * Nout + t0 * 16 + 4 * g, a0[0] * sc, a0[1] * sc, a0[2] * sc, a0[3] * sc);
-    if (t1 != t0) store4<OutT>(Y + (size_t)t * Nout + t1 * 16 + 4 * g, a1[0] * sc, a1[1] * sc, a1[2] * sc, a1[3] * sc);
+    if (act) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        a0[i] = relu2<OutT>(a0[i]);
+        a1[i] = relu2<OutT>(a1[i]);
+      }
+    }
+    store4<OutT>(Y + (size_t)t * Nout + t0 * 16 + 4 * g, a0[0], a0[1], a0[2], a0[3]);
+    if (t1 != t0) store4<OutT>(Y + (size_t)t * Nout + t1 * 16 + 4 * g, a1[0], a1[1], a1[2], a1[3]);
   }
 }
 
@@ -165,7 +178,7 @@ __device__ __forceinline__ void finish_pair(OutT* __restrict__ Y, int t, const f
 template <bool SWIGLU, typename OutT, int WAVES, int NTL>
 __device__ __forceinline__ void stream_block(const bf16_t* __restrict__ X, const bf16_t* __restrict__ w0,
                                              const bf16_t* __restrict__ w1, OutT* __restrict__ Y,
-                                             const int* __restrict__ a_rows, const float* __restrict__ scale,
+                                             const int* __restrict__ a_rows, const float* __restrict__ scale, int act,
                                              bf16_t (&sX)[2][kRows * BK], int tok0, int live, int K, int Nout, int t0,
                                              int t1, bool wave_ok, int first, int nstage, f32x4* __restrict__ piece) {
   constexpr int THREADS = WAVES * 64;
@@ -279,7 +292,7 @@ __device__ __forceinline__ void stream_block(const bf16_t* __restrict__ X, const
   for (int nt = 0; nt < NTL; ++nt) {
     const int row = nt * 16 + r;
     if (row >= live) continue;
-    finish_pair<SWIGLU>(Y, tok0 + row, scale, acc0[nt], acc1[nt], Nout, t0, t1, g);
+    finish_pair<SWIGLU>(Y, tok0 + row, scale, act, acc0[nt], acc1[nt], Nout, t0, t1, g);
   }
 }
 
@@ -292,7 +305,7 @@ struct StreamArgs {
   Items items;
   f32x4* pieces;     // null: nothing is cut
   size_t a_piece;    // f32x4 of a piece
-  int Nout, K, units;
+  int Nout, K, units, act;
 };
 
 // Item `left`'s group, how many passes the group has, and which of the group's items it is; `items` there are.
@@ -354,7 +367,7 @@ __global__ __launch_bounds__(WAVES * 64, 2) void gemm_stream_kernel(StreamArgs p
   const bf16_t* w0 = We + (size_t)t0 * nkb * 512 + lane * 8;
   const bf16_t* w1 = We + (size_t)t1 * nkb * 512 + lane * 8;
 #define GO(NTL_) \
-  stream_block<SWIGLU, OutT, WAVES, NTL_>(p.X, w0, w1, (OutT*)p.Y, p.a_rows, p.scale, sX, tok0, live, K, Nout, t0, t1, \
+  stream_block<SWIGLU, OutT, WAVES, NTL_>(p.X, w0, w1, (OutT*)p.Y, p.a_rows, p.scale, p.act, sX, tok0, live, K, Nout, t0, t1, \
                                           wave_ok, first, stages, piece)
   if (live <= 32) GO(2);
   else if (live <= 64) GO(4);
@@ -388,7 +401,7 @@ __global__ __launch_bounds__(WAVES * 64) void add_pieces_kernel(StreamArgs p) {
       a1 += from[64];
     }
     if (nt * 16 + r < at.live)
-      finish_pair<SWIGLU>((OutT*)p.Y, at.tok0 + nt * 16 + r, p.scale, a0, a1, p.Nout, t0, t1, lane >> 4);
+      finish_pair<SWIGLU>((OutT*)p.Y, at.tok0 + nt * 16 + r, p.scale, p.act, a0, a1, p.Nout, t0, t1, lane >> 4);
   }
 }
 
@@ -416,8 +429,8 @@ constexpr uint32_t wide_stage(bool half) { return (uint32_t)wide_rows(half) * BK
 template <bool SWIGLU, bool HALF, int NT>
 __device__ __forceinline__ void wide_block(const bf16_t* __restrict__ X, const bf16_t* __restrict__ We,
                                            bf16_t* __restrict__ Y, const int* __restrict__ a_rows,
-                                           const float* __restrict__ scale, unsigned char* smem, int tok0, int live, int K,
-                                           int Nout, int nb) {
+                                           const float* __restrict__ scale, int act, unsigned char* smem, int tok0,
+                                           int live, int K, int Nout, int nb) {
   static_assert(NT % 2 == 0, "a wavefront brings NT / 2 kilobytes of a stage's rows");
   static_assert(!HALF || !SWIGLU, "half a block of rows of W: plain products only");
   constexpr int NW = HALF ? NT / 2 : NT;  // tiles of X a wavefront multiplies with
@@ -540,6 +553,7 @@ __device__ __forceinline__ void wide_block(const bf16_t* __restrict__ X, const b
           y[e] = gate / (1.0f + expf(-gate)) * up;
         } else {
           y[e] = acc[i][n][e] * sc;
+          if (act) y[e] = relu2<bf16_t>(y[e]);
         }
       }
       store4<bf16_t>(Y + (size_t)t * (SWIGLU ? half : Nout) + tile * 16 + 4 * g, y[0], y[1], y[2], y[3]);
@@ -551,7 +565,7 @@ template <bool SWIGLU, bool HALF>
 __global__ __launch_bounds__(256, 1) void wide_kernel(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W,
                                                       bf16_t* __restrict__ Y, const int* __restrict__ offsets,
                                                       const int* __restrict__ a_rows, const float* __restrict__ scale,
-                                                      int Nout, int K, int G, int nblk8) {
+                                                      int act, int Nout, int K, int G, int nblk8) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
   constexpr int kWideRows = wide_rows(HALF);
   const Items items = {offsets, 0, G, nblk8, kWideRows};
@@ -565,7 +579,7 @@ __global__ __launch_bounds__(256, 1) void wide_kernel(const bf16_t* __restrict__
   const int tok0 = lo + tile * per, live = min(per, rows - tile * per);
   if (live <= 0) return;
   const bf16_t* We = W + (size_t)e * Nout * K;
-#define GO(NT_) wide_block<SWIGLU, HALF, NT_>(X, We, Y, a_rows, scale, smem, tok0, live, K, Nout, nb)
+#define GO(NT_) wide_block<SWIGLU, HALF, NT_>(X, We, Y, a_rows, scale, act, smem, tok0, live, K, Nout, nb)
   if constexpr (HALF) {
     if (live > 256) {
       GO(18);
@@ -583,7 +597,7 @@ __global__ __launch_bounds__(256, 1) void wide_kernel(const bf16_t* __restrict__
 
 template <bool SW, bool HALF>
 int launch_wide(hipStream_t s, const void* X, const void* W, void* Y, const int* offsets, const int* a_rows,
-                const float* scale, int M, int Nout, int K, int G) {
+                const float* scale, int act, int M, int Nout, int K, int G) {
   constexpr uint32_t lds = 3 * wide_stage(HALF);
   if (const int rc = allow_lds(wide_kernel<SW, HALF>, lds)) return rc;
   constexpr int of8 = SW || HALF ? 1024 : 2048;  // columns of Y of eight blocks
@@ -591,7 +605,7 @@ int launch_wide(hipStream_t s, const void* X, const void* W, void* Y, const int*
   const long long items = ((long long)M / wide_rows(HALF) + G) * nblk8;
   if (items > (1ll << 30)) return JLE_BAD_ARG;
   hipLaunchKernelGGL((wide_kernel<SW, HALF>), dim3((unsigned)items), dim3(256), lds, s, (const bf16_t*)X, (const bf16_t*)W,
-                     (bf16_t*)Y, offsets, a_rows, scale, Nout, K, G, nblk8);
+                     (bf16_t*)Y, offsets, a_rows, scale, act, Nout, K, G, nblk8);
   JLE_LAUNCH_CHECK();
   return 0;
 }
@@ -620,20 +634,20 @@ JLE_API int jle_gemm_stream_piece(int M) { return (M < kRows ? (M + 31) / 32 * 3
 
 // X [*, K] bf16, W [G, Nout, K] bf16 in the streaming layout, Y [M, Nout] (or [M, Nout / 2] with swiglu) bf16 or
 // float32; X must have fewer than 2^32 elements (wide: 2^32 bytes).  wide: wide_kernel (groups, bfloat16 out), 2 (plain): HALF.
-// pieces: null, or room for `units` pieces (the compute units), and the items of the last, partly filled round are cut.
+// act 1 (plain): max(., 0)^2 of the rounded sums.  pieces: null, or room for `units` pieces (the compute units), and the items of the last, partly filled round are cut.
 // Blocks are 8 wavefronts (two per SIMD, one block per compute unit): measured against 4, 5 and 6 on expert
 // shapes with even and with skewed numbers of rows per expert.
 JLE_API int jle_gemm_stream(const void* X, const void* W, void* Y, const int* offsets, const int* a_rows,
-                            const float* scale, int swiglu, int out_f32, int M, int Nout, int K, int G,
+                            const float* scale, int swiglu, int act, int out_f32, int M, int Nout, int K, int G,
                             int wide, void* pieces, int units, hipStream_t s) {
   if (M <= 0 || Nout <= 0) return 0;
   if (wide) {
     if (offsets == nullptr || out_f32 || G < 1 || G > 65535 || !jle_gemm_stream_supported(Nout, K, swiglu) ||
         ((uintptr_t)X | (uintptr_t)W | (uintptr_t)Y) % 16)
       return JLE_BAD_ARG;
-    if (swiglu) return launch_wide<true, false>(s, X, W, Y, offsets, a_rows, scale, M, Nout, K, G);
-    return wide == 2 ? launch_wide<false, true>(s, X, W, Y, offsets, a_rows, scale, M, Nout, K, G)
-                     : launch_wide<false, false>(s, X, W, Y, offsets, a_rows, scale, M, Nout, K, G);
+    if (swiglu) return launch_wide<true, false>(s, X, W, Y, offsets, a_rows, scale, act, M, Nout, K, G);
+    return wide == 2 ? launch_wide<false, true>(s, X, W, Y, offsets, a_rows, scale, act, M, Nout, K, G)
+                     : launch_wide<false, false>(s, X, W, Y, offsets, a_rows, scale, act, M, Nout, K, G);
   }
   if (G < 1 || G > 65535 || (offsets == nullptr && G != 1) || !jle_gemm_stream_supported(Nout, K, swiglu)) return JLE_BAD_ARG;
   constexpr int kWaves = 8;
@@ -648,7 +662,7 @@ JLE_API int jle_gemm_stream(const void* X, const void* W, void* Y, const int* of
   }
   if (items > (1ll << 30)) return JLE_BAD_ARG;
   const StreamArgs p = {(const bf16_t*)X, (const bf16_t*)W, Y, a_rows, scale, {offsets, M, G, nblk, kRows}, (f32x4*)pieces,
-                        (size_t)jle_gemm_stream_piece(M) / 16, Nout, K, units};
+                        (size_t)jle_gemm_stream_piece(M) / 16, Nout, K, units, act};
   if (swiglu) return out_f32 ? launch_stream<true, float, kWaves>(p, items, s) : launch_stream<true, bf16_t, kWaves>(p, items, s);
   return out_f32 ? launch_stream<false, float, kWaves>(p, items, s) : launch_stream<false, bf16_t, kWaves>(p, items, s);
 }

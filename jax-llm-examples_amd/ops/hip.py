@@ -1880,11 +1880,11 @@ class HipOps:
         tail = groups * row_blocks * passes[0] % units
         return passes[0] != passes[1] or 0 < tail <= units // 2
 
-    def gemm_stream(self, a, b, *, offsets=None, a_rows=None, scale=None, swiglu=False, out_f32=False, rows=None,
+    def gemm_stream(self, a, b, *, offsets=None, a_rows=None, scale=None, swiglu=False, relu2=False, out_f32=False, rows=None,
                     expected=None):
         """bfloat16 product on MFMA for about a hundred rows per group and more, weights in the streaming layout and
         read once per 192 rows of a group, or per tile of up to 256 or 288 (:meth:`stream_wide`, :meth:`stream_half`; see
-        ``gemm_stream.hip``).  ``expected``: how many of the rows are expected to belong to a group, if not all."""
+        ``gemm_stream.hip``).  ``relu2``: of every rounded sum ``max(., 0)^2``.  ``expected``: how many of the rows are expected to belong to a group, if not all."""
         if b.dim() == 2:
             b = b.unsqueeze(0)
         g, nout, k = b.shape
@@ -1908,7 +1908,7 @@ class HipOps:
             room = self._query("jle_gemm_stream_piece", m) * self._compute_units
             pieces = torch.empty(room, dtype=torch.uint8, device=a.device)
         self._call("jle_gemm_stream", _p(a), _p(b), _p(out), _p(offsets), _p(a_rows), _p(scale), int(swiglu),
-                   int(out_f32), m, nout, k, g, int(wide), _p(pieces), self._compute_units)
+                   int(relu2), int(out_f32), m, nout, k, g, int(wide), _p(pieces), self._compute_units)
         return out
 
     @staticmethod
@@ -2516,6 +2516,8 @@ class HipOps:
             act = product(h, w_up, 2 * f, d, fused=True, a_rows=sorted_token)
         elif mfma and m <= 2 * self.SKINNY_MAX_ROWS and self._few_fits(h, w_up):  # (the activation of the rounded sums too)
             act = self.gemm_few(h, w_up, offsets=offsets, a_rows=sorted_token, tiled=tiled, relu2=True)
+        elif mfma and m > 2 * self.SKINNY_MAX_ROWS and tiled and self.stream_supported(f, d, False):
+            act = product(h, w_up, f, d, a_rows=sorted_token, relu2=True)
         else:
             act = self.relu2(product(h, w_up, f, d, a_rows=sorted_token))
         routed = product(act, w_down, d, f, scale=sorted_weight)

@@ -1246,6 +1246,22 @@ def test_wide_tiles_of_the_weight_streaming_product(ops, counts, nout, k, swiglu
     assert torch.equal(*got)
 
 
+@pytest.mark.parametrize("way", ["passes", "cut", "wide", "half"])
+def test_squared_relu_behind_the_weight_streaming_product(ops, way):
+    """The bits of the product and the activation as launches of their own, by every kernel that takes such rows."""
+    from jax_llm_examples_amd.ops.layout import tile_
+    counts, nout, k = [3, 0, 200, 70], 272, 4096
+    x, w = _rand(sum(counts), k, dt=torch.bfloat16, seed=1), _rand(4, nout, k, dt=torch.bfloat16, scale=0.02, seed=2)
+    x[5, 7], x[9] = float("nan"), 0.0
+    tile_(w)
+    off = torch.tensor([0] + counts).cumsum(0).int().to(DEV)
+    ops.stream_wide, ops.stream_half, ops.stream_cuts = (lambda *a: way == "wide"), (lambda *a: way == "half"), (lambda *a: way == "cut")
+    got = ops.gemm_stream(x, w, offsets=off, relu2=True)
+    want = ops.relu2(ops.gemm_stream(x, w, offsets=off))
+    del ops.stream_wide, ops.stream_half, ops.stream_cuts
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16)) and bool((got >= 0).sum() > 0)
+
+
 @pytest.mark.parametrize("counts,nout,k,swiglu", [
     ([5, 0, 192, 193, 31, 385], 272, 4096, False),   # several passes, two blocks of W, the second of one tile
     ([100, 33, 64], 544, 4352, True),                # pieces of unequal length
