@@ -89,7 +89,7 @@ _SIGNATURES = {
     "jle_conv_rows": [_vp, _i, _i, _vp, _vp, _vp, _i, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _vp],
     "jle_conv_qk_prepare": [_vp, _i, _vp, _vp, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _f, _f, _vp, _vp, _i, _i,
                             _i, _i, _i, _i, _i, _i, _i, _vp],
-    "jle_gemm_stream": [_vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _vp, _i, _vp],
+    "jle_gemm_stream": [_vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _i, _vp, _i, _vp],
     "jle_streams_mix_norm": [_vp, _i, _vp, _vp, _vp, _i, _vp, _i, _vp, _vp, _vp, _vp, _f, _vp, _i, _vp, _i, _i, _i, _i,
                              _vp],
     "jle_embed_sinusoid": [_vp, _vp, _vp, _i, _f, _vp, _vp, _i, _i, _i, _vp],
@@ -1085,7 +1085,8 @@ class HipOps:
         takes weights of fewer than 2^24 numbers (8 rows of 2048 x 2048 12 -> 6.6), and of up to 2^25 with a k of 5,120 or
         more (2048 x 8192 23 -> 16, 5120 x 5120 29 -> 25) or with the activation, which is a launch of its own behind the
         library's; others it does not gain (8 rows of 8192 x 2048 15.8 against 17.6, 4096 x 4096 15.7 against 17.4).  Many
-        rows: see :meth:`split_ranges`.  In between neither gains."""
+        rows: see :meth:`split_ranges`.  In between the experts' kernel for few rows where its blocks are about one round
+        (:meth:`f32_tiles_pay`); else neither gains."""
         if h.dtype != torch.float32 or w.dtype != torch.float32 or h.dim() != 2 or w.dim() != 2:
             return None
         rows, k = h.shape
@@ -1096,10 +1097,27 @@ class HipOps:
             return None
         if rows <= 4 or rows <= 8 and (n * k < 1 << 24 or n * k <= 1 << 25 and (k >= 5120 or act >= 0)):
             return self.gemm_f32_rows(h, w, act)
+        if (act <= 0 and HipOps.f32_tiles_pay(rows, n, k, act == 0)
+                and not (torch.is_grad_enabled() and (h.requires_grad or w.requires_grad))):
+            return self.gemm_f32_skinny(h, w, swiglu=act == 0)
         ranges = self.split_ranges(rows, n, k, act >= 0, self._compute_units)
         if ranges:
             return self.gemm_f32_split(h, w, act, ranges)
         return None
+
+    @staticmethod
+    def f32_tiles_pay(rows: int, n: int, k: int, gated: bool) -> bool:
+        """Whether a dense float32 product goes through the kernel of the experts' few rows, a block for 16 columns and 16 rows
+        (``gemm_f32.hip``; on the float32 matrix instructions, errors against 64 bits from a third to three quarters of the
+        library's).  A block takes 4 us and 3 more per 1,024 of k, so it is the faster one while its blocks are one round of
+        the compute units (two with a short k) and k is no longer than 2,048.  The library's | this, us: 64 x 64, 32 rows 4.7 |
+        4.1, 128 rows 6.3 | 4.2; 64 x 256, 32 rows 9.1 | 5.0; 512 x 512, 128 rows 11.1 | 5.8; 1,024 x 1,024, 64 rows
+        11.8 | 6.2, 128 rows (512 blocks) 11.9 | 9.4; 2,048 x 2,048, 16 rows 12.9 | 10.2, 32 rows 13.4 | 10.6, 48 rows (384
+        blocks) 13.5 | 15.9; 2,048 x 4,096, 16 rows 15.1 | 18.5.  Gate and up, with the activation, of 512 x 64, 32 rows 7.0 |
+        4.7; 2,048 x 2,048, 64 rows 17.3 | 14.1; 8,192 x 2,048, 16 rows 23.9 | 19.6.  (And the library's product costs the host
+        20 us a call, this one 7.)"""
+        tiles = -(-(n // 2 if gated else n) // 16) * -(-rows // 16)
+        return rows <= HipOps.F32_SKINNY_ROWS and k <= 2048 and tiles <= (512 if k <= 1024 and not gated else 256)
 
     def linear(self, h, w, out_dtype=None):
         """``h @ w.T``: through the BLAS library; up to a few tens of bfloat16 rows (:meth:`_few`), and few or many float32

@@ -26,6 +26,13 @@ def test_dense_float32_products_by_size():
     assert rule(tensor(1, 64), tensor(32, 60)) is None  # (the library's product refuses it)
 
 
+@pytest.mark.parametrize("rows, n, k, gated, pays", [(9, 64, 64, False, True), (128, 64, 64, False, True), (129, 64, 64, False, False),
+    (32, 2048, 2048, False, True), (33, 2048, 2048, False, False), (128, 1024, 1024, False, True), (128, 2048, 512, False, False),
+    (64, 2048, 2048, True, True), (65, 2048, 2048, True, False), (16, 512, 2052, False, False)])
+def test_dense_float32_products_of_tens_of_rows_by_size(rows, n, k, gated, pays):
+    assert HipOps.f32_tiles_pay(rows, n, k, gated) == pays
+
+
 @pytest.mark.parametrize("rows", [1, 512])
 @pytest.mark.parametrize("a, b", [("cuda:0", "cuda:1"), ("cuda:1", "cuda:0"), ("cuda:0", "cpu"), ("cpu", "cuda:0"),
                                   ("cuda:1", "cuda:1")])
