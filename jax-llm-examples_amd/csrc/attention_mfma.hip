@@ -52,8 +52,8 @@ struct Biasing {
   int L;
   float cap_in, cap_out;
 };
-constexpr int kNoBias = 0, kBiasTable = 1, kBiasPenalty = 2, kCapped = 3;  // what a kernel is compiled for
-constexpr bool light(int biased) { return biased == kNoBias || biased == kCapped; }  // (few registers beyond the plain kernel's)
+constexpr int kNoBias = 0, kBiasTable = 1, kBiasPenalty = 2, kCapped = 3, kKept = 4;  // what a kernel is compiled for (kKept: first keys kept beside a window)
+constexpr bool light(int biased) { return biased == kNoBias || biased == kCapped || biased == kKept; }  // (few registers beyond the plain kernel's)
 
 // cap tanh(s / cap) in the exponent's base-2 units from an unscaled score: tanh z = 1 - 2 / (exp(2 z) + 1)
 __device__ __forceinline__ float capped_log2(float v, const Biasing& b) {
@@ -811,10 +811,10 @@ __device__ __forceinline__ void softmax64_and_values(f32x4 (&st)[CT][4], int hal
                                                      const Columns (&col)[CT], int k_lo, int k_hi, float scale_log2,
                                                      float (&m)[CT], float (&l)[CT], f32x4 (&acc)[CT][DH / 16],
                                                      Biasing bias = Biasing{nullptr, 0, 0.f, 0.f}, bool far = false,
-                                                     const float* far_b = nullptr) {
+                                                     const float* far_b = nullptr, int keep = 0) {
   constexpr int DT = DH / 16;
   const int g = (threadIdx.x & 63) >> 4;
-  const float sc = BIASED ? 1.0f : scale_log2;  // (biased scores are scaled where the bias is added)
+  const float sc = light(BIASED) && BIASED != kCapped ? scale_log2 : 1.0f;  // (biased scores are scaled where the bias is added)
   bf16x8 pb[CT][2];
   bf16x8 pb_lo[BIASED == kBiasTable ? CT : 1][2];  // (see softmax_and_values)
   float corr[CT];
@@ -847,7 +847,7 @@ __device__ __forceinline__ void softmax64_and_values(f32x4 (&st)[CT][4], int hal
         }
         if (MASKED) {
           const int key = kb + 32 * (tt >> 1) + 8 * g + 4 * (tt & 1) + i;
-          const bool ok = key >= col[ct].lo && key <= col[ct].hi;
+          const bool ok = (key >= col[ct].lo || (BIASED == kKept && key < keep)) && key <= col[ct].hi;
           v = ok ? v : -INFINITY;
           st[ct][tt][i] = v;
         }
@@ -905,22 +905,22 @@ __device__ __forceinline__ void softmax64_and_values(f32x4 (&st)[CT][4], int hal
     }
     if (MASKED) {
       // values: keys outside [k_lo, k_hi] may never have been written: they are read as zero
-      uint32_t keep[2][2];
+      uint32_t live[2][2];
 #pragma unroll
       for (int t2 = 0; t2 < 2; ++t2)
 #pragma unroll
         for (int h2 = 0; h2 < 2; ++h2) {
           const int key = kb + 32 * hf + 8 * g + 4 * t2 + 2 * h2;
-          const uint32_t lo_ok = (key >= k_lo && key <= k_hi) ? 0x0000ffffu : 0u;
-          const uint32_t hi_ok = (key + 1 >= k_lo && key + 1 <= k_hi) ? 0xffff0000u : 0u;
-          keep[t2][h2] = lo_ok | hi_ok;
+          const uint32_t lo_ok = ((key >= k_lo || (BIASED == kKept && key < keep)) && key <= k_hi) ? 0x0000ffffu : 0u;
+          const uint32_t hi_ok = ((key + 1 >= k_lo || (BIASED == kKept && key + 1 < keep)) && key + 1 <= k_hi) ? 0xffff0000u : 0u;
+          live[t2][h2] = lo_ok | hi_ok;
         }
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt) {
-        vraw[dt].x &= keep[0][0];
-        vraw[dt].y &= keep[0][1];
-        vraw[dt].z &= keep[1][0];
-        vraw[dt].w &= keep[1][1];
+        vraw[dt].x &= live[0][0];
+        vraw[dt].y &= live[0][1];
+        vraw[dt].z &= live[1][0];
+        vraw[dt].w &= live[1][1];
       }
     }
 #pragma unroll
@@ -942,7 +942,7 @@ __global__ __launch_bounds__(256, 2) void attention_prefill_lds_kernel(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ kv, bf16_t* __restrict__ out,
     const int* __restrict__ positions, const int* __restrict__ token_segment, const int* __restrict__ block_table,
     int table_width, const int* __restrict__ tiles, const int* __restrict__ groups, int ret_mode, int ret_param,
-    float scale_log2, int Hq, int Hkv, int ps, Biasing bias, const float* __restrict__ sink) {
+    float scale_log2, int Hq, int Hkv, int ps, Biasing bias, const float* __restrict__ sink, int keep) {
   constexpr int DH = 128, CT = 2, KC = DH / 32, DT = DH / 16;
   constexpr int NB = 2;
   constexpr int TILE = 16 * DH * 2;  // bytes of a key tile, and of a value tile
@@ -986,7 +986,7 @@ __global__ __launch_bounds__(256, 2) void attention_prefill_lds_kernel(
     col[ct].token = c < nt ? n0 + c : n0;
     col[ct].head = h;
     col[ct].lo = ok ? first_key(ret_mode, ret_param, pos) : 1;
-    col[ct].hi = ok ? pos : 0;
+    col[ct].hi = ok ? pos : BIASED == kKept ? -1 : 0;  // (kept: key 0 is everyone's)
     col[ct].pos = pos;
     const bf16_t* qrow = q + ((size_t)col[ct].token * Hq + h) * DH + g * 8;
 #pragma unroll
@@ -1044,14 +1044,20 @@ __global__ __launch_bounds__(256, 2) void attention_prefill_lds_kernel(
   const uint32_t v_rd = (uint32_t)(c16 * 32 + (((g & 1) ^ ((c16 >> 2) & 1)) * 16));  // + dt * 512 + the page tile's
 
   bool bad = false;
-  const int kb_first = (k_lo / 64) * 64;
+  const int kb_window = (k_lo / 64) * 64;
+  // kept: the steps before the window's that hold kept keys, then on from the window's first
+  const int kept_end = BIASED == kKept ? (min(keep, kb_window) + 63) / 64 * 64 : 0;
+  const int kb_first = kept_end > 0 ? 0 : kb_window;
+  auto behind = [&](int kb) __attribute__((always_inline)) {  // the step behind the one at kb
+    return BIASED == kKept && kb + 64 >= kept_end && kb + 64 < kb_window ? kb_window : kb + 64;
+  };
   // this wavefront's tile of the next step to ask for: its first key, and where that lies in the pages
   int my_key = kb_first + 16 * wave;
   int page_index = my_key / ps, page_off = my_key % ps;
   int page = 0;
   bool need = false;
   auto look_up = [&]() {
-    need = my_key <= k_hi && my_key + 15 >= k_lo;
+    need = my_key <= k_hi && (my_key + 15 >= k_lo || (BIASED == kKept && my_key < keep));
     page = table[min(page_index, table_width - 1)];  // (asked for now, looked at when the step's loads are asked for)
   };
   look_up();
@@ -1067,14 +1073,20 @@ __global__ __launch_bounds__(256, 2) void attention_prefill_lds_kernel(
     for (int i = 0; i < 4; ++i) load_to_lds16(keys, k_src[i], dst + i * 1024);
 #pragma unroll
     for (int i = 0; i < 4; ++i) load_to_lds16(values, v_src[i], dst + 4 * TILE + i * 1024);
-    my_key += 64;
-    page_off += 64;  // a page holds at least 16 keys: at most four pages further
+    const int from = my_key;
+    my_key = behind(my_key - 16 * wave) + 16 * wave;
+    if (BIASED == kKept && my_key != from + 64) {
+      page_index = my_key / ps;
+      page_off = my_key % ps;
+    } else {
+      page_off += 64;  // a page holds at least 16 keys: at most four pages further
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      if (page_off >= ps) {
-        page_off -= ps;
-        ++page_index;
-      }
+      for (int i = 0; i < 4; ++i)
+        if (page_off >= ps) {
+          page_off -= ps;
+          ++page_index;
+        }
+    }
     look_up();
   };
 
@@ -1082,11 +1094,11 @@ __global__ __launch_bounds__(256, 2) void attention_prefill_lds_kernel(
   asm volatile("" ::: "memory");
   load_step(0);
   int buf = 0;
-  for (int kb = kb_first; kb <= k_hi; kb += 64) {
+  for (int kb = kb_first; kb <= k_hi; kb = behind(kb)) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this step's eight loads have landed
     __syncthreads();
     load_step(buf ^ 1);  // the next step, into the buffer that every wavefront has just left
-    if (head_ok && kb + 63 >= my_lo && kb <= my_hi) {
+    if (head_ok && (kb + 63 >= my_lo || (BIASED == kKept && kb < keep)) && kb <= my_hi) {
       const unsigned char* sb = smem + buf * BUF;
       const int halves = kb + 32 <= my_hi ? 2 : 1;  // (tiles 2 and 3 lie past this wavefront's last key)
       f32x4 st[CT][4];
@@ -1114,7 +1126,7 @@ __global__ __launch_bounds__(256, 2) void attention_prefill_lds_kernel(
             for (int ct = 0; ct < CT; ++ct)
               st[ct][2 * hf + t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kt[t][c], qb[ct][c], st[ct][2 * hf + t], 0, 0, 0);
       }
-      if (BIASED) {
+      if (BIASED && BIASED != kKept) {
         const bool far = kb + 63 <= far_until;
         if (kb >= all_lo && kb + 63 <= all_hi)
           softmax64_and_values<DH, CT, false, BIASED>(st, 2, sb + 4 * TILE, v_rd, TILE, kb, col, k_lo, k_hi, scale_log2, m,
@@ -1123,9 +1135,10 @@ __global__ __launch_bounds__(256, 2) void attention_prefill_lds_kernel(
           softmax64_and_values<DH, CT, true, BIASED>(st, halves, sb + 4 * TILE, v_rd, TILE, kb, col, k_lo, k_hi,
                                                    scale_log2, m, l, acc, bias, far, far_b);
       } else if (kb >= all_lo && kb + 63 <= all_hi)  // the same for the whole wavefront
-        softmax64_and_values<DH, CT, false>(st, 2, sb + 4 * TILE, v_rd, TILE, kb, col, k_lo, k_hi, scale_log2, m, l, acc);
+        softmax64_and_values<DH, CT, false, BIASED>(st, 2, sb + 4 * TILE, v_rd, TILE, kb, col, k_lo, k_hi, scale_log2, m, l, acc);
       else  // (keys outside a column's range, those of tiles that were not asked for among them, count for nothing)
-        softmax64_and_values<DH, CT, true>(st, halves, sb + 4 * TILE, v_rd, TILE, kb, col, k_lo, k_hi, scale_log2, m, l, acc);
+        softmax64_and_values<DH, CT, true, BIASED>(st, halves, sb + 4 * TILE, v_rd, TILE, kb, col, k_lo, k_hi, scale_log2, m, l,
+                                                   acc, bias, false, nullptr, keep);
     }
     buf ^= 1;
   }
@@ -1601,19 +1614,19 @@ JLE_API int jle_attention_prefill(const void* q, const void* kv, void* out, cons
         if (bias_len < 0)
           hipLaunchKernelGGL(attention_prefill_lds_kernel<kBiasPenalty>, gs, dim3(kGroupWaves * 64), 0, s, (const bf16_t*)q,
                              (const bf16_t*)kv, (bf16_t*)out, positions, token_segment, block_table, table_width, tiles,
-                             groups, ret_mode, ret_param, sl, Hq, Hkv, ps, bs, sink);
+                             groups, ret_mode, ret_param, sl, Hq, Hkv, ps, bs, sink, 0);
         else if (cap > 0.f)
           hipLaunchKernelGGL(attention_prefill_lds_kernel<kCapped>, gs, dim3(kGroupWaves * 64), 0, s, (const bf16_t*)q,
                              (const bf16_t*)kv, (bf16_t*)out, positions, token_segment, block_table, table_width, tiles,
-                             groups, ret_mode, ret_param, sl, Hq, Hkv, ps, bs, sink);
+                             groups, ret_mode, ret_param, sl, Hq, Hkv, ps, bs, sink, 0);
         else if (bias != nullptr)
           hipLaunchKernelGGL(attention_prefill_lds_kernel<kBiasTable>, gs, dim3(kGroupWaves * 64), 0, s, (const bf16_t*)q,
                              (const bf16_t*)kv, (bf16_t*)out, positions, token_segment, block_table, table_width, tiles,
-                             groups, ret_mode, ret_param, sl, Hq, Hkv, ps, bs, sink);
+                             groups, ret_mode, ret_param, sl, Hq, Hkv, ps, bs, sink, 0);
         else
           hipLaunchKernelGGL(attention_prefill_lds_kernel<kNoBias>, gs, dim3(kGroupWaves * 64), 0, s, (const bf16_t*)q,
                              (const bf16_t*)kv, (bf16_t*)out, positions, token_segment, block_table, table_width, tiles,
-                             groups, ret_mode, ret_param, sl, Hq, Hkv, ps, bs, sink);
+                             groups, ret_mode, ret_param, sl, Hq, Hkv, ps, bs, sink, 0);
         break;
       case 256: PICK_S(256); break;
     }
@@ -1654,17 +1667,26 @@ JLE_API int jle_attention_prefill(const void* q, const void* kv, void* out, cons
 }
 
 // A window of `window` keys whose queries also see the sequence's first `keep` keys; tiles of 16 or 32 tokens, one
-// wavefront per (tile, query head).
+// wavefront per (tile, query head), or (groups, as jle_attention_prefill has them; heads of 128, tiles of 32) those of a kv
+// head sharing keys.
 JLE_API int jle_attention_prefill_kept(const void* q, const void* kv, void* out, const int* positions,
                                        const int* token_segment, const int* block_table, int table_width,
-                                       const int* tiles, int num_tiles, int tile_tokens, int window, int keep,
-                                       float scale, int Hq, int Hkv, int dh, int ps, hipStream_t s) {
+                                       const int* tiles, int num_tiles, int tile_tokens, const int* groups, int num_groups,
+                                       int window, int keep, float scale, int Hq, int Hkv, int dh, int ps, hipStream_t s) {
   if (num_tiles <= 0) return 0;
   if (!jle_attention_mfma_supported(dh, Hq, Hkv, ps)) return JLE_BAD_ARG;
   if (window <= 0 || keep < 0 || (tile_tokens != 16 && tile_tokens != 32)) return JLE_BAD_ARG;
   const long long items = (long long)num_tiles * Hq;
   dim3 g((unsigned)((items + 3) / 4)), b(256);
   const float sl = scale * kLog2e;
+  if (groups != nullptr) {
+    if (tile_tokens != 32 || num_groups <= 0 || dh != 128) return JLE_BAD_ARG;
+    hipLaunchKernelGGL(attention_prefill_lds_kernel<kKept>, dim3((unsigned)((long long)num_groups * Hkv)), dim3(kGroupWaves * 64),
+                       0, s, (const bf16_t*)q, (const bf16_t*)kv, (bf16_t*)out, positions, token_segment, block_table,
+                       table_width, tiles, groups, 2, window, sl, Hq, Hkv, ps, Biasing{nullptr, 0, 0.f, 0.f}, nullptr, keep);
+    JLE_LAUNCH_CHECK();
+    return 0;
+  }
 #define LAUNCH_K(DH, CT)                                                                                             \
   hipLaunchKernelGGL((attention_prefill_kept_kernel<DH, CT>), g, b, 0, s, (const bf16_t*)q, (const bf16_t*)kv,       \
                      (bf16_t*)out, positions, token_segment, block_table, table_width, tiles, num_tiles, window,     \

@@ -122,7 +122,7 @@ _SIGNATURES = {
     "jle_latent_expanded_gather": [_vp, _vp, _vp, _i, _vp, _i, _vp, _vp, _i, _i, _i, _vp],
     "jle_latent_expanded_attention": [_vp, _i, _vp, _vp, _vp, _i, _vp, _vp, _vp, _i, _i, _f, _i, _vp, _vp],
     "jle_relu2": [_vp, _vp, _i, _ll, _vp],
-    "jle_attention_prefill_kept": [_vp, _vp, _vp, _vp, _vp, _vp, _i, _vp, _i, _i, _i, _i, _f, _i, _i, _i, _i, _vp],
+    "jle_attention_prefill_kept": [_vp, _vp, _vp, _vp, _vp, _vp, _i, _vp, _i, _i, _vp, _i, _i, _i, _f, _i, _i, _i, _i, _vp],
     "jle_paged_attention_kept": [_vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _f, _i, _i, _i, _i, _i, _i, _i, _i, _vp,
                                  _vp, _vp],
     "jle_paged_attention_biased": [_vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _f, _i, _i, _i, _i, _i, _i, _i, _i, _vp,
@@ -2138,10 +2138,10 @@ class HipOps:
         return whole
 
     def attention_plan(self, seg_lens, seg_starts, retention, device, num_kv_heads=1, group_size=1, decode_bucket=None,
-                       tile=None):
+                       tile=None, single_tiles=False):
         """Work lists of the MFMA attention kernels for one step and one retention rule: the rows that are
-        single decode tokens (and into how many keys their work is split), tiles of up to 32 consecutive
-        tokens of longer segments and, with ``group_size`` > 1 query heads per kv head, the packing of the
+        single decode tokens (and into how many keys their work is split; ``single_tiles``: these are tiles too), tiles of up
+        to 32 consecutive tokens of longer segments and, with ``group_size`` > 1 query heads per kv head, the packing of the
         (tile, head) items of a kv head into blocks of wavefronts that share keys.  ``decode_bucket``: the step
         holds single tokens only, none beyond this context length: the split is then chosen from the number of
         tokens and this bound alone (not from where each request stands), so the same launch fits every such
@@ -2152,7 +2152,7 @@ class HipOps:
         tile = tile or self.PREFILL_TILE
         o = 0
         for i, n in enumerate(seg_lens):
-            if n == 1:
+            if n == 1 and not single_tiles:
                 dec.append(o)
                 if decode_bucket is None:
                     spans.append((first_needed_position(retention, seg_starts[i]), seg_starts[i]))
@@ -2370,24 +2370,21 @@ class HipOps:
         single = meta is not None and meta.decode_bucket is not None
         if (not single and q.dtype == torch.bfloat16 and hq // hk <= 32
                 and self._query("jle_attention_mfma_supported", dh, hq, hk, ps)):
-            # portions of prompts in bfloat16: the matrix-core kernel, a wavefront per (tile of 32 tokens, head),
-            # which takes the kept keys before a tile's window as a range of its own; a step of single tokens
-            # goes on below (a query's keys shared between wavefronts)
+            # portions of prompts in bfloat16: the matrix-core kernels, which take the kept keys before a tile's window as a
+            # range of their own: with heads of 128 that share kv heads the one whose wavefronts share keys, else a wavefront
+            # per (tile of 32 tokens, head); a step of single tokens goes on below (a query's keys shared between wavefronts)
             seg_lens, _ = self._segments(meta, token_segment, positions)
             if any(ln > 1 for ln in seg_lens):
-                tiles = meta.meta.get("kept_tiles") if meta is not None else None
-                if tiles is None:
-                    flat, o = [], 0
-                    for ln in seg_lens:
-                        for t in range(0, ln, self.PREFILL_TILE):
-                            flat += [o + t, min(self.PREFILL_TILE, ln - t)]
-                        o += ln
-                    tiles = to_device(torch.tensor(flat, dtype=torch.int32), q.device)
+                plan = meta.meta.get("kept_plan") if meta is not None else None
+                if plan is None:
+                    seg_lens, seg_starts = self._segments(meta, token_segment, positions)
+                    plan = self.attention_plan(seg_lens, seg_starts, ("window", param), q.device, hk, hq // hk if dh == 128 else 1,
+                                               single_tiles=True)
                     if meta is not None:
-                        meta.meta["kept_tiles"] = tiles
+                        meta.meta["kept_plan"] = plan
                 self._call("jle_attention_prefill_kept", _p(q), _p(kv_cache), _p(out), _p(positions),
-                           _p(token_segment), _p(block_table), block_table.shape[1], _p(tiles), tiles.numel() // 2,
-                           self.PREFILL_TILE, param, keep, float(scale), hq, hk, dh, ps)
+                           _p(token_segment), _p(block_table), block_table.shape[1], _p(plan["tiles"]), plan["num_tiles"],
+                           self.PREFILL_TILE, _p(plan["groups"]), plan["num_groups"], param, keep, float(scale), hq, hk, dh, ps)
                 return out
         splits, tiles_per_split, ws_ml, ws_o = 1, 0, None, None
         waves = n * hq

@@ -304,6 +304,39 @@ def test_paged_attention_of_long_portions_at_head_size_128(ops, ref, hq, hk, ps,
     _assert_close_to_scale(got, want, dt)
 
 
+@pytest.mark.parametrize("hq,hk,ps", [(10, 2, 16), (16, 8, 16), (9, 3, 48), (4, 2, 64), (3, 3, 16)])
+@pytest.mark.parametrize("window,keep", [(150, 5), (70, 64), (64, 65), (100, 200), (1, 1), (33, 0), (2000, 8)])
+def test_attention_with_kept_tokens_of_long_portions_at_head_size_128(ops, ref, monkeypatch, hq, hk, ps, window, keep):
+    """Kept keys in steps of their own before the window's, beside it and within it, kept ranges that end inside a step and
+    inside a page, portions that lie before, across and behind the window's first move, a single token between them.  Pages
+    that no query sees are given back, and what lies beside the visible keys of the others is poisoned."""
+    dt = torch.bfloat16
+    specs = [(0, 333), (190, 130), (517, 1), (64, 64), (1000, 35)]
+    q, kv, bt, pos, seg = _attention_case(hq, hk, 128, ps, dt, specs, seed=3)
+    want = ref.paged_attention(q, kv, bt, pos, seg, ("window_keep", window, keep), 128 ** -0.5)
+    plain = kv.clone()
+    for i, (a, b) in enumerate(specs):
+        first = max(0, a - window + 1)
+        for j in range(-(-(a + b) // ps)):
+            page = int(bt[i, j])
+            for o in range(ps):
+                if j * ps + o >= a + b or keep <= j * ps + o < first:
+                    kv[page, 0, :, o] = float("nan")
+                    kv[page, 1].view(hk, 128, ps)[:, :, o] = float("nan")  # (values lie transposed)
+            if keep <= j * ps and (j + 1) * ps <= first:
+                bt[i, j] = -1
+    calls = []
+    inner = ops._call
+    monkeypatch.setattr(ops, "_call", lambda name, *a: (calls.append(name), inner(name, *a))[1])
+    got = ops.paged_attention(q, kv, bt, pos, seg, ("window_keep", window, keep), 128 ** -0.5)
+    assert calls == ["jle_attention_prefill_kept"]
+    _assert_close_to_scale(got, want, dt)
+    if window == 2000:  # (nothing lies before the window: the plain kernel's bits)
+        alone = [ops.paged_attention(q[:333].contiguous(), plain, bt, pos[:333].contiguous(), seg[:333].contiguous(), r, 128 ** -0.5)
+                 for r in (("window_keep", window, keep), ("all",))]
+        assert hq == hk or torch.equal(*alone)
+
+
 class _Segments:
     """What the matrix-memory kernels read of a step."""
 
