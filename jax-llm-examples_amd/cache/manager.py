@@ -229,6 +229,7 @@ class CacheManager:
         for k, named in (run_states or {}).items():
             self.run_state[k] = {name: torch.zeros((max_requests, 2, *shape), dtype=dt or torch.float32,
                                                    device=self.device) for name, (shape, dt) in named.items()}
+        self._slot_rows: dict[int, list] = {}  # per slot: its rows of all state tensors, by type
         fill = float("nan") if poison else 0.0
         for g in self.groups:
             for cid in g.cache_ids:
@@ -248,12 +249,15 @@ class CacheManager:
         slot = self.slots.alloc()
         # The slot's state in all layers, a launch for each of their types (one for each tensor was seven a request of
         # Sudilorn's, 448 where 64 start together: 5 us of host time and 3 of the GPU's each).
-        fresh = {}
-        for named in (self.state, *self.run_state.values(), *self.named_state.values()):
-            for t in named.values():
-                fresh.setdefault(t.dtype, []).append(t[slot])
-        for rows in fresh.values():
-            torch._foreach_zero_(rows)
+        rows = self._slot_rows.get(slot)
+        if rows is None:
+            fresh = {}
+            for named in (self.state, *self.run_state.values(), *self.named_state.values()):
+                for t in named.values():
+                    fresh.setdefault(t.dtype, []).append(t[slot])
+            rows = self._slot_rows[slot] = list(fresh.values())
+        for same in rows:
+            torch._foreach_zero_(same)
         self._lives += 1
         e = RequestEntry(slot=slot, tables=[[] for _ in self.groups], versions=[0 for _ in self.groups],
                          serial=self._lives, freed_upto=[0 for _ in self.groups])
@@ -268,6 +272,8 @@ class CacheManager:
         table = e.tables[g.index]
         first = e.num_tokens // self.page_size
         last = (upto - 1) // self.page_size
+        if first >= len(table):
+            return list(range(first, last + 1))
         return [j for j in range(first, last + 1) if j >= len(table) or table[j] < 0]
 
     def pages_needed(self, rid, n_new: int) -> list[int]:
@@ -311,6 +317,9 @@ class CacheManager:
             got = g.pool.alloc(len(m))
             if got:
                 e.versions[g.index] += 1
+            if got and m[0] == len(table):  # (a run of new places at the table's end)
+                table += got
+                continue
             for j, p in zip(m, got):
                 while len(table) <= j:
                     table.append(-1)
@@ -361,7 +370,9 @@ class CacheManager:
     def free(self, rid) -> None:
         e = self.requests.pop(rid)
         for g in self.groups:
-            pages = [p for p in e.tables[g.index] if p >= 0]
+            pages = e.tables[g.index]
+            if -1 in pages:
+                pages = [p for p in pages if p >= 0]
             if pages:
                 self._release(g, pages)
         self.slots.release(e.slot)

@@ -33,21 +33,26 @@ class PagePool:
     def alloc(self, n: int) -> list[int]:
         if n > len(self._free):
             raise OutOfPages(f"asked for {n} pages, {len(self._free)} of {self.num_pages} free")
-        out = [self._free.pop() for _ in range(n)]
+        if n < 1:
+            return []
+        out = self._free[: -n - 1: -1]
+        del self._free[-n:]
         self.handed_out += n
+        held = self._held
+        if any(map(held.__getitem__, out)):
+            raise AssertionError(f"page {next(p for p in out if held[p])} handed out twice")
         for p in out:
-            if self._held[p]:
-                raise AssertionError(f"page {p} handed out twice")
-            self._held[p] = 1
+            held[p] = 1
         return out
 
     def release(self, pages) -> None:
+        held, num = self._held, self.num_pages
         for p in pages:
-            if not 0 <= p < self.num_pages:
+            if not 0 <= p < num:
                 raise AssertionError(f"page {p} does not belong to this pool")
-            if not self._held[p]:
+            if not held[p]:
                 raise AssertionError(f"page {p} given back twice")
-            self._held[p] = 0
+            held[p] = 0
             self._free.append(p)
 
     def check(self) -> None:

@@ -125,6 +125,7 @@ def fill_step(layout: StepLayout, flat: np.ndarray, cache, entries: Sequence[Ste
     tables = [v(f"block_table{g.index}") for g in cache.groups]
     maps = [v(f"slot_mapping{g.index}") for g in cache.groups]
     seg_lens, seg_starts = [], []
+    in_page = np.arange(ps, dtype=np.int32)
     o = w = 0
     cu[0] = 0
     for i, e in enumerate(entries):
@@ -140,7 +141,7 @@ def fill_step(layout: StepLayout, flat: np.ndarray, cache, entries: Sequence[Ste
             prev[o] = cache.last_token(e.rid)
         else:
             t = np.asarray(e.tokens, dtype=np.int64)
-            if t.min() < 0 or t.max() >= vocab_size:
+            if t.view(np.uint64).max() >= vocab_size:  # (a negative one is a very large one so)
                 raise ValueError(f"request {e.rid!r}: token id outside 0..{vocab_size - 1}")
             tok[o: o + n] = t
             prev[o] = cache.last_token(e.rid)
@@ -171,11 +172,12 @@ def fill_step(layout: StepLayout, flat: np.ndarray, cache, entries: Sequence[Ste
                     raise AssertionError(f"request {e.rid!r}: a new token has no page in group {g.index}")
                 sm[o] = page * ps + start % ps
             else:
-                p = pos[o: o + n]
-                pages = np.asarray(table, np.int64)[p // ps] if (start + n - 1) // ps < len(table) else np.array([-1])
-                if (pages < 0).any():
+                first, last = start // ps, (start + n - 1) // ps
+                pages = table[first: last + 1]
+                if len(pages) <= last - first or min(pages) < 0:
                     raise AssertionError(f"request {e.rid!r}: a new token has no page in group {g.index}")
-                sm[o: o + n] = pages * ps + p % ps
+                slots_of = np.add.outer(np.array(pages, np.int32) * np.int32(ps), in_page).reshape(-1)
+                sm[o: o + n] = slots_of[start - first * ps: start - first * ps + n]
         if stamps is not None:
             stamps[i] = stamp
         seg_lens.append(n)
