@@ -273,6 +273,92 @@ __global__ __launch_bounds__(1024) void moe_topk_align_kernel(const float* __res
   align_by_block(ids_s, gates_s, smem, smem + E, offsets, sorted_token, sorted_gate, inv, M, E, k, extra, k);
 }
 
+constexpr int kTokenExperts = 16;  // of norm_route_token_kernel
+
+// The grouping of up to 64 pairs by up to 63 experts by one wavefront: lane r has pair r's expert and gate.  What align_by_block
+// writes, without its barriers and trips through shared memory.
+__device__ __forceinline__ void align_by_wave(int id, float gate, int M, int E, int k, int extra, int inv_ld,
+                                              int* __restrict__ offsets, int* __restrict__ sorted_token,
+                                              float* __restrict__ sorted_gate, int* __restrict__ inv) {
+  const int lane = threadIdx.x & 63;
+  int pos = 0, off = 0;  // pairs that come before this lane's; pairs of experts below this lane's number
+  for (int i = 0; i < M; ++i) {
+    const int other = __builtin_amdgcn_readlane(id, i);
+    pos += (other < id || (other == id && i < lane)) ? 1 : 0;
+    off += other < lane ? 1 : 0;
+  }
+  const int total = __builtin_amdgcn_readlane(off, E);
+  if (lane <= E) offsets[lane] = off;
+  if (lane < M) {
+    const bool has_row = id < E;  // (an identity expert has none)
+    if (has_row) {
+      sorted_token[pos] = lane / k;
+      sorted_gate[pos] = gate;
+    }
+    inv[lane / k * inv_ld + lane % k] = has_row ? pos : -1;
+  }
+  if (extra > 0) {
+    if (lane == 0) offsets[E + 1] = total + extra;
+    if (lane < extra) {
+      sorted_token[total + lane] = lane;
+      sorted_gate[total + lane] = 1.0f;
+      if (inv_ld > k) inv[lane * inv_ld + k] = total + lane;
+    }
+  }
+}
+
+// The residual row n and what is added to it, normed: into shared memory (all threads of the block), and by the writer stored.
+template <typename DT, typename OT, int CPT>
+__device__ __forceinline__ void normed_row(const float* __restrict__ x, const Delta<DT>& delta, const float* __restrict__ w,
+                                           float eps, float* __restrict__ x_out, OT* __restrict__ h_out, size_t n, int D,
+                                           bool writer, float* row, float* red) {
+  constexpr int THREADS = 256;
+  f32x4_t wv[CPT];
+#pragma unroll
+  for (int i = 0; i < CPT; ++i) {
+    const int d = (threadIdx.x + THREADS * i) * 4;
+    wv[i] = (w != nullptr && d < D) ? load4<float>(w + d) : f32x4_t{1.f, 1.f, 1.f, 1.f};
+  }
+  f32x4_t v[CPT];
+  float ss = 0.f;
+  const bool add = delta.any();
+  const DeltaRow<DT> drow = delta_row(delta, n, D);
+#pragma unroll
+  for (int i = 0; i < CPT; ++i) {
+    const int d = (threadIdx.x + THREADS * i) * 4;
+    v[i] = d < D ? load4<float>(x + d) : f32x4_t{0.f, 0.f, 0.f, 0.f};
+  }
+  // (every load before the first store: see add_rmsnorm_vec_kernel)
+  if (add) {
+#pragma unroll
+    for (int i = 0; i < CPT; ++i) {
+      const int d = (threadIdx.x + THREADS * i) * 4;
+      v[i] += d < D ? delta_row_at4<false, DT>(delta, drow, n, d, D) : f32x4_t{0.f, 0.f, 0.f, 0.f};
+    }
+  }
+  if (writer) {
+#pragma unroll
+    for (int i = 0; i < CPT; ++i) {
+      const int d = (threadIdx.x + THREADS * i) * 4;
+      if (d < D) store4<float>(x_out + d, v[i]);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < CPT; ++i) ss = add_squares4(ss, v[i]);
+  const float tot = block_sum<THREADS>(ss, red);
+  const float rs = 1.0f / sqrtf(tot / (float)D + eps);
+#pragma unroll
+  for (int i = 0; i < CPT; ++i) {
+    const int d = (threadIdx.x + THREADS * i) * 4;
+    if (d < D) {
+      f32x4_t h = v[i] * rs;
+      if (w != nullptr) h *= wv[i];
+      *reinterpret_cast<f32x4_t*>(row + d) = h;
+      if (writer && h_out != nullptr) store4<OT>(h_out + d, h);
+    }
+  }
+}
+
 // Steps of few tokens: the addition of the pending branch output to the residual, the norm of the sum, the
 // router's logits, the choice of experts and the grouping of the choices, in one launch.  A block is (token,
 // four experts): it forms the token's normed row (every block of a token the same row, with the arithmetic of
@@ -302,50 +388,7 @@ __global__ __launch_bounds__(256) void norm_route_kernel(const float* __restrict
   const size_t n = blockIdx.x;
   const size_t base = n * D;
   const bool writer = blockIdx.y == 0;
-  f32x4_t wv[CPT];
-#pragma unroll
-  for (int i = 0; i < CPT; ++i) {
-    const int d = (threadIdx.x + THREADS * i) * 4;
-    wv[i] = (w != nullptr && d < D) ? load4<float>(w + d) : f32x4_t{1.f, 1.f, 1.f, 1.f};
-  }
-  f32x4_t v[CPT];
-  float ss = 0.f;
-  const bool add = delta.any();
-  const DeltaRow<DT> drow = delta_row(delta, n, D);
-#pragma unroll
-  for (int i = 0; i < CPT; ++i) {
-    const int d = (threadIdx.x + THREADS * i) * 4;
-    v[i] = d < D ? load4<float>(x + base + d) : f32x4_t{0.f, 0.f, 0.f, 0.f};
-  }
-  // (every load before the first store: see add_rmsnorm_vec_kernel)
-  if (add) {
-#pragma unroll
-    for (int i = 0; i < CPT; ++i) {
-      const int d = (threadIdx.x + THREADS * i) * 4;
-      v[i] += d < D ? delta_row_at4<false, DT>(delta, drow, n, d, D) : f32x4_t{0.f, 0.f, 0.f, 0.f};
-    }
-  }
-  if (writer) {
-#pragma unroll
-    for (int i = 0; i < CPT; ++i) {
-      const int d = (threadIdx.x + THREADS * i) * 4;
-      if (d < D) store4<float>(x_out + base + d, v[i]);
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < CPT; ++i) ss = add_squares4(ss, v[i]);
-  const float tot = block_sum<THREADS>(ss, red);
-  const float rs = 1.0f / sqrtf(tot / (float)D + eps);
-#pragma unroll
-  for (int i = 0; i < CPT; ++i) {
-    const int d = (threadIdx.x + THREADS * i) * 4;
-    if (d < D) {
-      f32x4_t h = v[i] * rs;
-      if (w != nullptr) h *= wv[i];
-      *reinterpret_cast<f32x4_t*>(row + d) = h;
-      if (writer && h_out != nullptr) store4<OT>(h_out + base + d, h);
-    }
-  }
+  normed_row<DT, OT, CPT>(x + base, delta, w, eps, x_out + base, h_out != nullptr ? h_out + base : nullptr, n, D, writer, row, red);
   __syncthreads();
   // one expert's logit per wavefront
   const int lane = threadIdx.x & 63;
@@ -453,6 +496,104 @@ __global__ __launch_bounds__(256) void norm_route_kernel(const float* __restrict
   }
   __syncthreads();
   align_by_block(ids_s, gates_s, ismem, ismem + E, offsets, sorted_token, sorted_gate, inv, M, E, k, extra, k);
+}
+
+// norm_route_kernel for choices by scores of up to 16 experts, up to 64 pairs of more than a few tokens: a block takes a token
+// with all its experts, EPW a wavefront, chooses from its own shared memory, and only the choices are handed to the block that
+// groups.  Where norm_route_kernel's time goes (16 tokens of 2,048, 10 experts, two by scores): row and addition 2.6 us, sum of
+// squares and row 0.9, logits 1.4, handed over 0.8, choice 10.3 (the last block alone, four tokens a wavefront one after the
+// other), grouping 1.8.  Here all tokens are chosen for at once, the router's first rows come while the token's row is added and
+// normed, and one wavefront groups in registers.  norm_route_kernel | this, us, 10 experts: 16 tokens of 2,048 19.0 | 13.5, 32
+// 30.0 | 15.0; 16 of 4,096 21.6 | 16.3; 8 of 3,072, 16 experts 17.2 | 14.4; 16 of 6,144, 8 experts 22.8 | 16.8; but a lone token,
+// whose experts are shared out over compute units there, 9.7 | 10.3, and 4 of 4,096, 16 experts 13.5 | 13.8.
+template <typename DT, typename OT, int CPT, int EPW>
+__global__ __launch_bounds__(256) void norm_route_token_kernel(const float* __restrict__ x, Delta<DT> delta,
+                                                               const float* __restrict__ w, float eps,
+                                                               float* __restrict__ x_out, OT* __restrict__ h_out,
+                                                               const float* __restrict__ router,
+                                                               float* __restrict__ logits, int* __restrict__ ids,
+                                                               float* __restrict__ gates, int* __restrict__ offsets,
+                                                               int* __restrict__ sorted_token,
+                                                               float* __restrict__ sorted_gate, int* __restrict__ inv,
+                                                               int* __restrict__ ticket, int N, int D, int E, int k,
+                                                               int extra, Choice choice, int experts) {
+  constexpr int U = 4;  // pieces of a router row a lane asks for at once
+  extern __shared__ int smem[];  // the normed row [D] (floats)
+  float* row = reinterpret_cast<float*>(smem);
+  __shared__ float red[4];
+  __shared__ float z[kTokenExperts], scores[kTokenExperts], choices[kTokenExperts];
+  const size_t n = blockIdx.x;
+  const int lane = threadIdx.x & 63, wave = wave_index();
+  const int D4 = D >> 2;
+  const float4* we[EPW];
+#pragma unroll
+  for (int j = 0; j < EPW; ++j) we[j] = reinterpret_cast<const float4*>(router + (size_t)min(wave + 4 * j, E - 1) * D);
+  float4 rv[U][EPW];
+  auto ask = [&](int c0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int j = 0; j < EPW; ++j) rv[u][j] = we[j][min(c0 + 64 * u, D4 - 1)];
+  };
+  ask(lane);
+  normed_row<DT, OT, CPT>(x + n * D, delta, w, eps, x_out + n * D, h_out != nullptr ? h_out + n * D : nullptr, n, D, true, row, red);
+  __syncthreads();
+  float acc[EPW];
+#pragma unroll
+  for (int j = 0; j < EPW; ++j) acc[j] = 0.f;
+  for (int c0 = lane; c0 - lane < D4; c0 += 64 * U) {  // (a lane's terms in the order of moe_logits_kernel)
+    float4 cur[U][EPW];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int j = 0; j < EPW; ++j) cur[u][j] = rv[u][j];
+    if (c0 - lane + 64 * U < D4) ask(c0 + 64 * U);
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int c = c0 + 64 * u;
+      if (c >= D4) continue;
+      const float4 h = *reinterpret_cast<const float4*>(row + 4 * c);
+#pragma unroll
+      for (int j = 0; j < EPW; ++j) {
+        acc[j] = __builtin_fmaf(h.x, cur[u][j].x, acc[j]);
+        acc[j] = __builtin_fmaf(h.y, cur[u][j].y, acc[j]);
+        acc[j] = __builtin_fmaf(h.z, cur[u][j].z, acc[j]);
+        acc[j] = __builtin_fmaf(h.w, cur[u][j].w, acc[j]);
+      }
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < EPW; ++j) {
+    const int e = wave + 4 * j;
+    const float v = wave_sum(acc[j]);
+    if (lane == 0 && e < E) {
+      z[e] = v;
+      logits[n * E + e] = v;
+    }
+  }
+  __syncthreads();
+  if (wave != 0) return;
+  int id = 0;  // lane r < k: the token's r-th choice
+  float gate = 0.f;
+  choose_by_wave<false>(z, choice, scores, choices, id, gate);
+  const int M = N * k;
+  // handed over as norm_route_kernel hands over its logits
+  if (lane < k) {
+    __hip_atomic_store(ids + n * k + lane, id, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    put_shared(gates + n * k + lane, gate);
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  int t = 0;
+  if (lane == 0) t = __hip_atomic_fetch_add(ticket, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (__builtin_amdgcn_readfirstlane(t) != N - 1) return;
+  if (lane == 0) __hip_atomic_store(ticket, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  if (lane < M) {
+    id = __hip_atomic_load(ids + lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    gate = get_shared(gates + lane);
+  }
+  align_by_wave(id, gate, M, experts, k, extra, extra > 0 ? k + 1 : k, offsets, sorted_token, sorted_gate, inv);
 }
 
 static int launch_logits(const float* h, const float* w, float* logits, int N, int D, int E, hipStream_t s) {
@@ -580,6 +721,18 @@ JLE_API int jle_norm_route(const float* x, int delta_kind, const void* delta, co
   hipLaunchKernelGGL((norm_route_kernel<DT, OT, SCORED, CPT>), g, b, lds, s, x, dl, w, eps, x_out, (OT*)h_out,   \
                      router, logits, ids, gates, offsets, sorted_token, sorted_gate, inv, ticket, N, D, E, k,    \
                      extra_group ? N : 0, choice, experts)
+  // (the same bits: which of the two is a question of time alone)
+  const bool by_token = scored && E <= kTokenExperts && N > 4 && N * k <= 64;
+#define LAUNCH_T(DT, OT, CPT, EPW)                                                                               \
+  hipLaunchKernelGGL((norm_route_token_kernel<DT, OT, CPT, EPW>), dim3(N), b, D * sizeof(float), s, x, dl, w, eps, x_out, \
+                     (OT*)h_out, router, logits, ids, gates, offsets, sorted_token, sorted_gate, inv, ticket, N, D, E, k, \
+                     extra_group ? N : 0, choice, experts)
+#define TOKEN_BY_WIDTH(DT, OT, EPW)                                                                              \
+  do {                                                                                                           \
+    if (D <= 2048) LAUNCH_T(DT, OT, 2, EPW);                                                                     \
+    else if (D <= 4096) LAUNCH_T(DT, OT, 4, EPW);                                                                \
+    else LAUNCH_T(DT, OT, 8, EPW);                                                                               \
+  } while (0)
 #define BY_WIDTH(DT, OT, SCORED)                                                                                 \
   do {                                                                                                           \
     if (D <= 2048) LAUNCH(DT, OT, SCORED, 2);                                                                    \
@@ -592,7 +745,9 @@ JLE_API int jle_norm_route(const float* x, int delta_kind, const void* delta, co
     Delta<DT> dl = {delta_kind == 1 ? (const DT*)delta : nullptr,                                                \
                     delta_kind == 2 ? (const DT*)routed : nullptr, inv_in, (const DT*)shared, k_in,              \
                     (const DT*)self, self_w, self_k};                                                            \
-    if (scored) BY_WIDTH(DT, OT, true);                                                                          \
+    if (by_token && E <= 8) TOKEN_BY_WIDTH(DT, OT, 2);                                                           \
+    else if (by_token) TOKEN_BY_WIDTH(DT, OT, 4);                                                                \
+    else if (scored) BY_WIDTH(DT, OT, true);                                                                     \
     else BY_WIDTH(DT, OT, false);                                                                                \
   } while (0)
   if (delta_is_bf16) {
@@ -602,6 +757,8 @@ JLE_API int jle_norm_route(const float* x, int delta_kind, const void* delta, co
   }
 #undef GO
 #undef BY_WIDTH
+#undef TOKEN_BY_WIDTH
+#undef LAUNCH_T
 #undef LAUNCH
   JLE_LAUNCH_CHECK();
   return 0;

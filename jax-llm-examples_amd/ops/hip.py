@@ -2430,7 +2430,8 @@ class HipOps:
         how = (0 if groups is None else int(groups), 0 if groups is None else int(keep_groups), int(group_terms),
                1 if scores == "softmax" else 0, -1.0 if normalize is None else float(normalize), float(weight_scale))
         if isinstance(h32, PendingNorm):
-            fused = None if h32.done or hasattr(h32.delta, "terms") or n > self.NORM_CHOOSE_ROWS else \
+            most = self.NORM_CHOOSE_TOKENS // top_k if e <= self.NORM_CHOOSE_EXPERTS else self.NORM_CHOOSE_ROWS
+            fused = None if h32.done or hasattr(h32.delta, "terms") or n > max(most, self.NORM_CHOOSE_ROWS) else \
                 self._norm_route(h32, router, top_k, scored=(experts, correction, how, extra_group))
             if fused is not None:
                 ids, weights, _, grouping = fused
@@ -2455,7 +2456,9 @@ class HipOps:
         return ids, weights, self.moe_align(ids, weights, experts, extra_group=extra_group, note_extra=extra_group)
 
     NORM_CHOOSE_ROWS = 16  # up to here the choice by scores is made in the launch that norms the rows (whose last block
-    # chooses for all tokens: 17 us at 8 tokens, 52 at 64, where the separate launches take 22)
+    # chooses for all tokens: 17 us at 8 tokens, 52 at 64, where the separate launches take 22); of up to 16 experts and 64
+    # choices every token's own block chooses (15 us at 32 tokens)
+    NORM_CHOOSE_EXPERTS, NORM_CHOOSE_TOKENS = 16, 64
 
     @staticmethod
     def _grouping_arrays(n: int, k: int, experts: int, extra: bool, dev):

@@ -337,6 +337,42 @@ def test_attention_with_kept_tokens_of_long_portions_at_head_size_128(ops, ref, 
         assert hq == hk or torch.equal(*alone)
 
 
+@pytest.mark.parametrize("n,d,e,k,experts,groups", [
+    (5, 1032, 2, 1, 2, None), (5, 2048, 10, 2, 8, (5, 3)), (8, 2056, 16, 8, 16, (4, 2)), (16, 2048, 9, 4, 8, None),
+    (17, 4096, 16, 3, 12, (8, 5)), (32, 2048, 10, 2, 8, (5, 3)), (64, 8192, 8, 1, 8, None), (64, 4104, 16, 1, 16, (2, 1))])
+@pytest.mark.parametrize("extra", [False, True])
+def test_choices_by_scores_token_by_token_equal_the_separate_kernels(ops, n, d, e, k, experts, groups, extra):
+    """A block a token with all its experts (up to 16, up to 64 choices): the bits of norm, logits, choice and grouping as
+    launches of their own, launch after launch, with equal scores, a token that is not finite and identity experts."""
+    x, w, router = _rand(n, d, seed=1), _rand(d, seed=2) + 1.0, _rand(e, d, scale=0.05, seed=3)
+    router[e - 1] = router[0]
+    delta = _rand(n, d, dt=torch.bfloat16, seed=4)
+    x[n - 1, 3] = float("inf")
+    correction = _rand(e, scale=0.1, seed=5)
+    g, keep = groups or (None, None)
+    calls = []
+    inner = ops._call
+    for scores in ("sigmoid", "softmax"):
+        args = dict(groups=g, keep_groups=keep, group_terms=1, scores=scores, normalize=1e-20 if extra else None, weight_scale=1.5,
+                    num_experts=experts, extra_group=extra)
+        for _ in range(2):
+            ops._call = lambda name, *a: (calls.append(name), inner(name, *a))[1]
+            pending = ops.defer_norm(x.clone(), delta, w, 1e-5, torch.bfloat16)
+            ids, weights, grouping = ops.moe_choose(pending, router, correction, k, **args)
+            del ops._call
+            assert calls[-1] == "jle_norm_route"
+            h, h32 = ops.add_rmsnorm(x.clone(), delta, w, 1e-5, torch.bfloat16, want32=True)
+            want = ops.moe_choose(h32, router, correction, k, **args)
+            ok = torch.arange(n, device=DEV) < n - 1  # (the last token's numbers are NaN: any order will do, its rows exist)
+            assert torch.equal(ids[ok], want[0][ok]) and torch.equal(weights[ok], want[1][ok])
+            assert torch.equal(pending.rows()[ok], h[ok]) and bool(((ids >= 0) & (ids < e)).all())
+            off, tok, gate, inv = (t.cpu() for t in grouping)
+            again = [t.cpu() for t in ops.moe_align(ids, weights, experts, extra_group=len(off) == experts + 2, note_extra=True)]
+            rows = int(again[0][-1])  # (behind them nothing is written: identity experts)
+            assert torch.equal(off, again[0]) and torch.equal(inv, again[3]) and torch.equal(tok[:rows], again[1][:rows])
+            assert torch.equal(gate[:rows].view(torch.int32), again[2][:rows].view(torch.int32))
+
+
 class _Segments:
     """What the matrix-memory kernels read of a step."""
 
