@@ -8,6 +8,11 @@
 //   scores: one key per lane (the lane reads its key's row; q is read at a wave-uniform address)
 //   softmax: running maximum and sum across tiles, float32
 //   values: one head element per lane (+64, +128, +192), probabilities broadcast by shuffle
+// bfloat16 with 64 or 128 elements a head and pages of whole sixteens of keys (DH): the same sums in the same order, but a
+// tile's keys and values are all asked for before the first is used.  A wavefront has a tile or a few, so the kernel is a
+// chain of trips to memory: 64 single tokens of about 90 keys, 16 heads on 8 kv heads of 128, two wavefronts a query, 24.2 ->
+// 15.2 us (of which the code, fetched once by every compute unit, is a part).  Other sizes and float32 keep the loops: with
+// a length known at run time only, the loads cannot be laid out in registers.
 // Page layout per kv head: keys [page_size][head_dim], values [head_dim][page_size].
 #include "common.h"
 
@@ -39,8 +44,18 @@ __device__ __forceinline__ int retention_first_key(int mode, int param, int pos)
   return 0;
 }
 
-template <typename T>
-__global__ __launch_bounds__(256) void paged_attention_generic_kernel(
+// A key's score beyond the product: the cap, then a learned number per head and distance; every key further back than the
+// table is long takes its last entry (a negative length: a penalty that grows with the distance, two numbers per head)
+__device__ __forceinline__ float adjusted(float s, float cap, const float* __restrict__ bias, int bias_len, int h, int back) {
+  if (cap > 0.f) s = cap * tanhf(s / cap);
+  if (bias_len < 0) s -= bias[2 * h] * log1pf(bias[2 * h + 1] * (float)back);
+  else if (bias != nullptr) s += bias[(size_t)h * bias_len + min(back, bias_len - 1)];
+  return s;
+}
+
+// DH > 0: bfloat16 with dh == DH and ps % 16 == 0.
+template <typename T, int DH>
+__global__ __launch_bounds__(256, DH > 0 ? 2 : 1) void paged_attention_generic_kernel(
     const T* __restrict__ q, const T* __restrict__ kv, T* __restrict__ out, const int* __restrict__ positions,
     const int* __restrict__ token_segment, const int* __restrict__ block_table, int table_width, int ret_mode,
     int ret_param, float scale, int N, int Hq, int Hkv, int dh, int ps, int splits, int tiles_per_split,
@@ -80,6 +95,64 @@ __global__ __launch_bounds__(256) void paged_attention_generic_kernel(
   const int r_lo = range == 0 ? 0 : t_lo, r_hi = range == 0 ? r_last : t_hi;
   for (int t0 = r_lo; t0 <= r_hi; t0 += 64) {
     const int key = t0 + lane;
+    if constexpr (DH > 0) {
+      static_assert(sizeof(T) == 2 && DH % 64 == 0, "a lane has DH / 64 elements of a head's values");
+      constexpr int KV = DH / 8, E = DH / 64;
+      // (lanes without a key of their own read the nearest visible one: no branch stands between the loads)
+      const int lo = max(r_first - t0, 0), last = min(r_last - t0, 63);
+      const int mine = min(max(lane, lo), last);
+      const int page = table[(t0 + mine) / ps], slot = (t0 + mine) % ps;
+      if (__any(page < 0)) {  // a visible key's page is missing: the result is NaN whatever else is read
+        bad = true;
+        break;
+      }
+      const T* krow = kv + (size_t)page * page_stride + head_off + (size_t)slot * DH;
+      Vec16<T> k[KV], v[4][E][2];
+#pragma unroll
+      for (int c = 0; c < KV; ++c) k[c].load(krow + 8 * c);
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {  // sixteen keys' values a lane and element; groups without a visible key: the nearest one's
+        const int at = min(max(c, lo / 16), last / 16) * 16, who = max(at, lo);
+        const T* vplane = kv + (size_t)__builtin_amdgcn_readlane(page, who) * page_stride + head_off + v_off +
+                          __builtin_amdgcn_readlane(slot, who) / 16 * 16 + (size_t)lane * ps;
+#pragma unroll
+        for (int i = 0; i < E; ++i) {
+          v[c][i][0].load(vplane + (size_t)64 * i * ps);
+          v[c][i][1].load(vplane + (size_t)64 * i * ps + 8);
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);  // every load is on its way before the first is waited for
+      float dot = 0.f;
+#pragma unroll
+      for (int c = 0; c < KV; ++c) {
+        Vec16<T> qv;
+        qv.load(qrow + 8 * c);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) dot += qv.get(i) * k[c].get(i);
+      }
+      float s = adjusted(dot * scale, cap, bias, bias_len, h, pos - t0 - mine);
+      s = mine == lane ? s : -INFINITY;
+      const float m_new = fmaxf(m, wave_max(s));
+      const float corr = expf(m - m_new);  // first tile: exp(-inf) = 0
+      const float p = (s == -INFINITY) ? 0.f : expf(s - m_new);
+      l = l * corr + wave_sum(p);
+      m = m_new;
+#pragma unroll
+      for (int i = 0; i < E; ++i) acc[i] *= corr;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        if (c * 16 > last || c * 16 + 15 < lo) continue;
+#pragma unroll
+        for (int kk = 0; kk < 16; ++kk) {
+          const int at = 16 * c + kk;
+          const float pk = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(p), at));
+          const bool seen = at >= lo && at <= last;  // (slots that no visible key fills may hold anything)
+#pragma unroll
+          for (int i = 0; i < E; ++i) acc[i] += pk * (seen ? v[c][i][kk / 8].get(kk % 8) : 0.f);
+        }
+      }
+      continue;
+    }
     const bool valid = key >= r_first && key <= r_last;
     float s = -INFINITY;
     const T* krow = nullptr;
@@ -99,12 +172,7 @@ __global__ __launch_bounds__(256) void paged_attention_generic_kernel(
 #pragma unroll
           for (int i = 0; i < Vec16<T>::kN; ++i) dot += qv.get(i) * kvv.get(i);
         }
-        s = dot * scale;
-        if (cap > 0.f) s = cap * tanhf(s / cap);
-        // a learned number per head and distance; every key further back than the table is long takes its last entry
-        // (a negative length: a penalty that grows with the distance, two numbers per head)
-        if (bias_len < 0) s -= bias[2 * h] * log1pf(bias[2 * h + 1] * (float)(pos - key));
-        else if (bias != nullptr) s += bias[(size_t)h * bias_len + min(pos - key, bias_len - 1)];
+        s = adjusted(dot * scale, cap, bias, bias_len, h, pos - key);
       }
     }
     const float m_new = fmaxf(m, wave_max(s));
@@ -271,25 +339,23 @@ static int launch_generic(const void* q, const void* kv, void* out, const int* p
   if (items > (1ll << 31) - 8) return JLE_BAD_ARG;
   dim3 g((unsigned)((items + 3) / 4)), b(256);
   dim3 gm((unsigned)(((long long)N * Hq + 3) / 4));
-  if (is_bf16) {
-    hipLaunchKernelGGL(paged_attention_generic_kernel<bf16_t>, g, b, 0, s, (const bf16_t*)q, (const bf16_t*)kv,
-                       (bf16_t*)out, positions, token_segment, block_table, table_width, ret_mode, ret_param, scale,
-                       N, Hq, Hkv, dh, ps, splits, tiles_per_split, ws_ml, ws_o, bias, bias_len, sink, keep,
-                       cap);
-    JLE_LAUNCH_CHECK();
-    if (splits > 1)
-      hipLaunchKernelGGL(paged_attention_generic_merge_kernel<bf16_t>, gm, b, 0, s, ws_ml, ws_o, (bf16_t*)out, N * Hq,
-                         dh, splits, sink, Hq);
-  } else {
-    hipLaunchKernelGGL(paged_attention_generic_kernel<float>, g, b, 0, s, (const float*)q, (const float*)kv,
-                       (float*)out, positions, token_segment, block_table, table_width, ret_mode, ret_param, scale, N,
-                       Hq, Hkv, dh, ps, splits, tiles_per_split, ws_ml, ws_o, bias, bias_len, sink, keep,
-                       cap);
-    JLE_LAUNCH_CHECK();
-    if (splits > 1)
-      hipLaunchKernelGGL(paged_attention_generic_merge_kernel<float>, gm, b, 0, s, ws_ml, ws_o, (float*)out, N * Hq, dh,
-                         splits, sink, Hq);
-  }
+  const bool ahead = is_bf16 && ps % 16 == 0 && ((uintptr_t)q | (uintptr_t)kv) % 16 == 0;
+#define GO(T_, DH_)                                                                                                          \
+  hipLaunchKernelGGL((paged_attention_generic_kernel<T_, DH_>), g, b, 0, s, (const T_*)q, (const T_*)kv, (T_*)out, positions, \
+                     token_segment, block_table, table_width, ret_mode, ret_param, scale, N, Hq, Hkv, dh, ps, splits,        \
+                     tiles_per_split, ws_ml, ws_o, bias, bias_len, sink, keep, cap)
+  if (!is_bf16) GO(float, 0);
+  else if (ahead && dh == 128) GO(bf16_t, 128);
+  else if (ahead && dh == 64) GO(bf16_t, 64);
+  else GO(bf16_t, 0);
+#undef GO
+  JLE_LAUNCH_CHECK();
+  if (splits > 1 && is_bf16)
+    hipLaunchKernelGGL(paged_attention_generic_merge_kernel<bf16_t>, gm, b, 0, s, ws_ml, ws_o, (bf16_t*)out, N * Hq, dh,
+                       splits, sink, Hq);
+  else if (splits > 1)
+    hipLaunchKernelGGL(paged_attention_generic_merge_kernel<float>, gm, b, 0, s, ws_ml, ws_o, (float*)out, N * Hq, dh,
+                       splits, sink, Hq);
   JLE_LAUNCH_CHECK();
   return 0;
 }

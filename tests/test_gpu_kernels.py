@@ -304,6 +304,40 @@ def test_paged_attention_of_long_portions_at_head_size_128(ops, ref, hq, hk, ps,
     _assert_close_to_scale(got, want, dt)
 
 
+@pytest.mark.parametrize("hq,hk,dh,ps", [(10, 2, 128, 16), (16, 8, 128, 48), (3, 3, 64, 16), (4, 2, 64, 64), (6, 3, 64, 8)])
+@pytest.mark.parametrize("window,keep", [(150, 5), (70, 64), (64, 65), (1, 1), (33, 0), (2000, 8)])
+@pytest.mark.parametrize("shared", [0, 1 << 20])
+def test_single_tokens_with_kept_ones_at_the_edges_of_tiles(ops, ref, monkeypatch, hq, hk, dh, ps, window, keep, shared):
+    """Whole tiles' loads asked for ahead (64 and 128 elements, pages of sixteens; another page size for the other form): last
+    keys at the edges of sixteens, tiles and pages, windows and kept ranges that begin and end inside them, a query's keys in
+    one wavefront and shared.  Slots that no query sees are poisoned, pages of nothing else are given back, and a token whose
+    own page is missing gets NaN."""
+    monkeypatch.setattr(type(ops), "GENERIC_SPLIT_BELOW", shared)
+    dt = torch.bfloat16
+    ends = [0, 1, 15, 16, 31, 47, 48, 63, 64, 65, 127, 128, 191, 250, 600]
+    q, kv, bt, pos, seg = _attention_case(hq, hk, dh, ps, dt, [(a, 1) for a in ends], seed=5)
+    want = ref.paged_attention(q, kv, bt, pos, seg, ("window_keep", window, keep), dh ** -0.5)
+    for i, a in enumerate(ends):
+        first = max(0, a - window + 1)
+        for j in range(-(-(a + 1) // ps)):
+            page = int(bt[i, j])
+            for o in range(ps):
+                if j * ps + o > a or keep <= j * ps + o < first:
+                    kv[page, 0].view(hk, ps, dh)[:, o] = float("nan")
+                    kv[page, 1].view(hk, dh, ps)[:, :, o] = float("nan")  # (values lie transposed)
+            if keep <= j * ps and (j + 1) * ps <= first:
+                bt[i, j] = -1
+    calls = []
+    inner = ops._call
+    monkeypatch.setattr(ops, "_call", lambda name, *a: (calls.append(name), inner(name, *a))[1])
+    got = ops.paged_attention(q, kv, bt, pos, seg, ("window_keep", window, keep), dh ** -0.5)
+    assert calls == ["jle_paged_attention_kept"]
+    _assert_close_to_scale(got, want, dt)
+    bt[-1, 600 // ps] = -1
+    gone = ops.paged_attention(q, kv, bt, pos, seg, ("window_keep", window, keep), dh ** -0.5)
+    assert torch.isnan(gone[-1]).all() and torch.equal(gone[:-1], got[:-1])
+
+
 @pytest.mark.parametrize("hq,hk,ps", [(10, 2, 16), (16, 8, 16), (9, 3, 48), (4, 2, 64), (3, 3, 16)])
 @pytest.mark.parametrize("window,keep", [(150, 5), (70, 64), (64, 65), (100, 200), (1, 1), (33, 0), (2000, 8)])
 def test_attention_with_kept_tokens_of_long_portions_at_head_size_128(ops, ref, monkeypatch, hq, hk, ps, window, keep):
