@@ -39,9 +39,9 @@ class PagePool:
         del self._free[-n:]
         self.handed_out += n
         held = self._held
-        if any(map(held.__getitem__, out)):
-            raise AssertionError(f"page {next(p for p in out if held[p])} handed out twice")
         for p in out:
+            if held[p]:
+                raise AssertionError(f"page {p} handed out twice")
             held[p] = 1
         return out
 
