@@ -273,37 +273,112 @@ __global__ __launch_bounds__(1024) void moe_topk_align_kernel(const float* __res
   align_by_block(ids_s, gates_s, smem, smem + E, offsets, sorted_token, sorted_gate, inv, M, E, k, extra, k);
 }
 
-constexpr int kTokenExperts = 16;  // of norm_route_token_kernel
+constexpr int kTokenExperts = 16;  // of the kernels whose block takes a token with all its experts
 
-// The grouping of up to 64 pairs by up to 63 experts by one wavefront: lane r has pair r's expert and gate.  What align_by_block
-// writes, without its barriers and trips through shared memory.
-__device__ __forceinline__ void align_by_wave(int id, float gate, int M, int E, int k, int extra, int inv_ld,
-                                              int* __restrict__ offsets, int* __restrict__ sorted_token,
+// The grouping of up to 64 R pairs by up to 63 experts by one wavefront: lane l has the experts and gates of the pairs l, l + 64,
+// ...  What align_by_block writes, without its barriers and trips through shared memory.
+template <int R>
+__device__ __forceinline__ void align_by_wave(const int (&id)[R], const float (&gate)[R], int M, int E, int k, int extra,
+                                              int inv_ld, int* __restrict__ offsets, int* __restrict__ sorted_token,
                                               float* __restrict__ sorted_gate, int* __restrict__ inv) {
   const int lane = threadIdx.x & 63;
-  int pos = 0, off = 0;  // pairs that come before this lane's; pairs of experts below this lane's number
-  for (int i = 0; i < M; ++i) {
-    const int other = __builtin_amdgcn_readlane(id, i);
-    pos += (other < id || (other == id && i < lane)) ? 1 : 0;
-    off += other < lane ? 1 : 0;
-  }
-  const int total = __builtin_amdgcn_readlane(off, E);
-  if (lane <= E) offsets[lane] = off;
-  if (lane < M) {
-    const bool has_row = id < E;  // (an identity expert has none)
-    if (has_row) {
-      sorted_token[pos] = lane / k;
-      sorted_gate[pos] = gate;
+  int pos[R], off = 0, run = 0;
+#pragma unroll
+  for (int r = 0; r < R; ++r) pos[r] = -1;  // (an identity expert's pair has no row)
+  for (int e = 0; e < E; ++e) {
+    if (lane == e) off = run;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const bool match = id[r] == e && lane + 64 * r < M;
+      const unsigned long long bal = __ballot(match);
+      if (match) pos[r] = run + __popcll(bal & ((1ull << lane) - 1ull));
+      run += __popcll(bal);
     }
-    inv[lane / k * inv_ld + lane % k] = has_row ? pos : -1;
+  }
+  if (lane < E) offsets[lane] = off;
+  if (lane == 0) offsets[E] = run;
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int pair = lane + 64 * r;
+    if (pair >= M) continue;
+    inv[pair / k * inv_ld + pair % k] = pos[r];
+    if (pos[r] < 0) continue;
+    sorted_token[pos[r]] = pair / k;
+    sorted_gate[pos[r]] = gate[r];
   }
   if (extra > 0) {
-    if (lane == 0) offsets[E + 1] = total + extra;
-    if (lane < extra) {
-      sorted_token[total + lane] = lane;
-      sorted_gate[total + lane] = 1.0f;
-      if (inv_ld > k) inv[lane * inv_ld + k] = total + lane;
+    if (lane == 0) offsets[E + 1] = run + extra;
+    for (int t = lane; t < extra; t += 64) {
+      sorted_token[run + t] = t;
+      sorted_gate[run + t] = 1.0f;
+      if (inv_ld > k) inv[t * inv_ld + k] = run + t;
     }
+  }
+}
+
+// The same as a launch of its own, for few pairs that lie in memory: 128 pairs of 8 experts 5.6 us
+// in moe_align_kernel, whose thousand threads meet at eight barriers, about 3 so.
+template <int R>
+__global__ __launch_bounds__(64) void moe_align_wave_kernel(const int* __restrict__ ids, const float* __restrict__ gates,
+                                                            int* __restrict__ offsets, int* __restrict__ sorted_token,
+                                                            float* __restrict__ sorted_gate, int* __restrict__ inv, int M,
+                                                            int E, int k, int extra, int inv_ld) {
+  int id[R];
+  float gate[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int pair = min((int)threadIdx.x + 64 * r, M - 1);
+    id[r] = ids[pair];
+    gate[r] = gates[pair];
+  }
+  align_by_wave(id, gate, M, E, k, extra, inv_ld, offsets, sorted_token, sorted_gate, inv);
+}
+
+// The router and the choice by scores of up to 16 experts, a block a token, a wavefront an expert (its sum in the order of
+// moe_logits_kernel: the same bits).  Launches of their own, 4.6 and 4.8 us for 64 tokens, are mostly their start and end.  With
+// the grouping behind it, before | so, us: 8 experts of 2,048, two a token: 17 tokens 9.0 | 7.0, 64 9.2 | 7.3, 256 10.9 | 9.2; 10 of
+// 4,096: 64 10.4 | 8.7, 256 12.7 | 10.9.
+template <int WAVES>
+__global__ __launch_bounds__(WAVES * 64) void moe_logits_choose_kernel(const float* __restrict__ h,
+                                                                       const float* __restrict__ router, int* __restrict__ ids,
+                                                                       float* __restrict__ weights, int D, Choice choice) {
+  constexpr int U = 8;  // pieces of a row a lane asks for at once
+  __shared__ float z[kTokenExperts], scores[kTokenExperts], choices[kTokenExperts];
+  const size_t n = blockIdx.x;
+  const int lane = threadIdx.x & 63, wave = wave_index();
+  const int D4 = D >> 2;
+  if (wave < choice.E) {
+    const float4* x = reinterpret_cast<const float4*>(h + n * D);
+    const float4* w = reinterpret_cast<const float4*>(router + (size_t)wave * D);
+    float acc = 0.f;
+    for (int c0 = lane; c0 - lane < D4; c0 += 64 * U) {
+      float4 xv[U], wv[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int c = min(c0 + 64 * u, D4 - 1);
+        xv[u] = x[c];
+        wv[u] = w[c];
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        if (c0 + 64 * u >= D4) continue;
+        acc = __builtin_fmaf(xv[u].x, wv[u].x, acc);
+        acc = __builtin_fmaf(xv[u].y, wv[u].y, acc);
+        acc = __builtin_fmaf(xv[u].z, wv[u].z, acc);
+        acc = __builtin_fmaf(xv[u].w, wv[u].w, acc);
+      }
+    }
+    acc = wave_sum(acc);
+    if (lane == 0) z[wave] = acc;
+  }
+  __syncthreads();
+  if (wave != 0) return;
+  int id;
+  float weight;
+  choose_by_wave<false>(z, choice, scores, choices, id, weight);
+  if (lane < choice.top_k) {
+    ids[n * choice.top_k + lane] = id;
+    weights[n * choice.top_k + lane] = weight;
   }
 }
 
@@ -573,14 +648,14 @@ __global__ __launch_bounds__(256) void norm_route_token_kernel(const float* __re
   }
   __syncthreads();
   if (wave != 0) return;
-  int id = 0;  // lane r < k: the token's r-th choice
-  float gate = 0.f;
-  choose_by_wave<false>(z, choice, scores, choices, id, gate);
+  int id[1];  // lane r < k: the token's r-th choice
+  float gate[1];
+  choose_by_wave<false>(z, choice, scores, choices, id[0], gate[0]);
   const int M = N * k;
   // handed over as norm_route_kernel hands over its logits
   if (lane < k) {
-    __hip_atomic_store(ids + n * k + lane, id, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    put_shared(gates + n * k + lane, gate);
+    __hip_atomic_store(ids + n * k + lane, id[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    put_shared(gates + n * k + lane, gate[0]);
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -590,8 +665,8 @@ __global__ __launch_bounds__(256) void norm_route_token_kernel(const float* __re
   if (lane == 0) __hip_atomic_store(ticket, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   if (lane < M) {
-    id = __hip_atomic_load(ids + lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    gate = get_shared(gates + lane);
+    id[0] = __hip_atomic_load(ids + lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    gate[0] = get_shared(gates + lane);
   }
   align_by_wave(id, gate, M, experts, k, extra, extra > 0 ? k + 1 : k, offsets, sorted_token, sorted_gate, inv);
 }
@@ -634,6 +709,17 @@ static int launch_logits(const float* h, const float* w, float* logits, int N, i
 
 static int launch_align(const int* ids, const float* gates, int* offsets, int* sorted_token, float* sorted_gate,
                         int* inv, int M, int E, int k, int extra, int inv_ld, hipStream_t s) {
+  if (M <= 256 && E <= 63) {
+#define WAVE(R_) \
+  hipLaunchKernelGGL(moe_align_wave_kernel<R_>, dim3(1), dim3(64), 0, s, ids, gates, offsets, sorted_token, sorted_gate, inv, M, E, \
+                     k, extra, inv_ld)
+    if (M <= 64) WAVE(1);
+    else if (M <= 128) WAVE(2);
+    else WAVE(4);
+#undef WAVE
+    JLE_LAUNCH_CHECK();
+    return 0;
+  }
   // (shared memory: 64 KB; the pieces take what the experts' counters leave, at most 2,048 pairs)
   int piece = (16384 - (3 * E + 1)) / 2;
   piece = piece > 2048 ? 2048 : piece / 64 * 64;
@@ -660,6 +746,20 @@ JLE_API int jle_moe_logits(const float* h, const float* w, float* logits, int N,
   if (N <= 0) return 0;
   if (E < 1 || E > 4096 || logits == nullptr) return JLE_BAD_ARG;
   return launch_logits(h, w, logits, N, D, E, s);
+}
+
+// The router of up to 16 experts and the choice by scores (the same results as jle_moe_logits, then jle_moe_choose).
+JLE_API int jle_moe_logits_choose(const float* h, const float* w, const float* correction, int* ids, float* weights, int N, int D,
+                                  int E, int top_k, int groups, int keep, int terms, int softmax, float floor_, float scale,
+                                  hipStream_t s) {
+  if (N <= 0) return 0;
+  const Choice a = {correction, E, top_k, groups, keep, terms, softmax, floor_, scale};
+  if (!choice_ok(a) || E > kTokenExperts || D <= 0 || D % 4 || (((uintptr_t)h | (uintptr_t)w) & 15) != 0) return JLE_BAD_ARG;
+  if (E <= 4) hipLaunchKernelGGL(moe_logits_choose_kernel<4>, dim3(N), dim3(256), 0, s, h, w, ids, weights, D, a);
+  else if (E <= 8) hipLaunchKernelGGL(moe_logits_choose_kernel<8>, dim3(N), dim3(512), 0, s, h, w, ids, weights, D, a);
+  else hipLaunchKernelGGL(moe_logits_choose_kernel<16>, dim3(N), dim3(1024), 0, s, h, w, ids, weights, D, a);
+  JLE_LAUNCH_CHECK();
+  return 0;
 }
 
 // The router and the grouping of its choices in one call (the same results as jle_moe_route, then jle_moe_align).

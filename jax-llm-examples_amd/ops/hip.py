@@ -114,6 +114,7 @@ _SIGNATURES = {
                         _i, _i, _i, _i, _f, _f, _vp, _i, _vp, _i, _i, _i, _vp, _vp],
     "jle_gated_delta_single": [_vp, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _f, _f, _vp],
     "jle_moe_choose": [_vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _f, _f, _i, _vp, _vp, _vp, _vp, _i, _i, _vp],
+    "jle_moe_logits_choose": [_vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _i, _f, _f, _vp],
     "jle_moe_choose_groups": [_i, _i, _i, _i],
     "jle_mamba2": [_vp, _i, _vp, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _f, _i,
                    _vp],
@@ -2442,6 +2443,11 @@ class HipOps:
         if correction is not None:
             self._chk(correction, torch.float32, (e,), "correction")
         dev = h32.device
+        if self.choose_by_token(n, d, e) and not (h32.data_ptr() | router.data_ptr()) % 16:
+            ids = torch.empty(n, top_k, dtype=torch.int32, device=dev)
+            weights = torch.empty(n, top_k, dtype=torch.float32, device=dev)
+            self._call("jle_moe_logits_choose", _p(h32), _p(router), _p(correction), _p(ids), _p(weights), n, d, e, top_k, *how)
+            return ids, weights, self.moe_align(ids, weights, experts, extra_group=extra_group, note_extra=extra_group)
         logits = torch.empty(n, e, dtype=torch.float32, device=dev)
         self._call("jle_moe_logits", _p(h32), _p(router), _p(logits), n, d, e)
         ids = torch.empty(n, top_k, dtype=torch.int32, device=dev)
@@ -2459,6 +2465,17 @@ class HipOps:
     # chooses for all tokens: 17 us at 8 tokens, 52 at 64, where the separate launches take 22); of up to 16 experts and 64
     # choices every token's own block chooses (15 us at 32 tokens)
     NORM_CHOOSE_EXPERTS, NORM_CHOOSE_TOKENS = 16, 64
+    CHOOSE_TOKENS = 256
+
+    @staticmethod
+    def choose_by_token(n: int, d: int, experts: int) -> bool:
+        """Whether logits and choice by scores are one launch, a block a token with all its experts (up to 16): as long as the
+        blocks are one round, and the router, which every block reads for itself through one first-level cache, is small.
+        Separate | one, us with the grouping: 8 experts of 2,048, one token 6.6 | 6.3, 256 10.9 | 9.2 (512 in two launches
+        12.8); 10 of 4,096, one token 7.4 | 7.9, 17 9.8 | 8.5, 256 12.7 | 10.9; 16 of 5,120, 17 tokens 10.2 | 12.0, 128 13.0 |
+        13.6."""
+        return (n <= HipOps.CHOOSE_TOKENS and experts <= HipOps.NORM_CHOOSE_EXPERTS and d % 4 == 0
+                and d * experts <= (24576 if n < 16 else 40960))
 
     @staticmethod
     def _grouping_arrays(n: int, k: int, experts: int, extra: bool, dev):

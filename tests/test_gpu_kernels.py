@@ -407,6 +407,48 @@ def test_choices_by_scores_token_by_token_equal_the_separate_kernels(ops, n, d, 
             assert torch.equal(gate[:rows].view(torch.int32), again[2][:rows].view(torch.int32))
 
 
+@pytest.mark.parametrize("n,d,e,k,experts,groups", [
+    (1, 4, 1, 1, 1, None), (1, 2048, 10, 2, 8, (5, 3)), (16, 2052, 4, 4, 3, None), (17, 1020, 5, 1, 5, None), (32, 2048, 8, 2, 8, (4, 2)),
+    (33, 2048, 8, 2, 8, (4, 2)), (64, 4100, 9, 2, 7, None), (65, 2048, 16, 2, 16, (4, 2)), (128, 512, 16, 2, 12, (8, 5)),
+    (129, 2048, 8, 2, 8, None), (200, 256, 16, 16, 16, None), (256, 2048, 10, 1, 8, None), (257, 2048, 10, 1, 8, None),
+    (15, 4096, 10, 2, 8, None), (64, 4096, 16, 4, 16, None)])
+@pytest.mark.parametrize("extra", [False, True])
+def test_router_and_choice_in_one_launch_equal_the_separate_kernels(ops, monkeypatch, n, d, e, k, experts, groups, extra):
+    """A block a token with all its experts: the bits of logits and choice as launches of their own, at the edges of a
+    wavefront's experts, of the pieces of a row and of the pairs that one wavefront groups; the grouping against a stable sort."""
+    h, router, correction = _rand(n, d, seed=1), _rand(e, d, scale=0.05, seed=2), _rand(e, scale=0.1, seed=3)
+    router[e - 1] = router[0]
+    g, keep = groups or (None, None)
+    calls = []
+    inner = ops._call
+    monkeypatch.setattr(ops, "_call", lambda name, *a: (calls.append(name), inner(name, *a))[1])
+    for scores, corr in (("sigmoid", correction), ("softmax", None)):
+        args = dict(groups=g, keep_groups=keep, group_terms=1, scores=scores, normalize=1e-20 if extra else None, weight_scale=1.5,
+                    num_experts=experts, extra_group=extra)
+        calls.clear()
+        ids, weights, grouping = ops.moe_choose(h, router, corr, k, **args)
+        assert calls[0] == ("jle_moe_logits" if (n, d, e) in ((257, 2048, 10), (15, 4096, 10), (64, 4096, 16)) else "jle_moe_logits_choose")
+        with monkeypatch.context() as m:
+            m.setattr(type(ops), "CHOOSE_TOKENS", 0)
+            want = ops.moe_choose(h, router, corr, k, **args)
+        assert torch.equal(ids, want[0]) and torch.equal(weights, want[1])
+        assert all(a.shape == b.shape for a, b in zip(grouping, want[2]))
+        off, tok, gate, inv = (t.cpu() for t in grouping)
+        flat = ids.cpu().reshape(-1)
+        order = [int(r) for r in torch.argsort(flat, stable=True) if flat[r] < experts]
+        counts = torch.bincount(flat.long(), minlength=e)[:experts]
+        assert off[: experts + 1].tolist() == [0, *torch.cumsum(counts, 0).tolist()]
+        assert tok[: len(order)].tolist() == [r // k for r in order]
+        assert torch.equal(gate[: len(order)], weights.cpu().reshape(-1)[order])
+        ld = inv.numel() // n
+        row = {r: i for i, r in enumerate(order)}
+        assert inv.view(n, ld)[:, :k].reshape(-1).tolist() == [row.get(r, -1) for r in range(n * k)]
+        if len(off) == experts + 2:  # (a shared expert's rows behind the others)
+            assert int(off[-1]) == len(order) + n and tok[len(order): len(order) + n].tolist() == list(range(n))
+            assert ld == k + 1 and inv.view(n, ld)[:, k].tolist() == [len(order) + t for t in range(n)]
+            assert bool((gate[len(order): len(order) + n] == 1).all())
+
+
 class _Segments:
     """What the matrix-memory kernels read of a step."""
 
