@@ -2380,13 +2380,14 @@ class HipOps:
             # per (tile of 32 tokens, head); a step of single tokens goes on below (a query's keys shared between wavefronts)
             seg_lens, _ = self._segments(meta, token_segment, positions)
             if any(ln > 1 for ln in seg_lens):
-                plan = meta.meta.get("kept_plan") if meta is not None else None
+                group = hq // hk if dh == 128 else 1
+                key = ("kept_plan", hk, group)  # (the lists ask neither for the window nor for how many keys are kept)
+                plan = meta.meta.get(key) if meta is not None else None
                 if plan is None:
                     seg_lens, seg_starts = self._segments(meta, token_segment, positions)
-                    plan = self.attention_plan(seg_lens, seg_starts, ("window", param), q.device, hk, hq // hk if dh == 128 else 1,
-                                               single_tiles=True)
+                    plan = self.attention_plan(seg_lens, seg_starts, ("window", param), q.device, hk, group, single_tiles=True)
                     if meta is not None:
-                        meta.meta["kept_plan"] = plan
+                        meta.meta[key] = plan
                 self._call("jle_attention_prefill_kept", _p(q), _p(kv_cache), _p(out), _p(positions),
                            _p(token_segment), _p(block_table), block_table.shape[1], _p(plan["tiles"]), plan["num_tiles"],
                            self.PREFILL_TILE, _p(plan["groups"]), plan["num_groups"], param, keep, float(scale), hq, hk, dh, ps)
