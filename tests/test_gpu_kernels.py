@@ -371,6 +371,18 @@ def test_attention_with_kept_tokens_of_long_portions_at_head_size_128(ops, ref, 
         assert hq == hk or torch.equal(*alone)
 
 
+def test_attention_with_kept_tokens_of_layers_with_other_heads_in_one_step(ops, ref):
+    """Layers of one step with other numbers of heads find lists laid out for their own; window and kept range change none."""
+    import types
+
+    ctx = types.SimpleNamespace(meta={}, seg_lens=[100, 70], seg_starts=[0, 300], decode_bucket=None)
+    for hq, hk, retention in ((16, 8, ("window_keep", 90, 5)), (12, 2, ("window_keep", 90, 5)), (4, 2, ("window_keep", 90, 5)),
+                              (16, 8, ("window_keep", 33, 70))):
+        q, kv, bt, pos, seg = _attention_case(hq, hk, 128, 16, torch.bfloat16, [(0, 100), (300, 70)], seed=hq)
+        got = ops.paged_attention(q, kv, bt, pos, seg, retention, 128 ** -0.5, meta=ctx)
+        _assert_close_to_scale(got, ref.paged_attention(q, kv, bt, pos, seg, retention, 128 ** -0.5), torch.bfloat16)
+
+
 @pytest.mark.parametrize("n,d,e,k,experts,groups", [
     (5, 1032, 2, 1, 2, None), (5, 2048, 10, 2, 8, (5, 3)), (8, 2056, 16, 8, 16, (4, 2)), (16, 2048, 9, 4, 8, None),
     (17, 4096, 16, 3, 12, (8, 5)), (32, 2048, 10, 2, 8, (5, 3)), (64, 8192, 8, 1, 8, None), (64, 4104, 16, 1, 16, (2, 1))])
