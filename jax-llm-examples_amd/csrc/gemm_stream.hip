@@ -21,10 +21,10 @@
 // (The grid once had an item for every pass that any group could have: those without rows lay between those with, and where
 // their number was even only some of the chiplets got work: 64 groups of 256 x 2,048 with 190 rows 328 us, counted 48; 32 of
 // 1,536 x 2,048, gate and up, with 48 rows 78 -> 41; 12 of 2,560 x 6,144 with 250 237 -> 108.)
-// A block has a compute unit to itself, and those left over behind the last full round would keep a few of them busy for a
-// round's time: they are cut along k into as many pieces as the round has places (Cut), whose float32 sums add_pieces_kernel
-// adds up in their order and finishes.  16 groups of 5,120 x 8,192 with 128 rows, 320 blocks: 297 -> 269 us, what reading the
-// weights alone takes in this arrangement 234.
+// A block has a compute unit to itself, and those left over behind the last full round keep a few of them busy for a round's
+// time.  With one group (an output head) they are cut along k into as many pieces as the round has places, whose float32 sums
+// add_pieces_kernel adds up in their order and finishes (CUT).  With several groups they are not: which blocks are left over
+// follows from how all tokens of the step were shared out, and a row's sums are to have one order whatever rows lie beside it.
 #include "common.h"
 
 using namespace jle;
@@ -117,23 +117,8 @@ struct Items {
   }
 };
 
-// How the items of the last, partly filled round are cut along k: into `pieces` each, one for every compute unit at most, none
-// shorter than kLeastStages.
-constexpr int kLeastStages = 16, kMostPieces = 8, kMostCutGroups = 1024;
-struct Cut {
-  int whole, tail, pieces;  // items taken whole, items behind them, pieces of each of those
-
-  __device__ __forceinline__ Cut(int items, int units, int nstage) {
-    tail = items % units;
-    pieces = tail > 0 ? min(min(units / tail, kMostPieces), nstage / kLeastStages) : 1;
-    if (pieces < 2) tail = 0;
-    whole = items - tail;
-  }
-  // the stages that a piece begins at: whole rounds of four
-  static __device__ __forceinline__ int stage(int piece, int pieces, int nstage) {
-    return (int)((long long)(nstage / WAHEAD) * piece / pieces) * WAHEAD;
-  }
-};
+// The stages that a piece of a cut item begins at: whole rounds of four.
+__device__ __forceinline__ int piece_stage(int piece, int cuts, int nstage) { return nstage / WAHEAD * piece / cuts * WAHEAD; }
 
 // Rows of a tile: a group's rows as even as multiples of 32 allow.
 __device__ __forceinline__ int rows_a_tile(int rows, int tiles) { return ((rows + tiles - 1) / tiles + 31) / 32 * 32; }
@@ -175,7 +160,7 @@ __device__ __forceinline__ void finish_pair(OutT* __restrict__ Y, int t, const f
 // tiles land in tiles that nobody reads).  The main loop has no branch but its own: every load is asked for unconditionally (rows past
 // the live ones read the pass's first row again, into their own places), so that the waits for the loads of
 // two stages ago never include the loads asked for since.
-template <bool SWIGLU, typename OutT, int WAVES, int NTL>
+template <bool SWIGLU, typename OutT, int WAVES, bool CUT, int NTL>
 __device__ __forceinline__ void stream_block(const bf16_t* __restrict__ X, const bf16_t* __restrict__ w0,
                                              const bf16_t* __restrict__ w1, OutT* __restrict__ Y,
                                              const int* __restrict__ a_rows, const float* __restrict__ scale, int act,
@@ -186,9 +171,11 @@ __device__ __forceinline__ void stream_block(const bf16_t* __restrict__ X, const
   constexpr int CPT = (CHUNKS + THREADS - 1) / THREADS;  // per thread
   const int lane = threadIdx.x & 63;
   const int r = lane & 15, g = lane >> 4;
-  X += (size_t)first * BK;  // (this block's stages: nstage of them, a multiple of 4)
-  w0 += (size_t)first * 1024;
-  w1 += (size_t)first * 1024;
+  if constexpr (CUT) {  // (this block's stages: nstage of them, a multiple of 4)
+    X += (size_t)first * BK;
+    w0 += (size_t)first * 1024;
+    w1 += (size_t)first * 1024;
+  }
 
   // who brings which pieces of X: piece c is 8 k of row c / 8, 8 consecutive threads a row's 128 bytes
   uint32_t xsrc[CPT];  // elements from X (the host checks that X has fewer than 2^32)
@@ -278,13 +265,15 @@ __device__ __forceinline__ void stream_block(const bf16_t* __restrict__ X, const
   STAGE(xb, wd, 1, s + 3, false, false);
 #undef STAGE
   if (!wave_ok) return;
-  if (piece != nullptr) {  // a piece of k: its sums as they are
+  if constexpr (CUT) {
+    if (piece != nullptr) {  // a piece of k: its sums as they are
 #pragma unroll
-    for (int nt = 0; nt < NTL; ++nt) {
-      piece[(nt * WAVES * 2 + (threadIdx.x >> 6) * 2) * 64 + lane] = acc0[nt];
-      piece[(nt * WAVES * 2 + (threadIdx.x >> 6) * 2 + 1) * 64 + lane] = acc1[nt];
+      for (int nt = 0; nt < NTL; ++nt) {
+        piece[(nt * WAVES * 2 + (threadIdx.x >> 6) * 2) * 64 + lane] = acc0[nt];
+        piece[(nt * WAVES * 2 + (threadIdx.x >> 6) * 2 + 1) * 64 + lane] = acc1[nt];
+      }
+      return;
     }
-    return;
   }
 
   // accumulators: element i of tile nt in lane (g, r) = weight row 4 g + i of the tile, row 16 nt + r of the pass
@@ -303,8 +292,9 @@ struct StreamArgs {
   const int* a_rows;
   const float* scale;
   Items items;
-  f32x4* pieces;     // null: nothing is cut
-  size_t a_piece;    // f32x4 of a piece
+  f32x4* pieces;             // CUT: the sums of the items behind the `whole` ones, of each in `cuts` pieces
+  size_t a_piece;            // f32x4 of a piece
+  int whole, tail, cuts;
   int Nout, K, units, act;
 };
 
@@ -336,26 +326,23 @@ __device__ __forceinline__ bool tiles_of(int nb, int wave, int Nout, int& t0, in
   return ft < ntile;
 }
 
-template <bool SWIGLU, typename OutT, int WAVES>
+template <bool SWIGLU, typename OutT, int WAVES, bool CUT>
 __global__ __launch_bounds__(WAVES * 64, 2) void gemm_stream_kernel(StreamArgs p) {
   __shared__ __attribute__((aligned(16))) bf16_t sX[2][kRows * BK];
   const int K = p.K, Nout = p.Nout;
-  const int items = p.items.count(), all = K / BK;
-  int left = blockIdx.x, first = 0, stages = all;
+  int left = blockIdx.x, first = 0, stages = K / BK;
   f32x4* piece = nullptr;
-  if (p.pieces != nullptr) {
-    const Cut c(items, p.units, all);
-    const int slot = left - c.whole;
-    if (slot >= c.tail * c.pieces) return;
+  if constexpr (CUT) {
+    const int slot = left - p.whole;
     if (slot >= 0) {
-      left = c.whole + slot % c.tail;
-      first = Cut::stage(slot / c.tail, c.pieces, all);
-      stages = Cut::stage(slot / c.tail + 1, c.pieces, all) - first;
+      left = p.whole + slot % p.tail;
+      first = piece_stage(slot / p.tail, p.cuts, K / BK);
+      stages = piece_stage(slot / p.tail + 1, p.cuts, K / BK) - first;
       piece = p.pieces + (size_t)slot * p.a_piece;
     }
   }
   int passes;
-  const int e = locate(p, items, left, passes);
+  const int e = locate(p, p.items.count(), left, passes);
   if (e < 0) return;  // (the grid is laid out for the most items that so many rows can make)
   const Pass at(p.items, e, left, passes);
   const int tok0 = at.tok0, live = at.live, nb = at.nb;
@@ -367,8 +354,8 @@ __global__ __launch_bounds__(WAVES * 64, 2) void gemm_stream_kernel(StreamArgs p
   const bf16_t* w0 = We + (size_t)t0 * nkb * 512 + lane * 8;
   const bf16_t* w1 = We + (size_t)t1 * nkb * 512 + lane * 8;
 #define GO(NTL_) \
-  stream_block<SWIGLU, OutT, WAVES, NTL_>(p.X, w0, w1, (OutT*)p.Y, p.a_rows, p.scale, p.act, sX, tok0, live, K, Nout, t0, t1, \
-                                          wave_ok, first, stages, piece)
+  stream_block<SWIGLU, OutT, WAVES, CUT, NTL_>(p.X, w0, w1, (OutT*)p.Y, p.a_rows, p.scale, p.act, sX, tok0, live, K, Nout, t0, \
+                                               t1, wave_ok, first, stages, piece)
   if (live <= 32) GO(2);
   else if (live <= 64) GO(4);
   else if (live <= 96) GO(6);
@@ -380,28 +367,25 @@ __global__ __launch_bounds__(WAVES * 64, 2) void gemm_stream_kernel(StreamArgs p
 
 // The cut items' pieces, added up in their order and finished: blockIdx.x is the item behind the whole ones, blockIdx.y
 // which of its tiles of rows.
-template <bool SWIGLU, typename OutT, int WAVES>
+template <typename OutT, int WAVES>
 __global__ __launch_bounds__(WAVES * 64) void add_pieces_kernel(StreamArgs p) {
-  const int items = p.items.count();
-  const Cut c(items, p.units, p.K / BK);
-  if ((int)blockIdx.x >= c.tail) return;
-  int left = c.whole + blockIdx.x, passes;
-  const int e = locate(p, items, left, passes);
+  int left = p.whole + blockIdx.x, passes;
+  const int e = locate(p, p.items.count(), left, passes);
   if (e < 0) return;
   const Pass at(p.items, e, left, passes);
   const int lane = threadIdx.x & 63, r = lane & 15, wave = wave_index();
   int t0, t1;
-  if (!tiles_of<SWIGLU, WAVES>(at.nb, wave, p.Nout, t0, t1)) return;
+  if (!tiles_of<false, WAVES>(at.nb, wave, p.Nout, t0, t1)) return;
   for (int nt = blockIdx.y; nt * 16 < at.live; nt += gridDim.y) {
     const f32x4* from = p.pieces + (size_t)blockIdx.x * p.a_piece + (nt * WAVES * 2 + wave * 2) * 64 + lane;
     f32x4 a0 = from[0], a1 = from[64];
-    for (int i = 1; i < c.pieces; ++i) {
-      from += (size_t)c.tail * p.a_piece;
+    for (int i = 1; i < p.cuts; ++i) {
+      from += (size_t)p.tail * p.a_piece;
       a0 += from[0];
       a1 += from[64];
     }
     if (nt * 16 + r < at.live)
-      finish_pair<SWIGLU>((OutT*)p.Y, at.tok0 + nt * 16 + r, p.scale, p.act, a0, a1, p.Nout, t0, t1, lane >> 4);
+      finish_pair<false>((OutT*)p.Y, at.tok0 + nt * 16 + r, p.scale, p.act, a0, a1, p.Nout, t0, t1, lane >> 4);
   }
 }
 
@@ -612,10 +596,7 @@ int launch_wide(hipStream_t s, const void* X, const void* W, void* Y, const int*
 
 template <bool SW, typename OT, int WV>
 int launch_stream(const StreamArgs& p, long long items, hipStream_t s) {
-  hipLaunchKernelGGL((gemm_stream_kernel<SW, OT, WV>), dim3((unsigned)items), dim3(WV * 64), 0, s, p);
-  JLE_LAUNCH_CHECK();
-  if (p.pieces == nullptr) return 0;
-  hipLaunchKernelGGL((add_pieces_kernel<SW, OT, WV>), dim3(p.units / 2, 4), dim3(WV * 64), 0, s, p);
+  hipLaunchKernelGGL((gemm_stream_kernel<SW, OT, WV, false>), dim3((unsigned)items), dim3(WV * 64), 0, s, p);
   JLE_LAUNCH_CHECK();
   return 0;
 }
@@ -629,17 +610,18 @@ JLE_API int jle_gemm_stream_supported(int Nout, int K, int swiglu) {
   return Nout > 0 && Nout % 16 == 0;
 }
 
-// Bytes that a piece's sums take, of the most rows that an item of M rows can have.
+// Bytes that the sums of a piece of an item take, of the most rows that an item of M rows can have.
 JLE_API int jle_gemm_stream_piece(int M) { return (M < kRows ? (M + 31) / 32 * 32 : kRows) * 256 * 4; }
 
 // X [*, K] bf16, W [G, Nout, K] bf16 in the streaming layout, Y [M, Nout] (or [M, Nout / 2] with swiglu) bf16 or
 // float32; X must have fewer than 2^32 elements (wide: 2^32 bytes).  wide: wide_kernel (groups, bfloat16 out), 2 (plain): HALF.
-// act 1 (plain): max(., 0)^2 of the rounded sums.  pieces: null, or room for `units` pieces (the compute units), and the items of the last, partly filled round are cut.
+// act 1 (plain): max(., 0)^2 of the rounded sums.  pieces (one group, no offsets, plain, float32 out): room for tail * cuts
+// pieces: the last `tail` of the items (256 rows of W by up to 192 rows) are cut into `cuts` along k.
 // Blocks are 8 wavefronts (two per SIMD, one block per compute unit): measured against 4, 5 and 6 on expert
 // shapes with even and with skewed numbers of rows per expert.
 JLE_API int jle_gemm_stream(const void* X, const void* W, void* Y, const int* offsets, const int* a_rows,
                             const float* scale, int swiglu, int act, int out_f32, int M, int Nout, int K, int G,
-                            int wide, void* pieces, int units, hipStream_t s) {
+                            int wide, void* pieces, int tail, int cuts, int units, hipStream_t s) {
   if (M <= 0 || Nout <= 0) return 0;
   if (wide) {
     if (offsets == nullptr || out_f32 || G < 1 || G > 65535 || !jle_gemm_stream_supported(Nout, K, swiglu) ||
@@ -653,16 +635,21 @@ JLE_API int jle_gemm_stream(const void* X, const void* W, void* Y, const int* of
   constexpr int kWaves = 8;
   const int pairs = swiglu ? Nout / 32 : (Nout / 16 + 1) / 2;  // pairs of weight tiles = wavefronts needed per group
   const int nblk = (pairs + kWaves - 1) / kWaves;
-  long long items = ((long long)M / kRows + (offsets == nullptr ? 1 : G)) * nblk;
-  if (pieces != nullptr) {
-    if (units < 2 || units > 65535 || K / BK < 2 * kLeastStages || G > kMostCutGroups ||
-        (uintptr_t)pieces % 16)
-      return JLE_BAD_ARG;
-    items += units;
-  }
+  const long long items = offsets == nullptr ? ((long long)M + kRows - 1) / kRows * nblk : ((long long)M / kRows + G) * nblk;
   if (items > (1ll << 30)) return JLE_BAD_ARG;
-  const StreamArgs p = {(const bf16_t*)X, (const bf16_t*)W, Y, a_rows, scale, {offsets, M, G, nblk, kRows}, (f32x4*)pieces,
-                        (size_t)jle_gemm_stream_piece(M) / 16, Nout, K, units, act};
+  StreamArgs p = {(const bf16_t*)X, (const bf16_t*)W, Y, a_rows, scale, {offsets, M, G, nblk, kRows}, (f32x4*)pieces,
+                  (size_t)jle_gemm_stream_piece(M) / 16, (int)items - tail, tail, cuts, Nout, K, units, act};
+  if (pieces != nullptr) {
+    if (offsets != nullptr || swiglu || !out_f32 || tail < 1 || tail > items || tail > 65535 || cuts < 2 ||
+        cuts > K / (BK * WAHEAD) || (uintptr_t)pieces % 16)
+      return JLE_BAD_ARG;
+    hipLaunchKernelGGL((gemm_stream_kernel<false, float, kWaves, true>), dim3((unsigned)(p.whole + (long long)tail * cuts)),
+                       dim3(kWaves * 64), 0, s, p);
+    JLE_LAUNCH_CHECK();
+    hipLaunchKernelGGL((add_pieces_kernel<float, kWaves>), dim3(tail, 4), dim3(kWaves * 64), 0, s, p);
+    JLE_LAUNCH_CHECK();
+    return 0;
+  }
   if (swiglu) return out_f32 ? launch_stream<true, float, kWaves>(p, items, s) : launch_stream<true, bf16_t, kWaves>(p, items, s);
   return out_f32 ? launch_stream<false, float, kWaves>(p, items, s) : launch_stream<false, bf16_t, kWaves>(p, items, s);
 }

@@ -90,7 +90,7 @@ _SIGNATURES = {
     "jle_conv_rows": [_vp, _i, _i, _vp, _vp, _vp, _i, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _vp],
     "jle_conv_qk_prepare": [_vp, _i, _vp, _vp, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _f, _f, _vp, _vp, _i, _i,
                             _i, _i, _i, _i, _i, _i, _i, _vp],
-    "jle_gemm_stream": [_vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _i, _vp, _i, _vp],
+    "jle_gemm_stream": [_vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _i, _vp, _i, _i, _i, _vp],
     "jle_streams_mix_norm": [_vp, _i, _vp, _vp, _vp, _i, _vp, _i, _vp, _vp, _vp, _vp, _f, _vp, _i, _vp, _i, _i, _i, _i,
                              _vp],
     "jle_embed_sinusoid": [_vp, _vp, _vp, _i, _f, _vp, _vp, _i, _i, _i, _vp],
@@ -1882,23 +1882,21 @@ class HipOps:
 
     @staticmethod
     @functools.lru_cache(maxsize=4096)
-    def stream_cuts(rows: int, groups: int, row_blocks: int, k: int, units: int) -> bool:
-        """Whether the products in passes cut the blocks left over behind the last full round of ``units`` compute units along
-        k (``row_blocks`` blocks of 256 rows of W a group; see ``gemm_stream.hip``).  How many are left over is known on the
-        device only, where nothing is cut if they fill more than half of the round; the launch that adds the pieces up is made
-        all the same, so this asks whether groups whose sizes scatter about their mean by twice its root can leave such a
-        rest.  Writing and adding up the pieces takes about 12 us, more than the round is shorter by with a short k.  Whole |
-        cut, us: 16 groups of 5,120 x 8,192 (320 blocks) with 64 rows 285 | 254, 128 309 | 276, 192 356 | 300; 8 of
-        4,096 x 7,168 (128) with 64 101 | 90, 190 140 | 117; 8 of 2,048 x 4,096 (64) with 64 55 | 42; an output head of
-        32,000 x 4,096 (125), 64 rows 67 | 61; but 16 of 2,048 x 3,072 (128) with 128 57 | 68, 8 of 4,096 x 2,048 (128) with
-        64 30 | 39."""
-        if k // 64 < HipOps.CUT_STAGES or groups > 1024:
-            return False
-        mean = rows / groups
-        spread = 2 * mean ** 0.5 if groups > 1 else 0.0
-        passes = [max(1, -(-int(mean + d) // 192)) for d in (-spread, spread)]
-        tail = groups * row_blocks * passes[0] % units
-        return passes[0] != passes[1] or 0 < tail <= units // 2
+    def stream_cuts(rows: int, row_blocks: int, k: int, units: int) -> tuple[int, int]:
+        """How many blocks of an output head's product in passes (``row_blocks`` blocks of 256 rows of W a pass) are cut along
+        k, and into how many pieces each (see ``gemm_stream.hip``): those left over behind the last full round of ``units``
+        compute units, into one for every place of the round, no shorter than 16 stages of 64 k; none if they fill more than
+        half of the round.  Writing and adding up the pieces takes about 12 us, more than the round is shorter by with a short
+        k.  Whole | cut, us: 32,000 x 4,096 (125 blocks), 17 rows 67 | 58, 64 68 | 63, 192 90 | 79; 202,048 x 5,120 (790), 17
+        rows 380 | 348, 64 403 | 370, 192 495 | 461, 400 (three passes) 1,239 | 1,229.
+
+        Experts' products, which gained as much, are not cut: their blocks are known on the device only, and which of them are
+        left over depends on every token of the step."""
+        blocks = row_blocks * -(-rows // 192)
+        tail = blocks % units
+        if k // 64 < HipOps.CUT_STAGES or not 0 < tail <= units // 2:
+            return 0, 1
+        return tail, min(units // tail, 8, k // 64 // 16)
 
     def gemm_stream(self, a, b, *, offsets=None, a_rows=None, scale=None, swiglu=False, relu2=False, out_f32=False, rows=None,
                     expected=None):
@@ -1923,12 +1921,13 @@ class HipOps:
         wide, among = 0, m if expected is None else expected
         if offsets is not None and not out_f32 and a.numel() < 2 ** 31 and not (a.data_ptr() | b.data_ptr()) % 16:
             wide = 2 if not swiglu and self.stream_half(among, g, -(-nout // 128)) else self.stream_wide(among, g, -(-nout // 256))
-        pieces = None  # (sums of the pieces: 192 KiB each at most)
-        if not wide and self.stream_cuts(among, g, -(-nout // 256), k, self._compute_units):
-            room = self._query("jle_gemm_stream_piece", m) * self._compute_units
-            pieces = torch.empty(room, dtype=torch.uint8, device=a.device)
+        pieces, tail, cuts = None, 0, 1  # (sums of the pieces: 192 KiB each at most)
+        if offsets is None and g == 1 and out_f32 and not swiglu:
+            tail, cuts = self.stream_cuts(m, -(-nout // 256), k, self._compute_units)
+            if tail:
+                pieces = torch.empty(self._query("jle_gemm_stream_piece", m) * tail * cuts, dtype=torch.uint8, device=a.device)
         self._call("jle_gemm_stream", _p(a), _p(b), _p(out), _p(offsets), _p(a_rows), _p(scale), int(swiglu),
-                   int(relu2), int(out_f32), m, nout, k, g, int(wide), _p(pieces), self._compute_units)
+                   int(relu2), int(out_f32), m, nout, k, g, int(wide), _p(pieces), tail, cuts, self._compute_units)
         return out
 
     @staticmethod

@@ -118,11 +118,12 @@ def test_narrower_tiles_are_one_round_however_the_rows_are_shared_out(groups):
     assert taken
 
 
-@pytest.mark.parametrize("groups, rows, blocks, k, cut", [
-    (16, 128, 20, 8192, True), (16, 128, 64, 5120, False), (8, 64, 16, 7168, True), (8, 64, 8, 4096, True), (8, 512, 8, 4096, False),
-    (8, 190, 16, 7168, True), (8, 128, 16, 4032, False), (1025, 64, 1, 8192, False), (1, 64, 125, 4096, True), (1, 64, 196, 4096, False)])
-def test_which_launches_can_cut_their_last_round(groups, rows, blocks, k, cut):
-    assert HipOps.stream_cuts(rows * groups, groups, blocks, k, 256) == cut
+@pytest.mark.parametrize("rows, blocks, k, units, cut", [
+    (64, 125, 4096, 256, (125, 2)), (64, 196, 4096, 256, (0, 1)), (64, 256, 4096, 256, (0, 1)), (64, 257, 4096, 256, (1, 4)),
+    (192, 790, 5120, 256, (22, 5)), (193, 790, 5120, 256, (44, 5)), (1000, 8, 16384, 256, (48, 5)), (64, 125, 4032, 256, (0, 1)),
+    (64, 125, 4096, 64, (0, 1)), (64, 80, 4096, 64, (16, 4)), (64, 125, 4096, 1, (0, 1))])
+def test_which_blocks_of_an_output_head_are_cut(rows, blocks, k, units, cut):
+    assert HipOps.stream_cuts(rows, blocks, k, units) == cut
 
 
 @pytest.mark.parametrize("n, k, least, most", [(16000, 2048, 5, 64), (28672, 4096, 5, 64), (28688, 4096, 5, 32), (32768, 2048, 5, 32),

@@ -1423,7 +1423,7 @@ def test_wide_tiles_of_the_weight_streaming_product(ops, counts, nout, k, swiglu
     assert torch.equal(*got)
 
 
-@pytest.mark.parametrize("way", ["passes", "cut", "wide", "half"])
+@pytest.mark.parametrize("way", ["passes", "wide", "half"])
 def test_squared_relu_behind_the_weight_streaming_product(ops, way):
     """The bits of the product and the activation as launches of their own, by every kernel that takes such rows."""
     from jax_llm_examples_amd.ops.layout import tile_
@@ -1432,21 +1432,57 @@ def test_squared_relu_behind_the_weight_streaming_product(ops, way):
     x[5, 7], x[9] = float("nan"), 0.0
     tile_(w)
     off = torch.tensor([0] + counts).cumsum(0).int().to(DEV)
-    ops.stream_wide, ops.stream_half, ops.stream_cuts = (lambda *a: way == "wide"), (lambda *a: way == "half"), (lambda *a: way == "cut")
+    ops.stream_wide, ops.stream_half = (lambda *a: way == "wide"), (lambda *a: way == "half")
     got = ops.gemm_stream(x, w, offsets=off, relu2=True)
     want = ops.relu2(ops.gemm_stream(x, w, offsets=off))
-    del ops.stream_wide, ops.stream_half, ops.stream_cuts
+    del ops.stream_wide, ops.stream_half
     assert torch.equal(got.view(torch.int16), want.view(torch.int16)) and bool((got >= 0).sum() > 0)
+
+
+@pytest.mark.parametrize("rows,nout,k,tail,cuts", [
+    (77, 2048, 16384, 8, 8),    # one pass, all of it is cut
+    (33, 272, 4352, 2, 4),      # pieces of unequal length, a second block of W of one tile
+    (400, 544, 4096, 5, 3),     # three passes of three blocks of W: the first four items whole
+    (193, 4096, 4096, 1, 4)])   # two passes, the last item alone
+def test_blocks_cut_along_k_of_an_output_head(ops, monkeypatch, rows, nout, k, tail, cuts):
+    from jax_llm_examples_amd.ops.layout import tile_
+    x, w = _rand(rows, k, dt=torch.bfloat16, seed=1), _rand(nout, k, dt=torch.bfloat16, scale=0.02, seed=2)
+    want = x.double() @ w.double().T.contiguous()
+    tile_(w)
+    monkeypatch.setattr(ops, "stream_cuts", lambda *a: (tail, cuts))
+    got = [ops.gemm_stream(x, w, out_f32=True) for _ in range(2)]
+    monkeypatch.setattr(ops, "stream_cuts", lambda *a: (0, 1))
+    whole = ops.gemm_stream(x, w, out_f32=True)
+    assert torch.equal(got[0], got[1]) and not torch.equal(got[0], whole)
+    # float32 sums of k products of bfloat16 numbers: sqrt(k) 2^-24 of the terms' size is 4e-6 at 4,096 in the worst
+    # order and a tenth of that as the matrix units add up
+    for y in (got[0], whole):
+        assert float((y.double() - want).norm() / want.norm()) <= 4e-6
+
+
+@pytest.mark.parametrize("swiglu", [False, True])
+@pytest.mark.parametrize("counts", [[3] * 257, [3, 0, 200] * 50, [190] * 8, [3] + [400] * 40])
+def test_experts_products_of_a_row_do_not_depend_on_the_other_rows(ops, counts, swiglu):
+    """The first expert's rows beside full groups, beside empty ones and beside one that has most of the rows: the same bits."""
+    from jax_llm_examples_amd.ops.layout import tile_
+    nout, k, first = 64, 4096, counts[0]
+    x = _rand(sum(counts), k, dt=torch.bfloat16, seed=1)
+    w = _rand(1, nout, k, dt=torch.bfloat16, scale=0.02, seed=2).repeat(len(counts), 1, 1)
+    tile_(w)
+    got = []
+    for others in (counts[1:], [0] * (len(counts) - 1), [0] * (len(counts) - 2) + [sum(counts[1:])]):
+        off = torch.tensor([0, first] + others).cumsum(0).int().to(DEV)
+        got.append(ops.gemm_stream(x[: int(off[-1])].contiguous(), w, offsets=off, swiglu=swiglu)[:first])
+    assert torch.equal(got[0], got[1]) and torch.equal(got[0], got[2])
 
 
 @pytest.mark.parametrize("counts,nout,k,swiglu", [
     ([5, 0, 192, 193, 31, 385], 272, 4096, False),   # several passes, two blocks of W, the second of one tile
-    ([100, 33, 64], 544, 4352, True),                # pieces of unequal length
-    ([3] * 256, 64, 4096, False),                    # exactly a round of blocks: nothing to cut
-    ([3] * 257, 64, 4096, False),                    # one left over, in as many pieces as its stages allow
-    ([200] * 65, 512, 4096, True),                   # more groups than a look takes, blocks left over that stay whole
-    ([77], 2048, 16384, False)])                     # one group: all of it is cut
-def test_blocks_cut_along_k_of_the_weight_streaming_product(ops, counts, nout, k, swiglu):
+    ([190, 200, 260, 385, 193], 272, 512, False),    # two or three passes in every group
+    ([100, 33, 64], 544, 4352, True),                # one pass a group
+    ([3] * 257, 64, 4096, False),                    # more groups than compute units
+    ([200] * 65, 512, 1024, True)])                  # more groups than a look takes, two passes each
+def test_passes_of_the_weight_streaming_product_against_64_bits(ops, monkeypatch, counts, nout, k, swiglu):
     from jax_llm_examples_amd.ops.layout import tile_
     m, e = sum(counts), len(counts)
     x, w = _rand(m + 3, k, dt=torch.bfloat16, seed=1), _rand(e, nout, k, dt=torch.bfloat16, scale=0.02, seed=2)
@@ -1455,21 +1491,16 @@ def test_blocks_cut_along_k_of_the_weight_streaming_product(ops, counts, nout, k
     off = torch.tensor([0] + counts).cumsum(0).int().to(DEV)
     rows = torch.randperm(m + 3, generator=torch.Generator().manual_seed(3))[:m].int().to(DEV)
     scale = _rand(m, seed=4)
-    ops.stream_wide, ops.stream_half, ops.stream_cuts = (lambda *a: False), (lambda *a: False), (lambda *a: True)
-    got = [ops.gemm_stream(x, stored, offsets=off, a_rows=rows, scale=scale, swiglu=swiglu, rows=m, out_f32=True) for _ in range(2)]
-    if e == 1:
-        got.append(ops.gemm_stream(x[rows.long()], stored[0], out_f32=True) * scale[:, None])  # (no offsets)
-    del ops.stream_wide, ops.stream_half, ops.stream_cuts
-    assert torch.equal(got[0], got[1]) and torch.equal(got[0], got[-1])
+    monkeypatch.setattr(ops, "stream_wide", lambda *a: False)
+    monkeypatch.setattr(ops, "stream_half", lambda *a: False)
+    got = ops.gemm_stream(x, stored, offsets=off, a_rows=rows, scale=scale, swiglu=swiglu, rows=m, out_f32=True)
     o = 0
     for c, we in zip(counts, w):
-        want = x[rows[o: o + c].long()].double() @ we.double().T * scale[o: o + c, None].double()
+        want = x[rows[o: o + c].long()].double() @ we.double().T.contiguous() * scale[o: o + c, None].double()
         if swiglu:
             want = torch.nn.functional.silu(want[:, : nout // 2]) * want[:, nout // 2:]
-        if c:
-            # float32 sums of k products of bfloat16 numbers: sqrt(k) 2^-24 of the terms' size is 4e-6 at 4,096 in the worst
-            # order and a tenth of that as the matrix units add up; the activation doubles it
-            assert float((got[0][o: o + c].double() - want).norm() / want.norm()) <= 4e-6
+        if c:  # (see above; the activation doubles it)
+            assert float((got[o: o + c].double() - want).norm() / want.norm()) <= 4e-6
         o += c
 
 
