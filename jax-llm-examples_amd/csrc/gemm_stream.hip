@@ -16,7 +16,8 @@
 // four stages.  Groups with more than 192 rows are done in passes (each reads the weights again).
 //
 // Work items are (group, pass, block of WAVES * 32 weight rows), the last fastest, so the blocks of a group
-// are dealt to all dies in turn and a group with many rows slows all of them alike.  How many there are is known on the
+// are dealt to all dies in turn and a group with many rows slows all of them alike; where a group's blocks are no multiple of
+// the eight dies and there are up to two rounds of items, (pass, group, block) (locate).  How many there are is known on the
 // device only (Items): every block counts the groups' passes itself, so that items are those with rows and nothing else.
 // (The grid once had an item for every pass that any group could have: those without rows lay between those with, and where
 // their number was even only some of the chiplets got work: 64 groups of 256 x 2,048 with 190 rows 328 us, counted 48; 32 of
@@ -58,7 +59,7 @@ struct Items {
   int M, G, nblk, most;
 
   __device__ __forceinline__ int rows_of(int g) const {
-    return offsets == nullptr ? (g == 0 ? M : 0) : g < G ? offsets[g + 1] - offsets[g] : 0;
+    return offsets == nullptr ? M : g < G ? offsets[g + 1] - offsets[g] : 0;
   }
   __device__ __forceinline__ int count() const {
     const int lane = threadIdx.x & 63;
@@ -95,10 +96,7 @@ struct Items {
     const int mine = (rows_of(threadIdx.x & 63) + most - 1) / most, of = __builtin_amdgcn_readfirstlane(mine);
     return G <= 64 && __ballot((int)(threadIdx.x & 63) < G && (mine > of + 1 || mine < of - 1)) == 0;
   }
-  // find() of such groups with every group's first tile before all second ones: with a round or two of blocks in all the last
-  // ones are then those with the fewest rows (8 groups of 4,096 x 2,048 with 512 rows, three passes of 192, 192 and 128: 106
-  // us group after group, 94 so; where one group has most of the rows its last tiles would come last: 16 of 5,120 x 8,192
-  // with 128, 40 % in one, 287 | 352).
+  // find() of such groups with every group's first tile before all second ones (see locate).
   __device__ __forceinline__ int find_by_tile(int& left, int& tiles) const {
     const int mine = (rows_of(threadIdx.x & 63) + most - 1) / most;
     for (int t = 0;; ++t) {
@@ -298,10 +296,23 @@ struct StreamArgs {
   int Nout, K, units, act;
 };
 
-// Item `left`'s group, how many passes the group has, and which of the group's items it is; `items` there are.
-__device__ __forceinline__ int locate(const StreamArgs& p, int items, int& left, int& passes) {
+// Item `left`'s group, how many passes the group has, and which of the group's items it is.
+// The passes of a block of W are to run on one die, whose cache then has the weights for the second one.  Items are dealt to
+// the eight dies in turn, so they do group after group if a group's blocks are a multiple of eight; else every group's first
+// pass comes before all second ones.  Group after group | so, us: 16 groups of 1,024 x 4,096 (four blocks) with 250 rows
+// 73 | 62, 400 99 | 85, 600 117 | 96; 32 of 1,024 x 2,048 with 300 86 | 60; 64 of 512 x 1,024 with 300 48 | 39; 12 of
+// 2,560 x 6,144 (ten) with 250 155 | 116; but 8 of 4,096 x 2,048 (sixteen) with 450 85 | 91, 570 99 | 104, 700 107 | 121.  Where one
+// group has most of the rows its last tiles would come last (16 of 5,120 x 8,192 with 128, 40 % in one, 287 | 352).
+__device__ __forceinline__ int locate(const StreamArgs& p, int& left, int& passes) {
+  const Items& it = p.items;
+  if (it.offsets == nullptr) {
+    passes = (it.M + it.most - 1) / it.most;
+    return left < passes * it.nblk ? 0 : -1;
+  }
+  if (it.nblk % 8 == 0) return it.find(left, passes);
+  const int items = it.count();
   if (left >= items) return -1;
-  return items <= 2 * p.units && p.items.even() ? p.items.find_by_tile(left, passes) : p.items.find(left, passes);
+  return items <= 2 * p.units && it.even() ? it.find_by_tile(left, passes) : it.find(left, passes);
 }
 
 // The rows of item `left` of a group with `tiles` passes, the first of its block's pairs of tiles of W
@@ -342,7 +353,7 @@ __global__ __launch_bounds__(WAVES * 64, 2) void gemm_stream_kernel(StreamArgs p
     }
   }
   int passes;
-  const int e = locate(p, p.items.count(), left, passes);
+  const int e = locate(p, left, passes);
   if (e < 0) return;  // (the grid is laid out for the most items that so many rows can make)
   const Pass at(p.items, e, left, passes);
   const int tok0 = at.tok0, live = at.live, nb = at.nb;
@@ -370,7 +381,7 @@ __global__ __launch_bounds__(WAVES * 64, 2) void gemm_stream_kernel(StreamArgs p
 template <typename OutT, int WAVES>
 __global__ __launch_bounds__(WAVES * 64) void add_pieces_kernel(StreamArgs p) {
   int left = p.whole + blockIdx.x, passes;
-  const int e = locate(p, p.items.count(), left, passes);
+  const int e = locate(p, left, passes);
   if (e < 0) return;
   const Pass at(p.items, e, left, passes);
   const int lane = threadIdx.x & 63, r = lane & 15, wave = wave_index();

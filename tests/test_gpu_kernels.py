@@ -1479,6 +1479,7 @@ def test_experts_products_of_a_row_do_not_depend_on_the_other_rows(ops, counts, 
 @pytest.mark.parametrize("counts,nout,k,swiglu", [
     ([5, 0, 192, 193, 31, 385], 272, 4096, False),   # several passes, two blocks of W, the second of one tile
     ([190, 200, 260, 385, 193], 272, 512, False),    # two or three passes in every group
+    ([190, 385, 260, 385, 193], 2048, 256, False),   # the same with blocks of W for every die
     ([100, 33, 64], 544, 4352, True),                # one pass a group
     ([3] * 257, 64, 4096, False),                    # more groups than compute units
     ([200] * 65, 512, 1024, True)])                  # more groups than a look takes, two passes each
