@@ -23,9 +23,9 @@
 // their number was even only some of the chiplets got work: 64 groups of 256 x 2,048 with 190 rows 328 us, counted 48; 32 of
 // 1,536 x 2,048, gate and up, with 48 rows 78 -> 41; 12 of 2,560 x 6,144 with 250 237 -> 108.)
 // A block has a compute unit to itself, and those left over behind the last full round keep a few of them busy for a round's
-// time.  With one group (an output head) they are cut along k into as many pieces as the round has places, whose float32 sums
-// add_pieces_kernel adds up in their order and finishes (CUT).  With several groups they are not: which blocks are left over
-// follows from how all tokens of the step were shared out, and a row's sums are to have one order whatever rows lie beside it.
+// time.  So some blocks of W, the last ones of every group, are cut along k into as many pieces as the round has places, whose
+// float32 sums add_pieces_kernel adds up in their order and finishes (CUT).  Which blocks these are is known before the launch,
+// from the numbers of groups and of their blocks: a row's sums have one order whatever rows lie beside it.
 #include "common.h"
 
 using namespace jle;
@@ -61,16 +61,21 @@ struct Items {
   __device__ __forceinline__ int rows_of(int g) const {
     return offsets == nullptr ? M : g < G ? offsets[g + 1] - offsets[g] : 0;
   }
-  __device__ __forceinline__ int count() const {
+  __device__ __forceinline__ int tiles_of_all() const {
+    if (offsets == nullptr) return (M + most - 1) / most;
     const int lane = threadIdx.x & 63;
     int n = 0;
     for (int g0 = 0; g0 < G; g0 += 64) n += (rows_of(g0 + lane) + most - 1) / most;
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) n += __shfl_xor(n, o, 64);
-    return __builtin_amdgcn_readfirstlane(n) * nblk;
+    return __builtin_amdgcn_readfirstlane(n);
   }
   // Item `left`'s group (-1: no such item), how many tiles the group has, and which of the group's items it is.
   __device__ __forceinline__ int find(int& left, int& tiles) const {
+    if (offsets == nullptr) {
+      tiles = (M + most - 1) / most;
+      return left < tiles * nblk ? 0 : -1;
+    }
     const int lane = threadIdx.x & 63;
     for (int g0 = 0; g0 < G; g0 += 64) {
       const int mine = (rows_of(g0 + lane) + most - 1) / most;
@@ -290,9 +295,8 @@ struct StreamArgs {
   const int* a_rows;
   const float* scale;
   Items items;
-  f32x4* pieces;             // CUT: the sums of the items behind the `whole` ones, of each in `cuts` pieces
-  size_t a_piece;            // f32x4 of a piece
-  int whole, tail, cuts;
+  f32x4* pieces;        // CUT: the sums of the last `cut` blocks of every group, each in `cuts` pieces of k
+  int cut, cuts, room;  // room: tiles of 16 rows that a piece of one of the blocks has place for, of all passes
   int Nout, K, units, act;
 };
 
@@ -305,12 +309,8 @@ struct StreamArgs {
 // group has most of the rows its last tiles would come last (16 of 5,120 x 8,192 with 128, 40 % in one, 287 | 352).
 __device__ __forceinline__ int locate(const StreamArgs& p, int& left, int& passes) {
   const Items& it = p.items;
-  if (it.offsets == nullptr) {
-    passes = (it.M + it.most - 1) / it.most;
-    return left < passes * it.nblk ? 0 : -1;
-  }
-  if (it.nblk % 8 == 0) return it.find(left, passes);
-  const int items = it.count();
+  if (it.offsets == nullptr || it.nblk % 8 == 0) return it.find(left, passes);
+  const int items = it.tiles_of_all() * it.nblk;
   if (left >= items) return -1;
   return items <= 2 * p.units && it.even() ? it.find_by_tile(left, passes) : it.find(left, passes);
 }
@@ -337,26 +337,58 @@ __device__ __forceinline__ bool tiles_of(int nb, int wave, int Nout, int& t0, in
   return ft < ntile;
 }
 
+// A block of a CUT launch: the whole items come first, then the first pieces of all cut ones, their second pieces, and so on.
+struct CutItem {
+  Items items;         // of which it is one: the whole or the cut blocks of the groups
+  int at, piece, nb0;  // which one, which piece (-1: whole), the first of the groups' blocks that are meant
+
+  __device__ __forceinline__ CutItem(const StreamArgs& p, int block) : items(p.items), at(block), piece(-1), nb0(0) {
+    const int passes = items.tiles_of_all(), whole = passes * (items.nblk - p.cut), a_piece = passes * p.cut;
+    if (block < whole) {
+      items.nblk -= p.cut;
+      return;
+    }
+    nb0 = items.nblk - p.cut;
+    items.nblk = p.cut;
+    piece = a_piece > 0 ? (block - whole) / a_piece : p.cuts;
+    at = block - whole - piece * a_piece;
+  }
+};
+
+// Where the sums of a piece of cut item `at` begin, whose rows begin at tok0.  The tiles of rows of all passes lie behind each
+// other; a pass of n rows has 2 * ceil(n / 32) of them, no more than floor(n / 16) + 2.
+__device__ __forceinline__ f32x4* piece_sums(const StreamArgs& p, int piece, int at, int tok0) {
+  return p.pieces + ((size_t)(piece * p.cut + at % p.cut) * p.room + (tok0 >> 4) + 2 * (at / p.cut)) * 1024;
+}
+
 template <bool SWIGLU, typename OutT, int WAVES, bool CUT>
 __global__ __launch_bounds__(WAVES * 64, 2) void gemm_stream_kernel(StreamArgs p) {
+  static_assert(WAVES == 8, "a tile of a piece's sums is 16 rows by 256 of W");
   __shared__ __attribute__((aligned(16))) bf16_t sX[2][kRows * BK];
   const int K = p.K, Nout = p.Nout;
-  int left = blockIdx.x, first = 0, stages = K / BK;
-  f32x4* piece = nullptr;
+  int e, left = blockIdx.x, passes, nb0 = 0, first = 0, stages = K / BK, at_piece = -1, item = 0;
   if constexpr (CUT) {
-    const int slot = left - p.whole;
-    if (slot >= 0) {
-      left = p.whole + slot % p.tail;
-      first = piece_stage(slot / p.tail, p.cuts, K / BK);
-      stages = piece_stage(slot / p.tail + 1, p.cuts, K / BK) - first;
-      piece = p.pieces + (size_t)slot * p.a_piece;
+    const CutItem c(p, left);
+    if (c.piece >= p.cuts) return;
+    p.items = c.items;
+    nb0 = c.nb0;
+    at_piece = c.piece;
+    left = item = c.at;
+    e = p.items.find(left, passes);
+    if (at_piece >= 0) {
+      first = piece_stage(at_piece, p.cuts, K / BK);
+      stages = piece_stage(at_piece + 1, p.cuts, K / BK) - first;
     }
+  } else {
+    e = locate(p, left, passes);
   }
-  int passes;
-  const int e = locate(p, left, passes);
   if (e < 0) return;  // (the grid is laid out for the most items that so many rows can make)
   const Pass at(p.items, e, left, passes);
-  const int tok0 = at.tok0, live = at.live, nb = at.nb;
+  const int tok0 = at.tok0, live = at.live, nb = nb0 + at.nb;
+  f32x4* piece = nullptr;
+  if constexpr (CUT) {
+    if (at_piece >= 0) piece = piece_sums(p, at_piece, item, tok0);
+  }
   const int lane = threadIdx.x & 63, wave = wave_index();
   const int nkb = K >> 5;
   const bf16_t* We = p.W + (size_t)e * Nout * K;
@@ -376,22 +408,23 @@ __global__ __launch_bounds__(WAVES * 64, 2) void gemm_stream_kernel(StreamArgs p
 #undef GO
 }
 
-// The cut items' pieces, added up in their order and finished: blockIdx.x is the item behind the whole ones, blockIdx.y
-// which of its tiles of rows.
+// The cut items' pieces, added up in their order and finished: blockIdx.x is the item, blockIdx.y which of its tiles of rows.
 template <typename OutT, int WAVES>
 __global__ __launch_bounds__(WAVES * 64) void add_pieces_kernel(StreamArgs p) {
-  int left = p.whole + blockIdx.x, passes;
-  const int e = locate(p, left, passes);
+  const int nb0 = p.items.nblk - p.cut;
+  p.items.nblk = p.cut;
+  int left = blockIdx.x, passes;
+  const int e = p.items.find(left, passes);
   if (e < 0) return;
   const Pass at(p.items, e, left, passes);
   const int lane = threadIdx.x & 63, r = lane & 15, wave = wave_index();
   int t0, t1;
-  if (!tiles_of<false, WAVES>(at.nb, wave, p.Nout, t0, t1)) return;
+  if (!tiles_of<false, WAVES>(nb0 + at.nb, wave, p.Nout, t0, t1)) return;
   for (int nt = blockIdx.y; nt * 16 < at.live; nt += gridDim.y) {
-    const f32x4* from = p.pieces + (size_t)blockIdx.x * p.a_piece + (nt * WAVES * 2 + wave * 2) * 64 + lane;
+    const f32x4* from = piece_sums(p, 0, blockIdx.x, at.tok0) + (nt * WAVES * 2 + wave * 2) * 64 + lane;
     f32x4 a0 = from[0], a1 = from[64];
     for (int i = 1; i < p.cuts; ++i) {
-      from += (size_t)p.tail * p.a_piece;
+      from += (size_t)p.cut * p.room * 1024;
       a0 += from[0];
       a1 += from[64];
     }
@@ -605,9 +638,21 @@ int launch_wide(hipStream_t s, const void* X, const void* W, void* Y, const int*
   return 0;
 }
 
+// passes: the most that so many rows can make
 template <bool SW, typename OT, int WV>
-int launch_stream(const StreamArgs& p, long long items, hipStream_t s) {
-  hipLaunchKernelGGL((gemm_stream_kernel<SW, OT, WV, false>), dim3((unsigned)items), dim3(WV * 64), 0, s, p);
+int launch_stream(const StreamArgs& p, long long passes, hipStream_t s) {
+  hipLaunchKernelGGL((gemm_stream_kernel<SW, OT, WV, false>), dim3((unsigned)(passes * p.items.nblk)), dim3(WV * 64), 0, s, p);
+  JLE_LAUNCH_CHECK();
+  return 0;
+}
+
+template <typename OT, int WV>
+int launch_cut(const StreamArgs& p, long long passes, hipStream_t s) {
+  const long long blocks = passes * (p.items.nblk - p.cut + p.cut * p.cuts);
+  if (blocks > (1ll << 30)) return JLE_BAD_ARG;
+  hipLaunchKernelGGL((gemm_stream_kernel<false, OT, WV, true>), dim3((unsigned)blocks), dim3(WV * 64), 0, s, p);
+  JLE_LAUNCH_CHECK();
+  hipLaunchKernelGGL((add_pieces_kernel<OT, WV>), dim3((unsigned)(passes * p.cut), 4), dim3(WV * 64), 0, s, p);
   JLE_LAUNCH_CHECK();
   return 0;
 }
@@ -621,18 +666,18 @@ JLE_API int jle_gemm_stream_supported(int Nout, int K, int swiglu) {
   return Nout > 0 && Nout % 16 == 0;
 }
 
-// Bytes that the sums of a piece of an item take, of the most rows that an item of M rows can have.
-JLE_API int jle_gemm_stream_piece(int M) { return (M < kRows ? (M + 31) / 32 * 32 : kRows) * 256 * 4; }
+// Tiles of rows that the pieces of a cut block of all groups have place for; 16 KB a tile and piece.
+JLE_API int jle_gemm_stream_room(int M, int G) { return (M >> 4) + 2 * (M / kRows + G); }
 
 // X [*, K] bf16, W [G, Nout, K] bf16 in the streaming layout, Y [M, Nout] (or [M, Nout / 2] with swiglu) bf16 or
 // float32; X must have fewer than 2^32 elements (wide: 2^32 bytes).  wide: wide_kernel (groups, bfloat16 out), 2 (plain): HALF.
-// act 1 (plain): max(., 0)^2 of the rounded sums.  pieces (one group, no offsets, plain, float32 out): room for tail * cuts
-// pieces: the last `tail` of the items (256 rows of W by up to 192 rows) are cut into `cuts` along k.
+// act 1 (plain): max(., 0)^2 of the rounded sums.  cuts > 1 (plain, not wide): the last `cut` of a group's blocks of 256 rows of
+// W are cut into `cuts` pieces along k; pieces: place for jle_gemm_stream_room(M, G) * cut * cuts tiles of 16 KB.
 // Blocks are 8 wavefronts (two per SIMD, one block per compute unit): measured against 4, 5 and 6 on expert
 // shapes with even and with skewed numbers of rows per expert.
 JLE_API int jle_gemm_stream(const void* X, const void* W, void* Y, const int* offsets, const int* a_rows,
                             const float* scale, int swiglu, int act, int out_f32, int M, int Nout, int K, int G,
-                            int wide, void* pieces, int tail, int cuts, int units, hipStream_t s) {
+                            int wide, void* pieces, int cut, int cuts, int units, hipStream_t s) {
   if (M <= 0 || Nout <= 0) return 0;
   if (wide) {
     if (offsets == nullptr || out_f32 || G < 1 || G > 65535 || !jle_gemm_stream_supported(Nout, K, swiglu) ||
@@ -646,21 +691,15 @@ JLE_API int jle_gemm_stream(const void* X, const void* W, void* Y, const int* of
   constexpr int kWaves = 8;
   const int pairs = swiglu ? Nout / 32 : (Nout / 16 + 1) / 2;  // pairs of weight tiles = wavefronts needed per group
   const int nblk = (pairs + kWaves - 1) / kWaves;
-  const long long items = offsets == nullptr ? ((long long)M + kRows - 1) / kRows * nblk : ((long long)M / kRows + G) * nblk;
-  if (items > (1ll << 30)) return JLE_BAD_ARG;
-  StreamArgs p = {(const bf16_t*)X, (const bf16_t*)W, Y, a_rows, scale, {offsets, M, G, nblk, kRows}, (f32x4*)pieces,
-                  (size_t)jle_gemm_stream_piece(M) / 16, (int)items - tail, tail, cuts, Nout, K, units, act};
-  if (pieces != nullptr) {
-    if (offsets != nullptr || swiglu || !out_f32 || tail < 1 || tail > items || tail > 65535 || cuts < 2 ||
-        cuts > K / (BK * WAHEAD) || (uintptr_t)pieces % 16)
+  const long long passes = offsets == nullptr ? ((long long)M + kRows - 1) / kRows : (long long)M / kRows + G;
+  if (passes * nblk > (1ll << 30)) return JLE_BAD_ARG;
+  const StreamArgs p = {(const bf16_t*)X, (const bf16_t*)W, Y, a_rows, scale, {offsets, M, G, nblk, kRows}, (f32x4*)pieces,
+                        cut, cuts, jle_gemm_stream_room(M, G), Nout, K, units, act};
+  if (cuts > 1) {
+    if (swiglu || cut < 1 || cut > nblk || cuts > K / (BK * WAHEAD) || pieces == nullptr || (uintptr_t)pieces % 16)
       return JLE_BAD_ARG;
-    hipLaunchKernelGGL((gemm_stream_kernel<false, float, kWaves, true>), dim3((unsigned)(p.whole + (long long)tail * cuts)),
-                       dim3(kWaves * 64), 0, s, p);
-    JLE_LAUNCH_CHECK();
-    hipLaunchKernelGGL((add_pieces_kernel<float, kWaves>), dim3(tail, 4), dim3(kWaves * 64), 0, s, p);
-    JLE_LAUNCH_CHECK();
-    return 0;
+    return out_f32 ? launch_cut<float, kWaves>(p, passes, s) : launch_cut<bf16_t, kWaves>(p, passes, s);
   }
-  if (swiglu) return out_f32 ? launch_stream<true, float, kWaves>(p, items, s) : launch_stream<true, bf16_t, kWaves>(p, items, s);
-  return out_f32 ? launch_stream<false, float, kWaves>(p, items, s) : launch_stream<false, bf16_t, kWaves>(p, items, s);
+  if (swiglu) return out_f32 ? launch_stream<true, float, kWaves>(p, passes, s) : launch_stream<true, bf16_t, kWaves>(p, passes, s);
+  return out_f32 ? launch_stream<false, float, kWaves>(p, passes, s) : launch_stream<false, bf16_t, kWaves>(p, passes, s);
 }

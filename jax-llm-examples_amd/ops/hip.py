@@ -195,7 +195,7 @@ def _bind(path: str):
             fn.argtypes = args
             fn.restype = ctypes.c_int
     for name, args in (("jle_attention_mfma_supported", [_i, _i, _i, _i]),  # queries, not launches: no stream
-                       ("jle_greedy_blocks", [_i]), ("jle_gemm_stream_supported", [_i, _i, _i]), ("jle_gemm_stream_piece", [_i]), ("jle_gemm_f32_stream_supported", [_i, _i, _i]),
+                       ("jle_greedy_blocks", [_i]), ("jle_gemm_stream_supported", [_i, _i, _i]), ("jle_gemm_stream_room", [_i, _i]), ("jle_gemm_f32_stream_supported", [_i, _i, _i]),
                        ("jle_gemm_few_tiles", [_i] * 7),
                        ("jle_latent_attention_mfma_supported", [_i, _i, _i, _i, _i]),
                        ("jle_latent_values_supported", [_i] * 6),
@@ -1882,21 +1882,26 @@ class HipOps:
 
     @staticmethod
     @functools.lru_cache(maxsize=4096)
-    def stream_cuts(rows: int, row_blocks: int, k: int, units: int) -> tuple[int, int]:
-        """How many blocks of an output head's product in passes (``row_blocks`` blocks of 256 rows of W a pass) are cut along
-        k, and into how many pieces each (see ``gemm_stream.hip``): those left over behind the last full round of ``units``
-        compute units, into one for every place of the round, no shorter than 16 stages of 64 k; none if they fill more than
-        half of the round.  Writing and adding up the pieces takes about 12 us, more than the round is shorter by with a short
-        k.  Whole | cut, us: 32,000 x 4,096 (125 blocks), 17 rows 67 | 58, 64 68 | 63, 192 90 | 79; 202,048 x 5,120 (790), 17
-        rows 380 | 348, 64 403 | 370, 192 495 | 461, 400 (three passes) 1,239 | 1,229.
-
-        Experts' products, which gained as much, are not cut: their blocks are known on the device only, and which of them are
-        left over depends on every token of the step."""
-        blocks = row_blocks * -(-rows // 192)
-        tail = blocks % units
-        if k // 64 < HipOps.CUT_STAGES or not 0 < tail <= units // 2:
+    def stream_cuts(rows: int, groups: int, row_blocks: int, k: int, units: int) -> tuple[int, int]:
+        """How many blocks of 256 rows of W of every group a plain product in passes cuts along k, and into how many pieces
+        (see ``gemm_stream.hip``): as many as are left over behind the last full round of ``units`` compute units where every
+        group has one pass, into one piece for every place of that round, none shorter than 16 stages of 64 k; none if they fill
+        more than half of the round, or if groups one and a half times the root of their mean fuller than it have two passes.
+        Which blocks those are follows from the sizes and the number of rows alone, so a token's sums do not depend on how
+        the others were shared out.  Writing and adding up the pieces takes about 12 us, more than the round is shorter by with
+        a short k.  Whole | cut, us, drawn groups: 16 of 5,120 x 8,192 (four of twenty blocks in four) with 24 rows 271 | 226, 100
+        300 | 261, 170 348 | 302, 178 355 | 365; 8 of 4,096 x 7,168 (all in two) with 48 99 | 88, 170 141 | 116, 178 144 | 158; 8 of
+        2,048 x 4,096 (all in four) with 100 60 | 56; 12 of 2,560 x 6,144 with 165 121 | 112; 32 of 1,024 x 8,192 with 100 123 | 126;
+        an output head of 32,000 x 4,096, 17 rows 67 | 55, 64 67 | 61, 192 90 | 74, of 202,048 x 5,120 380 | 346, 402 | 368,
+        498 | 468; but 8 of 4,096 x 2,048 with 64, in two, 34 | 44.  With 40 % of the rows in one group it loses where it gains
+        least: 16 of 5,120 x 8,192 with 100 270 | 285, 12 of 2,560 x 6,144 with 48 100 | 112, 170 130 | 142."""
+        mean = rows / groups
+        tail = groups * row_blocks % units
+        if k // 64 < HipOps.CUT_STAGES or not 0 < tail <= units // 2 or mean + (1.5 * mean ** 0.5 if groups > 1 else 0) > 192:
             return 0, 1
-        return tail, min(units // tail, 8, k // 64 // 16)
+        columns = -(-tail // groups)
+        pieces = min(units // (columns * groups), 8, k // 64 // 16)
+        return (columns, pieces) if pieces > 1 else (0, 1)
 
     def gemm_stream(self, a, b, *, offsets=None, a_rows=None, scale=None, swiglu=False, relu2=False, out_f32=False, rows=None,
                     expected=None):
@@ -1921,13 +1926,13 @@ class HipOps:
         wide, among = 0, m if expected is None else expected
         if offsets is not None and not out_f32 and a.numel() < 2 ** 31 and not (a.data_ptr() | b.data_ptr()) % 16:
             wide = 2 if not swiglu and self.stream_half(among, g, -(-nout // 128)) else self.stream_wide(among, g, -(-nout // 256))
-        pieces, tail, cuts = None, 0, 1  # (sums of the pieces: 192 KiB each at most)
-        if offsets is None and g == 1 and out_f32 and not swiglu:
-            tail, cuts = self.stream_cuts(m, -(-nout // 256), k, self._compute_units)
-            if tail:
-                pieces = torch.empty(self._query("jle_gemm_stream_piece", m) * tail * cuts, dtype=torch.uint8, device=a.device)
+        pieces, cut, cuts = None, 0, 1
+        if not wide and not swiglu:
+            cut, cuts = self.stream_cuts(among, g, -(-nout // 256), k, self._compute_units)
+            if cuts > 1:  # (tiles of 16 KB)
+                pieces = torch.empty(self._query("jle_gemm_stream_room", m, g) * cut * cuts << 14, dtype=torch.uint8, device=a.device)
         self._call("jle_gemm_stream", _p(a), _p(b), _p(out), _p(offsets), _p(a_rows), _p(scale), int(swiglu),
-                   int(relu2), int(out_f32), m, nout, k, g, int(wide), _p(pieces), tail, cuts, self._compute_units)
+                   int(relu2), int(out_f32), m, nout, k, g, int(wide), _p(pieces), cut, cuts, self._compute_units)
         return out
 
     @staticmethod

@@ -118,12 +118,14 @@ def test_narrower_tiles_are_one_round_however_the_rows_are_shared_out(groups):
     assert taken
 
 
-@pytest.mark.parametrize("rows, blocks, k, units, cut", [
-    (64, 125, 4096, 256, (125, 2)), (64, 196, 4096, 256, (0, 1)), (64, 256, 4096, 256, (0, 1)), (64, 257, 4096, 256, (1, 4)),
-    (192, 790, 5120, 256, (22, 5)), (193, 790, 5120, 256, (44, 5)), (1000, 8, 16384, 256, (48, 5)), (64, 125, 4032, 256, (0, 1)),
-    (64, 125, 4096, 64, (0, 1)), (64, 80, 4096, 64, (16, 4)), (64, 125, 4096, 1, (0, 1))])
-def test_which_blocks_of_an_output_head_are_cut(rows, blocks, k, units, cut):
-    assert HipOps.stream_cuts(rows, blocks, k, units) == cut
+@pytest.mark.parametrize("rows, groups, blocks, k, units, cut", [
+    (64, 1, 125, 4096, 256, (125, 2)), (64, 1, 196, 4096, 256, (0, 1)), (64, 1, 256, 4096, 256, (0, 1)), (64, 1, 257, 4096, 256, (1, 4)),
+    (192, 1, 790, 5120, 256, (22, 5)), (193, 1, 790, 5120, 256, (0, 1)), (64, 1, 125, 4032, 256, (0, 1)), (64, 1, 125, 4096, 64, (0, 1)),
+    (64, 1, 80, 4096, 64, (16, 4)), (64, 1, 125, 4096, 1, (0, 1)), (16 * 128, 16, 20, 8192, 256, (4, 4)), (16 * 172, 16, 20, 8192, 256, (4, 4)), (16 * 173, 16, 20, 8192, 256, (0, 1)),
+    (16 * 128, 16, 64, 5120, 256, (0, 1)), (8 * 64, 8, 16, 7168, 256, (16, 2)), (8 * 64, 8, 8, 4096, 256, (8, 4)), (3 * 64, 3, 86, 4096, 256, (1, 4)),
+    (100 * 3, 100, 3, 4096, 256, (1, 2)), (0, 129, 1, 8192, 256, (0, 1))])
+def test_which_blocks_of_a_product_in_passes_are_cut(rows, groups, blocks, k, units, cut):
+    assert HipOps.stream_cuts(rows, groups, blocks, k, units) == cut
 
 
 @pytest.mark.parametrize("n, k, least, most", [(16000, 2048, 5, 64), (28672, 4096, 5, 64), (28688, 4096, 5, 32), (32768, 2048, 5, 32),

@@ -1423,8 +1423,8 @@ def test_wide_tiles_of_the_weight_streaming_product(ops, counts, nout, k, swiglu
     assert torch.equal(*got)
 
 
-@pytest.mark.parametrize("way", ["passes", "wide", "half"])
-def test_squared_relu_behind_the_weight_streaming_product(ops, way):
+@pytest.mark.parametrize("way", ["passes", "cut", "wide", "half"])
+def test_squared_relu_behind_the_weight_streaming_product(ops, monkeypatch, way):
     """The bits of the product and the activation as launches of their own, by every kernel that takes such rows."""
     from jax_llm_examples_amd.ops.layout import tile_
     counts, nout, k = [3, 0, 200, 70], 272, 4096
@@ -1432,47 +1432,68 @@ def test_squared_relu_behind_the_weight_streaming_product(ops, way):
     x[5, 7], x[9] = float("nan"), 0.0
     tile_(w)
     off = torch.tensor([0] + counts).cumsum(0).int().to(DEV)
-    ops.stream_wide, ops.stream_half = (lambda *a: way == "wide"), (lambda *a: way == "half")
+    monkeypatch.setattr(ops, "stream_wide", lambda *a: way == "wide")
+    monkeypatch.setattr(ops, "stream_half", lambda *a: way == "half")
+    monkeypatch.setattr(ops, "stream_cuts", lambda *a: (2, 3) if way == "cut" else (0, 1))
     got = ops.gemm_stream(x, w, offsets=off, relu2=True)
     want = ops.relu2(ops.gemm_stream(x, w, offsets=off))
-    del ops.stream_wide, ops.stream_half
     assert torch.equal(got.view(torch.int16), want.view(torch.int16)) and bool((got >= 0).sum() > 0)
 
 
-@pytest.mark.parametrize("rows,nout,k,tail,cuts", [
-    (77, 2048, 16384, 8, 8),    # one pass, all of it is cut
-    (33, 272, 4352, 2, 4),      # pieces of unequal length, a second block of W of one tile
-    (400, 544, 4096, 5, 3),     # three passes of three blocks of W: the first four items whole
-    (193, 4096, 4096, 1, 4)])   # two passes, the last item alone
-def test_blocks_cut_along_k_of_an_output_head(ops, monkeypatch, rows, nout, k, tail, cuts):
+@pytest.mark.parametrize("counts,nout,k,cut,cuts", [
+    ([77], 2048, 16384, 8, 8),                       # one group, all of it is cut
+    ([192], 272, 4352, 2, 4),                        # pieces of unequal length, a second block of W of one tile
+    ([33], 4096, 4096, 1, 3),                        # the last block alone
+    ([5, 0, 192, 193, 31, 385], 800, 2048, 1, 2),    # groups without rows, with one, two and three passes; fifteen tiles and three
+    ([5, 0, 192, 193, 31, 385], 800, 2048, 4, 7),    # all blocks
+    ([1, 47, 17] * 50, 528, 1024, 2, 4),             # more groups than a look takes; pieces of a round of stages
+    ([0, 0], 272, 1024, 1, 2)])                      # no rows at all
+def test_blocks_cut_along_k_of_the_weight_streaming_product(ops, monkeypatch, counts, nout, k, cut, cuts):
+    """One group with and without offsets, picked and scaled rows, float32 and bfloat16 results."""
     from jax_llm_examples_amd.ops.layout import tile_
-    x, w = _rand(rows, k, dt=torch.bfloat16, seed=1), _rand(nout, k, dt=torch.bfloat16, scale=0.02, seed=2)
-    want = x.double() @ w.double().T.contiguous()
-    tile_(w)
-    monkeypatch.setattr(ops, "stream_cuts", lambda *a: (tail, cuts))
-    got = [ops.gemm_stream(x, w, out_f32=True) for _ in range(2)]
+    m, e = sum(counts), len(counts)
+    x, w = _rand(m + 3, k, dt=torch.bfloat16, seed=1), _rand(e, nout, k, dt=torch.bfloat16, scale=0.02, seed=2)
+    stored = w.clone()
+    tile_(stored)
+    off = torch.tensor([0] + counts).cumsum(0).int().to(DEV)
+    rows = torch.randperm(m + 3, generator=torch.Generator().manual_seed(3))[:m].int().to(DEV)
+    scale = _rand(m, seed=4)
+    monkeypatch.setattr(ops, "stream_wide", lambda *a: False)
+    monkeypatch.setattr(ops, "stream_half", lambda *a: False)
+    monkeypatch.setattr(ops, "stream_cuts", lambda *a: (cut, cuts))
+    m = max(m, 7)  # (rows that no group has are left as they are)
+    args = dict(offsets=off, a_rows=rows, scale=scale, rows=m)
+    got, low = (ops.gemm_stream(x, stored, out_f32=f, **args) for f in (True, False))
+    assert torch.equal(got, ops.gemm_stream(x, stored, out_f32=True, **args)) or m > sum(counts)
+    assert torch.equal(low[: sum(counts)], got[: sum(counts)].bfloat16())
+    if e == 1:
+        assert torch.equal(got, ops.gemm_stream(x[rows.long()], stored[0], out_f32=True) * scale[:, None])
     monkeypatch.setattr(ops, "stream_cuts", lambda *a: (0, 1))
-    whole = ops.gemm_stream(x, w, out_f32=True)
-    assert torch.equal(got[0], got[1]) and not torch.equal(got[0], whole)
-    # float32 sums of k products of bfloat16 numbers: sqrt(k) 2^-24 of the terms' size is 4e-6 at 4,096 in the worst
-    # order and a tenth of that as the matrix units add up
-    for y in (got[0], whole):
-        assert float((y.double() - want).norm() / want.norm()) <= 4e-6
+    uncut = ops.gemm_stream(x, stored, out_f32=True, **args)
+    o, from_cut = 0, (-(-nout // 256) - cut) * 256
+    assert torch.equal(got[: sum(counts), :from_cut], uncut[: sum(counts), :from_cut])
+    for c, we in zip(counts, w):
+        want = x[rows[o: o + c].long()].double() @ we.double().T.contiguous() * scale[o: o + c, None].double()
+        # float32 sums of k products of bfloat16 numbers: sqrt(k) 2^-24 of the terms' size is 8e-6 at 16,384 in the worst
+        # order and a tenth of that as the matrix units add up
+        for y in (got, uncut) if c else ():
+            assert float((y[o: o + c].double() - want).norm() / want.norm()) <= 4e-6
+        o += c
 
 
 @pytest.mark.parametrize("swiglu", [False, True])
-@pytest.mark.parametrize("counts", [[3] * 257, [3, 0, 200] * 50, [190] * 8, [3] + [400] * 40])
-def test_experts_products_of_a_row_do_not_depend_on_the_other_rows(ops, counts, swiglu):
-    """The first expert's rows beside full groups, beside empty ones and beside one that has most of the rows: the same bits."""
+@pytest.mark.parametrize("counts", [[3] * 257, [3, 0, 200] * 50, [100] * 8, [3] + [120] * 20, [190] * 8, [3] + [400] * 40])
+def test_experts_products_of_a_row_do_not_depend_on_how_the_others_are_shared_out(ops, counts, swiglu):
+    """The first expert's rows beside full groups, beside empty ones and one that has all the rows, beside odd ones: the same bits."""
     from jax_llm_examples_amd.ops.layout import tile_
-    nout, k, first = 64, 4096, counts[0]
+    nout, k, first, rest = 544, 4096, counts[0], sum(counts[1:])
     x = _rand(sum(counts), k, dt=torch.bfloat16, seed=1)
     w = _rand(1, nout, k, dt=torch.bfloat16, scale=0.02, seed=2).repeat(len(counts), 1, 1)
     tile_(w)
     got = []
-    for others in (counts[1:], [0] * (len(counts) - 1), [0] * (len(counts) - 2) + [sum(counts[1:])]):
+    for others in (counts[1:], [0] * (len(counts) - 2) + [rest], [rest // 3] + [0] * (len(counts) - 3) + [rest - rest // 3]):
         off = torch.tensor([0, first] + others).cumsum(0).int().to(DEV)
-        got.append(ops.gemm_stream(x[: int(off[-1])].contiguous(), w, offsets=off, swiglu=swiglu)[:first])
+        got.append(ops.gemm_stream(x, w, offsets=off, swiglu=swiglu)[:first])
     assert torch.equal(got[0], got[1]) and torch.equal(got[0], got[2])
 
 
