@@ -348,7 +348,6 @@ def test_attention_with_kept_tokens_of_long_portions_at_head_size_128(ops, ref, 
     specs = [(0, 333), (190, 130), (517, 1), (64, 64), (1000, 35)]
     q, kv, bt, pos, seg = _attention_case(hq, hk, 128, ps, dt, specs, seed=3)
     want = ref.paged_attention(q, kv, bt, pos, seg, ("window_keep", window, keep), 128 ** -0.5)
-    plain = kv.clone()
     for i, (a, b) in enumerate(specs):
         first = max(0, a - window + 1)
         for j in range(-(-(a + b) // ps)):
@@ -365,10 +364,23 @@ def test_attention_with_kept_tokens_of_long_portions_at_head_size_128(ops, ref, 
     got = ops.paged_attention(q, kv, bt, pos, seg, ("window_keep", window, keep), 128 ** -0.5)
     assert calls == ["jle_attention_prefill_kept"]
     _assert_close_to_scale(got, want, dt)
-    if window == 2000:  # (nothing lies before the window: the plain kernel's bits)
-        alone = [ops.paged_attention(q[:333].contiguous(), plain, bt, pos[:333].contiguous(), seg[:333].contiguous(), r, 128 ** -0.5)
-                 for r in (("window_keep", window, keep), ("all",))]
-        assert hq == hk or torch.equal(*alone)
+
+
+@pytest.mark.parametrize("window,keep,n", [(1024, 8, 80), (150, 70, 1111), (1024, 8, 2048)])
+def test_keys_shared_between_wavefronts_lose_no_precision(ops, window, keep, n):
+    """Query heads that share kv heads against the same kv heads given to each (whose wavefronts read their own keys): both
+    take a running maximum every 32 keys and round the same probabilities, so that only the orders of float32 sums differ."""
+    q, kv, bt, pos, seg = _attention_case(8, 4, 128, 16, torch.bfloat16, [(0, n)], seed=11)
+    pages, twice = bt[0].long(), kv.repeat_interleave(2, dim=2)
+    keys = twice[pages, 0].permute(1, 0, 2, 3).reshape(8, -1, 128)[:, :n].double()
+    values = twice[pages, 1].reshape(-1, 8, 128, 16).permute(1, 0, 3, 2).reshape(8, -1, 128)[:, :n].double()  # (stored transposed)
+    at = torch.arange(n, device=DEV)
+    hidden = (at[None] > at[:, None]) | (at[:, None] - at[None] >= window) & (at[None] >= keep)
+    want = torch.stack([torch.softmax((q[:, h].double() @ keys[h].T.contiguous() * 128 ** -0.5).masked_fill(hidden, -math.inf), -1) @ values[h]
+                        for h in range(8)], 1)
+    err = [float((ops.paged_attention(q, pool, bt, pos, seg, ("window_keep", window, keep), 128 ** -0.5).view(n, 8, 128).double() - want).norm())
+           for pool in (kv, twice)]
+    assert err[0] <= 1.001 * err[1]
 
 
 def test_attention_with_kept_tokens_of_layers_with_other_heads_in_one_step(ops, ref):
