@@ -1099,7 +1099,7 @@ class HipOps:
             return None
         if rows <= 4 or rows <= 8 and (n * k < 1 << 24 or n * k <= 1 << 25 and (k >= 5120 or act >= 0)):
             return self.gemm_f32_rows(h, w, act)
-        if (act <= 0 and HipOps.f32_tiles_pay(rows, n, k, act == 0)
+        if (act <= 0 and HipOps.f32_tiles_pay(rows, n, k, act == 0, self._compute_units)
                 and not (torch.is_grad_enabled() and (h.requires_grad or w.requires_grad))):
             return self.gemm_f32_skinny(h, w, swiglu=act == 0)
         ranges = self.split_ranges(rows, n, k, act >= 0, self._compute_units)
@@ -1108,18 +1108,18 @@ class HipOps:
         return None
 
     @staticmethod
-    def f32_tiles_pay(rows: int, n: int, k: int, gated: bool) -> bool:
+    def f32_tiles_pay(rows: int, n: int, k: int, gated: bool, units: int = 256) -> bool:
         """Whether a dense float32 product goes through the kernel of the experts' few rows, a block for 16 columns and 16 rows
         (``gemm_f32.hip``; on the float32 matrix instructions, errors against 64 bits from a third to three quarters of the
         library's).  A block takes 4 us and 3 more per 1,024 of k, so it is the faster one while its blocks are one round of
-        the compute units (two with a short k) and k is no longer than 2,048.  The library's | this, us: 64 x 64, 32 rows 4.7 |
+        the ``units`` compute units (two with a short k) and k is no longer than 2,048.  The library's | this, us: 64 x 64, 32 rows 4.7 |
         4.1, 128 rows 6.3 | 4.2; 64 x 256, 32 rows 9.1 | 5.0; 512 x 512, 128 rows 11.1 | 5.8; 1,024 x 1,024, 64 rows
         11.8 | 6.2, 128 rows (512 blocks) 11.9 | 9.4; 2,048 x 2,048, 16 rows 12.9 | 10.2, 32 rows 13.4 | 10.6, 48 rows (384
         blocks) 13.5 | 15.9; 2,048 x 4,096, 16 rows 15.1 | 18.5.  Gate and up, with the activation, of 512 x 64, 32 rows 7.0 |
         4.7; 2,048 x 2,048, 64 rows 17.3 | 14.1; 8,192 x 2,048, 16 rows 23.9 | 19.6.  (And the library's product costs the host
         20 us a call, this one 7.)"""
         tiles = -(-(n // 2 if gated else n) // 16) * -(-rows // 16)
-        return rows <= HipOps.F32_SKINNY_ROWS and k <= 2048 and tiles <= (512 if k <= 1024 and not gated else 256)
+        return rows <= HipOps.F32_SKINNY_ROWS and k <= 2048 and tiles <= (2 * units if k <= 1024 and not gated else units)
 
     def linear(self, h, w, out_dtype=None):
         """``h @ w.T``: through the BLAS library; up to a few tens of bfloat16 rows (:meth:`_few`), and few or many float32

@@ -33,6 +33,13 @@ def test_dense_float32_products_of_tens_of_rows_by_size(rows, n, k, gated, pays)
     assert HipOps.f32_tiles_pay(rows, n, k, gated) == pays
 
 
+@pytest.mark.parametrize("units", [32, 64, 128, 256])
+def test_dense_float32_products_of_tens_of_rows_are_one_round_of_any_device(units):
+    """A device with fewer compute units, as a part of one has: as many blocks are several rounds of it."""
+    assert HipOps.f32_tiles_pay(16, 32 * units, 1024, True, units) and not HipOps.f32_tiles_pay(16, 32 * units + 32, 1024, True, units)
+    assert HipOps.f32_tiles_pay(48, 32 * (units // 3), 512, True, units) and not HipOps.f32_tiles_pay(49, 32 * (units // 3), 512, True, units)
+
+
 @pytest.mark.parametrize("rows", [1, 512])
 @pytest.mark.parametrize("a, b", [("cuda:0", "cuda:1"), ("cuda:1", "cuda:0"), ("cuda:0", "cpu"), ("cpu", "cuda:0"),
                                   ("cuda:1", "cuda:1")])
