@@ -1111,15 +1111,23 @@ class HipOps:
     def f32_tiles_pay(rows: int, n: int, k: int, gated: bool, units: int = 256) -> bool:
         """Whether a dense float32 product goes through the kernel of the experts' few rows, a block for 16 columns and 16 rows
         (``gemm_f32.hip``; on the float32 matrix instructions, errors against 64 bits from a third to three quarters of the
-        library's).  A block takes 4 us and 3 more per 1,024 of k, so it is the faster one while its blocks are one round of
-        the ``units`` compute units (two with a short k) and k is no longer than 2,048.  The library's | this, us: 64 x 64, 32 rows 4.7 |
-        4.1, 128 rows 6.3 | 4.2; 64 x 256, 32 rows 9.1 | 5.0; 512 x 512, 128 rows 11.1 | 5.8; 1,024 x 1,024, 64 rows
-        11.8 | 6.2, 128 rows (512 blocks) 11.9 | 9.4; 2,048 x 2,048, 16 rows 12.9 | 10.2, 32 rows 13.4 | 10.6, 48 rows (384
-        blocks) 13.5 | 15.9; 2,048 x 4,096, 16 rows 15.1 | 18.5.  Gate and up, with the activation, of 512 x 64, 32 rows 7.0 |
-        4.7; 2,048 x 2,048, 64 rows 17.3 | 14.1; 8,192 x 2,048, 16 rows 23.9 | 19.6.  (And the library's product costs the host
-        20 us a call, this one 7.)"""
-        tiles = -(-(n // 2 if gated else n) // 16) * -(-rows // 16)
-        return rows <= HipOps.F32_SKINNY_ROWS and k <= 2048 and tiles <= (2 * units if k <= 1024 and not gated else units)
+        library's).  A block takes 4 us and 3 more per 1,024 of k however few blocks there are, so it is the faster one while its
+        blocks are one round of the ``units`` compute units, and with more than 1,024 of k only where the library, which shares
+        k out among blocks while the matrix is small, no longer does.  The library's is the faster one too for up to 16 rows of
+        matrices with 512 columns and more and a short k, where both are mostly launch.  The library's | this, us on the
+        device, launches recorded: 64 x 64, 32 rows 3.9 | 3.7, 128 rows 5.8 | 3.8; 512 x 256, 16 rows 4.0 | 5.0, 64 rows 5.6 | 5.1;
+        512 x 640, 16 rows 6.5 | 5.6; 1,024 x 1,024, 16 rows 8.4 | 6.0, 64 rows 8.5 | 7.1, 128 rows (512 blocks) 8.8 | 9.7; 2,048 x 1,024,
+        48 rows (384 blocks) 8.7 | 9.8; 32 x 2,048, 16 rows 8.3 | 8.6, 64 rows 9.2 | 11.2; 1,024 x 2,048, 64 rows 9.1 | 11.3; 1,024 x
+        1,536, 64 rows 7.8 | 10.4; 1,536 x 2,048, 32 rows 12.3 | 11.3; 2,048 x 2,048, 16 rows 12.2 | 11.5, 32 rows 12.7 | 11.9;
+        2,048 x 1,536, 16 rows 9.8 | 9.8; 4,096 x 1,152, 16 rows 10.2 | 10.0.  Gate and up, with the activation: 512 x 64, 32 rows
+        5.9 | 4.6; 512 x 256, 16 rows 5.9 | 6.4, 64 rows 7.5 | 6.5; 2,048 x 1,024, 64 rows 11.9 | 9.3; 512 x 2,048, 64 rows 11.1 | 14.5;
+        2,048 x 1,536, 32 rows 12.5 | 13.7; 2,048 x 2,048, 32 rows 14.9 | 15.0, 64 rows 17.0 | 15.3; 4,096 x 1,152, 16 rows 12.2 | 11.4.
+        (And the library's product costs the host 20 us a call, this one 7.)"""
+        if rows > HipOps.F32_SKINNY_ROWS or k > 2048 or -(-(n // 2 if gated else n) // 16) * -(-rows // 16) > units:
+            return False
+        if k > 1024:
+            return n * k >= (4 if gated else 3) << 20
+        return gated or n < 512 or k >= 512 or rows > 16 and k >= 128
 
     def linear(self, h, w, out_dtype=None):
         """``h @ w.T``: through the BLAS library; up to a few tens of bfloat16 rows (:meth:`_few`), and few or many float32

@@ -27,8 +27,12 @@ def test_dense_float32_products_by_size():
 
 
 @pytest.mark.parametrize("rows, n, k, gated, pays", [(9, 64, 64, False, True), (128, 64, 64, False, True), (129, 64, 64, False, False),
-    (32, 2048, 2048, False, True), (33, 2048, 2048, False, False), (128, 1024, 1024, False, True), (128, 2048, 512, False, False),
-    (64, 2048, 2048, True, True), (65, 2048, 2048, True, False), (16, 512, 2052, False, False)])
+    (32, 2048, 2048, False, True), (33, 2048, 2048, False, False), (64, 1024, 1024, False, True), (65, 1024, 1024, False, False), (128, 2048, 512, False, False),
+    (64, 2048, 2048, True, True), (65, 2048, 2048, True, False), (16, 512, 2052, False, False),
+    (64, 32, 2048, False, False), (64, 32, 2048, True, False), (32, 1535, 2048, False, False), (32, 1536, 2048, False, True),
+    (16, 2046, 2048, True, False), (16, 2048, 2048, True, True), (64, 32, 1024, False, True), (9, 32, 1028, False, False),
+    (16, 512, 508, False, False), (16, 512, 512, False, True), (16, 511, 64, False, True), (17, 512, 128, False, True),
+    (17, 512, 124, False, False), (16, 512, 64, True, True)])
 def test_dense_float32_products_of_tens_of_rows_by_size(rows, n, k, gated, pays):
     assert HipOps.f32_tiles_pay(rows, n, k, gated) == pays
 

@@ -1075,7 +1075,7 @@ def test_dense_float32_products(ops, rows, nout, k):
         assert torch.equal(ops.linear(x, w), ops.gemm_f32_split(x, w, -1, ranges) if ranges else ops.gemm_f32_rows(x, w))
 
 
-@pytest.mark.parametrize("rows,nout,k", [(9, 2, 4), (16, 64, 64), (17, 130, 36), (33, 1000, 516), (64, 1024, 1024), (128, 512, 2048),
+@pytest.mark.parametrize("rows,nout,k", [(9, 2, 4), (16, 64, 64), (17, 130, 36), (33, 1000, 516), (64, 1024, 1024), (128, 512, 2048), (32, 2048, 2048),
                                          (127, 62, 2044), (48, 2048, 300)])
 def test_dense_float32_products_of_tens_of_rows(ops, rows, nout, k):
     """The experts' kernel for few rows with one group, the way the dense products of such sizes go.  A wavefront adds up every
@@ -1083,12 +1083,12 @@ def test_dense_float32_products_of_tens_of_rows(ops, rows, nout, k):
     x, w = _rand(rows, k, seed=41), _rand(nout, k, seed=42)
     want, size = x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t()
     bound = size * (k / 32 + 40) * 2.0 ** -24
-    assert ops.f32_tiles_pay(rows, nout, k, False)
-    got = ops.linear(x, w)
-    assert torch.equal(got, ops.gemm_f32_skinny(x, w)) and bool(((got.double() - want).abs() <= bound).all())
+    got = ops.gemm_f32_skinny(x, w)
+    assert bool(((got.double() - want).abs() <= bound).all())
+    assert torch.equal(got, ops.linear(x, w)) or not ops.f32_tiles_pay(rows, nout, k, False)
     gate, up = want.chunk(2, -1)
-    got = ops.swiglu_linear(x, w)
-    assert torch.equal(got, ops.gemm_f32_skinny(x, w, swiglu=True))
+    got = ops.gemm_f32_skinny(x, w, swiglu=True)
+    assert torch.equal(got, ops.swiglu_linear(x, w)) or not ops.f32_tiles_pay(rows, nout, k, True)
     b = 1.13 * bound[:, :nout // 2] * up.abs() + (gate.abs() + 2.0 ** -19 * gate.abs()) * bound[:, nout // 2:]
     assert bool(((got.double() - torch.nn.functional.silu(gate) * up).abs() <= 1.01 * b + 2.0 ** -19 * (gate * up).abs() + 1e-30).all())
     gelu = ops.swiglu_linear(x, w, "gelu_tanh").double()  # (has no kernel here: the library's and a pass of its own)
