@@ -316,8 +316,7 @@ __device__ __forceinline__ void align_by_wave(const int (&id)[R], const float (&
   }
 }
 
-// The same as a launch of its own, for few pairs that lie in memory: 128 pairs of 8 experts 5.6 us
-// in moe_align_kernel, whose thousand threads meet at eight barriers, about 3 so.
+// The same as a launch of its own, for few pairs of few experts that lie in memory (see launch_align).
 template <int R>
 __global__ __launch_bounds__(64) void moe_align_wave_kernel(const int* __restrict__ ids, const float* __restrict__ gates,
                                                             int* __restrict__ offsets, int* __restrict__ sorted_token,
@@ -709,7 +708,10 @@ static int launch_logits(const float* h, const float* w, float* logits, int N, i
 
 static int launch_align(const int* ids, const float* gates, int* offsets, int* sorted_token, float* sorted_gate,
                         int* inv, int M, int E, int k, int extra, int inv_ld, hipStream_t s) {
-  if (M <= 256 && E <= 63) {
+  // A wavefront looks at all its pairs for every expert; moe_align_kernel's thousand threads share them and meet at eight
+  // barriers.  Threads | wavefront, us: 64 pairs of 8 experts 2.9 | 2.3, of 32 3.8 | 3.6, of 48 5.1 | 5.4; 128 of 8 3.1 | 2.6, of 16
+  // 3.6 | 3.2; 256 of 8 3.5 | 3.1, of 16 3.6 | 4.1, of 32 4.9 | 6.1, of 63 7.0 | 9.7.
+  if (M <= 256 && (M + 63) / 64 * E <= 40) {
 #define WAVE(R_) \
   hipLaunchKernelGGL(moe_align_wave_kernel<R_>, dim3(1), dim3(64), 0, s, ids, gates, offsets, sorted_token, sorted_gate, inv, M, E, \
                      k, extra, inv_ld)

@@ -979,6 +979,21 @@ def test_moe_experts_with_128_experts_most_of_them_empty_or_nearly(ops, ref, n):
     _assert_close_to_scale(normed, ref_normed, dt)
 
 
+@pytest.mark.parametrize("n,k,e", [(64, 1, 40), (64, 1, 41), (65, 1, 20), (32, 4, 20), (64, 2, 21), (43, 3, 13), (64, 3, 14), (128, 2, 10),
+                                   (256, 1, 11), (257, 1, 3), (1, 1, 1)])
+def test_moe_align_at_the_edges_of_one_wavefront(ops, n, k, e):
+    """As many pairs and experts as one wavefront groups, and one more of either; choices beyond the experts have no row."""
+    ids = torch.randint(0, e + 2, (n, k), generator=torch.Generator().manual_seed(n)).int()
+    gates = _rand(n, k, seed=5)
+    off, tok, gate, inv = (t.cpu() for t in ops.moe_align(ids.to(DEV), gates, e, extra_group=True, note_extra=True))
+    flat, order = ids.reshape(-1), [int(r) for r in torch.argsort(ids.reshape(-1), stable=True) if ids.reshape(-1)[r] < e]
+    assert off.tolist() == [sum(int(f < i) for f in flat) for i in range(e + 1)] + [len(order) + n]
+    assert tok.tolist()[: len(order) + n] == [r // k for r in order] + list(range(n))
+    assert torch.equal(gate[: len(order)], gates.cpu().reshape(-1)[order]) and bool((gate[len(order): len(order) + n] == 1).all())
+    row = {r: i for i, r in enumerate(order)}
+    assert inv.view(n, k + 1).tolist() == [[row.get(t * k + j, -1) for j in range(k)] + [len(order) + t] for t in range(n)]
+
+
 def test_moe_align_is_a_stable_grouping(ops):
     g = torch.Generator().manual_seed(0)
     ids = torch.randint(0, 7, (300, 2), generator=g).to(torch.int32).to(DEV)
