@@ -2486,8 +2486,9 @@ class HipOps:
         blocks are one round, and the router, which every block reads for itself through one first-level cache, is small.
         Separate | one, us with the grouping: 8 experts of 2,048, one token 6.6 | 6.3, 256 10.9 | 9.2 (512 in two launches
         12.8); 10 of 4,096, one token 7.4 | 7.9, 17 9.8 | 8.5, 256 12.7 | 10.9; 16 of 5,120, 17 tokens 10.2 | 12.0, 128 13.0 |
-        13.6."""
-        return (n <= HipOps.CHOOSE_TOKENS and experts <= HipOps.NORM_CHOOSE_EXPERTS and d % 4 == 0
+        13.6.  A block with more than ten wavefronts is there later, which few tokens wait for: 16 experts of 1,032, one token
+        7.7 | 8.1, 4 7.9 | 8.7, 8 8.5 | 8.8, 16 9.0 | 8.8."""
+        return (n <= HipOps.CHOOSE_TOKENS and experts <= (10 if n < 16 else HipOps.NORM_CHOOSE_EXPERTS) and d % 4 == 0
                 and d * experts <= (24576 if n < 16 else 40960))
 
     @staticmethod

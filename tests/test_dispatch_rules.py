@@ -190,3 +190,9 @@ def test_many_rows_of_float32_with_a_short_k():
     sizes = [(777, 16384, 96), (2048, 5120, 96), (777, 16384, 2048), (1554, 2048, 8192), (512, 4096, 4096)]
     assert [HipOps.split_ranges(*s, False, 256) > 0 for s in sizes] == [False, False, True, True, True]
     assert HipOps.split_ranges(1024, 7168, 96, True, 256) == 1  # (the activation is a pass of its own behind the library's)
+
+
+@pytest.mark.parametrize("n, d, experts, one", [(1, 2048, 10, True), (1, 1032, 10, True), (1, 1032, 11, False), (15, 512, 16, False), (16, 512, 16, True),
+                                                (16, 2048, 16, True), (15, 2460, 10, False), (256, 2560, 16, True), (257, 64, 2, False), (1, 62, 2, False)])
+def test_logits_and_choice_in_one_launch_by_size(n, d, experts, one):
+    assert HipOps.choose_by_token(n, d, experts) == one
