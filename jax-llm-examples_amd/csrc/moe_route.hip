@@ -579,7 +579,8 @@ __global__ __launch_bounds__(256) void norm_route_kernel(const float* __restrict
 // other), grouping 1.8.  Here all tokens are chosen for at once, the router's first rows come while the token's row is added and
 // normed, and one wavefront groups in registers.  norm_route_kernel | this, us, 10 experts: 16 tokens of 2,048 19.0 | 13.5, 32
 // 30.0 | 15.0; 16 of 4,096 21.6 | 16.3; 8 of 3,072, 16 experts 17.2 | 14.4; 16 of 6,144, 8 experts 22.8 | 16.8; but a lone token,
-// whose experts are shared out over compute units there, 9.7 | 10.3, and 4 of 4,096, 16 experts 13.5 | 13.8.
+// whose experts are shared out over compute units there, 9.7 | 10.3, and 4 of 4,096, 16 experts 13.5 | 13.8; nor up to 8 whose rows
+// with more than 8 experts are long: 5 of 8,192, 10 experts 16.1 | 17.5, 8 16.7 | 17.6, 16 19.6 | 17.6.
 template <typename DT, typename OT, int CPT, int EPW>
 __global__ __launch_bounds__(256) void norm_route_token_kernel(const float* __restrict__ x, Delta<DT> delta,
                                                                const float* __restrict__ w, float eps,
@@ -824,7 +825,7 @@ JLE_API int jle_norm_route(const float* x, int delta_kind, const void* delta, co
                      router, logits, ids, gates, offsets, sorted_token, sorted_gate, inv, ticket, N, D, E, k,    \
                      extra_group ? N : 0, choice, experts)
   // (the same bits: which of the two is a question of time alone)
-  const bool by_token = scored && E <= kTokenExperts && N > 4 && N * k <= 64;
+  const bool by_token = scored && E <= kTokenExperts && N > (E > 8 && D > 4096 ? 8 : 4) && N * k <= 64;
 #define LAUNCH_T(DT, OT, CPT, EPW)                                                                               \
   hipLaunchKernelGGL((norm_route_token_kernel<DT, OT, CPT, EPW>), dim3(N), b, D * sizeof(float), s, x, dl, w, eps, x_out, \
                      (OT*)h_out, router, logits, ids, gates, offsets, sorted_token, sorted_gate, inv, ticket, N, D, E, k, \

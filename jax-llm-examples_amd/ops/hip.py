@@ -2444,8 +2444,7 @@ class HipOps:
         how = (0 if groups is None else int(groups), 0 if groups is None else int(keep_groups), int(group_terms),
                1 if scores == "softmax" else 0, -1.0 if normalize is None else float(normalize), float(weight_scale))
         if isinstance(h32, PendingNorm):
-            most = self.NORM_CHOOSE_TOKENS // top_k if e <= self.NORM_CHOOSE_EXPERTS else self.NORM_CHOOSE_ROWS
-            fused = None if h32.done or hasattr(h32.delta, "terms") or n > max(most, self.NORM_CHOOSE_ROWS) else \
+            fused = None if h32.done or hasattr(h32.delta, "terms") or n > self.norm_choose_rows(d, e, top_k) else \
                 self._norm_route(h32, router, top_k, scored=(experts, correction, how, extra_group))
             if fused is not None:
                 ids, weights, _, grouping = fused
@@ -2475,10 +2474,19 @@ class HipOps:
         return ids, weights, self.moe_align(ids, weights, experts, extra_group=extra_group, note_extra=extra_group)
 
     NORM_CHOOSE_ROWS = 16  # up to here the choice by scores is made in the launch that norms the rows (whose last block
-    # chooses for all tokens: 17 us at 8 tokens, 52 at 64, where the separate launches take 22); of up to 16 experts and 64
-    # choices every token's own block chooses (15 us at 32 tokens)
+    # chooses for all tokens: 17 us at 8 tokens, 52 at 64, where the separate launches take 22)
     NORM_CHOOSE_EXPERTS, NORM_CHOOSE_TOKENS = 16, 64
     CHOOSE_TOKENS = 256
+
+    @staticmethod
+    def norm_choose_rows(d: int, experts: int, top_k: int) -> int:
+        """Up to how many tokens the choice by scores is made in the launch that norms them: 16, and with up to 16 experts, where
+        every token's own block chooses, as many as have 64 choices (15 us at 32 tokens) unless more than 8 experts' rows are
+        longer than 4,096, which a block then waits for: separate launches | one, us, two of 10 experts of 8,192, 17 tokens
+        16.1 | 17.6, 32 15.8 | 17.8, of 5,120, 32 14.0 | 14.7; two of 16 of 8,192, 32 17.4 | 19.1; but two of 8 of 8,192, 32
+        16.0 | 14.6, of 16 of 4,096, 32 14.3 | 13.5."""
+        fits = experts <= HipOps.NORM_CHOOSE_EXPERTS and (experts <= 8 or d <= 4096)
+        return max(HipOps.NORM_CHOOSE_ROWS, HipOps.NORM_CHOOSE_TOKENS // top_k if fits else 0)
 
     @staticmethod
     def choose_by_token(n: int, d: int, experts: int) -> bool:

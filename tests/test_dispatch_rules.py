@@ -196,3 +196,9 @@ def test_many_rows_of_float32_with_a_short_k():
                                                 (16, 2048, 16, True), (15, 2460, 10, False), (256, 2560, 16, True), (257, 64, 2, False), (1, 62, 2, False)])
 def test_logits_and_choice_in_one_launch_by_size(n, d, experts, one):
     assert HipOps.choose_by_token(n, d, experts) == one
+
+
+@pytest.mark.parametrize("d, experts, top_k, rows", [(2048, 10, 2, 32), (4096, 16, 1, 64), (4104, 16, 1, 16), (8192, 8, 2, 32), (8192, 9, 2, 16),
+                                                     (2048, 17, 1, 16), (2048, 16, 8, 16)])
+def test_rows_normed_and_chosen_for_in_one_launch(d, experts, top_k, rows):
+    assert HipOps.norm_choose_rows(d, experts, top_k) == rows

@@ -397,7 +397,8 @@ def test_attention_with_kept_tokens_of_layers_with_other_heads_in_one_step(ops, 
 
 @pytest.mark.parametrize("n,d,e,k,experts,groups", [
     (5, 1032, 2, 1, 2, None), (5, 2048, 10, 2, 8, (5, 3)), (8, 2056, 16, 8, 16, (4, 2)), (16, 2048, 9, 4, 8, None),
-    (17, 4096, 16, 3, 12, (8, 5)), (32, 2048, 10, 2, 8, (5, 3)), (64, 8192, 8, 1, 8, None), (64, 4104, 16, 1, 16, (2, 1))])
+    (17, 4096, 16, 3, 12, (8, 5)), (32, 2048, 10, 2, 8, (5, 3)), (64, 8192, 8, 1, 8, None), (64, 4096, 16, 1, 16, (2, 1)),
+    (8, 4104, 9, 2, 8, None), (9, 4104, 9, 2, 8, None), (16, 8192, 16, 4, 12, (4, 2))])
 @pytest.mark.parametrize("extra", [False, True])
 def test_choices_by_scores_token_by_token_equal_the_separate_kernels(ops, n, d, e, k, experts, groups, extra):
     """A block a token with all its experts (up to 16, up to 64 choices): the bits of norm, logits, choice and grouping as
