@@ -58,6 +58,12 @@ __device__ __forceinline__ void load_to_lds16(const void* base, uint32_t byte_of
   asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1\n" ::"v"(byte_off), "s"(base), "s"(lds_addr) : "memory");
 }
 
+// max(v, 0)^2; what is not a number stays so (fmaxf would give the other operand)
+__device__ __forceinline__ float relu2(float v) {
+  const float u = v > 0.f || v != v ? v : 0.f;
+  return u * u;
+}
+
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);

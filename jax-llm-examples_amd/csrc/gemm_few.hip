@@ -224,10 +224,7 @@ __global__ __launch_bounds__(kWaves * 64) void gemm_few_kernel(FewArgs p) {
       }
     } else if (p.act == 1) {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const float u = fmaxf(rounded<OutT>(v[j]), 0.f);
-        v[j] = u * u;
-      }
+      for (int j = 0; j < 4; ++j) v[j] = relu2(rounded<OutT>(v[j]));
     }
     const int c = n0 + i * 16 + 4 * g;
     OutT* y = (OutT*)p.Y + (size_t)t * width + c;

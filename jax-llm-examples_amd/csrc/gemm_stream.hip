@@ -126,13 +126,6 @@ __device__ __forceinline__ int piece_stage(int piece, int cuts, int nstage) { re
 // Rows of a tile: a group's rows as even as multiples of 32 allow.
 __device__ __forceinline__ int rows_a_tile(int rows, int tiles) { return ((rows + tiles - 1) / tiles + 31) / 32 * 32; }
 
-// max(., 0)^2 of a sum as it would be stored
-template <typename OutT>
-__device__ __forceinline__ float relu2(float v) {
-  const float u = fmaxf(Num<OutT>::round(v), 0.f);
-  return u * u;
-}
-
 // A lane's sums of a row, four neighbouring rows of two tiles of W, scaled and stored.
 template <bool SWIGLU, typename OutT>
 __device__ __forceinline__ void finish_pair(OutT* __restrict__ Y, int t, const float* __restrict__ scale, int act, f32x4 a0,
@@ -149,8 +142,8 @@ __device__ __forceinline__ void finish_pair(OutT* __restrict__ Y, int t, const f
     if (act) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        a0[i] = relu2<OutT>(a0[i]);
-        a1[i] = relu2<OutT>(a1[i]);
+        a0[i] = relu2(Num<OutT>::round(a0[i]));
+        a1[i] = relu2(Num<OutT>::round(a1[i]));
       }
     }
     store4<OutT>(Y + (size_t)t * Nout + t0 * 16 + 4 * g, a0[0], a0[1], a0[2], a0[3]);
@@ -581,7 +574,7 @@ __device__ __forceinline__ void wide_block(const bf16_t* __restrict__ X, const b
           y[e] = gate / (1.0f + expf(-gate)) * up;
         } else {
           y[e] = acc[i][n][e] * sc;
-          if (act) y[e] = relu2<bf16_t>(y[e]);
+          if (act) y[e] = relu2(Num<bf16_t>::round(y[e]));
         }
       }
       store4<bf16_t>(Y + (size_t)t * (SWIGLU ? half : Nout) + tile * 16 + 4 * g, y[0], y[1], y[2], y[3]);

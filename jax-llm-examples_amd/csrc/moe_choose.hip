@@ -57,8 +57,7 @@ template <typename T>
 __global__ __launch_bounds__(256) void relu2_kernel(const T* __restrict__ x, T* __restrict__ y, long long count) {
   const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
   if (i >= count) return;
-  const float v = fmaxf(Num<T>::load(x + i), 0.f);
-  Num<T>::store(y + i, v * v);
+  Num<T>::store(y + i, relu2(Num<T>::load(x + i)));
 }
 
 }  // namespace

@@ -1451,6 +1451,20 @@ def test_wide_tiles_of_the_weight_streaming_product(ops, counts, nout, k, swiglu
     assert torch.equal(*got)
 
 
+@pytest.mark.parametrize("dt", DT)
+def test_squared_relu_keeps_what_is_not_a_number(ops, dt):
+    """Of plain numbers, infinities and NaN what torch gives, as a launch of its own and behind the product of a few rows."""
+    x = torch.cat([_rand(300, dt=dt, seed=1), torch.tensor([0.0, -0.0, math.inf, -math.inf, math.nan, -math.nan], dtype=dt, device=DEV)])
+    got, want = ops.relu2(x), (torch.relu(x.float()) ** 2).to(dt)
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.nan_to_num(7.0), want.nan_to_num(7.0))
+    rows, w = _rand(7, 256, dt=torch.bfloat16, seed=2), _rand(2, 64, 256, dt=torch.bfloat16, seed=3)
+    rows[4, 100] = math.nan
+    off = torch.tensor([0, 3, 7], dtype=torch.int32, device=DEV)
+    got = ops.gemm_few(rows, w, offsets=off, relu2=True)
+    assert bool(got[4].isnan().all())
+    assert torch.equal(got.isnan().any(1), torch.arange(7, device=DEV) == 4) and bool((got[5] > 0).any())
+
+
 @pytest.mark.parametrize("way", ["passes", "cut", "wide", "half"])
 def test_squared_relu_behind_the_weight_streaming_product(ops, monkeypatch, way):
     """The bits of the product and the activation as launches of their own, by every kernel that takes such rows."""
@@ -1465,7 +1479,9 @@ def test_squared_relu_behind_the_weight_streaming_product(ops, monkeypatch, way)
     monkeypatch.setattr(ops, "stream_cuts", lambda *a: (2, 3) if way == "cut" else (0, 1))
     got = ops.gemm_stream(x, w, offsets=off, relu2=True)
     want = ops.relu2(ops.gemm_stream(x, w, offsets=off))
-    assert torch.equal(got.view(torch.int16), want.view(torch.int16)) and bool((got >= 0).sum() > 0)
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16)) and bool(got[5].isnan().all()) and not got[9].any()
+    others = torch.cat([got[:5], got[10:]])
+    assert not others.isnan().any() and bool((others > 0).any()) and bool((others == 0).any())
 
 
 @pytest.mark.parametrize("counts,nout,k,cut,cuts", [
