@@ -400,7 +400,7 @@ def test_attention_with_kept_tokens_of_layers_with_other_heads_in_one_step(ops, 
     (17, 4096, 16, 3, 12, (8, 5)), (32, 2048, 10, 2, 8, (5, 3)), (64, 8192, 8, 1, 8, None), (64, 4096, 16, 1, 16, (2, 1)),
     (8, 4104, 9, 2, 8, None), (9, 4104, 9, 2, 8, None), (16, 8192, 16, 4, 12, (4, 2))])
 @pytest.mark.parametrize("extra", [False, True])
-def test_choices_by_scores_token_by_token_equal_the_separate_kernels(ops, n, d, e, k, experts, groups, extra):
+def test_choices_by_scores_token_by_token_equal_the_separate_kernels(ops, monkeypatch, n, d, e, k, experts, groups, extra):
     """A block a token with all its experts (up to 16, up to 64 choices): the bits of norm, logits, choice and grouping as
     launches of their own, launch after launch, with equal scores, a token that is not finite and identity experts."""
     x, w, router = _rand(n, d, seed=1), _rand(d, seed=2) + 1.0, _rand(e, d, scale=0.05, seed=3)
@@ -415,10 +415,10 @@ def test_choices_by_scores_token_by_token_equal_the_separate_kernels(ops, n, d, 
         args = dict(groups=g, keep_groups=keep, group_terms=1, scores=scores, normalize=1e-20 if extra else None, weight_scale=1.5,
                     num_experts=experts, extra_group=extra)
         for _ in range(2):
-            ops._call = lambda name, *a: (calls.append(name), inner(name, *a))[1]
-            pending = ops.defer_norm(x.clone(), delta, w, 1e-5, torch.bfloat16)
-            ids, weights, grouping = ops.moe_choose(pending, router, correction, k, **args)
-            del ops._call
+            with monkeypatch.context() as m:
+                m.setattr(ops, "_call", lambda name, *a: (calls.append(name), inner(name, *a))[1])
+                pending = ops.defer_norm(x.clone(), delta, w, 1e-5, torch.bfloat16)
+                ids, weights, grouping = ops.moe_choose(pending, router, correction, k, **args)
             assert calls[-1] == "jle_norm_route"
             h, h32 = ops.add_rmsnorm(x.clone(), delta, w, 1e-5, torch.bfloat16, want32=True)
             want = ops.moe_choose(h32, router, correction, k, **args)
@@ -1433,7 +1433,7 @@ def test_weight_streaming_product_of_fuller_groups(ops, counts, nout, k, tiled):
     ([224, 225, 256, 257, 512, 513, 700], 544, 768, True),  # one, two and three tiles of rows; gate and up
     ([3, 0, 280] * 50, 64, 256, False),                     # more groups than a look takes
     ([256], 2304, 256, True)])                              # more than eight blocks of W
-def test_wide_tiles_of_the_weight_streaming_product(ops, counts, nout, k, swiglu):
+def test_wide_tiles_of_the_weight_streaming_product(ops, monkeypatch, counts, nout, k, swiglu):
     """The kernel for many rows a group gives the bits of the one that takes them in passes (the same sums in the same
     order), with the rows gathered and scaled; that one is tested against the general product elsewhere."""
     from jax_llm_examples_amd.ops.layout import tile_
@@ -1445,9 +1445,8 @@ def test_wide_tiles_of_the_weight_streaming_product(ops, counts, nout, k, swiglu
     scale = _rand(m, seed=4)
     got = []
     for wide in (False, True):
-        ops.stream_wide = lambda *a, wide=wide: wide
+        monkeypatch.setattr(ops, "stream_wide", lambda *a, wide=wide: wide)
         got.append(ops.gemm_stream(x, w, offsets=off, a_rows=rows, scale=scale, swiglu=swiglu, rows=m))
-    del ops.stream_wide
     assert torch.equal(*got)
 
 
@@ -1570,7 +1569,7 @@ def test_passes_of_the_weight_streaming_product_against_64_bits(ops, monkeypatch
         o += c
 
 
-def test_rows_off_their_16_bytes_take_the_passes(ops):
+def test_rows_off_their_16_bytes_take_the_passes(ops, monkeypatch):
     """Rows that begin at 8 bytes, where the wide tiles want 16."""
     from jax_llm_examples_amd.ops.layout import tile_
     x, w = _rand(400, 256, dt=torch.bfloat16, seed=1), _rand(1, 64, 256, dt=torch.bfloat16, scale=0.1, seed=2)
@@ -1578,9 +1577,8 @@ def test_rows_off_their_16_bytes_take_the_passes(ops):
     off = torch.tensor([0, 400], dtype=torch.int32, device=DEV)
     elsewhere = torch.empty(400 * 256 + 4, dtype=torch.bfloat16, device=DEV)[4:].view(400, 256)
     elsewhere.copy_(x)
-    ops.stream_wide = lambda *a: True
+    monkeypatch.setattr(ops, "stream_wide", lambda *a: True)
     got = [ops.gemm_stream(t, w, offsets=off) for t in (x, elsewhere)]
-    del ops.stream_wide
     assert torch.equal(*got)
 
 
