@@ -1840,29 +1840,31 @@ class HipOps:
     def stream_wide(rows: int, groups: int, row_blocks: int) -> bool:
         """Which of ``gemm_stream.hip``'s kernels takes ``rows`` rows in ``groups`` groups (``row_blocks`` blocks of 256 rows
         of W a group): passes of 192 rows or wide tiles of 256.  A block fills a compute unit, so what counts is how many
-        rounds of blocks there are on the 256 compute units and how long one takes; measured per stage of 64 k,
-        microseconds: passes 0.9 + 0.0037 a row, tiles 0.95 + 0.003.  A group's rows are taken to scatter about their mean by
-        its root: how they are shared out is known on the device only.  With fewer than WIDE_GROUPS groups one that is far
-        fuller than the others is what the launch takes, and is better cut in more pieces: 2 groups of 4,096 x 2,048 with 300
-        rows on average in even groups 43 | 38, with 90 and 510 42 | 53; 4 with 40 % of the rows in one 45 | 55.  Over 180
-        sizes of 8, 16 and 64 groups, even, from 0.3 to 1.7 of the mean, and one with 40 % of the rows, the choice is 15 %
-        faster than passes on the average and 2 % from the better of the two, at worst 13 % slower than passes (groups of
-        192 rows each, what a pass holds; beside that 8 %: one group far fuller at 192 on average).  Both sides measured (passes | tiles,
-        us): 8 groups of 14,336 x 4,096 gate and up with 192 rows each 286 | 226, 256 368 | 309, 410 529 | 401, 700
-        743 | 643; of 4,096 x 7,168 with 192 152 | 154, 410 275 | 163, 512 281 | 298, 700 302 | 329; of 8,192 x 2,048 gate
-        and up with 410 152 | 121, 512 152 | 167; 16 of 16,384 x 5,120 with 160 523 | 541, 410 1,508 | 1,023, 700
-        1,920 | 1,709."""
+        rounds of blocks there are on the 256 compute units and how long one takes; measured per stage of 64 k, microseconds:
+        passes 0.9 + 0.0037 a row, tiles 0.95 + 0.003.  Fewer than 16 row blocks of tiles count in eights, as they are dealt to the
+        eight chiplets (of 10 groups of 3,072 x 3,072 with 384 rows half of the chiplets get two thirds: 80 | 147).  A group's rows
+        are taken to scatter about their mean by its root: how they are shared out is known on the device only.  With fewer than WIDE_GROUPS groups one that is far fuller than the others is what the launch takes, and is better cut in
+        more pieces: 2 groups of 4,096 x 2,048 with 300 rows on average in even groups 41 | 43, 40 % in one 45 | 59; 4 42 | 60.
+        Over 26 matrices of 8 to 128 groups with 48 to 900 rows each, even, drawn, and with 40 % of the rows in one group, the
+        choice between these and :meth:`stream_half`'s is 3 % from the best, and where it is not passes 7 % faster than these; at
+        worst 1.65 times their time (8 of 5,120 x 4,096 with 256, 40 % in one: 110 | 181; drawn 1.42 times, 32 of 1,024 x 2,048
+        with 176: 51 | 73).  Both sides measured (passes | tiles, us, drawn groups): 8 groups of 14,336 x 4,096 gate and up with 192 rows 264 | 232, 256
+        341 | 293, 410 494 | 409, 700 767 | 650; of 4,096 x 7,168 with 192 155 | 161, 410 267 | 198, 512 312 | 298, 700
+        348 | 351; of 8,192 x 2,048 gate and up with 410 151 | 127, 512 183 | 170; 16 of 16,384 x 5,120 with 160 551 | 579, 410
+        1,440 | 1,084, 700 2,117 | 1,780; of 5,120 x 8,192 with 300 557 | 505; 64 of 1,024 x 2,048 (four row blocks) with 192
+        114 | 142, 300 156 | 200; of 512 x 2,048 with 290 68 | 191."""
         mean = rows / groups
         if mean < HipOps.WIDE_GROUP_ROWS or groups < HipOps.WIDE_GROUPS:
             return False
 
-        def cost(most, start, a_row):
+        def cost(most, a_tile, start, a_row):
             tiles = sum(-(-max(1.0, mean + d * mean ** 0.5) // most) for d in (-1, 0, 1)) / 3
-            blocks = row_blocks * groups * tiles
+            blocks = a_tile * groups * tiles
             rounds = -(-blocks // 256) if blocks < 1024 else blocks / 256 + 0.5
             return rounds * (start + a_row * mean / tiles)
 
-        return cost(256, 0.95, 0.003) < cost(192, 0.9, 0.0037)
+        a_tile = -(-row_blocks // 8) * 8 if row_blocks < 16 else row_blocks
+        return cost(256, a_tile, 0.95, 0.003) < cost(192, row_blocks, 0.9, 0.0037)
 
     @staticmethod
     @functools.lru_cache(maxsize=4096)
@@ -1875,13 +1877,11 @@ class HipOps:
         (of groups of 256 rows of W all blocks are on two of them: 64 such groups up to 2.1 times the time of passes).  Few rows a group are
         the time of their weights' bytes.
 
-        Measured over 22 matrices, 8 to 128 groups and 24 means from 48 to 800 rows, each even, drawn, uneven by a quarter,
-        from 0.3 to 1.7 of the mean and with 40 % of the rows in one group: where these tiles are taken they are 12 % faster
-        than what else would be on the average, at worst 16 % slower (24 groups of 1,024 x 4,096 with 145 rows, 40 % in one).
-        Taken wherever even groups would fill one round or two, they were up to 67 % slower (8 of 4,096 x 7,168 with 256 rows:
-        even 199 | 168 us, 40 % in one 154 | 257).  What else would be | these, us, even and with 40 % in one: 8 of 2,048 x 4,096
-        with 128 rows 62 | 59 and 79 | 67, 230 84 | 74 and 79 | 72, 300 80 | 64 and 100 | 73; 8 of 1,024 x 8,192 with 512
-        152 | 133 and 151 | 147."""
+        Measured as :meth:`stream_wide` is: where these tiles are taken they are 7 % faster than passes on the average, at worst
+        24 % slower (16 groups of 1,024 x 2,048 with 256 rows, two passes of 128: 37 | 46 us).  Taken wherever even groups would
+        fill one round or two, they were up to 67 % slower.  Passes | these, us, drawn and with 40 % in one: 8 of 2,048 x 4,096 with
+        128 rows 62 | 57 and 69 | 63, 230 63 | 70 and 80 | 68, 300 81 | 80 and 82 | 70; 8 of 1,024 x 8,192 with 512 147 | 141 and
+        147 | 140; 16 of 1,024 x 2,048 with 190 48 | 42 and 48 | 45; but 8 of 4,096 x 7,168 with 256 160 | 166 and 151 | 214."""
         slots = -(-row_blocks // 8) * 8 * groups
         mean = rows / groups
         return groups >= HipOps.WIDE_GROUPS and mean >= 90 and slots <= 192 and slots * (mean / 288 + 0.5) <= 224

@@ -103,6 +103,13 @@ def test_few_groups_stay_with_passes(groups, rows, blocks, wide):
     assert HipOps.stream_wide(rows * groups, groups, blocks) == wide
 
 
+@pytest.mark.parametrize("groups, rows, blocks, wide", [(64, 290, 2, False), (32, 330, 2, False), (24, 290, 4, False), (64, 192, 4, False), (128, 176, 3, False),
+                                                        (16, 300, 20, True), (8, 410, 16, True), (16, 700, 64, True), (10, 384, 12, False), (16, 512, 20, True), (16, 160, 64, False)])
+def test_wide_tiles_where_their_row_blocks_reach_every_chiplet(groups, rows, blocks, wide):
+    """Few row blocks of wide tiles are on a few of the eight chiplets only, where passes are dealt to all of them."""
+    assert HipOps.stream_wide(rows * groups, groups, blocks) == wide
+
+
 @pytest.mark.parametrize("groups, rows, blocks, half", [
     (8, 512, 32, False), (8, 512, 16, False), (8, 410, 32, False), (8, 190, 32, False), (8, 330, 32, False), (8, 128, 32, False),
     (8, 64, 32, False), (8, 64, 16, False), (16, 128, 40, False), (16, 256, 40, False), (4, 512, 16, False), (8, 700, 16, False),
