@@ -435,8 +435,8 @@ __global__ __launch_bounds__(WAVES * 64) void add_pieces_kernel(StreamArgs p) {
 // memory serves 64 operations.  With one wavefront a SIMD nothing hides a wait, so there is none: a B operand is asked for
 // four products of tiles before its use, the barrier that says that the next stage's rows have come (and that the ring's
 // oldest place is free) stands in the middle of a stage, and the next stage's first operands are read at this one's end.
-// 16 groups of 16,384 x 5,120 (gate and up) with 410 rows each: 1,023 us (1.08 PFLOP/s) against 1,508 in passes of 192; 8 of
-// 4,096 x 7,168 163 (1.18) against 275.  (With eight wavefronts of 64 x half the rows and the weights through shared memory
+// 16 groups of 16,384 x 5,120 (gate and up) with 410 rows each: 1,080 us (1.02 PFLOP/s) against 1,474 in passes of 192; 8 of
+// 4,096 x 7,168 194 (0.99) against 269.  (With eight wavefronts of 64 x half the rows and the weights through shared memory
 // too 422 and 188 at 8 groups: reading and bringing in together took shared memory as long as the products.)
 // HALF (plain products): a block takes 128 rows of W and up to 288 of X, its wavefronts in twos by twos, 64 rows of W and half
 // of X each.  It reads twice as much for a product, but where blocks of 256 would fill a part of the compute units or of their

@@ -1111,18 +1111,19 @@ class HipOps:
     def f32_tiles_pay(rows: int, n: int, k: int, gated: bool, units: int = 256) -> bool:
         """Whether a dense float32 product goes through the kernel of the experts' few rows, a block for 16 columns and 16 rows
         (``gemm_f32.hip``; on the float32 matrix instructions, errors against 64 bits from a third to three quarters of the
-        library's).  A block takes 4 us and 3 more per 1,024 of k however few blocks there are, so it is the faster one while its
-        blocks are one round of the ``units`` compute units, and with more than 1,024 of k only where the library, which shares
-        k out among blocks while the matrix is small, no longer does.  The library's is the faster one too for up to 16 rows of
-        matrices with 512 columns and more and a short k, where both are mostly launch.  The library's | this, us on the
-        device, launches recorded: 64 x 64, 32 rows 3.9 | 3.7, 128 rows 5.8 | 3.8; 512 x 256, 16 rows 4.0 | 5.0, 64 rows 5.6 | 5.1;
-        512 x 640, 16 rows 6.5 | 5.6; 1,024 x 1,024, 16 rows 8.4 | 6.0, 64 rows 8.5 | 7.1, 128 rows (512 blocks) 8.8 | 9.7; 2,048 x 1,024,
-        48 rows (384 blocks) 8.7 | 9.8; 32 x 2,048, 16 rows 8.3 | 8.6, 64 rows 9.2 | 11.2; 1,024 x 2,048, 64 rows 9.1 | 11.3; 1,024 x
-        1,536, 64 rows 7.8 | 10.4; 1,536 x 2,048, 32 rows 12.3 | 11.3; 2,048 x 2,048, 16 rows 12.2 | 11.5, 32 rows 12.7 | 11.9;
-        2,048 x 1,536, 16 rows 9.8 | 9.8; 4,096 x 1,152, 16 rows 10.2 | 10.0.  Gate and up, with the activation: 512 x 64, 32 rows
-        5.9 | 4.6; 512 x 256, 16 rows 5.9 | 6.4, 64 rows 7.5 | 6.5; 2,048 x 1,024, 64 rows 11.9 | 9.3; 512 x 2,048, 64 rows 11.1 | 14.5;
-        2,048 x 1,536, 32 rows 12.5 | 13.7; 2,048 x 2,048, 32 rows 14.9 | 15.0, 64 rows 17.0 | 15.3; 4,096 x 1,152, 16 rows 12.2 | 11.4.
-        (And the library's product costs the host 20 us a call, this one 7.)"""
+        library's). A block takes 4 us and 3 more per 1,024 of k however few blocks there are, so it is the faster one while
+        its blocks are one round of the ``units`` compute units, and with more than 1,024 of k only where the library, which
+        shares k out among blocks while the matrix is small, no longer does. The library's is the faster one too for up to 16
+        rows of matrices with 512 columns and more and a short k, where both are mostly launch. The library's | this, us on the
+        device, launches recorded: 64 x 64, 32 rows 3.9 | 3.7, 128 rows 5.8 | 3.8; 512 x 256, 16 rows 4.0 | 5.0, 64 rows 5.6 |
+        5.1; 512 x 640, 16 rows 6.5 | 5.6; 1,024 x 1,024, 16 rows 8.4 | 6.0, 64 rows 8.5 | 7.1, 128 rows (512 blocks) 8.8 |
+        9.7; 2,048 x 1,024, 48 rows (384 blocks) 8.7 | 9.8; 32 x 2,048, 16 rows 8.3 | 8.6, 64 rows 9.2 | 11.2; 1,024 x 2,048,
+        64 rows 9.1 | 11.3; 1,024 x 1,536, 64 rows 7.8 | 10.4; 1,536 x 2,048, 32 rows 12.3 | 11.3; 2,048 x 2,048, 16 rows 12.2
+        | 11.5, 32 rows 12.7 | 11.9; 2,048 x 1,536, 16 rows 9.8 | 9.8; 4,096 x 1,152, 16 rows 10.2 | 10.0. Gate and up, with
+        the activation: 512 x 64, 32 rows 5.9 | 4.6; 512 x 256, 16 rows 5.9 | 6.4, 64 rows 7.5 | 6.5; 2,048 x 1,024, 64 rows
+        11.9 | 9.3; 512 x 2,048, 64 rows 11.1 | 14.5; 2,048 x 1,536, 32 rows 12.5 | 13.7; 2,048 x 2,048, 32 rows 14.9 | 15.0,
+        64 rows 17.0 | 15.3; 4,096 x 1,152, 16 rows 12.2 | 11.4. (And the library's product costs the host 20 us a call, this
+        one 7.)"""
         if rows > HipOps.F32_SKINNY_ROWS or k > 2048 or -(-(n // 2 if gated else n) // 16) * -(-rows // 16) > units:
             return False
         if k > 1024:
@@ -1842,17 +1843,18 @@ class HipOps:
         of W a group): passes of 192 rows or wide tiles of 256.  A block fills a compute unit, so what counts is how many
         rounds of blocks there are on the 256 compute units and how long one takes; measured per stage of 64 k, microseconds:
         passes 0.9 + 0.0037 a row, tiles 0.95 + 0.003.  Fewer than 16 row blocks of tiles count in eights, as they are dealt to the
-        eight chiplets (of 10 groups of 3,072 x 3,072 with 384 rows half of the chiplets get two thirds: 80 | 147).  A group's rows
-        are taken to scatter about their mean by its root: how they are shared out is known on the device only.  With fewer than WIDE_GROUPS groups one that is far fuller than the others is what the launch takes, and is better cut in
-        more pieces: 2 groups of 4,096 x 2,048 with 300 rows on average in even groups 41 | 43, 40 % in one 45 | 59; 4 42 | 60.
-        Over 26 matrices of 8 to 128 groups with 48 to 900 rows each, even, drawn, and with 40 % of the rows in one group, the
-        choice between these and :meth:`stream_half`'s is 3 % from the best, and where it is not passes 7 % faster than these; at
-        worst 1.65 times their time (8 of 5,120 x 4,096 with 256, 40 % in one: 110 | 181; drawn 1.42 times, 32 of 1,024 x 2,048
-        with 176: 51 | 73).  Both sides measured (passes | tiles, us, drawn groups): 8 groups of 14,336 x 4,096 gate and up with 192 rows 264 | 232, 256
-        341 | 293, 410 494 | 409, 700 767 | 650; of 4,096 x 7,168 with 192 155 | 161, 410 267 | 198, 512 312 | 298, 700
-        348 | 351; of 8,192 x 2,048 gate and up with 410 151 | 127, 512 183 | 170; 16 of 16,384 x 5,120 with 160 551 | 579, 410
-        1,440 | 1,084, 700 2,117 | 1,780; of 5,120 x 8,192 with 300 557 | 505; 64 of 1,024 x 2,048 (four row blocks) with 192
-        114 | 142, 300 156 | 200; of 512 x 2,048 with 290 68 | 191."""
+        eight chiplets (of 10 groups of 3,072 x 3,072 with 384 rows half of the chiplets get two thirds: 80 | 147). A group's
+        rows are taken to scatter about their mean by its root: how they are shared out is known on the device only. With fewer
+        than WIDE_GROUPS groups one that is far fuller than the others is what the launch takes, and is better cut in more
+        pieces: 2 groups of 4,096 x 2,048 with 300 rows on average in even groups 41 | 43, 40 % in one 45 | 59; 4 42 | 60. Over
+        26 matrices of 8 to 128 groups with 48 to 900 rows each, even, drawn, and with 40 % of the rows in one group, the
+        choice between these and :meth:`stream_half`'s is 3 % from the best, and where it is not passes it is 7 % faster than
+        they, at worst 1.65 times their time (8 of 5,120 x 4,096 with 256, 40 % in one: 110 | 181; drawn 1.42 times, 32 of 1,024 x
+        2,048 with 176: 51 | 73). Both sides measured (passes | tiles, us, drawn groups): 8 groups of 14,336 x 4,096 gate and
+        up with 192 rows 264 | 232, 256 341 | 293, 410 494 | 409, 700 767 | 650; of 4,096 x 7,168 with 192 155 | 161, 410 267 |
+        198, 512 312 | 298, 700 348 | 351; of 8,192 x 2,048 gate and up with 410 151 | 127, 512 183 | 170; 16 of 16,384 x 5,120
+        with 160 551 | 579, 410 1,440 | 1,084, 700 2,117 | 1,780; of 5,120 x 8,192 with 300 557 | 505; 64 of 1,024 x 2,048
+        (four row blocks) with 192 114 | 142, 300 156 | 200; of 512 x 2,048 with 290 68 | 191."""
         mean = rows / groups
         if mean < HipOps.WIDE_GROUP_ROWS or groups < HipOps.WIDE_GROUPS:
             return False
@@ -1874,8 +1876,7 @@ class HipOps:
         if all of them start together and is lost if one is left over.  So they have to fit one round of the 256 compute units
         however the rows are shared out, which is known on the device only: a group is taken to have half a tile more than its
         rows fill, and an eighth of the round stays free.  Row blocks count in eights, as they are dealt to the eight chiplets
-        (of groups of 256 rows of W all blocks are on two of them: 64 such groups up to 2.1 times the time of passes).  Few rows a group are
-        the time of their weights' bytes.
+        (of groups of 256 rows of W all blocks are on two of them).  Few rows a group are the time of their weights' bytes.
 
         Measured as :meth:`stream_wide` is: where these tiles are taken they are 7 % faster than passes on the average, at worst
         24 % slower (16 groups of 1,024 x 2,048 with 256 rows, two passes of 128: 37 | 46 us).  Taken wherever even groups would
