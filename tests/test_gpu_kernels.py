@@ -1542,7 +1542,8 @@ def test_experts_products_of_a_row_do_not_depend_on_how_the_others_are_shared_ou
 
 @pytest.mark.parametrize("counts,nout,k,swiglu", [
     ([5, 0, 192, 193, 31, 385], 272, 4096, False),   # several passes, two blocks of W, the second of one tile
-    ([190, 200, 260, 385, 193], 272, 512, False),    # two or three passes in every group
+    ([200, 190, 260, 385, 193], 272, 512, False),    # passes that differ from the first group's two by one: pass after pass
+    ([410, 577, 500], 2336, 256, True),              # the same with three and four, the last group's blocks in the last round
     ([190, 385, 260, 385, 193], 2048, 256, False),   # the same with blocks of W for every die
     ([100, 33, 64], 544, 4352, True),                # one pass a group
     ([3] * 257, 64, 4096, False),                    # more groups than compute units
