@@ -13,6 +13,7 @@ from typing import Optional
 
 import numpy as np
 import torch
+from torch.autograd import forward_ad
 
 from . import build as _build
 from .transfer import to_device
@@ -50,6 +51,7 @@ _SIGNATURES = {
                        _vp, _vp, _i, _i, _i, _i, _i, _vp, _vp, _i, _i, _vp, _i, _i, _i, _i, _f, _f, _vp],
     "jle_moe_align": [_vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _vp],
     "jle_moe_route_align": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _vp],
+    "jle_gemm_dense": [_vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _vp],
     "jle_gemm_generic": [_vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _vp],
     "jle_gemm_f32_skinny": [_vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _vp],
     "jle_gemm_f32_rows": [_vp, _vp, _vp, _i, _i, _i, _i, _vp],
@@ -225,6 +227,12 @@ def load_library(kernel_sources=None):
 
 def _p(t: Optional[torch.Tensor]):
     return None if t is None else t.data_ptr()
+
+
+def _watched() -> bool:
+    """Whether the operations are looked at while they run: derivatives in forward mode, function transforms, dispatch modes."""
+    return (forward_ad._current_level >= 0 or torch._C._functorch.peek_interpreter_stack() is not None
+            or torch._C._len_torch_dispatch_stack() > 0)
 
 
 class HipOps:
@@ -891,8 +899,8 @@ class HipOps:
         kr = torch.empty(rows, dr, dtype=q.dtype, device=q.device)
         self._call("jle_latent_expanded_gather", _p(latent_pages), _p(rope_pages), _p(block_table), block_table.shape[1],
                    _p(table), ns // 4, _p(c), _p(kr), r, dr, ps)
-        kn = torch.matmul(c, w_uk.t())  # [rows, H * nope]
-        vt = torch.matmul(w_uv, c.t())  # [H * value_dim, rows]
+        kn = self._product(c, w_uk)  # [rows, H * nope]
+        vt = self._product(w_uv, c)  # [H * value_dim, rows]
         out = torch.empty(n, H * dv, dtype=q.dtype, device=q.device)
         self._call("jle_latent_expanded_attention", _p(q), q.stride(0), _p(kn), _p(kr), _p(vt), rows, _p(out),
                    _p(positions), _p(table[ns:]), (table.numel() - ns) // 4, w, float(scale), H, _p(sink))
@@ -1131,8 +1139,8 @@ class HipOps:
         return gated or n < 512 or k >= 512 or rows > 16 and k >= 128
 
     def linear(self, h, w, out_dtype=None):
-        """``h @ w.T``: through the BLAS library; up to a few tens of bfloat16 rows (:meth:`_few`), and few or many float32
-        rows, through kernels of their own."""
+        """``h @ w.T``: up to a few tens of bfloat16 rows (:meth:`_few`), many of them (:meth:`dense_tile`), and few or many
+        float32 rows go through kernels of their own, others through the BLAS library."""
         h = self._rows(h)
         out = self._dense_float32(h, w)
         if out is not None:
@@ -1144,8 +1152,87 @@ class HipOps:
                 and w.dtype == torch.bfloat16 and w.shape[1] % 8 == 0 and h.is_contiguous() and w.is_contiguous()):
             out = self.gemm_skinny(h, w)
             return out if out_dtype is None or out_dtype == out.dtype else out.to(out_dtype)
-        out = torch.matmul(h, w.t())
+        out = self._product(h, w)
         return out if out_dtype is None or out_dtype == out.dtype else out.to(out_dtype)
+
+    # gemm_dense.hip's tiles, 32 rows of X by 32 of W: (how many blocks a compute unit takes, and of a launch the microseconds
+    # there are at all, a round of blocks, a round's stage of 64 k, and what that takes longer where all compute units have a block)
+    DENSE_TILES = {(8, 8): (1, -1.3, 9.2, 0.960, 0.375), (8, 7): (1, -1.8, 9.2, 0.886, 0.295), (8, 6): (1, -2.0, 9.2, 0.733, 0.256),
+                   (6, 8): (1, -0.9, 7.2, 0.783, 0.249), (8, 5): (1, -1.3, 7.6, 0.639, 0.215), (8, 4): (1, 0.2, 4.9, 0.546, 0.204),
+                   (6, 4): (1, 0.9, 3.4, 0.459, 0.153), (4, 5): (1, 1.3, 2.5, 0.457, 0.123), (4, 4): (2, 2.3, 0.7, 0.442, 0.503)}
+    DENSE_GATED_TILES = {(8, 8): (1, 2.5, 8.7, 1.019, 0.369), (8, 6): (1, 0.0, 8.3, 0.828, 0.216), (6, 8): (1, 2.7, 4.5, 0.925, 0.189),
+                         (8, 4): (1, 3.2, 2.5, 0.648, 0.172), (4, 6): (1, 6.9, -3.3, 0.705, 0.083), (4, 4): (2, 8.5, -7.6, 0.633, 0.527)}
+
+    @staticmethod
+    @functools.lru_cache(maxsize=4096)
+    def dense_tile(rows: int, n: int, k: int, gated: bool, units: int = 256) -> int:
+        """The tile of ``gemm_dense.hip`` for ``rows`` rows by ``n`` columns of the result, or 0: the library's product.
+
+        The tile is the one whose launch takes the least time by DENSE_TILES, which are fits to 22 numbers of rows by 22
+        matrices, each with every tile (what they say is a twentieth off, and the choice 2.4 % behind the best tile on the average).
+
+        Of the library's products it takes those that it does faster, 1.15 times on the average (library | this kernel, us, weights
+        not in the caches): 2,048 rows of 4,096 x 4,096 58 | 54, of 5,120 x 5,120 89 | 79, of 7,168 x 5,120 120 | 103, of 4,096 x
+        14,336 (k) 208 | 181, of 2,048 x 2,048 22 | 20, of 18,560 x 4,096 339 | 239; 1,024 of 5,120 x 5,120 60 | 52, 608 of 7,168 x
+        5,120 60 | 49; 2,048 of 4,096 x 512 (k) 18.6 | 13.2, where the library's launch alone is 18.  It leaves the library those
+        that fill whole rounds of 256 x 256 tiles (8,191 of 4,096 x 4,096 177 | 190, 4,096 of 8,192 x 2,048 96 | 106: there the
+        chip's power is what both wait for), and those with too few tiles for its compute units and a long k, which the library
+        cuts along k (704 of 4,096 x 7,168 (k) 51 | 63, 1,024 of 2,048 x 8,192 (k) 49 | 65).  With the gate it is measured against the
+        library's product and the activation's launch: 2,048 rows of 8,192 x 5,120 277 | 247, 953 150 | 123, 8,191 of 14,336 x
+        4,096 1,385 | 1,366, 256 of 8,192 x 5,120 70 | 67, but 97 47 | 65."""
+        if rows < 1 or n < 8 or n % 8 or k < 64 or k % 64 or k >= 1 << 23 or gated and 4 * n * k >= 1 << 32:
+            return 0
+        wide = 2 * n if gated else n  # rows of W
+        small = -(-rows // 128) * -(-wide // 128)
+        if gated:
+            if rows < 256 or small < 0.9 * units:
+                return 0
+        else:
+            if not (rows >= 192 and k <= 2048 or rows >= 256 and small >= (0.93 if k <= 6144 else 1.17) * units):
+                return 0
+            full = -(-rows // 256) * (wide // 256) / units  # rounds of whole tiles of 256 x 256
+            if wide % 256 == 0 and full >= 0.95 and full / math.ceil(full) >= 0.9:
+                return 0
+        tiles = HipOps.DENSE_GATED_TILES if gated else HipOps.DENSE_TILES
+
+        def cost(tile):
+            blocks, start, a_round, a_stage, full = tiles[tile]
+            count = -(-rows // (32 * tile[0])) * -(-wide // (32 * tile[1]))
+            rounds = -(-count // (units * blocks))
+            return start + rounds * (a_round + k / 64 * a_stage) + k / 64 * full * count / (units * blocks)
+
+        best = min(tiles, key=cost)
+        return best[0] * 16 + best[1]
+
+    def _dense(self, h, w, gated: bool = False, bias=None):
+        """``h @ w.T`` (``+ bias``; gated: ``silu(gate) * up``) of many bfloat16 rows by ``gemm_dense.hip``, or None: not its sizes,
+        or not the faster one, or a call that others look into."""
+        if (h.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or h.dim() != 2 or w.dim() != 2 or h.shape[1] != w.shape[1]
+                or gated and w.shape[0] % 2):
+            return None
+        m, k = h.shape
+        n = w.shape[0] // 2 if gated else w.shape[0]
+        tile = HipOps.dense_tile(m, n, k, gated, self._compute_units)
+        if (not tile or not h.get_device() == w.get_device() == self._device_index or not (h.is_contiguous() and w.is_contiguous())
+                or (h.data_ptr() | w.data_ptr()) % 16
+                or bias is not None and (bias.dtype != torch.bfloat16 or bias.shape != (n,) or not bias.is_contiguous()
+                                         or bias.get_device() != self._device_index or bias.data_ptr() % 8)
+                or torch.is_grad_enabled() and (h.requires_grad or w.requires_grad or bias is not None and bias.requires_grad)
+                or _watched()):
+            return None
+        return self.gemm_dense(h, w, tile, gated, bias)
+
+    def gemm_dense(self, h, w, tile: int, gated: bool = False, bias=None):
+        """The product of :meth:`_dense` with a tile of ``tile // 16 * 32`` rows of ``h`` by ``tile % 16 * 32`` of ``w``."""
+        m, k = h.shape
+        n = w.shape[0] // 2 if gated else w.shape[0]
+        self._chk(h, torch.bfloat16, (m, k), "rows")
+        self._chk(w, torch.bfloat16, (2 * n if gated else n, k), "W")
+        if bias is not None:
+            self._chk(bias, torch.bfloat16, (n,), "bias")
+        out = torch.empty(m, n, dtype=torch.bfloat16, device=h.device)
+        self._call("jle_gemm_dense", _p(h), _p(w), _p(out), _p(bias), int(gated), m, n, k, tile, self._compute_units)
+        return out
 
     FEW_ROWS = 64
 
@@ -1189,7 +1276,8 @@ class HipOps:
             return self.gemm_skinny(h, w, out_f32=True), bias
         if bias_run is None:
             bias_run = bias.to(h.dtype)
-        return torch.addmm(bias_run, h, w.t()), None
+        out = self._dense(h, w, bias=bias_run)
+        return torch.addmm(bias_run, h, w.t()) if out is None else out, None
 
     _ACTS = {"silu": 0, "gelu_tanh": 1}
 
@@ -1202,7 +1290,14 @@ class HipOps:
             product = self.gemm_few if self._few(h, w_gate_up) else self.gemm_skinny
             return product(h, w_gate_up, swiglu=1 + act)  # (the activation in the product's epilogue)
         out = self._dense_float32(h, w_gate_up, act)
-        return self.silu_mul(torch.matmul(h, w_gate_up.t()), activation) if out is None else out
+        if out is None and act == 0:
+            out = self._dense(h, w_gate_up, gated=True)
+        return self.silu_mul(self._product(h, w_gate_up), activation) if out is None else out
+
+    def _product(self, h, w):
+        """``h @ w.T`` of many bfloat16 rows: :meth:`_dense`'s, else the library's."""
+        out = self._dense(h, w)
+        return torch.matmul(h, w.t()) if out is None else out
 
     def sigmoid_mul(self, o, gate):
         """``o * sigmoid(gate)``; ``gate`` may be a slice of wider rows (its last axis contiguous), and narrower than ``o``:

@@ -30,7 +30,7 @@ class FolivikArchitecture:
                       "attention_generic.hip", "attention_mfma.hip", "attention_f32.hip", "attention_prep.hip",
                       "moe_route.hip", "moe_choose.hip", "gemm_skinny.hip", "gemm_few.hip", "gemm_stream.hip",
                       "gemm_grouped.hip",
-                      "gemm_generic.hip", "gemm_f32.hip", "gemm_f32_dense.hip", "parallel.hip", "sampling.hip")
+                      "gemm_generic.hip", "gemm_f32.hip", "gemm_f32_dense.hip", "gemm_dense.hip", "parallel.hip", "sampling.hip")
 
     def parse_config(self, top: Mapping[str, Any]) -> FolivikConfig:
         return FolivikConfig.from_dict(top)

@@ -26,7 +26,7 @@ class LifesunArchitecture:
     kernel_sources = ("elementwise.hip", "parallel.hip", "terms.hip", "retention.hip", "gated_unit.hip",
                       "attention_heads.hip", "attention_conv.hip", "attention_span.hip", "attention_generic.hip",
                       "attention_mfma.hip", "attention_f32.hip", "gemm_skinny.hip", "gemm_few.hip", "gemm_stream.hip",
-                      "gemm_grouped.hip", "gemm_generic.hip", "gemm_f32.hip", "gemm_f32_dense.hip", "sampling.hip")
+                      "gemm_grouped.hip", "gemm_generic.hip", "gemm_f32.hip", "gemm_f32_dense.hip", "gemm_dense.hip", "sampling.hip")
 
     def parse_config(self, top: Mapping[str, Any]) -> LifesunConfig:
         return LifesunConfig.from_dict(top)

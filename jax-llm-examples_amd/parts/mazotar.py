@@ -28,7 +28,7 @@ class MazotarArchitecture:
     # what of csrc/ a model of this design calls (a first run on a machine without a built library compiles these)
     kernel_sources = ("elementwise.hip", "streams.hip", "mlstm.hip", "attention_span.hip", "attention_generic.hip",
                       "attention_mfma.hip", "attention_f32.hip", "attention_prep.hip", "moe_route.hip", "gemm_skinny.hip", "gemm_few.hip",
-                      "gemm_stream.hip", "gemm_grouped.hip", "gemm_generic.hip", "gemm_f32.hip", "gemm_f32_dense.hip",
+                      "gemm_stream.hip", "gemm_grouped.hip", "gemm_generic.hip", "gemm_f32.hip", "gemm_f32_dense.hip", "gemm_dense.hip",
                       "sampling.hip")
 
     def parse_config(self, top: Mapping[str, Any]) -> MazotarConfig:

@@ -23,7 +23,7 @@ class RovidraArchitecture:
     # what of csrc/ a model of this design calls (a first run on a machine without a built library compiles these)
     kernel_sources = ("elementwise.hip", "sandwich.hip", "attention_latent.hip",
                       "attention_expanded.hip", "gemm_skinny.hip", "gemm_few.hip", "gemm_stream.hip",
-                      "gemm_grouped.hip", "gemm_generic.hip", "gemm_f32.hip", "gemm_f32_dense.hip", "sampling.hip")
+                      "gemm_grouped.hip", "gemm_generic.hip", "gemm_f32.hip", "gemm_f32_dense.hip", "gemm_dense.hip", "sampling.hip")
 
     def parse_config(self, top: Mapping[str, Any]) -> RovidraConfig:
         return RovidraConfig.from_dict(top)

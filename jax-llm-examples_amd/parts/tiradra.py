@@ -25,7 +25,7 @@ class TiradraArchitecture:
     kernel_sources = ("elementwise.hip", "parallel.hip", "attention_conv.hip", "attention_prep.hip", "attention_latent.hip",
                       "attention_expanded.hip",
                       "attention_mfma.hip", "attention_generic.hip", "attention_f32.hip", "gemm_skinny.hip", "gemm_few.hip",
-                      "gemm_stream.hip", "gemm_grouped.hip", "gemm_generic.hip", "gemm_f32.hip", "gemm_f32_dense.hip", "sampling.hip")
+                      "gemm_stream.hip", "gemm_grouped.hip", "gemm_generic.hip", "gemm_f32.hip", "gemm_f32_dense.hip", "gemm_dense.hip", "sampling.hip")
 
     def parse_config(self, top: Mapping[str, Any]) -> TiradraConfig:
         return TiradraConfig.from_dict(top)

@@ -2030,3 +2030,53 @@ def test_sum_with_factors_of_rows_off_their_16_bytes(ops, d, k):
     assert ((x.double() - want).abs() <= 8 * 2.0 ** -24 * size).all()
     assert ((h32.double() - normed).abs() <= 32 * 2.0 ** -24 * (size + normed.abs())).all()
     assert torch.equal(h, h32.bfloat16())
+
+
+@pytest.mark.parametrize("tile,gated", [(t, False) for t in ((8, 8), (8, 7), (8, 6), (6, 8), (8, 5), (8, 4), (6, 4), (4, 5), (4, 4))]
+                         + [(t, True) for t in ((8, 8), (8, 6), (6, 8), (8, 4), (4, 6), (4, 4))])
+def test_dense_product_of_many_rows(ops, tile, gated):
+    """Every tile: one row and eight columns over, one less, several tiles each way, one to six stages; with a bias and with the gate."""
+    bm, bn = 32 * tile[0], 32 * tile[1] // (2 if gated else 1)
+    for m, n, k in ((1, 8, 64), (bm, bn, 128), (bm + 1, bn + 8, 192), (2 * bm - 1, 2 * bn - 8, 256), (3 * bm + 17, 9 * bn + 16, 384)):
+        g = torch.Generator().manual_seed(m + n + k)
+        x = torch.randn(m, k, generator=g).to(DEV, torch.bfloat16)
+        w = (torch.randn(2 * n if gated else n, k, generator=g) * k ** -0.5).to(DEV, torch.bfloat16)
+        bias = None if gated else torch.randn(n, generator=g).to(DEV, torch.bfloat16)
+        want, sums = x.double() @ w.double().t(), (k + 2) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t())
+        for b in (None, bias) if bias is not None else (None,):
+            got = ops.gemm_dense(x, w, tile[0] * 16 + tile[1], gated, b).double()
+            if gated:  # (silu's slope is at most 1.1, its value at most the gate's; its float32 form adds a few roundings)
+                gate, up = want.split(n, 1)
+                y = torch.nn.functional.silu(gate) * up
+                off = 1.1 * sums[:, :n] * up.abs() + gate.abs() * sums[:, n:] + 1.1 * sums[:, :n] * sums[:, n:] + 16 * 2.0 ** -24 * y.abs()
+            else:
+                y = want if b is None else want + b.double()
+                off = sums + 2.0 ** -24 * y.abs()
+            assert ((got - y).abs() <= 2.0 ** -8 * y.abs() + off + 1e-30).all()
+            again = ops.gemm_dense(x[m // 2:].contiguous(), w, 4 * 16 + 4, gated, b)
+            assert torch.equal(again.double(), got[m // 2:])  # (a row's sums have one order whatever the tile and the other rows)
+
+
+def test_dense_product_keeps_what_is_not_a_number_in_its_row(ops):
+    x, w = (torch.randn(300, 128, device=DEV).bfloat16() for _ in range(2))
+    want = ops.gemm_dense(x, w[:296].contiguous(), 8 * 16 + 8)
+    x[299, 5], x[7, 127] = math.nan, math.inf
+    got = ops.gemm_dense(x, w[:296].contiguous(), 8 * 16 + 8)
+    keep = torch.ones(300, dtype=torch.bool)
+    keep[[7, 299]] = False
+    assert got[299].isnan().all() and not got[7].isfinite().any() and torch.equal(got[keep], want[keep])
+
+
+def test_dense_products_replayed(ops):
+    """In a graph, pass after pass with other rows in between."""
+    x, w = torch.randn(512, 1024, device=DEV).bfloat16(), torch.randn(2048, 1024, device=DEV).bfloat16()
+    ops.linear(x, w)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        y = ops.linear(x, w)
+        z = ops.swiglu_linear(y[:, :1024].contiguous(), w)
+    for _ in range(3):
+        x.copy_(torch.randn(512, 1024, device=DEV))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, ops.linear(x, w)) and torch.equal(z, ops.swiglu_linear(y[:, :1024].contiguous(), w))
