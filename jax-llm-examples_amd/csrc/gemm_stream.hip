@@ -27,6 +27,7 @@
 // float32 sums add_pieces_kernel adds up in their order and finishes (CUT).  Which blocks these are is known before the launch,
 // from the numbers of groups and of their blocks: a row's sums have one order whatever rows lie beside it.
 #include "common.h"
+#include "dense_block.h"
 
 using namespace jle;
 
@@ -427,206 +428,75 @@ __global__ __launch_bounds__(WAVES * 64) void add_pieces_kernel(StreamArgs p) {
 }
 
 // ------------------------------------------------------------------ groups of many rows
-// A block of four wavefronts, one a SIMD, takes 256 rows of W (SWIGLU: 128 gate rows and their up rows) and up to 256 rows
-// of a group; a wavefront 64 of those rows of W, four tiles, and all the rows of X: 4 x NT tiles of accumulators.  Its
-// weights go from memory straight into the A operand (no other wavefront of the block wants them), four stages of 64 k in
-// registers; X comes through shared memory, brought by the load unit itself (a kilobyte an instruction in the lanes' order,
-// the rows' 16-byte pieces swizzled by which piece a lane fetches) into a ring of three stages.  A byte read from shared
-// memory serves 64 operations.  With one wavefront a SIMD nothing hides a wait, so there is none: a B operand is asked for
-// four products of tiles before its use, the barrier that says that the next stage's rows have come (and that the ring's
-// oldest place is free) stands in the middle of a stage, and the next stage's first operands are read at this one's end.
-// 16 groups of 16,384 x 5,120 (gate and up) with 410 rows each: 1,080 us (1.02 PFLOP/s) against 1,474 in passes of 192; 8 of
-// 4,096 x 7,168 194 (0.99) against 269.  (With eight wavefronts of 64 x half the rows and the weights through shared memory
-// too 422 and 188 at 8 groups: reading and bringing in together took shared memory as long as the products.)
-// HALF (plain products): a block takes 128 rows of W and up to 288 of X, its wavefronts in twos by twos, 64 rows of W and half
-// of X each.  It reads twice as much for a product, but where blocks of 256 would fill a part of the compute units or of their
-// last round it is the faster: 8 groups of 2,048 x 4,096 with 300 rows 84 us in passes, 80 in wide tiles (128
-// blocks, two tiles a group), 64 so.  (All of 288 rows in wide tiles spills registers: 10 times slower.)
-// Work items: a group's rows in tiles of at most 256 (288), as even as multiples of 32 allow; item = ((row block / 8) * tiles +
-// tile) * 8 + row block % 8 within a group, so that the tiles that read the same weights run on one chiplet.
-constexpr int wide_rows(bool half) { return half ? 288 : 256; }                            // of X, of a block
-constexpr uint32_t wide_stage(bool half) { return (uint32_t)wide_rows(half) * BK * 2; }  // bytes of a stage's rows
+// A block of dense_block.h takes 32 * FN rows of W (SWIGLU: half of them gate rows, half their up rows) and up to 256 (FN = 4:
+// 288) rows of a group.  A group's rows are cut into tiles as even as multiples of 32 allow, and a block multiplies no more than
+// its tile has (full tiles and what is left instead: 8 groups of 14,336 x 4,096, gate and up, with 300 rows 298 -> 400 us).
+// Work items: item = ((row block / 8) * tiles + tile) * 8 + row block % 8 within a group, so that the tiles that read the
+// same weights run on one chiplet.  All blocks go through k from its beginning: begun elsewhere by row block, so that they read
+// other channels of the memory, they no longer find each other's rows of X in the caches (with 410 rows 403 -> 490).
+// In us, drawn groups, passes of 192 | tiles whose weights went straight into registers, X through a ring in shared memory | these:
+// gate and up of 8 of 14,336 x 4,096 with 192 rows 258 | 234 | 221, 410 483 | 389 | 364 (1.06 PFLOP/s), 700 743 | 635 | 559; 16
+// of 16,384 x 5,120 with 410 1,418 | 1,032 | 968; plain, 8 of 4,096 x 7,168 with 410 256 | 186 | 172, 16 of 5,120 x 8,192 762 |
+// 572 | 552; FN = 4: 8 of 2,048 x 4,096 with 192 80 | 69 | 58, 410 82 | 72 | 62, 16 of 1,024 x 2,048 with 176 46 | 41 | 35.
+// What bounds them is the last round of blocks and, below some 250 rows, the weights' bytes and the products that do not quite
+// overlap: with all groups' weights in the caches 410 rows take 352 for 400, 128 rows 129 for 197 (full tiles and rest).
+constexpr int wide_rows(int fn) { return fn == 8 ? 256 : 288; }  // of X, of a block
 
-template <bool SWIGLU, bool HALF, int NT>
-__device__ __forceinline__ void wide_block(const bf16_t* __restrict__ X, const bf16_t* __restrict__ We,
-                                           bf16_t* __restrict__ Y, const int* __restrict__ a_rows,
-                                           const float* __restrict__ scale, int act, unsigned char* smem, int tok0,
-                                           int live, int K, int Nout, int nb) {
-  static_assert(NT % 2 == 0, "a wavefront brings NT / 2 kilobytes of a stage's rows");
-  static_assert(!HALF || !SWIGLU, "half a block of rows of W: plain products only");
-  constexpr int NW = HALF ? NT / 2 : NT;  // tiles of X a wavefront multiplies with
-  static_assert(NW >= 4, "a stage's first operands are read behind the barrier in the middle of the stage before");
-  constexpr int PF = 4;  // operands asked for ahead
-  const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
-  const int wave = wave_index();
-  const uint32_t lds0 = (uint32_t)(uintptr_t)smem;
-  const int half = Nout >> 1, ntile = (SWIGLU ? half : Nout) >> 4;
-  const int nstage = K / BK;  // a multiple of 4
-  // this wavefront's tiles of W (SWIGLU: two of the gate, two of up); those behind the end: the last one, not stored
-  const bf16_t* w_src[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int tile = SWIGLU ? min(nb * 8 + wave * 2 + (i & 1), ntile - 1) + (i >= 2 ? half >> 4 : 0)
-                            : min(HALF ? nb * 8 + (wave & 1) * 4 + i : nb * 16 + wave * 4 + i, ntile - 1);
-    w_src[i] = We + (size_t)tile * 16 * K + lane * 8;
-  }
-  uint32_t x_src[NT / 2];
-#pragma unroll
-  for (int i = 0; i < NT / 2; ++i) {
-    const int t = tok0 + min(8 * (wave + 4 * i) + (lane >> 3), live - 1);
-    x_src[i] = (uint32_t)(a_rows != nullptr ? a_rows[t] : t) * (uint32_t)(K * 2) + (uint32_t)(((lane & 7) ^ (lane >> 3)) * 16);
-  }
-  auto ask_rows = [&](int s, uint32_t place) __attribute__((always_inline)) {
-#pragma unroll
-    for (int i = 0; i < NT / 2; ++i)
-      load_to_lds16(X + (size_t)s * BK, x_src[i], lds0 + place + (uint32_t)((wave + 4 * i) * 1024));
-  };
-  auto ask_weights = [&](u32x4 (&w)[2][4], int s) __attribute__((always_inline)) {
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) w[ks][i] = *reinterpret_cast<const u32x4*>(w_src[i] + (size_t)(2 * s + ks) * 512);
-  };
-  const int n0 = HALF ? (wave >> 1) * NW : 0;  // the first of its tiles of X
-  const uint32_t b_rd = (uint32_t)(n0 * 2048 + r * 128 + ((g ^ (r & 7)) * 16));  // (k step 1: bit 6 the other way)
-  auto operand = [&](uint32_t place, int j) __attribute__((always_inline)) {
-    return *reinterpret_cast<const bf16x8*>(smem + place + (b_rd ^ (j >= NW ? 64 : 0)) + (j % NW) * 2048);
-  };
-  f32x4 acc[4][NW];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int n = 0; n < NW; ++n) acc[i][n] = f32x4{0.f, 0.f, 0.f, 0.f};
-  u32x4 wa[2][4], wb[2][4], wc[2][4], wd[2][4];
-  bf16x8 ahead[PF];
-  constexpr uint32_t STAGE = wide_stage(HALF);
-  uint32_t here = 0, next = STAGE, free_ = 2 * STAGE;  // the ring: this stage's rows, the next one's, the one after
+struct WideArgs {
+  const bf16_t* X;
+  const bf16_t* W;
+  bf16_t* Y;
+  const int* offsets;
+  const int* a_rows;
+  const float* scale;
+  int act, Nout, K, G, nblk8;
+};
 
-  // rows_next: how many of the loads on their way are younger than the next stage's rows (-1: there is no next stage)
-#define WIDE_STAGE(w_, s_, rows_next, ASKX, ASKW)                                                       \
-  do {                                                                                                  \
-    bf16x8 b_[2 * NW + PF];                                                                             \
-    _Pragma("unroll") for (int p = 0; p < PF; ++p) b_[p] = ahead[p];                                    \
-    _Pragma("unroll") for (int j = 0; j < 2 * NW; ++j) {                                                \
-      if (j == NW && rows_next >= 0) {                                                                  \
-        if (rows_next > 0) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");                             \
-        else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                                           \
-        __syncthreads();                                                                                \
-        if (ASKX) ask_rows((s_) + 2, free_);                                                            \
-      }                                                                                                 \
-      if (j + PF < 2 * NW) b_[j + PF] = operand(here, j + PF);                                          \
-      else if (rows_next >= 0) b_[j + PF] = operand(next, j + PF - 2 * NW);                             \
-      _Pragma("unroll") for (int i = 0; i < 4; ++i) {                                                   \
-        acc[i][j % NW] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, w_[j / NW][i]), b_[j], \
-                                                                 acc[i][j % NW], 0, 0, 0);              \
-      }                                                                                                 \
-      __builtin_amdgcn_sched_barrier(0);                                                                \
-    }                                                                                                   \
-    if (rows_next >= 0) {                                                                               \
-      _Pragma("unroll") for (int p = 0; p < PF; ++p) ahead[p] = b_[2 * NW + p];                         \
-    }                                                                                                   \
-    if (ASKW) ask_weights(w_, (s_) + WAHEAD);                                                           \
-    const uint32_t t_ = here;                                                                           \
-    here = next;                                                                                        \
-    next = free_;                                                                                       \
-    free_ = t_;                                                                                         \
-  } while (0)
-
-  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the rows' numbers have come; from here on only the stages' loads count
-  asm volatile("" ::: "memory");
-  ask_rows(0, 0);
-  ask_rows(1, STAGE);
-  ask_weights(wa, 0);
-  ask_weights(wb, 1);
-  ask_weights(wc, 2);
-  ask_weights(wd, 3);
-  asm volatile("s_waitcnt vmcnt(24)" ::: "memory");
-  __syncthreads();
-#pragma unroll
-  for (int p = 0; p < PF; ++p) ahead[p] = operand(0, p);
-  int s = 0;
-  for (; s < nstage - WAHEAD; s += WAHEAD) {
-    WIDE_STAGE(wa, s, 8, true, true);
-    WIDE_STAGE(wb, s + 1, 8, true, true);
-    WIDE_STAGE(wc, s + 2, 8, true, true);
-    WIDE_STAGE(wd, s + 3, 8, true, true);
-  }
-  WIDE_STAGE(wa, s, 8, true, false);
-  WIDE_STAGE(wb, s + 1, 0, true, false);
-  WIDE_STAGE(wc, s + 2, 0, false, false);
-  WIDE_STAGE(wd, s + 3, -1, false, false);
-#undef WIDE_STAGE
-#pragma unroll
-  for (int n = 0; n < NW; ++n) {
-    const int row = (n0 + n) * 16 + r;
-    if (row >= live) continue;
-    const int t = tok0 + row;
-    const float sc = scale != nullptr ? scale[t] : 1.f;
-#pragma unroll
-    for (int i = 0; i < (SWIGLU ? 2 : 4); ++i) {
-      const int tile = SWIGLU ? nb * 8 + wave * 2 + i : HALF ? nb * 8 + (wave & 1) * 4 + i : nb * 16 + wave * 4 + i;
-      if (tile >= ntile) continue;
-      float y[4];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        if (SWIGLU) {
-          const float gate = acc[i][n][e] * sc, up = acc[i + 2][n][e] * sc;
-          y[e] = gate / (1.0f + expf(-gate)) * up;
-        } else {
-          y[e] = acc[i][n][e] * sc;
-          if (act) y[e] = relu2(Num<bf16_t>::round(y[e]));
-        }
-      }
-      store4<bf16_t>(Y + (size_t)t * (SWIGLU ? half : Nout) + tile * 16 + 4 * g, y[0], y[1], y[2], y[3]);
-    }
-  }
-}
-
-template <bool SWIGLU, bool HALF>
-__global__ __launch_bounds__(256, 1) void wide_kernel(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W,
-                                                      bf16_t* __restrict__ Y, const int* __restrict__ offsets,
-                                                      const int* __restrict__ a_rows, const float* __restrict__ scale,
-                                                      int act, int Nout, int K, int G, int nblk8) {
+template <int FN, bool SWIGLU>
+__global__ __launch_bounds__(256, 1) void wide_kernel(WideArgs p) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
-  constexpr int kWideRows = wide_rows(HALF);
-  const Items items = {offsets, 0, G, nblk8, kWideRows};
+  constexpr int BN = SWIGLU ? FN * 16 : FN * 32;
+  const Items items = {p.offsets, 0, p.G, p.nblk8, wide_rows(FN)};
   int left = blockIdx.x, tiles;
   const int e = items.find(left, tiles);
   if (e < 0) return;  // (the grid is laid out for the most tiles that so many rows can make)
-  const int nb = left / (8 * tiles) * 8 + (left & 7), tile = (left >> 3) % tiles;
-  if (nb * (SWIGLU || HALF ? 128 : 256) >= (SWIGLU ? Nout / 2 : Nout)) return;
-  const int lo = offsets[e], rows = offsets[e + 1] - lo;
-  const int per = rows_a_tile(rows, tiles);
-  const int tok0 = lo + tile * per, live = min(per, rows - tile * per);
+  const int nb = left / (8 * tiles) * 8 + (left & 7), tile = (left >> 3) % tiles, N = SWIGLU ? p.Nout >> 1 : p.Nout;
+  if (nb * BN >= N) return;
+  const int rows = p.offsets[e + 1] - p.offsets[e], per = rows_a_tile(rows, tiles), lo = p.offsets[e] + tile * per, live = min(per, rows - tile * per);
   if (live <= 0) return;
-  const bf16_t* We = W + (size_t)e * Nout * K;
-#define GO(NT_) wide_block<SWIGLU, HALF, NT_>(X, We, Y, a_rows, scale, act, smem, tok0, live, K, Nout, nb)
-  if constexpr (HALF) {
-    if (live > 256) {
-      GO(18);
-      return;
-    }
+  const dense::DenseBlock b = {p.X, p.W + (size_t)e * p.Nout * p.K, p.Y, nullptr, p.a_rows, p.scale, p.act, lo, live, nb * BN, N, p.K};
+#define GO(FM, RX, RW) dense::dense_block<FM, FN, RX, RW, SWIGLU, true>(b, smem)
+  if constexpr (FN == 8) {
+    if (live <= 64) GO(2, 6, 6);
+    else if (live <= 96) GO(3, 6, 6);
+    else if (live <= 128) GO(4, 6, 6);
+    else if (live <= 160) GO(5, 6, 6);
+    else if (live <= 192) GO(6, 5, 6);
+    else if (live <= 224) GO(7, 4, 6);
+    else GO(8, 4, 6);
+  } else {
+    if (live <= 64) GO(2, 6, 6);
+    else if (live <= 96) GO(3, 6, 6);
+    else if (live <= 128) GO(4, 6, 6);
+    else if (live <= 160) GO(5, 6, 6);
+    else if (live <= 192) GO(6, 6, 6);
+    else if (live <= 224) GO(7, 6, 6);
+    else if (live <= 256) GO(8, 6, 6);
+    else GO(9, 6, 6);
   }
-  if (live <= 64) GO(HALF ? 8 : 4);
-  else if (live <= 128) GO(8);
-  else if (live <= 160) GO(10);
-  else if (live <= 192) GO(12);
-  else if (live <= 224) GO(14);
-  else GO(16);
 #undef GO
 }
 
-template <bool SW, bool HALF>
-int launch_wide(hipStream_t s, const void* X, const void* W, void* Y, const int* offsets, const int* a_rows,
-                const float* scale, int act, int M, int Nout, int K, int G) {
-  constexpr uint32_t lds = 3 * wide_stage(HALF);
-  if (const int rc = allow_lds(wide_kernel<SW, HALF>, lds)) return rc;
-  constexpr int of8 = SW || HALF ? 1024 : 2048;  // columns of Y of eight blocks
-  const int nblk8 = ((SW ? Nout / 2 : Nout) + of8 - 1) / of8 * 8;
-  const long long items = ((long long)M / wide_rows(HALF) + G) * nblk8;
+template <int FN, bool SW>
+int launch_wide(WideArgs p, int M, hipStream_t s) {
+  constexpr uint32_t lds = 160 * 1024;  // (a compute unit's: the largest tile's rings take it all or most of it)
+  static_assert(dense::dense_bytes<8, FN, 4, 6, SW>() <= lds && dense::dense_bytes<9, 4, 6, 6, SW>() <= lds, "");
+  if (const int rc = allow_lds(wide_kernel<FN, SW>, lds)) return rc;
+  constexpr int of8 = 8 * (SW ? FN * 16 : FN * 32);  // columns of Y of eight blocks
+  p.nblk8 = ((SW ? p.Nout / 2 : p.Nout) + of8 - 1) / of8 * 8;
+  const long long items = ((long long)M / wide_rows(FN) + p.G) * p.nblk8;
   if (items > (1ll << 30)) return JLE_BAD_ARG;
-  hipLaunchKernelGGL((wide_kernel<SW, HALF>), dim3((unsigned)items), dim3(256), lds, s, (const bf16_t*)X, (const bf16_t*)W,
-                     (bf16_t*)Y, offsets, a_rows, scale, act, Nout, K, G, nblk8);
+  hipLaunchKernelGGL((wide_kernel<FN, SW>), dim3((unsigned)items), dim3(256), lds, s, p);
   JLE_LAUNCH_CHECK();
   return 0;
 }
@@ -663,7 +533,8 @@ JLE_API int jle_gemm_stream_supported(int Nout, int K, int swiglu) {
 JLE_API int jle_gemm_stream_room(int M, int G) { return (M >> 4) + 2 * (M / kRows + G); }
 
 // X [*, K] bf16, W [G, Nout, K] bf16 in the streaming layout, Y [M, Nout] (or [M, Nout / 2] with swiglu) bf16 or
-// float32; X must have fewer than 2^32 elements (wide: 2^32 bytes).  wide: wide_kernel (groups, bfloat16 out), 2 (plain): HALF.
+// float32; X must have fewer than 2^32 elements (wide: 2^32 bytes).  wide: wide_kernel (groups, bfloat16 out, a group's W of fewer than
+// 2^32 bytes), 2 (plain): with FN = 4.
 // act 1 (plain): max(., 0)^2 of the rounded sums.  cuts > 1 (plain, not wide): the last `cut` of a group's blocks of 256 rows of
 // W are cut into `cuts` pieces along k; pieces: place for jle_gemm_stream_room(M, G) * cut * cuts tiles of 16 KB.
 // Blocks are 8 wavefronts (two per SIMD, one block per compute unit): measured against 4, 5 and 6 on expert
@@ -674,11 +545,11 @@ JLE_API int jle_gemm_stream(const void* X, const void* W, void* Y, const int* of
   if (M <= 0 || Nout <= 0) return 0;
   if (wide) {
     if (offsets == nullptr || out_f32 || G < 1 || G > 65535 || !jle_gemm_stream_supported(Nout, K, swiglu) ||
-        ((uintptr_t)X | (uintptr_t)W | (uintptr_t)Y) % 16)
+        (long long)Nout * K * 2 >= (1ll << 32) || ((uintptr_t)X | (uintptr_t)W | (uintptr_t)Y) % 16)
       return JLE_BAD_ARG;
-    if (swiglu) return launch_wide<true, false>(s, X, W, Y, offsets, a_rows, scale, act, M, Nout, K, G);
-    return wide == 2 ? launch_wide<false, true>(s, X, W, Y, offsets, a_rows, scale, act, M, Nout, K, G)
-                     : launch_wide<false, false>(s, X, W, Y, offsets, a_rows, scale, act, M, Nout, K, G);
+    const WideArgs p = {(const bf16_t*)X, (const bf16_t*)W, (bf16_t*)Y, offsets, a_rows, scale, act, Nout, K, G, 0};
+    if (swiglu) return launch_wide<8, true>(p, M, s);
+    return wide == 2 ? launch_wide<4, false>(p, M, s) : launch_wide<8, false>(p, M, s);
   }
   if (G < 1 || G > 65535 || (offsets == nullptr && G != 1) || !jle_gemm_stream_supported(Nout, K, swiglu)) return JLE_BAD_ARG;
   constexpr int kWaves = 8;

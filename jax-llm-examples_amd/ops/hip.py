@@ -1936,20 +1936,19 @@ class HipOps:
     def stream_wide(rows: int, groups: int, row_blocks: int) -> bool:
         """Which of ``gemm_stream.hip``'s kernels takes ``rows`` rows in ``groups`` groups (``row_blocks`` blocks of 256 rows
         of W a group): passes of 192 rows or wide tiles of 256.  A block fills a compute unit, so what counts is how many
-        rounds of blocks there are on the 256 compute units and how long one takes; measured per stage of 64 k, microseconds:
+        rounds of blocks there are on the 256 compute units and how long one takes, per stage of 64 k, microseconds:
         passes 0.9 + 0.0037 a row, tiles 0.95 + 0.003.  Fewer than 16 row blocks of tiles count in eights, as they are dealt to the
-        eight chiplets (of 10 groups of 3,072 x 3,072 with 384 rows half of the chiplets get two thirds: 80 | 147). A group's
+        eight chiplets (of 10 groups of 3,072 x 3,072 with 384 rows half of the chiplets get two thirds: 115 | 126). A group's
         rows are taken to scatter about their mean by its root: how they are shared out is known on the device only. With fewer
         than WIDE_GROUPS groups one that is far fuller than the others is what the launch takes, and is better cut in more
-        pieces: 2 groups of 4,096 x 2,048 with 300 rows on average in even groups 41 | 43, 40 % in one 45 | 59; 4 42 | 60. Over
-        26 matrices of 8 to 128 groups with 48 to 900 rows each, even, drawn, and with 40 % of the rows in one group, the
-        choice between these and :meth:`stream_half`'s is 3 % from the best, and where it is not passes it is 7 % faster than
-        they, at worst 1.65 times their time (8 of 5,120 x 4,096 with 256, 40 % in one: 110 | 181; drawn 1.42 times, 32 of 1,024 x
-        2,048 with 176: 51 | 73). Both sides measured (passes | tiles, us, drawn groups): 8 groups of 14,336 x 4,096 gate and
-        up with 192 rows 264 | 232, 256 341 | 293, 410 494 | 409, 700 767 | 650; of 4,096 x 7,168 with 192 155 | 161, 410 267 |
-        198, 512 312 | 298, 700 348 | 351; of 8,192 x 2,048 gate and up with 410 151 | 127, 512 183 | 170; 16 of 16,384 x 5,120
-        with 160 551 | 579, 410 1,440 | 1,084, 700 2,117 | 1,780; of 5,120 x 8,192 with 300 557 | 505; 64 of 1,024 x 2,048
-        (four row blocks) with 192 114 | 142, 300 156 | 200; of 512 x 2,048 with 290 68 | 191."""
+        pieces.  The line was drawn when the tiles took 6 % longer than they do.  Over 34 matrices of 4 to 128 groups with 96 to 900
+        rows each, even, drawn, and with 40 % of the rows in one group, the choice between these and :meth:`stream_half`'s is 4.5 %
+        from the best; a line drawn anew would be 3.9 % from it, but up to 1.8 times slower at single sizes than this one. Both
+        sides measured (passes | tiles, us, drawn groups): 8 groups of 14,336 x 4,096 gate and up with 176 rows 193 | 210, 192
+        258 | 221, 256 314 | 264, 410 483 | 364, 700 743 | 559; of 4,096 x 7,168 with 192 137 | 150, 300 158 | 145, 410 256 |
+        172, 512 289 | 282, 700 320 | 314; of 8,192 x 2,048 gate and up with 410 139 | 111, 512 164 | 153; 16 of 16,384 x 5,120
+        with 160 527 | 506, 410 1,418 | 968, 700 2,057 | 1,525; of 5,120 x 8,192 with 300 542 | 441; 64 of 1,024 x 2,048
+        (four row blocks) with 192 108 | 140, 300 152 | 191; of 512 x 2,048 with 300 65 | 174."""
         mean = rows / groups
         if mean < HipOps.WIDE_GROUP_ROWS or groups < HipOps.WIDE_GROUPS:
             return False
@@ -1973,11 +1972,10 @@ class HipOps:
         rows fill, and an eighth of the round stays free.  Row blocks count in eights, as they are dealt to the eight chiplets
         (of groups of 256 rows of W all blocks are on two of them).  Few rows a group are the time of their weights' bytes.
 
-        Measured as :meth:`stream_wide` is: where these tiles are taken they are 7 % faster than passes on the average, at worst
-        24 % slower (16 groups of 1,024 x 2,048 with 256 rows, two passes of 128: 37 | 46 us).  Taken wherever even groups would
-        fill one round or two, they were up to 67 % slower.  Passes | these, us, drawn and with 40 % in one: 8 of 2,048 x 4,096 with
-        128 rows 62 | 57 and 69 | 63, 230 63 | 70 and 80 | 68, 300 81 | 80 and 82 | 70; 8 of 1,024 x 8,192 with 512 147 | 141 and
-        147 | 140; 16 of 1,024 x 2,048 with 190 48 | 42 and 48 | 45; but 8 of 4,096 x 7,168 with 256 160 | 166 and 151 | 214."""
+        Measured as :meth:`stream_wide` is.  Passes | these, us, drawn and with 40 % in one: 8 of 2,048 x 4,096 with 128 rows 62 | 46
+        and 69 | 57, 224 64 | 59 and 77 | 63, 300 79 | 67 and 79 | 62, 410 82 | 62 and 81 | 67; 16 of 1,024 x 2,048 with 192 46 | 35
+        and 46 | 41, 256 43 | 42 and 47 | 41; 8 of 1,024 x 8,192 with 192 144 | 102 and 144 | 99, but with 128, where passes are cut
+        along k, 55 | 86 and 70 | 103; 8 of 4,096 x 7,168 (not taken) with 256 143 | 139 and 138 | 175."""
         slots = -(-row_blocks // 8) * 8 * groups
         mean = rows / groups
         return groups >= HipOps.WIDE_GROUPS and mean >= 90 and slots <= 192 and slots * (mean / 288 + 0.5) <= 224
@@ -2028,7 +2026,8 @@ class HipOps:
         out = torch.empty(m, nout // 2 if swiglu else nout, dtype=torch.float32 if out_f32 else torch.bfloat16,
                           device=a.device)
         wide, among = 0, m if expected is None else expected
-        if offsets is not None and not out_f32 and a.numel() < 2 ** 31 and not (a.data_ptr() | b.data_ptr()) % 16:
+        if (offsets is not None and not out_f32 and a.numel() < 2 ** 31 and nout * k < 2 ** 31
+                and not (a.data_ptr() | b.data_ptr()) % 16):
             wide = 2 if not swiglu and self.stream_half(among, g, -(-nout // 128)) else self.stream_wide(among, g, -(-nout // 256))
         pieces, cut, cuts = None, 0, 1
         if not wide and not swiglu:

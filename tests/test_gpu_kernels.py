@@ -1450,6 +1450,28 @@ def test_wide_tiles_of_the_weight_streaming_product(ops, monkeypatch, counts, no
     assert torch.equal(*got)
 
 
+@pytest.mark.parametrize("counts,nout,k", [
+    ([1, 0, 32, 33, 64, 65, 96, 97, 128, 129], 128, 256),        # every number of row tiles
+    ([160, 161, 192, 193, 224, 225, 256, 257], 144, 512),        # a second block of W of one tile
+    ([288, 0, 289, 576, 577, 900], 1168, 256)])                  # the most rows of a tile and one more; more than eight blocks of W
+def test_narrower_wide_tiles_of_the_weight_streaming_product(ops, monkeypatch, counts, nout, k):
+    """The bits of the kernel that takes the rows in passes, rows gathered and scaled; rows that no group has are left alone."""
+    from jax_llm_examples_amd.ops.layout import tile_
+    m, e = sum(counts), len(counts)
+    x, w = _rand(m + 3, k, dt=torch.bfloat16, seed=1), _rand(e, nout, k, dt=torch.bfloat16, scale=0.1, seed=2)
+    tile_(w)
+    off = torch.tensor([0] + counts).cumsum(0).int().to(DEV)
+    rows = torch.randperm(m + 3, generator=torch.Generator().manual_seed(3)).int().to(DEV)
+    scale = _rand(m + 3, seed=4)
+    got = []
+    monkeypatch.setattr(ops, "stream_wide", lambda *a: False)
+    monkeypatch.setattr(ops, "stream_cuts", lambda *a: (0, 1))
+    for half in (False, True):
+        monkeypatch.setattr(ops, "stream_half", lambda *a, half=half: half)
+        got.append(ops.gemm_stream(x, w, offsets=off, a_rows=rows, scale=scale, rows=m + 3)[:m])
+    assert torch.equal(*got)
+
+
 @pytest.mark.parametrize("dt", DT)
 def test_squared_relu_keeps_what_is_not_a_number(ops, dt):
     """Of plain numbers, infinities and NaN what torch gives, as a launch of its own and behind the product of a few rows."""
