@@ -179,67 +179,99 @@ __global__ void moe_topk_kernel(const float* __restrict__ logits, int* __restric
   }
 }
 
-// The same grouping for any number of pairs that lie in memory, a piece of the pairs at a time: all threads bring
-// the piece's experts into shared memory (whole lines); every wavefront looks through the piece for its experts
-// and notes each pair's row there; then all threads write the rows' tokens and gates.  Nothing in a wavefront's
-// look through 64 pairs waits for memory (with the gate fetched inside it, every look waited for that load:
-// 2,048 pairs took 18 us, now 6).  The order of the rows is the same.
-__global__ __launch_bounds__(1024) void moe_align_kernel(const int* __restrict__ ids, const float* __restrict__ gates,
-                                                         int* __restrict__ offsets, int* __restrict__ sorted_token,
-                                                         float* __restrict__ sorted_gate, int* __restrict__ inv,
-                                                         int M, int E, int k, int extra, int piece_len, int inv_ld) {
-  extern __shared__ int smem[];  // counts[E], starts[E + 1], runs[E], piece[piece_len], rows[piece_len]
-  int* counts = smem;
-  int* starts = smem + E;
-  int* runs = smem + 2 * E + 1;
-  int* piece = smem + 3 * E + 1;
-  int* rows = piece + piece_len;
-  for (int e = threadIdx.x; e < E; e += blockDim.x) counts[e] = 0;
-  __syncthreads();
-  for (int r = threadIdx.x; r < M; r += blockDim.x)
-    if (ids[r] < E) atomicAdd(&counts[ids[r]], 1);
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    int run = 0;
-    for (int e = 0; e < E; ++e) {
-      starts[e] = run;
-      runs[e] = run;
-      run += counts[e];
+// The same grouping for any number of pairs that lie in memory.  Every wavefront has a run of the pairs: it counts them by
+// expert; from all wavefronts' counts follows where each one's pairs of an expert begin; then it goes through its run once
+// more, 64 pairs at a time, and a pair's row is its expert's next one plus how many of the lanes before it have the same expert,
+// which a ballot for each bit of the experts' numbers tells.  Counting and placing are shared by all wavefronts whatever the
+// number of experts.  (With a wavefront for every expert that looks through all pairs, 64 at a time and each look behind
+// the last, us: 1,024 pairs of 8 experts 5.4 -> 4.4, 2,048 8.0 -> 5.4, 4,096 14.0 -> 7.2, 16,384 51 -> 20; 2,048 of 128 39 -> 6.0.)
+// What is left is one block's trips to memory and shared memory, one behind the other.  The order of the rows is the pairs'.
+constexpr int kAlignWaves = 16, kAlignAhead = 4;  // (pairs a lane asks for at once)
+__global__ __launch_bounds__(kAlignWaves * 64) void moe_align_kernel(const int* __restrict__ ids, const float* __restrict__ gates,
+                                                                     int* __restrict__ offsets, int* __restrict__ sorted_token,
+                                                                     float* __restrict__ sorted_gate, int* __restrict__ inv,
+                                                                     int M, int E, int k, int extra, int inv_ld) {
+  extern __shared__ int smem[];  // counts[waves][E], starts[E + 1]
+  const int lane = threadIdx.x & 63, wave = wave_index(), waves = blockDim.x >> 6;
+  int* mine = smem + wave * E;
+  int* starts = smem + waves * E;
+  const int per = ((M + 63) / 64 + waves - 1) / waves * 64, lo = wave * per, hi = min(M, lo + per);
+  int e[kAlignAhead];
+  auto ask = [&](int base) __attribute__((always_inline)) {  // (E: no pair, or one without a row)
+#pragma unroll
+    for (int j = 0; j < kAlignAhead; ++j) {
+      const int r = base + 64 * j + lane;
+      e[j] = r < hi ? min(ids[r], E) : E;
     }
-    starts[E] = run;
+  };
+  ask(lo);
+  for (int i = threadIdx.x; i < waves * E; i += blockDim.x) smem[i] = 0;
+  __syncthreads();
+  for (int base = lo; base < hi; base += 64 * kAlignAhead) {
+    if (base != lo) ask(base);
+#pragma unroll
+    for (int j = 0; j < kAlignAhead; ++j)
+      if (e[j] < E) atomicAdd(&mine[e[j]], 1);
+  }
+  __syncthreads();
+  for (int x = threadIdx.x; x < E; x += blockDim.x) {
+    int c[kAlignWaves], run = 0;
+#pragma unroll
+    for (int w = 0; w < kAlignWaves; ++w) c[w] = w < waves ? smem[w * E + x] : 0;
+#pragma unroll
+    for (int w = 0; w < kAlignWaves; ++w) {
+      if (w < waves) smem[w * E + x] = run;
+      run += c[w];
+    }
+    starts[x] = run;
+  }
+  __syncthreads();
+  if (wave == 0) {
+    int before = 0;
+    for (int x0 = 0; x0 < E; x0 += 64) {
+      const int own = x0 + lane < E ? starts[x0 + lane] : 0;
+      int upto = own;
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const int v = __shfl_up(upto, o, 64);
+        if (lane >= o) upto += v;
+      }
+      if (x0 + lane < E) starts[x0 + lane] = before + upto - own;
+      before += __shfl(upto, 63, 64);
+    }
+    if (lane == 0) starts[E] = before;
   }
   __syncthreads();
   extra_group(starts[E], offsets, sorted_token, sorted_gate, inv, E, k, extra, inv_ld);
-  for (int e = threadIdx.x; e <= E; e += blockDim.x) offsets[e] = starts[e];
-  const int lane = threadIdx.x & 63, wave = wave_index(), waves = blockDim.x >> 6;
-  for (int c0 = 0; c0 < M; c0 += piece_len) {
-    const int n = min(piece_len, M - c0);
-    for (int i = threadIdx.x; i < n; i += blockDim.x) {
-      piece[i] = ids[c0 + i];
-      rows[i] = -1;
-    }
-    __syncthreads();
-    for (int e = wave; e < E; e += waves) {
-      if (counts[e] == 0) continue;
-      int run = runs[e];
-      for (int base = 0; base < n; base += 64) {
-        const int r = base + lane;
-        const bool match = r < n && piece[r] == e;
-        const unsigned long long bal = __ballot(match);
-        if (match) rows[r] = run + __popcll(bal & ((1ull << lane) - 1ull));
-        run += __popcll(bal);
+  for (int x = threadIdx.x; x <= E; x += blockDim.x) offsets[x] = starts[x];
+  const int bits = 32 - __clz(E);
+  for (int base = lo; base < hi; base += 64 * kAlignAhead) {
+    float gate[kAlignAhead];
+    if (hi - lo > 64 * kAlignAhead) ask(base);  // (else they are still here)
+#pragma unroll
+    for (int j = 0; j < kAlignAhead; ++j) gate[j] = e[j] < E ? gates[base + 64 * j + lane] : 0.f;
+#pragma unroll
+    for (int j = 0; j < kAlignAhead; ++j) {
+      const int r = base + 64 * j + lane;
+      if (base + 64 * j >= hi) break;
+      unsigned long long same = ~0ull;
+      for (int b = 0; b < bits; ++b) {
+        const bool one = e[j] >> b & 1;
+        const unsigned long long with = __ballot(one);
+        same &= one ? with : ~with;
       }
-      if (lane == 0) runs[e] = run;
+      const int rank = __popcll(same & ((1ull << lane) - 1ull));
+      int first = 0;
+      if (rank == 0 && e[j] < E) first = starts[e[j]] + atomicAdd(&mine[e[j]], __popcll(same));
+      first = __shfl(first, __ffsll((long long)same) - 1, 64);
+      if (r >= hi) continue;
+      const int pos = e[j] < E ? first + rank : -1, t = r / k;
+      inv[t * inv_ld + r - t * k] = pos;
+      if (pos >= 0) {
+        sorted_token[pos] = t;
+        sorted_gate[pos] = gate[j];
+      }
     }
-    __syncthreads();
-    for (int i = threadIdx.x; i < n; i += blockDim.x) {
-      const int pos = rows[i], t = (c0 + i) / k;
-      inv[t * inv_ld + (c0 + i) - t * k] = pos;
-      if (pos < 0) continue;
-      sorted_token[pos] = t;
-      sorted_gate[pos] = gates[c0 + i];
-    }
-    __syncthreads();
   }
 }
 
@@ -709,9 +741,9 @@ static int launch_logits(const float* h, const float* w, float* logits, int N, i
 
 static int launch_align(const int* ids, const float* gates, int* offsets, int* sorted_token, float* sorted_gate,
                         int* inv, int M, int E, int k, int extra, int inv_ld, hipStream_t s) {
-  // A wavefront looks at all its pairs for every expert; moe_align_kernel's thousand threads share them and meet at eight
-  // barriers.  Threads | wavefront, us: 64 pairs of 8 experts 2.9 | 2.3, of 32 3.8 | 3.6, of 48 5.1 | 5.4; 128 of 8 3.1 | 2.6, of 16
-  // 3.6 | 3.2; 256 of 8 3.5 | 3.1, of 16 3.6 | 4.1, of 32 4.9 | 6.1, of 63 7.0 | 9.7.
+  // A wavefront looks at all its pairs for every expert; moe_align_kernel's meet at four barriers, 3.6 to 3.7 us up to 256 pairs
+  // whatever the experts.  One wavefront, us: 64 pairs of 8 experts 2.3, of 32 3.6, of 48 5.4; 128 of 8 2.6, of 16 3.2; 256 of 8
+  // 3.1, of 16 4.1, of 32 6.1.
   if (M <= 256 && (M + 63) / 64 * E <= 40) {
 #define WAVE(R_) \
   hipLaunchKernelGGL(moe_align_wave_kernel<R_>, dim3(1), dim3(64), 0, s, ids, gates, offsets, sorted_token, sorted_gate, inv, M, E, \
@@ -723,12 +755,11 @@ static int launch_align(const int* ids, const float* gates, int* offsets, int* s
     JLE_LAUNCH_CHECK();
     return 0;
   }
-  // (shared memory: 64 KB; the pieces take what the experts' counters leave, at most 2,048 pairs)
-  int piece = (16384 - (3 * E + 1)) / 2;
-  piece = piece > 2048 ? 2048 : piece / 64 * 64;
-  if (piece < 64) return JLE_BAD_ARG;
-  hipLaunchKernelGGL(moe_align_kernel, dim3(1), dim3(1024), (3 * E + 1 + 2 * piece) * sizeof(int), s, ids, gates, offsets,
-                     sorted_token, sorted_gate, inv, M, E, k, extra, piece, inv_ld);
+  // (64 KB of counts: fewer wavefronts with thousands of experts)
+  const int waves = min(min(kAlignWaves, (M + 63) / 64), (16384 - (E + 1)) / E);
+  if (waves < 1) return JLE_BAD_ARG;
+  hipLaunchKernelGGL(moe_align_kernel, dim3(1), dim3(64 * waves), ((waves + 1) * E + 1) * sizeof(int), s, ids, gates, offsets,
+                     sorted_token, sorted_gate, inv, M, E, k, extra, inv_ld);
   JLE_LAUNCH_CHECK();
   return 0;
 }

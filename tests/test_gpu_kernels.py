@@ -995,6 +995,26 @@ def test_moe_align_at_the_edges_of_one_wavefront(ops, n, k, e):
     assert inv.view(n, k + 1).tolist() == [[row.get(t * k + j, -1) for j in range(k)] + [len(order) + t] for t in range(n)]
 
 
+@pytest.mark.parametrize("n,k,e", [(257, 1, 8), (1024, 1, 63), (1025, 4, 64), (4096, 1, 1), (4097, 1, 300), (8193, 2, 10), (700, 1, 4096), (333, 1, 2048)])
+def test_moe_align_of_many_pairs(ops, n, k, e):
+    """Runs of pairs that end within 64 and past the ones that a wavefront asks for at once, more experts than a look takes and than
+    sixteen wavefronts count; even, all of one expert, and with choices that have no row."""
+    g = torch.Generator().manual_seed(n)
+    for ids in (torch.randint(0, e + 2, (n, k), generator=g), torch.full((n, k), e - 1), torch.randint(0, min(e, 3), (n, k), generator=g)):
+        gates = _rand(n, k, seed=5)
+        off, tok, gate, inv = (t.cpu() for t in ops.moe_align(ids.int().to(DEV), gates, e, extra_group=True, note_extra=True))
+        flat = ids.reshape(-1)
+        order = torch.argsort(flat, stable=True)
+        order = order[flat[order] < e]
+        rows = order.numel()
+        assert torch.equal(off[: e + 1].long(), torch.cat([torch.zeros(1), torch.bincount(flat[flat < e], minlength=e)]).cumsum(0).long())
+        assert off[e + 1] == rows + n and torch.equal(tok[: rows + n].long(), torch.cat([order // k, torch.arange(n)]))
+        assert torch.equal(gate[:rows], gates.cpu().reshape(-1)[order])
+        want = torch.full((n * k,), -1)
+        want[order] = torch.arange(rows)
+        assert torch.equal(inv.view(n, k + 1).long(), torch.cat([want.view(n, k), rows + torch.arange(n)[:, None]], 1))
+
+
 def test_moe_align_is_a_stable_grouping(ops):
     g = torch.Generator().manual_seed(0)
     ids = torch.randint(0, 7, (300, 2), generator=g).to(torch.int32).to(DEV)
