@@ -7,8 +7,13 @@
 //     rows [N, Hq dk + Hk dk + Hv dv] (or the leading part of wider rows)  ->  q_out [N, Hq, D],  pages [.., 2, Hk, ps, D] (values [D][ps])
 // and the combination of two score maps' outputs into one head's:
 //     d = a1 - lam a2;  d / sqrt(mean(d^2) + eps) * scale * sigmoid(gate)
-// One wavefront per (token, head); a lane holds elements lane, lane + 64, ...  Everything in float32; the order of
-// every sum depends on the sizes only.
+// One wavefront per (token, head); a lane holds elements lane, lane + 64, ... (PER of them, so that a step of few tokens runs
+// through no more code than its heads need).  Everything in float32; the order of every sum depends on the sizes only.
+// Values lie transposed in their pages: a token's are single elements a row of the page apart, so many tokens' are brought
+// sixteen at a time through shared memory and written in runs of a page's row.
+// 16 query and 8 key heads of 128 on 8 value heads of 128, us: 2,048 tokens 31 -> 23.7 (34 MB: what is left is a wavefront's work
+// for every head; with eight heads a wavefront, which share sines and cosines, the same), 300 7.1 -> 5.5, 8 3.6 -> 3.3; on 4 of 256,
+// 2,048 38 -> 27.8.
 #include "common.h"
 
 using namespace jle;
@@ -33,18 +38,53 @@ struct HeadsArgs {
   int wq_stride;  // from one query head's norm weights to the next's (0: one for all)
 };
 
+// A block's sixteen tokens of a value head into their pages, 128 elements at a time.
+constexpr int kTileTokens = 16, kTileWidth = 128;  // (256 threads: two rows at a time)
 template <typename T>
-__global__ __launch_bounds__(64) void heads_prepare_kernel(HeadsArgs<T> a) {
-  __shared__ float sh[kMaxPerLane * 64];
-  const int n = blockIdx.x, h = blockIdx.y, lane = threadIdx.x;
+__device__ __forceinline__ void write_values(const HeadsArgs<T>& a, T (&tile)[kTileTokens][kTileWidth + 8], int N, int block) {
+  const int vh = block % a.Hv, t0 = block / a.Hv * kTileTokens;
+  const int share = a.Hk / a.Hv, j = threadIdx.x & 15;
+  const size_t plane = (size_t)a.Hk * a.ps * a.D;
+  const int slot = t0 + j < N ? a.slot_mapping[t0 + j] : -1;
+  const T* src = a.rows + (size_t)t0 * a.ld + (a.Hq + a.Hk) * a.dk + vh * a.dv;
+  for (int d0 = 0; d0 < a.D; d0 += kTileWidth) {
+    if (d0 > 0) __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kTileTokens * kTileWidth / 256; ++i) {  // (zeros behind the real elements)
+      const int t = 2 * i + (threadIdx.x >> 7), e = threadIdx.x & (kTileWidth - 1);
+      tile[t][e] = t0 + t < N && d0 + e < a.dv ? src[(size_t)t * a.ld + d0 + e] : T(0);
+    }
+    __syncthreads();
+    if (slot < 0) continue;
+    const int width = min(kTileWidth, a.D - d0);
+    for (int s = 0; s < share; ++s) {
+      T* dst = a.kv_cache + (size_t)(slot / a.ps) * 2 * plane + plane + ((size_t)(vh * share + s) * a.D + d0) * a.ps + slot % a.ps;
+      for (int d = threadIdx.x >> 4; d < width; d += 16) dst[(size_t)d * a.ps] = tile[j][d];
+    }
+  }
+}
+
+// value_blocks: the first blocks, which write the values sixteen tokens at a time (0: a wavefront per token and value head)
+template <typename T, int PER>
+__global__ __launch_bounds__(256) void heads_prepare_kernel(HeadsArgs<T> a, int N, int value_blocks) {
+  __shared__ float sh_all[4][PER * 64];
+  __shared__ T tile[kTileTokens][kTileWidth + 8];
+  if ((int)blockIdx.x < value_blocks) {
+    write_values(a, tile, N, blockIdx.x);
+    return;
+  }
+  const int lane = threadIdx.x & 63, wave = wave_index();
+  float* sh = sh_all[wave];
+  const int heads = a.kv_cache == nullptr ? a.Hq : a.Hq + a.Hk + (value_blocks > 0 ? 0 : a.Hv);
+  const int item = (int)(blockIdx.x - value_blocks) * (int)(blockDim.x >> 6) + wave, n = item / heads, h = item - n * heads;
+  if (n >= N) return;
   const bool is_q = h < a.Hq, is_v = h >= a.Hq + a.Hk;
-  if (!is_q && a.kv_cache == nullptr) return;
   const int dim = is_v ? a.dv : a.dk;
   const int c0 = is_v ? (a.Hq + a.Hk) * a.dk + (h - a.Hq - a.Hk) * a.dv : h * a.dk;
   const T* src = a.rows + (size_t)n * a.ld + c0;
-  float x[kMaxPerLane];
+  float x[PER];
 #pragma unroll
-  for (int i = 0; i < kMaxPerLane; ++i) {
+  for (int i = 0; i < PER; ++i) {
     const int e = lane + 64 * i;
     x[i] = e < dim ? Num<T>::load(src + e) : 0.f;
   }
@@ -53,10 +93,10 @@ __global__ __launch_bounds__(64) void heads_prepare_kernel(HeadsArgs<T> a) {
     if (a.norm_eps >= 0.f && a.norm_first) {
       float ss = 0.f;
 #pragma unroll
-      for (int i = 0; i < kMaxPerLane; ++i) ss = __builtin_fmaf(x[i], x[i], ss);
+      for (int i = 0; i < PER; ++i) ss = __builtin_fmaf(x[i], x[i], ss);
       const float inv = 1.0f / sqrtf(wave_sum(ss) / (float)dim + a.norm_eps);
 #pragma unroll
-      for (int i = 0; i < kMaxPerLane; ++i) {
+      for (int i = 0; i < PER; ++i) {
         const int e = lane + 64 * i;
         if (e < dim) x[i] = w != nullptr ? x[i] * inv * w[e] : x[i] * inv;
       }
@@ -65,10 +105,11 @@ __global__ __launch_bounds__(64) void heads_prepare_kernel(HeadsArgs<T> a) {
       const int rd = a.rotary_dim, hr = rd / 2;
       const float pos = (float)a.positions[n];
 #pragma unroll
-      for (int i = 0; i < kMaxPerLane; ++i) sh[lane + 64 * i] = x[i];
-      __syncthreads();
+      for (int i = 0; i < PER; ++i) sh[lane + 64 * i] = x[i];
+      asm volatile("" ::: "memory");  // (the wavefront's own place: its writes come before its reads)
+      __builtin_amdgcn_wave_barrier();
 #pragma unroll
-      for (int i = 0; i < kMaxPerLane; ++i) {
+      for (int i = 0; i < PER; ++i) {
         const int e = lane + 64 * i;
         if (e < rd) {
           const bool first = a.half_pairs ? e < hr : (e & 1) == 0;
@@ -86,10 +127,10 @@ __global__ __launch_bounds__(64) void heads_prepare_kernel(HeadsArgs<T> a) {
     if (a.norm_eps >= 0.f && !a.norm_first) {
       float ss = 0.f;
 #pragma unroll
-      for (int i = 0; i < kMaxPerLane; ++i) ss = __builtin_fmaf(x[i], x[i], ss);
+      for (int i = 0; i < PER; ++i) ss = __builtin_fmaf(x[i], x[i], ss);
       const float inv = 1.0f / sqrtf(wave_sum(ss) / (float)dim + a.norm_eps);
 #pragma unroll
-      for (int i = 0; i < kMaxPerLane; ++i) {
+      for (int i = 0; i < PER; ++i) {
         const int e = lane + 64 * i;
         if (e < dim) x[i] = w != nullptr ? x[i] * inv * w[e] : x[i] * inv;
       }
@@ -98,7 +139,7 @@ __global__ __launch_bounds__(64) void heads_prepare_kernel(HeadsArgs<T> a) {
   if (is_q) {
     T* dst = a.q_out + ((size_t)n * a.Hq + h) * a.D;
 #pragma unroll
-    for (int i = 0; i < kMaxPerLane; ++i) {
+    for (int i = 0; i < PER; ++i) {
       const int e = lane + 64 * i;
       if (e < a.D) Num<T>::store(dst + e, x[i]);  // (zeros behind the real elements)
     }
@@ -111,7 +152,7 @@ __global__ __launch_bounds__(64) void heads_prepare_kernel(HeadsArgs<T> a) {
   if (!is_v) {
     T* dst = a.kv_cache + page * 2 * plane + ((size_t)(h - a.Hq) * a.ps + off) * a.D;
 #pragma unroll
-    for (int i = 0; i < kMaxPerLane; ++i) {
+    for (int i = 0; i < PER; ++i) {
       const int e = lane + 64 * i;
       if (e < a.D) Num<T>::store(dst + e, x[i]);
     }
@@ -121,7 +162,7 @@ __global__ __launch_bounds__(64) void heads_prepare_kernel(HeadsArgs<T> a) {
   for (int s = 0; s < share; ++s) {
     T* dst = a.kv_cache + page * 2 * plane + plane + (size_t)(vh * share + s) * a.ps * a.D + off;
 #pragma unroll
-    for (int i = 0; i < kMaxPerLane; ++i) {
+    for (int i = 0; i < PER; ++i) {
       const int e = lane + 64 * i;
       if (e < a.D) Num<T>::store(dst + (size_t)e * a.ps, x[i]);
     }
@@ -172,16 +213,25 @@ JLE_API int jle_heads_prepare(const void* rows, int ld, const int* positions, co
   if (kv_cache != nullptr && slot_mapping == nullptr) return JLE_BAD_ARG;
   if (wq_stride != 0 && wq_stride != dk) return JLE_BAD_ARG;
   if (ld < (Hq + Hk) * dk + Hv * dv) return JLE_BAD_ARG;
-  const dim3 grid(N, Hq + Hk + Hv);
+  // Values through shared memory from 256 tokens on (fewer are mostly single tokens of several requests, each in a page of its
+  // own); four wavefronts a block then.
+  const long long value_blocks = kv_cache != nullptr && N >= 256 ? (long long)(N + kTileTokens - 1) / kTileTokens * Hv : 0;
+  const long long items = (long long)N * (kv_cache == nullptr ? Hq : Hq + Hk + (value_blocks > 0 ? 0 : Hv));
+  const int waves = value_blocks > 0 ? 4 : 1;
+  const long long blocks = value_blocks + (items + waves - 1) / waves;
+  if (blocks > (1ll << 28)) return JLE_BAD_ARG;
+#define GO(T, PER)                                                                                                            \
+  hipLaunchKernelGGL((heads_prepare_kernel<T, PER>), dim3((unsigned)blocks), dim3(64 * waves), 0, s,                          \
+                     HeadsArgs<T>{(const T*)rows, positions, slot_mapping, inv_freq, wq, wk, (T*)q_out, (T*)kv_cache, magnitude, \
+                                  norm_eps, rotary_dim, half_pairs, norm_first, Hq, Hk, Hv, dk, dv, D, ps, ld, wq_stride},     \
+                     N, (int)value_blocks)
+  const int per = D <= 128 ? 2 : D <= 256 ? 4 : kMaxPerLane;
   if (is_bf16) {
-    HeadsArgs<bf16_t> a{(const bf16_t*)rows, positions, slot_mapping, inv_freq, wq, wk, (bf16_t*)q_out, (bf16_t*)kv_cache,
-                        magnitude, norm_eps, rotary_dim, half_pairs, norm_first, Hq, Hk, Hv, dk, dv, D, ps, ld, wq_stride};
-    hipLaunchKernelGGL(heads_prepare_kernel<bf16_t>, grid, dim3(64), 0, s, a);
+    if (per == 2) GO(bf16_t, 2); else if (per == 4) GO(bf16_t, 4); else GO(bf16_t, kMaxPerLane);
   } else {
-    HeadsArgs<float> a{(const float*)rows, positions, slot_mapping, inv_freq, wq, wk, (float*)q_out, (float*)kv_cache,
-                       magnitude, norm_eps, rotary_dim, half_pairs, norm_first, Hq, Hk, Hv, dk, dv, D, ps, ld, wq_stride};
-    hipLaunchKernelGGL(heads_prepare_kernel<float>, grid, dim3(64), 0, s, a);
+    if (per == 2) GO(float, 2); else if (per == 4) GO(float, 4); else GO(float, kMaxPerLane);
   }
+#undef GO
   JLE_LAUNCH_CHECK();
   return 0;
 }

@@ -2122,3 +2122,28 @@ def test_dense_products_replayed(ops):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(y, ops.linear(x, w)) and torch.equal(z, ops.swiglu_linear(y[:, :1024].contiguous(), w))
+
+
+@pytest.mark.parametrize("dt", DT)
+@pytest.mark.parametrize("hq,hk,hv,dk,dv,page,ps", [(4, 2, 2, 128, 128, 128, 16), (2, 4, 2, 64, 136, 144, 16), (3, 3, 1, 96, 300, 320, 32), (2, 1, 1, 20, 12, 24, 8)])
+def test_heads_of_many_tokens_prepared(ops, dt, hq, hk, hv, dk, dv, page, ps):
+    """Values written sixteen tokens at a time: what the same tokens give in calls of fewer than 256, in scattered slots of pages."""
+    import types
+    n = 259
+    rows = _rand(n, (hq + hk) * dk + hv * dv, dt=dt, seed=1)
+    rot = types.SimpleNamespace(inv_freq=_rand(dk // 4, seed=2).abs(), rotary_dim=dk // 4 * 2, magnitude=1.1, pairing="half")
+    prep = types.SimpleNamespace(query_scale=None, norm_span="head", rotation=rot, norm_weight_q=_rand(dk, seed=3), norm_weight_k=None,
+                                 norm_eps=1e-5, norm_first=True)
+    slots = torch.randperm((n // ps + 3) * ps, generator=torch.Generator().manual_seed(4))[:n].int().to(DEV)
+    positions = torch.arange(n, dtype=torch.int32, device=DEV)
+    got = []
+    for cuts in ((0, n), (0, 200, n)):
+        pages = torch.full((n // ps + 3, 2, hk, ps, page), 7.0, dtype=dt, device=DEV)
+        q = [ops.heads_prepare(rows[a:b], hq, hk, hv, dk, dv, page, prep, positions[a:b], pages, slots[a:b]) for a, b in zip(cuts, cuts[1:])]
+        got.append((torch.cat(q), pages))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+    plain = torch.cat([ops.heads_prepare(rows[a:b], hq, hk, hv, dk, dv, page, prep, positions[a:b], None, None) for a, b in ((0, 3), (3, n))])
+    assert torch.equal(plain, got[0][0])
+    values = got[0][1][:, 1].reshape(-1, hk, page, ps)[(slots // ps).long(), :, :, (slots % ps).long()]  # [n, hk, page]
+    want = rows[:, (hq + hk) * dk:].reshape(n, hv, dv).repeat_interleave(hk // hv, 1)
+    assert torch.equal(values[..., :dv], want) and not values[..., dv:].any()
