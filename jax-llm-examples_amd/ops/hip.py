@@ -1179,16 +1179,13 @@ class HipOps:
         chip's power is what both wait for), and those with too few tiles for its compute units and a long k, which the library
         cuts along k (704 of 4,096 x 7,168 (k) 51 | 63, 1,024 of 2,048 x 8,192 (k) 49 | 65).  With the gate it is measured against the
         library's product and the activation's launch: 2,048 rows of 8,192 x 5,120 277 | 247, 953 150 | 123, 8,191 of 14,336 x
-        4,096 1,385 | 1,366, but 97 of 8,192 x 5,120 47 | 65; with
-        256 rows it gains 4 %, 70 | 67, and the line lies above them: in mixed steps of a few hundred rows the activation of gate and
-        up that were not rounded first took the worst of 64 requests' logits from 0.0147 of the largest to 0.0151, where 0.015 is
-        allowed (the errors of whole prompts against 64 bits are smaller with it, 2.4e-3 -> 2.1e-3: it is the tail that moved)."""
+        4,096 1,385 | 1,366, but 97 of 8,192 x 5,120 47 | 65, and with 256 70 | 67."""
         if rows < 1 or n < 8 or n % 8 or k < 64 or k % 64 or k >= 1 << 23 or gated and 4 * n * k >= 1 << 32:
             return 0
         wide = 2 * n if gated else n  # rows of W
         small = -(-rows // 128) * -(-wide // 128)
         if gated:
-            if rows < 384 or small < 0.9 * units:
+            if rows < 256 or small < 0.9 * units:
                 return 0
         else:
             if not (rows >= 192 and k <= 2048 or rows >= 256 and small >= (0.93 if k <= 6144 else 1.17) * units):
@@ -1293,8 +1290,8 @@ class HipOps:
             product = self.gemm_few if self._few(h, w_gate_up) else self.gemm_skinny
             return product(h, w_gate_up, swiglu=1 + act)  # (the activation in the product's epilogue)
         out = self._dense_float32(h, w_gate_up, act)
-        if out is None and act == 0:
-            out = self._dense(h, w_gate_up, gated=True)
+        # (not gemm_dense.hip's epilogue: a launch of 18 us less, but gate and up that are not rounded first took the worst of 64
+        # requests' logits in mixed steps of up to 1,709 rows from 0.0147 of the largest to 0.0151, where 0.015 is allowed)
         return self.silu_mul(self._product(h, w_gate_up), activation) if out is None else out
 
     def _product(self, h, w):
