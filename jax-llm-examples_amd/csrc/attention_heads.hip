@@ -11,9 +11,9 @@
 // through no more code than its heads need).  Everything in float32; the order of every sum depends on the sizes only.
 // Values lie transposed in their pages: a token's are single elements a row of the page apart, so many tokens' are brought
 // sixteen at a time through shared memory and written in runs of a page's row.
-// 16 query and 8 key heads of 128 on 8 value heads of 128, us: 2,048 tokens 31 -> 23.7 (34 MB: what is left is a wavefront's work
-// for every head; with eight heads a wavefront, which share sines and cosines, the same), 300 7.1 -> 5.5, 8 3.6 -> 3.3; on 4 of 256,
-// 2,048 38 -> 27.8.
+// 16 query and 8 key heads of 128 on 8 value heads of 128, us: 2,048 tokens 31 -> 22.6 (34 MB: what is left is a wavefront's work
+// for every head; with eight heads a wavefront, which share sines and cosines, the same), 300 6.9 -> 5.3, 255 7.0 -> 6.5, 8 3.6 ->
+// 3.3; on 4 of 256, 2,048 36 -> 26.1; queries alone, 2,048 19 -> 11.5.
 #include "common.h"
 
 using namespace jle;
@@ -21,6 +21,7 @@ using namespace jle;
 namespace {
 
 constexpr int kMaxPerLane = 8;  // heads of up to 512 elements
+constexpr int per_lane(int D) { return D <= 128 ? 2 : D <= 256 ? 4 : kMaxPerLane; }
 
 template <typename T>
 struct HeadsArgs {
@@ -38,46 +39,48 @@ struct HeadsArgs {
   int wq_stride;  // from one query head's norm weights to the next's (0: one for all)
 };
 
-// A block's sixteen tokens of a value head into their pages, 128 elements at a time.
-constexpr int kTileTokens = 16, kTileWidth = 128;  // (256 threads: two rows at a time)
+// A block's sixteen tokens and 128 elements of a value head into their pages.
+constexpr int kTileTokens = 16, kTileWidth = 128, kTilePitch = kTileWidth + 8;  // (256 threads: two rows at a time)
 template <typename T>
-__device__ __forceinline__ void write_values(const HeadsArgs<T>& a, T (&tile)[kTileTokens][kTileWidth + 8], int N, int block) {
-  const int vh = block % a.Hv, t0 = block / a.Hv * kTileTokens;
+__device__ __forceinline__ void write_values(const HeadsArgs<T>& a, T* tile, int N, int block) {
+  const int columns = (a.D + kTileWidth - 1) / kTileWidth, d0 = block % columns * kTileWidth;
+  const int vh = block / columns % a.Hv, t0 = block / columns / a.Hv * kTileTokens;
   const int share = a.Hk / a.Hv, j = threadIdx.x & 15;
   const size_t plane = (size_t)a.Hk * a.ps * a.D;
   const int slot = t0 + j < N ? a.slot_mapping[t0 + j] : -1;
   const T* src = a.rows + (size_t)t0 * a.ld + (a.Hq + a.Hk) * a.dk + vh * a.dv;
-  for (int d0 = 0; d0 < a.D; d0 += kTileWidth) {
-    if (d0 > 0) __syncthreads();
 #pragma unroll
-    for (int i = 0; i < kTileTokens * kTileWidth / 256; ++i) {  // (zeros behind the real elements)
-      const int t = 2 * i + (threadIdx.x >> 7), e = threadIdx.x & (kTileWidth - 1);
-      tile[t][e] = t0 + t < N && d0 + e < a.dv ? src[(size_t)t * a.ld + d0 + e] : T(0);
-    }
-    __syncthreads();
-    if (slot < 0) continue;
-    const int width = min(kTileWidth, a.D - d0);
-    for (int s = 0; s < share; ++s) {
-      T* dst = a.kv_cache + (size_t)(slot / a.ps) * 2 * plane + plane + ((size_t)(vh * share + s) * a.D + d0) * a.ps + slot % a.ps;
-      for (int d = threadIdx.x >> 4; d < width; d += 16) dst[(size_t)d * a.ps] = tile[j][d];
-    }
+  for (int i = 0; i < kTileTokens * kTileWidth / 256; ++i) {  // (zeros behind the real elements)
+    const int t = 2 * i + (threadIdx.x >> 7), e = threadIdx.x & (kTileWidth - 1);
+    tile[t * kTilePitch + e] = t0 + t < N && d0 + e < a.dv ? src[(size_t)t * a.ld + d0 + e] : T(0);
+  }
+  __syncthreads();
+  if (slot < 0) return;
+  const int width = min(kTileWidth, a.D - d0);
+  for (int s = 0; s < share; ++s) {
+    T* dst = a.kv_cache + (size_t)(slot / a.ps) * 2 * plane + plane + ((size_t)(vh * share + s) * a.D + d0) * a.ps + slot % a.ps;
+    for (int d = threadIdx.x >> 4; d < width; d += 16) dst[(size_t)d * a.ps] = tile[j * kTilePitch + d];
   }
 }
 
-// value_blocks: the first blocks, which write the values sixteen tokens at a time (0: a wavefront per token and value head)
-template <typename T, int PER>
-__global__ __launch_bounds__(256) void heads_prepare_kernel(HeadsArgs<T> a, int N, int value_blocks) {
-  __shared__ float sh_all[4][PER * 64];
-  __shared__ T tile[kTileTokens][kTileWidth + 8];
-  if ((int)blockIdx.x < value_blocks) {
-    write_values(a, tile, N, blockIdx.x);
+// TILES: the first value_blocks blocks write the values sixteen tokens at a time, four wavefronts of the others a token's head each.
+// Else a block is a wavefront of token blockIdx.x and head blockIdx.y, the values' heads behind the keys'.
+template <typename T, int PER, bool TILES>
+__global__ __launch_bounds__(TILES ? 256 : 64) void heads_prepare_kernel(HeadsArgs<T> a, int N, int value_blocks) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];  // a value tile, or PER * 64 floats a wavefront
+  if (TILES && (int)blockIdx.x < value_blocks) {
+    write_values(a, reinterpret_cast<T*>(smem), N, blockIdx.x);
     return;
   }
-  const int lane = threadIdx.x & 63, wave = wave_index();
-  float* sh = sh_all[wave];
-  const int heads = a.kv_cache == nullptr ? a.Hq : a.Hq + a.Hk + (value_blocks > 0 ? 0 : a.Hv);
-  const int item = (int)(blockIdx.x - value_blocks) * (int)(blockDim.x >> 6) + wave, n = item / heads, h = item - n * heads;
-  if (n >= N) return;
+  const int lane = threadIdx.x & 63, wave = TILES ? wave_index() : 0;
+  float* sh = reinterpret_cast<float*>(smem) + wave * PER * 64;
+  int n = blockIdx.x, h = blockIdx.y;
+  if (TILES) {
+    const int heads = a.Hq + a.Hk, item = (int)(blockIdx.x - value_blocks) * 4 + wave;
+    n = item / heads;
+    h = item - n * heads;
+    if (n >= N) return;
+  }
   const bool is_q = h < a.Hq, is_v = h >= a.Hq + a.Hk;
   const int dim = is_v ? a.dv : a.dk;
   const int c0 = is_v ? (a.Hq + a.Hk) * a.dk + (h - a.Hq - a.Hk) * a.dv : h * a.dk;
@@ -198,7 +201,47 @@ __global__ __launch_bounds__(64) void diff_combine_kernel(const T* __restrict__ 
   }
 }
 
+// How N tokens are prepared.  Values through shared memory from 256 tokens on (fewer are mostly single tokens of several requests,
+// each in a page of its own).  A block has the shared memory of what it does and no more, and blocks of one wavefront are dealt
+// out head by head: with room for four wavefronts and a tile in every block, token by token, us: 255 tokens of 16, 8 and 8 heads of 64
+// in bfloat16 6.9, now 5.4; queries alone, float32, 16 heads of 256, 2,048 tokens 29.6, now 16.2.  Wide heads' values are
+// written by a block for every 128 elements: 256 tokens of 2 value heads of 512 10.0, now 5.4.
+struct HeadsPlan {
+  bool tiles;
+  int columns;  // parts of 128 elements of a value head
+  uint32_t lds;
+};
+HeadsPlan heads_plan(int N, int D, bool paged, bool rotary, int size) {
+  HeadsPlan p;
+  p.tiles = paged && N >= 256;
+  p.columns = (D + kTileWidth - 1) / kTileWidth;
+  const uint32_t rows = rotary ? (p.tiles ? 4 : 1) * per_lane(D) * 256 : 0, tile = p.tiles ? kTileTokens * kTilePitch * size : 0;
+  p.lds = rows > tile ? rows : tile;
+  return p;
+}
+
+template <typename T, int PER>
+int launch_heads(const HeadsArgs<T>& a, int N, hipStream_t s) {
+  const HeadsPlan plan = heads_plan(N, a.D, a.kv_cache != nullptr, a.rotary_dim > 0, sizeof(T));
+  if (plan.tiles) {
+    const long long value_blocks = (long long)(N + kTileTokens - 1) / kTileTokens * a.Hv * plan.columns;
+    const long long blocks = value_blocks + ((long long)N * (a.Hq + a.Hk) + 3) / 4;
+    if (blocks > (1ll << 28)) return JLE_BAD_ARG;
+    hipLaunchKernelGGL((heads_prepare_kernel<T, PER, true>), dim3((unsigned)blocks), dim3(256), plan.lds, s, a, N, (int)value_blocks);
+  } else {
+    const int heads = a.kv_cache == nullptr ? a.Hq : a.Hq + a.Hk + a.Hv;
+    hipLaunchKernelGGL((heads_prepare_kernel<T, PER, false>), dim3(N, heads), dim3(64), plan.lds, s, a, N, 0);
+  }
+  JLE_LAUNCH_CHECK();
+  return 0;
+}
+
 }  // namespace
+
+// Bytes of shared memory of a block that prepares some of N tokens.
+JLE_API int jle_heads_prepare_shared(int N, int D, int paged, int rotary, int is_bf16) {
+  return (int)heads_plan(N, D, paged != 0, rotary != 0, is_bf16 ? 2 : 4).lds;
+}
 
 JLE_API int jle_heads_prepare(const void* rows, int ld, const int* positions, const int* slot_mapping, const float* inv_freq,
                               int rotary_dim, int half_pairs, float magnitude, float norm_eps, int norm_first,
@@ -213,27 +256,13 @@ JLE_API int jle_heads_prepare(const void* rows, int ld, const int* positions, co
   if (kv_cache != nullptr && slot_mapping == nullptr) return JLE_BAD_ARG;
   if (wq_stride != 0 && wq_stride != dk) return JLE_BAD_ARG;
   if (ld < (Hq + Hk) * dk + Hv * dv) return JLE_BAD_ARG;
-  // Values through shared memory from 256 tokens on (fewer are mostly single tokens of several requests, each in a page of its
-  // own); four wavefronts a block then.
-  const long long value_blocks = kv_cache != nullptr && N >= 256 ? (long long)(N + kTileTokens - 1) / kTileTokens * Hv : 0;
-  const long long items = (long long)N * (kv_cache == nullptr ? Hq : Hq + Hk + (value_blocks > 0 ? 0 : Hv));
-  const int waves = value_blocks > 0 ? 4 : 1;
-  const long long blocks = value_blocks + (items + waves - 1) / waves;
-  if (blocks > (1ll << 28)) return JLE_BAD_ARG;
-#define GO(T, PER)                                                                                                            \
-  hipLaunchKernelGGL((heads_prepare_kernel<T, PER>), dim3((unsigned)blocks), dim3(64 * waves), 0, s,                          \
-                     HeadsArgs<T>{(const T*)rows, positions, slot_mapping, inv_freq, wq, wk, (T*)q_out, (T*)kv_cache, magnitude, \
-                                  norm_eps, rotary_dim, half_pairs, norm_first, Hq, Hk, Hv, dk, dv, D, ps, ld, wq_stride},     \
-                     N, (int)value_blocks)
-  const int per = D <= 128 ? 2 : D <= 256 ? 4 : kMaxPerLane;
-  if (is_bf16) {
-    if (per == 2) GO(bf16_t, 2); else if (per == 4) GO(bf16_t, 4); else GO(bf16_t, kMaxPerLane);
-  } else {
-    if (per == 2) GO(float, 2); else if (per == 4) GO(float, 4); else GO(float, kMaxPerLane);
-  }
-#undef GO
-  JLE_LAUNCH_CHECK();
-  return 0;
+  const HeadsArgs<bf16_t> a = {(const bf16_t*)rows, positions, slot_mapping, inv_freq, wq, wk, (bf16_t*)q_out, (bf16_t*)kv_cache, magnitude,
+                               norm_eps, rotary_dim, half_pairs, norm_first, Hq, Hk, Hv, dk, dv, D, ps, ld, wq_stride};
+  const HeadsArgs<float> f = {(const float*)rows, positions, slot_mapping, inv_freq, wq, wk, (float*)q_out, (float*)kv_cache, magnitude,
+                              norm_eps, rotary_dim, half_pairs, norm_first, Hq, Hk, Hv, dk, dv, D, ps, ld, wq_stride};
+  if (per_lane(D) == 2) return is_bf16 ? launch_heads<bf16_t, 2>(a, N, s) : launch_heads<float, 2>(f, N, s);
+  if (per_lane(D) == 4) return is_bf16 ? launch_heads<bf16_t, 4>(a, N, s) : launch_heads<float, 4>(f, N, s);
+  return is_bf16 ? launch_heads<bf16_t, kMaxPerLane>(a, N, s) : launch_heads<float, kMaxPerLane>(f, N, s);
 }
 
 // o [N, 2 H, D] in the order [kv head][map][query head of the group]; gate [N, H dv] or null; out [N, H dv].

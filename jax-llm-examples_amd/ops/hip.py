@@ -198,7 +198,7 @@ def _bind(path: str):
             fn.restype = ctypes.c_int
     for name, args in (("jle_attention_mfma_supported", [_i, _i, _i, _i]),  # queries, not launches: no stream
                        ("jle_greedy_blocks", [_i]), ("jle_gemm_stream_supported", [_i, _i, _i]), ("jle_gemm_stream_room", [_i, _i]), ("jle_gemm_f32_stream_supported", [_i, _i, _i]),
-                       ("jle_gemm_few_tiles", [_i] * 7),
+                       ("jle_gemm_few_tiles", [_i] * 7), ("jle_heads_prepare_shared", [_i] * 5),
                        ("jle_latent_attention_mfma_supported", [_i, _i, _i, _i, _i]),
                        ("jle_latent_values_supported", [_i] * 6),
                        ("jle_latent_expanded_supported", [_i, _i, _i, _i, _i]), ("jle_attention_group_waves", []),

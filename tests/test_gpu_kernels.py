@@ -2125,7 +2125,7 @@ def test_dense_products_replayed(ops):
 
 
 @pytest.mark.parametrize("dt", DT)
-@pytest.mark.parametrize("hq,hk,hv,dk,dv,page,ps", [(4, 2, 2, 128, 128, 128, 16), (2, 4, 2, 64, 136, 144, 16), (3, 3, 1, 96, 300, 320, 32), (2, 1, 1, 20, 12, 24, 8)])
+@pytest.mark.parametrize("hq,hk,hv,dk,dv,page,ps", [(4, 2, 2, 128, 128, 128, 16), (2, 4, 2, 64, 136, 144, 16), (3, 3, 1, 96, 300, 320, 32), (2, 1, 1, 20, 12, 24, 8), (2, 4, 2, 256, 512, 512, 16)])
 def test_heads_of_many_tokens_prepared(ops, dt, hq, hk, hv, dk, dv, page, ps):
     """Values written sixteen tokens at a time: what the same tokens give in calls of fewer than 256, in scattered slots of pages."""
     import types
@@ -2147,3 +2147,11 @@ def test_heads_of_many_tokens_prepared(ops, dt, hq, hk, hv, dk, dv, page, ps):
     values = got[0][1][:, 1].reshape(-1, hk, page, ps)[(slots // ps).long(), :, :, (slots % ps).long()]  # [n, hk, page]
     want = rows[:, (hq + hk) * dk:].reshape(n, hv, dv).repeat_interleave(hk // hv, 1)
     assert torch.equal(values[..., :dv], want) and not values[..., dv:].any()
+
+
+@pytest.mark.parametrize("n,dim,paged,rotary,bf16,bytes_", [
+    (255, 64, 1, 1, 1, 512), (9, 128, 1, 1, 0, 512), (200, 256, 1, 1, 0, 1024), (255, 512, 1, 1, 1, 2048), (2048, 512, 0, 1, 0, 2048), (300, 128, 0, 0, 1, 0),
+    (256, 128, 1, 1, 1, 4352), (256, 128, 1, 1, 0, 8704), (256, 512, 1, 1, 1, 8192), (256, 64, 1, 0, 1, 4352)])
+def test_heads_take_the_shared_memory_of_what_a_block_does(ops, n, dim, paged, rotary, bf16, bytes_):
+    """A wavefront of its own: its head and no room for others or for a value tile, so that 32 of them fit a compute unit's 160 KB."""
+    assert ops._query("jle_heads_prepare_shared", n, dim, paged, rotary, bf16) == bytes_
