@@ -210,29 +210,37 @@ struct HeadsPlan {
   bool tiles;
   int columns;  // parts of 128 elements of a value head
   uint32_t lds;
+  int step;  // tokens a launch: its threads are fewer than 2^32
 };
-HeadsPlan heads_plan(int N, int D, bool paged, bool rotary, int size) {
+HeadsPlan heads_plan(int N, int heads, int D, bool paged, bool rotary, int size) {
   HeadsPlan p;
   p.tiles = paged && N >= 256;
   p.columns = (D + kTileWidth - 1) / kTileWidth;
   const uint32_t rows = rotary ? (p.tiles ? 4 : 1) * per_lane(D) * 256 : 0, tile = p.tiles ? kTileTokens * kTilePitch * size : 0;
   p.lds = rows > tile ? rows : tile;
+  p.step = max(kTileTokens, (1 << 25) / heads / kTileTokens * kTileTokens);
   return p;
 }
 
 template <typename T, int PER>
-int launch_heads(const HeadsArgs<T>& a, int N, hipStream_t s) {
-  const HeadsPlan plan = heads_plan(N, a.D, a.kv_cache != nullptr, a.rotary_dim > 0, sizeof(T));
-  if (plan.tiles) {
-    const long long value_blocks = (long long)(N + kTileTokens - 1) / kTileTokens * a.Hv * plan.columns;
-    const long long blocks = value_blocks + ((long long)N * (a.Hq + a.Hk) + 3) / 4;
-    if (blocks > (1ll << 28)) return JLE_BAD_ARG;
-    hipLaunchKernelGGL((heads_prepare_kernel<T, PER, true>), dim3((unsigned)blocks), dim3(256), plan.lds, s, a, N, (int)value_blocks);
-  } else {
-    const int heads = a.kv_cache == nullptr ? a.Hq : a.Hq + a.Hk + a.Hv;
-    hipLaunchKernelGGL((heads_prepare_kernel<T, PER, false>), dim3(N, heads), dim3(64), plan.lds, s, a, N, 0);
+int launch_heads(HeadsArgs<T> a, int N, hipStream_t s) {
+  const HeadsPlan plan = heads_plan(N, a.Hq + a.Hk + a.Hv, a.D, a.kv_cache != nullptr, a.rotary_dim > 0, sizeof(T));
+  for (int left = N; left > 0; left -= plan.step) {
+    const int n = min(left, plan.step);
+    if (plan.tiles) {
+      const int value_blocks = (n + kTileTokens - 1) / kTileTokens * a.Hv * plan.columns;
+      const int blocks = value_blocks + (n * (a.Hq + a.Hk) + 3) / 4;
+      hipLaunchKernelGGL((heads_prepare_kernel<T, PER, true>), dim3((unsigned)blocks), dim3(256), plan.lds, s, a, n, value_blocks);
+    } else {
+      const int heads = a.kv_cache == nullptr ? a.Hq : a.Hq + a.Hk + a.Hv;
+      hipLaunchKernelGGL((heads_prepare_kernel<T, PER, false>), dim3(n, heads), dim3(64), plan.lds, s, a, n, 0);
+    }
+    JLE_LAUNCH_CHECK();
+    a.rows += (size_t)n * a.ld;
+    a.q_out += (size_t)n * a.Hq * a.D;
+    if (a.positions != nullptr) a.positions += n;
+    if (a.slot_mapping != nullptr) a.slot_mapping += n;
   }
-  JLE_LAUNCH_CHECK();
   return 0;
 }
 
@@ -240,7 +248,7 @@ int launch_heads(const HeadsArgs<T>& a, int N, hipStream_t s) {
 
 // Bytes of shared memory of a block that prepares some of N tokens.
 JLE_API int jle_heads_prepare_shared(int N, int D, int paged, int rotary, int is_bf16) {
-  return (int)heads_plan(N, D, paged != 0, rotary != 0, is_bf16 ? 2 : 4).lds;
+  return (int)heads_plan(N, 1, D, paged != 0, rotary != 0, is_bf16 ? 2 : 4).lds;
 }
 
 JLE_API int jle_heads_prepare(const void* rows, int ld, const int* positions, const int* slot_mapping, const float* inv_freq,

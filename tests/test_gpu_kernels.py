@@ -2155,3 +2155,23 @@ def test_heads_of_many_tokens_prepared(ops, dt, hq, hk, hv, dk, dv, page, ps):
 def test_heads_take_the_shared_memory_of_what_a_block_does(ops, n, dim, paged, rotary, bf16, bytes_):
     """A wavefront of its own: its head and no room for others or for a value tile, so that 32 of them fit a compute unit's 160 KB."""
     assert ops._query("jle_heads_prepare_shared", n, dim, paged, rotary, bf16) == bytes_
+
+
+def test_heads_of_more_tokens_than_a_launch_takes(ops):
+    """2^26 heads and more: threads of two launches and a rest; the same as in calls of a part each."""
+    import types
+    n, hq, d, ps = (1 << 20) + 37, 64, 2, 16
+    rows = _rand(n, (hq + 2) * d, dt=torch.bfloat16, seed=1)
+    prep = types.SimpleNamespace(query_scale=None, norm_span="head", rotation=None, norm_weight_q=None, norm_weight_k=None, norm_eps=1e-5,
+                                 norm_first=True)
+    slots = torch.randperm(n + 11, generator=torch.Generator().manual_seed(2))[:n].int().to(DEV)
+    positions = torch.arange(n, dtype=torch.int32, device=DEV)
+    got = []
+    for cuts in ((0, n), (0, 1 << 19, n)):
+        pages = torch.zeros(n // ps + 2, 2, 1, ps, d, dtype=torch.bfloat16, device=DEV)
+        q = torch.cat([ops.heads_prepare(rows[a:b], hq, 1, 1, d, d, d, prep, positions[a:b], pages, slots[a:b]) for a, b in zip(cuts, cuts[1:])])
+        got.append((q, pages))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+    assert torch.equal(ops.heads_prepare(rows, hq, 1, 1, d, d, d, prep, positions, None, None), got[0][0])
+    values = got[0][1][:, 1].reshape(-1, d, ps)[(slots // ps).long(), :, (slots % ps).long()]
+    assert torch.equal(values, rows[:, -d:])
