@@ -743,14 +743,15 @@ static int launch_align(const int* ids, const float* gates, int* offsets, int* s
                         int* inv, int M, int E, int k, int extra, int inv_ld, hipStream_t s) {
   // A wavefront looks at all its pairs for every expert; moe_align_kernel's meet at four barriers, 3.6 to 3.7 us up to 256 pairs
   // whatever the experts.  One wavefront, us: 64 pairs of 8 experts 2.3, of 32 3.6, of 48 5.4; 128 of 8 2.6, of 16 3.2; 256 of 8
-  // 3.1, of 16 4.1, of 32 6.1.
-  if (M <= 256 && (M + 63) / 64 * E <= 40) {
+  // 3.1, of 16 4.1, of 32 6.1.  Above 256 pairs, one | all: 320 of 2 experts 2.7 | 3.7, of 4 3.0 | 3.7, of 6 3.4 | 3.7, of 8 3.7 | 3.7.
+  if (M <= (E <= 6 ? 384 : 256) && (M + 63) / 64 * E <= 40) {
 #define WAVE(R_) \
   hipLaunchKernelGGL(moe_align_wave_kernel<R_>, dim3(1), dim3(64), 0, s, ids, gates, offsets, sorted_token, sorted_gate, inv, M, E, \
                      k, extra, inv_ld)
     if (M <= 64) WAVE(1);
     else if (M <= 128) WAVE(2);
-    else WAVE(4);
+    else if (M <= 256) WAVE(4);
+    else WAVE(6);
 #undef WAVE
     JLE_LAUNCH_CHECK();
     return 0;

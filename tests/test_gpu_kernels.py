@@ -995,7 +995,7 @@ def test_moe_align_at_the_edges_of_one_wavefront(ops, n, k, e):
     assert inv.view(n, k + 1).tolist() == [[row.get(t * k + j, -1) for j in range(k)] + [len(order) + t] for t in range(n)]
 
 
-@pytest.mark.parametrize("n,k,e", [(257, 1, 8), (1024, 1, 63), (1025, 4, 64), (4096, 1, 1), (4097, 1, 300), (8193, 2, 10), (700, 1, 4096), (333, 1, 2048)])
+@pytest.mark.parametrize("n,k,e", [(257, 1, 6), (160, 2, 3), (384, 1, 6), (385, 1, 6), (257, 1, 7), (257, 1, 8), (1024, 1, 63), (1025, 4, 64), (4096, 1, 1), (4097, 1, 300), (8193, 2, 10), (700, 1, 4096), (333, 1, 2048)])
 def test_moe_align_of_many_pairs(ops, n, k, e):
     """Runs of pairs that end within 64 and past the ones that a wavefront asks for at once, more experts than a look takes and than
     sixteen wavefronts count; even, all of one expert, and with choices that have no row."""
