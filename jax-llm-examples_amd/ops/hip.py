@@ -14,6 +14,7 @@ from typing import Optional
 import numpy as np
 import torch
 from torch.autograd import forward_ad
+from torch.utils._device import DeviceContext
 
 from . import build as _build
 from .transfer import to_device
@@ -230,9 +231,18 @@ def _p(t: Optional[torch.Tensor]):
 
 
 def _watched() -> bool:
-    """Whether the operations are looked at while they run: derivatives in forward mode, function transforms, dispatch modes."""
-    return (forward_ad._current_level >= 0 or torch._C._functorch.peek_interpreter_stack() is not None
-            or torch._C._len_torch_dispatch_stack() > 0)
+    """Whether the operations are looked at, or changed, while they run: compiled or traced, derivatives in forward mode, function
+    transforms, dispatch modes, function modes (but a default device's, which concerns new tensors only), autocast."""
+    return (torch.compiler.is_compiling() or forward_ad._current_level >= 0
+            or torch._C._functorch.peek_interpreter_stack() is not None or torch._C._len_torch_dispatch_stack() > 0
+            or torch._C._len_torch_function_stack() > 0
+            and not all(isinstance(m, DeviceContext) for m in torch.overrides._get_current_function_mode_stack())
+            or torch.is_autocast_enabled("cuda") or torch._C._get_tracing_state() is not None)
+
+
+def _plain(t) -> bool:
+    """Whether a tensor is of no class of its own, which may have no memory and whose products may be something else."""
+    return type(t) is torch.Tensor or type(t) is torch.nn.Parameter or not isinstance(t, torch.Tensor)
 
 
 class HipOps:
@@ -1214,11 +1224,11 @@ class HipOps:
         n = w.shape[0] // 2 if gated else w.shape[0]
         tile = HipOps.dense_tile(m, n, k, gated, self._compute_units)
         if (not tile or not h.get_device() == w.get_device() == self._device_index or not (h.is_contiguous() and w.is_contiguous())
-                or (h.data_ptr() | w.data_ptr()) % 16
+                or _watched() or not (_plain(h) and _plain(w) and _plain(bias))
+                or not h.data_ptr() or not w.data_ptr() or (h.data_ptr() | w.data_ptr()) % 16
                 or bias is not None and (bias.dtype != torch.bfloat16 or bias.shape != (n,) or not bias.is_contiguous()
                                          or bias.get_device() != self._device_index or bias.data_ptr() % 8)
-                or torch.is_grad_enabled() and (h.requires_grad or w.requires_grad or bias is not None and bias.requires_grad)
-                or _watched()):
+                or torch.is_grad_enabled() and (h.requires_grad or w.requires_grad or bias is not None and bias.requires_grad)):
             return None
         return self.gemm_dense(h, w, tile, gated, bias)
 

@@ -240,3 +240,46 @@ def test_dense_products_that_are_left_to_the_library():
         assert not taken(h, w)
     with torch.no_grad():
         assert taken(at(2048, 4096, requires_grad=True), w)
+
+
+class Elsewhere(torch.Tensor):
+    """A class of its own around no memory, whose operations it answers itself."""
+    __torch_function__ = torch._C._disabled_torch_function_impl
+
+    @staticmethod
+    def __new__(cls, rows, cols):
+        return torch.Tensor._make_wrapper_subclass(cls, (rows, cols), dtype=torch.bfloat16, device="cuda:0")
+
+    @classmethod
+    def __torch_dispatch__(cls, func, types, args=(), kwargs=None):
+        return func
+
+
+def test_dense_products_that_others_look_into_are_left_to_the_library():
+    def at(rows, cols, address=4096):
+        return types.SimpleNamespace(dtype=torch.bfloat16, shape=(rows, cols), dim=lambda: 2, get_device=lambda: 0, is_contiguous=lambda: True,
+                                     data_ptr=lambda: address, requires_grad=False)
+
+    ops = types.SimpleNamespace(_compute_units=256, _device_index=0, gemm_dense=lambda h, w, tile, gated, bias: tile)
+    h, w = at(2048, 4096), at(4096, 4096)
+    taken = lambda h=h, w=w, **kw: HipOps._dense(ops, h, w, **kw) is not None
+    assert taken() and not taken(h=Elsewhere(2048, 4096)) and not taken(w=Elsewhere(4096, 4096)) and not taken(h=at(2048, 4096, address=0))
+
+    class Mode(torch.overrides.TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    with Mode():
+        assert not taken()
+    with torch.device("cpu"):
+        assert taken()
+        with Mode():
+            assert not taken()
+    try:
+        torch.set_autocast_enabled("cuda", True)
+        assert not taken()
+    finally:
+        torch.set_autocast_enabled("cuda", False)
+    seen = []
+    torch.jit.trace(lambda x: (seen.append(taken()), x)[1], torch.zeros(1), check_trace=False)
+    assert seen and not any(seen) and taken()
