@@ -104,11 +104,12 @@ struct DenseBlock {
   int N, K;            // columns of Y
 };
 
-// TILED: W in the streaming layout, whose kilobytes (16 rows of 32 k) are fragments as a wavefront reads them.
+// TILED: W in the streaming layout, whose kilobytes (16 rows of 32 k) are fragments as a wavefront reads them.  GATED: gate rows
+// first, silu(gate) * up of the sums.
 template <int FM, int FN, int RX, int RW, bool GATED, bool TILED>
 __device__ __forceinline__ void dense_block(const DenseBlock& p, unsigned char* smem) {
   using R = Ring<FM, FN, RX, RW>;
-  static_assert(!GATED || FN % 2 == 0, "a wavefront has a gate's fragments and their up's");
+  static_assert(!GATED || (TILED && FN % 2 == 0), "a wavefront has a gate's fragments and their up's");
   constexpr int U = FM + FN, MF = FM * FN;
   constexpr uint32_t KX = BK * 2, KW = TILED ? BK * 32 : BK * 2;  // bytes from one stage to the next
   // Of a step's MF products: the reads of fragments are dealt out to the first SPAN; the barrier is behind product BP of a
@@ -141,7 +142,7 @@ __device__ __forceinline__ void dense_block(const DenseBlock& p, unsigned char* 
   for (int i = 0; i < FN; ++i) {
     if constexpr (TILED) {  // a wavefront brings a fragment: 16 rows of one of the stage's two steps
       int row = 32 * i + 16 * (wave >> 1);
-      if constexpr (GATED) {
+      if constexpr (GATED) {  // every half: FN * 8 rows of the gate and their rows of up
         const int in = row % (FN * 16), at = in % (FN * 8);
         row = min(n0 + row / (FN * 16) * (FN * 8) + at, p.N - 16) + (in >= FN * 8 ? p.N : 0);
       } else {
@@ -150,14 +151,7 @@ __device__ __forceinline__ void dense_block(const DenseBlock& p, unsigned char* 
       wsrc[i] = (uint32_t)row * (uint32_t)(p.K * 2) + (uint32_t)((wave & 1) * 1024 + lane * 16);
       continue;
     }
-    int row = 32 * i + 8 * wave + (lane >> 3);
-    if constexpr (GATED) {  // every half: FN * 8 rows of the gate and their rows of up
-      const int in = row % (FN * 16), at = in % (FN * 8);
-      row = min(n0 + row / (FN * 16) * (FN * 8) + at, p.N - 1) + (in >= FN * 8 ? p.N : 0);
-    } else {
-      row = min(row, p.N - 1 - n0);
-    }
-    wsrc[i] = (uint32_t)row * (uint32_t)(p.K * 2) + piece;
+    wsrc[i] = (uint32_t)min(32 * i + 8 * wave + (lane >> 3), p.N - 1 - n0) * (uint32_t)(p.K * 2) + piece;
   }
   auto load = [&](bool w, uint32_t live, uint32_t src, uint32_t k) __attribute__((always_inline)) {
     const u32x4 rsrc = {w ? w_lo : x_lo, w ? w_hi : x_hi, live, 0x00020000u};
@@ -262,7 +256,7 @@ __device__ __forceinline__ void dense_block(const DenseBlock& p, unsigned char* 
       if constexpr (GATED) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          const float gate = TILED ? acc[i][j][e] * sc : acc[i][j][e], up = TILED ? acc[i + FN / 2][j][e] * sc : acc[i + FN / 2][j][e];
+          const float gate = acc[i][j][e] * sc, up = acc[i + FN / 2][j][e] * sc;
           y[e] = gate_act<0>(gate) * up;
         }
       } else {

@@ -1,7 +1,6 @@
 // Dense matrix product of many rows: bfloat16 in and out, float32 accumulate on MFMA.
 //
 //   Y[t, n] = sum_k X[t, k] * W[n, k]  (+ bias[n])
-//   Y[t, f] = silu(gate) * up,  gate/up = the sums of rows f and N + f of W   (GATED)
 //
 // Tiles of 128 x 128 to 256 x 256, each a block's work (dense_block.h).
 #include "dense_block.h"
@@ -31,22 +30,22 @@ __device__ __forceinline__ void tile_of(const DenseArgs& p, int& tm, int& tn) {
   tn = in / rows;
 }
 
-template <int FM, int FN, int RX, int RW, bool GATED, int BLOCKS>
+template <int FM, int FN, int RX, int RW, int BLOCKS>
 __global__ __launch_bounds__(256, BLOCKS) void dense_kernel(DenseArgs p) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
   int tm, tn;
   tile_of(p, tm, tn);
   const int m0 = tm * FM * 32;
-  const DenseBlock b = {p.X, p.W, p.Y, p.bias, nullptr, nullptr, 0, m0, p.M - m0, tn * (GATED ? FN * 16 : FN * 32), p.N, p.K};
-  dense_block<FM, FN, RX, RW, GATED, false>(b, smem);
+  const DenseBlock b = {p.X, p.W, p.Y, p.bias, nullptr, nullptr, 0, m0, p.M - m0, tn * FN * 32, p.N, p.K};
+  dense_block<FM, FN, RX, RW, false, false>(b, smem);
 }
 
-template <int FM, int FN, int RX, int RW, bool GATED, int BLOCKS>
+template <int FM, int FN, int RX, int RW, int BLOCKS>
 int launch(DenseArgs p, int units, hipStream_t s) {
-  constexpr int BM = FM * 32, BN = GATED ? FN * 16 : FN * 32;
-  constexpr uint32_t lds = dense_bytes<FM, FN, RX, RW, GATED>();
+  constexpr int BM = FM * 32, BN = FN * 32;
+  constexpr uint32_t lds = dense_bytes<FM, FN, RX, RW, false>();
   static_assert(lds * BLOCKS <= 160 * 1024, "");
-  const auto k = dense_kernel<FM, FN, RX, RW, GATED, BLOCKS>;
+  const auto k = dense_kernel<FM, FN, RX, RW, BLOCKS>;
   if (const int rc = allow_lds(k, lds)) return rc;
   p.mt = (p.M + BM - 1) / BM;
   p.nt = (p.N + BN - 1) / BN;
@@ -68,37 +67,27 @@ int launch(DenseArgs p, int units, hipStream_t s) {
 
 }  // namespace
 
-// X [M, K], W [N, K] (gated: [2 N, K], gate rows first), Y [M, N], bias [N] or null (not gated): bfloat16, 16-byte aligned
-// rows.  K a multiple of 64, N of 8; a tile's rows of X and all of a gated W have fewer than 2^32 bytes.  act: gate_act's.
-// tile: FM * 16 + FN; units: compute units.
-JLE_API int jle_gemm_dense(const void* X, const void* W, void* Y, const void* bias, int gated, int M, int N, int K, int tile,
-                            int units, hipStream_t s) {
+// X [M, K], W [N, K], Y [M, N], bias [N] or null: bfloat16, 16-byte aligned rows.  K a multiple of 64, N of 8; a tile's rows have
+// fewer than 2^32 bytes.  tile: FM * 16 + FN; units: compute units.
+JLE_API int jle_gemm_dense(const void* X, const void* W, void* Y, const void* bias, int M, int N, int K, int tile, int units, hipStream_t s) {
   if (M <= 0 || N <= 0) return 0;
   if (K < BK || K % BK || N % 8 || units < 8 || ((uintptr_t)X | (uintptr_t)W | (uintptr_t)Y) % 16 || (uintptr_t)bias % 8 ||
-      (long long)K * 512 >= (1ll << 32) || (gated && ((long long)N * K * 4 >= (1ll << 32) || bias != nullptr)))
+      (long long)K * 512 >= (1ll << 32))
     return JLE_BAD_ARG;
   const DenseArgs p = {(const bf16_t*)X, (const bf16_t*)W, (bf16_t*)Y, (const bf16_t*)bias, M, N, K, 0, 0, 1};
-#define GO(FM, FN, RX, RW, BLOCKS)                                          \
-  case FM * 16 + FN:                                                        \
-    if (gated) return launch<FM, FN, RX, RW, true, BLOCKS>(p, units, s);    \
-    return launch<FM, FN, RX, RW, false, BLOCKS>(p, units, s)
-#define GO_PLAIN(FM, FN, RX, RW, BLOCKS) \
-  case FM * 16 + FN:                     \
-    return gated ? JLE_BAD_ARG : launch<FM, FN, RX, RW, false, BLOCKS>(p, units, s)
+#define GO(FM, FN, RX, RW, BLOCKS) \
+  case FM * 16 + FN: return launch<FM, FN, RX, RW, BLOCKS>(p, units, s)
   switch (tile) {
     GO(8, 8, 5, 5, 1);
+    GO(8, 7, 5, 4, 1);
     GO(8, 6, 5, 6, 1);
     GO(6, 8, 6, 5, 1);
+    GO(8, 5, 6, 6, 1);
     GO(8, 4, 6, 6, 1);
+    GO(6, 4, 6, 6, 1);
+    GO(4, 5, 6, 6, 1);
     GO(4, 4, 5, 5, 2);
-    GO_PLAIN(8, 7, 5, 4, 1);
-    GO_PLAIN(8, 5, 6, 6, 1);
-    GO_PLAIN(6, 4, 6, 6, 1);
-    GO_PLAIN(4, 5, 6, 6, 1);
-    case 4 * 16 + 6:
-      return gated ? launch<4, 6, 6, 6, true, 1>(p, units, s) : JLE_BAD_ARG;
   }
 #undef GO
-#undef GO_PLAIN
   return JLE_BAD_ARG;
 }

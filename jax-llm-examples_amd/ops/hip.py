@@ -52,7 +52,7 @@ _SIGNATURES = {
                        _vp, _vp, _i, _i, _i, _i, _i, _vp, _vp, _i, _i, _vp, _i, _i, _i, _i, _f, _f, _vp],
     "jle_moe_align": [_vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _vp],
     "jle_moe_route_align": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _vp],
-    "jle_gemm_dense": [_vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _vp],
+    "jle_gemm_dense": [_vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _vp],
     "jle_gemm_generic": [_vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _vp],
     "jle_gemm_f32_skinny": [_vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _vp],
     "jle_gemm_f32_rows": [_vp, _vp, _vp, _i, _i, _i, _i, _vp],
@@ -1170,12 +1170,10 @@ class HipOps:
     DENSE_TILES = {(8, 8): (1, -1.3, 9.2, 0.960, 0.375), (8, 7): (1, -1.8, 9.2, 0.886, 0.295), (8, 6): (1, -2.0, 9.2, 0.733, 0.256),
                    (6, 8): (1, -0.9, 7.2, 0.783, 0.249), (8, 5): (1, -1.3, 7.6, 0.639, 0.215), (8, 4): (1, 0.2, 4.9, 0.546, 0.204),
                    (6, 4): (1, 0.9, 3.4, 0.459, 0.153), (4, 5): (1, 1.3, 2.5, 0.457, 0.123), (4, 4): (2, 2.3, 0.7, 0.442, 0.503)}
-    DENSE_GATED_TILES = {(8, 8): (1, 2.5, 8.7, 1.019, 0.369), (8, 6): (1, 0.0, 8.3, 0.828, 0.216), (6, 8): (1, 2.7, 4.5, 0.925, 0.189),
-                         (8, 4): (1, 3.2, 2.5, 0.648, 0.172), (4, 6): (1, 6.9, -3.3, 0.705, 0.083), (4, 4): (2, 8.5, -7.6, 0.633, 0.527)}
 
     @staticmethod
     @functools.lru_cache(maxsize=4096)
-    def dense_tile(rows: int, n: int, k: int, gated: bool, units: int = 256) -> int:
+    def dense_tile(rows: int, n: int, k: int, units: int = 256) -> int:
         """The tile of ``gemm_dense.hip`` for ``rows`` rows by ``n`` columns of the result, or 0: the library's product.
 
         The tile is the one whose launch takes the least time by DENSE_TILES, which are fits to 22 numbers of rows by 22
@@ -1187,42 +1185,33 @@ class HipOps:
         5,120 60 | 49; 2,048 of 4,096 x 512 (k) 18.6 | 13.2, where the library's launch alone is 18.  It leaves the library those
         that fill whole rounds of 256 x 256 tiles (8,191 of 4,096 x 4,096 177 | 190, 4,096 of 8,192 x 2,048 96 | 106: there the
         chip's power is what both wait for), and those with too few tiles for its compute units and a long k, which the library
-        cuts along k (704 of 4,096 x 7,168 (k) 51 | 63, 1,024 of 2,048 x 8,192 (k) 49 | 65).  With the gate it is measured against the
-        library's product and the activation's launch: 2,048 rows of 8,192 x 5,120 277 | 247, 953 150 | 123, 8,191 of 14,336 x
-        4,096 1,385 | 1,366, but 97 of 8,192 x 5,120 47 | 65, and with 256 70 | 67."""
-        if rows < 1 or n < 8 or n % 8 or k < 64 or k % 64 or k >= 1 << 23 or gated and 4 * n * k >= 1 << 32:
+        cuts along k (704 of 4,096 x 7,168 (k) 51 | 63, 1,024 of 2,048 x 8,192 (k) 49 | 65)."""
+        if rows < 1 or n < 8 or n % 8 or k < 64 or k % 64 or k >= 1 << 23:
             return 0
-        wide = 2 * n if gated else n  # rows of W
-        small = -(-rows // 128) * -(-wide // 128)
-        if gated:
-            if rows < 256 or small < 0.9 * units:
-                return 0
-        else:
-            if not (rows >= 192 and k <= 2048 or rows >= 256 and small >= (0.93 if k <= 6144 else 1.17) * units):
-                return 0
-            full = -(-rows // 256) * (wide // 256) / units  # rounds of whole tiles of 256 x 256
-            if wide % 256 == 0 and full >= 0.95 and full / math.ceil(full) >= 0.9:
-                return 0
-        tiles = HipOps.DENSE_GATED_TILES if gated else HipOps.DENSE_TILES
+        small = -(-rows // 128) * -(-n // 128)
+        if not (rows >= 192 and k <= 2048 or rows >= 256 and small >= (0.93 if k <= 6144 else 1.17) * units):
+            return 0
+        full = -(-rows // 256) * (n // 256) / units  # rounds of whole tiles of 256 x 256
+        if n % 256 == 0 and full >= 0.95 and full / math.ceil(full) >= 0.9:
+            return 0
 
         def cost(tile):
-            blocks, start, a_round, a_stage, full = tiles[tile]
-            count = -(-rows // (32 * tile[0])) * -(-wide // (32 * tile[1]))
+            blocks, start, a_round, a_stage, full = HipOps.DENSE_TILES[tile]
+            count = -(-rows // (32 * tile[0])) * -(-n // (32 * tile[1]))
             rounds = -(-count // (units * blocks))
             return start + rounds * (a_round + k / 64 * a_stage) + k / 64 * full * count / (units * blocks)
 
-        best = min(tiles, key=cost)
+        best = min(HipOps.DENSE_TILES, key=cost)
         return best[0] * 16 + best[1]
 
-    def _dense(self, h, w, gated: bool = False, bias=None):
-        """``h @ w.T`` (``+ bias``; gated: ``silu(gate) * up``) of many bfloat16 rows by ``gemm_dense.hip``, or None: not its sizes,
+    def _dense(self, h, w, bias=None):
+        """``h @ w.T`` (``+ bias``) of many bfloat16 rows by ``gemm_dense.hip``, or None: not its sizes,
         or not the faster one, or a call that others look into."""
-        if (h.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or h.dim() != 2 or w.dim() != 2 or h.shape[1] != w.shape[1]
-                or gated and w.shape[0] % 2):
+        if h.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or h.dim() != 2 or w.dim() != 2 or h.shape[1] != w.shape[1]:
             return None
         m, k = h.shape
-        n = w.shape[0] // 2 if gated else w.shape[0]
-        tile = HipOps.dense_tile(m, n, k, gated, self._compute_units)
+        n = w.shape[0]
+        tile = HipOps.dense_tile(m, n, k, self._compute_units)
         if (not tile or not h.get_device() == w.get_device() == self._device_index or not (h.is_contiguous() and w.is_contiguous())
                 or _watched() or not (_plain(h) and _plain(w) and _plain(bias))
                 or not h.data_ptr() or not w.data_ptr() or (h.data_ptr() | w.data_ptr()) % 16
@@ -1230,18 +1219,18 @@ class HipOps:
                                          or bias.get_device() != self._device_index or bias.data_ptr() % 8)
                 or torch.is_grad_enabled() and (h.requires_grad or w.requires_grad or bias is not None and bias.requires_grad)):
             return None
-        return self.gemm_dense(h, w, tile, gated, bias)
+        return self.gemm_dense(h, w, tile, bias)
 
-    def gemm_dense(self, h, w, tile: int, gated: bool = False, bias=None):
+    def gemm_dense(self, h, w, tile: int, bias=None):
         """The product of :meth:`_dense` with a tile of ``tile // 16 * 32`` rows of ``h`` by ``tile % 16 * 32`` of ``w``."""
         m, k = h.shape
-        n = w.shape[0] // 2 if gated else w.shape[0]
+        n = w.shape[0]
         self._chk(h, torch.bfloat16, (m, k), "rows")
-        self._chk(w, torch.bfloat16, (2 * n if gated else n, k), "W")
+        self._chk(w, torch.bfloat16, (n, k), "W")
         if bias is not None:
             self._chk(bias, torch.bfloat16, (n,), "bias")
         out = torch.empty(m, n, dtype=torch.bfloat16, device=h.device)
-        self._call("jle_gemm_dense", _p(h), _p(w), _p(out), _p(bias), int(gated), m, n, k, tile, self._compute_units)
+        self._call("jle_gemm_dense", _p(h), _p(w), _p(out), _p(bias), m, n, k, tile, self._compute_units)
         return out
 
     FEW_ROWS = 64
@@ -1300,8 +1289,8 @@ class HipOps:
             product = self.gemm_few if self._few(h, w_gate_up) else self.gemm_skinny
             return product(h, w_gate_up, swiglu=1 + act)  # (the activation in the product's epilogue)
         out = self._dense_float32(h, w_gate_up, act)
-        # (not gemm_dense.hip's epilogue: a launch of 18 us less, but gate and up that are not rounded first took the worst of 64
-        # requests' logits in mixed steps of up to 1,709 rows from 0.0147 of the largest to 0.0151, where 0.015 is allowed)
+        # (gate and up are rounded before the activation: in an epilogue that did not, the worst of 64 requests' logits in mixed steps of
+        # up to 1,709 rows went from 0.0147 of the largest to 0.0151, where 0.015 is allowed)
         return self.silu_mul(self._product(h, w_gate_up), activation) if out is None else out
 
     def _product(self, h, w):

@@ -211,13 +211,13 @@ def test_rows_normed_and_chosen_for_in_one_launch(d, experts, top_k, rows):
     assert HipOps.norm_choose_rows(d, experts, top_k) == rows
 
 
-@pytest.mark.parametrize("rows, n, k, gated, tile", [
-    (2048, 4096, 4096, False, (8, 4)), (2048, 5120, 5120, False, (8, 5)), (2048, 7168, 5120, False, (8, 7)), (2048, 4096, 512, False, (4, 4)),
-    (8191, 4096, 4096, False, None), (4096, 8192, 2048, False, None), (704, 4096, 7168, False, None), (1024, 2048, 8192, False, None),
-    (2048, 8192, 5120, True, (8, 8)), (97, 8192, 5120, True, None), (65, 2048, 2048, False, None), (192, 2048, 2048, False, (4, 4)),
-    (2048, 4096, 4100, False, None), (2048, 4100, 4096, False, None), (0, 4096, 4096, False, None), (2048, 0, 4096, False, None), (2048, 4096, 0, False, None)])
-def test_dense_products_of_many_rows_by_size(rows, n, k, gated, tile):
-    assert HipOps.dense_tile(rows, n, k, gated) == (0 if tile is None else tile[0] * 16 + tile[1])
+@pytest.mark.parametrize("rows, n, k, tile", [
+    (2048, 4096, 4096, (8, 4)), (2048, 5120, 5120, (8, 5)), (2048, 7168, 5120, (8, 7)), (2048, 4096, 512, (4, 4)),
+    (8191, 4096, 4096, None), (4096, 8192, 2048, None), (704, 4096, 7168, None), (1024, 2048, 8192, None),
+    (65, 2048, 2048, None), (192, 2048, 2048, (4, 4)),
+    (2048, 4096, 4100, None), (2048, 4100, 4096, None), (0, 4096, 4096, None), (2048, 0, 4096, None), (2048, 4096, 0, None)])
+def test_dense_products_of_many_rows_by_size(rows, n, k, tile):
+    assert HipOps.dense_tile(rows, n, k) == (0 if tile is None else tile[0] * 16 + tile[1])
 
 
 def test_dense_products_that_are_left_to_the_library():
@@ -227,10 +227,10 @@ def test_dense_products_that_are_left_to_the_library():
                   requires_grad=False)
         return types.SimpleNamespace(**{**of, **other})
 
-    ops = types.SimpleNamespace(_compute_units=256, _device_index=0, gemm_dense=lambda h, w, tile, gated, bias: tile)
+    ops = types.SimpleNamespace(_compute_units=256, _device_index=0, gemm_dense=lambda h, w, tile, bias: tile)
     h, w = at(2048, 4096), at(4096, 4096)
     taken = lambda *a, **kw: HipOps._dense(ops, *a, **kw) is not None
-    assert taken(h, w) and taken(h, w, gated=True) and not taken(h, at(4096, 4032)) and not taken(h, at(4095, 4096), gated=True)
+    assert taken(h, w) and not taken(h, at(4096, 4032))
     for other in (dict(dtype=torch.float32), dict(dim=lambda: 3), dict(get_device=lambda: 1), dict(get_device=lambda: -1),
                   dict(is_contiguous=lambda: False), dict(data_ptr=lambda: 4104), dict(requires_grad=True)):
         assert not taken(at(2048, 4096, **other), w) and not taken(h, at(4096, 4096, **other))
@@ -260,7 +260,7 @@ def test_dense_products_that_others_look_into_are_left_to_the_library():
         return types.SimpleNamespace(dtype=torch.bfloat16, shape=(rows, cols), dim=lambda: 2, get_device=lambda: 0, is_contiguous=lambda: True,
                                      data_ptr=lambda: address, requires_grad=False)
 
-    ops = types.SimpleNamespace(_compute_units=256, _device_index=0, gemm_dense=lambda h, w, tile, gated, bias: tile)
+    ops = types.SimpleNamespace(_compute_units=256, _device_index=0, gemm_dense=lambda h, w, tile, bias: tile)
     h, w = at(2048, 4096), at(4096, 4096)
     taken = lambda h=h, w=w, **kw: HipOps._dense(ops, h, w, **kw) is not None
     assert taken() and not taken(h=Elsewhere(2048, 4096)) and not taken(w=Elsewhere(4096, 4096)) and not taken(h=at(2048, 4096, address=0))

@@ -2074,28 +2074,21 @@ def test_sum_with_factors_of_rows_off_their_16_bytes(ops, d, k):
     assert torch.equal(h, h32.bfloat16())
 
 
-@pytest.mark.parametrize("tile,gated", [(t, False) for t in ((8, 8), (8, 7), (8, 6), (6, 8), (8, 5), (8, 4), (6, 4), (4, 5), (4, 4))]
-                         + [(t, True) for t in ((8, 8), (8, 6), (6, 8), (8, 4), (4, 6), (4, 4))])
-def test_dense_product_of_many_rows(ops, tile, gated):
-    """Every tile: one row and eight columns over, one less, several tiles each way, one to six stages; with a bias and with the gate."""
-    bm, bn = 32 * tile[0], 32 * tile[1] // (2 if gated else 1)
+@pytest.mark.parametrize("tile", [(8, 8), (8, 7), (8, 6), (6, 8), (8, 5), (8, 4), (6, 4), (4, 5), (4, 4)])
+def test_dense_product_of_many_rows(ops, tile):
+    """Every tile: one row and eight columns over, one less, several tiles each way, one to six stages; with a bias."""
+    bm, bn = 32 * tile[0], 32 * tile[1]
     for m, n, k in ((1, 8, 64), (bm, bn, 128), (bm + 1, bn + 8, 192), (2 * bm - 1, 2 * bn - 8, 256), (3 * bm + 17, 9 * bn + 16, 384)):
         g = torch.Generator().manual_seed(m + n + k)
         x = torch.randn(m, k, generator=g).to(DEV, torch.bfloat16)
-        w = (torch.randn(2 * n if gated else n, k, generator=g) * k ** -0.5).to(DEV, torch.bfloat16)
-        bias = None if gated else torch.randn(n, generator=g).to(DEV, torch.bfloat16)
+        w = (torch.randn(n, k, generator=g) * k ** -0.5).to(DEV, torch.bfloat16)
+        bias = torch.randn(n, generator=g).to(DEV, torch.bfloat16)
         want, sums = x.double() @ w.double().t(), (k + 2) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t())
-        for b in (None, bias) if bias is not None else (None,):
-            got = ops.gemm_dense(x, w, tile[0] * 16 + tile[1], gated, b).double()
-            if gated:  # (silu's slope is at most 1.1, its value at most the gate's; its float32 form adds a few roundings)
-                gate, up = want.split(n, 1)
-                y = torch.nn.functional.silu(gate) * up
-                off = 1.1 * sums[:, :n] * up.abs() + gate.abs() * sums[:, n:] + 1.1 * sums[:, :n] * sums[:, n:] + 16 * 2.0 ** -24 * y.abs()
-            else:
-                y = want if b is None else want + b.double()
-                off = sums + 2.0 ** -24 * y.abs()
-            assert ((got - y).abs() <= 2.0 ** -8 * y.abs() + off + 1e-30).all()
-            again = ops.gemm_dense(x[m // 2:].contiguous(), w, 4 * 16 + 4, gated, b)
+        for b in (None, bias):
+            got = ops.gemm_dense(x, w, tile[0] * 16 + tile[1], b).double()
+            y = want if b is None else want + b.double()
+            assert ((got - y).abs() <= 2.0 ** -8 * y.abs() + sums + 2.0 ** -24 * y.abs() + 1e-30).all()
+            again = ops.gemm_dense(x[m // 2:].contiguous(), w, 4 * 16 + 4, b)
             assert torch.equal(again.double(), got[m // 2:])  # (a row's sums have one order whatever the tile and the other rows)
 
 
