@@ -1936,11 +1936,12 @@ class HipOps:
         """Which of ``gemm_stream.hip``'s kernels takes ``rows`` rows in ``groups`` groups (``row_blocks`` blocks of 256 rows
         of W a group): passes of 192 rows or wide tiles of 256.  A block fills a compute unit, so what counts is how many
         rounds of blocks there are on the 256 compute units and how long one takes, per stage of 64 k, microseconds:
-        passes 0.9 + 0.0037 a row, tiles 0.95 + 0.003.  Fewer than 16 row blocks of tiles count in eights, as they are dealt to the
+        passes 0.9 + 0.0037 a row, tiles 0.95 + 0.003 (the tiles' constants are those of the kernel before this one, which took 6 %
+        longer on the average).  Fewer than 16 row blocks of tiles count in eights, as they are dealt to the
         eight chiplets (of 10 groups of 3,072 x 3,072 with 384 rows half of the chiplets get two thirds: 115 | 126). A group's
         rows are taken to scatter about their mean by its root: how they are shared out is known on the device only. With fewer
         than WIDE_GROUPS groups one that is far fuller than the others is what the launch takes, and is better cut in more
-        pieces.  The line was drawn when the tiles took 6 % longer than they do.  Over 34 matrices of 4 to 128 groups with 96 to 900
+        pieces.  Over 34 matrices of 4 to 128 groups with 96 to 900
         rows each, even, drawn, and with 40 % of the rows in one group, the choice between these and :meth:`stream_half`'s is 4.5 %
         from the best; a line drawn anew would be 3.9 % from it, but up to 1.8 times slower at single sizes than this one. Both
         sides measured (passes | tiles, us, drawn groups): 8 groups of 14,336 x 4,096 gate and up with 176 rows 193 | 210, 192
@@ -1973,11 +1974,22 @@ class HipOps:
 
         Measured as :meth:`stream_wide` is.  Passes | these, us, drawn and with 40 % in one: 8 of 2,048 x 4,096 with 128 rows 62 | 46
         and 69 | 57, 224 64 | 59 and 77 | 63, 300 79 | 67 and 79 | 62, 410 82 | 62 and 81 | 67; 16 of 1,024 x 2,048 with 192 46 | 35
-        and 46 | 41, 256 43 | 42 and 47 | 41; 8 of 1,024 x 8,192 with 192 144 | 102 and 144 | 99, but with 128, where passes are cut
-        along k, 55 | 86 and 70 | 103; 8 of 4,096 x 7,168 (not taken) with 256 143 | 139 and 138 | 175."""
+        and 46 | 41, 256 43 | 42 and 47 | 41; 8 of 1,024 x 8,192 with 192 144 | 102 and 144 | 99; 8 of 4,096 x 7,168 (not taken) with 256
+        143 | 139 and 138 | 175.  Where passes can be cut along k see :meth:`cut_passes_pay`."""
         slots = -(-row_blocks // 8) * 8 * groups
         mean = rows / groups
         return groups >= HipOps.WIDE_GROUPS and mean >= 90 and slots <= 192 and slots * (mean / 288 + 0.5) <= 224
+
+    @staticmethod
+    def cut_passes_pay(groups: int, row_blocks: int, k: int, cuts: int, units: int) -> bool:
+        """Whether passes cut along k into ``cuts`` pieces (:meth:`stream_cuts`) are taken before the tiles of :meth:`stream_half`
+        (``row_blocks`` of 128 rows of W a group): with a long k in three pieces or more, or where the tiles would leave three quarters
+        of the ``units`` compute units without a block.  Two pieces gain less than they lose with 40 % of the rows in one group.
+        Cut | tiles, us, drawn groups of 128 and so shared out: 8 of 1,024 x 4,096 37 | 42 and 37 | 51, x 8,192 56 | 86 and 71 | 100; 16
+        of 512 x 4,096 36 | 48 and 40 | 55; 8 of 2,048 x 6,144 68 | 74 and 78 | 93, x 8,192 85 | 99 and 106 | 122; 16 of 1,024 x 8,192 85 |
+        99 and 107 | 120; 10 of 2,048 x 6,144 76 | 77 and 91 | 89; but 8 of 2,048 x 4,096 61 | 48 and 70 | 60, x 5,120 59 | 59 and
+        70 | 71; 8 of 1,536 x 4,096 45 | 45 and, with 160, 66 | 50; 8 of 3,072 x 8,192, in two, 96 | 103 and, with 160, 150 | 119."""
+        return cuts > 1 and (k >= 6144 and cuts >= 3 or 4 * groups * row_blocks <= units)
 
     CUT_STAGES = 64  # stages of 64 k from which on it pays
 
@@ -2025,14 +2037,16 @@ class HipOps:
         out = torch.empty(m, nout // 2 if swiglu else nout, dtype=torch.float32 if out_f32 else torch.bfloat16,
                           device=a.device)
         wide, among = 0, m if expected is None else expected
+        cut, cuts = (0, 1) if swiglu else self.stream_cuts(among, g, -(-nout // 256), k, self._compute_units)
         if (offsets is not None and not out_f32 and a.numel() < 2 ** 31 and nout * k < 2 ** 31
                 and not (a.data_ptr() | b.data_ptr()) % 16):
-            wide = 2 if not swiglu and self.stream_half(among, g, -(-nout // 128)) else self.stream_wide(among, g, -(-nout // 256))
-        pieces, cut, cuts = None, 0, 1
-        if not wide and not swiglu:
-            cut, cuts = self.stream_cuts(among, g, -(-nout // 256), k, self._compute_units)
-            if cuts > 1:  # (tiles of 16 KB)
-                pieces = torch.empty(self._query("jle_gemm_stream_room", m, g) * cut * cuts << 14, dtype=torch.uint8, device=a.device)
+            half = not swiglu and self.stream_half(among, g, -(-nout // 128)) and not self.cut_passes_pay(g, -(-nout // 128), k, cuts, self._compute_units)
+            wide = 2 if half else self.stream_wide(among, g, -(-nout // 256))
+        pieces = None
+        if wide:
+            cut, cuts = 0, 1
+        elif cuts > 1:  # (tiles of 16 KB)
+            pieces = torch.empty(self._query("jle_gemm_stream_room", m, g) * cut * cuts << 14, dtype=torch.uint8, device=a.device)
         self._call("jle_gemm_stream", _p(a), _p(b), _p(out), _p(offsets), _p(a_rows), _p(scale), int(swiglu),
                    int(relu2), int(out_f32), m, nout, k, g, int(wide), _p(pieces), cut, cuts, self._compute_units)
         return out

@@ -146,6 +146,26 @@ def test_which_blocks_of_a_product_in_passes_are_cut(rows, groups, blocks, k, un
     assert HipOps.stream_cuts(rows, groups, blocks, k, units) == cut
 
 
+@pytest.mark.parametrize("groups, nout, k, rows, way", [
+    (8, 1024, 8192, 128, "cut"), (8, 1024, 8192, 96, "cut"), (8, 1024, 8192, 192, "tiles"), (8, 1024, 4096, 160, "cut"), (16, 512, 4096, 128, "cut"),
+    (8, 2048, 4096, 128, "tiles"), (8, 2048, 5120, 128, "tiles"), (8, 2048, 6144, 128, "cut"), (16, 1024, 8192, 128, "cut"), (16, 1024, 4096, 128, "tiles"),
+    (8, 1536, 4096, 160, "tiles"), (8, 1536, 8192, 160, "cut"), (8, 3072, 8192, 160, "tiles"), (24, 1024, 8192, 128, "tiles"), (8, 2048, 2048, 128, "tiles"),
+    (8, 14336, 4096, 410, "wide"), (8, 4096, 7168, 48, "cut"), (8, 4096, 2048, 64, "whole")])
+def test_plain_products_of_groups_by_size(monkeypatch, groups, nout, k, rows, way):
+    """Of passes, passes cut along k and the two kinds of tiles the one that a call of drawn groups launches."""
+    called = []
+    ops = types.SimpleNamespace(_compute_units=256, _chk=lambda *a: None, stream_supported=lambda *a: True, _query=lambda *a: 1,
+                                _call=lambda name, *a: called.append((a[13], a[16])))
+    for rule_ in ("stream_half", "stream_wide", "stream_cuts", "cut_passes_pay"):
+        setattr(ops, rule_, getattr(HipOps, rule_, lambda *a: False))
+    a = torch.empty(1, dtype=torch.bfloat16).expand(groups * rows, k)
+    b = torch.empty(1, dtype=torch.bfloat16).expand(groups, nout, k)
+    monkeypatch.setattr(torch, "empty", lambda *a, **kw: None)
+    HipOps.gemm_stream(ops, a, b, offsets=torch.zeros(groups + 1, dtype=torch.int32))
+    assert called == [{"wide": (1, 1), "tiles": (2, 1), "whole": (0, 1), "cut": (0, HipOps.stream_cuts(groups * rows, groups, -(-nout // 256), k, 256)[1])}[way]]
+    assert (called[0][1] > 1) == (way == "cut")
+
+
 @pytest.mark.parametrize("n, k, least, most", [(16000, 2048, 5, 64), (28672, 4096, 5, 64), (28688, 4096, 5, 32), (32768, 2048, 5, 32),
                                                  (32784, 2048, 5, 16), (50000, 3072, 5, 16), (65536, 4096, 5, 24), (202048, 5120, 5, 24)])
 def test_output_heads_by_size(n, k, least, most):
