@@ -126,7 +126,7 @@ __device__ __forceinline__ void dense_block(const DenseBlock& p, unsigned char* 
   const int nstage = p.K / BK;
   const int* const a_rows = TILED ? p.a_rows : nullptr;
   const uint64_t xa = (uint64_t)(uintptr_t)(a_rows != nullptr ? p.X : p.X + (size_t)m0 * p.K);
-  const uint64_t wa = (uint64_t)(uintptr_t)(p.W + (GATED ? (size_t)0 : (size_t)n0 * p.K));
+  const uint64_t wa = (uint64_t)(uintptr_t)(p.W + (size_t)n0 * p.K);
   auto same = [](uint32_t v) __attribute__((always_inline)) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); };
   uint32_t x_lo = same((uint32_t)xa), x_hi = same((uint32_t)(xa >> 32)), w_lo = same((uint32_t)wa), w_hi = same((uint32_t)(wa >> 32));
   asm volatile("s_nop 4" : "+s"(x_lo), "+s"(x_hi), "+s"(w_lo), "+s"(w_hi));  // (before a load reads what vector instructions wrote)
@@ -144,7 +144,7 @@ __device__ __forceinline__ void dense_block(const DenseBlock& p, unsigned char* 
       int row = 32 * i + 16 * (wave >> 1);
       if constexpr (GATED) {  // every half: FN * 8 rows of the gate and their rows of up
         const int in = row % (FN * 16), at = in % (FN * 8);
-        row = min(n0 + row / (FN * 16) * (FN * 8) + at, p.N - 16) + (in >= FN * 8 ? p.N : 0);
+        row = min(row / (FN * 16) * (FN * 8) + at, p.N - 16 - n0) + (in >= FN * 8 ? p.N : 0);
       } else {
         row = min(row, p.N - 16 - n0);
       }

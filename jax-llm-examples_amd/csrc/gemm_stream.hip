@@ -533,8 +533,8 @@ JLE_API int jle_gemm_stream_supported(int Nout, int K, int swiglu) {
 JLE_API int jle_gemm_stream_room(int M, int G) { return (M >> 4) + 2 * (M / kRows + G); }
 
 // X [*, K] bf16, W [G, Nout, K] bf16 in the streaming layout, Y [M, Nout] (or [M, Nout / 2] with swiglu) bf16 or
-// float32; X must have fewer than 2^32 elements (wide: 2^32 bytes).  wide: wide_kernel (groups, bfloat16 out, a group's W of fewer than
-// 2^32 bytes), 2 (plain): with FN = 4.
+// float32; X must have fewer than 2^32 elements (wide: 2^32 bytes).  wide: wide_kernel (groups, bfloat16 out, K below 2^23; with
+// swiglu half of a group's W, and 128 rows more, have fewer than 2^32 bytes), 2 (plain): with FN = 4.
 // act 1 (plain): max(., 0)^2 of the rounded sums.  cuts > 1 (plain, not wide): the last `cut` of a group's blocks of 256 rows of
 // W are cut into `cuts` pieces along k; pieces: place for jle_gemm_stream_room(M, G) * cut * cuts tiles of 16 KB.
 // Blocks are 8 wavefronts (two per SIMD, one block per compute unit): measured against 4, 5 and 6 on expert
@@ -545,7 +545,7 @@ JLE_API int jle_gemm_stream(const void* X, const void* W, void* Y, const int* of
   if (M <= 0 || Nout <= 0) return 0;
   if (wide) {
     if (offsets == nullptr || out_f32 || G < 1 || G > 65535 || !jle_gemm_stream_supported(Nout, K, swiglu) ||
-        (long long)Nout * K * 2 >= (1ll << 32) || ((uintptr_t)X | (uintptr_t)W | (uintptr_t)Y) % 16)
+        K >= 1 << 23 || (swiglu && ((long long)Nout / 2 + 128) * K >= (1ll << 31)) || ((uintptr_t)X | (uintptr_t)W | (uintptr_t)Y) % 16)
       return JLE_BAD_ARG;
     const WideArgs p = {(const bf16_t*)X, (const bf16_t*)W, (bf16_t*)Y, offsets, a_rows, scale, act, Nout, K, G, 0};
     if (swiglu) return launch_wide<8, true>(p, M, s);

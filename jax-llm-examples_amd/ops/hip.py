@@ -2038,8 +2038,8 @@ class HipOps:
                           device=a.device)
         wide, among = 0, m if expected is None else expected
         cut, cuts = (0, 1) if swiglu else self.stream_cuts(among, g, -(-nout // 256), k, self._compute_units)
-        if (offsets is not None and not out_f32 and a.numel() < 2 ** 31 and nout * k < 2 ** 31
-                and not (a.data_ptr() | b.data_ptr()) % 16):
+        if (offsets is not None and not out_f32 and a.numel() < 2 ** 31 and k < 2 ** 23
+                and not (swiglu and (nout // 2 + 128) * k >= 2 ** 31) and not (a.data_ptr() | b.data_ptr()) % 16):
             half = not swiglu and self.stream_half(among, g, -(-nout // 128)) and not self.cut_passes_pay(g, -(-nout // 128), k, cuts, self._compute_units)
             wide = 2 if half else self.stream_wide(among, g, -(-nout // 256))
         pieces = None

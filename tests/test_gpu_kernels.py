@@ -2168,3 +2168,23 @@ def test_heads_of_more_tokens_than_a_launch_takes(ops):
     assert torch.equal(ops.heads_prepare(rows, hq, 1, 1, d, d, d, prep, positions, None, None), got[0][0])
     values = got[0][1][:, 1].reshape(-1, d, ps)[(slots // ps).long(), :, (slots % ps).long()]
     assert torch.equal(values, rows[:, -d:])
+
+
+def test_wide_tiles_of_weights_of_more_than_four_gib(ops, monkeypatch):
+    """A group's matrix past 2^32 bytes goes to the tiles where the rule says so, plain and with the gate, and gives the passes' bits."""
+    k, nout, m = 4096, (1 << 19) + 32, 70
+    w = torch.empty(1, nout, k, dtype=torch.bfloat16, device=DEV)
+    w.normal_(std=0.02, generator=torch.Generator(DEV).manual_seed(1))
+    x = _rand(m, k, dt=torch.bfloat16, seed=2)
+    off = torch.tensor([0, m], dtype=torch.int32, device=DEV)
+    took, call = [], ops._call
+    monkeypatch.setattr(ops, "_call", lambda name, *a: (took.append(a[13]), call(name, *a))[1])
+    monkeypatch.setattr(ops, "stream_cuts", lambda *a: (0, 1))
+    for swiglu in (False, True):
+        got = []
+        for half, wide in ((False, False), (False, True)) + (() if swiglu else ((True, False),)):
+            monkeypatch.setattr(ops, "stream_half", lambda *a: half)
+            monkeypatch.setattr(ops, "stream_wide", lambda *a: wide)
+            got.append(ops.gemm_stream(x, w, offsets=off, swiglu=swiglu, rows=m))
+        assert all(torch.equal(g, got[0]) for g in got[1:]) and got[0].isfinite().all() and got[0][-1, -16:].any()
+    assert took == [0, 1, 2, 0, 1]
