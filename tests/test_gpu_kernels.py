@@ -1452,7 +1452,10 @@ def test_weight_streaming_product_of_fuller_groups(ops, counts, nout, k, tiled):
     ([128, 129, 160, 161, 192, 193], 528, 512, False),      # every number of row tiles; a second block of W of one tile
     ([224, 225, 256, 257, 512, 513, 700], 544, 768, True),  # one, two and three tiles of rows; gate and up
     ([3, 0, 280] * 50, 64, 256, False),                     # more groups than a look takes
-    ([256], 2304, 256, True)])                              # more than eight blocks of W
+    ([256], 2304, 256, True),                               # more than eight blocks of W
+    # every number of row tiles and one row more, full tiles among them, over twelve stages: every ring goes round more than once
+    ([1, 32, 64, 65, 96, 97, 128, 129, 160, 161, 192, 193, 224, 225, 256, 257, 512], 288, 768, False),
+    ([1, 32, 64, 65, 96, 97, 128, 129, 160, 161, 192, 193, 224, 225, 256, 257, 512], 288, 768, True)])
 def test_wide_tiles_of_the_weight_streaming_product(ops, monkeypatch, counts, nout, k, swiglu):
     """The kernel for many rows a group gives the bits of the one that takes them in passes (the same sums in the same
     order), with the rows gathered and scaled; that one is tested against the general product elsewhere."""
@@ -1464,6 +1467,7 @@ def test_wide_tiles_of_the_weight_streaming_product(ops, monkeypatch, counts, no
     rows = torch.randperm(m + 3, generator=torch.Generator().manual_seed(3))[:m].int().to(DEV)
     scale = _rand(m, seed=4)
     got = []
+    monkeypatch.setattr(ops, "stream_half", lambda *a: False)
     for wide in (False, True):
         monkeypatch.setattr(ops, "stream_wide", lambda *a, wide=wide: wide)
         got.append(ops.gemm_stream(x, w, offsets=off, a_rows=rows, scale=scale, swiglu=swiglu, rows=m))
@@ -1473,7 +1477,8 @@ def test_wide_tiles_of_the_weight_streaming_product(ops, monkeypatch, counts, no
 @pytest.mark.parametrize("counts,nout,k", [
     ([1, 0, 32, 33, 64, 65, 96, 97, 128, 129], 128, 256),        # every number of row tiles
     ([160, 161, 192, 193, 224, 225, 256, 257], 144, 512),        # a second block of W of one tile
-    ([288, 0, 289, 576, 577, 900], 1168, 256)])                  # the most rows of a tile and one more; more than eight blocks of W
+    ([288, 0, 289, 576, 577, 900], 1168, 256),                   # the most rows of a tile and one more; more than eight blocks of W
+    ([1, 32, 64, 65, 96, 97, 128, 129, 160, 161, 192, 193, 224, 225, 256, 257, 288, 289, 576], 144, 768)])  # twelve stages
 def test_narrower_wide_tiles_of_the_weight_streaming_product(ops, monkeypatch, counts, nout, k):
     """The bits of the kernel that takes the rows in passes, rows gathered and scaled; rows that no group has are left alone."""
     from jax_llm_examples_amd.ops.layout import tile_
@@ -2102,19 +2107,57 @@ def test_dense_product_keeps_what_is_not_a_number_in_its_row(ops):
     assert got[299].isnan().all() and not got[7].isfinite().any() and torch.equal(got[keep], want[keep])
 
 
-def test_dense_products_replayed(ops):
-    """In a graph, pass after pass with other rows in between."""
+def _dense_calls(ops, monkeypatch):
+    """The sizes that the kernel of many rows is called with from here on."""
+    called, kernel = [], ops.gemm_dense
+    monkeypatch.setattr(ops, "gemm_dense", lambda h, w, *a, **kw: (called.append((h.shape[0], *w.shape)), kernel(h, w, *a, **kw))[1])
+    return called
+
+
+def test_dense_products_replayed(ops, monkeypatch):
+    """In a graph, pass after pass with other rows in between; the kernel of many rows is what the graph holds."""
     x, w = torch.randn(512, 1024, device=DEV).bfloat16(), torch.randn(2048, 1024, device=DEV).bfloat16()
     ops.linear(x, w)
     graph = torch.cuda.CUDAGraph()
+    called = _dense_calls(ops, monkeypatch)
     with torch.cuda.graph(graph):
         y = ops.linear(x, w)
         z = ops.swiglu_linear(y[:, :1024].contiguous(), w)
+    assert called == [(512, 2048, 1024)] * 2
+    sums = lambda a: 2.0 ** -8 * (a.double() @ w.double().t()).abs() + 1026 * 2.0 ** -24 * (a.double().abs() @ w.double().abs().t())
     for _ in range(3):
         x.copy_(torch.randn(512, 1024, device=DEV))
         graph.replay()
         torch.cuda.synchronize()
+        assert ((y.double() - x.double() @ w.double().t()).abs() <= sums(x)).all()
         assert torch.equal(y, ops.linear(x, w)) and torch.equal(z, ops.swiglu_linear(y[:, :1024].contiguous(), w))
+
+
+def test_which_products_of_many_rows_are_the_dense_kernels(ops, monkeypatch):
+    """Plain, with a bias, under the activation, and a latent's keys and values; not where a gradient is wanted or a mode looks on."""
+    from torch.utils.flop_counter import FlopCounterMode
+    from jax_llm_examples_amd.engine.batch import GroupContext
+    called = _dense_calls(ops, monkeypatch)
+    x, w = torch.randn(384, 512, device=DEV).bfloat16(), torch.randn(1024, 512, device=DEV).bfloat16()
+    bias = torch.randn(1024, device=DEV).bfloat16()
+    for call in (lambda: ops.linear(x, w), lambda: ops.linear_bias(x, w, bias)[0], lambda: ops.swiglu_linear(x, w)):
+        del called[:]
+        call()
+        assert called == [(384, 1024, 512)]
+    del called[:]
+    ops.linear(x, w.requires_grad_())
+    with torch.no_grad(), FlopCounterMode(display=False) as seen:
+        ops.linear(x, w)
+    assert not called and seen.get_total_flops() == 2 * 384 * 1024 * 512
+    n, H, R, ps = 256, 4, 512, 16
+    zeros = lambda *s: torch.zeros(*s, dtype=torch.bfloat16, device=DEV)
+    table = torch.arange(n // ps, dtype=torch.int32, device=DEV).view(1, -1)
+    pos, seg = torch.arange(n, dtype=torch.int32, device=DEV), torch.zeros(n, dtype=torch.int32, device=DEV)
+    meta = GroupContext(block_table=None, slot_mapping=None, width=n // ps, retention=("all",), seg_lens=[n], seg_starts=[0])
+    monkeypatch.setattr(ops, "LATENT_EXPAND_PAIRS", 0)
+    assert ops.latent_attention_expanded(zeros(n, H, 192), 128, zeros(H * 128, R), zeros(H * 128, R), zeros(n // ps, ps, R),
+                                         zeros(n // ps, ps, 64), table, pos, seg, None, 0.1, meta) is not None
+    assert called == [(n, H * 128, R), (H * 128, n, R)]
 
 
 @pytest.mark.parametrize("dt", DT)
