@@ -1179,8 +1179,9 @@ class HipOps:
         The tile is the one whose launch takes the least time by DENSE_TILES, which are fits to 22 numbers of rows by 22
         matrices, each with every tile (what they say is a twentieth off, and the choice 2.4 % behind the best tile on the average).
 
-        Of the library's products it takes those that it does faster, 1.15 times on the average (library | this kernel, us, weights
-        not in the caches): 2,048 rows of 4,096 x 4,096 58 | 54, of 5,120 x 5,120 89 | 79, of 7,168 x 5,120 120 | 103, of 4,096 x
+        Of the library's products it takes those that it does faster, 1.15 times on the average; over 300 other sizes of up to 8,192
+        rows, odd ones among them, 1.34 times, of which 13 are 5 to 9 % slower (876 rows of 28,672 x 4,096 173 | 185; no line that
+        leaves them out keeps what lies beside them).  Library | this kernel, us, weights not in the caches: 2,048 rows of 4,096 x 4,096 58 | 54, of 5,120 x 5,120 89 | 79, of 7,168 x 5,120 120 | 103, of 4,096 x
         14,336 (k) 208 | 181, of 2,048 x 2,048 22 | 20, of 18,560 x 4,096 339 | 239; 1,024 of 5,120 x 5,120 60 | 52, 608 of 7,168 x
         5,120 60 | 49; 2,048 of 4,096 x 512 (k) 18.6 | 13.2, where the library's launch alone is 18.  It leaves the library those
         that fill whole rounds of 256 x 256 tiles (8,191 of 4,096 x 4,096 177 | 190, 4,096 of 8,192 x 2,048 96 | 106: there the
